@@ -95,14 +95,21 @@ int lr_ladder_norms(const void* resid_in, const void* d1, const void* d2, const 
  * (utils.py:146, 148), wqkv1 (utils.py:311), output (gpt_ladder_TP.py:283).
  * K % 8 == 0.  The kernel is chosen from the shape: M <= 4 (and M <= 8 with act_swiglu) the
  * weight-streaming GEMV (v_dot2 on packed pairs, every weight read once); 4 < M <= 64 the
- * weight-streaming matrix-core kernel of lr_linear_multi; M >= 512 on a large enough grid the
- * 256 x 256 tile matrix-core GEMM; everything else the 128 x 128 tile matrix-core GEMM.  All of
- * them accumulate in fp32 and round once; the summation order, hence the last bit, depends on the
- * kernel.
+ * weight-streaming matrix-core kernel of lr_linear_multi; beyond that the matrix-core GEMM, in tiles
+ * that its shape picks.  All of them accumulate in fp32 and round once; the summation order, hence the
+ * last bit, depends on the kernel.
  * act_swiglu != 0: x is taken to be [M, 2K] = [u | g] (row stride ldx) and the kernel consumes
  * bf16( bf16(silu(g)) * u ) in its place -- w2(silu(g) * u), utils.py:147-148. */
 int lr_linear(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, int act_swiglu,
               lr_stream_t stream);
+
+/* lr_linear (act_swiglu = 0) with memory for partial sums: where the tiles of the matrix-core GEMM would leave compute
+ * units idle, tiles are cut along K, the pieces' fp32 sums go to `scratch` and a second launch adds them, in a fixed order.
+ * Any size is legal, a larger one allows more pieces; lr_linear_scratch_bytes(M) bytes are always enough (0: none would be
+ * used).  Calls that may overlap need memory of their own.  No counterpart in the reference. */
+size_t lr_linear_scratch_bytes(int M);
+int lr_linear_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, void* scratch,
+                      size_t scratch_bytes, lr_stream_t stream);
 
 /* lr_linear with the launch configuration of the GEMV given by the caller instead of chosen from
  * the shape: gemv_cfg = rows per wave * 100 + K-split * 10 + unroll, one of 144, 212, 222, 242, 244,
@@ -152,21 +159,25 @@ int lr_linear_multi(const lr_projection_t* projections, int n_projections, int M
  * y[M, N] = x[M, K] w[N, K]^T with N = (n_head + 2 n_kv_head) * head_dim, then q rotated in y, rotated k and
  * v stored at slot pos[s] of the caches, k and v left as projected in y (Attention.forward, utils.py:188-198, and
  * KVCache.update, :50-59) -- bit for bit what lr_linear followed by lr_rope_kv_write (table_is_gathered = 0)
- * leaves, in one launch of the prefill GEMM where that kernel applies (M >= 512 and enough tiles), in those two
- * calls otherwise.  A position outside the cache or the table sets *rope->err = LR_DEV_POS_RANGE and leaves that
+ * leaves, in the output pass of the prefill GEMM (M > 64), in those two calls otherwise.  A position outside the cache or the table sets *rope->err = LR_DEV_POS_RANGE and leaves that
  * row as projected.  ldy % 8 == 0. */
 int lr_linear_rope_kv(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int K, int S,
                       const lr_rope_kv_t* rope, lr_stream_t stream);
+/* The same with memory for partial sums, as lr_linear_scratch is lr_linear. */
+int lr_linear_rope_kv_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int K, int S,
+                              const lr_rope_kv_t* rope, void* scratch, size_t scratch_bytes, lr_stream_t stream);
 
 /* The MLP's first projection with the activation applied on the way out (utils.py:145-148):
  *     y[M, I] = bf16( bf16(silu(g)) * u ),  [u | g] = bf16(x w^T),  w [2 I, K] = [up; gate] rows, N = 2 I.
- * M <= 64: lr_linear_multi's LR_EPI_SWIGLU; M >= 512 on a large enough grid: the 256 x 256 tile
- * matrix-core GEMM on tiles of 128 row PAIRS (a lane holds both halves of a pair); otherwise the
- * projection goes to `scratch` ([M, N] bf16, scratch_bytes >= 2 M N, then ldy must equal I) and
- * lr_swiglu follows.  scratch may be NULL when one of the first two cases applies.  Same bits as
- * lr_linear followed by lr_swiglu. */
+ * M <= 64: lr_linear_multi's LR_EPI_SWIGLU; beyond: the matrix-core GEMM on row PAIRS (a lane holds both
+ * halves of a pair).  `scratch` ([M, N] bf16, scratch_bytes >= 2 M N) may be NULL for M <= 64 and for
+ * M >= 512 with at least 192 tiles of 256 rows x 128 pairs; it holds the projection where a shape is
+ * served by lr_linear followed by lr_swiglu.  Same bits as those two. */
 int lr_linear_swiglu_out(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K,
                          void* scratch, size_t scratch_bytes, lr_stream_t stream);
+/* The same with memory for partial sums (`sums`), as lr_linear_scratch is lr_linear. */
+int lr_linear_swiglu_out_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K,
+                                 void* scratch, size_t scratch_bytes, void* sums, size_t sums_bytes, lr_stream_t stream);
 
 /* lr_attn_decode and one projection of lr_linear_multi in ONE launch: the first workgroups of the grid are the
  * attention's (split, kv head, sequence) items, the rest the bands of the projection, so the projection's weight

@@ -1,7 +1,9 @@
-// LDS-tiled MFMA bf16 GEMM for prefill (and for decode batches above 8 rows):
-//   y[m, n] = bf16( sum_k x[m, k] * w[n, k] ),  fp32 accumulation in v_mfma_f32_32x32x16_bf16.
+// Matrix-core bf16 GEMMs for prefill and for more than 64 rows:
+//   y[m, n] = bf16( sum_k x[m, k] * w[n, k] ),  fp32 accumulation.
+// k_gemm_dma (below) is the one that matters; k_gemm here serves an input that is activated on its way in, and rows longer
+// than the 2 GiB offsets of k_gemm_dma's requests reach.
 //
-// Workgroup tile 128 x 128 x 64, four waves in a 2 x 2 arrangement, each wave owning a 64 x 64
+// k_gemm: v_mfma_f32_32x32x16_bf16, workgroup tile 128 x 128 x 64, four waves in a 2 x 2 arrangement, each wave owning a 64 x 64
 // block = 2 x 2 MFMA tiles (64 accumulator VGPRs).  Both operands are K-contiguous in memory, so
 // the same staging path serves them: 128-bit global loads -> registers -> LDS rows padded by 16
 // bytes (stride 144 B keeps ds_read_b128 of 16 consecutive rows on distinct banks) -> 128-bit LDS
@@ -129,30 +131,41 @@ __global__ __launch_bounds__(256) void k_gemm(const u16* __restrict__ x, int64_t
 }
 
 // ---------------------------------------------------------------------------------------------
-// Large-tile variant for prefill-sized problems (M >= 512): workgroup tile 256 x 256 x 64, four
-// waves in a 2 x 2 arrangement, each owning 128 x 128 = 4 x 4 MFMA tiles (256 accumulator
-// registers; one workgroup per CU, so a wave has the whole 512-register budget).  The point is LDS
-// traffic: a 64 x 64 wave tile reads 1 KiB of LDS per MFMA, which at 128 B/clk per CU takes as long
-// as the MFMAs themselves; a 128 x 128 wave tile reads half of that.  Staging is the same as in
-// k_gemm (128-bit global loads -> registers -> padded LDS rows, double-buffered, next tile's
-// loads in flight during the multiply).  Tiles are dealt so that the 32 workgroups an XCD runs
-// together cover 4 row tiles x 8 column tiles: they share operand rows in that XCD's L2
-// (blockIdx % 8 is the XCD), which keeps the HBM demand ~5x below the L2 demand.
+// The prefill GEMM.  A workgroup of four waves (2 x 2) multiplies a tile of 128 AH input rows x 128 BH weight rows;
+// AH x BH is 2 x 2, 1 x 2 or 1 x 1 (gemm_plan picks).  Bound: the matrix cores, at the clock the chip's power allows --
+// 16384 x 4096 x 14336: 1.50 PFLOP/s, matrix cores busy 86 % of the cycles at 1.57 GHz -- from a few hundred rows on; the
+// weights' HBM traffic below.
+//
+// Operands go from memory to LDS directly (buffer_load ... lds, 16 bytes per lane, 8 rows x 64 k per instruction): no
+// registers, no LDS write instructions.  An instruction fills 1 KiB of LDS in lane order, so rows cannot be padded; the
+// sixteen-byte groups of a row are exchanged instead (group g of row r lies at g ^ (r & 7)), by the address a lane loads
+// from and again by the address a fragment is read at: conflict-free for the 16-row fragments of
+// v_mfma_f32_16x16x32_bf16.
+//
+// A k-tile is 64 elements; its operand rows come in two halves each (A: input rows, B: weight rows) and the tile's four
+// quarter products follow one another in four phases, (A0 B0) (A0 B1) (A1 B1) (A1 B0).  Every phase reads ONE half from
+// LDS into registers for a later phase and requests the half of two k-tiles ahead into the LDS slot that the phase before
+// it emptied: a request has seven phases to land, a slot is read in exactly one phase, and one barrier per phase orders
+// both.  The reads and requests stand between the matrix instructions, one at a time, and every request is made whatever
+// the tile (a k-tile past the end is a resource of no records: zeros, no traffic), so the waits are exact.  The next
+// k-tile's A0 and B0 take the registers that A0 and B1 leave, so B0 and B1 change registers from one k-tile to the next:
+// the loop walks two.
+//
+// Before (128 x 128 wave tiles of v_mfma_f32_32x32x16_bf16, operands staged through registers and padded LDS rows):
+// 16384 rows x (N x K), us before / now: 6144 x 4096 646 / 560, 4096 x 4096 428 / 381, 28672 x 4096 with SwiGLU 3112 /
+// 2755, 4096 x 14336 1462 / 1281.  The chip is power-limited under either: with the same loop on 32x32x16 instructions the
+// matrix cores were busy 92 % of the cycles at 1.43 GHz (1337 us): twice the accumulator traffic per product.  The matrix
+// instruction is assembler text because its accumulator has to be one register block in and out: left to the compiler,
+// 180 accumulator moves per two k-tiles (1.15 PFLOP/s).
 // ---------------------------------------------------------------------------------------------
-constexpr int GM = 256, GN = 256;
-
-// KTAIL: K is not a multiple of the 64-element k-tile, so the last tile needs a per-lane range check.  Without it the
-// k position of a load is a scalar added by the load instruction itself and the row part of the address never
-// changes: no vector instruction per load (with the check: add, select and a 16-register offset update per tile,
-// ~60 vector instructions that the matrix instructions wait behind).
-// ROPE: the projection is the fused q/k/v projection of a prefill (row b * S + s sits at position rpos[s]) and its
-// output pass does what k_rope_kv_write would do to the stored rows: q rotated in y, rotated k and plain v into the
-// caches, k and v left as projected in y; a position outside the cache or the table sets the error word and leaves
-// the plain row.
-struct GemmRope {
+struct GemmRope {   // the projection is the fused q/k/v projection of a prefill: see lr_linear_rope_kv
+  const u16* table;
+  const int32_t* pos;
+  u16 *k_cache, *v_cache;
+  int32_t* err;
   int S, Hq, Hkv, hd, Smax, block_size;
 };
-// GROUP: the rows of a tile are entries of a list, tile (matrix, first entry, entries) as a device table says: input row
+// The rows of a tile are entries of a list, tile (matrix, first entry, entries) as a device table says: input row
 // entry / xdiv, output row entry, weights of one of several matrices that lie `wstride` elements apart.
 struct GemmGroup {
   const int32_t* tiles;    // [][3]
@@ -161,493 +174,534 @@ struct GemmGroup {
   int xdiv;
   int64_t wstride;
 };
-template <bool KTAIL, bool ROPE, bool GROUP = false>
-__global__ __launch_bounds__(256) void k_gemm_big(const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
-                                                  u16* __restrict__ y, int64_t ldy, int M, int N, int K, int tm,
-                                                  int tn, int pair_off, const u16* __restrict__ rtable,
-                                                  const int32_t* __restrict__ rpos, u16* __restrict__ rk,
-                                                  u16* __restrict__ rv, int32_t* rerr, const GemmRope rp,
-                                                  const GemmGroup gp = {}) {
-  extern __shared__ __attribute__((aligned(16))) u16 gsm[];
-  u16* xs = gsm;                      // [2][GM * LDT]
-  u16* ws = gsm + 2 * GM * LDT;       // [2][GN * LDT]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  // ---- tile of this workgroup
-  int mt, nt;
-  int32_t* const entry = reinterpret_cast<int32_t*>(gsm + 2 * (GM + GN) * LDT);   // (GROUP) the tile's entries
-  if constexpr (GROUP) {   // an XCD takes a contiguous run of tiles, a row tile's column tiles one after the other
-    const int n = gridDim.x, xcd = blockIdx.x & 7, base = n >> 3, rem = n & 7;
-    const int id = xcd * base + (xcd < rem ? xcd : rem) + (blockIdx.x >> 3);
-    mt = id / tn;
-    nt = id - mt * tn;
-    if (mt >= gp.ntiles[0]) return;
-    const int32_t* tile = gp.tiles + 3 * mt;
-    w += tile[0] * gp.wstride;
-    M = tile[2];
-    entry[tid] = gp.entries[tile[1] + (tid < M ? tid : 0)];
-    mt = 0;
-    __syncthreads();
-  } else {
-    const int id = blockIdx.x;
-    if (tm % 32 == 0) {  // XCD-aware: XCD x owns a band of tm / 8 row tiles, walked 4 row tiles x all column tiles at a time
-      const int xcd = id & 7, j = id >> 3;
-      const int per_group = 4 * tn;
-      const int grp = j / per_group, r = j - grp * per_group;
-      mt = xcd * (tm / 8) + grp * 4 + (r & 3);
-      nt = r >> 2;
-    } else {
-      mt = id / tn;
-      nt = id - mt * tn;
-    }
-  }
-  // pair_off != 0: w holds [up; gate] rows (pair_off = number of pairs) and the tile covers 128 PAIRS: each wave's
-  // 128 weight rows are 64 up rows followed by the 64 gate rows of the same pairs, so that a lane ends up with
-  // both halves of a pair and stores bf16(bf16(silu(g)) * u) -- N is then the number of pairs
-  const int m0 = mt * GM, n0 = nt * (pair_off ? GN / 2 : GN);
+// Tiles [0, full) are computed whole; each of the `rem` tiles after them is cut along K into `splits` pieces, whose fp32
+// sums go to `part` in the order a wave holds them (k_gemm_sum adds them in order and finishes the tile).
+struct GemmSplit {
+  float* part;
+  int full, rem, splits;
+};
+enum { GEMM_PLAIN, GEMM_PAIR, GEMM_ROPE };   // PAIR: w holds [up; gate] rows, N counts pairs, output silu(gate) * up
 
-  // staging assignment: 2048 16-byte chunks per operand tile, 8 per thread
-  f32x16_t acc[4][4];
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
+template <int AH, int BH>
+struct GemmTile {
+  static constexpr int TM = 128 * AH, TN = 128 * BH;
+  static constexpr int HA = 8192 * AH, HB = 8192 * BH;   // bytes of half an operand's k-tile
+  static constexpr int NA = 2 * AH, NB = 2 * BH;         // DMA instructions of a wave for it
+  static constexpr int RING = 4 * (HA + HB);
+  static constexpr int EPITCH = 64 * BH + 8;             // row pitch of a wave's output piece (plain), in elements
+  static constexpr int EBYTES = 4 * 64 * AH * EPITCH * 2;
+  static constexpr int LDS = RING > EBYTES ? RING : EBYTES;
+};
 
-  const int srow0 = tid >> 3, scol = (tid & 7) * 8;  // chunk i sits 32 rows below chunk i - 1
-  // Operand rows are read through buffer resources based at the tile's first row; a chunk beyond M,
-  // N or K gets an offset outside the resource and reads as zero: no branches around the loads.
-  const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(x + (int64_t)m0 * ldx), 0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(w + (int64_t)n0 * K), 0, 0x7fffffff, 0x00020000);
-  int xoff[8], woff[8];
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
+// One wave instruction: 64 x 16 bytes from memory to LDS at `lds` + 16 * lane.  (s_nop: the wait state between a write of
+// M0 and its use; the scalar operands come from scalar instructions.)
+__device__ __forceinline__ void dma16(const i32x4_t& rsrc, int voff, int soff, u32 lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
+               : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_requests_and_lds() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+
+// Which of `n` tiles workgroup `id` of `count` takes: an XCD (id % 8) has a contiguous run of them.
+__device__ __forceinline__ int xcd_run(int id, int n) {
+  const int xcd = id & 7, base = n >> 3, rem = n & 7;
+  return xcd * base + (xcd < rem ? xcd : rem) + (id >> 3);
+}
+// Tile number -> (row tile, column tile): bands of up to four row tiles, a band's columns one after the other, so that the
+// workgroups an XCD runs at the same time share operand rows in its L2.
+__device__ __forceinline__ void gemm_tile_at(int t, int tm, int tn, int& mt, int& nt) {
+  const int band = t / (4 * tn), r = t - band * 4 * tn;
+  const int h = tm - band * 4 < 4 ? tm - band * 4 : 4;
+  nt = r / h;
+  mt = band * 4 + r - nt * h;
+}
+
+// The outputs of R16 groups of 16 rows of a wave's part of a tile.  The products are W-tile x X-tile^T: a lane of
+// acc[a][b] holds four consecutive columns 4 (lane / 16) .. of row lane % 16; b < 2 BH are columns of the tile's first half
+// of weight rows, the others of its second.  Stored from there an instruction would touch 32 bytes in each of 16 rows: they
+// take one trip through LDS (`eb`, a piece of the wave's own) and leave as whole rows.  `row0`: first of the wave's row
+// groups here, m = tile row of group g is row_of(g).
+template <int AH, int BH, int MODE, int R16>
+__device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u16* eb, int g0, int wm, int wn, int m0, int n0, u16* __restrict__ y,
+                                           int64_t ldy, int M, int N, const GemmRope& rp, const int32_t* entry) {
+  int lane = threadIdx.x & 63;   // (laundered: the addresses below are not formed before the k loop and kept through it)
+  asm volatile("" : "+v"(lane));
+  constexpr bool P = MODE == GEMM_PAIR;
+  constexpr int HC = 32 * BH;                        // a wave's columns in one half
+  constexpr int EP = (P ? HC : 2 * HC) + 8;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = srow0 + i * 32;
-    const int xrow = GROUP ? entry[r] / gp.xdiv : r;
-    xoff[i] = m0 + r < M ? (int)((int64_t)xrow * ldx * 2) : (int)0x80000000;
-    if (pair_off) {
-      const int wv = i >> 2, b = i & 3;                      // r = wv * 128 + b * 32 + srow0
-      const int pr = wv * 64 + (b & 1) * 32 + srow0;          // pair inside the tile
-      woff[i] = n0 + pr < N ? (int)((int64_t)((b >> 1) * pair_off + pr) * K * 2) : (int)0x80000000;
-    } else {
-      woff[i] = n0 + r < N ? r * K * 2 : (int)0x80000000;
-    }
-  }
-  // k = first element of the k-tile (the same for all lanes); a tile beyond K is only ever requested, never used
-  // (the two tiles asked for past the end): without the per-lane check it is replaced by the last real tile
-  const int klast = ((K + BK - 1) / BK - 1) * BK;
-  if (!KTAIL) {
+  for (int a = 0; a < R16; ++a) {
+    const int ml = a * 16 + (lane & 15);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (xoff[i] >= 0) xoff[i] += scol * 2;
-      if (woff[i] >= 0) woff[i] += scol * 2;
+    for (int b = 0; b < (P ? 2 * BH : 4 * BH); ++b) {
+      float o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = P ? swiglu_bf(round_bf(acc[a][b][e]), round_bf(acc[a][b + 2 * BH][e])) : acc[a][b][e];
+      *reinterpret_cast<uint2*>(&eb[ml * EP + b * 16 + (lane >> 4) * 4]) = make_uint2(pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]));
     }
+    __builtin_amdgcn_sched_barrier(0);   // (not all accumulators out of their half of the register file at once)
   }
-  auto fetch = [&](const __amdgpu_buffer_rsrc_t& res, int rowoff, int k) -> uint4 {
-    u32x4_t v;
-    if (KTAIL) {
-      const int off = (k + scol < K && rowoff >= 0) ? rowoff + (k + scol) * 2 : (int)0x80000000;
-      v = __builtin_amdgcn_raw_buffer_load_b128(res, off, 0, 0);
-    } else {
-      v = __builtin_amdgcn_raw_buffer_load_b128(res, rowoff, (k < klast ? k : klast) * 2, 0);
-    }
-    return make_uint4(v.x, v.y, v.z, v.w);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // a wave reads back only what it wrote itself
+  constexpr int LPR = HC / 8, RPI = 64 / LPR;         // lanes per row, rows per instruction
+  const int cl = (lane % LPR) * 8;
+  const bool vec_ok = (ldy & 7) == 0;
+  auto row_of = [&](int ml) {
+    const int g = g0 + (ml >> 4);
+    return m0 + (g / (2 * AH)) * 64 * AH + wm * 32 * AH + (g % (2 * AH)) * 16 + (ml & 15);
   };
-  // Global -> LDS staging one tile ahead through ONE register set, in quarters: while tile kt is
-  // multiplied, quarter q of tile kt + 1 (requested a whole iteration earlier, so it has landed) is
-  // written to the other LDS buffer behind the MFMA group of k-step q, and the same registers are
-  // at once refilled with quarter q of tile kt + 2.
-  uint4 xr[8], wr[8];
-  const int nk = (K + BK - 1) / BK;
+  auto store_row = [&](int m, int n, const uint4& v) {
+    if (m >= M) return;
+    if (entry != nullptr) m = entry[m];
+    if (vec_ok && n + 7 < N) {
+      st16(y + (int64_t)m * ldy + n, v);
+    } else {
+      const u32 q[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    xr[i] = fetch(xres, xoff[i], 0);
-    wr[i] = fetch(wres, woff[i], 0);
-  }
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    st16(&xs[(srow0 + i * 32) * LDT + scol], xr[i]);
-    st16(&ws[(srow0 + i * 32) * LDT + scol], wr[i]);
-  }
-  // (requests beyond K read as zero: every load and LDS write below is unconditional, so the number of
-  // loads in flight never depends on a branch and the waits can be exact)
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    xr[i] = fetch(xres, xoff[i], BK);
-    wr[i] = fetch(wres, woff[i], BK);
-  }
-  __syncthreads();
-
-  const int arow = lane & 31, akq = (lane >> 5) * 8;
-  // Fragments of k-step ks + 1 are read from LDS while the matrix instructions of k-step ks run; those of the next
-  // tile's k-step 0 during this tile's last k-step, behind the one workgroup barrier of the iteration.
-  bf16x8_t af[2][4], bfr[2][4];
-#pragma unroll
-  for (int a = 0; a < 4; ++a) af[0][a] = *reinterpret_cast<const bf16x8_t*>(&xs[(wm * 128 + a * 32 + arow) * LDT + akq]);
-#pragma unroll
-  for (int b = 0; b < 4; ++b) bfr[0][b] = *reinterpret_cast<const bf16x8_t*>(&ws[(wn * 128 + b * 32 + arow) * LDT + akq]);
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    const u16* xc = xs + cur * GM * LDT;
-    const u16* wc = ws + cur * GN * LDT;
-    u16* xn = xs + (cur ^ 1) * GM * LDT;
-    u16* wn_ = ws + (cur ^ 1) * GN * LDT;
-    const int k2 = (kt + 2) * BK;
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      const int c = ks & 1, nx = c ^ 1;
-      const bool last = ks + 1 == BK / 16;
-      // One non-matrix instruction in the shadow of every matrix instruction (a wave issues in order: grouped, the
-      // sixteen matrix instructions of a k-step would be followed by ~16 LDS / global instructions with the matrix
-      // pipe idle).  K-steps 0..2: the eight fragment reads of the next k-step, the four LDS writes of the staged
-      // quarter, the four global loads of the quarter after it.  Last k-step: the writes first, then the barrier
-      // (every wave has written the next tile and has read all it needs of this one), the loads, and the fragment
-      // reads of the NEXT tile's k-step 0 -- so that an iteration does not open with the matrix pipe waiting for LDS.
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int a4 = j >> 2, b4 = j & 3;
-        acc[a4][b4] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[c][b4], af[c][a4], acc[a4][b4], 0, 0, 0);
-        const int rd = last ? j - 8 : j;       // slot of the eight fragment reads
-        const int wr_ = last ? j : j - 8;      // slot of the four LDS writes
-        const int ft = last ? j - 4 : j - 12;  // slot of the four global loads
-        if (rd >= 0 && rd < 8) {
-          const u16* xf = last ? xn : xc;
-          const u16* wf = last ? wn_ : wc;
-          const int kk = last ? 0 : (ks + 1) * 16;
-          if (rd < 4) af[nx][rd] = *reinterpret_cast<const bf16x8_t*>(&xf[(wm * 128 + rd * 32 + arow) * LDT + kk + akq]);
-          else bfr[nx][rd - 4] = *reinterpret_cast<const bf16x8_t*>(&wf[(wn * 128 + (rd - 4) * 32 + arow) * LDT + kk + akq]);
-        } else if (wr_ >= 0 && wr_ < 4) {
-          const int i = 2 * ks + (wr_ >> 1);
-          if ((wr_ & 1) == 0) st16(&xn[(srow0 + i * 32) * LDT + scol], xr[i]);
-          else st16(&wn_[(srow0 + i * 32) * LDT + scol], wr[i]);
-        } else if (ft >= 0 && ft < 4) {
-          const int i = 2 * ks + (ft >> 1);
-          if ((ft & 1) == 0) xr[i] = fetch(xres, xoff[i], k2);
-          else wr[i] = fetch(wres, woff[i], k2);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        if (last && j == 3) {
-          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // LDS only: the global loads stay in flight
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
+      for (int e = 0; e < 8; ++e)
+        if (n + e < N) y[(int64_t)m * ldy + n + e] = (u16)(q[e >> 1] >> ((e & 1) * 16));
     }
-  }
-
-  // The products were formed as W-tile x X-tile^T, so accumulator element v of a 32 x 32 tile is
-  // output column n = (v / 4) * 8 + (lane / 32) * 4 + v % 4 of output row m = lane % 32: a lane holds
-  // four consecutive n of one row per group of four registers.  Stored from there, an instruction would
-  // touch 16 bytes in each of 32 rows (32 partial cache lines, every line eight times per tile): the
-  // tile's outputs take one trip through LDS instead (the operand tiles are dead; every wave has a piece
-  // of its own) and leave as whole rows, an instruction covering 256 contiguous bytes of each of 4 rows
-  // (128 bytes of 8 rows in pair mode).
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // nobody still reads the operand tiles
-  u16* const eb = gsm + wave * (128 * (128 + 8));
-  auto emit = [&](auto PAIR) {
-    int lane = threadIdx.x & 63;  // (laundered: the addresses below are not formed before the k loop and kept through it)
-    asm volatile("" : "+v"(lane));
-    constexpr bool P = decltype(PAIR)::value;
-    constexpr int WN = P ? 64 : 128;   // output columns of a wave
-    constexpr int EP = WN + 8;         // row pitch of the wave's piece, in elements
-    constexpr int LPR = WN / 8;        // lanes per row in the read-back
-    constexpr int RPI = 64 / LPR;      // rows per instruction
+  };
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int ml = a * 32 + (lane & 31);
-#pragma unroll
-      for (int b = 0; b < (P ? 2 : 4); ++b)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int nl = b * 32 + g * 8 + (lane >> 5) * 4;
-          uint2 pk;
-          if constexpr (P) {
-            float o[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = swiglu_bf(round_bf(acc[a][b][4 * g + e]), round_bf(acc[a][b + 2][4 * g + e]));
-            pk.x = pack_bf2(o[0], o[1]);
-            pk.y = pack_bf2(o[2], o[3]);
-          } else {
-            pk.x = pack_bf2(acc[a][b][4 * g], acc[a][b][4 * g + 1]);
-            pk.y = pack_bf2(acc[a][b][4 * g + 2], acc[a][b][4 * g + 3]);
-          }
-          *reinterpret_cast<uint2*>(&eb[ml * EP + nl]) = pk;
-        }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // a wave reads back only what it wrote itself
-    const bool vec_ok = (ldy & 7) == 0;
-    const int cl = (lane % LPR) * 8;
-    const int ncol0 = n0 + wn * WN + cl;
-    // ROPE: the lane's eight columns lie in one head of one section (head_dim % 8 == 0); its rows are RPI apart
-    int rb = 0, rs = 0, sect = 0, hh = 0, dd = 0;
-    if constexpr (ROPE && !P) {
-      const int mfirst = m0 + wm * 128 + lane / LPR;
-      rb = mfirst / rp.S;
-      rs = mfirst - rb * rp.S;
+  for (int hb = 0; hb < (P ? 1 : 2); ++hb) {
+    const int n = n0 + hb * 64 * BH + wn * HC + cl;
+    if constexpr (MODE == GEMM_ROPE) {
+      // What k_rope_kv_write would do to the stored rows.  The lane's eight columns lie in one head of one section
+      // (head_dim % 8 == 0).  Positions of several rows first, then their table entries, then the arithmetic: two memory
+      // round trips per RB rows (row by row the position and the entry it selects are a chain of two loads per row, and
+      // the output pass of a tile took three times as long).
+      constexpr int RB = R16 * 16 / RPI < 8 ? R16 * 16 / RPI : 8;
       const int nq = rp.Hq * rp.hd, nkv = rp.Hkv * rp.hd;
-      sect = ncol0 < nq ? 0 : (ncol0 < nq + nkv ? 1 : 2);
-      const int cc = ncol0 - (sect == 0 ? 0 : (sect == 1 ? nq : nq + nkv));
-      hh = cc / rp.hd;
-      dd = cc - hh * rp.hd;
-    }
-    auto store_row = [&](int m, const uint4& v) {
-      if (m < M) {
-        if constexpr (GROUP) m = entry[m];
-        if (vec_ok && ncol0 + 7 < N) {
-          *reinterpret_cast<uint4*>(y + (int64_t)m * ldy + ncol0) = v;
-        } else {
-          const u32 q[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (ncol0 + e < N) y[(int64_t)m * ldy + ncol0 + e] = (u16)(q[e >> 1] >> ((e & 1) * 16));
-        }
-      }
-    };
-    if constexpr (ROPE && !P) {
-      // Sixteen rows at a time: all their positions first, then all their table entries, then the arithmetic -- two
-      // memory round trips per sixteen rows (row by row the position and the table entry it selects are a chain of
-      // two dependent loads per row, and the output pass of a tile took three times as long).
-      constexpr int RB = 16;
-      for (int h0 = 0; h0 < 128 / RPI; h0 += RB) {
+      const int sect = n < nq ? 0 : (n < nq + nkv ? 1 : 2), cc = n - (sect == 0 ? 0 : (sect == 1 ? nq : nq + nkv));
+      const int hh = cc / rp.hd, dd = cc - hh * rp.hd;
+      for (int i0 = 0; i0 < R16 * 16 / RPI; i0 += RB) {
         int ps[RB], bb[RB];
 #pragma unroll
         for (int i = 0; i < RB; ++i) {
-          bb[i] = rb;
-          const int m = m0 + wm * 128 + (h0 + i) * RPI + lane / LPR;
-          ps[i] = (m < M && ncol0 < N) ? rpos[rs] : -1;  // (N % 8 == 0 and ldy % 8 == 0 here: the column group is whole)
-          rs += RPI;
-          while (rs >= rp.S) { rs -= rp.S; ++rb; }
+          const int m = row_of((i0 + i) * RPI + lane / LPR);
+          bb[i] = m / rp.S;
+          ps[i] = (m < M && n < N) ? rp.pos[m - bb[i] * rp.S] : -1;  // (N % 8 == 0 and ldy % 8 == 0: the columns are whole)
         }
         uint4 tv[RB];
         bool ok[RB];
 #pragma unroll
         for (int i = 0; i < RB; ++i) {
           ok[i] = ps[i] >= 0 && ps[i] < rp.Smax && ps[i] < rp.block_size;
-          tv[i] = (ok[i] && sect < 2) ? ld16(rtable + (int64_t)ps[i] * rp.hd + dd) : make_uint4(0, 0, 0, 0);
+          tv[i] = (ok[i] && sect < 2) ? ld16(rp.table + (int64_t)ps[i] * rp.hd + dd) : make_uint4(0, 0, 0, 0);
         }
 #pragma unroll
         for (int i = 0; i < RB; ++i) {
-          const int ml = (h0 + i) * RPI + lane / LPR;
-          const int m = m0 + wm * 128 + ml;
-          uint4 v = *reinterpret_cast<const uint4*>(&eb[ml * EP + cl]);
+          const int ml = (i0 + i) * RPI + lane / LPR, m = row_of(ml);
+          uint4 v = *reinterpret_cast<const uint4*>(&eb[ml * EP + hb * HC + cl]);
           if (ok[i]) {
             const uint4 r = sect < 2 ? rope8(v, tv[i]) : v;
             if (sect == 0) v = r;
-            else st16((sect == 1 ? rk : rv) + (((int64_t)bb[i] * rp.Hkv + hh) * rp.Smax + ps[i]) * rp.hd + dd, r);
-          } else if (m < M && ncol0 < N && rerr && cl == 0 && wn == 0) {
-            *rerr = LR_DEV_POS_RANGE;
+            else st16((sect == 1 ? rp.k_cache : rp.v_cache) + (((int64_t)bb[i] * rp.Hkv + hh) * rp.Smax + ps[i]) * rp.hd + dd, r);
+          } else if (m < M && n == 0 && rp.err) {
+            *rp.err = LR_DEV_POS_RANGE;
           }
-          store_row(m, v);
+          store_row(m, n, v);
         }
       }
-      return;
-    }
+    } else {
 #pragma unroll 4
-    for (int r0 = 0; r0 < 128; r0 += RPI) {
-      const int ml = r0 + lane / LPR;
-      store_row(m0 + wm * 128 + ml, *reinterpret_cast<const uint4*>(&eb[ml * EP + cl]));
+      for (int r0 = 0; r0 < R16 * 16; r0 += RPI) {
+        const int ml = r0 + lane / LPR;
+        store_row(row_of(ml), n, *reinterpret_cast<const uint4*>(&eb[ml * EP + hb * HC + cl]));
+      }
     }
-  };
-  if (pair_off) emit(std::true_type{});
-  else emit(std::false_type{});
+  }
 }
 
-// pair_off != 0: N counts [up; gate] row pairs (see the kernel); rope != nullptr: the q/k/v projection of a prefill
-// of S tokens per sequence (pair_off == 0, ldy % 8 == 0)
-template <bool KTAIL, bool ROPE>
-static int launch_gemm_big_as(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K,
-                              int pair_off, const lr_rope_kv_t* rope, int S, hipStream_t s) {
-  constexpr size_t lds = (size_t)2 * (GM + GN) * LDT * sizeof(u16);
-  static std::atomic<unsigned long long> lds_raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_big<KTAIL, ROPE>), lds, lds_raised)) return LR_E_LAUNCH;
-  const int gn = pair_off ? GN / 2 : GN;
-  const int tm = (M + GM - 1) / GM, tn = (N + gn - 1) / gn;
-  GemmRope rp = {};
-  if (ROPE) rp = GemmRope{S, rope->n_head, rope->n_kv_head, rope->head_dim, rope->smax, rope->block_size};
-  k_gemm_big<KTAIL, ROPE><<<dim3((unsigned)(tm * tn)), dim3(256), lds, s>>>(
-      (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, M, N, K, tm, tn, pair_off, ROPE ? (const u16*)rope->table : nullptr,
-      ROPE ? rope->pos : nullptr, ROPE ? (u16*)rope->k_cache : nullptr, ROPE ? (u16*)rope->v_cache : nullptr,
-      ROPE ? rope->err : nullptr, rp);
-  return lr_launch_status();
-}
-
-static int launch_gemm_big(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K,
-                           int pair_off, hipStream_t s, const lr_rope_kv_t* rope = nullptr, int S = 0) {
-  const bool ktail = K % BK != 0;
-  if (rope)
-    return ktail ? launch_gemm_big_as<true, true>(x, ldx, w, y, ldy, M, N, K, pair_off, rope, S, s)
-                 : launch_gemm_big_as<false, true>(x, ldx, w, y, ldy, M, N, K, pair_off, rope, S, s);
-  return ktail ? launch_gemm_big_as<true, false>(x, ldx, w, y, ldy, M, N, K, pair_off, nullptr, 0, s)
-               : launch_gemm_big_as<false, false>(x, ldx, w, y, ldy, M, N, K, pair_off, nullptr, 0, s);
-}
-
-// Grouped products (lr_moe): rows of several matrices' tiles, see GemmGroup.  pair_off as in launch_gemm_big.
-namespace lr_detail {
-template <bool KTAIL>
-static int gemm_grouped_as(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int N, int K, int pair_off,
-                           const GemmGroup& gp, int max_tiles, hipStream_t s) {
-  constexpr size_t lds = (size_t)2 * (GM + GN) * LDT * sizeof(u16) + GM * sizeof(int32_t);
-  static std::atomic<unsigned long long> lds_raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_big<KTAIL, false, true>), lds, lds_raised)) return LR_E_LAUNCH;
-  const int gn = pair_off ? GN / 2 : GN, tn = (N + gn - 1) / gn;
-  k_gemm_big<KTAIL, false, true><<<dim3((unsigned)(max_tiles * tn)), dim3(256), lds, s>>>(
-      (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, GM, N, K, max_tiles, tn, pair_off, nullptr, nullptr, nullptr, nullptr, nullptr,
-      GemmRope{}, gp);
-  return lr_launch_status();
-}
-// Grouped products in 128 x 128 tiles, for problems with few 256-row tiles: the loop of k_gemm with gathered rows, buffer
-// loads instead of branches and, in pair mode, a wave's 64 weight rows as 32 up rows followed by their gate rows.
-__global__ __launch_bounds__(256) void k_gemm_grouped(const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w, u16* __restrict__ y,
-                                                      int64_t ldy, int N, int K, int tn, int pair_off, const GemmGroup gp) {
-  __shared__ __attribute__((aligned(16))) u16 xs[2][BM * LDT];
-  __shared__ __attribute__((aligned(16))) u16 ws[2][BN * LDT];
-  __shared__ int32_t entry[BM];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// KTAIL: K is not a multiple of the 64-element k-tile, so the last one needs a per-lane range check.
+template <int AH, int BH, bool KTAIL, int MODE, bool GROUP>
+__global__ __launch_bounds__(256, AH * BH == 1 ? 2 : 1) void k_gemm_dma(const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
+                                                                        u16* __restrict__ y, int64_t ldy, int M, int N, int K, int tm, int tn,
+                                                                        const GemmRope rp, const GemmSplit sp, const GemmGroup gp) {
+  using T = GemmTile<AH, BH>;
+  constexpr int HA = T::HA, HB = T::HB, NA = T::NA, NB = T::NB, BOFF = 4 * HA;
+  extern __shared__ __attribute__((aligned(1024))) u16 gsm[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
-  int mt, nt, M;
-  {
-    const int n = gridDim.x, xcd = blockIdx.x & 7, base = n >> 3, rem = n & 7;
-    const int id = xcd * base + (xcd < rem ? xcd : rem) + (blockIdx.x >> 3);
+  int mt, nt, piece = -1, kt0 = 0, nk = (K + 63) / 64;
+  int32_t* const entry = reinterpret_cast<int32_t*>(gsm + T::LDS / 2);   // (GROUP) the tile's entries
+  if constexpr (GROUP) {
+    const int id = xcd_run(blockIdx.x, gridDim.x);   // a row tile's column tiles one after the other
     mt = id / tn;
     nt = id - mt * tn;
     if (mt >= gp.ntiles[0]) return;
     const int32_t* tile = gp.tiles + 3 * mt;
     w += tile[0] * gp.wstride;
     M = tile[2];
-    if (tid < BM) entry[tid] = gp.entries[tile[1] + (tid < M ? tid : 0)];
+    if (tid < T::TM) entry[tid] = gp.entries[tile[1] + (tid < M ? tid : 0)];
+    mt = 0;
     __syncthreads();
-  }
-  const int n0 = nt * (pair_off ? BN / 2 : BN);
-  const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(x), 0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(w + (int64_t)n0 * K), 0, 0x7fffffff, 0x00020000);
-  const int srow0 = tid >> 3, scol = (tid & 7) * 8;
-  int xoff[4], woff[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = srow0 + 32 * i;
-    xoff[i] = r < M ? (int)((int64_t)(entry[r] / gp.xdiv) * ldx * 2) : (int)0x80000000;
-    if (pair_off) {
-      const int pr = (r >> 6) * 32 + (r & 31);
-      woff[i] = n0 + pr < N ? (int)((int64_t)(((r >> 5) & 1) * pair_off + pr) * K * 2) : (int)0x80000000;
+  } else {
+    int t = blockIdx.x;
+    if (t < sp.full) {
+      t = xcd_run(t, sp.full);
     } else {
-      woff[i] = n0 + r < N ? r * K * 2 : (int)0x80000000;
+      const int q = xcd_run(t - sp.full, sp.rem * sp.splits), split = q / sp.rem;
+      t = sp.full + q - split * sp.rem;
+      piece = (t - sp.full) * sp.splits + split;
+      const int pairs = (nk + 1) / 2, p0 = (int)((int64_t)pairs * split / sp.splits), p1 = (int)((int64_t)pairs * (split + 1) / sp.splits);
+      kt0 = 2 * p0;
+      nk = (nk < 2 * p1 ? nk : 2 * p1) - kt0;
+    }
+    gemm_tile_at(t, tm, tn, mt, nt);
+  }
+  const int m0 = mt * T::TM, n0 = nt * (MODE == GEMM_PAIR ? T::TN / 2 : T::TN);
+
+  // Requests.  Instruction i of a wave's share of a half covers the half's rows (wave * n + i) * 8 + lane / 8, a lane 16
+  // bytes of one.  Operand rows are read through buffer resources based at the tile's first row; a row beyond M or N has an
+  // offset outside the resource and reads as zero.
+  const u16* const xb = x + (int64_t)m0 * ldx + kt0 * 64;
+  const u16* const wb = w + (int64_t)n0 * K + kt0 * 64;
+  constexpr int OUT = (int)0x80000000;
+  const int klen = K - kt0 * 64;
+  const int chunk = ((lane & 7) ^ (lane >> 3)) * 8;      // (row % 8 == lane / 8)
+  int xo[2][NA], wo[2][NB];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      const int r = h * 64 * AH + (wave * NA + i) * 8 + (lane >> 3);
+      const int row = GROUP ? entry[r] / gp.xdiv : r;
+      xo[h][i] = m0 + r < M ? (int)((int64_t)row * ldx * 2) + chunk * 2 : OUT;
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int r = (wave * NB + i) * 8 + (lane >> 3);
+      if (MODE == GEMM_PAIR) wo[h][i] = n0 + r < N ? (int)((int64_t)(h * N + r) * K * 2) + chunk * 2 : OUT;   // (half 0 up, half 1 gate)
+      else wo[h][i] = n0 + h * 64 * BH + r < N ? (int)((int64_t)(h * 64 * BH + r) * K * 2) + chunk * 2 : OUT;
     }
   }
-  uint4 xr[4], wr[4];
-  auto fetch = [&](int k) {
-    const bool in = k + scol < K;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const u32x4_t a = __builtin_amdgcn_raw_buffer_load_b128(xres, in && xoff[i] >= 0 ? xoff[i] + (k + scol) * 2 : (int)0x80000000, 0, 0);
-      const u32x4_t b = __builtin_amdgcn_raw_buffer_load_b128(wres, in && woff[i] >= 0 ? woff[i] + (k + scol) * 2 : (int)0x80000000, 0, 0);
-      xr[i] = make_uint4(a.x, a.y, a.z, a.w);
-      wr[i] = make_uint4(b.x, b.y, b.z, b.w);
-    }
+  const u32 lds0 = __builtin_amdgcn_readfirstlane((u32)(uintptr_t)(__attribute__((address_space(3))) u16*)gsm);
+  auto request = [&](const u16* base, int voff, int t, u32 lds) {
+    const bool in = t < nk;
+    i32x4_t r;
+    r.x = (int)(u32)(unsigned long long)base;
+    r.y = (int)(u32)((unsigned long long)base >> 32) & 0xffff;
+    r.z = in ? 0x7fffffff : 0;
+    r.w = 0x00020000;
+    if (KTAIL) voff = t * 64 + chunk < klen ? voff : OUT;
+    dma16(r, voff, in ? t * 128 : 0, lds);
   };
-  auto stage = [&](int buf) {
+  auto dma_a = [&](int t, int par, int h, int i) { request(xb, xo[h][i], t, lds0 + (par * 2 + h) * HA + (wave * NA + i) * 1024); };
+  auto dma_b = [&](int t, int par, int h, int i) { request(wb, wo[h][i], t, lds0 + BOFF + (par * 2 + h) * HB + (wave * NB + i) * 1024); };
+
+  f32x4_t acc[4 * AH][4 * BH];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      st16(&xs[buf][(srow0 + 32 * i) * LDT + scol], xr[i]);
-      st16(&ws[buf][(srow0 + 32 * i) * LDT + scol], wr[i]);
-    }
-  };
-  f32x16_t acc[2][2];
+  for (int a = 0; a < 4 * AH; ++a)
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+    for (int b = 0; b < 4 * BH; ++b)
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+      for (int v = 0; v < 4; ++v) acc[a][b][v] = 0.0f;
+  bf16x8_t af[2][2 * AH][2], bf[2][2 * BH][2];
+  const char* const smb = reinterpret_cast<const char*>(gsm);
+  int fa[2], fb[2];
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
-  const int nk = (K + BK - 1) / BK, arow = lane & 31, akq = (lane >> 5) * 8;
-  fetch(0);
-  stage(0);
-  __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < nk) fetch((kt + 1) * BK);
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 16) {
-      bf16x8_t af[2], bfr[2];
-#pragma unroll
-      for (int a = 0; a < 2; ++a) af[a] = *reinterpret_cast<const bf16x8_t*>(&xs[cur][(wm * 64 + a * 32 + arow) * LDT + kk + akq]);
-#pragma unroll
-      for (int b = 0; b < 2; ++b) bfr[b] = *reinterpret_cast<const bf16x8_t*>(&ws[cur][(wn * 64 + b * 32 + arow) * LDT + kk + akq]);
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[b], af[a], acc[a][b], 0, 0, 0);
-    }
-    if (kt + 1 < nk) stage(cur ^ 1);
-    __syncthreads();
+  for (int ks = 0; ks < 2; ++ks) {
+    const int c = ((4 * ks + (lane >> 4)) ^ (lane & 7)) * 16;
+    fa[ks] = (wm * 32 * AH + (lane & 15)) * 128 + c;
+    fb[ks] = (wn * 32 * BH + (lane & 15)) * 128 + c + BOFF;
   }
-  // The products were W-tile x X-tile^T: accumulator element v of a 32 x 32 tile is output column (v / 4) * 8 + (lane / 32) * 4
-  // + v % 4 of row lane % 32.  Outputs leave through LDS (a piece per wave) as whole rows.
-  u16* eb = &xs[0][0] + wave * 64 * LDT;      // (2 BM LDT elements in all; the operand tiles are dead)
-  auto emit = [&](auto PAIR) {
-    constexpr bool P = decltype(PAIR)::value;
-    constexpr int WN = P ? 32 : 64, LPR = WN / 8, RPI = 64 / LPR;
+  auto read_a = [&](int par, int h, int t, int ks) {
+    af[h][t][ks] = *reinterpret_cast<const bf16x8_t*>(smb + fa[ks] + (par * 2 + h) * HA + t * 2048);
+  };
+  auto read_b = [&](int set, int par, int h, int t, int ks) {
+    bf[set][t][ks] = *reinterpret_cast<const bf16x8_t*>(smb + fb[ks] + (par * 2 + h) * HB + t * 2048);
+  };
+  auto barrier = [&] {
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+  for (int t = 0; t < 2; ++t) {
 #pragma unroll
-      for (int b = 0; b < (P ? 1 : 2); ++b)
+    for (int i = 0; i < NA; ++i) dma_a(t, t, 0, i);
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          float o[4];
+    for (int i = 0; i < NB; ++i) dma_b(t, t, 0, i);
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            o[e] = P ? swiglu_bf(round_bf(acc[a][0][4 * g + e]), round_bf(acc[a][1][4 * g + e])) : acc[a][b][4 * g + e];
-          *reinterpret_cast<uint2*>(&eb[(a * 32 + (lane & 31)) * LDT + b * 32 + g * 8 + (lane >> 5) * 4]) =
-              make_uint2(pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]));
+    for (int i = 0; i < NB; ++i) dma_b(t, t, 1, i);
+#pragma unroll
+    for (int i = 0; i < NA; ++i) dma_a(t, t, 1, i);
+  }
+  wait_requests_and_lds<3 * NA + 3 * NB>();
+  barrier();
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+    for (int t = 0; t < 2 * AH; ++t) read_a(0, 0, t, ks);
+#pragma unroll
+    for (int t = 0; t < 2 * BH; ++t) read_b(0, 0, 0, t, ks);
+  }
+  wait_requests_and_lds<3 * NA + 3 * NB>();
+  barrier();
+#pragma unroll
+  for (int i = 0; i < NA; ++i) dma_a(2, 0, 0, i);
+
+  // Phase P of k-tile t (even: PAR 0).  Reads B1 of this tile, A1 of this tile, A0 of the next, B0 of the next; requests
+  // B0, B1, A1 of tile t + 2 and A0 of tile t + 3.
+  auto phase = [&](auto PAR_, auto P_, int t) {
+    constexpr int PAR = decltype(PAR_)::value, P = decltype(P_)::value;
+    constexpr int ah = P >> 1, bh = (P == 1 || P == 2), set = bh ^ PAR;
+    // requests younger than the slot read here: those of the six phases since
+    wait_requests_and_lds<(P == 0 ? 4 * NA + 2 * NB : P == 2 ? 2 * NA + 4 * NB : 3 * NA + 3 * NB)>();
+    barrier();
+    constexpr int J = 8 * AH * BH, RD = (P == 1 || P == 2) ? 4 * AH : 4 * BH, RQ = (P == 2 || P == 3) ? NA : NB;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int tb = j % (2 * BH), ta = j / (2 * BH) % (2 * AH), ks = j / (4 * AH * BH);
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+                   : "+a"(acc[ah * 2 * AH + ta][bh * 2 * BH + tb])
+                   : "v"(bf[set][tb][ks]), "v"(af[ah][ta][ks]));
+      if (j < J / 2) {
+#pragma unroll
+        for (int e = j * RD / (J / 2); e < (j + 1) * RD / (J / 2); ++e) {
+          if (P == 0) read_b(1 ^ PAR, PAR, 1, e % (2 * BH), e / (2 * BH));
+          if (P == 1) read_a(PAR, 1, e % (2 * AH), e / (2 * AH));
+          if (P == 2) read_a(PAR ^ 1, 0, e % (2 * AH), e / (2 * AH));
+          if (P == 3) read_b(1 ^ PAR, PAR ^ 1, 0, e % (2 * BH), e / (2 * BH));
         }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // a wave reads back only what it wrote itself
-    const int cl = (lane % LPR) * 8, n = n0 + wn * WN + cl;
+      } else {
 #pragma unroll
-    for (int r0 = 0; r0 < 64; r0 += RPI) {
-      const int ml = r0 + lane / LPR, m = wm * 64 + ml;
-      if (m < M && n < N)      // (N and ldy are multiples of 8)
-        st16(y + (int64_t)entry[m] * ldy + n, *reinterpret_cast<const uint4*>(&eb[ml * LDT + cl]));
+        for (int e = (j - J / 2) * RQ / (J / 2); e < (j + 1 - J / 2) * RQ / (J / 2); ++e) {
+          if (P == 0) dma_b(t + 2, PAR, 0, e);
+          if (P == 1) dma_b(t + 2, PAR, 1, e);
+          if (P == 2) dma_a(t + 2, PAR, 1, e);
+          if (P == 3) dma_a(t + 3, PAR ^ 1, 0, e);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
-  if (pair_off) emit(std::true_type{});
-  else emit(std::false_type{});
+  {
+    std::integral_constant<int, 0> c0;
+    std::integral_constant<int, 1> c1;
+    std::integral_constant<int, 2> c2;
+    std::integral_constant<int, 3> c3;
+    for (int t = 0; t < nk; t += 2) {   // (an odd number of k-tiles ends with one of zeros)
+      phase(c0, c0, t);
+      phase(c0, c1, t);
+      phase(c0, c2, t);
+      phase(c0, c3, t);
+      phase(c1, c0, t + 1);
+      phase(c1, c1, t + 1);
+      phase(c1, c2, t + 1);
+      phase(c1, c3, t + 1);
+    }
+  }
+  // the last matrix instructions' results can be read (they are assembler text: the wait states are ours), nothing is on its
+  // way into LDS, nobody still reads it
+  asm volatile("s_nop 15\n\ts_nop 15\n\ts_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if constexpr (!GROUP) {
+    if (piece >= 0) {
+      float* p = sp.part + (int64_t)piece * (T::TM * T::TN) + (int64_t)wave * (16 * AH * BH * 256) + lane * 4;
+#pragma unroll
+      for (int a = 0; a < 4 * AH; ++a) {
+#pragma unroll
+        for (int b = 0; b < 4 * BH; ++b) *reinterpret_cast<f32x4_t*>(p + (a * 4 * BH + b) * 256) = acc[a][b];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      return;
+    }
+  }
+  gemm_store<AH, BH, MODE, 4 * AH>(acc, gsm + wave * (T::EBYTES / 8), 0, wm, wn, m0, n0, y, ldy, M, N, rp, GROUP ? entry : nullptr);
 }
 
-// tile_rows: 128 or 256, the height the tile table was made for
+// The cut tiles: a workgroup adds the pieces of a 1 / (4 AH) part of one (16 rows per wave, four pieces' loads in flight
+// together, summed in order) and finishes it.  Bound: memory, mostly the last-level cache: the pieces were just written.
+template <int AH, int BH, int MODE>
+__global__ __launch_bounds__(256) void k_gemm_sum(u16* __restrict__ y, int64_t ldy, int M, int N, int tm, int tn, const GemmRope rp, const GemmSplit sp) {
+  using T = GemmTile<AH, BH>;
+  __shared__ __attribute__((aligned(16))) u16 sm[4 * 16 * T::EPITCH];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int rt = blockIdx.x / (4 * AH), g0 = blockIdx.x - rt * 4 * AH;
+  int mt, nt;
+  gemm_tile_at(sp.full + rt, tm, tn, mt, nt);
+  const int m0 = mt * T::TM, n0 = nt * (MODE == GEMM_PAIR ? T::TN / 2 : T::TN);
+  if (m0 + (g0 / (2 * AH)) * 64 * AH + (g0 % (2 * AH)) * 16 >= M) return;   // (its lowest row; no barrier follows)
+  constexpr int C = 4 * BH, STEP = T::TM * T::TN;
+  const float* p = sp.part + (int64_t)rt * sp.splits * STEP + ((int64_t)wave * 4 * AH + g0) * (C * 256) + lane * 4;
+  f32x4_t acc[1][C], v[4][C];
+#pragma unroll
+  for (int b = 0; b < C; ++b) acc[0][b] = *reinterpret_cast<const f32x4_t*>(p + b * 256);
+  for (int s = 1; s < sp.splits; s += 4) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int b = 0; b < C; ++b)
+        v[i][b] = *reinterpret_cast<const f32x4_t*>(p + (int64_t)(s + i < sp.splits ? s + i : 0) * STEP + b * 256);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (s + i < sp.splits) {
+#pragma unroll
+        for (int b = 0; b < C; ++b) acc[0][b] += v[i][b];
+      }
+  }
+  gemm_store<AH, BH, MODE, 1>(acc, sm + wave * (16 * T::EPITCH), g0, wave >> 1, wave & 1, m0, n0, y, ldy, M, N, rp, nullptr);
+}
+
+// ---- which tile, and which tiles are cut along K
+struct GemmPlan {
+  int tile;        // index into GEMM_TILES; -1: no tile serves the shape
+  int full, rem, splits;
+};
+// What decides, measured (us; N x K; the plan's choice first, then whole tiles of 256 x 256 / 128 x 256 / 128 x 128):
+//   777 rows,  4096 x 14336   98 (64 tiles of 256 x 256 in 4 pieces)     235 / 158 / 106
+//   777 rows,  4096 x  4096   33 (224 tiles of 128 x 128)                 74 /  47 /  33
+//   300 rows,  4096 x 14336   58 (48 tiles of 128 x 256 in 4 pieces)     235 / 170 / 104
+//   128 rows,  2048 x  8192   20 (16 tiles of 128 x 128 in 8 pieces)     134 /  83 /  58
+//   128 rows, 16384 x  2048   23 (128 pair tiles of 128 x 128 in 2)       48 /  35 /  26
+//  2048 rows,  4096 x 14336  184 (128 tiles of 256 x 256 in 2 pieces)    242 / 199 / 239
+//  3002 rows, 28672 x  4096  564 (1280 tiles whole, 64 in 3 pieces)      586 / 635 / 660
+// A workgroup's time is nk * (ktile + busy * slope) + fixed, `busy` the workgroups per CU: the more CUs are at work, the
+// lower the clock and the more of them ask the L2s (256 x 256: 1.05 us per k-tile on a quarter of the chip, 1.41 on all of
+// it).  Two 128 x 128 tiles on one CU take twice the time of one.  Pieces cost a launch and their trip through memory.
+struct GemmTileCost {
+  int ah, bh, per_cu;
+  float ktile, slope, fixed;
+};
+constexpr GemmTileCost GEMM_TILES[3] = {{2, 2, 1, 0.95f, 0.46f, 5.0f}, {1, 2, 1, 0.58f, 0.29f, 3.0f}, {1, 1, 2, 0.44f, 0.06f, 3.0f}};
+constexpr size_t GEMM_SCRATCH = (size_t)64 << 20;   // pieces of one round of the largest tiles
+
+static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
+  int cus = lr_num_cus();
+  if (cus <= 0) cus = 256;
+  const int nk = (K + 63) / 64;
+  GemmPlan best{-1, 0, 0, 1};
+  float best_us = 0;
+  for (int c = 0; c < 3; ++c) {
+    const GemmTileCost& t = GEMM_TILES[c];
+    const int TM = 128 * t.ah, TN = (mode == GEMM_PAIR ? 64 : 128) * t.bh, slots = cus * t.per_cu;
+    const int64_t tiles = (int64_t)((M + TM - 1) / TM) * ((N + TN - 1) / TN), rounds = tiles / slots;
+    if (tiles > 0x3fffffff) continue;
+    const int left = (int)(tiles - rounds * slots);
+    auto round_us = [&](int workgroups, int k) {
+      const float busy = (float)workgroups / cus;
+      return k * (busy > 1.0f ? 2 * (t.ktile + t.slope) : t.ktile + busy * t.slope) + t.fixed;
+    };
+    auto consider = [&](float us, const GemmPlan& p) {
+      if (best.tile < 0 || us < best_us) {
+        best = p;
+        best_us = us;
+      }
+    };
+    const float whole = rounds * round_us(slots, nk);
+    consider(whole + (left ? round_us(left, nk) : 0.0f), GemmPlan{c, (int)tiles, 0, 1});
+    for (int s = 2; left && s <= 16 && 4 * s <= nk && left * s <= slots; ++s) {
+      const size_t bytes = (size_t)left * s * (128 * t.ah) * (128 * t.bh) * sizeof(float);
+      if (bytes > scratch) break;
+      consider(whole + round_us(left * s, (nk + s - 1) / s) + 4.5f + bytes / 6.5e6f, GemmPlan{c, (int)tiles - left, left, s});
+    }
+  }
+  return best;
+}
+
+template <int AH, int BH, bool KTAIL, int MODE>
+static int gemm_run_as(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, const GemmRope& rp,
+                       const GemmPlan& p, void* scratch, hipStream_t s) {
+  using T = GemmTile<AH, BH>;
+  static std::atomic<unsigned long long> raised{0};
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_dma<AH, BH, KTAIL, MODE, false>), T::LDS, raised)) return LR_E_LAUNCH;
+  const int gn = MODE == GEMM_PAIR ? T::TN / 2 : T::TN, tm = (M + T::TM - 1) / T::TM, tn = (N + gn - 1) / gn;
+  const GemmSplit sp{(float*)scratch, p.full, p.rem, p.splits};
+  k_gemm_dma<AH, BH, KTAIL, MODE, false><<<dim3((unsigned)(p.full + p.rem * p.splits)), dim3(256), T::LDS, s>>>(
+      (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, M, N, K, tm, tn, rp, sp, GemmGroup{});
+  if (p.rem) k_gemm_sum<AH, BH, MODE><<<dim3((unsigned)(p.rem * 4 * AH)), dim3(256), 0, s>>>((u16*)y, ldy, M, N, tm, tn, rp, sp);
+  return lr_launch_status();
+}
+template <int AH, int BH, bool KTAIL>
+static int gemm_run_mode(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, int mode, const GemmRope& rp,
+                         const GemmPlan& p, void* scratch, hipStream_t s) {
+  if (mode == GEMM_PAIR) return gemm_run_as<AH, BH, KTAIL, GEMM_PAIR>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+  if (mode == GEMM_ROPE) return gemm_run_as<AH, BH, KTAIL, GEMM_ROPE>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+  return gemm_run_as<AH, BH, KTAIL, GEMM_PLAIN>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+}
+static int gemm_run(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, int mode, const GemmRope& rp,
+                    const GemmPlan& p, void* scratch, hipStream_t s) {
+  const bool kt = K % 64 != 0;
+  if (p.tile == 0)
+    return kt ? gemm_run_mode<2, 2, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
+              : gemm_run_mode<2, 2, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+  if (p.tile == 1)
+    return kt ? gemm_run_mode<1, 2, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
+              : gemm_run_mode<1, 2, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+  return kt ? gemm_run_mode<1, 1, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
+            : gemm_run_mode<1, 1, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+}
+// whether a tile's rows lie within the 2 GiB that an offset of a request reaches (N: pairs in PAIR mode)
+static bool gemm_reaches(int64_t ldx, int N, int K, int mode) {
+  return 256 * ldx * 2 < 0x7fffffff && ((mode == GEMM_PAIR ? (int64_t)N : 0) + 256) * K * 2 < 0x7fffffff;
+}
+static int gemm(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, int mode, const GemmRope& rp, void* scratch,
+                size_t scratch_bytes, hipStream_t s) {
+  if (!gemm_reaches(ldx, N, K, mode)) return LR_E_UNSUPPORTED;
+  const GemmPlan p = gemm_plan(M, N, K, mode, scratch == nullptr || lr_misaligned(scratch) ? 0 : scratch_bytes);
+  if (p.tile < 0) return LR_E_UNSUPPORTED;
+  return gemm_run(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+}
+
+// Grouped products (lr_moe): rows of several matrices' tiles, see GemmGroup; pair_off != 0: GEMM_PAIR (N counts pairs).
+// tile_rows: 128 or 256, the height the tile table was made for.
+namespace lr_detail {
+template <int AH, int BH, bool KTAIL, int MODE>
+static int gemm_grouped_as(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int N, int K, const GemmGroup& gp, int max_tiles,
+                           hipStream_t s) {
+  using T = GemmTile<AH, BH>;
+  constexpr size_t lds = T::LDS + T::TM * sizeof(int32_t);
+  static std::atomic<unsigned long long> raised{0};
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_dma<AH, BH, KTAIL, MODE, true>), lds, raised)) return LR_E_LAUNCH;
+  const int gn = MODE == GEMM_PAIR ? T::TN / 2 : T::TN, tn = (N + gn - 1) / gn;
+  k_gemm_dma<AH, BH, KTAIL, MODE, true><<<dim3((unsigned)(max_tiles * tn)), dim3(256), lds, s>>>(
+      (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, T::TM, N, K, max_tiles, tn, GemmRope{}, GemmSplit{}, gp);
+  return lr_launch_status();
+}
 int gemm_grouped(const void* x, int64_t ldx, int64_t xrows, const void* w, void* y, int64_t ldy, int N, int K, int pair_off, int64_t wstride,
                  const int32_t* tiles, const int32_t* ntiles, const int32_t* entries, int xdiv, int max_tiles, int tile_rows, hipStream_t s) {
-  if (xrows * ldx * 2 >= 0x7fffffff || ((int64_t)pair_off + GN) * K * 2 >= 0x7fffffff) return LR_E_UNSUPPORTED;
+  if (xrows * ldx * 2 >= 0x7fffffff || ((int64_t)pair_off + 256) * K * 2 >= 0x7fffffff) return LR_E_UNSUPPORTED;
   const GemmGroup gp = {tiles, ntiles, entries, xdiv, wstride};
-  if (tile_rows == BM) {
-    const int gn = pair_off ? BN / 2 : BN, tn = (N + gn - 1) / gn;
-    k_gemm_grouped<<<dim3((unsigned)(max_tiles * tn)), dim3(256), 0, s>>>((const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, N, K, tn, pair_off, gp);
-    return lr_launch_status();
+  const bool kt = K % 64 != 0;
+  if (tile_rows == 128) {
+    if (pair_off)
+      return kt ? gemm_grouped_as<1, 1, true, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
+                : gemm_grouped_as<1, 1, false, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
+    return kt ? gemm_grouped_as<1, 1, true, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
+              : gemm_grouped_as<1, 1, false, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
   }
-  return K % BK ? gemm_grouped_as<true>(x, ldx, w, y, ldy, N, K, pair_off, gp, max_tiles, s)
-                : gemm_grouped_as<false>(x, ldx, w, y, ldy, N, K, pair_off, gp, max_tiles, s);
+  if (pair_off)
+    return kt ? gemm_grouped_as<2, 2, true, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
+              : gemm_grouped_as<2, 2, false, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
+  return kt ? gemm_grouped_as<2, 2, true, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
+            : gemm_grouped_as<2, 2, false, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
 }
 }  // namespace lr_detail
 
-extern "C" int lr_linear_tuned(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K,
-                               int act_swiglu, int gemv_cfg, lr_stream_t stream) {
+static int linear_rows(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, int act_swiglu, int gemv_cfg,
+                       void* scratch, size_t scratch_bytes, hipStream_t s) {
   LR_REQUIRE_PTR(x);
   LR_REQUIRE_PTR(w);
   LR_REQUIRE_PTR(y);
   if (M <= 0 || N <= 0 || K <= 0) return LR_E_SHAPE;
   if (ldx < (act_swiglu ? 2 : 1) * (int64_t)K || ldy < N) return LR_E_SHAPE;
   if (K % 8 || ldx % 8) return LR_E_ALIGN;
-  hipStream_t s = (hipStream_t)stream;
   if (M <= 4 || ((act_swiglu || gemv_cfg) && M <= 8))
     return lr_gemv_dispatch(x, ldx, w, y, ldy, M, N, K, act_swiglu, gemv_cfg, s);
   if (!act_swiglu && M <= 64) {
     // decode batches: the weight-streaming matrix-core kernel (stream_gemm.hip); shapes it declines fall through
     lr_projection_t pr;
     pr.x = x; pr.ldx = ldx; pr.w = w; pr.y = y; pr.ldy = ldy; pr.N = N; pr.K = K; pr.epilogue = LR_EPI_NONE; pr.rope = nullptr;
-    const int rc = lr_linear_multi(&pr, 1, M, stream);
+    const int rc = lr_linear_multi(&pr, 1, M, s);
     if (rc != LR_E_UNSUPPORTED) return rc;
   }
-  if (!act_swiglu && M >= 512 && N >= 256 && ((M + GM - 1) / GM) * ((N + GN - 1) / GN) >= 192 &&
-      (int64_t)GM * ldx * 2 < 0x7fffffff && (int64_t)GN * K * 2 < 0x7fffffff)
-    return launch_gemm_big(x, ldx, w, y, ldy, M, N, K, 0, s);
+  if (!act_swiglu) {
+    const int rc = gemm(x, ldx, w, y, ldy, M, N, K, GEMM_PLAIN, GemmRope{}, scratch, scratch_bytes, s);
+    if (rc != LR_E_UNSUPPORTED) return rc;
+  }
   const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
   if (grid.y > 65535) return LR_E_UNSUPPORTED;
   if (act_swiglu)
@@ -657,18 +711,33 @@ extern "C" int lr_linear_tuned(const void* x, int64_t ldx, const void* w, void* 
   return lr_launch_status();
 }
 
+extern "C" int lr_linear_tuned(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K,
+                               int act_swiglu, int gemv_cfg, lr_stream_t stream) {
+  return linear_rows(x, ldx, w, y, ldy, M, N, K, act_swiglu, gemv_cfg, nullptr, 0, (hipStream_t)stream);
+}
+
 extern "C" int lr_linear(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K,
                          int act_swiglu, lr_stream_t stream) {
-  return lr_linear_tuned(x, ldx, w, y, ldy, M, N, K, act_swiglu, 0, stream);
+  return linear_rows(x, ldx, w, y, ldy, M, N, K, act_swiglu, 0, nullptr, 0, (hipStream_t)stream);
+}
+
+extern "C" size_t lr_linear_scratch_bytes(int M) { return M > 64 ? GEMM_SCRATCH : 0; }
+
+extern "C" int lr_linear_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, void* scratch,
+                                 size_t scratch_bytes, lr_stream_t stream) {
+  LR_OPTIONAL_PTR(scratch);
+  return linear_rows(x, ldx, w, y, ldy, M, N, K, 0, 0, scratch, scratch_bytes, (hipStream_t)stream);
 }
 
 // The fused q/k/v projection of M = B * S rows (S tokens per sequence, row b * S + s at position pos[s]) finished as
-// lr_rope_kv_write would finish it.  One launch where the 256 x 256-tile GEMM applies; otherwise the two calls.
-extern "C" int lr_linear_rope_kv(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int K, int S,
-                                 const lr_rope_kv_t* rope, lr_stream_t stream) {
+// lr_rope_kv_write would finish it, in the GEMM's output pass; up to 64 rows (and rows out of the requests' reach) in the
+// two calls.
+extern "C" int lr_linear_rope_kv_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int K, int S,
+                                         const lr_rope_kv_t* rope, void* scratch, size_t scratch_bytes, lr_stream_t stream) {
   LR_REQUIRE_PTR(x);
   LR_REQUIRE_PTR(w);
   LR_REQUIRE_PTR(y);
+  LR_OPTIONAL_PTR(scratch);
   if (rope == nullptr || rope->pos == nullptr) return LR_E_NULL;
   LR_REQUIRE_PTR(rope->table);
   LR_REQUIRE_PTR(rope->k_cache);
@@ -681,22 +750,31 @@ extern "C" int lr_linear_rope_kv(const void* x, int64_t ldx, const void* w, void
   if (K % 8 || ldx % 8 || ldy % 8 || rope->head_dim % 8) return LR_E_ALIGN;
   const int N = (int)n64;
   hipStream_t s = (hipStream_t)stream;
-  if (M >= 512 && N >= 256 && ((M + GM - 1) / GM) * ((N + GN - 1) / GN) >= 192 && (int64_t)GM * ldx * 2 < 0x7fffffff &&
-      (int64_t)GN * K * 2 < 0x7fffffff)
-    return launch_gemm_big(x, ldx, w, y, ldy, M, N, K, 0, s, rope, S);
-  const int rc = lr_linear(x, ldx, w, y, ldy, M, N, K, 0, stream);
+  if (M > 64) {
+    const GemmRope rp{(const u16*)rope->table, rope->pos, (u16*)rope->k_cache, (u16*)rope->v_cache, rope->err, S, rope->n_head,
+                      rope->n_kv_head, rope->head_dim, rope->smax, rope->block_size};
+    const int rc = gemm(x, ldx, w, y, ldy, M, N, K, GEMM_ROPE, rp, scratch, scratch_bytes, s);
+    if (rc != LR_E_UNSUPPORTED) return rc;
+  }
+  const int rc = linear_rows(x, ldx, w, y, ldy, M, N, K, 0, 0, scratch, scratch_bytes, s);
   if (rc != LR_OK) return rc;
   return lr_rope_kv_write(y, ldy, rope->table, 0, rope->pos, rope->k_cache, rope->v_cache, M / S, S, rope->n_head,
                           rope->n_kv_head, rope->head_dim, rope->smax, rope->block_size, rope->err, stream);
 }
 
+extern "C" int lr_linear_rope_kv(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int K, int S,
+                                 const lr_rope_kv_t* rope, lr_stream_t stream) {
+  return lr_linear_rope_kv_scratch(x, ldx, w, y, ldy, M, K, S, rope, nullptr, 0, stream);
+}
+
 // y[M, I] = bf16( bf16(silu(g)) * u ) for [u | g] = x w^T with w = [up; gate] rows (N = 2 I): the MLP's first
 // projection with the activation applied on the way out (utils.py:145-148 without the [M, 2 I] tensor).
-extern "C" int lr_linear_swiglu_out(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K,
-                                    void* scratch, size_t scratch_bytes, lr_stream_t stream) {
+extern "C" int lr_linear_swiglu_out_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K,
+                                            void* scratch, size_t scratch_bytes, void* sums, size_t sums_bytes, lr_stream_t stream) {
   LR_REQUIRE_PTR(x);
   LR_REQUIRE_PTR(w);
   LR_REQUIRE_PTR(y);
+  LR_OPTIONAL_PTR(sums);
   if (M <= 0 || N <= 0 || K <= 0 || N % 2 || ldx < K || ldy < N / 2) return LR_E_SHAPE;
   if (K % 8 || ldx % 8) return LR_E_ALIGN;
   const int I = N / 2;
@@ -706,13 +784,20 @@ extern "C" int lr_linear_swiglu_out(const void* x, int64_t ldx, const void* w, v
     const int rc = lr_linear_multi(&pr, 1, M, stream);
     if (rc != LR_E_UNSUPPORTED) return rc;
   }
-  if (M >= 512 && I >= 128 && ((M + GM - 1) / GM) * ((I + GN / 2 - 1) / (GN / 2)) >= 192 &&
-      (int64_t)GM * ldx * 2 < 0x7fffffff && ((int64_t)I + GN) * K * 2 < 0x7fffffff)
-    return launch_gemm_big(x, ldx, w, y, ldy, M, I, K, I, (hipStream_t)stream);
-  // other sizes: the projection into `scratch` [M, N], then the activation
-  LR_REQUIRE_PTR(scratch);
-  if (scratch_bytes < (size_t)M * N * sizeof(u16)) return LR_E_SHAPE;
-  const int rc = lr_linear(x, ldx, w, scratch, N, M, N, K, 0, stream);
+  // (a caller of other than large problems brings `scratch` [M, N]; used where the weights are out of the requests' reach)
+  const bool large = M >= 512 && I >= 128 && (int64_t)((M + 255) / 256) * ((I + 127) / 128) >= 192 && gemm_reaches(ldx, I, K, GEMM_PAIR);
+  if (!large) {
+    LR_REQUIRE_PTR(scratch);
+    if (scratch_bytes < (size_t)M * N * sizeof(u16)) return LR_E_SHAPE;
+  }
+  int rc = gemm(x, ldx, w, y, ldy, M, I, K, GEMM_PAIR, GemmRope{}, sums, sums_bytes, (hipStream_t)stream);
+  if (rc != LR_E_UNSUPPORTED) return rc;
+  rc = linear_rows(x, ldx, w, scratch, N, M, N, K, 0, 0, nullptr, 0, (hipStream_t)stream);
   if (rc != LR_OK) return rc;
   return lr_detail::swiglu_rows(scratch, N, y, ldy, M, I, stream);
+}
+
+extern "C" int lr_linear_swiglu_out(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K,
+                                    void* scratch, size_t scratch_bytes, lr_stream_t stream) {
+  return lr_linear_swiglu_out_scratch(x, ldx, w, y, ldy, M, N, K, scratch, scratch_bytes, nullptr, 0, stream);
 }

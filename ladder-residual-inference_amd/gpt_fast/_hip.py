@@ -25,9 +25,14 @@ _PROTOS = {
     "lr_linear": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_void_p]),
     "lr_linear_tuned": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int,
                                 c_void_p]),
+    "lr_linear_scratch_bytes": (c_size_t, [c_int]),
+    "lr_linear_scratch": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_size_t,
+                                  c_void_p]),
     "lr_linear_multi": (c_int, [c_void_p, c_int, c_int, c_void_p]),
     "lr_linear_swiglu_out": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p,
                                      c_size_t, c_void_p]),
+    "lr_linear_swiglu_out_scratch": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p,
+                                             c_size_t, c_void_p, c_size_t, c_void_p]),
     "lr_linear_fp8_scratch_bytes": (c_size_t, [c_int, c_int, c_int]),
     "lr_linear_fp8_multi": (c_int, [c_void_p, c_int, c_int, c_void_p]),
     "lr_linear_fp8": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p,
@@ -39,6 +44,8 @@ _PROTOS = {
                              c_int, c_int, c_int, c_void_p, c_void_p]),
     "lr_linear_rope_kv": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p,
                                   c_void_p]),
+    "lr_linear_rope_kv_scratch": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p,
+                                          c_void_p, c_size_t, c_void_p]),
     "lr_attn_decode_scratch_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
     "lr_attn_decode": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int,
                                c_int, c_int, c_void_p, c_size_t, c_void_p]),
@@ -223,9 +230,18 @@ def ladder_norms(resid_in, d1, d2, gain1, gain2, resid_out, normed1, normed2, ep
                                   _dev(normed2), rows, dim, float(eps), _stream()), "lr_ladder_norms")
 
 
-def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, act_swiglu: bool = False, gemv_cfg: int = 0):
+def linear_scratch_bytes(rows: int) -> int:
+    return int(load().lr_linear_scratch_bytes(rows))
+
+
+def _scratch_args(t):
+    return (None, 0) if t is None else (t.data_ptr(), t.numel() * t.element_size())
+
+
+def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, act_swiglu: bool = False, gemv_cfg: int = 0, scratch=None):
     """out[M, N] = x[M, K] @ w[N, K]^T (x = [u | g] of width 2K when act_swiglu).  gemv_cfg != 0 goes
-    through lr_linear_tuned (an explicit GEMV launch configuration for this one call)."""
+    through lr_linear_tuned (an explicit GEMV launch configuration for this one call).  `scratch`: device memory for partial
+    sums (linear_scratch_bytes), not shared with calls that may overlap."""
     M, xc, ldx = _rows_ld(x)
     N, K = w.shape
     assert w.is_contiguous() and xc == (2 * K if act_swiglu else K), (x.shape, w.shape, act_swiglu)
@@ -238,6 +254,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, act_swiglu: bool
     elif gemv_cfg:
         _check(load().lr_linear_tuned(_dev(x), ldx, _dev(w), _dev(out), ldy, M, N, K, int(act_swiglu), int(gemv_cfg),
                                       _stream()), "lr_linear_tuned")
+    elif scratch is not None and not act_swiglu:
+        _check(load().lr_linear_scratch(_dev(x), ldx, _dev(w), _dev(out), ldy, M, N, K, *_scratch_args(scratch), _stream()),
+               "lr_linear_scratch")
     else:
         _check(load().lr_linear(_dev(x), ldx, _dev(w), _dev(out), ldy, M, N, K, int(act_swiglu), _stream()),
                "lr_linear")
@@ -272,16 +291,16 @@ def rope_kv_epilogue(table, pos, k_cache, v_cache, Hq, Hkv, hd, n_pos=1):
                    device_error_word(k_cache.device).data_ptr(), Hq, Hkv, hd, Smax, table.shape[0])
 
 
-def linear_rope_kv(x, w, out, table, pos, k_cache, v_cache, B, S, Hq, Hkv, hd):
+def linear_rope_kv(x, w, out, table, pos, k_cache, v_cache, B, S, Hq, Hkv, hd, scratch=None):
     """The fused q/k/v projection of B * S rows, rotated and cached on its way out (lr_linear_rope_kv): what
-    linear(x, w, out) followed by rope_kv_write(out, table, False, pos, ...) leaves."""
+    linear(x, w, out, scratch=scratch) followed by rope_kv_write(out, table, False, pos, ...) leaves."""
     M, K, ldx = _rows_ld(x)
     Mo, N, ldy = _rows_ld(out)
     assert M == Mo == B * S and w.is_contiguous() and tuple(w.shape) == ((Hq + 2 * Hkv) * hd, K) and N == w.shape[0]
     assert B <= k_cache.shape[0]
     rope = rope_kv_epilogue(table, pos, k_cache, v_cache, Hq, Hkv, hd, n_pos=S)
-    _check(load().lr_linear_rope_kv(_dev(x), ldx, _dev(w), _dev(out), ldy, M, K, S, ctypes.byref(rope), _stream()),
-           "lr_linear_rope_kv")
+    _check(load().lr_linear_rope_kv_scratch(_dev(x), ldx, _dev(w), _dev(out), ldy, M, K, S, ctypes.byref(rope),
+                                            *_scratch_args(scratch), _stream()), "lr_linear_rope_kv_scratch")
     return out
 
 
@@ -393,7 +412,7 @@ def linear_fp8(x: torch.Tensor, w8: torch.Tensor, scales: torch.Tensor, out: tor
     return out
 
 
-def linear_swiglu(h: torch.Tensor, w: torch.Tensor, out: torch.Tensor, act: torch.Tensor = None):
+def linear_swiglu(h: torch.Tensor, w: torch.Tensor, out: torch.Tensor, act: torch.Tensor = None, scratch=None):
     """out = (silu(g) * u) @ w^T for h = [u | g].  Up to 4 rows the activation is fused into the
     weight-streaming GEMV; above that it is materialised once (in `act`, or a new tensor) and fed to
     the plain MFMA GEMM, whose operand loader is then a pure copy."""
@@ -403,35 +422,36 @@ def linear_swiglu(h: torch.Tensor, w: torch.Tensor, out: torch.Tensor, act: torc
     if act is None:
         act = h.new_empty(M, two_k // 2)
     swiglu(h, act)
-    return linear(act, w, out)
+    return linear(act, w, out, scratch=scratch)
 
 
-def linear_swiglu_out(x: torch.Tensor, w1: torch.Tensor, act: torch.Tensor, scratch: torch.Tensor = None):
+def linear_swiglu_out(x: torch.Tensor, w1: torch.Tensor, act: torch.Tensor, scratch: torch.Tensor = None, sums=None):
     """act[M, I] = silu(g) * u for [u | g] = x @ w1^T, w1 = [up; gate] rows: the activation is applied in the
-    projection's epilogue where the shape allows (lr_linear_swiglu_out); `scratch` [M, 2 I] serves the rest."""
+    projection's epilogue where the shape allows (lr_linear_swiglu_out); `scratch` [M, 2 I] serves the rest.  `sums`: as
+    linear's scratch."""
     M, K, ldx = _rows_ld(x)
     N, Kw = w1.shape
     Mo, Io, ldy = _rows_ld(act)
     assert w1.is_contiguous() and Kw == K and N % 2 == 0 and (Mo, Io) == (M, N // 2), (x.shape, w1.shape, act.shape)
     sp, sb = (None, 0) if scratch is None else (_dev(scratch), scratch.numel() * scratch.element_size())
-    _check(load().lr_linear_swiglu_out(_dev(x), ldx, _dev(w1), _dev(act), ldy, M, N, K, sp, sb, _stream()),
-           "lr_linear_swiglu_out")
+    _check(load().lr_linear_swiglu_out_scratch(_dev(x), ldx, _dev(w1), _dev(act), ldy, M, N, K, sp, sb, *_scratch_args(sums),
+                                               _stream()), "lr_linear_swiglu_out_scratch")
     return act
 
 
-def module_linear(x: torch.Tensor, mod, out: torch.Tensor):
+def module_linear(x: torch.Tensor, mod, out: torch.Tensor, scratch=None):
     """mod(x) for an nn.Linear (bf16 weight) or a weight-only fp8 replacement (`weight` e4m3 + `scales`)."""
     scales = getattr(mod, "scales", None)
     if scales is not None:
         return linear_fp8(x, mod.weight, scales, out)
-    return linear(x, mod.weight, out)
+    return linear(x, mod.weight, out, scratch=scratch)
 
 
-def module_linear_swiglu(h: torch.Tensor, mod, out: torch.Tensor, act: torch.Tensor = None):
+def module_linear_swiglu(h: torch.Tensor, mod, out: torch.Tensor, act: torch.Tensor = None, scratch=None):
     """mod(silu(g) * u) for h = [u | g]."""
     scales = getattr(mod, "scales", None)
     if scales is None:
-        return linear_swiglu(h, mod.weight, out, act)
+        return linear_swiglu(h, mod.weight, out, act, scratch)
     M, two_k, _ = _rows_ld(h)
     if act is None:
         act = h.new_empty(M, two_k // 2)

@@ -23,6 +23,8 @@ class HybridWorkspace:
         self.xc = e(rows, D)                      # in the compute type: the input of the next product
         self.d = e(rows, D)                       # what the current sublayer adds to the residual
         self.proj = e(rows, pad8(max(m.proj_cols for m in mixers)))
+        n = _hip.linear_scratch_bytes(rows) if dtype == torch.bfloat16 else 0
+        self.sums = e(n, dt=torch.uint8) if n else None      # partial sums of products
         n = max(m.scratch_bytes(B, S) for m in mixers)
         self.scratch = e(n, dt=torch.uint8) if n else None
         n = max((r * c for r, c in (m.window_rows(B, S) for m in mixers)), default=0)

@@ -45,6 +45,9 @@ class Workspace:
         self.next_token = torch.empty(B, 1, dtype=torch.int32, device=device)
         self.next_token_valid_for = None   # set by a fused decode step that already chose the token
         self.scratch = None
+        # partial sums of the prefill GEMM (only for prompts: a decode step's chains may run on two streams)
+        n = _hip.linear_scratch_bytes(rows) if S > 1 else 0
+        self.sums = torch.empty(n, dtype=torch.uint8, device=device) if n else None
         if S == 1:
             n = _hip.attn_decode_scratch_bytes(B, cfg.n_head_local, hd, smax) // 4
             self.scratch = torch.empty(n, dtype=torch.float32, device=device)
@@ -179,10 +182,10 @@ class GPTBase(nn.Module):
             last = lambda t, out: None if t is None else _hip.embed(t.view(B * S, -1), ws.last_rows, out)
             _hip.add_rmsnorm(last(ws.x, ws.xl), last(final_d1, ws.d1l), last(final_d2, ws.d2l), self.norm.weight, None,
                              ws.xnl, cfg.norm_eps)
-            _hip.module_linear(ws.xnl, self.output, ws.logits.view(B, -1))
+            _hip.module_linear(ws.xnl, self.output, ws.logits.view(B, -1), ws.sums)
         else:
             _hip.add_rmsnorm(ws.x, final_d1, final_d2, self.norm.weight, None, ws.xn, cfg.norm_eps)
-            _hip.module_linear(ws.xn, self.output, ws.logits.view(B * S, -1))
+            _hip.module_linear(ws.xn, self.output, ws.logits.view(B * S, -1), ws.sums)
         return ws.logits
 
     def _run_layers(self, ws: Workspace, pos: Tensor):
@@ -219,10 +222,10 @@ class GPTBase(nn.Module):
         elif (wqkv is not None and S > 1 and not roped and not hasattr(wqkv, "scales")
               and wqkv.weight.shape[0] == (Hq + 2 * Hkv) * hd):   # (not the parallel family's wider projection)
             # prefill: the projection rotates q and caches rotated k and v on its way out (one launch of the GEMM)
-            _hip.linear_rope_kv(ws.xn, wqkv.weight, ws.qkv, self.freqs_cis, pos, kc, vc, B, S, Hq, Hkv, hd)
+            _hip.linear_rope_kv(ws.xn, wqkv.weight, ws.qkv, self.freqs_cis, pos, kc, vc, B, S, Hq, Hkv, hd, ws.sums)
             roped = True
         elif wqkv is not None:
-            _hip.module_linear(ws.xn, wqkv, ws.qkv)
+            _hip.module_linear(ws.xn, wqkv, ws.qkv, ws.sums)
         if not roped:
             _hip.rope_kv_write(ws.qkv, self.freqs_cis, False, pos, kc, vc, B, S, Hq, Hkv, hd)
         if S == 1:
@@ -234,7 +237,7 @@ class GPTBase(nn.Module):
         if bands:
             _hip.linear_multi((ws.y, blk.attention.wo.weight, out, _hip.EPI_NONE))
         else:
-            _hip.module_linear(ws.y, blk.attention.wo, out)
+            _hip.module_linear(ws.y, blk.attention.wo, out, ws.sums)
 
     def _mlp(self, ws: Workspace, blk, out: Tensor, xn: Optional[Tensor] = None):
         ff = blk.feed_forward
@@ -245,8 +248,8 @@ class GPTBase(nn.Module):
             return
         if xin.shape[0] > 4 and not hasattr(ff.w1, "scales"):
             # the activation in the first projection's epilogue; up to 4 rows it is fused into w2's GEMV instead
-            _hip.linear_swiglu_out(xin, ff.w1.weight, ws.act, ws.h)
-            _hip.module_linear(ws.act, ff.w2, out)
+            _hip.linear_swiglu_out(xin, ff.w1.weight, ws.act, ws.h, ws.sums)
+            _hip.module_linear(ws.act, ff.w2, out, ws.sums)
             return
         _hip.module_linear(xin, ff.w1, ws.h)
         _hip.module_linear_swiglu(ws.h, ff.w2, out, ws.act)

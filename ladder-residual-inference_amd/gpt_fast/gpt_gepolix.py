@@ -110,7 +110,7 @@ class GPTGepolix(GPTHybrid):
             blk.mixer.mix(ws, pos, proj, y)
             if m is not None:
                 _hip.moe(routed)
-            following.after(both, blk.mixer.out_proj, ws.d, ws.x, ws.xc, experts)
+            following.after(both, blk.mixer.out_proj, ws.d, ws.x, ws.xc, experts, ws.sums)
         return None, None
 
     def _project_in(self, ws, blk, act, routed):
@@ -128,18 +128,18 @@ class GPTGepolix(GPTHybrid):
                 _hip.linear_multi(*todo)
             return proj
         if blk.w1 is None:
-            return project(ws.xc, blk.mixer.in_proj, proj)
+            return project(ws.xc, blk.mixer.in_proj, proj, ws.sums)
         h = ws.h[:ws.rows * 2 * blk.beside].view(ws.rows, -1)
         if ws.xc.dtype == torch.float32:
             _hip.linear(ws.xc, blk.w1.weight, h)
             _hip.swiglu(h, act)
             _hip.linear(ws.xc, w, proj)
         else:
-            _hip.linear_swiglu_out(ws.xc, blk.w1.weight, act, h)
-            _hip.linear(ws.xc, w, proj)
+            _hip.linear_swiglu_out(ws.xc, blk.w1.weight, act, h, ws.sums)
+            _hip.linear(ws.xc, w, proj, scratch=ws.sums)
         return proj
 
     def _head(self, ws, d1, d2):
         xc = ws.xc if ws.last_rows is None else self._last(ws, ws.xc)[1]
-        project(xc, self.output, ws.logits.flatten(0, 1))
+        project(xc, self.output, ws.logits.flatten(0, 1), ws.sums)
         return ws.logits

@@ -84,8 +84,8 @@ class GPTLasivik(GPTHybrid):
             _hip.linear(ws.xc, ff.w1.weight, h)
             _hip.swiglu(h, act)
         else:
-            _hip.linear_swiglu_out(ws.xc, ff.w1.weight, act, h)
-        project(act, ff.w2, ws.d)
+            _hip.linear_swiglu_out(ws.xc, ff.w1.weight, act, h, ws.sums)
+        project(act, ff.w2, ws.d, ws.sums)
 
     def _head(self, ws, d1, d2):
         cfg = self.config
@@ -94,6 +94,6 @@ class GPTLasivik(GPTHybrid):
             x, xc = self._last(ws, ws.x)
         _hip.residual_rmsnorm(x, 1.0, None, self.norm.weight, None, xc, cfg.norm_eps, cfg.width, gain_offset=1.0)
         logits = ws.logits.flatten(0, 1)
-        project(xc, self.output, logits)
+        project(xc, self.output, logits, ws.sums)
         _hip.logit_cap(logits, cfg.logit_scale, cfg.logit_softcap)
         return ws.logits

@@ -50,13 +50,13 @@ class MixerArgs:
     taps: int = 1                   # mamba2: of the convolution ahead of the state space
 
 
-def project(x: Tensor, lin: nn.Linear, out: Tensor) -> Tensor:
+def project(x: Tensor, lin: nn.Linear, out: Tensor, sums: Optional[Tensor] = None) -> Tensor:
     """lin(x) for the rows of a step: the weight-streaming kernel from two to 64 rows (as the other families' decode
-    steps use it), what the shape picks otherwise."""
+    steps use it), what the shape picks otherwise.  `sums`: the workspace's memory for partial sums."""
     if x.dtype == torch.bfloat16 and 2 <= x.shape[0] <= 64:
         _hip.linear_multi((x, lin.weight, out, _hip.EPI_NONE))
         return out
-    return _hip.linear(x, lin.weight, out)
+    return _hip.linear(x, lin.weight, out, scratch=sums)
 
 
 def rotate_half_table(length: int, dims: int, base: float) -> Tensor:
@@ -106,7 +106,7 @@ class Mixer(nn.Module):
         raise NotImplementedError
 
     def _project_in(self, ws) -> Tensor:
-        return project(ws.xc, self.in_proj, ws.proj[:, :self.proj_cols])
+        return project(ws.xc, self.in_proj, ws.proj[:, :self.proj_cols], ws.sums)
 
     def _y(self, ws) -> Tensor:
         return ws.y_of(self.y_cols, self.args.heads * self.args.vdim)
@@ -118,7 +118,7 @@ class Mixer(nn.Module):
     def run(self, ws, pos: Tensor):
         y = self._y(ws)
         self.mix(ws, pos, self._project_in(ws), y)
-        project(y, self.out_proj, ws.d)
+        project(y, self.out_proj, ws.d, ws.sums)
 
 
 class _LinearAttention(Mixer):
@@ -231,7 +231,7 @@ class LatentAttention(Mixer):
                 rows = cache[:ws.B].view(ws.B * n, self.rank_p)
             else:
                 _hip.latent_window(cache, pos, rows.view(ws.B, n, self.rank_p), ws.B, a.window)
-            _hip.linear(rows, self.kv_up.weight, kv)
+            _hip.linear(rows, self.kv_up.weight, kv, scratch=ws.sums)
             _hip.window_attention(proj[:, :nq], kv, y, pos, ws.B, ws.S, a.heads, a.dim, a.vdim, a.window, n,
                                   cache.shape[1], a.scale)
 

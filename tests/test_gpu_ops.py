@@ -821,3 +821,59 @@ def test_stream_read_runs_and_leaves_the_sink_alone(hip):
     assert sink.item() == 1234
     with pytest.raises(hip.LadderHipError):
         hip.stream_read(buf[:1024], sink)
+
+
+# ------------------------------------------------------------------------------------ the prefill GEMM's tiles and pieces
+
+@pytest.mark.parametrize("M,N,K", [
+    (65, 8, 8), (100, 72, 64), (129, 264, 520), (256, 256, 128), (257, 512, 192), (300, 520, 200), (513, 40, 4096),
+    (777, 1032, 1000),                                   # one row, column or k too many for every tile; odd numbers of k-tiles
+    (128, 1024, 8192), (300, 2048, 4160), (777, 2048, 7168),   # cut along K where there is memory for it: 128 x 128,
+    (2100, 2560, 8192),                                        # 128 x 256 and 256 x 256 tiles; whole rounds first
+])
+def test_linear_tiles_and_pieces(hip, M, N, K):
+    """Whole tiles, and tiles cut along K with their sums added by a second launch, against the float64 product: fp32
+    accumulation and one rounding either way (the assert allows the rounding to fall on the other side).  The cut form
+    repeats bit for bit and writes no row or column beyond its own."""
+    x, w = rnd(M, K, seed=90), rnd(N, K, seed=91, scale=K ** -0.5)
+    want = (x.double() @ w.double().T).to(BF)
+    sums = torch.empty(hip.linear_scratch_bytes(M), dtype=torch.uint8, device=DEV)
+    outs = []
+    for scratch in (None, sums, sums):
+        y = torch.full((M + 1, N + 8), 5.0, dtype=BF, device=DEV)
+        hip.linear(x, w, y[:M, :N], scratch=scratch)
+        assert_close_ulp(y[:M, :N].contiguous(), want, what=f"{M} x {N} x {K}")
+        assert (y[M:] == 5.0).all() and (y[:, N:] == 5.0).all()
+        outs.append(y)
+    assert torch.equal(outs[1], outs[2])
+
+
+@pytest.mark.parametrize("M,I,K", [(128, 512, 4096), (300, 1000, 4104), (777, 2048, 4096)])
+def test_linear_swiglu_out_pieces(hip, M, I, K):
+    """[up; gate] pairs in cut tiles: the activation after the sums are complete."""
+    x, w1 = rnd(M, K, seed=92), rnd(2 * I, K, seed=93, scale=K ** -0.5)
+    act, h = torch.empty(M, I, dtype=BF, device=DEV), torch.empty(M, 2 * I, dtype=BF, device=DEV)
+    hip.linear_swiglu_out(x, w1, act, h, torch.empty(hip.linear_scratch_bytes(M), dtype=torch.uint8, device=DEV))
+    u, g = (x.double() @ w1.double().T).to(BF).float().chunk(2, 1)
+    want = ((g / (1 + torch.exp(-g))).to(BF).float() * u).to(BF)
+    # up, gate and silu(gate) are each rounded: one step of any of them is at most 2^-7 of the result
+    assert ((act.float() - want.float()).abs() <= 2.0 ** -7 * 3 * want.float().abs() + 2.0 ** -12).all()
+    assert (ulp_diff(act, want) > 0).float().mean().item() < 0.05
+
+
+@pytest.mark.parametrize("B,S,Hq,Hkv,hd,K", [(1, 128, 8, 2, 64, 4096), (3, 100, 4, 1, 128, 4104), (2, 389, 16, 4, 128, 4096)])
+def test_linear_rope_kv_pieces(hip, B, S, Hq, Hkv, hd, K):
+    """The q/k/v projection in cut tiles, rotated and cached after the sums: the two calls on the same plan, bit for bit."""
+    N, Smax, start = (Hq + 2 * Hkv) * hd, S + 11, 5
+    x, w = rnd(B * S, K, seed=94), rnd(N, K, seed=95, scale=K ** -0.5)
+    sums = torch.empty(hip.linear_scratch_bytes(B * S), dtype=torch.uint8, device=DEV)
+    pos = torch.arange(start, start + S, dtype=torch.int32, device=DEV)
+    table = O.rope_table(start + S, hd, 500000, BF).to(DEV)
+    out = [torch.empty(B * S, N, dtype=BF, device=DEV) for _ in range(2)]
+    kc = [torch.zeros(B, Hkv, Smax, hd, dtype=BF, device=DEV) for _ in range(2)]
+    vc = [torch.zeros_like(kc[0]) for _ in range(2)]
+    hip.linear(x, w, out[0], scratch=sums)
+    hip.rope_kv_write(out[0], table, False, pos, kc[0], vc[0], B, S, Hq, Hkv, hd)
+    hip.linear_rope_kv(x, w, out[1], table, pos, kc[1], vc[1], B, S, Hq, Hkv, hd, sums)
+    assert torch.equal(out[0], out[1]) and torch.equal(kc[0], kc[1]) and torch.equal(vc[0], vc[1])
+    hip.raise_on_device_error(out[0].device)
