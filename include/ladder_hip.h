@@ -106,7 +106,8 @@ int lr_linear(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, i
 /* lr_linear (act_swiglu = 0) with memory for partial sums: where the tiles of the matrix-core GEMM would leave compute
  * units idle, tiles are cut along K, the pieces' fp32 sums go to `scratch` and a second launch adds them, in a fixed order.
  * Any size is legal, a larger one allows more pieces; lr_linear_scratch_bytes(M) bytes are always enough (0: none would be
- * used).  Calls that may overlap need memory of their own.  No counterpart in the reference. */
+ * used).  With scratch the GEMM also serves M of 33 to 64, where it is then faster than the weight-streaming kernel.
+ * Calls that may overlap need memory of their own.  No counterpart in the reference. */
 size_t lr_linear_scratch_bytes(int M);
 int lr_linear_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, void* scratch,
                       size_t scratch_bytes, lr_stream_t stream);

@@ -131,8 +131,8 @@ __global__ __launch_bounds__(256) void k_gemm(const u16* __restrict__ x, int64_t
 }
 
 // ---------------------------------------------------------------------------------------------
-// The prefill GEMM.  A workgroup of four waves (2 x 2) multiplies a tile of 128 AH input rows x 128 BH weight rows;
-// AH x BH is 2 x 2, 1 x 2 or 1 x 1 (gemm_plan picks).  Bound: the matrix cores, at the clock the chip's power allows --
+// The GEMM of prompts and of decode batches above 32.  A workgroup of four waves (2 x 2) multiplies a tile of 64 A16 input
+// rows x 128 BH weight rows: 256 x 256, 128 x 256, 128 x 128 or 64 x 128 (gemm_plan picks).  Bound: the matrix cores, at the clock the chip's power allows --
 // 16384 x 4096 x 14336: 1.50 PFLOP/s, matrix cores busy 86 % of the cycles at 1.57 GHz -- from a few hundred rows on; the
 // weights' HBM traffic below.
 //
@@ -182,23 +182,28 @@ struct GemmSplit {
 };
 enum { GEMM_PLAIN, GEMM_PAIR, GEMM_ROPE };   // PAIR: w holds [up; gate] rows, N counts pairs, output silu(gate) * up
 
-template <int AH, int BH>
+template <int A16, int BH>
 struct GemmTile {
-  static constexpr int TM = 128 * AH, TN = 128 * BH;
-  static constexpr int HA = 8192 * AH, HB = 8192 * BH;   // bytes of half an operand's k-tile
-  static constexpr int NA = 2 * AH, NB = 2 * BH;         // DMA instructions of a wave for it
+  static constexpr int TM = 64 * A16, TN = 128 * BH;
+  static constexpr int HA = 4096 * A16, HB = 8192 * BH;   // bytes of half an operand's k-tile
+  static constexpr int NA = A16, NB = 2 * BH;         // DMA instructions of a wave for it
   static constexpr int RING = 4 * (HA + HB);
   static constexpr int EPITCH = 64 * BH + 8;             // row pitch of a wave's output piece (plain), in elements
-  static constexpr int EBYTES = 4 * 64 * AH * EPITCH * 2;
+  static constexpr int EBYTES = 4 * 32 * A16 * EPITCH * 2;
   static constexpr int LDS = RING > EBYTES ? RING : EBYTES;
 };
 
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
 // One wave instruction: 64 x 16 bytes from memory to LDS at `lds` + 16 * lane.  (s_nop: the wait state between a write of
 // M0 and its use; the scalar operands come from scalar instructions.)
+template <bool NT>
 __device__ __forceinline__ void dma16(const i32x4_t& rsrc, int voff, int soff, u32 lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
-               : "memory");
+  if (NT)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
+                 : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
+                 : "memory");
 }
 template <int N>
 __device__ __forceinline__ void wait_requests_and_lds() {
@@ -224,7 +229,7 @@ __device__ __forceinline__ void gemm_tile_at(int t, int tm, int tn, int& mt, int
 // of weight rows, the others of its second.  Stored from there an instruction would touch 32 bytes in each of 16 rows: they
 // take one trip through LDS (`eb`, a piece of the wave's own) and leave as whole rows.  `row0`: first of the wave's row
 // groups here, m = tile row of group g is row_of(g).
-template <int AH, int BH, int MODE, int R16>
+template <int A16, int BH, int MODE, int R16>
 __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u16* eb, int g0, int wm, int wn, int m0, int n0, u16* __restrict__ y,
                                            int64_t ldy, int M, int N, const GemmRope& rp, const int32_t* entry) {
   int lane = threadIdx.x & 63;   // (laundered: the addresses below are not formed before the k loop and kept through it)
@@ -250,7 +255,7 @@ __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u1
   const bool vec_ok = (ldy & 7) == 0;
   auto row_of = [&](int ml) {
     const int g = g0 + (ml >> 4);
-    return m0 + (g / (2 * AH)) * 64 * AH + wm * 32 * AH + (g % (2 * AH)) * 16 + (ml & 15);
+    return m0 + (g / (A16)) * 32 * A16 + wm * 16 * A16 + (g % (A16)) * 16 + (ml & 15);
   };
   auto store_row = [&](int m, int n, const uint4& v) {
     if (m >= M) return;
@@ -315,12 +320,13 @@ __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u1
   }
 }
 
-// KTAIL: K is not a multiple of the 64-element k-tile, so the last one needs a per-lane range check.
-template <int AH, int BH, bool KTAIL, int MODE, bool GROUP>
-__global__ __launch_bounds__(256, AH * BH == 1 ? 2 : 1) void k_gemm_dma(const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
+// KTAIL: K is not a multiple of the 64-element k-tile, so the last one needs a per-lane range check.  NT: weights are loaded
+// non-temporally.
+template <int A16, int BH, bool KTAIL, int MODE, bool GROUP, bool NT = false>
+__global__ __launch_bounds__(256, A16 * BH <= 2 ? 2 : 1) void k_gemm_dma(const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
                                                                         u16* __restrict__ y, int64_t ldy, int M, int N, int K, int tm, int tn,
                                                                         const GemmRope rp, const GemmSplit sp, const GemmGroup gp) {
-  using T = GemmTile<AH, BH>;
+  using T = GemmTile<A16, BH>;
   constexpr int HA = T::HA, HB = T::HB, NA = T::NA, NB = T::NB, BOFF = 4 * HA;
   extern __shared__ __attribute__((aligned(1024))) u16 gsm[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -367,7 +373,7 @@ __global__ __launch_bounds__(256, AH * BH == 1 ? 2 : 1) void k_gemm_dma(const u1
   for (int h = 0; h < 2; ++h) {
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
-      const int r = h * 64 * AH + (wave * NA + i) * 8 + (lane >> 3);
+      const int r = h * 32 * A16 + (wave * NA + i) * 8 + (lane >> 3);
       const int row = GROUP ? entry[r] / gp.xdiv : r;
       xo[h][i] = m0 + r < M ? (int)((int64_t)row * ldx * 2) + chunk * 2 : OUT;
     }
@@ -379,7 +385,7 @@ __global__ __launch_bounds__(256, AH * BH == 1 ? 2 : 1) void k_gemm_dma(const u1
     }
   }
   const u32 lds0 = __builtin_amdgcn_readfirstlane((u32)(uintptr_t)(__attribute__((address_space(3))) u16*)gsm);
-  auto request = [&](const u16* base, int voff, int t, u32 lds) {
+  auto request = [&](auto ONCE, const u16* base, int voff, int t, u32 lds) {
     const bool in = t < nk;
     i32x4_t r;
     r.x = (int)(u32)(unsigned long long)base;
@@ -387,25 +393,25 @@ __global__ __launch_bounds__(256, AH * BH == 1 ? 2 : 1) void k_gemm_dma(const u1
     r.z = in ? 0x7fffffff : 0;
     r.w = 0x00020000;
     if (KTAIL) voff = t * 64 + chunk < klen ? voff : OUT;
-    dma16(r, voff, in ? t * 128 : 0, lds);
+    dma16<decltype(ONCE)::value>(r, voff, in ? t * 128 : 0, lds);
   };
-  auto dma_a = [&](int t, int par, int h, int i) { request(xb, xo[h][i], t, lds0 + (par * 2 + h) * HA + (wave * NA + i) * 1024); };
-  auto dma_b = [&](int t, int par, int h, int i) { request(wb, wo[h][i], t, lds0 + BOFF + (par * 2 + h) * HB + (wave * NB + i) * 1024); };
+  auto dma_a = [&](int t, int par, int h, int i) { request(std::false_type{}, xb, xo[h][i], t, lds0 + (par * 2 + h) * HA + (wave * NA + i) * 1024); };
+  auto dma_b = [&](int t, int par, int h, int i) { request(std::bool_constant<NT>{}, wb, wo[h][i], t, lds0 + BOFF + (par * 2 + h) * HB + (wave * NB + i) * 1024); };
 
-  f32x4_t acc[4 * AH][4 * BH];
+  f32x4_t acc[2 * A16][4 * BH];
 #pragma unroll
-  for (int a = 0; a < 4 * AH; ++a)
+  for (int a = 0; a < 2 * A16; ++a)
 #pragma unroll
     for (int b = 0; b < 4 * BH; ++b)
 #pragma unroll
       for (int v = 0; v < 4; ++v) acc[a][b][v] = 0.0f;
-  bf16x8_t af[2][2 * AH][2], bf[2][2 * BH][2];
+  bf16x8_t af[2][A16][2], bf[2][2 * BH][2];
   const char* const smb = reinterpret_cast<const char*>(gsm);
   int fa[2], fb[2];
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
     const int c = ((4 * ks + (lane >> 4)) ^ (lane & 7)) * 16;
-    fa[ks] = (wm * 32 * AH + (lane & 15)) * 128 + c;
+    fa[ks] = (wm * 16 * A16 + (lane & 15)) * 128 + c;
     fb[ks] = (wn * 32 * BH + (lane & 15)) * 128 + c + BOFF;
   }
   auto read_a = [&](int par, int h, int t, int ks) {
@@ -435,7 +441,7 @@ __global__ __launch_bounds__(256, AH * BH == 1 ? 2 : 1) void k_gemm_dma(const u1
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-    for (int t = 0; t < 2 * AH; ++t) read_a(0, 0, t, ks);
+    for (int t = 0; t < A16; ++t) read_a(0, 0, t, ks);
 #pragma unroll
     for (int t = 0; t < 2 * BH; ++t) read_b(0, 0, 0, t, ks);
   }
@@ -452,19 +458,19 @@ __global__ __launch_bounds__(256, AH * BH == 1 ? 2 : 1) void k_gemm_dma(const u1
     // requests younger than the slot read here: those of the six phases since
     wait_requests_and_lds<(P == 0 ? 4 * NA + 2 * NB : P == 2 ? 2 * NA + 4 * NB : 3 * NA + 3 * NB)>();
     barrier();
-    constexpr int J = 8 * AH * BH, RD = (P == 1 || P == 2) ? 4 * AH : 4 * BH, RQ = (P == 2 || P == 3) ? NA : NB;
+    constexpr int J = 4 * A16 * BH, RD = (P == 1 || P == 2) ? 2 * A16 : 4 * BH, RQ = (P == 2 || P == 3) ? NA : NB;
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-      const int tb = j % (2 * BH), ta = j / (2 * BH) % (2 * AH), ks = j / (4 * AH * BH);
+      const int tb = j % (2 * BH), ta = j / (2 * BH) % (A16), ks = j / (2 * A16 * BH);
       asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
-                   : "+a"(acc[ah * 2 * AH + ta][bh * 2 * BH + tb])
+                   : "+a"(acc[ah * A16 + ta][bh * 2 * BH + tb])
                    : "v"(bf[set][tb][ks]), "v"(af[ah][ta][ks]));
       if (j < J / 2) {
 #pragma unroll
         for (int e = j * RD / (J / 2); e < (j + 1) * RD / (J / 2); ++e) {
           if (P == 0) read_b(1 ^ PAR, PAR, 1, e % (2 * BH), e / (2 * BH));
-          if (P == 1) read_a(PAR, 1, e % (2 * AH), e / (2 * AH));
-          if (P == 2) read_a(PAR ^ 1, 0, e % (2 * AH), e / (2 * AH));
+          if (P == 1) read_a(PAR, 1, e % (A16), e / (A16));
+          if (P == 2) read_a(PAR ^ 1, 0, e % (A16), e / (A16));
           if (P == 3) read_b(1 ^ PAR, PAR ^ 1, 0, e % (2 * BH), e / (2 * BH));
         }
       } else {
@@ -500,9 +506,9 @@ __global__ __launch_bounds__(256, AH * BH == 1 ? 2 : 1) void k_gemm_dma(const u1
   asm volatile("s_nop 15\n\ts_nop 15\n\ts_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   if constexpr (!GROUP) {
     if (piece >= 0) {
-      float* p = sp.part + (int64_t)piece * (T::TM * T::TN) + (int64_t)wave * (16 * AH * BH * 256) + lane * 4;
+      float* p = sp.part + (int64_t)piece * (T::TM * T::TN) + (int64_t)wave * (8 * A16 * BH * 256) + lane * 4;
 #pragma unroll
-      for (int a = 0; a < 4 * AH; ++a) {
+      for (int a = 0; a < 2 * A16; ++a) {
 #pragma unroll
         for (int b = 0; b < 4 * BH; ++b) *reinterpret_cast<f32x4_t*>(p + (a * 4 * BH + b) * 256) = acc[a][b];
         __builtin_amdgcn_sched_barrier(0);
@@ -510,23 +516,23 @@ __global__ __launch_bounds__(256, AH * BH == 1 ? 2 : 1) void k_gemm_dma(const u1
       return;
     }
   }
-  gemm_store<AH, BH, MODE, 4 * AH>(acc, gsm + wave * (T::EBYTES / 8), 0, wm, wn, m0, n0, y, ldy, M, N, rp, GROUP ? entry : nullptr);
+  gemm_store<A16, BH, MODE, 2 * A16>(acc, gsm + wave * (T::EBYTES / 8), 0, wm, wn, m0, n0, y, ldy, M, N, rp, GROUP ? entry : nullptr);
 }
 
-// The cut tiles: a workgroup adds the pieces of a 1 / (4 AH) part of one (16 rows per wave, four pieces' loads in flight
+// The cut tiles: a workgroup adds the pieces of a 1 / (2 A16) part of one (16 rows per wave, four pieces' loads in flight
 // together, summed in order) and finishes it.  Bound: memory, mostly the last-level cache: the pieces were just written.
-template <int AH, int BH, int MODE>
+template <int A16, int BH, int MODE>
 __global__ __launch_bounds__(256) void k_gemm_sum(u16* __restrict__ y, int64_t ldy, int M, int N, int tm, int tn, const GemmRope rp, const GemmSplit sp) {
-  using T = GemmTile<AH, BH>;
+  using T = GemmTile<A16, BH>;
   __shared__ __attribute__((aligned(16))) u16 sm[4 * 16 * T::EPITCH];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int rt = blockIdx.x / (4 * AH), g0 = blockIdx.x - rt * 4 * AH;
+  const int rt = blockIdx.x / (2 * A16), g0 = blockIdx.x - rt * 2 * A16;
   int mt, nt;
   gemm_tile_at(sp.full + rt, tm, tn, mt, nt);
   const int m0 = mt * T::TM, n0 = nt * (MODE == GEMM_PAIR ? T::TN / 2 : T::TN);
-  if (m0 + (g0 / (2 * AH)) * 64 * AH + (g0 % (2 * AH)) * 16 >= M) return;   // (its lowest row; no barrier follows)
+  if (m0 + (g0 / (A16)) * 32 * A16 + (g0 % (A16)) * 16 >= M) return;   // (its lowest row; no barrier follows)
   constexpr int C = 4 * BH, STEP = T::TM * T::TN;
-  const float* p = sp.part + (int64_t)rt * sp.splits * STEP + ((int64_t)wave * 4 * AH + g0) * (C * 256) + lane * 4;
+  const float* p = sp.part + (int64_t)rt * sp.splits * STEP + ((int64_t)wave * 2 * A16 + g0) * (C * 256) + lane * 4;
   f32x4_t acc[1][C], v[4][C];
 #pragma unroll
   for (int b = 0; b < C; ++b) acc[0][b] = *reinterpret_cast<const f32x4_t*>(p + b * 256);
@@ -543,7 +549,7 @@ __global__ __launch_bounds__(256) void k_gemm_sum(u16* __restrict__ y, int64_t l
         for (int b = 0; b < C; ++b) acc[0][b] += v[i][b];
       }
   }
-  gemm_store<AH, BH, MODE, 1>(acc, sm + wave * (16 * T::EPITCH), g0, wave >> 1, wave & 1, m0, n0, y, ldy, M, N, rp, nullptr);
+  gemm_store<A16, BH, MODE, 1>(acc, sm + wave * (16 * T::EPITCH), g0, wave >> 1, wave & 1, m0, n0, y, ldy, M, N, rp, nullptr);
 }
 
 // ---- which tile, and which tiles are cut along K
@@ -559,78 +565,93 @@ struct GemmPlan {
 //   128 rows, 16384 x  2048   23 (128 pair tiles of 128 x 128 in 2)       48 /  35 /  26
 //  2048 rows,  4096 x 14336  184 (128 tiles of 256 x 256 in 2 pieces)    242 / 199 / 239
 //  3002 rows, 28672 x  4096  564 (1280 tiles whole, 64 in 3 pieces)      586 / 635 / 660
+//    64 rows,  1280 x  8192   15 (10 tiles of 64 x 128 in 12 pieces)       -  /  -  / 100   (the bands of stream_band.h 24)
+//    64 rows, 28672 x  4096   47 (224 pair tiles of 64 x 128)              -  /  65 /  52   (bands 76)
 // A workgroup's time is nk * (ktile + busy * slope) + fixed, `busy` the workgroups per CU: the more CUs are at work, the
 // lower the clock and the more of them ask the L2s (256 x 256: 1.05 us per k-tile on a quarter of the chip, 1.41 on all of
-// it).  Two 128 x 128 tiles on one CU take twice the time of one.  Pieces cost a launch and their trip through memory.
+// it); `cold` in place of the slope where a single row tile reads every weight from HBM itself; `pair` where two share a CU.
+// The weights need their time on the way from HBM whatever the tiles.  Pieces cost a launch and their trip through memory.
 struct GemmTileCost {
-  int ah, bh, per_cu;
-  float ktile, slope, fixed;
+  int a16, bh, per_cu;
+  float ktile, slope, cold, pair, fixed;
 };
-constexpr GemmTileCost GEMM_TILES[3] = {{2, 2, 1, 0.95f, 0.46f, 5.0f}, {1, 2, 1, 0.58f, 0.29f, 3.0f}, {1, 1, 2, 0.44f, 0.06f, 3.0f}};
+constexpr GemmTileCost GEMM_TILES[4] = {{4, 2, 1, 0.95f, 0.46f, 1.4f, 0.0f, 5.0f},
+                                         {2, 2, 1, 0.58f, 0.29f, 1.6f, 0.0f, 3.0f},
+                                         {2, 1, 2, 0.44f, 0.06f, 0.5f, 0.92f, 3.0f},
+                                         {1, 1, 2, 0.27f, 0.26f, 0.4f, 0.72f, 2.5f}};
 constexpr size_t GEMM_SCRATCH = (size_t)64 << 20;   // pieces of one round of the largest tiles
+constexpr int GEMM_SCRATCH_FROM = 33;               // rows from which a projection that has memory for pieces is one of this file's
 
 static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
   int cus = lr_num_cus();
   if (cus <= 0) cus = 256;
   const int nk = (K + 63) / 64;
+  const float weights_us = (float)N * (mode == GEMM_PAIR ? 2 : 1) * K * 2 / 5.5e6f;
   GemmPlan best{-1, 0, 0, 1};
   float best_us = 0;
-  for (int c = 0; c < 3; ++c) {
+  for (int c = 0; c < 4; ++c) {
     const GemmTileCost& t = GEMM_TILES[c];
-    const int TM = 128 * t.ah, TN = (mode == GEMM_PAIR ? 64 : 128) * t.bh, slots = cus * t.per_cu;
+    const int TM = 64 * t.a16, TN = (mode == GEMM_PAIR ? 64 : 128) * t.bh, slots = cus * t.per_cu;
     const int64_t tiles = (int64_t)((M + TM - 1) / TM) * ((N + TN - 1) / TN), rounds = tiles / slots;
     if (tiles > 0x3fffffff) continue;
     const int left = (int)(tiles - rounds * slots);
     auto round_us = [&](int workgroups, int k) {
       const float busy = (float)workgroups / cus;
-      return k * (busy > 1.0f ? 2 * (t.ktile + t.slope) : t.ktile + busy * t.slope) + t.fixed;
+      return k * (busy > 1.0f ? t.pair : t.ktile + busy * (M <= TM ? t.cold : t.slope));
     };
-    auto consider = [&](float us, const GemmPlan& p) {
+    auto consider = [&](float us, float more, const GemmPlan& p) {
+      us = (us > weights_us ? us : weights_us) + more;
       if (best.tile < 0 || us < best_us) {
         best = p;
         best_us = us;
       }
     };
-    const float whole = rounds * round_us(slots, nk);
-    consider(whole + (left ? round_us(left, nk) : 0.0f), GemmPlan{c, (int)tiles, 0, 1});
+    const float whole = rounds * round_us(slots, nk), fixed = (rounds + (left ? 1 : 0)) * t.fixed;
+    consider(whole + (left ? round_us(left, nk) : 0.0f), fixed, GemmPlan{c, (int)tiles, 0, 1});
     for (int s = 2; left && s <= 16 && 4 * s <= nk && left * s <= slots; ++s) {
-      const size_t bytes = (size_t)left * s * (128 * t.ah) * (128 * t.bh) * sizeof(float);
+      const size_t bytes = (size_t)left * s * (64 * t.a16) * (128 * t.bh) * sizeof(float);
       if (bytes > scratch) break;
-      consider(whole + round_us(left * s, (nk + s - 1) / s) + 4.5f + bytes / 6.5e6f, GemmPlan{c, (int)tiles - left, left, s});
+      consider(whole + round_us(left * s, (nk + s - 1) / s), fixed + 6.0f + bytes / 6.5e6f, GemmPlan{c, (int)tiles - left, left, s});
     }
   }
   return best;
 }
 
-template <int AH, int BH, bool KTAIL, int MODE>
+template <int A16, int BH, bool KTAIL, int MODE, bool NT = false>
 static int gemm_run_as(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, const GemmRope& rp,
                        const GemmPlan& p, void* scratch, hipStream_t s) {
-  using T = GemmTile<AH, BH>;
+  using T = GemmTile<A16, BH>;
   static std::atomic<unsigned long long> raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_dma<AH, BH, KTAIL, MODE, false>), T::LDS, raised)) return LR_E_LAUNCH;
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_dma<A16, BH, KTAIL, MODE, false, NT>), T::LDS, raised)) return LR_E_LAUNCH;
   const int gn = MODE == GEMM_PAIR ? T::TN / 2 : T::TN, tm = (M + T::TM - 1) / T::TM, tn = (N + gn - 1) / gn;
   const GemmSplit sp{(float*)scratch, p.full, p.rem, p.splits};
-  k_gemm_dma<AH, BH, KTAIL, MODE, false><<<dim3((unsigned)(p.full + p.rem * p.splits)), dim3(256), T::LDS, s>>>(
+  k_gemm_dma<A16, BH, KTAIL, MODE, false, NT><<<dim3((unsigned)(p.full + p.rem * p.splits)), dim3(256), T::LDS, s>>>(
       (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, M, N, K, tm, tn, rp, sp, GemmGroup{});
-  if (p.rem) k_gemm_sum<AH, BH, MODE><<<dim3((unsigned)(p.rem * 4 * AH)), dim3(256), 0, s>>>((u16*)y, ldy, M, N, tm, tn, rp, sp);
+  if (p.rem) k_gemm_sum<A16, BH, MODE><<<dim3((unsigned)(p.rem * 2 * A16)), dim3(256), 0, s>>>((u16*)y, ldy, M, N, tm, tn, rp, sp);
   return lr_launch_status();
 }
-template <int AH, int BH, bool KTAIL>
+template <int A16, int BH, bool KTAIL, bool NT = false>
 static int gemm_run_mode(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, int mode, const GemmRope& rp,
                          const GemmPlan& p, void* scratch, hipStream_t s) {
-  if (mode == GEMM_PAIR) return gemm_run_as<AH, BH, KTAIL, GEMM_PAIR>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
-  if (mode == GEMM_ROPE) return gemm_run_as<AH, BH, KTAIL, GEMM_ROPE>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
-  return gemm_run_as<AH, BH, KTAIL, GEMM_PLAIN>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+  if (mode == GEMM_PAIR) return gemm_run_as<A16, BH, KTAIL, GEMM_PAIR, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+  if (mode == GEMM_ROPE) return gemm_run_as<A16, BH, KTAIL, GEMM_ROPE, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+  return gemm_run_as<A16, BH, KTAIL, GEMM_PLAIN, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
 }
 static int gemm_run(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, int mode, const GemmRope& rp,
                     const GemmPlan& p, void* scratch, hipStream_t s) {
   const bool kt = K % 64 != 0;
   if (p.tile == 0)
+    return kt ? gemm_run_mode<4, 2, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
+              : gemm_run_mode<4, 2, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+  if (p.tile == 1)
     return kt ? gemm_run_mode<2, 2, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
               : gemm_run_mode<2, 2, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
-  if (p.tile == 1)
-    return kt ? gemm_run_mode<1, 2, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
-              : gemm_run_mode<1, 2, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+  if (p.tile == 2)
+    return kt ? gemm_run_mode<2, 1, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
+              : gemm_run_mode<2, 1, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+  if (M <= 64)   // every weight is used once: non-temporal (28672 x 4096 at 64 rows 50.0 -> 46.7 us, 16032 x 8192 61.9 -> 57.5)
+    return kt ? gemm_run_mode<1, 1, true, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
+              : gemm_run_mode<1, 1, false, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
   return kt ? gemm_run_mode<1, 1, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
             : gemm_run_mode<1, 1, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
 }
@@ -649,15 +670,15 @@ static int gemm(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy,
 // Grouped products (lr_moe): rows of several matrices' tiles, see GemmGroup; pair_off != 0: GEMM_PAIR (N counts pairs).
 // tile_rows: 128 or 256, the height the tile table was made for.
 namespace lr_detail {
-template <int AH, int BH, bool KTAIL, int MODE>
+template <int A16, int BH, bool KTAIL, int MODE>
 static int gemm_grouped_as(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int N, int K, const GemmGroup& gp, int max_tiles,
                            hipStream_t s) {
-  using T = GemmTile<AH, BH>;
+  using T = GemmTile<A16, BH>;
   constexpr size_t lds = T::LDS + T::TM * sizeof(int32_t);
   static std::atomic<unsigned long long> raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_dma<AH, BH, KTAIL, MODE, true>), lds, raised)) return LR_E_LAUNCH;
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_dma<A16, BH, KTAIL, MODE, true>), lds, raised)) return LR_E_LAUNCH;
   const int gn = MODE == GEMM_PAIR ? T::TN / 2 : T::TN, tn = (N + gn - 1) / gn;
-  k_gemm_dma<AH, BH, KTAIL, MODE, true><<<dim3((unsigned)(max_tiles * tn)), dim3(256), lds, s>>>(
+  k_gemm_dma<A16, BH, KTAIL, MODE, true><<<dim3((unsigned)(max_tiles * tn)), dim3(256), lds, s>>>(
       (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, T::TM, N, K, max_tiles, tn, GemmRope{}, GemmSplit{}, gp);
   return lr_launch_status();
 }
@@ -668,16 +689,16 @@ int gemm_grouped(const void* x, int64_t ldx, int64_t xrows, const void* w, void*
   const bool kt = K % 64 != 0;
   if (tile_rows == 128) {
     if (pair_off)
-      return kt ? gemm_grouped_as<1, 1, true, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
-                : gemm_grouped_as<1, 1, false, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
-    return kt ? gemm_grouped_as<1, 1, true, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
-              : gemm_grouped_as<1, 1, false, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
+      return kt ? gemm_grouped_as<2, 1, true, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
+                : gemm_grouped_as<2, 1, false, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
+    return kt ? gemm_grouped_as<2, 1, true, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
+              : gemm_grouped_as<2, 1, false, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
   }
   if (pair_off)
-    return kt ? gemm_grouped_as<2, 2, true, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
-              : gemm_grouped_as<2, 2, false, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
-  return kt ? gemm_grouped_as<2, 2, true, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
-            : gemm_grouped_as<2, 2, false, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
+    return kt ? gemm_grouped_as<4, 2, true, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
+              : gemm_grouped_as<4, 2, false, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
+  return kt ? gemm_grouped_as<4, 2, true, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
+            : gemm_grouped_as<4, 2, false, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
 }
 }  // namespace lr_detail
 
@@ -691,7 +712,7 @@ static int linear_rows(const void* x, int64_t ldx, const void* w, void* y, int64
   if (K % 8 || ldx % 8) return LR_E_ALIGN;
   if (M <= 4 || ((act_swiglu || gemv_cfg) && M <= 8))
     return lr_gemv_dispatch(x, ldx, w, y, ldy, M, N, K, act_swiglu, gemv_cfg, s);
-  if (!act_swiglu && M <= 64) {
+  if (!act_swiglu && M <= 64 && !(M >= GEMM_SCRATCH_FROM && scratch)) {
     // decode batches: the weight-streaming matrix-core kernel (stream_gemm.hip); shapes it declines fall through
     lr_projection_t pr;
     pr.x = x; pr.ldx = ldx; pr.w = w; pr.y = y; pr.ldy = ldy; pr.N = N; pr.K = K; pr.epilogue = LR_EPI_NONE; pr.rope = nullptr;
@@ -721,7 +742,7 @@ extern "C" int lr_linear(const void* x, int64_t ldx, const void* w, void* y, int
   return linear_rows(x, ldx, w, y, ldy, M, N, K, act_swiglu, 0, nullptr, 0, (hipStream_t)stream);
 }
 
-extern "C" size_t lr_linear_scratch_bytes(int M) { return M > 64 ? GEMM_SCRATCH : 0; }
+extern "C" size_t lr_linear_scratch_bytes(int M) { return M >= GEMM_SCRATCH_FROM ? GEMM_SCRATCH : 0; }
 
 extern "C" int lr_linear_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, void* scratch,
                                  size_t scratch_bytes, lr_stream_t stream) {
@@ -730,8 +751,8 @@ extern "C" int lr_linear_scratch(const void* x, int64_t ldx, const void* w, void
 }
 
 // The fused q/k/v projection of M = B * S rows (S tokens per sequence, row b * S + s at position pos[s]) finished as
-// lr_rope_kv_write would finish it, in the GEMM's output pass; up to 64 rows (and rows out of the requests' reach) in the
-// two calls.
+// lr_rope_kv_write would finish it, in the GEMM's output pass; decode batches without scratch (and rows out of the requests'
+// reach) in the two calls.
 extern "C" int lr_linear_rope_kv_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int K, int S,
                                          const lr_rope_kv_t* rope, void* scratch, size_t scratch_bytes, lr_stream_t stream) {
   LR_REQUIRE_PTR(x);
@@ -750,7 +771,7 @@ extern "C" int lr_linear_rope_kv_scratch(const void* x, int64_t ldx, const void*
   if (K % 8 || ldx % 8 || ldy % 8 || rope->head_dim % 8) return LR_E_ALIGN;
   const int N = (int)n64;
   hipStream_t s = (hipStream_t)stream;
-  if (M > 64) {
+  if (M > 64 || (M >= GEMM_SCRATCH_FROM && scratch)) {
     const GemmRope rp{(const u16*)rope->table, rope->pos, (u16*)rope->k_cache, (u16*)rope->v_cache, rope->err, S, rope->n_head,
                       rope->n_kv_head, rope->head_dim, rope->smax, rope->block_size};
     const int rc = gemm(x, ldx, w, y, ldy, M, N, K, GEMM_ROPE, rp, scratch, scratch_bytes, s);
@@ -778,7 +799,7 @@ extern "C" int lr_linear_swiglu_out_scratch(const void* x, int64_t ldx, const vo
   if (M <= 0 || N <= 0 || K <= 0 || N % 2 || ldx < K || ldy < N / 2) return LR_E_SHAPE;
   if (K % 8 || ldx % 8) return LR_E_ALIGN;
   const int I = N / 2;
-  if (M <= 64) {
+  if (M <= 64 && !(M >= GEMM_SCRATCH_FROM && sums)) {
     lr_projection_t pr;
     pr.x = x; pr.ldx = ldx; pr.w = w; pr.y = y; pr.ldy = ldy; pr.N = N; pr.K = K; pr.epilogue = LR_EPI_SWIGLU; pr.rope = nullptr;
     const int rc = lr_linear_multi(&pr, 1, M, stream);
@@ -786,12 +807,12 @@ extern "C" int lr_linear_swiglu_out_scratch(const void* x, int64_t ldx, const vo
   }
   // (a caller of other than large problems brings `scratch` [M, N]; used where the weights are out of the requests' reach)
   const bool large = M >= 512 && I >= 128 && (int64_t)((M + 255) / 256) * ((I + 127) / 128) >= 192 && gemm_reaches(ldx, I, K, GEMM_PAIR);
-  if (!large) {
+  if (!large && !(M <= 64 && sums)) {
     LR_REQUIRE_PTR(scratch);
     if (scratch_bytes < (size_t)M * N * sizeof(u16)) return LR_E_SHAPE;
   }
   int rc = gemm(x, ldx, w, y, ldy, M, I, K, GEMM_PAIR, GemmRope{}, sums, sums_bytes, (hipStream_t)stream);
-  if (rc != LR_E_UNSUPPORTED) return rc;
+  if (rc != LR_E_UNSUPPORTED || scratch == nullptr || scratch_bytes < (size_t)M * N * sizeof(u16)) return rc;
   rc = linear_rows(x, ldx, w, scratch, N, M, N, K, 0, 0, nullptr, 0, (hipStream_t)stream);
   if (rc != LR_OK) return rc;
   return lr_detail::swiglu_rows(scratch, N, y, ldy, M, I, stream);

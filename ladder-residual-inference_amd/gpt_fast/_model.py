@@ -45,9 +45,13 @@ class Workspace:
         self.next_token = torch.empty(B, 1, dtype=torch.int32, device=device)
         self.next_token_valid_for = None   # set by a fused decode step that already chose the token
         self.scratch = None
-        # partial sums of the prefill GEMM (only for prompts: a decode step's chains may run on two streams)
-        n = _hip.linear_scratch_bytes(rows) if S > 1 else 0
-        self.sums = torch.empty(n, dtype=torch.uint8, device=device) if n else None
+        # partial sums of products; the MLP's may run beside the attention's in a decode step
+        n = _hip.linear_scratch_bytes(rows)
+        self.sums = self.sums_mlp = torch.empty(n, dtype=torch.uint8, device=device) if n else None
+        if n and S == 1:
+            # (room for the pieces of three quarters of the compute units, 32 KiB each: the attention's products keep the
+            # rest -- 70B rank shard, batch 64: 7.6 ms per step, 8.2 with as many pieces as pay for a product alone)
+            self.sums_mlp = torch.empty(min(n, 200 << 15), dtype=torch.uint8, device=device)
         if S == 1:
             n = _hip.attn_decode_scratch_bytes(B, cfg.n_head_local, hd, smax) // 4
             self.scratch = torch.empty(n, dtype=torch.float32, device=device)
@@ -198,14 +202,17 @@ class GPTBase(nn.Module):
     # is the faster one -- dense family on the 70B rank shard, ms per step at batch 1 / 4: 5.7 / 8.5 without bands,
     # 6.1 / 6.2 with)
     band_rows_from = 2
+    # and up to which: above, the GEMM with its partial sums is the faster one (64 rows of the 70B rank shard, us: up/gate
+    # 38.9 in bands / 30.7, q/k/v 23.6 / 14.8, w2 23.0 / 18.6, wo 13.9 / 10.7)
+    band_rows_to = 32
 
     def _decode_bands(self, ws: Workspace, *linears) -> bool:
-        """A decode step of up to 64 rows on bf16 weights: every projection of a block is a launch of the
+        """A decode step of up to 32 rows on bf16 weights: every projection of a block is a launch of the
         weight-streaming kernel (lr_linear_multi), the q/k/v one rotating and caching on its way out and the up/gate one
         storing silu(gate) * up -- also below 5 rows, where lr_linear alone would pick the matrix-vector kernel: fewer
         launches per block weigh more than the kernel.  (`linears`: the modules
         in question; weight-only quantised ones have kernels of their own.)"""
-        return ws.S == 1 and self.band_rows_from <= ws.B <= 64 and not any(hasattr(m, "scales") for m in linears)
+        return ws.S == 1 and self.band_rows_from <= ws.B <= self.band_rows_to and not any(hasattr(m, "scales") for m in linears)
 
     def _attention(self, ws: Workspace, blk, pos: Tensor, wqkv: nn.Module, out: Tensor, roped: bool = False):
         """ws.xn -> fused projection -> RoPE + cache write -> attention -> wo -> out (partial sum).
@@ -219,9 +226,9 @@ class GPTBase(nn.Module):
         if wqkv is not None and bands and not roped:
             _hip.linear_multi((ws.xn, wqkv.weight, ws.qkv, _hip.rope_kv_epilogue(self.freqs_cis, pos, kc, vc, Hq, Hkv, hd)))
             roped = True
-        elif (wqkv is not None and S > 1 and not roped and not hasattr(wqkv, "scales")
+        elif (wqkv is not None and (S > 1 or ws.sums is not None) and not roped and not hasattr(wqkv, "scales")
               and wqkv.weight.shape[0] == (Hq + 2 * Hkv) * hd):   # (not the parallel family's wider projection)
-            # prefill: the projection rotates q and caches rotated k and v on its way out (one launch of the GEMM)
+            # prefill, large decode batches: the projection rotates q and caches rotated k and v on its way out (one launch of the GEMM)
             _hip.linear_rope_kv(ws.xn, wqkv.weight, ws.qkv, self.freqs_cis, pos, kc, vc, B, S, Hq, Hkv, hd, ws.sums)
             roped = True
         elif wqkv is not None:
@@ -248,8 +255,8 @@ class GPTBase(nn.Module):
             return
         if xin.shape[0] > 4 and not hasattr(ff.w1, "scales"):
             # the activation in the first projection's epilogue; up to 4 rows it is fused into w2's GEMV instead
-            _hip.linear_swiglu_out(xin, ff.w1.weight, ws.act, ws.h, ws.sums)
-            _hip.module_linear(ws.act, ff.w2, out, ws.sums)
+            _hip.linear_swiglu_out(xin, ff.w1.weight, ws.act, ws.h, ws.sums_mlp)
+            _hip.module_linear(ws.act, ff.w2, out, ws.sums_mlp)
             return
         _hip.module_linear(xin, ff.w1, ws.h)
         _hip.module_linear_swiglu(ws.h, ff.w2, out, ws.act)

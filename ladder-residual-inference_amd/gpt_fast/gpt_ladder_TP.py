@@ -148,10 +148,10 @@ class GPTLadder(GPTBase):
         fp8 = hasattr(self.layers[0].attention.wqkv, "scales")
         multi = side is None and ws.B <= 64 and not fp8
         beside = multi and ws.B <= 16
-        # Above 32 rows a band workgroup fills the register file of its waves but not the CU: the MLP chain (up/gate,
+        # Above 32 rows the projections are products with partial sums, whose launches leave room: the MLP chain (up/gate,
         # w2) runs as a second branch of the captured graph beside the attention chain (q/k/v, attention, wo) --
-        # 70B rank shard, batch 64: 10.4 -> 9.9 ms per step; at batch 32 nothing moves (7.35 / 7.31), below that
-        # the attention shares the up/gate launch instead
+        # 70B rank shard, batch 64: 7.6 ms per step, one after the other 10.0 (in bands 9.45 and 9.96); at batch 32 nothing
+        # moves (7.35 / 7.31, in bands), below that the attention shares the up/gate launch instead
         two_chains = multi and not beside and ws.B >= self.two_chains_from
         if two_chains:
             cur = torch.cuda.current_stream()
@@ -181,11 +181,8 @@ class GPTLadder(GPTBase):
                 elif two_chains:
                     chain.wait_stream(cur)
                     with torch.cuda.stream(chain):
-                        _hip.linear_multi(up_gate)
-                        _hip.linear_multi((ws.act, blk.feed_forward.w2.weight, ws.m, _hip.EPI_NONE))
-                    _hip.linear_multi((ws.xn, blk.attention.wqkv.weight, ws.qkv, rope))
-                    self._attention(ws, blk, pos, None, None, roped=True)
-                    _hip.linear_multi((ws.y, blk.attention.wo.weight, ws.a, _hip.EPI_NONE))
+                        self._mlp(ws, blk, ws.m, ws.xn2)
+                    self._attention(ws, blk, pos, blk.attention.wqkv, ws.a)
                     cur.wait_stream(chain)
                     pending_a, pending_m = ws.a, ws.m
                     continue

@@ -48,7 +48,7 @@ class GPTParallel(GPTBase):
         cfg = self.config
         nqkv = (cfg.n_head_local + 2 * cfg.n_kv_local) * cfg.head_dim
         att0 = self.layers[0].attention
-        if self._decode_bands(ws, att0.wqkv1, att0.wo, att0.w2):
+        if ws.S == 1 and ws.B <= 64 and not any(hasattr(m, "scales") for m in (att0.wqkv1, att0.wo, att0.w2)):
             return self._run_layers_decode(ws, pos, nqkv)
         for blk in self.layers:
             att = blk.attention
@@ -67,7 +67,8 @@ class GPTParallel(GPTBase):
         of the same input: [q | k | v], rotated and cached on the way out, and [up | gate], stored as silu(gate) * up
         -- the second independent of the attention, so up to 16 sequences its bands share the attention's launch
         (lr_attn_decode_beside) and above that the q/k/v launch; wo and w2 share a launch; y + x is left to the next
-        block's norm launch (x + y: the same sum).  Six launches per block instead of nine."""
+        block's norm launch (x + y: the same sum).  Six launches per block instead of nine.  Above 32 sequences each
+        projection is a product of its own, with partial sums."""
         cfg = self.config
         Hq, Hkv, hd = cfg.n_head_local, cfg.n_kv_local, cfg.head_dim
         q = ws.qkv[:, :nqkv]
@@ -79,7 +80,13 @@ class GPTParallel(GPTBase):
             w = att.wqkv1.weight
             qkv = (ws.xn, w[:nqkv], q, _hip.rope_kv_epilogue(self.freqs_cis, pos, kv.k_cache, kv.v_cache, Hq, Hkv, hd))
             up_gate = (ws.xn, w[nqkv:], ws.act, _hip.EPI_SWIGLU)
-            if ws.B <= 16:
+            if ws.B > self.band_rows_to:
+                _hip.linear_rope_kv(ws.xn, w[:nqkv], q, self.freqs_cis, pos, kv.k_cache, kv.v_cache, ws.B, 1, Hq, Hkv, hd, ws.sums)
+                _hip.linear_swiglu_out(ws.xn, w[nqkv:], ws.act, sums=ws.sums)
+                _hip.attn_decode(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd)
+                _hip.linear(ws.y, att.wo.weight, ws.a, scratch=ws.sums)
+                _hip.linear(ws.act, att.w2.weight, ws.m, scratch=ws.sums)
+            elif ws.B <= 16:
                 _hip.linear_multi(qkv)
                 if not _hip.attn_decode_beside(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd, up_gate):
                     _hip.linear_multi(up_gate)
@@ -87,7 +94,8 @@ class GPTParallel(GPTBase):
             else:
                 _hip.linear_multi(qkv, up_gate)
                 _hip.attn_decode(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd)
-            _hip.linear_multi((ws.y, att.wo.weight, ws.a, _hip.EPI_NONE), (ws.act, att.w2.weight, ws.m, _hip.EPI_NONE))
+            if ws.B <= self.band_rows_to:
+                _hip.linear_multi((ws.y, att.wo.weight, ws.a, _hip.EPI_NONE), (ws.act, att.w2.weight, ws.m, _hip.EPI_NONE))
             _hip.add(ws.m, ws.a, ws.m)                               # w2(...) + wo(...)
             if blk.keeps_residual:
                 pending = ws.m                                       # y + x: with the next norm

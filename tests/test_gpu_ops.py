@@ -826,6 +826,7 @@ def test_stream_read_runs_and_leaves_the_sink_alone(hip):
 # ------------------------------------------------------------------------------------ the prefill GEMM's tiles and pieces
 
 @pytest.mark.parametrize("M,N,K", [
+    (33, 264, 520), (64, 1280, 8192), (40, 24, 64),      # decode batches: with memory for sums 64-row tiles
     (65, 8, 8), (100, 72, 64), (129, 264, 520), (256, 256, 128), (257, 512, 192), (300, 520, 200), (513, 40, 4096),
     (777, 1032, 1000),                                   # one row, column or k too many for every tile; odd numbers of k-tiles
     (128, 1024, 8192), (300, 2048, 4160), (777, 2048, 7168),   # cut along K where there is memory for it: 128 x 128,
@@ -848,7 +849,7 @@ def test_linear_tiles_and_pieces(hip, M, N, K):
     assert torch.equal(outs[1], outs[2])
 
 
-@pytest.mark.parametrize("M,I,K", [(128, 512, 4096), (300, 1000, 4104), (777, 2048, 4096)])
+@pytest.mark.parametrize("M,I,K", [(40, 1000, 2056), (128, 512, 4096), (300, 1000, 4104), (777, 2048, 4096)])
 def test_linear_swiglu_out_pieces(hip, M, I, K):
     """[up; gate] pairs in cut tiles: the activation after the sums are complete."""
     x, w1 = rnd(M, K, seed=92), rnd(2 * I, K, seed=93, scale=K ** -0.5)
@@ -861,7 +862,7 @@ def test_linear_swiglu_out_pieces(hip, M, I, K):
     assert (ulp_diff(act, want) > 0).float().mean().item() < 0.05
 
 
-@pytest.mark.parametrize("B,S,Hq,Hkv,hd,K", [(1, 128, 8, 2, 64, 4096), (3, 100, 4, 1, 128, 4104), (2, 389, 16, 4, 128, 4096)])
+@pytest.mark.parametrize("B,S,Hq,Hkv,hd,K", [(48, 1, 8, 2, 64, 4096), (1, 128, 8, 2, 64, 4096), (3, 100, 4, 1, 128, 4104), (2, 389, 16, 4, 128, 4096)])
 def test_linear_rope_kv_pieces(hip, B, S, Hq, Hkv, hd, K):
     """The q/k/v projection in cut tiles, rotated and cached after the sums: the two calls on the same plan, bit for bit."""
     N, Smax, start = (Hq + 2 * Hkv) * hd, S + 11, 5
