@@ -250,12 +250,6 @@ __global__ __launch_bounds__(64) void k_attn_prefill(const u16* __restrict__ q, 
 // an assembler statement that reads its result, and the statement then reads the registers too early.)
 __device__ __forceinline__ float max_med3(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, INFINITY); }
 __device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
-// two fp32 -> one dword of two bf16 (round to nearest even): a single v_cvt_pk_bf16_f32
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ u32 cvt_pk_bf2(float lo, float hi) {
-  return __builtin_bit_cast(u32, __builtin_convertvector(f32x2_t{lo, hi}, bf16x2_t));
-}
 constexpr float PREFILL_TAU2 = 8.0f;  // log2 of the largest softmax weight before the reference point moves
 
 struct WindowKeys {
@@ -445,9 +439,9 @@ __global__ __launch_bounds__(256) void k_attn_prefill_mfma(const u16* __restrict
         const float a0 = exp2_hw(fmaf(sacc[8 * h2 + 2 * j], c2, nmc));  // masked -> 0
         const float a1 = exp2_hw(fmaf(sacc[8 * h2 + 2 * j + 1], c2, nmc));
         l += a0 + a1;
-        const u32 hi = cvt_pk_bf2(a0, a1);
+        const u32 hi = pack_bf2(a0, a1);
         phi[h2][j] = hi;
-        plo[h2][j] = cvt_pk_bf2(a0 - __uint_as_float(hi << 16), a1 - __uint_as_float(hi & 0xffff0000u));
+        plo[h2][j] = pack_bf2(a0 - __uint_as_float(hi << 16), a1 - __uint_as_float(hi & 0xffff0000u));
       }
     // ---- O^T += V^T P^T ; k-step h2 covers keys 16 h2 + {0..3, 8..11} + 4 half, in the order of sacc
     const bool rescale = __any(grow);

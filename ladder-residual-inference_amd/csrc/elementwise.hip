@@ -3,6 +3,7 @@
 // position advance.  All of them move 128 bits per lane and round to bf16 exactly where the eager
 // reference materialises a tensor.
 #include "lr_common.h"
+#include <type_traits>
 
 // ------------------------------------------------------------------------------------ embed
 __global__ __launch_bounds__(256) void k_embed(const u16* __restrict__ table, const void* __restrict__ idx,
@@ -63,49 +64,67 @@ extern "C" int lr_add(const void* a, const void* b, float b_div, void* out, int6
 
 // ------------------------------------------------------------------------------------ add + RMSNorm
 // One workgroup per row; the updated residual row stays in registers between the two passes.
-constexpr int NORM_MAXIT = 8;  // 256 threads x 8 elements x 8 iterations = 16384 columns
+constexpr int NORM_MAX_DIM = 16384;
 
-__global__ __launch_bounds__(256) void k_add_rmsnorm(const u16* __restrict__ rin, const u16* __restrict__ d1,
+// the waves' sums, in a fixed order
+template <int W>
+__device__ __forceinline__ float norm_sum(const float* red) {
+  if constexpr (W == 1) return red[0];
+  else return norm_sum<W / 2>(red) + norm_sum<W / 2>(red + W / 2);
+}
+// Lanes per row, the same in both norm kernels and at any number of rows (the order of a sum depends on it).  A decode
+// batch has a CU per row, so its time is one memory round trip and the arithmetic of a lane's columns; a prompt's rows
+// have more loads in flight.  256 lanes against 1024, us, with two values per rounding conversion in both (one at a time
+// before: both norms of 8 x 8192 4.47): both norms of 8 x 8192 3.97 -> 3.43, of 128 x 8192 4.97 -> 4.32, of 1024 x 8192
+// 18.4 -> 16.3; one norm of 128 x 8192 3.56 -> 3.05.  Up to 4096 columns a wider workgroup gives 0.2 us at most and
+// loses at 2048 (2.34 -> 2.48): those rows keep the order of their sums.
+static int norm_lanes(int dim) { return dim <= 4096 ? 256 : 1024; }
+
+template <int T>
+__global__ __launch_bounds__(T) void k_add_rmsnorm(const u16* __restrict__ rin, const u16* __restrict__ d1,
                                                      const u16* __restrict__ d2, const u16* __restrict__ gain,
                                                      u16* rout, u16* __restrict__ nout, int dim, float eps) {
-  __shared__ float red[4];
+  __shared__ float red[T / 64];
+  constexpr int IT = NORM_MAX_DIM / (8 * T), W = T / 64;
   const int tid = threadIdx.x;
   const int64_t base = (int64_t)blockIdx.x * dim;
   // Every load of the row (residual, both addends, gain) is requested before the first one is
   // used: columns past `dim` are clamped to column 0 and ignored, so no branch separates the loads
   // and the kernel costs one memory round trip instead of one per iteration.
-  uint4 qr[NORM_MAXIT], q1[NORM_MAXIT], q2[NORM_MAXIT], qg[NORM_MAXIT];
+  uint4 qr[IT], q1[IT], q2[IT], qg[IT];
 #pragma unroll
-  for (int it = 0; it < NORM_MAXIT; ++it) {
-    const int c0 = (tid + it * 256) * 8;
-    if (it * 256 * 8 >= dim) break;  // uniform
+  for (int it = 0; it < IT; ++it) {
+    const int c0 = (tid + it * T) * 8;
+    if (it * T * 8 >= dim) break;  // uniform
     const int c = c0 < dim ? c0 : 0;
     qr[it] = ld16(rin + base + c);
     q1[it] = d1 ? ld16(d1 + base + c) : make_uint4(0, 0, 0, 0);
     q2[it] = d2 ? ld16(d2 + base + c) : make_uint4(0, 0, 0, 0);
     qg[it] = ld16(gain + c);
   }
-  float r[NORM_MAXIT][8];
+  float r[IT][8];
   float ss = 0.0f;
 #pragma unroll
-  for (int it = 0; it < NORM_MAXIT; ++it) {
-    const int c = (tid + it * 256) * 8;
-    if (it * 256 * 8 >= dim) break;
+  for (int it = 0; it < IT; ++it) {
+    const int c = (tid + it * T) * 8;
+    if (it * T * 8 >= dim) break;
     unpack8(qr[it], r[it]);
     if (d1) {
       float t[8];
       unpack8(q1[it], t);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) r[it][j] = round_bf(r[it][j] + t[j]);
+      for (int j = 0; j < 8; ++j) r[it][j] += t[j];
+      qr[it] = round8(r[it]);
     }
     if (d2) {
       float t[8];
       unpack8(q2[it], t);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) r[it][j] = round_bf(r[it][j] + t[j]);
+      for (int j = 0; j < 8; ++j) r[it][j] += t[j];
+      qr[it] = round8(r[it]);
     }
     if (c < dim) {
-      if (rout) st16(rout + base + c, pack8(r[it]));
+      if (rout) st16(rout + base + c, qr[it]);
 #pragma unroll
       for (int j = 0; j < 8; ++j) ss += r[it][j] * r[it][j];
     }
@@ -113,25 +132,28 @@ __global__ __launch_bounds__(256) void k_add_rmsnorm(const u16* __restrict__ rin
   ss = wave_sum(ss);
   if ((tid & 63) == 0) red[tid >> 6] = ss;
   __syncthreads();
-  ss = (red[0] + red[1]) + (red[2] + red[3]);
+  ss = norm_sum<W>(red);
   const float inv = rsqrtf(ss / (float)dim + eps);
   // (all results first, in registers of their own, then all stores: a store's data registers cannot be reused
   // before the store has completed, and with one set of them the compiler waits for the previous store in front of
   // every conversion)
-  uint4 on[NORM_MAXIT];
+  uint4 on[IT];
 #pragma unroll
-  for (int it = 0; it < NORM_MAXIT; ++it) {
-    if (it * 256 * 8 >= dim) break;
+  for (int it = 0; it < IT; ++it) {
+    if (it * T * 8 >= dim) break;
     float g[8], o[8];
     unpack8(qg[it], g);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = round_bf(r[it][j] * inv) * g[j];
+    for (int j = 0; j < 8; ++j) o[j] = r[it][j] * inv;
+    round8(o);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] *= g[j];
     on[it] = pack8(o);
   }
 #pragma unroll
-  for (int it = 0; it < NORM_MAXIT; ++it) {
-    const int c = (tid + it * 256) * 8;
-    if (it * 256 * 8 >= dim) break;
+  for (int it = 0; it < IT; ++it) {
+    const int c = (tid + it * T) * 8;
+    if (it * T * 8 >= dim) break;
     if (c < dim) st16(nout + base + c, on[it]);
   }
 }
@@ -146,10 +168,14 @@ extern "C" int lr_add_rmsnorm(const void* resid_in, const void* d1, const void* 
   LR_OPTIONAL_PTR(resid_out);
   if (rows <= 0 || dim <= 0) return LR_E_SHAPE;
   if (dim % 8) return LR_E_ALIGN;
-  if (dim > 256 * 8 * NORM_MAXIT) return LR_E_UNSUPPORTED;
-  k_add_rmsnorm<<<dim3(rows), dim3(256), 0, (hipStream_t)stream>>>((const u16*)resid_in, (const u16*)d1,
-                                                                   (const u16*)d2, (const u16*)gain, (u16*)resid_out,
-                                                                   (u16*)normed_out, dim, eps);
+  if (dim > NORM_MAX_DIM) return LR_E_UNSUPPORTED;
+  auto launch = [&](auto T) {
+    constexpr int lanes = decltype(T)::value;
+    k_add_rmsnorm<lanes><<<dim3(rows), dim3(lanes), 0, (hipStream_t)stream>>>(
+        (const u16*)resid_in, (const u16*)d1, (const u16*)d2, (const u16*)gain, (u16*)resid_out, (u16*)normed_out, dim, eps);
+  };
+  if (norm_lanes(dim) == 1024) launch(std::integral_constant<int, 1024>{});
+  else launch(std::integral_constant<int, 256>{});
   return lr_launch_status();
 }
 
@@ -157,18 +183,20 @@ extern "C" int lr_add_rmsnorm(const void* resid_in, const void* d1, const void* 
 // r1 = bf16(r + d1), n1 = norm(r1) * g1;  r2 = bf16(r1 + d2), n2 = norm(r2) * g2;  r <- r2.
 // In the ladder schedule the MLP's input does not contain the attention output of the same block, so
 // both residual updates and both norms of a block can be done before either module runs.
-__global__ __launch_bounds__(256) void k_ladder_norms(const u16* __restrict__ rin, const u16* __restrict__ d1,
+template <int T>
+__global__ __launch_bounds__(T) void k_ladder_norms(const u16* __restrict__ rin, const u16* __restrict__ d1,
                                                       const u16* __restrict__ d2, const u16* __restrict__ g1,
                                                       const u16* __restrict__ g2, u16* rout, u16* __restrict__ n1,
                                                       u16* __restrict__ n2, int dim, float eps) {
-  __shared__ float red[8];
+  __shared__ float red[2 * (T / 64)];
+  constexpr int IT = NORM_MAX_DIM / (8 * T), W = T / 64;
   const int tid = threadIdx.x;
   const int64_t base = (int64_t)blockIdx.x * dim;
-  uint4 qr[NORM_MAXIT], q1[NORM_MAXIT], q2[NORM_MAXIT], qg1[NORM_MAXIT], qg2[NORM_MAXIT];
+  uint4 qr[IT], q1[IT], q2[IT], qg1[IT], qg2[IT];
 #pragma unroll
-  for (int it = 0; it < NORM_MAXIT; ++it) {
-    const int c0 = (tid + it * 256) * 8;
-    if (it * 256 * 8 >= dim) break;  // uniform
+  for (int it = 0; it < IT; ++it) {
+    const int c0 = (tid + it * T) * 8;
+    if (it * T * 8 >= dim) break;  // uniform
     const int c = c0 < dim ? c0 : 0;
     qr[it] = ld16(rin + base + c);
     q1[it] = d1 ? ld16(d1 + base + c) : make_uint4(0, 0, 0, 0);
@@ -178,17 +206,17 @@ __global__ __launch_bounds__(256) void k_ladder_norms(const u16* __restrict__ ri
   }
   float ss1 = 0.0f, ss2 = 0.0f;
 #pragma unroll
-  for (int it = 0; it < NORM_MAXIT; ++it) {
-    const int c = (tid + it * 256) * 8;
-    if (it * 256 * 8 >= dim) break;
+  for (int it = 0; it < IT; ++it) {
+    const int c = (tid + it * T) * 8;
+    if (it * T * 8 >= dim) break;
     float r[8], t[8];
     unpack8(qr[it], r);
     if (d1) {
       unpack8(q1[it], t);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) r[j] = round_bf(r[j] + t[j]);
-    }
-    qr[it] = pack8(r);  // r1, exact in bf16
+      for (int j = 0; j < 8; ++j) r[j] += t[j];
+      qr[it] = round8(r);
+    }  // qr: r1
     if (c < dim) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) ss1 += r[j] * r[j];
@@ -196,9 +224,11 @@ __global__ __launch_bounds__(256) void k_ladder_norms(const u16* __restrict__ ri
     if (d2) {
       unpack8(q2[it], t);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) r[j] = round_bf(r[j] + t[j]);
-    }
-    q2[it] = pack8(r);  // r2
+      for (int j = 0; j < 8; ++j) r[j] += t[j];
+      q2[it] = round8(r);
+    } else {
+      q2[it] = qr[it];
+    }  // q2: r2
     if (c < dim) {
       st16(rout + base + c, q2[it]);
 #pragma unroll
@@ -209,34 +239,40 @@ __global__ __launch_bounds__(256) void k_ladder_norms(const u16* __restrict__ ri
   ss2 = wave_sum(ss2);
   if ((tid & 63) == 0) {
     red[tid >> 6] = ss1;
-    red[4 + (tid >> 6)] = ss2;
+    red[W + (tid >> 6)] = ss2;
   }
   __syncthreads();
-  const float inv1 = rsqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)dim + eps);
-  const float inv2 = rsqrtf(((red[4] + red[5]) + (red[6] + red[7])) / (float)dim + eps);
+  const float inv1 = rsqrtf(norm_sum<W>(red) / (float)dim + eps);
+  const float inv2 = rsqrtf(norm_sum<W>(red + W) / (float)dim + eps);
   // (all results first, in registers of their own, then all stores: a store's data registers cannot be reused
   // before the store has completed, and with one set of them the compiler waits for the previous stores in front of
   // every conversion)
-  uint4 o1[NORM_MAXIT], o2[NORM_MAXIT];
+  uint4 o1[IT], o2[IT];
 #pragma unroll
-  for (int it = 0; it < NORM_MAXIT; ++it) {
-    if (it * 256 * 8 >= dim) break;
+  for (int it = 0; it < IT; ++it) {
+    if (it * T * 8 >= dim) break;
     float r[8], g[8], o[8];
     unpack8(qr[it], r);
     unpack8(qg1[it], g);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = round_bf(r[j] * inv1) * g[j];
+    for (int j = 0; j < 8; ++j) o[j] = r[j] * inv1;
+    round8(o);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] *= g[j];
     o1[it] = pack8(o);
     unpack8(q2[it], r);
     unpack8(qg2[it], g);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = round_bf(r[j] * inv2) * g[j];
+    for (int j = 0; j < 8; ++j) o[j] = r[j] * inv2;
+    round8(o);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] *= g[j];
     o2[it] = pack8(o);
   }
 #pragma unroll
-  for (int it = 0; it < NORM_MAXIT; ++it) {
-    const int c = (tid + it * 256) * 8;
-    if (it * 256 * 8 >= dim) break;
+  for (int it = 0; it < IT; ++it) {
+    const int c = (tid + it * T) * 8;
+    if (it * T * 8 >= dim) break;
     if (c < dim) {
       st16(n1 + base + c, o1[it]);
       st16(n2 + base + c, o2[it]);
@@ -257,10 +293,15 @@ extern "C" int lr_ladder_norms(const void* resid_in, const void* d1, const void*
   LR_OPTIONAL_PTR(d2);
   if (rows <= 0 || dim <= 0) return LR_E_SHAPE;
   if (dim % 8) return LR_E_ALIGN;
-  if (dim > 256 * 8 * NORM_MAXIT) return LR_E_UNSUPPORTED;
-  k_ladder_norms<<<dim3(rows), dim3(256), 0, (hipStream_t)stream>>>(
-      (const u16*)resid_in, (const u16*)d1, (const u16*)d2, (const u16*)gain1, (const u16*)gain2, (u16*)resid_out,
-      (u16*)normed1, (u16*)normed2, dim, eps);
+  if (dim > NORM_MAX_DIM) return LR_E_UNSUPPORTED;
+  auto launch = [&](auto T) {
+    constexpr int lanes = decltype(T)::value;
+    k_ladder_norms<lanes><<<dim3(rows), dim3(lanes), 0, (hipStream_t)stream>>>(
+        (const u16*)resid_in, (const u16*)d1, (const u16*)d2, (const u16*)gain1, (const u16*)gain2, (u16*)resid_out,
+        (u16*)normed1, (u16*)normed2, dim, eps);
+  };
+  if (norm_lanes(dim) == 1024) launch(std::integral_constant<int, 1024>{});
+  else launch(std::integral_constant<int, 256>{});
   return lr_launch_status();
 }
 

@@ -18,7 +18,9 @@ constexpr int LR_FP8_GEMV_MAX_M = 1;
 
 typedef uint16_t u16;
 typedef uint32_t u32;
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
@@ -31,7 +33,10 @@ __device__ __forceinline__ u16 f_to_bf(float f) {
   __bf16 b = (__bf16)f;
   return __builtin_bit_cast(u16, b);
 }
-__device__ __forceinline__ u32 pack_bf2(float lo, float hi) { return (u32)f_to_bf(lo) | ((u32)f_to_bf(hi) << 16); }
+// two fp32 -> one dword of two bf16: a single v_cvt_pk_bf16_f32 (two separate conversions are three instructions)
+__device__ __forceinline__ u32 pack_bf2(float lo, float hi) {
+  return __builtin_bit_cast(u32, __builtin_convertvector(f32x2_t{lo, hi}, bf16x2_t));
+}
 // round an fp32 value to bf16 and back: the value a bf16 tensor would hold
 __device__ __forceinline__ float round_bf(float f) { return bf_to_f(f_to_bf(f)); }
 
@@ -62,6 +67,13 @@ __device__ __forceinline__ void unpack8(const uint4& v, float* f) {
 __device__ __forceinline__ uint4 pack8(const float* f) {
   uint4 v;
   v.x = pack_bf2(f[0], f[1]); v.y = pack_bf2(f[2], f[3]); v.z = pack_bf2(f[4], f[5]); v.w = pack_bf2(f[6], f[7]);
+  return v;
+}
+
+// round_bf of 8 values; the rounded values also packed
+__device__ __forceinline__ uint4 round8(float* f) {
+  const uint4 v = pack8(f);
+  unpack8(v, f);
   return v;
 }
 

@@ -80,6 +80,12 @@ def test_residual_rmsnorm(hip, dtype, rows, dim, width):
 
 
 @pytest.mark.parametrize("dtype", [F32, BF])
+@pytest.mark.parametrize("rows,dim,width", [(256, 4096, 4096), (257, 4096, 4096), (5, 1032, 1025), (2, 4104, 4104)])
+def test_residual_rmsnorm_at_the_edges_of_the_wide_workgroup(hip, dtype, rows, dim, width):
+    test_residual_rmsnorm(hip, dtype, rows, dim, width)
+
+
+@pytest.mark.parametrize("dtype", [F32, BF])
 def test_logit_cap(hip, dtype):
     l = rnd(5, 104, seed=4, dtype=dtype) * 30
     view, before = l[:, :99], l.clone()

@@ -495,6 +495,13 @@ def test_ladder_norms_equals_two_add_rmsnorm_calls(hip, rows, dim, first_block):
     assert_close_ulp(n2, O.rms_norm(r2, g2, 1e-5), max_ulp=2, max_frac=0.05, what="ladder_norms n2")
 
 
+@pytest.mark.parametrize("rows,dim", [(2, 4096), (2, 4104), (257, 8192), (3, 8200), (1, 16376)])
+def test_norms_at_the_edges_of_the_lanes_per_row(hip, rows, dim):
+    """256 lanes up to 4096 columns, 1024 above; the last columns leave most lanes of the last turn idle."""
+    test_add_rmsnorm(hip, rows, dim)
+    test_ladder_norms_equals_two_add_rmsnorm_calls(hip, rows, dim, False)
+
+
 # ------------------------------------------------------------------------------------ weight-only fp8 linear
 
 def test_linear_fp8_decodes_every_e4m3_value_exactly(hip):
