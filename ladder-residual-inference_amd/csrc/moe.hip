@@ -148,7 +148,7 @@ __global__ __launch_bounds__(64 * RW) void k_router(const Router a) {
 
 // One or two projections of a decode batch (the bands of lr_linear_multi) and its routing: the first workgroups route
 template <int MT, bool XL, int ET>
-__global__ __launch_bounds__(NWV * 64) void k_project_route(const Proj p0, const Proj p1, const int M, const Router a) {
+__global__ __launch_bounds__(NWV * 64, MT == 16 ? 2 : 0) void k_project_route(const Proj p0, const Proj p1, const int M, const Router a) {
   extern __shared__ __attribute__((aligned(16))) u16 sg_smem[];
   const int nr = (M + 15) / 16, id = (int)blockIdx.x - nr;
   if (id < 0) {
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(NWV * 64) void k_project_route(const Proj p0, const
   }
   const bool second = id >= p0.nwg;
   const Proj p = second ? p1 : p0;
-  stream_band<MT, 2, false, XL>(p, M, second ? id - p0.nwg : id, sg_smem);
+  stream_band<MT, 2, false, XL, false, false, NWV, 16, MT == 16, MT == 16 && !XL>(p, M, second ? id - p0.nwg : id, sg_smem);
 }
 
 // the shared expert's activations times their gate, four values per thread
@@ -325,7 +325,7 @@ __global__ __launch_bounds__(NWV * 64, 2) void k_expert_band(Proj p, const int64
   p.w += e * wstride;
   for (int i = 0; i < m; i += BAND_ENTRIES) {
     if (i) __syncthreads();
-    stream_band<16, UNITS, false, false, true, false, KW>(p, min(BAND_ENTRIES, m - i), blockIdx.x, sg_smem, list + i, xdiv);
+    stream_band<16, UNITS, false, false, true, false, KW, 16, false>(p, min(BAND_ENTRIES, m - i), blockIdx.x, sg_smem, list + i, xdiv);
   }
 }
 

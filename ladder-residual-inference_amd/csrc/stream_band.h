@@ -17,6 +17,7 @@ constexpr int OOB = (int)0x80000000;  // a buffer offset beyond every resource: 
 // 6.26 / 6.00; 8B, 16 rows: 4.00 / 3.78)
 constexpr int XLDS_MIN_MT = 32;       // band heights that always read their inputs in whole lines
 constexpr int XLDS_M16_FROM = 9;      // input rows from which the 16-row band does too
+static_assert(XLDS_M16_FROM <= 9, "the fragment layout of a bf16 band holds 8 input rows (X8)");
 constexpr int AUX_WEIGHTS = 2;        // weights: non-temporal (every line is used exactly once)
 
 #ifdef LR_BAND_PROFILE
@@ -78,8 +79,19 @@ struct BandResidual {
   int top;
 };
 // KW: waves that share a band's K, all of them or 1: then every wave has a band of its own (`band_` counts groups of NWV).
+// DEEP: the inputs are requested as far ahead as the weights.  Loads come back in the order of their requests, so a wait
+// for inputs that were asked for one chunk ago is a wait for nearly all the weights asked for before them; with both in
+// one order a wait leaves the younger chunks in flight.  (16-row bands; at 32 rows the registers for it cost more.)
+// X8: at most 8 input rows.  Fragment columns 8 to 15 would be empty, so their lanes carry the next 32 elements of K of
+// rows 0 to 7, and every second fragment is the previous load rotated by 8 lanes: half as many input loads (which were a
+// third of a bf16 band's requests and half of an e4m3 band's) and half their registers.
+// UROWS: weight rows of a unit that are loaded, 8 where no band has more: a load of absent rows takes its time too.
+// The three together, us, 8 rows: 1280 x 8192 9.43 -> 7.41, 4096 x 4096 9.37 -> 8.64, 10240 x 4096 19.25 -> 18.50, up/gate
+// 7168 x 8192 22.4 -> 21.9, 8192 x (1024 | 3584) 16.9 -> 16.3; 16 rows (DEEP alone) 4096 x 14336 25.1 -> 23.8; e4m3, 5 rows:
+// 1280 x 8192 7.80 -> 6.32, 8192 x (1024 | 3584) 11.9 -> 10.8, up/gate 14.2 -> 13.6.  The sums keep their order.
 // GATHER: input row m is row rows[m] / xdiv of x, output row m is row rows[m] of y (`rows`: M of them, in LDS).
-template <int MT, int UNITS, bool W8 = false, bool XL = (MT >= XLDS_MIN_MT), bool GATHER = false, bool RESID = false, int KW = NWV>
+template <int MT, int UNITS, bool W8 = false, bool XL = (MT >= XLDS_MIN_MT), bool GATHER = false, bool RESID = false, int KW = NWV,
+          int UROWS = 16, bool DEEP = true, bool X8 = false>
 __device__ __forceinline__ void stream_band(const Proj& p, const int M, const int band_, u16* sg_smem,
                                             const int32_t* rows = nullptr, const int xdiv = 1, const BandResidual rs = {}) {
   static_assert(!W8 || MT == 16, "the e4m3 path is built for up to 16 input rows");
@@ -87,9 +99,14 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
   constexpr int LRW = KCW + 8;         // LDS row length in elements
   constexpr int WB = W8 ? 1 : 2;       // bytes per weight
   // weight chunks in flight per wave: the e4m3 variant has twice the A fragments and input registers per chunk
-  // and gives up two of its four sets for a second workgroup per CU
-  constexpr int NS = W8 ? 2 : SETS;
-  constexpr int MTILES = MT / 16, KS = KCW / 32, NLD = UNITS * 4;
+  // and gives up two of its four sets for a second workgroup per CU (with half the input registers, X8, four sets would
+  // fit: up/gate of 5 rows 13.3 -> 15.0 us), except where a band is 8 rows (1280 x 8192: 6.9 us with two, 6.3 with four;
+  // a bf16 band of 8 rows with eight sets: 8.1, with four 7.4)
+  constexpr int NS = W8 && UROWS == 16 ? 2 : SETS;
+  constexpr int XS = DEEP ? NS : 2;
+  constexpr int MTILES = MT / 16, KS = KCW / 32, NLD = UNITS * UROWS / 4;
+  static_assert(!X8 || (MT == 16 && !XL), "one tile of inputs in fragment layout");
+  static_assert(UROWS == 16 || (UROWS == 8 && UNITS == 1), "a unit is loaded whole or by half");
   constexpr int NV = UNITS * MTILES * 4;  // accumulator registers per lane
   // XL: the inputs too are loaded in whole lines (4 rows x 256 bytes per instruction) and take the trip through
   // LDS into B-fragment layout: L2 serves whole-line reads 1.5 times as fast as the 16 rows x 64 bytes a
@@ -111,6 +128,7 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, l4 = lane >> 4;
+  const int la = lane & (UROWS - 1);  // the band row of a lane's A fragment (beyond UROWS the first rows again: unused sums)
   static_assert(KW == NWV || (KW == 1 && !W8 && !XL), "");
   const int band = KW == 1 ? band_ * NWV + wave : band_;
   const int kwave = KW == 1 ? 0 : wave;
@@ -147,16 +165,28 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
   } else {
 #pragma unroll
     for (int mt = 0; mt < MTILES; ++mt) {
-      const int m = mt * 16 + l16;
+      const int m = mt * 16 + (X8 ? l16 & 7 : l16);
       const int xm = GATHER ? (m < M ? rows[m] / xdiv : 0) : m;
-      xoff[mt] = m < M ? (int)((xm * ldx + l4 * 8) * 2) : OOB;
+      xoff[mt] = m < M ? (int)((xm * ldx + (X8 ? (l16 >> 3) * 32 : 0) + l4 * 8) * 2) : OOB;
     }
   }
+  // k-step ks of input tile mt as a B fragment
+  auto xfrag = [&](const u32x4_t (&r)[MTILES][X8 ? KS / 2 : KS], int mt, int ks) {
+    if constexpr (X8) {
+      u32x4_t v = r[0][ks / 2];
+      if (ks & 1)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = __builtin_amdgcn_update_dpp(v[e], v[e], 0x128, 0xf, 0xf, false);  // row_ror:8
+      return __builtin_bit_cast(bf16x8_t, v);
+    } else {
+      return __builtin_bit_cast(bf16x8_t, r[mt][ks]);
+    }
+  };
   u16* const my = sg_smem + wave * (WPIECE + XPIECE);
   u16* const myx = my + WPIECE;
 
   u32x4_t wr[NS][NLD];
-  u32x4_t xr[2][MTILES][KS];
+  u32x4_t xr[XS][MTILES][X8 ? KS / 2 : KS];
   f32x4_t acc[UNITS][MTILES];
 #pragma unroll
   for (int u = 0; u < UNITS; ++u)
@@ -176,23 +206,28 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
     for (int i = 0; i < NLD; ++i)
       dst[i] = __builtin_amdgcn_raw_buffer_load_b128(wres, (kok && woff[i] != OOB) ? woff[i] : OOB, k0 * WB, AUX_WEIGHTS);
   };
-  auto issue_x = [&](int ci, u32x4_t (&dst)[MTILES][KS]) {
+  auto issue_x = [&](int ci, u32x4_t (&dst)[MTILES][X8 ? KS / 2 : KS]) {
     const int k0 = (ci * KW + kwave) * KCW;
-    if (XLDS) {
+    if constexpr (XLDS) {
       const bool kok = k0 + l16 * 8 < K;
 #pragma unroll
       for (int i = 0; i < MT / 4; ++i)
         dst[i / KS][i % KS] =
             __builtin_amdgcn_raw_buffer_load_b128(xres, (kok && xoff[i] != OOB) ? xoff[i] : OOB, k0 * 2, 0);
-      return;
-    }
+    } else if constexpr (X8) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const bool kok = k0 + ks * 32 + l4 * 8 < K;
+      for (int j = 0; j < KS / 2; ++j)
+        dst[0][j] = __builtin_amdgcn_raw_buffer_load_b128(
+            xres, (k0 + (2 * j + (l16 >> 3)) * 32 + l4 * 8 < K && xoff[0] != OOB) ? xoff[0] : OOB, (k0 + 2 * j * 32) * 2, 0);
+    } else {
 #pragma unroll
-      for (int mt = 0; mt < MTILES; ++mt)
-        dst[mt][ks] = __builtin_amdgcn_raw_buffer_load_b128(xres, (kok && xoff[mt] != OOB) ? xoff[mt] : OOB,
-                                                           (k0 + ks * 32) * 2, 0);
+      for (int ks = 0; ks < KS; ++ks) {
+        const bool kok = k0 + ks * 32 + l4 * 8 < K;
+#pragma unroll
+        for (int mt = 0; mt < MTILES; ++mt)
+          dst[mt][ks] = __builtin_amdgcn_raw_buffer_load_b128(xres, (kok && xoff[mt] != OOB) ? xoff[mt] : OOB,
+                                                             (k0 + ks * 32) * 2, 0);
+      }
     }
   };
 
@@ -204,6 +239,7 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
   issue_x(0, xr[0]);
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
+    if (DEEP && s) issue_x(s, xr[s]);
     asm volatile("" ::: "memory");
     issue_w(s, wr[s]);
   }
@@ -213,7 +249,7 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       const int ci = c0 + s;
-      issue_x(ci + 1, xr[(s + 1) & 1]);
+      if (!DEEP) issue_x(ci + 1, xr[(s + 1) % XS]);
       // ---- this chunk's weights: registers -> LDS (row-major) -> A fragments
       asm volatile("" ::: "memory");
 #pragma unroll
@@ -245,18 +281,19 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
 #pragma unroll
             for (int k2 = 0; k2 < KS / 2; ++k2)
               ah[u][k2] =
-                  *reinterpret_cast<const bf16x8_t*>(my + (16 * u + l16) * LRW + (h * (KS / 2) + k2) * 32 + l4 * 8);
+                  *reinterpret_cast<const bf16x8_t*>(my + (16 * u + la) * LRW + (h * (KS / 2) + k2) * 32 + l4 * 8);
 #pragma unroll
           for (int k2 = 0; k2 < KS / 2; ++k2)
 #pragma unroll
             for (int mt = 0; mt < MTILES; ++mt) {
-              const bf16x8_t bx = __builtin_bit_cast(bf16x8_t, xr[s & 1][mt][h * (KS / 2) + k2]);
+              const bf16x8_t bx = xfrag(xr[s % XS], mt, h * (KS / 2) + k2);
 #pragma unroll
               for (int u = 0; u < UNITS; ++u)
                 acc[u][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[u][k2], bx, acc[u][mt], 0, 0, 0);
             }
         }
         asm volatile("" ::: "memory");
+        if (DEEP) issue_x(ci + NS, xr[s % XS]);
         continue;
       }
       bf16x8_t af[UNITS][KS];
@@ -264,14 +301,15 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
       for (int u = 0; u < UNITS; ++u)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
-          af[u][ks] = *reinterpret_cast<const bf16x8_t*>(my + (16 * u + l16) * LRW + ks * 32 + l4 * 8);
+          af[u][ks] = *reinterpret_cast<const bf16x8_t*>(my + (16 * u + la) * LRW + ks * 32 + l4 * 8);
       asm volatile("" ::: "memory");
       issue_w(ci + NS, wr[s]);
       if (XLDS) {
 #pragma unroll
         for (int i = 0; i < MT / 4; ++i)
-          *reinterpret_cast<u32x4_t*>(myx + (4 * i + l4) * LRW + l16 * 8) = xr[s & 1][i / KS][i % KS];
+          *reinterpret_cast<u32x4_t*>(myx + (4 * i + l4) * LRW + l16 * 8) = xr[s % XS][i / KS][i % KS];
         asm volatile("" ::: "memory");
+        if (DEEP) issue_x(ci + NS, xr[s % XS]);
       }
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
@@ -279,12 +317,13 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
         for (int mt = 0; mt < MTILES; ++mt) {
           bf16x8_t bx;
           if (XLDS) bx = *reinterpret_cast<const bf16x8_t*>(myx + (16 * mt + l16) * LRW + ks * 32 + l4 * 8);
-          else bx = __builtin_bit_cast(bf16x8_t, xr[s & 1][mt][ks]);
+          else bx = xfrag(xr[s % XS], mt, ks);
 #pragma unroll
           for (int u = 0; u < UNITS; ++u)
             acc[u][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[u][ks], bx, acc[u][mt], 0, 0, 0);
         }
       if (XLDS) asm volatile("" ::: "memory");
+      else if (DEEP) issue_x(ci + NS, xr[s % XS]);
     }
   }
 

@@ -13,8 +13,7 @@
 // 32 weight rows -- the number of rows is chosen so that every CU gets the same share -- and its
 // waves split K in 128-element chunks (wave w takes chunks w, w + 4, ...: together they read 1 KiB
 // contiguous per row and round).  Each wave keeps 4 chunks of weights (32 KiB) in flight in
-// registers, 128 KiB per CU.  The input rows come from L2 straight into B-fragment layout, one
-// chunk ahead.  The waves' partial sums meet in LDS and are added in a fixed order.
+// registers, 128 KiB per CU.  The input rows come from L2 straight into B-fragment layout.  The waves' partial sums meet in LDS and are added in a fixed order.
 //
 // Two projections that read the same layer input can share one launch (the band index selects the
 // projection), and a projection whose weight holds [up; gate] rows can take the band as row PAIRS
@@ -24,20 +23,20 @@
 
 namespace {
 
-template <int MT, int UNITS, bool W8, bool XL>
-__global__ __launch_bounds__(NWV * 64) void k_stream_gemm(const Proj p0, const Proj p1, const int M) {
+template <int MT, int UNITS, bool W8, bool XL, int UROWS, bool DEEP, bool X8>
+__global__ __launch_bounds__(NWV * 64, MT == 16 ? 2 : 0) void k_stream_gemm(const Proj p0, const Proj p1, const int M) {
   extern __shared__ __attribute__((aligned(16))) u16 sg_smem[];
   const bool second = (int)blockIdx.x >= p0.nwg;
   const Proj p = second ? p1 : p0;
-  stream_band<MT, UNITS, W8, XL>(p, M, second ? (int)blockIdx.x - p0.nwg : (int)blockIdx.x, sg_smem);
+  stream_band<MT, UNITS, W8, XL, false, false, NWV, UROWS, DEEP, X8>(p, M, second ? (int)blockIdx.x - p0.nwg : (int)blockIdx.x, sg_smem);
 }
 
-template <int MT, int UNITS, bool W8 = false, bool XL = (MT >= XLDS_MIN_MT)>
+template <int MT, int UNITS, bool W8 = false, bool XL = (MT >= XLDS_MIN_MT), int UROWS = 16, bool X8 = (MT == 16 && !XL && !W8), bool DEEP = (MT == 16)>
 static int launch_units(Proj& a, Proj& b, int M, hipStream_t s) {
   constexpr size_t lds = stream_band_lds_bytes<MT, UNITS, W8, XL>();
   static std::atomic<unsigned long long> lds_raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_stream_gemm<MT, UNITS, W8, XL>), lds, lds_raised)) return LR_E_LAUNCH;
-  k_stream_gemm<MT, UNITS, W8, XL><<<dim3((unsigned)(a.nwg + b.nwg)), dim3(NWV * 64), lds, s>>>(a, b, M);
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_stream_gemm<MT, UNITS, W8, XL, UROWS, DEEP, X8>), lds, lds_raised)) return LR_E_LAUNCH;
+  k_stream_gemm<MT, UNITS, W8, XL, UROWS, DEEP, X8><<<dim3((unsigned)(a.nwg + b.nwg)), dim3(NWV * 64), lds, s>>>(a, b, M);
   return LR_OK;
 }
 
@@ -45,7 +44,17 @@ template <int MT>
 static int launch(Proj& a, Proj& b, int M, int units, hipStream_t s) {
   if (MT == 16 && M >= XLDS_M16_FROM)  // the 16-row band with its inputs read in whole lines
     return units == 2 ? launch_units<MT, 2, false, true>(a, b, M, s) : launch_units<MT, 1, false, true>(a, b, M, s);
+  // bands of at most 8 weight rows load half a unit (8 input rows, 2048 x 2048: 4.83 -> 4.10 us; with 9 to 16 input rows,
+  // 1280 x 8192, nothing moves: 10.0 / 10.1)
+  if (MT == 16 && units == 1 && a.rpw <= 8 && b.rpw <= 8) return launch_units<16, 1, false, false, 8>(a, b, M, s);
   return units == 2 ? launch_units<MT, 2>(a, b, M, s) : launch_units<MT, 1>(a, b, M, s);
+}
+
+template <bool X8>
+static int launch_fp8(Proj& a, Proj& b, int M, int units, hipStream_t s) {
+  if (units == 2) return launch_units<16, 2, true, false, 16, X8>(a, b, M, s);
+  if (a.rpw <= 8 && b.rpw <= 8) return launch_units<16, 1, true, false, 8, X8>(a, b, M, s);
+  return launch_units<16, 1, true, false, 16, X8>(a, b, M, s);
 }
 
 // one 16-row unit per workgroup when every CU still gets a band that way; row pairs always take two units
@@ -83,9 +92,9 @@ extern "C" int lr_linear_multi(const lr_projection_t* proj, int n_proj, int M, l
 namespace {
 
 template <int MT, int UNITS, bool XL>
-__global__ __launch_bounds__(NWV * 64) void k_stream_residual(const Proj p, const int M, const BandResidual rs) {
+__global__ __launch_bounds__(NWV * 64, MT == 16 ? 2 : 0) void k_stream_residual(const Proj p, const int M, const BandResidual rs) {
   extern __shared__ __attribute__((aligned(16))) u16 sg_smem[];
-  stream_band<MT, UNITS, false, XL, false, true>(p, M, blockIdx.x, sg_smem, nullptr, 1, rs);
+  stream_band<MT, UNITS, false, XL, false, true, NWV, 16, MT == 16, MT == 16 && !XL>(p, M, blockIdx.x, sg_smem, nullptr, 1, rs);
 }
 
 template <int MT, int UNITS, bool XL>
@@ -158,7 +167,7 @@ int stream_fp8_multi(const lr_projection_fp8_t* proj, int n_proj, int M, lr_stre
   if (ncu < 1) return LR_E_LAUNCH;
   const int units = pick_units_and_plan(pr, n_proj, M, ncu);
   hipStream_t s = (hipStream_t)stream;
-  const int rc = units == 2 ? launch_units<16, 2, true>(pr[0], pr[1], M, s) : launch_units<16, 1, true>(pr[0], pr[1], M, s);
+  const int rc = M <= 8 ? launch_fp8<true>(pr[0], pr[1], M, units, s) : launch_fp8<false>(pr[0], pr[1], M, units, s);
   return rc != LR_OK ? rc : lr_launch_status();
 }
 }  // namespace lr_detail

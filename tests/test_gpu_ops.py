@@ -495,6 +495,26 @@ def test_ladder_norms_equals_two_add_rmsnorm_calls(hip, rows, dim, first_block):
     assert_close_ulp(n2, O.rms_norm(r2, g2, 1e-5), max_ulp=2, max_frac=0.05, what="ladder_norms n2")
 
 
+@pytest.mark.parametrize("M", [1, 2, 7, 8])
+@pytest.mark.parametrize("N,K", [(5, 16), (1280, 4112), (2048, 528), (2056, 144), (4104, 2064)])
+def test_bands_of_few_rows_equal_the_bands_of_many(hip, M, N, K):
+    """Up to 8 input rows share fragments and thin bands load half a unit; a sum keeps its order, so a row's results are
+    the bits it has in a call of 16 rows (inputs in whole lines, or e4m3 with full fragments)."""
+    x = torch.full((16, K + 24), float("nan"), dtype=BF, device=DEV)[:, :K]      # rows and columns beyond are not read
+    x.copy_(rnd(16, K, seed=90))
+    w, w8 = rnd(N, K, seed=91), rnd(N, K, seed=92).to(torch.float8_e4m3fn)
+    scales = rnd(N, seed=93).abs()
+    few, many = (torch.empty(m, N, dtype=BF, device=DEV) for m in (M, 16))
+    hip.linear_multi((x[:M], w, few, hip.EPI_NONE))
+    hip.linear_multi((x, w, many, hip.EPI_NONE))
+    assert torch.equal(few, many[:M])
+    assert_close_ulp(few, linear_ref(x[:M], w), what="few rows")
+    if M > 1:      # (one row of e4m3 weights is the matrix-vector kernel)
+        hip.linear_fp8_multi((x[:M], w8, scales, few, hip.EPI_NONE))
+        hip.linear_fp8_multi((x, w8, scales, many, hip.EPI_NONE))
+        assert torch.equal(few, many[:M])
+
+
 @pytest.mark.parametrize("rows,dim", [(2, 4096), (2, 4104), (257, 8192), (3, 8200), (1, 16376)])
 def test_norms_at_the_edges_of_the_lanes_per_row(hip, rows, dim):
     """256 lanes up to 4096 columns, 1024 above; the last columns leave most lanes of the last turn idle."""
