@@ -13,7 +13,8 @@
 // 32 weight rows -- the number of rows is chosen so that every CU gets the same share -- and its
 // waves split K in 128-element chunks (wave w takes chunks w, w + 4, ...: together they read 1 KiB
 // contiguous per row and round).  Each wave keeps 4 chunks of weights (32 KiB) in flight in
-// registers, 128 KiB per CU.  The input rows come from L2 straight into B-fragment layout.  The waves' partial sums meet in LDS and are added in a fixed order.
+// registers, 128 KiB per CU.  The input rows come from L2 straight into B-fragment layout.  The waves' partial sums
+// meet in LDS and are added in a fixed order.
 //
 // Two projections that read the same layer input can share one launch (the band index selects the
 // projection), and a projection whose weight holds [up; gate] rows can take the band as row PAIRS
