@@ -19,7 +19,7 @@ Prints ONE JSON line.  `value` = decoded tokens per second (whole job = the one 
                launch stream.  `traffic` = HBM bytes per launch from rocprofv3 FETCH_SIZE + WRITE_SIZE
                counter runs (a constant recorded from those runs, or null).  Other models / batches
                run the per-op path, whose dominant kernel is the up/gate projection (timed alone here:
-               the GEMV up to batch 4, the matrix-core band kernel above).
+               the GEMV up to batch 4, the matrix-core band kernel up to 32, above that the product with partial sums).
                `measured_read_ceiling` = GB/s of a plain streaming read of 8 GiB by every CU
                (lr_stream_read) on this machine in the same run; `frac` is against the nominal
                8 TB/s, `frac_of_measured_ceiling` against that.
@@ -63,12 +63,11 @@ TRAFFIC_BYTES_PER_LAUNCH = {
     ("gpt_ladder:ladder-70b-tp8", 1, 2048): 17.585e9,    # k_ladder_step, 1.007 x algorithmic
     # the up/gate projection alone (the kernel the batched workloads' roofline object is measured on):
     ("gpt_ladder:ladder-70b-tp8", 8, 2048): 118.75e6,    # k_stream_gemm<16,2>, 256 bands: 1.009 x algorithmic
-    ("gpt_ladder:ladder-70b-tp8", 64, 2048): 126.46e6,   # k_stream_gemm<64,2>, the decode step's 224 bands: 1.06 x
 }
 # HBM bytes of a whole decode step through the per-op kernels (all its launches), from the same kind of counter runs
 STEP_TRAFFIC_BYTES = {
     ("gpt_ladder:ladder-70b-tp8", 8, 2048): 22.41e9,     # 1.24 x algorithmic
-    ("gpt_ladder:ladder-70b-tp8", 64, 2048): 30.46e9,    # 1.34 x algorithmic
+    ("gpt_ladder:ladder-70b-tp8", 64, 2048): 27.52e9,    # 1.21 x algorithmic
 }
 
 
@@ -670,7 +669,9 @@ def main():
             run = lambda i: _hip.linear_fp8_multi((x, w1s[i], scs[i], y, _hip.EPI_NONE)) if B <= 16 else \
                 _hip.linear_fp8(x, w1s[i], scs[i], y)
         else:
-            run = lambda i: _hip.linear(x, w1s[i], y)
+            n = _hip.linear_scratch_bytes(B)   # (above 32 rows: the product with partial sums, as in the step)
+            sums = torch.empty(n, dtype=torch.uint8, device=dev) if n else None
+            run = lambda i: _hip.linear(x, w1s[i], y, scratch=sums)
         for i in range(8):
             run(i)
         reps = 3
@@ -685,7 +686,7 @@ def main():
         wbytes = 1 if args.fp8 else 2
         k_bytes = wbytes * N * Kdim + 2 * (B * Kdim + B * N)
         kern = ("k_gemv_fp8_multi" if B == 1 else "k_stream_gemm (e4m3 bands)") if args.fp8 else \
-            ("k_gemv" if B <= 4 else "k_stream_gemm")
+            ("k_gemv" if B <= 4 else "k_stream_gemm" if B <= 32 else "k_gemm_dma + k_gemm_sum")
         k_name = f"{kern} (w1 up+gate projection, [{N} x {Kdim}] {'e4m3' if args.fp8 else 'bf16'}, M={B})"
     k_gbps = k_bytes / (k_us * 1e-6) / 1e9
 
