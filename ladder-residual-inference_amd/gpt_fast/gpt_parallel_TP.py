@@ -48,7 +48,8 @@ class GPTParallel(GPTBase):
         cfg = self.config
         nqkv = (cfg.n_head_local + 2 * cfg.n_kv_local) * cfg.head_dim
         att0 = self.layers[0].attention
-        if ws.S == 1 and ws.B <= 64 and not any(hasattr(m, "scales") for m in (att0.wqkv1, att0.wo, att0.w2)):
+        if (ws.S == 1 and self.band_rows_from <= ws.B <= 64
+                and not any(hasattr(m, "scales") for m in (att0.wqkv1, att0.wo, att0.w2))):
             return self._run_layers_decode(ws, pos, nqkv)
         for blk in self.layers:
             att = blk.attention

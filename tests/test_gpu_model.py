@@ -807,7 +807,7 @@ def test_variants_on_70b_shard_shape_at_full_depth(family, B):
 @pytest.mark.parametrize("B", [3, 20])
 @pytest.mark.parametrize("semi", [False, True])
 @torch.no_grad()
-def test_variant_decode_on_the_bands_equals_the_single_projection_kernels(family, B, semi):
+def test_variant_decode_on_the_bands_equals_the_single_projection_kernels(family, B, semi, monkeypatch):
     """Decode steps of the other families through lr_linear_multi (q/k/v with the RoPE + cache epilogue, up/gate with
     the SwiGLU epilogue; parallel family: up/gate beside the attention up to 16 rows, beside q/k/v above, y + x left to
     the next norm) against the same steps through lr_linear and the separate kernels: the same tokens fed, logits
@@ -822,8 +822,15 @@ def test_variant_decode_on_the_bands_equals_the_single_projection_kernels(family
     g.manual_seed(3)
     toks = torch.randint(0, 512, (B, 10), device=DEV, generator=g)
 
+    from gpt_fast import _hip
+
+    launches = []
+    multi = _hip.linear_multi
+    monkeypatch.setattr(_hip, "linear_multi", lambda *a: (launches.append(len(a)), multi(*a))[1])
+
     def steps(rows_from):
         model.band_rows_from = rows_from
+        launches.clear()
         out = [model(toks[:, :6], torch.arange(6, device=DEV)).clone()]
         for t in range(6, 10):
             out.append(model(toks[:, t:t + 1], torch.tensor([t], device=DEV)).clone())
@@ -832,7 +839,9 @@ def test_variant_decode_on_the_bands_equals_the_single_projection_kernels(family
         return out, kv.k_cache[:B, :, :10].clone(), kv.v_cache[:B, :, :10].clone()
 
     plain, kp, vp = steps(10 ** 9)
+    assert not launches     # (two routes are compared)
     bands, kb, vb = steps(1)
+    assert launches
     assert torch.equal(plain[0], bands[0])   # prefill does not depend on the switch
     for a, b in zip(plain[1:], bands[1:]):
         assert rel_err(b, a) <= REL_TOL
