@@ -109,6 +109,16 @@ int lr_linear(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, i
  * used).  With scratch the GEMM also serves M of 33 to 64, where it is then faster than the weight-streaming kernel.
  * Calls that may overlap need memory of their own.  No counterpart in the reference. */
 size_t lr_linear_scratch_bytes(int M);
+/* How that GEMM would divide a product of M rows with `scratch_bytes` of such memory (rows within its reach, see
+ * lr_linear): pair = 0 for lr_linear_scratch and lr_linear_rope_kv_scratch, 1 for lr_linear_swiglu_out_scratch (N = 2 I
+ * there too).  A host computation, no launch: what to allocate for a given product is the sums_bytes of its plan at
+ * lr_linear_scratch_bytes(M), with which the plan stays what it is.  No counterpart in the reference. */
+typedef struct lr_linear_plan {
+  int32_t tile_rows, tile_cols; /* input rows and weight rows of a tile */
+  int32_t whole, cut, pieces;   /* tiles computed whole; tiles cut along K, and into how many pieces each */
+  size_t sums_bytes;            /* of the pieces' sums */
+} lr_linear_plan_t;
+int lr_linear_plan(int M, int N, int K, int pair, size_t scratch_bytes, lr_linear_plan_t* plan);
 int lr_linear_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, void* scratch,
                       size_t scratch_bytes, lr_stream_t stream);
 

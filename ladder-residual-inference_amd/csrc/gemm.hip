@@ -744,6 +744,21 @@ extern "C" int lr_linear(const void* x, int64_t ldx, const void* w, void* y, int
 
 extern "C" size_t lr_linear_scratch_bytes(int M) { return M >= GEMM_SCRATCH_FROM ? GEMM_SCRATCH : 0; }
 
+extern "C" int lr_linear_plan(int M, int N, int K, int pair, size_t scratch_bytes, lr_linear_plan_t* plan) {
+  if (plan == nullptr) return LR_E_NULL;
+  if (M <= 0 || N <= 0 || K <= 0 || (pair && N % 2)) return LR_E_SHAPE;
+  if (K % 8) return LR_E_ALIGN;
+  const GemmPlan p = gemm_plan(M, pair ? N / 2 : N, K, pair ? GEMM_PAIR : GEMM_PLAIN, scratch_bytes);
+  if (p.tile < 0) return LR_E_UNSUPPORTED;
+  plan->tile_rows = 64 * GEMM_TILES[p.tile].a16;
+  plan->tile_cols = 128 * GEMM_TILES[p.tile].bh;
+  plan->whole = p.full;
+  plan->cut = p.rem;
+  plan->pieces = p.splits;
+  plan->sums_bytes = p.rem ? (size_t)p.rem * p.splits * plan->tile_rows * plan->tile_cols * sizeof(float) : 0;
+  return LR_OK;
+}
+
 extern "C" int lr_linear_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, void* scratch,
                                  size_t scratch_bytes, lr_stream_t stream) {
   LR_OPTIONAL_PTR(scratch);

@@ -26,6 +26,7 @@ _PROTOS = {
     "lr_linear_tuned": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_int,
                                 c_void_p]),
     "lr_linear_scratch_bytes": (c_size_t, [c_int]),
+    "lr_linear_plan": (c_int, [c_int, c_int, c_int, c_int, c_size_t, c_void_p]),
     "lr_linear_scratch": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_size_t,
                                   c_void_p]),
     "lr_linear_multi": (c_int, [c_void_p, c_int, c_int, c_void_p]),
@@ -232,6 +233,25 @@ def ladder_norms(resid_in, d1, d2, gain1, gain2, resid_out, normed1, normed2, ep
 
 def linear_scratch_bytes(rows: int) -> int:
     return int(load().lr_linear_scratch_bytes(rows))
+
+
+class _LinearPlan(ctypes.Structure):   # lr_linear_plan_t
+    _fields_ = [(n, c_int32) for n in ("tile_rows", "tile_cols", "whole", "cut", "pieces")] + [("sums_bytes", c_size_t)]
+
+
+def linear_plan(rows: int, N: int, K: int, pair: bool = False, scratch_bytes: int = None) -> _LinearPlan:
+    """How the matrix-core GEMM divides a product (lr_linear_plan), by default with all the scratch it could use."""
+    p = _LinearPlan()
+    n = linear_scratch_bytes(rows) if scratch_bytes is None else scratch_bytes
+    _check(load().lr_linear_plan(rows, N, K, int(pair), n, ctypes.byref(p)), "lr_linear_plan")
+    return p
+
+
+def linear_sums_bytes(products) -> int:
+    """Bytes that serve all of `products` -- (rows, N, K, pair), any number of times each -- as `scratch` or `sums`, one at a
+    time; 0: none of them is a product that takes any."""
+    taken = [linear_plan(*p).sums_bytes for p in set(products) if linear_scratch_bytes(p[0]) and p[2] % 8 == 0]
+    return max(256, *taken) if taken else 0   # (what is given says which kernels run, also where no tile is cut)
 
 
 def _scratch_args(t):

@@ -23,7 +23,7 @@ class HybridWorkspace:
         self.xc = e(rows, D)                      # in the compute type: the input of the next product
         self.d = e(rows, D)                       # what the current sublayer adds to the residual
         self.proj = e(rows, pad8(max(m.proj_cols for m in mixers)))
-        n = _hip.linear_scratch_bytes(rows) if dtype == torch.bfloat16 else 0
+        n = model._sums_bytes(B, S)
         self.sums = e(n, dt=torch.uint8) if n else None      # partial sums of products
         n = max(m.scratch_bytes(B, S) for m in mixers)
         self.scratch = e(n, dt=torch.uint8) if n else None
@@ -72,6 +72,14 @@ class GPTHybrid(GPTBase):
         return int(it * (self._weights_per_step(batch_size) + batch_size * self.config.dim) + carried)
 
     # -- forward ----------------------------------------------------------------------------------
+    def _products(self, B, S):
+        for rows, N, K, pair in super()._products(B, S):
+            yield rows, N, K, pair
+        for blk in self.layers:
+            rows, cols = blk.mixer.window_rows(B, S)
+            if rows and self.output.weight.dtype == torch.bfloat16:
+                yield rows, *blk.mixer.kv_up.weight.shape, False
+
     def _new_workspace(self, B, S):
         w = self.output.weight
         return self.workspace_class(self, B, S, w.dtype, w.device, not self.last_logits_only)

@@ -22,7 +22,8 @@ from .utils import KVCache, RMSNorm, _pos_i32, precompute_freqs_cis
 class Workspace:
     """Activation buffers for one (batch, seq) shape, all bf16 [rows, *]."""
 
-    def __init__(self, cfg: ModelArgs, B: int, S: int, fused_width: int, device, dtype, smax: int, all_logits: bool):
+    def __init__(self, cfg: ModelArgs, B: int, S: int, fused_width: int, device, dtype, smax: int, all_logits: bool,
+                 sums_bytes: int):
         rows = B * S
         D, hd = cfg.dim, cfg.head_dim
         e = lambda *shape: torch.empty(*shape, dtype=dtype, device=device)
@@ -46,7 +47,7 @@ class Workspace:
         self.next_token_valid_for = None   # set by a fused decode step that already chose the token
         self.scratch = None
         # partial sums of products; the MLP's may run beside the attention's in a decode step
-        n = _hip.linear_scratch_bytes(rows)
+        n = sums_bytes
         self.sums = self.sums_mlp = torch.empty(n, dtype=torch.uint8, device=device) if n else None
         if n and S == 1:
             # (room for the pieces of three quarters of the compute units, 32 KiB each: the attention's products keep the
@@ -162,7 +163,18 @@ class GPTBase(nn.Module):
 
     def _new_workspace(self, B: int, S: int):
         return Workspace(self.config, B, S, self._fused_width(), self.output.weight.device, self.norm.weight.dtype,
-                         self.max_seq_length, not self.last_logits_only)
+                         self.max_seq_length, not self.last_logits_only, self._sums_bytes(B, S))
+
+    def _products(self, B: int, S: int):
+        """(rows, N, K, pair) of every bf16 projection of a (B, S) step, as linear_sums_bytes takes them."""
+        head = B if self.last_logits_only else B * S
+        for name, mod in self.named_modules():
+            if isinstance(mod, nn.Linear) and mod.weight.dtype == torch.bfloat16:
+                leaf = name.rpartition(".")[2]
+                yield head if leaf == "output" else B * S, *mod.weight.shape, leaf == "w1"
+
+    def _sums_bytes(self, B: int, S: int) -> int:
+        return _hip.linear_sums_bytes(self._products(B, S))
 
     # -- forward --------------------------------------------------------------------------------
     def forward(self, idx: Tensor, input_pos: Optional[Tensor] = None) -> Tensor:

@@ -44,6 +44,14 @@ class GPTParallel(GPTBase):
     def _fused_width(self) -> int:
         return super()._fused_width() + 2 * self.config.ffn_local
 
+    def _products(self, B, S):
+        nqkv = GPTBase._fused_width(self)
+        for rows, N, K, pair in super()._products(B, S):
+            yield rows, N, K, pair
+            if S == 1 and N == self._fused_width():   # (the decode step's two parts of the fused weight)
+                yield rows, nqkv, K, False
+                yield rows, N - nqkv, K, True
+
     def _run_layers(self, ws: Workspace, pos: Tensor):
         cfg = self.config
         nqkv = (cfg.n_head_local + 2 * cfg.n_kv_local) * cfg.head_dim

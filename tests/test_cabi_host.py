@@ -275,3 +275,53 @@ def test_setup_caches_refuses_a_sequence_longer_than_block_size():
         model = bm.GPTLadder(ModelArgs(block_size=64, vocab_size=512, n_layer=1, n_head=4, dim=256))
     with pytest.raises(ValueError):
         model.setup_caches(1, 65)
+
+
+FAMILIES = [("ladder", "ladder-70b-tp8"), ("dense", "ladder-8b"), ("desync", "ladder-8b"), ("parallel", "ladder-8b"),
+            ("lasivik", "lasivik-8b"), ("gepolix", "gepolix-8b")]
+
+
+def meta_model(family, name):
+    import gpt_fast
+
+    with torch.device("meta"):
+        m = getattr(gpt_fast, "GPT" + family.capitalize()).from_name(name).to(torch.bfloat16)
+    m.max_batch_size, m.max_seq_length = 96, 1024
+    if family in ("lasivik", "gepolix"):
+        m._build_caches(96, 1024, torch.bfloat16, torch.device("meta"))
+    return m
+
+
+@pytest.mark.parametrize("family,name", FAMILIES)
+@pytest.mark.parametrize("B,S", [(1, 1), (32, 1), (33, 1), (64, 1), (96, 1), (1, 33), (1, 777), (4, 512)])
+def test_memory_for_partial_sums_is_what_the_products_of_a_step_can_use(lib, family, name, B, S):
+    """Enough for every product to be divided as with all the memory it could ask for, and no more than that."""
+    from gpt_fast import _hip
+
+    model = meta_model(family, name)
+    for model.last_logits_only in (False, True):
+        products = set(model._products(B, S))
+        assert len(products) >= 4
+        ws = model._new_workspace(B, S)
+        if B * S <= 32:
+            assert ws.sums is None and not any(lib.lr_linear_scratch_bytes(p[0]) for p in products if p[0] == B * S)
+            continue
+        held = ws.sums.numel()
+        plans = [(p, _hip.linear_plan(*p)) for p in products if lib.lr_linear_scratch_bytes(p[0])]
+        assert held == max(256, *(q.sums_bytes for _, q in plans)) <= lib.lr_linear_scratch_bytes(B * S)
+        for p, full in plans:
+            assert bytes(full) == bytes(_hip.linear_plan(*p, scratch_bytes=held))
+        if S == 1 and B <= 64:
+            assert held <= 16 << 20
+
+
+def test_a_model_without_bf16_projections_holds_no_memory_for_partial_sums(lib):
+    from gpt_fast.quantize import WeightOnlyFp8Linear
+
+    model = meta_model("ladder", "ladder-70b-tp8")
+    for parent in list(model.modules()):
+        for name, child in list(parent.named_children()):
+            if isinstance(child, torch.nn.Linear):
+                setattr(parent, name, WeightOnlyFp8Linear(child.in_features, child.out_features, device="meta"))
+    for B, S in ((48, 1), (1, 777)):
+        assert model._new_workspace(B, S).sums is None
