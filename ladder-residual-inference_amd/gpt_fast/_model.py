@@ -46,13 +46,19 @@ class Workspace:
         self.next_token = torch.empty(B, 1, dtype=torch.int32, device=device)
         self.next_token_valid_for = None   # set by a fused decode step that already chose the token
         self.scratch = None
-        # partial sums of products; the MLP's may run beside the attention's in a decode step
+        # Partial sums of products, in a decode step two memories: the MLP's may run beside the attention's, and alternating
+        # ones are faster also one after the other (8B dense, 33 rows: 4.67 ms per step, 4.71 in one).  The MLP's of up to 64
+        # rows has room for the pieces of 25 of 32 compute units, 32 KiB each: beside the attention's products these keep
+        # the rest (70B rank shard, 64 rows: 7.6 ms per step, 8.2 with as many pieces as pay for a product alone), and
+        # alone more are no faster (w2 4096 x 14336 of 64 rows: 31.9 us in six pieces, 34.2 in seven).  More rows have
+        # larger tiles and one chain (70B rank shard, 96 rows: 9.7 ms per step, 10.9 with room for as little).
         n = sums_bytes
         self.sums = self.sums_mlp = torch.empty(n, dtype=torch.uint8, device=device) if n else None
         if n and S == 1:
-            # (room for the pieces of three quarters of the compute units, 32 KiB each: the attention's products keep the
-            # rest -- 70B rank shard, batch 64: 7.6 ms per step, 8.2 with as many pieces as pay for a product alone)
-            self.sums_mlp = torch.empty(min(n, 200 << 15), dtype=torch.uint8, device=device)
+            if rows <= 64:
+                cus = torch.cuda.get_device_properties(device).multi_processor_count if device.type == "cuda" else 256
+                n = min(n, cus * 25 // 32 << 15)
+            self.sums_mlp = torch.empty(n, dtype=torch.uint8, device=device)
         if S == 1:
             n = _hip.attn_decode_scratch_bytes(B, cfg.n_head_local, hd, smax) // 4
             self.scratch = torch.empty(n, dtype=torch.float32, device=device)

@@ -325,3 +325,12 @@ def test_a_model_without_bf16_projections_holds_no_memory_for_partial_sums(lib):
                 setattr(parent, name, WeightOnlyFp8Linear(child.in_features, child.out_features, device="meta"))
     for B, S in ((48, 1), (1, 777)):
         assert model._new_workspace(B, S).sums is None
+
+
+@pytest.mark.parametrize("family,name", FAMILIES[:3])
+@pytest.mark.parametrize("B", [33, 64, 65, 96])
+def test_partial_sums_of_the_mlp_are_limited_where_that_was_measured(lib, family, name, B):
+    """Memory of its own beside the attention's: a part as large up to 64 rows, all that the products can use above."""
+    ws = meta_model(family, name)._new_workspace(B, 1)
+    assert ws.sums_mlp is not ws.sums and ws.sums_mlp._base is None
+    assert ws.sums_mlp.numel() == (min(ws.sums.numel(), 200 << 15) if B <= 64 else ws.sums.numel())
