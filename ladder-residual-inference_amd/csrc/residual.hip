@@ -28,12 +28,17 @@ __global__ __launch_bounds__(256) void k_embed_residual(const T* __restrict__ ta
 
 // r = alpha x + d;  out = r / sqrt(mean(r^2) + eps) * (offset + gain), in fp32 and / or in the compute type.  The mean is
 // over the first `width` columns (the rest is padding: zero in, zero out).
+// Up to 4096 columns the squares are summed by blocks of 1024 columns, whether 256 lanes take one block after the other or
+// 1024 lanes all of them: a row's bits do not depend on how many rows there are.  (256 lanes with one sum each, x 4096, us:
+// 257 rows 3.49 instead of 3.74, 1024 rows 8.11 / 8.22, 16384 rows 138.1 / 138.7.)
 constexpr int RN_MAXIT = 16;  // 256 lanes x 4 columns x 16
 template <typename T, int RN_IT, int LANES = 256>
 __global__ __launch_bounds__(LANES) void k_residual_norm(const float* x, float alpha, const T* __restrict__ d,
                                                        const T* __restrict__ gain, float offset, float* xo,
                                                        T* __restrict__ xc, int dim, int width, float eps) {
-  __shared__ float red[LANES / 64];
+  constexpr int BLOCKS = RN_IT <= 4 ? RN_IT : 1;   // sums of a lane
+  constexpr int SUMS = BLOCKS * LANES / 64;
+  __shared__ float red[SUMS];
   const int tid = threadIdx.x;
   const int64_t base = (int64_t)blockIdx.x * dim;
   float4 qx[RN_IT];
@@ -45,7 +50,7 @@ __global__ __launch_bounds__(LANES) void k_residual_norm(const float* x, float a
     if (d) qd[i].load(d + base + c);
     qg[i].load(gain + c);
   }
-  float ss = 0.0f;
+  float ss[BLOCKS] = {};
 #pragma unroll
   for (int i = 0; i < RN_IT; ++i) {
     const int c = (tid + i * LANES) * 4;
@@ -55,18 +60,17 @@ __global__ __launch_bounds__(LANES) void k_residual_norm(const float* x, float a
     qx[i].y = fmaf(alpha, qx[i].y, f[1]);
     qx[i].z = fmaf(alpha, qx[i].z, f[2]);
     qx[i].w = fmaf(alpha, qx[i].w, f[3]);
-    if (c < dim) ss += (qx[i].x * qx[i].x + qx[i].y * qx[i].y) + (qx[i].z * qx[i].z + qx[i].w * qx[i].w);
+    if (c < dim) ss[i % BLOCKS] += fmaf(qx[i].x, qx[i].x, qx[i].y * qx[i].y) + fmaf(qx[i].z, qx[i].z, qx[i].w * qx[i].w);
   }
-  ss = wave_sum(ss);
-  if ((tid & 63) == 0) red[tid >> 6] = ss;
+#pragma unroll
+  for (int b = 0; b < BLOCKS; ++b) {
+    ss[b] = wave_sum(ss[b]);
+    if ((tid & 63) == 0) red[b * (LANES / 64) + (tid >> 6)] = ss[b];
+  }
   __syncthreads();
   float sum = 0.0f;
-  if constexpr (LANES == 256) {
-    sum = (red[0] + red[1]) + (red[2] + red[3]);
-  } else {
 #pragma unroll
-    for (int i = 0; i < LANES / 64; i += 4) sum += (red[i] + red[i + 1]) + (red[i + 2] + red[i + 3]);
-  }
+  for (int i = 0; i < SUMS; i += 4) sum += (red[i] + red[i + 1]) + (red[i + 2] + red[i + 3]);
   const float inv = 1.0f / sqrtf(sum / (float)width + eps);
 #pragma unroll
   for (int i = 0; i < RN_IT; ++i) {
@@ -224,9 +228,10 @@ void launch_residual_norm(const float* x, float alpha, const T* d, const T* gain
     k_residual_norm<T, IT><<<dim3(rows), dim3(256), 0, s>>>(x, alpha, d, gain, offset, xo, xc, dim, width, eps);      \
     return;                                                                                                          \
   }
+  const int cus = lr_num_cus();
   // No more rows than CUs: one memory round trip and a lane's arithmetic are the time, so four columns per lane (x 4096,
-  // us: 8 rows 2.52 -> 2.31, 128 rows 2.98 -> 2.77, 256 rows 3.48 -> 3.36; 1024 rows 6.90 -> 7.30).
-  if (rows <= 256 && dim > 1024 && dim <= 4096) {
+  // us: 8 rows 2.53 -> 2.29, 128 rows 2.90 -> 2.68, 256 rows 3.43 -> 3.26; at 1024 rows 0.4 us slower).
+  if (rows <= (cus > 0 ? cus : 256) && dim > 1024 && dim <= 4096) {
     k_residual_norm<T, 1, 1024><<<dim3(rows), dim3(1024), 0, s>>>(x, alpha, d, gain, offset, xo, xc, dim, width, eps);
     return;
   }

@@ -86,6 +86,19 @@ def test_residual_rmsnorm_at_the_edges_of_the_wide_workgroup(hip, dtype, rows, d
 
 
 @pytest.mark.parametrize("dtype", [F32, BF])
+@pytest.mark.parametrize("dim", [1024, 1032, 2048, 2056, 3072, 4096])
+def test_a_row_of_residual_rmsnorm_does_not_depend_on_the_number_of_rows(hip, dtype, dim):
+    x, d, gain = rnd(700, dim, seed=1), rnd(700, dim, seed=2).to(dtype), (0.3 * rnd(dim, seed=3)).to(dtype)
+    outs = []
+    for rows in (700, 257, 256, 31, 1):
+        xo, xc = torch.empty(rows, dim, device=DEV), torch.empty(rows, dim, dtype=dtype, device=DEV)
+        hip.residual_rmsnorm(x[:rows], 2.5, d[:rows], gain, xo, xc, 1e-5, dim, gain_offset=1.0)
+        outs.append((rows, xo, xc))
+    for rows, xo, xc in outs[1:]:
+        assert torch.equal(xo, outs[0][1][:rows]) and torch.equal(xc, outs[0][2][:rows])
+
+
+@pytest.mark.parametrize("dtype", [F32, BF])
 def test_logit_cap(hip, dtype):
     l = rnd(5, 104, seed=4, dtype=dtype) * 30
     view, before = l[:, :99], l.clone()
