@@ -84,6 +84,7 @@ class GPTBase(nn.Module):
         # of each sequence goes through the final norm and lm_head (prefill saves S-1 rows of it)
         self.last_logits_only = False
         self._ws: Dict[tuple, Workspace] = {}
+        self._shapes = None    # of the bf16 projections (_products), looked up by setup_caches
 
     # -- construction ---------------------------------------------------------------------------
     def _make_block(self, config, layer_idx):
@@ -117,6 +118,8 @@ class GPTBase(nn.Module):
                                       f"{dtype}")
         self._build_caches(max_batch_size, max_seq_length, dtype, device)
         self._ws.clear()
+        self._shapes = None
+        self._sums_bytes(1, 1)
         _hip.device_error_word(device)  # exists before any step is captured into a graph
 
     supported_dtypes = (torch.bfloat16,)
@@ -173,11 +176,11 @@ class GPTBase(nn.Module):
 
     def _products(self, B: int, S: int):
         """(rows, N, K, pair) of every bf16 projection of a (B, S) step, as linear_sums_bytes takes them."""
-        head = B if self.last_logits_only else B * S
-        for name, mod in self.named_modules():
-            if isinstance(mod, nn.Linear) and mod.weight.dtype == torch.bfloat16:
-                leaf = name.rpartition(".")[2]
-                yield head if leaf == "output" else B * S, *mod.weight.shape, leaf == "w1"
+        if self._shapes is None:
+            self._shapes = {(name.rpartition(".")[2], *mod.weight.shape) for name, mod in self.named_modules()
+                            if isinstance(mod, nn.Linear) and mod.weight.dtype == torch.bfloat16}
+        for leaf, N, K in self._shapes:
+            yield B if leaf == "output" and self.last_logits_only else B * S, N, K, leaf == "w1"
 
     def _sums_bytes(self, B: int, S: int) -> int:
         return _hip.linear_sums_bytes(self._products(B, S))
