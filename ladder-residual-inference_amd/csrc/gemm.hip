@@ -194,16 +194,15 @@ struct GemmTile {
 };
 
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
-// One wave instruction: 64 x 16 bytes from memory to LDS at `lds` + 16 * lane.  (s_nop: the wait state between a write of
-// M0 and its use; the scalar operands come from scalar instructions.)
+// One wave instruction: 64 x 16 bytes from memory to LDS at `lds` + 16 * lane.  M0, which holds `lds`, is an operand: the
+// compiler writes it and knows that it did.  (s_nop: the wait state between that and its use; the scalar operands come from
+// scalar instructions.)
 template <bool NT>
 __device__ __forceinline__ void dma16(const i32x4_t& rsrc, int voff, int soff, u32 lds) {
   if (NT)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
-                 : "memory");
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"{m0}"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
   else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
-                 : "memory");
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
 }
 template <int N>
 __device__ __forceinline__ void wait_requests_and_lds() {
