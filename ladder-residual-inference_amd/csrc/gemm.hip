@@ -173,6 +173,7 @@ struct GemmGroup {
   const int32_t* entries;
   int xdiv;
   int64_t wstride;
+  int64_t xrows;           // rows of x
 };
 // Tiles [0, full) are computed whole; each of the `rem` tiles after them is cut along K into `splits` pieces, whose fp32
 // sums go to `part` in the order a wave holds them (k_gemm_sum adds them in order and finishes the tile).
@@ -360,8 +361,8 @@ __global__ __launch_bounds__(256, A16 * BH <= 2 ? 2 : 1) void k_gemm_dma(const u
   const int m0 = mt * T::TM, n0 = nt * (MODE == GEMM_PAIR ? T::TN / 2 : T::TN);
 
   // Requests.  Instruction i of a wave's share of a half covers the half's rows (wave * n + i) * 8 + lane / 8, a lane 16
-  // bytes of one.  Operand rows are read through buffer resources based at the tile's first row; a row beyond M or N has an
-  // offset outside the resource and reads as zero.
+  // bytes of one.  Operand rows are read through buffer resources that hold the tile's rows and no more; a row beyond M or N
+  // has an offset outside the resource and reads as zero.
   const u16* const xb = x + (int64_t)m0 * ldx + kt0 * 64;
   const u16* const wb = w + (int64_t)n0 * K + kt0 * 64;
   constexpr int OUT = (int)0x80000000;
@@ -384,18 +385,21 @@ __global__ __launch_bounds__(256, A16 * BH <= 2 ? 2 : 1) void k_gemm_dma(const u
     }
   }
   const u32 lds0 = __builtin_amdgcn_readfirstlane((u32)(uintptr_t)(__attribute__((address_space(3))) u16*)gsm);
-  auto request = [&](auto ONCE, const u16* base, int voff, int t, u32 lds) {
+  const int64_t xlast = GROUP ? gp.xrows - 1 : (M - m0 < T::TM ? M - m0 : T::TM) - 1;
+  const int64_t wlast = MODE == GEMM_PAIR ? N + (int64_t)(N - n0 < T::TN / 2 ? N - n0 : T::TN / 2) - 1 : (N - n0 < T::TN ? N - n0 : T::TN) - 1;
+  const int xbytes = (int)((xlast * ldx + klen) * 2), wbytes = (int)((wlast * K + klen) * 2);   // (below 2 GiB: gemm_reaches)
+  auto request = [&](auto ONCE, const u16* base, int bytes, int voff, int t, u32 lds) {
     const bool in = t < nk;
     i32x4_t r;
     r.x = (int)(u32)(unsigned long long)base;
     r.y = (int)(u32)((unsigned long long)base >> 32) & 0xffff;
-    r.z = in ? 0x7fffffff : 0;
+    r.z = in ? bytes : 0;
     r.w = 0x00020000;
     if (KTAIL) voff = t * 64 + chunk < klen ? voff : OUT;
     dma16<decltype(ONCE)::value>(r, voff, in ? t * 128 : 0, lds);
   };
-  auto dma_a = [&](int t, int par, int h, int i) { request(std::false_type{}, xb, xo[h][i], t, lds0 + (par * 2 + h) * HA + (wave * NA + i) * 1024); };
-  auto dma_b = [&](int t, int par, int h, int i) { request(std::bool_constant<NT>{}, wb, wo[h][i], t, lds0 + BOFF + (par * 2 + h) * HB + (wave * NB + i) * 1024); };
+  auto dma_a = [&](int t, int par, int h, int i) { request(std::false_type{}, xb, xbytes, xo[h][i], t, lds0 + (par * 2 + h) * HA + (wave * NA + i) * 1024); };
+  auto dma_b = [&](int t, int par, int h, int i) { request(std::bool_constant<NT>{}, wb, wbytes, wo[h][i], t, lds0 + BOFF + (par * 2 + h) * HB + (wave * NB + i) * 1024); };
 
   f32x4_t acc[2 * A16][4 * BH];
 #pragma unroll
@@ -684,7 +688,7 @@ static int gemm_grouped_as(const void* x, int64_t ldx, const void* w, void* y, i
 int gemm_grouped(const void* x, int64_t ldx, int64_t xrows, const void* w, void* y, int64_t ldy, int N, int K, int pair_off, int64_t wstride,
                  const int32_t* tiles, const int32_t* ntiles, const int32_t* entries, int xdiv, int max_tiles, int tile_rows, hipStream_t s) {
   if (xrows * ldx * 2 >= 0x7fffffff || ((int64_t)pair_off + 256) * K * 2 >= 0x7fffffff) return LR_E_UNSUPPORTED;
-  const GemmGroup gp = {tiles, ntiles, entries, xdiv, wstride};
+  const GemmGroup gp = {tiles, ntiles, entries, xdiv, wstride, xrows};
   const bool kt = K % 64 != 0;
   if (tile_rows == 128) {
     if (pair_off)
