@@ -183,7 +183,8 @@ int lr_linear_rope_kv_scratch(const void* x, int64_t ldx, const void* w, void* y
  * M <= 64: lr_linear_multi's LR_EPI_SWIGLU; beyond: the matrix-core GEMM on row PAIRS (a lane holds both
  * halves of a pair).  `scratch` ([M, N] bf16, scratch_bytes >= 2 M N) may be NULL for M <= 64 and for
  * M >= 512 with at least 192 tiles of 256 rows x 128 pairs; it holds the projection where a shape is
- * served by lr_linear followed by lr_swiglu.  Same bits as those two. */
+ * served by lr_linear followed by lr_swiglu.  Same bits as those two.  Where it may not be NULL, I % 8 == 0 and
+ * ldy % 8 == 0, as lr_swiglu has it. */
 int lr_linear_swiglu_out(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K,
                          void* scratch, size_t scratch_bytes, lr_stream_t stream);
 /* The same with memory for partial sums (`sums`), as lr_linear_scratch is lr_linear. */

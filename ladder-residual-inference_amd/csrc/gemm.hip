@@ -827,7 +827,8 @@ extern "C" int lr_linear_swiglu_out_scratch(const void* x, int64_t ldx, const vo
   const bool large = M >= 512 && I >= 128 && (int64_t)((M + 255) / 256) * ((I + 127) / 128) >= 192 && gemm_reaches(ldx, I, K, GEMM_PAIR);
   if (!large && !(M <= 64 && sums)) {
     LR_REQUIRE_PTR(scratch);
-    if (scratch_bytes < (size_t)M * N * sizeof(u16)) return LR_E_SHAPE;
+    if (scratch_bytes < (size_t)M * N * sizeof(u16) || M > 65535 * 64) return LR_E_SHAPE;
+    if (I % 8 || ldy % 8) return LR_E_ALIGN;
   }
   int rc = gemm(x, ldx, w, y, ldy, M, I, K, GEMM_PAIR, GemmRope{}, sums, sums_bytes, (hipStream_t)stream);
   if (rc != LR_E_UNSUPPORTED || scratch == nullptr || scratch_bytes < (size_t)M * N * sizeof(u16)) return rc;

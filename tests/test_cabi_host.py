@@ -334,3 +334,22 @@ def test_partial_sums_of_the_mlp_are_limited_where_that_was_measured(lib, family
     ws = meta_model(family, name)._new_workspace(B, 1)
     assert ws.sums_mlp is not ws.sums and ws.sums_mlp._base is None
     assert ws.sums_mlp.numel() == (min(ws.sums.numel(), 200 << 15) if B <= 64 else ws.sums.numel())
+
+
+def test_swiglu_projection_of_many_rows_refuses_what_its_two_calls_refuse(lib):
+    """More than 64 rows on a small grid are specified as lr_linear into `scratch` and lr_swiglu: scratch of the projection's
+    size, multiples of 8 columns, and no more rows than lr_swiglu takes -- with memory for partial sums or without."""
+    E_NULL, E_ALIGN, E_SHAPE = -1, -2, -3
+    p, big = 4096, 1 << 40
+
+    def call(M, N, ldy, scratch, n, sums):
+        return lib.lr_linear_swiglu_out_scratch(p, 64, p, p, ldy, M, N, 64, scratch, n, sums, 1 << 20 if sums else 0, None)
+
+    for sums in (None, p):
+        assert call(65, 48, 24, None, 0, sums) == E_NULL
+        assert call(65, 48, 24, 8, big, sums) == E_ALIGN
+        assert call(65, 48, 24, p, 2 * 65 * 48 - 1, sums) == E_SHAPE
+        assert call(65, 36, 24, p, big, sums) == E_ALIGN            # 18 pairs
+        assert call(65, 48, 25, p, big, sums) == E_ALIGN            # rows of 25 elements
+        assert call(65535 * 64 + 1, 48, 24, p, big, sums) == E_SHAPE
+    assert lib.lr_linear_swiglu_out(p, 64, p, p, 24, 65, 36, 64, p, big, None) == E_ALIGN
