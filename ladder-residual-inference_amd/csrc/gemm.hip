@@ -715,7 +715,7 @@ static int linear_rows(const void* x, int64_t ldx, const void* w, void* y, int64
   if (K % 8 || ldx % 8) return LR_E_ALIGN;
   if (M <= 4 || ((act_swiglu || gemv_cfg) && M <= 8))
     return lr_gemv_dispatch(x, ldx, w, y, ldy, M, N, K, act_swiglu, gemv_cfg, s);
-  if (!act_swiglu && M <= 64 && !(M >= GEMM_SCRATCH_FROM && scratch)) {
+  if (!act_swiglu && M <= 64 && !(M >= GEMM_SCRATCH_FROM && scratch && gemm_reaches(ldx, N, K, GEMM_PLAIN))) {
     // decode batches: the weight-streaming matrix-core kernel (stream_gemm.hip); shapes it declines fall through
     lr_projection_t pr;
     pr.x = x; pr.ldx = ldx; pr.w = w; pr.y = y; pr.ldy = ldy; pr.N = N; pr.K = K; pr.epilogue = LR_EPI_NONE; pr.rope = nullptr;
@@ -817,7 +817,8 @@ extern "C" int lr_linear_swiglu_out_scratch(const void* x, int64_t ldx, const vo
   if (M <= 0 || N <= 0 || K <= 0 || N % 2 || ldx < K || ldy < N / 2) return LR_E_SHAPE;
   if (K % 8 || ldx % 8) return LR_E_ALIGN;
   const int I = N / 2;
-  if (M <= 64 && !(M >= GEMM_SCRATCH_FROM && sums)) {
+  const bool product = M <= 64 && M >= GEMM_SCRATCH_FROM && sums && gemm_reaches(ldx, I, K, GEMM_PAIR);   // of a decode batch
+  if (M <= 64 && !product) {
     lr_projection_t pr;
     pr.x = x; pr.ldx = ldx; pr.w = w; pr.y = y; pr.ldy = ldy; pr.N = N; pr.K = K; pr.epilogue = LR_EPI_SWIGLU; pr.rope = nullptr;
     const int rc = lr_linear_multi(&pr, 1, M, stream);
@@ -825,7 +826,7 @@ extern "C" int lr_linear_swiglu_out_scratch(const void* x, int64_t ldx, const vo
   }
   // (a caller of other than large problems brings `scratch` [M, N]; used where the weights are out of the requests' reach)
   const bool large = M >= 512 && I >= 128 && (int64_t)((M + 255) / 256) * ((I + 127) / 128) >= 192 && gemm_reaches(ldx, I, K, GEMM_PAIR);
-  if (!large && !(M <= 64 && sums)) {
+  if (!large && !product) {
     LR_REQUIRE_PTR(scratch);
     if (scratch_bytes < (size_t)M * N * sizeof(u16) || M > 65535 * 64) return LR_E_SHAPE;
     if (I % 8 || ldy % 8) return LR_E_ALIGN;

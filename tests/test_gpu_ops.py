@@ -905,3 +905,27 @@ def test_linear_rope_kv_pieces(hip, B, S, Hq, Hkv, hd, K):
     hip.linear_rope_kv(x, w, out[1], table, pos, kc[1], vc[1], B, S, Hq, Hkv, hd, sums)
     assert torch.equal(out[0], out[1]) and torch.equal(kc[0], kc[1]) and torch.equal(vc[0], vc[1])
     hip.raise_on_device_error(out[0].device)
+
+
+def test_decode_batches_beyond_the_reach_of_the_gemm_stay_with_the_bands(hip):
+    """A tile of 256 rows this far apart is out of the reach of a 2 GiB offset, 64 of them are not: with memory for partial
+    sums or without, the weight-streaming kernel serves them, to the same bits."""
+    M, K, ld = 40, 64, (1 << 22) + 8
+    wide = torch.zeros((M - 1) * ld + K, dtype=BF, device=DEV)
+    x = wide.as_strided((M, K), (ld, 1))
+    x.copy_(rnd(M, K, seed=70))
+    sums = torch.empty(1 << 20, dtype=torch.uint8, device=DEV)
+    w = rnd(48, K, seed=71)
+    plain, act = torch.empty(M, 48, dtype=BF, device=DEV), torch.empty(M, 24, dtype=BF, device=DEV)
+    want, want_act = torch.empty_like(plain), torch.empty_like(act)
+    hip.linear_multi((x.contiguous(), w, want, hip.EPI_NONE))
+    hip.linear_multi((x.contiguous(), w, want_act, hip.EPI_SWIGLU))
+    hip.linear(x, w, plain, scratch=sums)
+    hip.linear_swiglu_out(x, w, act, sums=sums)
+    assert torch.equal(plain, want) and torch.equal(act, want_act)
+    kc, vc = (torch.zeros(M, 1, 8, 8, dtype=BF, device=DEV) for _ in range(2))
+    pos, table = torch.tensor([3], dtype=torch.int32, device=DEV), O.rope_table(8, 8, 500000, BF).to(DEV)
+    hip.linear_rope_kv(x, w, plain, table, pos, kc, vc, M, 1, 4, 1, 8, sums)
+    hip.rope_kv_write(want, table, False, pos, *(torch.empty_like(kc) for _ in range(2)), M, 1, 4, 1, 8)
+    assert torch.equal(plain, want) and torch.equal(vc[:, 0, 3], want[:, 40:])
+    hip.raise_on_device_error(plain.device)
