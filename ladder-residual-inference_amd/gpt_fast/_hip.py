@@ -255,13 +255,16 @@ def linear_sums_bytes(products) -> int:
 
 
 def _scratch_args(t):
-    return (None, 0) if t is None else (t.data_ptr(), t.numel() * t.element_size())
+    if t is None:
+        return None, 0
+    assert t.is_contiguous(), "memory for partial sums is one piece"
+    return _dev(t, t.dtype), t.numel() * t.element_size()
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, act_swiglu: bool = False, gemv_cfg: int = 0, scratch=None):
     """out[M, N] = x[M, K] @ w[N, K]^T (x = [u | g] of width 2K when act_swiglu).  gemv_cfg != 0 goes
     through lr_linear_tuned (an explicit GEMV launch configuration for this one call).  `scratch`: device memory for partial
-    sums (linear_scratch_bytes), not shared with calls that may overlap."""
+    sums (linear_scratch_bytes), not shared with calls that may overlap; act_swiglu, gemv_cfg and fp32 take none."""
     M, xc, ldx = _rows_ld(x)
     N, K = w.shape
     assert w.is_contiguous() and xc == (2 * K if act_swiglu else K), (x.shape, w.shape, act_swiglu)

@@ -353,3 +353,12 @@ def test_swiglu_projection_of_many_rows_refuses_what_its_two_calls_refuse(lib):
         assert call(65, 48, 25, p, big, sums) == E_ALIGN            # rows of 25 elements
         assert call(65535 * 64 + 1, 48, 24, p, big, sums) == E_SHAPE
     assert lib.lr_linear_swiglu_out(p, 64, p, p, 24, 65, 36, 64, p, big, None) == E_ALIGN
+
+
+def test_only_contiguous_device_memory_is_handed_on_for_partial_sums():
+    from gpt_fast import _hip
+
+    assert _hip._scratch_args(None) == (None, 0)
+    for t in (torch.empty(64, dtype=torch.uint8), torch.empty(1, dtype=torch.uint8).expand(64), torch.empty(64)[::2]):
+        with pytest.raises(AssertionError):
+            _hip._scratch_args(t)
