@@ -586,11 +586,12 @@ constexpr size_t GEMM_SCRATCH = (size_t)64 << 20;   // pieces of one round of th
 constexpr int GEMM_SCRATCH_FROM = 33;               // rows from which a projection that has memory for pieces is one of this file's
 
 static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
+  GemmPlan best{-1, 0, 0, 1};
+  if (M > 0x7fffffff - 256 || N > 0x7fffffff - 256 || K > 0x7fffffff - 256) return best;   // (row, column and k of the last tile are ints)
   int cus = lr_num_cus();
   if (cus <= 0) cus = 256;
   const int nk = (K + 63) / 64;
   const float weights_us = (float)N * (mode == GEMM_PAIR ? 2 : 1) * K * 2 / 5.5e6f;
-  GemmPlan best{-1, 0, 0, 1};
   float best_us = 0;
   for (int c = 0; c < 4; ++c) {
     const GemmTileCost& t = GEMM_TILES[c];

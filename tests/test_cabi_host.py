@@ -362,3 +362,22 @@ def test_only_contiguous_device_memory_is_handed_on_for_partial_sums():
     for t in (torch.empty(64, dtype=torch.uint8), torch.empty(1, dtype=torch.uint8).expand(64), torch.empty(64)[::2]):
         with pytest.raises(AssertionError):
             _hip._scratch_args(t)
+
+
+def test_gemm_plan_covers_every_tile_and_refuses_sizes_beyond_its_integers(lib):
+    from gpt_fast import _hip
+
+    p = _hip._LinearPlan()
+    big = 0x7fffffff
+    for M, N, K in ((big, 8, 8), (8, big, 8), (8, 8, big - 7), (big - 255, 8, 8), (1 << 30, 1 << 30, 8)):
+        assert lib.lr_linear_plan(M, N, K, 0, 0, ctypes.byref(p)) == -4, (M, N, K)
+    assert lib.lr_linear_plan(8, 7, 8, 1, 0, ctypes.byref(p)) == -3 and lib.lr_linear_plan(0, 8, 8, 0, 0, ctypes.byref(p)) == -3
+    assert lib.lr_linear_plan(8, 8, 12, 0, 0, ctypes.byref(p)) == -2 and lib.lr_linear_plan(8, 8, 8, 0, 0, None) == -1
+    for M in (1, 33, 65, 777, 16384):
+        for N, K in ((8, 8), (1280, 8192), (28672, 4096), (4096, 14336)):
+            for pair in (False, True):
+                for scratch in (0, 1 << 20, 64 << 20):
+                    p = _hip.linear_plan(M, N, K, pair, scratch)
+                    assert p.whole + p.cut == -(-M // p.tile_rows) * -(-N // p.tile_cols)
+                    assert p.sums_bytes == p.cut * p.pieces * p.tile_rows * p.tile_cols * 4 <= scratch
+                    assert (p.pieces == 1) == (p.cut == 0) and p.pieces <= -(-K // 128)
