@@ -855,9 +855,9 @@ def test_stream_read_runs_and_leaves_the_sink_alone(hip):
 @pytest.mark.parametrize("M,N,K", [
     (33, 264, 520), (64, 1280, 8192), (40, 24, 64),      # decode batches: with memory for sums 64-row tiles
     (65, 8, 8), (100, 72, 64), (129, 264, 520), (256, 256, 128), (257, 512, 192), (300, 520, 200), (513, 40, 4096),
-    (777, 1032, 1000),                                   # one row, column or k too many for every tile; odd numbers of k-tiles
-    (128, 1024, 8192), (300, 2048, 4160), (777, 2048, 7168),   # cut along K where there is memory for it: 128 x 128,
-    (2100, 2560, 8192),                                        # 128 x 256 and 256 x 256 tiles; whole rounds first
+    (777, 1032, 1000),                                   # 64-row tiles: a row, column or k too many; odd numbers of k-tiles
+    (128, 1024, 8192), (300, 2048, 4160), (777, 2048, 7168),   # cut along K where there is memory for it: tiles of 64 x 128,
+    (2100, 2560, 8192),                                        # 128 x 128, 128 x 256 and 256 x 256
 ])
 def test_linear_tiles_and_pieces(hip, M, N, K):
     """Whole tiles, and tiles cut along K with their sums added by a second launch, against the float64 product: fp32
@@ -876,12 +876,66 @@ def test_linear_tiles_and_pieces(hip, M, N, K):
     assert torch.equal(outs[1], outs[2])
 
 
+def gemm_kind(plan):
+    return (plan.tile_rows, plan.tile_cols), "whole" if not plan.cut else "mixed" if plan.whole else "cut"
+
+
+# every tile with whole tiles only, with cut ones only and with both (64 x 128: never both); rows, columns and K that are no
+# whole tiles anywhere
+@pytest.mark.parametrize("tile,kind,M,N,K", [
+    ((64, 128), "whole", 43, 7, 72), ((64, 128), "cut", 70, 7, 2280),
+    ((128, 128), "whole", 5529, 279, 136), ((128, 128), "cut", 1730, 7, 3896), ((128, 128), "mixed", 5950, 1295, 2016),
+    ((128, 256), "whole", 5596, 655, 72), ((128, 256), "cut", 5424, 143, 2864), ((128, 256), "mixed", 796, 9583, 2016),
+    ((256, 256), "whole", 804, 9503, 72), ((256, 256), "cut", 385, 5415, 5304), ((256, 256), "mixed", 1762, 9351, 936),
+])
+def test_linear_of_every_tile_whole_and_cut(hip, tile, kind, M, N, K):
+    sums = torch.empty(hip.linear_scratch_bytes(M), dtype=torch.uint8, device=DEV)
+    with_sums = gemm_kind(hip.linear_plan(M, N, K)) == (tile, kind)
+    assert with_sums or gemm_kind(hip.linear_plan(M, N, K, scratch_bytes=0)) == (tile, kind)
+    x, w = rnd(M, K, seed=90), rnd(N, K, seed=91, scale=K ** -0.5)
+    want = (x.double() @ w.double().T).to(BF)
+    y = torch.full((M + 1, N + 8), 5.0, dtype=BF, device=DEV)
+    hip.linear(x, w, y[:M, :N], scratch=sums if with_sums else sums[:0])
+    assert_close_ulp(y[:M, :N].contiguous(), want, what=f"{M} x {N} x {K}")
+    assert (y[M:] == 5.0).all() and (y[:, N:] == 5.0).all()
+
+
+@pytest.mark.parametrize("tile,kind,M,I,K", [
+    ((64, 128), "whole", 43, 8, 72), ((64, 128), "cut", 70, 8, 2280),
+    ((128, 128), "whole", 137, 5776, 136), ((128, 128), "cut", 1730, 8, 3896), ((128, 128), "mixed", 2409, 1696, 2232),
+    ((128, 256), "whole", 203, 8312, 72), ((128, 256), "cut", 5999, 72, 3016), ((128, 256), "mixed", 545, 6600, 1960),
+    ((256, 256), "whole", 529, 6640, 72), ((256, 256), "cut", 2747, 456, 5400), ((256, 256), "mixed", 5927, 1352, 1048),
+])
+def test_linear_swiglu_out_of_every_tile_whole_and_cut(hip, tile, kind, M, I, K):
+    with_sums = gemm_kind(hip.linear_plan(M, 2 * I, K, True)) == (tile, kind)
+    assert with_sums or gemm_kind(hip.linear_plan(M, 2 * I, K, True, 0)) == (tile, kind)
+    check_swiglu_out(hip, M, I, K, hip.linear_scratch_bytes(M) if with_sums else 0)
+
+
+@pytest.mark.parametrize("tile,kind,B,S,Hq,Hkv,hd,K", [
+    ((64, 128), "cut", 5, 14, 1, 1, 8, 2280), ((128, 128), "whole", 3, 1843, 31, 2, 8, 136),
+    ((128, 128), "cut", 5, 346, 1, 1, 8, 3896), ((128, 128), "mixed", 7, 850, 65, 8, 16, 2016),
+    ((128, 256), "whole", 4, 1399, 37, 2, 16, 72), ((128, 256), "cut", 3, 1808, 14, 2, 8, 2864),
+    ((128, 256), "mixed", 4, 199, 583, 8, 16, 2016), ((256, 256), "whole", 4, 201, 281, 8, 32, 72),
+    ((256, 256), "cut", 5, 77, 661, 8, 8, 5304), ((256, 256), "mixed", 2, 881, 1153, 8, 8, 936),
+])
+def test_linear_rope_kv_of_every_tile_whole_and_cut(hip, tile, kind, B, S, Hq, Hkv, hd, K):
+    M, N = B * S, (Hq + 2 * Hkv) * hd
+    with_sums = gemm_kind(hip.linear_plan(M, N, K)) == (tile, kind)
+    assert with_sums or gemm_kind(hip.linear_plan(M, N, K, scratch_bytes=0)) == (tile, kind)
+    check_rope_kv(hip, B, S, Hq, Hkv, hd, K, hip.linear_scratch_bytes(M) if with_sums else 0)
+
+
 @pytest.mark.parametrize("M,I,K", [(40, 1000, 2056), (128, 512, 4096), (300, 1000, 4104), (777, 2048, 4096)])
 def test_linear_swiglu_out_pieces(hip, M, I, K):
     """[up; gate] pairs in cut tiles: the activation after the sums are complete."""
+    check_swiglu_out(hip, M, I, K, hip.linear_scratch_bytes(M))
+
+
+def check_swiglu_out(hip, M, I, K, sums_bytes):
     x, w1 = rnd(M, K, seed=92), rnd(2 * I, K, seed=93, scale=K ** -0.5)
     act, h = torch.empty(M, I, dtype=BF, device=DEV), torch.empty(M, 2 * I, dtype=BF, device=DEV)
-    hip.linear_swiglu_out(x, w1, act, h, torch.empty(hip.linear_scratch_bytes(M), dtype=torch.uint8, device=DEV))
+    hip.linear_swiglu_out(x, w1, act, h, torch.empty(max(16, sums_bytes), dtype=torch.uint8, device=DEV)[:sums_bytes])
     u, g = (x.double() @ w1.double().T).to(BF).float().chunk(2, 1)
     want = ((g / (1 + torch.exp(-g))).to(BF).float() * u).to(BF)
     # up, gate and silu(gate) are each rounded: one step of any of them is at most 2^-7 of the result
@@ -892,9 +946,13 @@ def test_linear_swiglu_out_pieces(hip, M, I, K):
 @pytest.mark.parametrize("B,S,Hq,Hkv,hd,K", [(48, 1, 8, 2, 64, 4096), (1, 128, 8, 2, 64, 4096), (3, 100, 4, 1, 128, 4104), (2, 389, 16, 4, 128, 4096)])
 def test_linear_rope_kv_pieces(hip, B, S, Hq, Hkv, hd, K):
     """The q/k/v projection in cut tiles, rotated and cached after the sums: the two calls on the same plan, bit for bit."""
+    check_rope_kv(hip, B, S, Hq, Hkv, hd, K, hip.linear_scratch_bytes(B * S))
+
+
+def check_rope_kv(hip, B, S, Hq, Hkv, hd, K, sums_bytes):
     N, Smax, start = (Hq + 2 * Hkv) * hd, S + 11, 5
     x, w = rnd(B * S, K, seed=94), rnd(N, K, seed=95, scale=K ** -0.5)
-    sums = torch.empty(hip.linear_scratch_bytes(B * S), dtype=torch.uint8, device=DEV)
+    sums = torch.empty(max(16, sums_bytes), dtype=torch.uint8, device=DEV)[:sums_bytes]
     pos = torch.arange(start, start + S, dtype=torch.int32, device=DEV)
     table = O.rope_table(start + S, hd, 500000, BF).to(DEV)
     out = [torch.empty(B * S, N, dtype=BF, device=DEV) for _ in range(2)]
