@@ -120,6 +120,64 @@ def test_a_batch_gives_every_sequence_what_it_gets_alone(case, dtype, batch):
         agrees(s.feed([r], [60])[0], g, dtype)
 
 
+@pytest.mark.parametrize("case", ["mixed", "odd", "large", "experts"])
+@pytest.mark.parametrize("batch", [33, 48, 70])
+def test_decode_batches_above_32_run_products(case, batch, monkeypatch):
+    """The products' route of dense layers in a decode step: every sequence as alone, and captured steps replay the eager
+    ones, bit for bit."""
+    from gpt_fast import _hip
+
+    s, cfg = served(case, BF, batch=batch)
+    launches = []
+    tanh = _hip.linear_residual_tanh
+    monkeypatch.setattr(_hip, "linear_residual_tanh", lambda *a: (launches.append(a), tanh(*a))[1])
+    rows = [C.tokens(cfg, 40, seed=i) for i in range(batch)]
+    got = s.feed(rows, [31] + [1] * 9)
+    assert not launches
+    for r, g in list(zip(rows, got))[::8]:
+        agrees(g, s.want(r), BF)
+        agrees(s.feed([r], [40])[0], g, BF)
+    replays_equal_eager(s, rows, 31)
+
+
+def replays_equal_eager(s, rows, T):
+    idx = torch.tensor(rows, dtype=torch.int32, device=DEV)
+    tok, pos = idx[:, :1].clone(), torch.tensor([T], dtype=torch.int32, device=DEV)
+
+    def start():
+        with torch.no_grad():
+            s.model(idx[:, :T].contiguous(), torch.arange(T, dtype=torch.int32, device=DEV))
+
+    def step():
+        with torch.no_grad():
+            return s.model(tok, pos)
+
+    start()
+    eager = []
+    for t in range(T, T + 4):
+        tok.copy_(idx[:, t:t + 1])
+        pos.fill_(t)
+        eager.append(step().clone())
+    start()
+    states = [x.clone() for x in s.model.recurrent_states()]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for x, y in zip(s.model.recurrent_states(), states):
+        x.copy_(y)
+    for t in range(T, T + 4):
+        tok.copy_(idx[:, t:t + 1])
+        pos.fill_(t)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager[t - T]), t
+
+
 @pytest.mark.parametrize("dtype", [F32, BF])
 def test_a_slot_is_used_again_without_a_trace_of_the_last_sequence(dtype):
     s, cfg = served("mixed", dtype)

@@ -99,6 +99,30 @@ def test_a_batch_gives_every_sequence_what_it_gets_alone(case, dtype):
         assert err(s.feed([r], [60])[0], g) < TOL[dtype]
 
 
+@pytest.mark.parametrize("case", ["mixed", "odd", "large"])
+@pytest.mark.parametrize("batch", [33, 48, 70])
+def test_decode_batches_above_32_run_products(case, batch, monkeypatch):
+    """The products' route of a decode step: every sequence as alone, and captured steps replay the eager ones, bit for bit."""
+    from gpt_fast import _hip
+    from test_gpu_gepolix_model import each, replays_equal_eager
+
+    s, cfg = served(case, BF, batch=batch)
+    launches = []
+    multi = _hip.linear_multi
+    monkeypatch.setattr(_hip, "linear_multi", lambda *a: (launches.append(a), multi(*a))[1])
+    rows = [C.tokens(cfg, 40, seed=i) for i in range(batch)]
+    got = s.feed(rows, [31] + [1] * 9)
+    assert not launches
+    # Single positions differ from float64 by up to 0.27 (a norm of a residual that nearly cancels), one sequence alone exactly
+    # as in a batch: nearly all must agree closely with float64, and all that do must agree with the sequence alone.
+    for r, g in list(zip(rows, got))[::8]:
+        want = s.want(r)
+        off, apart = each(g, want), each(s.feed([r], [40])[0], g)
+        assert off.median() < TOL[BF] / 2 and (off < TOL[BF]).double().mean() >= 0.9
+        assert (apart[off < TOL[BF]] < TOL[BF]).all()
+    replays_equal_eager(s, rows, 31)
+
+
 @pytest.mark.parametrize("dtype", [F32, BF])
 def test_a_slot_is_used_again_without_a_trace_of_the_last_sequence(dtype):
     s, cfg = served("mixed", dtype)

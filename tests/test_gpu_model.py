@@ -192,13 +192,74 @@ def test_tiny_ladder_per_op_decode_modes(B, mode):
 
 
 def test_tiny_ladder_mlp_chain_as_a_parallel_graph_branch():
-    """Above 16 sequences the MLP chain can run beside the attention chain as a second branch of the captured graph
-    (the default from 33 sequences on): same tokens and logits as the oracle, replays equal to eager."""
+    """Above 16 sequences the MLP chain can run beside the attention chain as a second branch of the captured graph, up to
+    32 in bands: same tokens and logits as the oracle, replays equal to eager.  (The default, from 33 sequences on and without
+    bands: test_decode_batches_above_32_run_products_with_partial_sums.)"""
     model = build("ladder", **dict(TINY, dim=512, n_head=8, n_local_heads=2, intermediate_size=640))
     model.two_chains_from = 17
     stats = run_parity(model, "ladder", B=20, T=20, new=12, fused=False)
     print(stats)
     check(stats)
+
+
+WIDER = dict(TINY, dim=512, n_head=8, n_local_heads=2, intermediate_size=2560)   # K long enough to be cut
+PATTERN = [{"attention": True, "mlp": False}, {"attention": False, "mlp": True}, {"attention": False, "mlp": False}]
+
+
+def wider(family):
+    shard = dict(reduce_pattern=PATTERN, tp_world_size=2, intermediate_size=5120)
+    return build(family, **(dict(WIDER, **shard) if family == "desync" else WIDER))
+
+
+@pytest.mark.parametrize("family", ["ladder", "dense", "desync", "parallel"])
+@pytest.mark.parametrize("B", [33, 40, 64, 70])
+def test_decode_batches_above_32_run_products_with_partial_sums(family, B):
+    """Their default route (the ladder's up to 64 with the MLP chain as a second branch of the captured graph): the oracle's
+    tokens and logits, replays equal to eager steps."""
+    from gpt_fast import _hip
+
+    model = wider(family)
+    model.setup_caches(B, 32)
+    assert any(_hip.linear_plan(*p).cut for p in model._products(B, 1))
+    stats = run_parity(model, family, B=B, T=20, new=12)
+    print(family, B, stats)
+    check(stats)
+    assert stats["graph_equals_eager"]
+
+
+@pytest.mark.parametrize("family", ["ladder", "dense", "desync", "parallel"])
+@pytest.mark.parametrize("B", [33, 48])
+@torch.no_grad()
+def test_decode_batches_above_32_equal_the_bands(family, B, monkeypatch):
+    """Different sequences in every row: products with partial sums against the weight-streaming bands that serve up to 32
+    rows, the same tokens fed: logits and caches within the tolerance of two summation orders."""
+    from gpt_fast import _hip
+
+    model = wider(family)
+    model.setup_caches(B, 32)
+    toks = torch.randint(0, 512, (B, 10), device=DEV, generator=torch.Generator(device=DEV).manual_seed(3))
+    launches = []
+    multi = _hip.linear_multi
+    monkeypatch.setattr(_hip, "linear_multi", lambda *a: (launches.append(len(a)), multi(*a))[1])
+
+    def steps(rows_to):
+        model.band_rows_to, model.two_chains_from = rows_to, rows_to + 1
+        launches.clear()
+        out = [model(toks[:, :6], torch.arange(6, device=DEV)).clone()]
+        for t in range(6, 10):
+            out.append(model(toks[:, t:t + 1], torch.tensor([t], device=DEV)).clone())
+        model.check_device_errors()
+        kv = model.layers[-1].attention.kv_cache
+        return out, kv.k_cache[:B, :, :10].clone(), kv.v_cache[:B, :, :10].clone()
+
+    sums, ks, vs = steps(32)
+    assert not launches
+    bands, kb, vb = steps(64)
+    assert launches
+    assert torch.equal(sums[0], bands[0])
+    for a, b in zip(sums[1:], bands[1:]):
+        assert rel_err(b, a) <= REL_TOL
+    assert rel_err(kb, ks) <= REL_TOL and rel_err(vb, vs) <= REL_TOL
 
 
 def test_tiny_ladder_fused_head_dim_128_many_kv_heads():
