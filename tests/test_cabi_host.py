@@ -381,3 +381,33 @@ def test_gemm_plan_covers_every_tile_and_refuses_sizes_beyond_its_integers(lib):
                     assert p.whole + p.cut == -(-M // p.tile_rows) * -(-N // p.tile_cols)
                     assert p.sums_bytes == p.cut * p.pieces * p.tile_rows * p.tile_cols * 4 <= scratch
                     assert (p.pieces == 1) == (p.cut == 0) and p.pieces <= -(-K // 128)
+
+
+def test_products_with_memory_for_partial_sums_refuse_what_the_ones_without_refuse(lib):
+    """Only refusals: nothing here may reach a launch."""
+    from gpt_fast._hip import _RopeKv
+
+    E_NULL, E_ALIGN, E_SHAPE = -1, -2, -3
+    p = 4096
+    rope = _RopeKv(p, p, p, p, None, 8, 1, 128, 64, 64)      # N = (8 + 2) * 128 = 1280
+
+    def linear(x=p, ldx=64, w=p, y=p, ldy=48, M=40, N=48, K=64, scratch=p):
+        return lib.lr_linear_scratch(x, ldx, w, y, ldy, M, N, K, scratch, 1 << 20, None)
+
+    def fused(x=p, ldx=64, y=p, ldy=1280, M=40, K=64, S=1, r=rope, scratch=p):
+        return lib.lr_linear_rope_kv_scratch(x, ldx, p, y, ldy, M, K, S, None if r is None else ctypes.byref(r), scratch, 1 << 20, None)
+
+    def swiglu(x=p, ldx=64, y=p, ldy=24, M=40, N=48, K=64, scratch=None, sums=p):
+        return lib.lr_linear_swiglu_out_scratch(x, ldx, p, y, ldy, M, N, K, scratch, 0, sums, 1 << 20, None)
+
+    for call in (linear, fused, swiglu):
+        assert call(x=None) == E_NULL and call(y=None) == E_NULL
+        assert call(x=p + 8) == E_ALIGN and call(y=p + 2) == E_ALIGN
+        assert call(M=0) == E_SHAPE and call(K=0) == E_SHAPE and call(ldx=56) == E_SHAPE and call(ldy=16) == E_SHAPE
+        assert call(K=60) == E_ALIGN and call(ldx=68) == E_ALIGN
+    assert linear(w=None) == E_NULL and linear(scratch=p + 8) == E_ALIGN and fused(scratch=p + 8) == E_ALIGN
+    assert swiglu(sums=p + 8) == E_ALIGN and swiglu(N=47) == E_SHAPE
+    assert fused(r=None) == E_NULL and fused(M=41, S=2) == E_SHAPE and fused(ldy=1284) == E_ALIGN
+    # the projection's buffer may be missing for up to 64 rows and for large grids, not in between
+    for M, N in ((65, 48), (511, 1 << 16), (1536, 7936)):      # (186 tiles of 256 rows x 128 pairs)
+        assert swiglu(M=M, N=N, ldy=N // 2) == E_NULL

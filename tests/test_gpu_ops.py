@@ -943,6 +943,20 @@ def check_swiglu_out(hip, M, I, K, sums_bytes):
     assert (ulp_diff(act, want) > 0).float().mean().item() < 0.05
 
 
+@pytest.mark.parametrize("M,I,K", [(33, 17, 64), (64, 1000, 520), (512, 12288, 64), (1536, 4090, 136)])
+def test_linear_swiglu_out_without_a_buffer_for_the_projection(hip, M, I, K):
+    """Up to 64 rows, and from 192 tiles of 256 rows x 128 pairs on: any number of pairs, the same bits as with a buffer."""
+    x, w1 = rnd(M, K, seed=96), rnd(2 * I, K, seed=97, scale=K ** -0.5)
+    sums = torch.empty(max(16, hip.linear_scratch_bytes(M)), dtype=torch.uint8, device=DEV)
+    got, want = (torch.full((M, I + 3), 5.0, dtype=BF, device=DEV) for _ in range(2))
+    hip.linear_swiglu_out(x, w1, got[:, :I], sums=sums)
+    hip.linear_swiglu_out(x, w1, want[:, :I], torch.empty(M, 2 * I, dtype=BF, device=DEV), sums)
+    assert torch.equal(got, want) and (got[:, I:] == 5.0).all()
+    u, g = (x.double() @ w1.double().T).to(BF).float().chunk(2, 1)
+    ref = ((g / (1 + torch.exp(-g))).to(BF).float() * u).to(BF)
+    assert ((got[:, :I].float() - ref.float()).abs() <= 2.0 ** -7 * 3 * ref.float().abs() + 2.0 ** -12).all()
+
+
 @pytest.mark.parametrize("B,S,Hq,Hkv,hd,K", [(48, 1, 8, 2, 64, 4096), (1, 128, 8, 2, 64, 4096), (3, 100, 4, 1, 128, 4104), (2, 389, 16, 4, 128, 4096)])
 def test_linear_rope_kv_pieces(hip, B, S, Hq, Hkv, hd, K):
     """The q/k/v projection in cut tiles, rotated and cached after the sums: the two calls on the same plan, bit for bit."""
