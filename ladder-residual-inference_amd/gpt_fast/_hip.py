@@ -231,6 +231,12 @@ def ladder_norms(resid_in, d1, d2, gain1, gain2, resid_out, normed1, normed2, ep
                                   _dev(normed2), rows, dim, float(eps), _stream()), "lr_ladder_norms")
 
 
+# Rows of a decode step up to which the weight-streaming bands are the faster kernel for projections that could have
+# partial sums, as in lr_linear_scratch_bytes.  ms per step, 33 rows, bands / products: ladder 1B 1.43 / 1.23, 8B 5.71 /
+# 4.55, 70B rank shard 7.98 / 6.25; Lasivik 1B 1.99 / 1.70, 8B 7.11 / 5.52; Gepolix 1B 2.03 / 1.77, 8B 7.49 / 6.62.
+BANDS_TO = 32
+
+
 def linear_scratch_bytes(rows: int) -> int:
     return int(load().lr_linear_scratch_bytes(rows))
 

@@ -225,10 +225,10 @@ class GPTBase(nn.Module):
     band_rows_from = 2
     # and up to which: above, the GEMM with its partial sums is the faster one (64 rows of the 70B rank shard, us: up/gate
     # 38.9 in bands / 30.7, q/k/v 23.6 / 14.8, w2 23.0 / 18.6, wo 13.9 / 10.7)
-    band_rows_to = 32
+    band_rows_to = _hip.BANDS_TO
 
     def _decode_bands(self, ws: Workspace, *linears) -> bool:
-        """A decode step of up to 32 rows on bf16 weights: every projection of a block is a launch of the
+        """A decode step of up to band_rows_to rows on bf16 weights: every projection of a block is a launch of the
         weight-streaming kernel (lr_linear_multi), the q/k/v one rotating and caching on its way out and the up/gate one
         storing silu(gate) * up -- also below 5 rows, where lr_linear alone would pick the matrix-vector kernel: fewer
         launches per block weigh more than the kernel.  (`linears`: the modules

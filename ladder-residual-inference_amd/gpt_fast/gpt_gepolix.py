@@ -118,7 +118,7 @@ class GPTGepolix(GPTHybrid):
         included."""
         proj = ws.proj[:, :blk.mixer.proj_cols]
         w = blk.mixer.in_proj.weight
-        if ws.xc.dtype == torch.bfloat16 and ws.rows <= (64 if routed is not None else 32):
+        if ws.xc.dtype == torch.bfloat16 and ws.rows <= (64 if routed is not None else _hip.BANDS_TO):
             todo = [(ws.xc, w, proj, _hip.EPI_NONE)]
             if blk.w1 is not None:
                 todo.append((ws.xc, blk.w1.weight, act, _hip.EPI_SWIGLU))

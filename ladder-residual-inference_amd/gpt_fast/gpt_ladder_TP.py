@@ -123,7 +123,7 @@ class GPTLadder(GPTBase):
     # shard, ms per step with / without: batch 8 8.6 / 8.3, batch 64 18.2 / 18.8).  Putting one step of each chain
     # into the same grid instead (wqkv beside w1, attention beside w2) was slower still: 10.3 ms at batch 8.
     overlap_modules = False
-    two_chains_from = 33   # decode batches from which the MLP chain is a parallel branch (see _run_layers_decode)
+    two_chains_from = _hip.BANDS_TO + 1   # decode batches from which the MLP chain is a parallel branch (see _run_layers_decode)
 
     def _run_layers_decode(self, ws: Workspace, pos: Tensor):
         """Decode step (S == 1) of an all-ladder model through the per-op kernels: one launch does both residual
@@ -140,7 +140,7 @@ class GPTLadder(GPTBase):
             if side is None or side.device != main.device:
                 side = self._side_stream = torch.cuda.Stream(device=main.device)
         pending_a = pending_m = None
-        # decode batches of up to 64 rows on bf16 weights: the block's two input projections share one launch of
+        # decode batches of up to 32 rows on bf16 weights: the block's two input projections share one launch of
         # the weight-streaming kernel (q/k/v -- rotated and cached on the way out -- next to up/gate, which stores
         # silu(gate) * up directly), and so do its two output projections (wo next to w2).  Also below 5 rows,
         # where single projections go to the matrix-vector kernel: five or six launches per block instead of nine
@@ -164,7 +164,13 @@ class GPTLadder(GPTBase):
         for blk in self.layers:
             _hip.ladder_norms(ws.x, pending_a, pending_m, blk.attention_norm.weight, blk.ffn_norm.weight, ws.x, ws.xn,
                               ws.xn2, eps)
-            if multi:
+            if two_chains:
+                chain.wait_stream(cur)
+                with torch.cuda.stream(chain):
+                    self._mlp(ws, blk, ws.m, ws.xn2)
+                self._attention(ws, blk, pos, blk.attention.wqkv, ws.a)
+                cur.wait_stream(chain)
+            elif multi:
                 kv = blk.attention.kv_cache
                 rope = _hip.rope_kv_epilogue(self.freqs_cis, pos, kv.k_cache, kv.v_cache, cfg.n_head_local,
                                              cfg.n_kv_local, cfg.head_dim)
@@ -178,14 +184,6 @@ class GPTLadder(GPTBase):
                     if not beside:
                         _hip.linear_multi(up_gate)
                         self._attention(ws, blk, pos, None, None, roped=True)
-                elif two_chains:
-                    chain.wait_stream(cur)
-                    with torch.cuda.stream(chain):
-                        self._mlp(ws, blk, ws.m, ws.xn2)
-                    self._attention(ws, blk, pos, blk.attention.wqkv, ws.a)
-                    cur.wait_stream(chain)
-                    pending_a, pending_m = ws.a, ws.m
-                    continue
                 else:
                     _hip.linear_multi((ws.xn, blk.attention.wqkv.weight, ws.qkv, rope), up_gate)
                     self._attention(ws, blk, pos, None, None, roped=True)

@@ -51,9 +51,9 @@ class MixerArgs:
 
 
 def project(x: Tensor, lin: nn.Linear, out: Tensor, sums: Optional[Tensor] = None) -> Tensor:
-    """lin(x) for the rows of a step: the weight-streaming kernel from two to 64 rows (32 with `sums`; as the other families' decode
+    """lin(x) for the rows of a step: the weight-streaming kernel from two to 64 rows (BANDS_TO with `sums`; as the other families' decode
     steps use it), what the shape picks otherwise.  `sums`: the workspace's memory for partial sums."""
-    if x.dtype == torch.bfloat16 and 2 <= x.shape[0] <= (64 if sums is None else 32):
+    if x.dtype == torch.bfloat16 and 2 <= x.shape[0] <= (64 if sums is None else _hip.BANDS_TO):
         _hip.linear_multi((x, lin.weight, out, _hip.EPI_NONE))
         return out
     return _hip.linear(x, lin.weight, out, scratch=sums)

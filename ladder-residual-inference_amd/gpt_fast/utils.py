@@ -85,8 +85,8 @@ class DynamicTanh(nn.Module):
 
     def after(self, h: Tensor, lin: nn.Linear, d: Tensor, x: Tensor, out: Tensor, experts=None, sums=None):
         """into() with lin(h) added to x in place: one launch for a decode batch, through `d` otherwise (with `sums`, memory for
-        partial sums, from 33 rows)."""
-        if h.dtype == torch.bfloat16 and h.shape[0] <= (64 if sums is None else 32):
+        partial sums, above BANDS_TO rows)."""
+        if h.dtype == torch.bfloat16 and h.shape[0] <= (64 if sums is None else _hip.BANDS_TO):
             _hip.linear_residual_tanh(h, lin.weight, x, self.alpha, self.weight, self.bias, out, experts)
         else:
             self.into(x, _hip.linear(h, lin.weight, d, scratch=sums), x, out, experts)

@@ -355,6 +355,12 @@ def test_swiglu_projection_of_many_rows_refuses_what_its_two_calls_refuse(lib):
     assert lib.lr_linear_swiglu_out(p, 64, p, p, 24, 65, 36, 64, p, big, None) == E_ALIGN
 
 
+def test_bands_end_where_products_with_partial_sums_begin(lib):
+    from gpt_fast import _hip
+
+    assert lib.lr_linear_scratch_bytes(_hip.BANDS_TO) == 0 and lib.lr_linear_scratch_bytes(_hip.BANDS_TO + 1) > 0
+
+
 def test_only_contiguous_device_memory_is_handed_on_for_partial_sums():
     from gpt_fast import _hip
 
