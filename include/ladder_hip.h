@@ -170,8 +170,9 @@ int lr_linear_multi(const lr_projection_t* projections, int n_projections, int M
  * y[M, N] = x[M, K] w[N, K]^T with N = (n_head + 2 n_kv_head) * head_dim, then q rotated in y, rotated k and
  * v stored at slot pos[s] of the caches, k and v left as projected in y (Attention.forward, utils.py:188-198, and
  * KVCache.update, :50-59) -- bit for bit what lr_linear followed by lr_rope_kv_write (table_is_gathered = 0)
- * leaves, in the output pass of the prefill GEMM (M > 64), in those two calls otherwise.  A position outside the cache or the table sets *rope->err = LR_DEV_POS_RANGE and leaves that
- * row as projected.  ldy % 8 == 0. */
+ * leaves, in the output pass of the matrix-core GEMM where that serves the sizes (M > 64, and M > 32 with memory for
+ * partial sums), in those two calls otherwise.  A position outside the cache or the table sets *rope->err =
+ * LR_DEV_POS_RANGE and leaves that row as projected.  ldy % 8 == 0. */
 int lr_linear_rope_kv(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int K, int S,
                       const lr_rope_kv_t* rope, lr_stream_t stream);
 /* The same with memory for partial sums, as lr_linear_scratch is lr_linear. */

@@ -1,4 +1,4 @@
-// Matrix-core bf16 GEMMs for prefill and for more than 64 rows:
+// Matrix-core bf16 GEMMs for prefill, decode batches above 64 rows, and from 33 rows on where there is memory for partial sums:
 //   y[m, n] = bf16( sum_k x[m, k] * w[n, k] ),  fp32 accumulation.
 // k_gemm_dma (below) is the one that matters; k_gemm here serves an input that is activated on its way in, and rows longer
 // than the 2 GiB offsets of k_gemm_dma's requests reach.
@@ -132,9 +132,9 @@ __global__ __launch_bounds__(256) void k_gemm(const u16* __restrict__ x, int64_t
 
 // ---------------------------------------------------------------------------------------------
 // The GEMM of prompts and of decode batches above 32.  A workgroup of four waves (2 x 2) multiplies a tile of 64 A16 input
-// rows x 128 BH weight rows: 256 x 256, 128 x 256, 128 x 128 or 64 x 128 (gemm_plan picks).  Bound: the matrix cores, at the clock the chip's power allows --
-// 16384 x 4096 x 14336: 1.50 PFLOP/s, matrix cores busy 86 % of the cycles at 1.57 GHz -- from a few hundred rows on; the
-// weights' HBM traffic below.
+// rows x 128 BH weight rows: 256 x 256, 128 x 256, 128 x 128 or 64 x 128 (gemm_plan picks).  Bound: the matrix cores, at the
+// clock the chip's power allows, from a few hundred rows on (16384 x 4096 x 14336, one counter run: 1302 us = 1.48 PFLOP/s,
+// matrix cores busy 79 % of the cycles at 1.78 GHz); the weights' HBM traffic below.
 //
 // Operands go from memory to LDS directly (buffer_load ... lds, 16 bytes per lane, 8 rows x 64 k per instruction): no
 // registers, no LDS write instructions.  An instruction fills 1 KiB of LDS in lane order, so rows cannot be padded; the
@@ -147,14 +147,16 @@ __global__ __launch_bounds__(256) void k_gemm(const u16* __restrict__ x, int64_t
 // LDS into registers for a later phase and requests the half of two k-tiles ahead into the LDS slot that the phase before
 // it emptied: a request has seven phases to land, a slot is read in exactly one phase, and one barrier per phase orders
 // both.  The reads and requests stand between the matrix instructions, one at a time, and every request is made whatever
-// the tile (a k-tile past the end is a resource of no records: zeros, no traffic), so the waits are exact.  The next
+// the tile (a k-tile past the end is a resource of no records: zeros, no traffic), so the waits are exact.  (They count the
+// youngest requests: memory operations that a compiler put between them, a spill's, would make them wait for more, not less.
+// There are none in any instance's loop.)  The next
 // k-tile's A0 and B0 take the registers that A0 and B1 leave, so B0 and B1 change registers from one k-tile to the next:
 // the loop walks two.
 //
 // Before (128 x 128 wave tiles of v_mfma_f32_32x32x16_bf16, operands staged through registers and padded LDS rows):
 // 16384 rows x (N x K), us before / now: 6144 x 4096 646 / 560, 4096 x 4096 428 / 381, 28672 x 4096 with SwiGLU 3112 /
-// 2755, 4096 x 14336 1462 / 1281.  The chip is power-limited under either: with the same loop on 32x32x16 instructions the
-// matrix cores were busy 92 % of the cycles at 1.43 GHz (1337 us): twice the accumulator traffic per product.  The matrix
+// 2755, 4096 x 14336 1462 / 1281 (from machine to machine 2750 - 2870 and 1275 - 1315).  The same loop on 32x32x16
+// instructions took 1337 us for the last: twice the accumulator traffic per product, at a power-limited clock.  The matrix
 // instruction is assembler text because its accumulator has to be one register block in and out: left to the compiler,
 // 180 accumulator moves per two k-tiles (1.15 PFLOP/s).
 // ---------------------------------------------------------------------------------------------
@@ -560,16 +562,20 @@ struct GemmPlan {
   int tile;        // index into GEMM_TILES; -1: no tile serves the shape
   int full, rem, splits;
 };
-// What decides, measured (us; N x K; the plan's choice first, then whole tiles of 256 x 256 / 128 x 256 / 128 x 128):
-//   777 rows,  4096 x 14336   98 (64 tiles of 256 x 256 in 4 pieces)     235 / 158 / 106
-//   777 rows,  4096 x  4096   33 (224 tiles of 128 x 128)                 74 /  47 /  33
-//   300 rows,  4096 x 14336   58 (48 tiles of 128 x 256 in 4 pieces)     235 / 170 / 104
-//   128 rows,  2048 x  8192   20 (16 tiles of 128 x 128 in 8 pieces)     134 /  83 /  58
-//   128 rows, 16384 x  2048   23 (128 pair tiles of 128 x 128 in 2)       48 /  35 /  26
-//  2048 rows,  4096 x 14336  184 (128 tiles of 256 x 256 in 2 pieces)    242 / 199 / 239
-//  3002 rows, 28672 x  4096  564 (1280 tiles whole, 64 in 3 pieces)      586 / 635 / 660
-//    64 rows,  1280 x  8192   15 (10 tiles of 64 x 128 in 12 pieces)       -  /  -  / 100   (the bands of stream_band.h 24)
-//    64 rows, 28672 x  4096   47 (224 pair tiles of 64 x 128)              -  /  65 /  52   (bands 76)
+// What it decides, measured (us, weights from HBM; rows, N x K: with all the memory it could use | without any):
+//   777 rows,  4096 x 14336   117 (64 tiles of 256 x 256 in 4 pieces)      | 110 (224 of 128 x 128)
+//   777 rows,  4096 x  4096    34 (224 tiles of 128 x 128)                 |  the same
+//   300 rows,  4096 x 14336    57 (48 tiles of 128 x 256 in 5)             | 102 (160 of 64 x 128)
+//   128 rows,  2048 x  8192    22 (32 tiles of 64 x 128 in 16)             |  55
+//   128 rows, 16384 x  2048    24 (256 pair tiles of 64 x 128)             |  the same
+//  2048 rows,  4096 x 14336   189 (128 tiles of 256 x 256 in 2)            | 198 (256 of 128 x 256)
+//  3002 rows, 28672 x  4096   564 (1280 pair tiles whole, 64 in 4)         | 577 (1344 whole)
+//    64 rows,  1280 x  8192    16 (10 tiles of 64 x 128 in 16)             |  55   (the bands of stream_band.h 24)
+//    64 rows,  7168 x  8192    34 (56 pair tiles of 64 x 128 in 4)         |  60   (bands 38)
+//    64 rows,  8192 x  3584    20 (64 tiles of 64 x 128 in 3)              |  29   (bands 24)
+//    64 rows, 28672 x  4096    53 (224 pair tiles of 64 x 128)             |  the same   (bands 78)
+//    64 rows,  4096 x 14336    34 (32 tiles of 64 x 128 in 7)              |  97   (in 6 pieces 32)
+// Where it errs: the first line (98 and 106 when the costs below were fitted) and the last.
 // A workgroup's time is nk * (ktile + busy * slope) + fixed, `busy` the workgroups per CU: the more CUs are at work, the
 // lower the clock and the more of them ask the L2s (256 x 256: 1.05 us per k-tile on a quarter of the chip, 1.41 on all of
 // it); `cold` in place of the slope where a single row tile reads every weight from HBM itself; `pair` where two share a CU.

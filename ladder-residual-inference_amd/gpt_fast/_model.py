@@ -224,7 +224,7 @@ class GPTBase(nn.Module):
     # 6.1 / 6.2 with)
     band_rows_from = 2
     # and up to which: above, the GEMM with its partial sums is the faster one (64 rows of the 70B rank shard, us: up/gate
-    # 38.9 in bands / 30.7, q/k/v 23.6 / 14.8, w2 23.0 / 18.6, wo 13.9 / 10.7)
+    # 37.6 in bands / 34.4, q/k/v 23.5 / 16.1, w2 23.8 / 20.1, wo 13.9 / 10.3)
     band_rows_to = _hip.BANDS_TO
 
     def _decode_bands(self, ws: Workspace, *linears) -> bool:
