@@ -119,7 +119,8 @@ class GPTBase(nn.Module):
         self._build_caches(max_batch_size, max_seq_length, dtype, device)
         self._ws.clear()
         self._shapes = None
-        self._sums_bytes(1, 1)
+        for _ in self._products(1, 1):
+            pass
         _hip.device_error_word(device)  # exists before any step is captured into a graph
 
     supported_dtypes = (torch.bfloat16,)
@@ -183,7 +184,7 @@ class GPTBase(nn.Module):
             yield B if leaf == "output" and self.last_logits_only else B * S, N, K, leaf == "w1"
 
     def _sums_bytes(self, B: int, S: int) -> int:
-        return _hip.linear_sums_bytes(self._products(B, S))
+        return _hip.linear_sums_bytes(self._products(B, S)) if B * S > _hip.BANDS_TO else 0
 
     # -- forward --------------------------------------------------------------------------------
     def forward(self, idx: Tensor, input_pos: Optional[Tensor] = None) -> Tensor:

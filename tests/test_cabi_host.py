@@ -293,7 +293,7 @@ def meta_model(family, name):
 
 
 @pytest.mark.parametrize("family,name", FAMILIES)
-@pytest.mark.parametrize("B,S", [(1, 1), (32, 1), (33, 1), (64, 1), (96, 1), (1, 33), (1, 777), (4, 512)])
+@pytest.mark.parametrize("B,S", [(1, 1), (32, 1), (1, 20), (2, 16), (33, 1), (64, 1), (96, 1), (1, 33), (1, 777), (4, 512)])
 def test_memory_for_partial_sums_is_what_the_products_of_a_step_can_use(lib, family, name, B, S):
     """Enough for every product to be divided as with all the memory it could ask for, and no more than that."""
     from gpt_fast import _hip
