@@ -70,4 +70,6 @@ def quantize_model_fp8(model: nn.Module, include_output: bool = True) -> nn.Modu
         model.output = WeightOnlyFp8Linear.from_linear(model.output)
     if hasattr(model, "_fused"):
         model._fused = {}
+    if hasattr(model, "_shapes"):
+        model._shapes = None
     return model
