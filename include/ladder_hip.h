@@ -165,6 +165,51 @@ typedef struct lr_projection {
 } lr_projection_t;
 int lr_linear_multi(const lr_projection_t* projections, int n_projections, int M, lr_stream_t stream);
 
+/* Input rows that have their norm's gain but are still to be divided by their root mean square,
+ *     sqrt(sum_i sums[m * count + i] / dim + eps),  dim = K:
+ * a projection divides its sums instead, in fp32 (normed rows of utils.py:68-78, with one rounding where those have two).
+ * sums NULL: the rows are as they should be.  count <= LR_ROW_NORM_MAX and M <= LR_ROW_NORM_MAX_ROWS, else
+ * LR_E_UNSUPPORTED.  `norms` holds one per projection. */
+typedef struct lr_row_norm {
+  const float* sums; /* [M, count] */
+  int32_t count, dim;
+  float eps;
+  /* fold_sums != NULL: [M, fold_count] parts of other rows' sums of squares, which the launch adds into fold_total [M], the
+   * sums (count 1) of a later launch whose many workgroups then need not.  LR_E_UNSUPPORTED where the projection has fewer
+   * than M bands (N < 4 M). */
+  const float* fold_sums;
+  float* fold_total;
+  int32_t fold_count;
+} lr_row_norm_t;
+#define LR_ROW_NORM_MAX 512
+#define LR_ROW_NORM_MAX_ROWS 16
+int lr_linear_multi_normed(const lr_projection_t* projections, const lr_row_norm_t* norms, int n_projections, int M,
+                           lr_stream_t stream);
+
+/* Output projections of a decode layer with the residual updates behind them and all that the norms of the next layer's
+ * projections need, M <= LR_ROW_NORM_MAX_ROWS rows (LR_E_UNSUPPORTED beyond):
+ *     r1 = bf16(resid_in + bf16(x1 w1^T)),  out1 = bf16(r1 * gain1),  sums1: sums of squares of r1
+ *     r2 = bf16(r1 + bf16(x2 w2^T)),        out2 = bf16(r2 * gain2),  sums2: of r2
+ * resid_out = r2 (may alias resid_in).  joint != 0: nothing is kept of r1 (gain1, out1, sums1 are not used) and
+ * r2 = bf16(resid_in + bf16(x2 w2^T + x1 w1^T)) of the two rounded products (gpt_parallel_TP.py:214-226).  (out1, sums1) and (out2, sums2) are
+ * inputs of lr_linear_multi_normed and its like, lr_linear_resid_sums(D) values per row.  In a ladder block x1 w1^T is the
+ * attention's, x2 w2^T the MLP's (gpt_ladder_TP.py:326-354: what lr_linear_multi and the next block's lr_ladder_norms compute).
+ * scales1 != NULL: both weights are e4m3 bytes with scales, as in lr_linear_fp8_multi. */
+typedef struct lr_linear_resid {
+  const void *x1, *w1, *scales1; /* x1 [M, K1], row stride ldx1; w1 [D, K1] */
+  const void *x2, *w2, *scales2;
+  int64_t ldx1, ldx2;
+  int32_t K1, K2, D;
+  const void* resid_in; /* [M, D], as are resid_out, out1, out2 */
+  void* resid_out;
+  const void *gain1, *gain2; /* [D] */
+  void *out1, *out2;
+  float *sums1, *sums2;
+  int32_t joint;
+} lr_linear_resid_t;
+int lr_linear_resid_sums(int D);
+int lr_linear_resid(const lr_linear_resid_t* desc, int M, lr_stream_t stream);
+
 /* The fused q/k/v projection of a PREFILL, finished as lr_rope_kv_write would finish it: M = B * S input rows (S
  * tokens per sequence, row b * S + s sits at position rope->pos[s], pos int32 [S] on the device),
  * y[M, N] = x[M, K] w[N, K]^T with N = (n_head + 2 n_kv_head) * head_dim, then q rotated in y, rotated k and
@@ -204,6 +249,11 @@ int lr_linear_swiglu_out_scratch(const void* x, int64_t ldx, const void* w, void
 int lr_attn_decode_beside(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos,
                           void* y, int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch,
                           size_t scratch_bytes, const lr_projection_t* projection, int M, lr_stream_t stream);
+/* The same for a projection whose input is as lr_linear_multi_normed takes it. */
+int lr_attn_decode_beside_normed(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos,
+                                 void* y, int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch,
+                                 size_t scratch_bytes, const lr_projection_t* projection, const lr_row_norm_t* norm, int M,
+                                 lr_stream_t stream);
 
 /* Weight-only fp8 linear:  y[m, n] = bf16( bf16( sum_k x[m, k] * w8[n, k] ) * scales[n] ).
  * w8 [N, K] dense float8 e4m3 (OCP "e4m3fn": bias 7, no infinities, max 448), one byte per weight;
@@ -240,6 +290,9 @@ typedef struct lr_projection_fp8 {
   const lr_rope_kv_t* rope; /* LR_EPI_ROPE_KV only, else ignored; read during the call */
 } lr_projection_fp8_t;
 int lr_linear_fp8_multi(const lr_projection_fp8_t* projections, int n_projections, int M, lr_stream_t stream);
+/* Inputs as in lr_linear_multi_normed, from 2 rows on. */
+int lr_linear_fp8_multi_normed(const lr_projection_fp8_t* projections, const lr_row_norm_t* norms, int n_projections, int M,
+                               lr_stream_t stream);
 
 /* lr_attn_decode_beside with a weight-only e4m3 projection (one lr_projection_fp8_t of lr_linear_fp8_multi) in
  * place of the bf16 one: the quantised ladder block's up/gate projection next to its attention.  Same bits as
@@ -250,6 +303,10 @@ int lr_attn_decode_beside_fp8(const void* q, int64_t ldq, const void* k_cache, c
                               const int32_t* pos, void* y, int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax,
                               void* scratch, size_t scratch_bytes, const lr_projection_fp8_t* projection, int M,
                               lr_stream_t stream);
+int lr_attn_decode_beside_fp8_normed(const void* q, int64_t ldq, const void* k_cache, const void* v_cache,
+                                     const int32_t* pos, void* y, int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax,
+                                     void* scratch, size_t scratch_bytes, const lr_projection_fp8_t* projection,
+                                     const lr_row_norm_t* norm, int M, lr_stream_t stream);
 
 /* out[r, i] = bf16( bf16(silu(h[r, I + i])) * h[r, i] ),  h [rows, 2I] = [u | g] (row stride ldh).
  * F.silu(g) * u after chunk(2), utils.py:147-148 and :386. */

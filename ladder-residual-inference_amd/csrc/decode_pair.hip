@@ -56,7 +56,7 @@ template <int HD, int G, bool W8, bool XL, bool EAGER, bool X8 = !W8 && !XL>
 static int launch_pair_as(const AttnItems& a, const Proj& p, int M, u16* y, int64_t ldy, int B, hipStream_t s) {
   const int Hq = a.Hkv * G;
   const size_t lds_att = (size_t)attn_item_lds_floats<HD, G>(a.chunk_max) * sizeof(float);
-  const size_t lds_band = stream_band_lds_bytes<PAIR_MT, PAIR_UNITS, W8, XL>();
+  const size_t lds_band = stream_band_lds_bytes<PAIR_MT, PAIR_UNITS, W8, XL>() + stream_band_norm_bytes(p, M);
   const size_t lds = lds_att > lds_band ? lds_att : lds_band;
   static std::atomic<unsigned long long> lds_raised{0};
   if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_attn_beside_band<HD, G, W8, XL, EAGER, X8>), lds, lds_raised)) return LR_E_LAUNCH;
@@ -83,7 +83,7 @@ static int launch_pair(const AttnItems& a, const Proj& p, int M, u16* y, int64_t
 template <bool W8, class Projection, class Fill>
 static int beside(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos, void* y,
                   int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch, size_t scratch_bytes,
-                  const Projection* proj, int M, int m_min, lr_stream_t stream, Fill fill) {
+                  const Projection* proj, const lr_row_norm_t* norm, int M, int m_min, lr_stream_t stream, Fill fill) {
   LR_REQUIRE_PTR(q);
   LR_REQUIRE_PTR(k_cache);
   LR_REQUIRE_PTR(v_cache);
@@ -98,7 +98,8 @@ static int beside(const void* q, int64_t ldq, const void* k_cache, const void* v
   // the projection must not touch the cache the attention reads, and only the 16-row band shares a CU
   if (proj->epilogue == LR_EPI_ROPE_KV || M > PAIR_MT || M < m_min) return LR_E_UNSUPPORTED;
   Proj p;
-  const int rc = fill(*proj, p);
+  int rc = fill(*proj, p);
+  if (rc == LR_OK) rc = sb_fill_norm(norm, p);
   if (rc != LR_OK) return rc;
   int G = Hq / Hkv;
   AttnItems a;
@@ -121,6 +122,7 @@ static int beside(const void* q, int64_t ldq, const void* k_cache, const void* v
   const int ncu = lr_num_cus();
   if (ncu < 1) return LR_E_LAUNCH;
   plan(p, M, p.pair_off ? 16 : 16 * PAIR_UNITS, ncu);
+  if (p.fold_sums && p.nwg < M) return LR_E_UNSUPPORTED;   // (a row per workgroup)
   hipStream_t s = (hipStream_t)stream;
 #define LR_PAIR(HDV, GV) \
   if (hd == HDV && G == GV) return launch_pair<HDV, GV, W8>(a, p, M, (u16*)y, ldy, B, s);
@@ -132,19 +134,36 @@ static int beside(const void* q, int64_t ldq, const void* k_cache, const void* v
 
 }  // namespace
 
+extern "C" int lr_attn_decode_beside_normed(const void* q, int64_t ldq, const void* k_cache, const void* v_cache,
+                                            const int32_t* pos, void* y, int64_t ldy, int B, int Hq, int Hkv, int hd,
+                                            int Smax, void* scratch, size_t scratch_bytes, const lr_projection_t* proj,
+                                            const lr_row_norm_t* norm, int M, lr_stream_t stream) {
+  return beside<false>(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj, norm, M, 1,
+                       stream, sb_fill_projection);
+}
+
 extern "C" int lr_attn_decode_beside(const void* q, int64_t ldq, const void* k_cache, const void* v_cache,
                                      const int32_t* pos, void* y, int64_t ldy, int B, int Hq, int Hkv, int hd,
                                      int Smax, void* scratch, size_t scratch_bytes, const lr_projection_t* proj,
                                      int M, lr_stream_t stream) {
-  return beside<false>(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj, M, 1,
-                       stream, sb_fill_projection);
+  return lr_attn_decode_beside_normed(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj,
+                                      nullptr, M, stream);
 }
 
 // (for one row lr_linear_fp8_multi uses the matrix-vector kernel, which has no band to put beside the attention)
+extern "C" int lr_attn_decode_beside_fp8_normed(const void* q, int64_t ldq, const void* k_cache, const void* v_cache,
+                                                const int32_t* pos, void* y, int64_t ldy, int B, int Hq, int Hkv, int hd,
+                                                int Smax, void* scratch, size_t scratch_bytes,
+                                                const lr_projection_fp8_t* proj, const lr_row_norm_t* norm, int M,
+                                                lr_stream_t stream) {
+  return beside<true>(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj, norm, M,
+                      LR_FP8_GEMV_MAX_M + 1, stream, sb_fill_projection_fp8);
+}
+
 extern "C" int lr_attn_decode_beside_fp8(const void* q, int64_t ldq, const void* k_cache, const void* v_cache,
                                          const int32_t* pos, void* y, int64_t ldy, int B, int Hq, int Hkv, int hd,
                                          int Smax, void* scratch, size_t scratch_bytes,
                                          const lr_projection_fp8_t* proj, int M, lr_stream_t stream) {
-  return beside<true>(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj, M,
-                      LR_FP8_GEMV_MAX_M + 1, stream, sb_fill_projection_fp8);
+  return lr_attn_decode_beside_fp8_normed(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj,
+                                          nullptr, M, stream);
 }

@@ -329,7 +329,7 @@ __global__ __launch_bounds__(256) void k_scale_cols(u16* __restrict__ y, int64_t
 }  // namespace
 
 namespace lr_detail {
-int stream_fp8_multi(const lr_projection_fp8_t* proj, int n_proj, int M, lr_stream_t stream);  // stream_gemm.hip
+int stream_fp8_multi(const lr_projection_fp8_t* proj, const lr_row_norm_t* norms, int n_proj, int M, lr_stream_t stream);  // stream_gemm.hip
 }
 
 extern "C" size_t lr_linear_fp8_scratch_bytes(int M, int N, int K) {
@@ -353,7 +353,7 @@ extern "C" int lr_linear_fp8(const void* x, int64_t ldx, const void* w8, const v
   if (M > LR_FP8_GEMV_MAX_M && M <= 16 && !lr_misaligned(scales)) {
     // decode batches: the matrix-core bands of lr_linear_fp8_multi (one projection, no epilogue)
     const lr_projection_fp8_t one = {x, ldx, w8, scales, y, ldy, N, K, LR_EPI_NONE, nullptr};
-    const int rc = lr_detail::stream_fp8_multi(&one, 1, M, stream);
+    const int rc = lr_detail::stream_fp8_multi(&one, nullptr, 1, M, stream);
     if (rc != LR_E_UNSUPPORTED || M > 8) return rc;
   }
   if (M <= 8) {
@@ -376,11 +376,18 @@ extern "C" int lr_linear_fp8(const void* x, int64_t ldx, const void* w8, const v
 }
 
 extern "C" int lr_linear_fp8_multi(const lr_projection_fp8_t* proj, int n_proj, int M, lr_stream_t stream) {
+  return lr_linear_fp8_multi_normed(proj, nullptr, n_proj, M, stream);
+}
+
+extern "C" int lr_linear_fp8_multi_normed(const lr_projection_fp8_t* proj, const lr_row_norm_t* norms, int n_proj, int M,
+                                          lr_stream_t stream) {
   if (proj == nullptr) return LR_E_NULL;
   if (n_proj < 1 || n_proj > 2 || M < 1) return LR_E_SHAPE;
   if (M > 16) return LR_E_UNSUPPORTED;
   // from 2 rows on the matrix cores: the dot products of the matrix-vector kernel grow with every row
-  if (M > LR_FP8_GEMV_MAX_M) return lr_detail::stream_fp8_multi(proj, n_proj, M, stream);
+  if (M > LR_FP8_GEMV_MAX_M) return lr_detail::stream_fp8_multi(proj, norms, n_proj, M, stream);
+  for (int i = 0; norms && i < n_proj; ++i)
+    if (norms[i].sums) return LR_E_UNSUPPORTED;
   P8 pr[2] = {};
   for (int i = 0; i < n_proj; ++i) {
     const int rc = fill_p8(proj[i], pr[i]);

@@ -108,11 +108,15 @@ __device__ __forceinline__ float lr_dpp(float v) {
 __device__ __forceinline__ float lr_lane(float v, int lane) {
   return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane));
 }
-__device__ __forceinline__ float wave_sum(float v) {
+__device__ __forceinline__ float row_sum(float v) {   // over the lane's row of 16
   v += lr_dpp<0x128>(v);  // row_ror:8
   v += lr_dpp<0x124>(v);  // row_ror:4
   v += lr_dpp<0x4e>(v);   // quad_perm [2,3,0,1]
   v += lr_dpp<0xb1>(v);   // quad_perm [1,0,3,2]
+  return v;
+}
+__device__ __forceinline__ float wave_sum(float v) {
+  v = row_sum(v);
   return (lr_lane(v, 0) + lr_lane(v, 16)) + (lr_lane(v, 32) + lr_lane(v, 48));
 }
 __device__ __forceinline__ float wave_max(float v) {

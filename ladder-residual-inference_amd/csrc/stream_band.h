@@ -49,6 +49,32 @@ struct Proj {
   u16 *k_cache, *v_cache;
   int32_t* err;
   int Hq, Hkv, hd, Smax, block_size;
+  // the input rows still have to be divided by their root mean square (norm_sums == nullptr: they do not): a row's sum of
+  // squares is the sum of its norm_count values, [M][norm_count]
+  const float* norm_sums;
+  int norm_count, norm_dim;
+  float norm_eps;
+  // the parts of another norm's sums of squares, [M][fold_count], which this launch adds to [M] sums for a later one
+  const float* fold_sums;
+  float* fold_total;
+  int fold_count;
+};
+__host__ __device__ constexpr int norm_pitch(int count) { return (count + 255) & ~255; }   // LDS row of parts: whole requests
+
+// What a layer's output projections leave for the next layer's input projections instead of their sums (stream_band, RN):
+// a = x w^T, and behind it with a second pair m = x2 w2^T; r1 = resid + a, r2 = r1 + m; out1 = r1 * gain1,
+// out2 = r2 * gain2 and the sums of squares of the band's columns of r1 and r2.
+struct ResidNorm {
+  const u16 *x2, *w2;
+  const u16* scales2;
+  int64_t ldx2;
+  int K2;
+  const u16* rin;          // [M, N]
+  u16* rout;
+  const u16 *gain1, *gain2;
+  u16 *out1, *out2;        // [M, N]
+  float *sums1, *sums2;    // [M][bands]
+  int joint;               // r2 = resid + (m + a), and nothing is kept of r1
 };
 
 // the low (HI == false) or high two e4m3 values of a dword as a packed bf16 pair (exact)
@@ -58,10 +84,26 @@ __device__ __forceinline__ u32 sb_fp8_pair(u32 v) {
   return __builtin_bit_cast(u32, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 1.0f, HI));
 }
 
-template <int MT, int UNITS, bool W8 = false, bool XL = (MT >= XLDS_MIN_MT)>
+template <int MT, int UNITS, bool W8 = false, bool XL = (MT >= XLDS_MIN_MT), int NW = NWV>
 constexpr size_t stream_band_lds_bytes() {
   constexpr int LRW = (W8 ? 2 * KC : KC) + 8;
-  return (size_t)NWV * (UNITS * 16 * LRW + (XL ? MT * LRW : 0)) * sizeof(u16);
+  return (size_t)NW * (UNITS * 16 * LRW + (XL ? MT * LRW : 0)) * sizeof(u16);
+}
+// and behind that, where the input's rows come with sums of squares: the sums, in whole requests, a factor per row, and a row
+// of the sums that are added for a later launch
+static inline size_t stream_band_norm_bytes(const Proj& p, int M) {
+  const int parts = (p.norm_count == 1 ? 256 : M * norm_pitch(p.norm_count)) + (p.fold_sums ? norm_pitch(p.fold_count) : 0);
+  return p.norm_sums ? (size_t)(parts + 64) * sizeof(float) : 0;
+}
+// One wave instruction: 64 x 16 bytes to LDS at `lds` + 16 * lane; what lies beyond `bytes` reads as zero.
+__device__ __forceinline__ void band_dma16(const void* base, int bytes, int voff, u32 lds) {
+  typedef int i32x4_t __attribute__((ext_vector_type(4)));
+  i32x4_t r;
+  r.x = (int)(u32)(unsigned long long)base;
+  r.y = (int)(u32)((unsigned long long)base >> 32) & 0xffff;
+  r.z = bytes;
+  r.w = 0x00020000;
+  asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"{m0}"(lds), "v"(voff), "s"(r) : "memory");
 }
 
 // One band of one projection, by the 256 lanes of a workgroup.  `sg_smem`: stream_band_lds_bytes<MT, UNITS>() bytes of LDS.
@@ -91,10 +133,12 @@ struct BandResidual {
 // 1280 x 8192 7.80 -> 6.32, 8192 x (1024 | 3584) 11.9 -> 10.8, up/gate 14.2 -> 13.6.  The sums keep their order.
 // GATHER: input row m is row rows[m] / xdiv of x, output row m is row rows[m] of y (`rows`: M of them, in LDS).
 template <int MT, int UNITS, bool W8 = false, bool XL = (MT >= XLDS_MIN_MT), bool GATHER = false, bool RESID = false, int KW = NWV,
-          int UROWS = 16, bool DEEP = true, bool X8 = false>
+          int UROWS = 16, bool DEEP = true, bool X8 = false, int NW = NWV, bool RN = false>
 __device__ __forceinline__ void stream_band(const Proj& p, const int M, const int band_, u16* sg_smem,
-                                            const int32_t* rows = nullptr, const int xdiv = 1, const BandResidual rs = {}) {
+                                            const int32_t* rows = nullptr, const int xdiv = 1, const BandResidual rs = {},
+                                            const ResidNorm& rn = {}) {
   static_assert(!W8 || MT == 16, "the e4m3 path is built for up to 16 input rows");
+  const bool has_norm = MT == 16 && KW == NW && !GATHER && !RESID && !RN && p.norm_sums != nullptr;
   constexpr int KCW = W8 ? 256 : 128;  // k elements per chunk
   constexpr int LRW = KCW + 8;         // LDS row length in elements
   constexpr int WB = W8 ? 1 : 2;       // bytes per weight
@@ -115,7 +159,7 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
   static_assert(!(XL && W8), "the e4m3 band reads its inputs in fragment layout");
   constexpr int WPIECE = UNITS * 16 * LRW, XPIECE = XLDS ? MT * LRW : 0;  // elements per wave
   // sg_smem: [NWV][WPIECE + XPIECE]
-  static_assert(sizeof(float) * NV * 64 <= sizeof(u16) * WPIECE, "the partial sums reuse the wave's weight piece");
+  static_assert(sizeof(float) * (RN ? 2 : 1) * NV * 64 <= sizeof(u16) * WPIECE, "the partial sums reuse the wave's weight piece");
 
   const u16* const xg = p.x;
   const u16* const wg_ = p.w;
@@ -129,8 +173,9 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, l4 = lane >> 4;
   const int la = lane & (UROWS - 1);  // the band row of a lane's A fragment (beyond UROWS the first rows again: unused sums)
-  static_assert(KW == NWV || (KW == 1 && !W8 && !XL), "");
-  const int band = KW == 1 ? band_ * NWV + wave : band_;
+  static_assert(KW == NW || (KW == 1 && !W8 && !XL), "");
+  static_assert(!RN || (KW == NW && MT == 16 && !GATHER && !RESID), "");
+  const int band = KW == 1 ? band_ * NW + wave : band_;
   const int kwave = KW == 1 ? 0 : wave;
   LR_BAND_STAMP(0)
   const int n_out = pair_off ? pair_off : N;         // output columns
@@ -182,6 +227,20 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
       return __builtin_bit_cast(bf16x8_t, r[mt][ks]);
     }
   };
+  // OOB where v >= n, else 0: no branch, and a scalar stays one
+  auto beyond = [](int v, int n) { return ~(v - n) & OOB; };
+  // (RN) the first pair's chunks of K come first, then the second's; a lane's offsets within each matrix, its rows' in scalars
+  const int nck1 = (K + KCW - 1) / KCW;
+  int wv1 = 0, wv2 = 0, xoff2[XLDS ? MT / 4 : MTILES];
+  if constexpr (RN) {
+    wv1 = l4 * K * WB + l16 * 16;
+    wv2 = l4 * rn.K2 * WB + l16 * 16;
+#pragma unroll
+    for (int i = 0; i < (XLDS ? MT / 4 : MTILES); ++i) {
+      const int m = XLDS ? 4 * i + l4 : (X8 ? l16 & 7 : l16);
+      xoff2[i] = m < M ? (int)((m * rn.ldx2 + (XLDS ? l16 * 8 : (X8 ? (l16 >> 3) * 32 : 0) + l4 * 8)) * 2) : OOB;
+    }
+  }
   u16* const my = sg_smem + wave * (WPIECE + XPIECE);
   u16* const myx = my + WPIECE;
 
@@ -200,6 +259,19 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
   // 1.5 % faster per step, 64-row bands 8 % slower -- their inputs come from L2, which likes the common window.
   // Not kept: the order of a sum would then depend on how the rows are cut into bands.)
   auto issue_w = [&](int ci, u32x4_t (&dst)[NLD]) {
+    if constexpr (RN) {
+      const int g = ci * KW + kwave;
+      const bool second = g >= nck1;
+      const int k0 = (second ? g - nck1 : g) * KCW, Kx = second ? rn.K2 : K;
+      const __amdgpu_buffer_rsrc_t res = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<unsigned char*>(reinterpret_cast<const unsigned char*>(second ? rn.w2 : wg_) + (int64_t)n0 * Kx * WB), 0, 0x7fffffff,
+          0x00020000);
+      const int at = (second ? wv2 : wv1) | beyond(k0 + l16 * (16 / WB), Kx);
+#pragma unroll
+      for (int i = 0; i < NLD; ++i)
+        dst[i] = __builtin_amdgcn_raw_buffer_load_b128(res, at | beyond(4 * i + l4, nrows), (k0 + 4 * i * Kx) * WB, AUX_WEIGHTS);
+      return;
+    }
     const int k0 = (ci * KW + kwave) * KCW;
     const bool kok = k0 + l16 * (16 / WB) < K;
 #pragma unroll
@@ -207,6 +279,22 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
       dst[i] = __builtin_amdgcn_raw_buffer_load_b128(wres, (kok && woff[i] != OOB) ? woff[i] : OOB, k0 * WB, AUX_WEIGHTS);
   };
   auto issue_x = [&](int ci, u32x4_t (&dst)[MTILES][X8 ? KS / 2 : KS]) {
+    if constexpr (RN) {
+      const int g = ci * KW + kwave;
+      const bool second = g >= nck1;
+      const int k0 = (second ? g - nck1 : g) * KCW, Kx = second ? rn.K2 : K;
+      const __amdgpu_buffer_rsrc_t res =
+          __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(second ? rn.x2 : xg), 0, 0x7fffffff, 0x00020000);
+      constexpr int NX = XLDS ? MT / 4 : (X8 ? KS / 2 : KS);
+#pragma unroll
+      for (int j = 0; j < NX; ++j) {
+        const int at = XLDS ? l16 * 8 : (X8 ? (2 * j + (l16 >> 3)) * 32 : j * 32) + l4 * 8;   // the lane's first k in the chunk
+        const int off = second ? xoff2[XLDS ? j : 0] : xoff[XLDS ? j : 0];
+        dst[XLDS ? j / KS : 0][XLDS ? j % KS : j] = __builtin_amdgcn_raw_buffer_load_b128(
+            res, off | beyond(k0 + at, Kx), (k0 + (XLDS ? 0 : (X8 ? 2 : 1) * j * 32)) * 2, 0);
+      }
+      return;
+    }
     const int k0 = (ci * KW + kwave) * KCW;
     if constexpr (XLDS) {
       const bool kok = k0 + l16 * 8 < K;
@@ -231,11 +319,57 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
     }
   };
 
-  const int nck = (K + KCW - 1) / KCW;
+  const int nck = nck1 + (RN ? (rn.K2 + KCW - 1) / KCW : 0);
   const int nch = kwave < nck ? (nck - kwave + KW - 1) / KW : 0;  // chunks of this wave
   // (the fences keep the requests in this order: the wait for chunk 0 counts the requests made after it, and the
   // scheduler, left alone, asks for chunk 0 last -- the loop then waited for all but the last 8 requests at the top
   // of every round of NS chunks)
+  // The parts of the sums of squares of rows wave, wave + NW, ... go to LDS ahead of everything else, and while the first
+  // weights are on their way the wave adds them.  Whole sums (norm_count 1) need one request.
+  const int npitch = norm_pitch(p.norm_count);
+  float* const nsum = reinterpret_cast<float*>(sg_smem + NW * (WPIECE + XPIECE));
+  float* const nscale = nsum + (p.norm_count == 1 ? 256 : M * npitch);
+  const bool folds = has_norm && p.fold_sums != nullptr && band < M && wave == NW - 1;   // the other norm's row `band`
+  float* const nfold = nscale + 64;
+  if (has_norm) {
+    const u32 at = __builtin_amdgcn_readfirstlane((u32)(uintptr_t)(__attribute__((address_space(3))) float*)nsum);
+    if (p.norm_count == 1) {
+      if (wave == 0) band_dma16(p.norm_sums, M * 4, lane * 16, at);
+    } else {
+      for (int m = wave; m < M; m += NW)
+        for (int o = 0; o < npitch; o += 256)
+          band_dma16(p.norm_sums + m * p.norm_count, p.norm_count * 4, (o + lane * 4) * 4, at + (m * npitch + o) * 4);
+    }
+    if (folds) {
+      const u32 fat = __builtin_amdgcn_readfirstlane((u32)(uintptr_t)(__attribute__((address_space(3))) float*)nfold);
+      for (int o = 0; o < norm_pitch(p.fold_count); o += 256)
+        band_dma16(p.fold_sums + band * p.fold_count, p.fold_count * 4, (o + lane * 4) * 4, fat + o * 4);
+    }
+  }
+  // the residual and the gains of the lane's output
+  u16 r_in = 0, ga1 = 0, ga2 = 0, sc1 = 0, sc2 = 0;
+  constexpr int ROWS_RN = 16 * UNITS;
+  static_assert(!RN || ROWS_RN * MT <= NW * 64, "an output per lane");
+  const int rn_r = tid % ROWS_RN, rn_m = tid / ROWS_RN;
+  const bool rn_ok = RN && rn_r < nrows && rn_m < M;
+  if constexpr (RN) {
+    // (no branch around a load: see above)
+    const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(rn.rin), 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t r1 = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(rn.gain1), 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t r2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(rn.gain2), 0, 0x7fffffff, 0x00020000);
+    r_in = __builtin_amdgcn_raw_buffer_load_b16(rr, rn_ok ? (rn_m * N + n0 + rn_r) * 2 : OOB, 0, 0);
+    ga1 = __builtin_amdgcn_raw_buffer_load_b16(r1, rn_ok ? (n0 + rn_r) * 2 : OOB, 0, 0);
+    ga2 = __builtin_amdgcn_raw_buffer_load_b16(r2, rn_ok ? (n0 + rn_r) * 2 : OOB, 0, 0);
+    if constexpr (W8) {
+      const __amdgpu_buffer_rsrc_t s1 = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(p.scales), 0, 0x7fffffff, 0x00020000);
+      const __amdgpu_buffer_rsrc_t s2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(rn.scales2), 0, 0x7fffffff, 0x00020000);
+      sc1 = __builtin_amdgcn_raw_buffer_load_b16(s1, rn_ok ? (n0 + rn_r) * 2 : OOB, 0, 0);
+      sc2 = __builtin_amdgcn_raw_buffer_load_b16(s2, rn_ok ? (n0 + rn_r) * 2 : OOB, 0, 0);
+    }
+    asm volatile("" ::: "memory");
+  }
+  f32x4_t acc1[UNITS][MTILES];   // (RN) the first pair's sums, once the wave has its last chunk of it
+  bool in_first = true;
   issue_x(0, xr[0]);
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
@@ -244,11 +378,53 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
     issue_w(s, wr[s]);
   }
   asm volatile("" ::: "memory");
+  if (has_norm) {
+    constexpr int YOUNGER = NS * NLD + (DEEP ? NS : 1) * (XLDS ? MT / 4 : MTILES * (X8 ? KS / 2 : KS));   // requests since
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(YOUNGER < 63 ? YOUNGER : 63) : "memory");
+    auto part = [&](const float* row, int pitch) {   // (zeros beyond the count)
+      float v = 0.0f;
+      for (int o = 0; o < pitch; o += 256) {
+        const float4 q = *reinterpret_cast<const float4*>(row + o + lane * 4);
+        v += (q.x + q.y) + (q.z + q.w);
+      }
+      return v;
+    };
+    if (p.norm_count == 1) {
+      if (wave == 0 && lane < M) nscale[lane] = rsqrtf(nsum[lane] / (float)p.norm_dim + p.norm_eps);
+    } else {
+      constexpr int R = MT / NW;   // rows of a wave, their sums side by side
+      float v[R];
+#pragma unroll
+      for (int i = 0; i < R; ++i) v[i] = part(nsum + (wave + i * NW < M ? wave + i * NW : 0) * npitch, npitch);
+#pragma unroll
+      for (int i = 0; i < R; ++i) v[i] = wave_sum(v[i]);
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+        if (lane == 0 && wave + i * NW < M) nscale[wave + i * NW] = rsqrtf(v[i] / (float)p.norm_dim + p.norm_eps);
+    }
+    if (folds) {
+      const float v = wave_sum(part(nfold, norm_pitch(p.fold_count)));
+      if (lane == 0) p.fold_total[band] = v;
+    }
+    asm volatile("" ::: "memory");
+  }
   LR_BAND_STAMP(1)
   for (int c0 = 0; c0 < nch; c0 += NS) {
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       const int ci = c0 + s;
+      if constexpr (RN) {
+        if (in_first && ci * KW + kwave >= nck1) {
+          in_first = false;
+#pragma unroll
+          for (int u = 0; u < UNITS; ++u)
+#pragma unroll
+            for (int mt = 0; mt < MTILES; ++mt) {
+              acc1[u][mt] = acc[u][mt];
+              acc[u][mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        }
+      }
       if (!DEEP) issue_x(ci + 1, xr[(s + 1) % XS]);
       // ---- this chunk's weights: registers -> LDS (row-major) -> A fragments
       asm volatile("" ::: "memory");
@@ -328,6 +504,17 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
   }
 
   LR_BAND_STAMP(3)
+  if constexpr (RN) {
+    if (in_first) {
+#pragma unroll
+      for (int u = 0; u < UNITS; ++u)
+#pragma unroll
+        for (int mt = 0; mt < MTILES; ++mt) {
+          acc1[u][mt] = acc[u][mt];
+          acc[u][mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
+  }
   // ---- the waves' partial sums meet in LDS (accumulator element e of tile (u, mt): band row
   //      16 u + 4 (lane / 16) + e, input row 16 mt + lane % 16) and are added in wave order
   __syncthreads();
@@ -338,9 +525,50 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
 #pragma unroll
     for (int mt = 0; mt < MTILES; ++mt)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) red[wave * WSTRIDE + ((u * MTILES + mt) * 4 + e) * 64 + lane] = acc[u][mt][e];
+      for (int e = 0; e < 4; ++e) {
+        red[wave * WSTRIDE + ((u * MTILES + mt) * 4 + e) * 64 + lane] = acc[u][mt][e];
+        if constexpr (RN) red[wave * WSTRIDE + NV * 64 + ((u * MTILES + mt) * 4 + e) * 64 + lane] = acc1[u][mt][e];
+      }
   __syncthreads();
+  // a sum, or that of the input's normed rows
+  auto normed = [&](float v, int m) { return has_norm ? v * nscale[m] : v; };
   LR_BAND_STAMP(4)
+  if constexpr (RN) {
+    float a = 0.0f, m2 = 0.0f;
+    const int ln = ((rn_r & 15) >> 2) * 16 + (rn_m & 15), e = rn_r & 3, u = rn_r >> 4;
+#pragma unroll
+    for (int wv = 0; wv < NW; ++wv) {
+      a += red[wv * WSTRIDE + NV * 64 + (u * 4 + e) * 64 + ln];
+      m2 += red[wv * WSTRIDE + (u * 4 + e) * 64 + ln];
+    }
+    a = round_bf(a);
+    m2 = round_bf(m2);
+    const int n = n0 + rn_r;
+    if constexpr (W8) {
+      a = round_bf(a * bf_to_f(sc1));
+      m2 = round_bf(m2 * bf_to_f(sc2));
+    }
+    const float r1 = round_bf(bf_to_f(r_in) + a), r2 = rn.joint ? round_bf(bf_to_f(r_in) + round_bf(m2 + a)) : round_bf(r1 + m2);
+    float s1 = rn_ok ? r1 * r1 : 0.0f, s2 = rn_ok ? r2 * r2 : 0.0f;
+    s1 = row_sum(s1);
+    s2 = row_sum(s2);
+    if (ROWS_RN == 32) {
+      s1 += __shfl_xor(s1, 16, LR_WAVE);
+      s2 += __shfl_xor(s2, 16, LR_WAVE);
+    }
+    if (rn_ok) {
+      const int64_t at = (int64_t)rn_m * N + n;
+      rn.rout[at] = f_to_bf(r2);
+      if (!rn.joint) rn.out1[at] = f_to_bf(r1 * bf_to_f(ga1));
+      rn.out2[at] = f_to_bf(r2 * bf_to_f(ga2));
+      if (rn_r == 0) {
+        if (!rn.joint) rn.sums1[rn_m * p.nwg + band] = s1;
+        rn.sums2[rn_m * p.nwg + band] = s2;
+      }
+    }
+    LR_BAND_STAMP(5)
+    return;
+  }
   const int rows_out = pair_off ? 16 : 16 * UNITS;
   if (rope_table != nullptr) {
     // The fused q/k/v projection of a decode step (one token per sequence: input row m is sequence m):
@@ -351,18 +579,18 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
     const int ps = pp.pos[0];
     const bool in_range = ps >= 0 && ps < pp.Smax && ps < pp.block_size;
     if (!in_range && pp.err && band == 0 && tid == 0) *pp.err = LR_DEV_POS_RANGE;
-    for (int o = tid; o < (rows_out / 2) * MT; o += NWV * 64) {
+    for (int o = tid; o < (rows_out / 2) * MT; o += NW * 64) {
       const int r = 2 * (o % (rows_out / 2)), m = o / (rows_out / 2);
       if (r >= nrows || m >= M) continue;
       const int mt = m >> 4, ln = ((r & 15) >> 2) * 16 + (m & 15), e = r & 3, u = r >> 4;
       float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll
-      for (int wv = 0; wv < NWV; ++wv) {
+      for (int wv = 0; wv < NW; ++wv) {
         s0 += red[wv * WSTRIDE + ((u * MTILES + mt) * 4 + e) * 64 + ln];
         s1 += red[wv * WSTRIDE + ((u * MTILES + mt) * 4 + e + 1) * 64 + ln];
       }
       const int n = n0 + r;
-      float x0 = round_bf(s0), x1 = round_bf(s1);
+      float x0 = round_bf(normed(s0, m)), x1 = round_bf(normed(s1, m));
       if constexpr (W8) {
         x0 = round_bf(x0 * bf_to_f(pp.scales[n]));
         x1 = round_bf(x1 * bf_to_f(pp.scales[n + 1]));
@@ -413,16 +641,16 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
 #pragma unroll
         for (int wv = 0; wv < KW; ++wv) s1 += red[(KW == 1 ? wave : wv) * WSTRIDE + ((MTILES + mt) * 4 + e) * 64 + ln];
       }
-      float u_ = round_bf(s0), g_ = round_bf(s1);
+      float u_ = round_bf(normed(s0, m)), g_ = round_bf(normed(s1, m));
       if constexpr (W8) {
         u_ = round_bf(u_ * bf_to_f(p.scales[n0 + r]));
         g_ = round_bf(g_ * bf_to_f(p.scales[pair_off + n0 + r]));
       }
       yg[(int64_t)ym * ldy + n0 + r] = f_to_bf(swiglu_bf(u_, g_));
     } else if constexpr (W8) {
-      yg[(int64_t)ym * ldy + n0 + r] = f_to_bf(round_bf(s0) * bf_to_f(p.scales[n0 + r]));
+      yg[(int64_t)ym * ldy + n0 + r] = f_to_bf(round_bf(normed(s0, m)) * bf_to_f(p.scales[n0 + r]));
     } else {
-      yg[(int64_t)ym * ldy + n0 + r] = f_to_bf(s0);
+      yg[(int64_t)ym * ldy + n0 + r] = f_to_bf(normed(s0, m));
     }
   }
   LR_BAND_STAMP(5)
@@ -442,6 +670,28 @@ static void plan(Proj& p, int M, int cap, int ncu) {
   if (rpw > cap) rpw = cap;
   p.rpw = rpw;
   p.nwg = (items + rpw - 1) / rpw;
+}
+
+// the sums of squares that come with a projection's input
+static int sb_fill_norm(const lr_row_norm_t* q, Proj& p) {
+  if (q == nullptr || q->sums == nullptr) return LR_OK;
+  LR_REQUIRE_PTR(q->sums);
+  if (q->count <= 0 || q->dim != p.K) return LR_E_SHAPE;
+  if (q->count > LR_ROW_NORM_MAX) return LR_E_UNSUPPORTED;
+  p.norm_sums = q->sums;
+  p.norm_count = q->count;
+  p.norm_dim = q->dim;
+  p.norm_eps = q->eps;
+  if (q->fold_sums) {
+    LR_REQUIRE_PTR(q->fold_sums);
+    if (q->fold_total == nullptr) return LR_E_NULL;
+    if (q->fold_count <= 0) return LR_E_SHAPE;
+    if (q->fold_count > LR_ROW_NORM_MAX) return LR_E_UNSUPPORTED;
+    p.fold_sums = q->fold_sums;
+    p.fold_total = q->fold_total;
+    p.fold_count = q->fold_count;
+  }
+  return LR_OK;
 }
 
 // lr_projection_t -> Proj (validated; rpw / nwg are set by plan())

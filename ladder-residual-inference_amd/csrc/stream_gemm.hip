@@ -34,7 +34,7 @@ __global__ __launch_bounds__(NWV * 64, MT == 16 ? 2 : 0) void k_stream_gemm(cons
 
 template <int MT, int UNITS, bool W8 = false, bool XL = (MT >= XLDS_MIN_MT), int UROWS = 16, bool X8 = (MT == 16 && !XL && !W8), bool DEEP = (MT == 16)>
 static int launch_units(Proj& a, Proj& b, int M, hipStream_t s) {
-  constexpr size_t lds = stream_band_lds_bytes<MT, UNITS, W8, XL>();
+  const size_t na = stream_band_norm_bytes(a, M), nb = stream_band_norm_bytes(b, M), lds = stream_band_lds_bytes<MT, UNITS, W8, XL>() + (na > nb ? na : nb);
   static std::atomic<unsigned long long> lds_raised{0};
   if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_stream_gemm<MT, UNITS, W8, XL, UROWS, DEEP, X8>), lds, lds_raised)) return LR_E_LAUNCH;
   k_stream_gemm<MT, UNITS, W8, XL, UROWS, DEEP, X8><<<dim3((unsigned)(a.nwg + b.nwg)), dim3(NWV * 64), lds, s>>>(a, b, M);
@@ -73,17 +73,25 @@ static int pick_units_and_plan(Proj* pr, int n_proj, int M, int ncu) {
 }  // namespace
 
 extern "C" int lr_linear_multi(const lr_projection_t* proj, int n_proj, int M, lr_stream_t stream) {
+  return lr_linear_multi_normed(proj, nullptr, n_proj, M, stream);
+}
+
+extern "C" int lr_linear_multi_normed(const lr_projection_t* proj, const lr_row_norm_t* norms, int n_proj, int M, lr_stream_t stream) {
   if (proj == nullptr) return LR_E_NULL;
   if (n_proj < 1 || n_proj > 2 || M < 1) return LR_E_SHAPE;
   if (M > 64) return LR_E_UNSUPPORTED;
   Proj pr[2] = {};
   for (int i = 0; i < n_proj; ++i) {
-    const int rc = sb_fill_projection(proj[i], pr[i]);
+    int rc = sb_fill_projection(proj[i], pr[i]);
+    if (rc == LR_OK && norms) rc = sb_fill_norm(norms + i, pr[i]);
     if (rc != LR_OK) return rc;
+    if (pr[i].norm_sums && M > LR_ROW_NORM_MAX_ROWS) return LR_E_UNSUPPORTED;
   }
   const int ncu = lr_num_cus();
   if (ncu < 1) return LR_E_LAUNCH;
   const int units = pick_units_and_plan(pr, n_proj, M, ncu);
+  for (int i = 0; i < n_proj; ++i)
+    if (pr[i].fold_sums && pr[i].nwg < M) return LR_E_UNSUPPORTED;   // (a row per workgroup)
   hipStream_t s = (hipStream_t)stream;
   const int rc = M <= 16 ? launch<16>(pr[0], pr[1], M, units, s)
                  : (M <= 32 ? launch<32>(pr[0], pr[1], M, units, s) : launch<64>(pr[0], pr[1], M, units, s));
@@ -139,6 +147,100 @@ extern "C" int lr_linear_residual_tanh(const void* x, int64_t ldx, const void* w
   return M >= XLDS_M16_FROM ? launch_residual<16, true>(pr[0], M, units, rs, s) : launch_residual<16, false>(pr[0], M, units, rs, s);
 }
 
+// ---- a layer's output projections with the residual updates and what the next norms need of the rows (lr_linear_resid)
+//
+// A norm between two projections is a launch that moves next to nothing and waits for everything.  Here the workgroup that
+// owns a band of columns forms both products of it, so it can update the residual there; it leaves the rows with their gains
+// and its share of their sums of squares, and the next projections divide their results by the rows' root mean squares
+// (stream_band: has_norm).  Bound: HBM, like the bands it replaces, whose two workgroups of four waves per CU become one of
+// eight: chunks of the first weight, then of the second, are dealt round the waves.  Measured, us per launch under a
+// profiler: 8192 x (1024 | 3584) e4m3 of 5 rows 10.7 -> 11.8 and q/k/v 7.0 -> 7.9, for a norm launch of 4.7; a step, us: 70B
+// rank shard, 8 rows 4617 -> 4403, e4m3 5 rows 3450 -> 3257; 8B 16 rows 3576 -> 3560; 8B parallel blocks, 6 rows 3220 -> 3114.
+// Not for 17 rows and more (the 32-row band fills the register file with four waves), nor where the norm stands between a
+// block's attention and its MLP: up/gate then has several bands per CU, each of which would add all the parts (12 rows of 8B
+// desync blocks 3755 -> 3772), and rounding the rows once instead of twice moves near-ties of two-row batches.
+namespace {
+
+constexpr int RN_WAVES = 8;
+
+template <int UNITS, bool W8, bool XL, int UROWS, bool X8>
+__global__ __launch_bounds__(RN_WAVES * 64) void k_stream_resid(const Proj p, const int M, const ResidNorm rn) {
+  extern __shared__ __attribute__((aligned(16))) u16 sg_smem[];
+  stream_band<16, UNITS, W8, XL, false, false, RN_WAVES, UROWS, !(XL && UNITS == 2), X8, RN_WAVES, true>(p, M, blockIdx.x, sg_smem, nullptr, 1, BandResidual{}, rn);
+}
+
+template <int UNITS, bool W8, bool XL, int UROWS, bool X8>
+int launch_resid_as(const Proj& p, int M, const ResidNorm& rn, hipStream_t s) {
+  constexpr size_t lds = stream_band_lds_bytes<16, UNITS, W8, XL, RN_WAVES>();
+  static std::atomic<unsigned long long> raised{0};
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_stream_resid<UNITS, W8, XL, UROWS, X8>), lds, raised)) return LR_E_LAUNCH;
+  k_stream_resid<UNITS, W8, XL, UROWS, X8><<<dim3((unsigned)p.nwg), dim3(RN_WAVES * 64), lds, s>>>(p, M, rn);
+  return lr_launch_status();
+}
+template <int UNITS, int UROWS>
+int launch_resid_rows(const Proj& p, int M, const ResidNorm& rn, hipStream_t s) {
+  if (p.scales) return M <= 8 ? launch_resid_as<UNITS, true, false, UROWS, true>(p, M, rn, s) : launch_resid_as<UNITS, true, false, UROWS, false>(p, M, rn, s);
+  return M >= XLDS_M16_FROM ? launch_resid_as<UNITS, false, true, UROWS, false>(p, M, rn, s) : launch_resid_as<UNITS, false, false, UROWS, true>(p, M, rn, s);
+}
+// bands of the columns: every CU the same number of rows
+void plan_resid(int D, int ncu, int& rows, int& bands) {
+  const int rounds = (D + 32 * ncu - 1) / (32 * ncu);
+  rows = (D + ncu * rounds - 1) / (ncu * rounds);
+  bands = (D + rows - 1) / rows;
+}
+
+}  // namespace
+
+extern "C" int lr_linear_resid_sums(int D) {
+  const int ncu = lr_num_cus();
+  if (D <= 0 || ncu < 1) return 0;
+  int rows, bands;
+  plan_resid(D, ncu, rows, bands);
+  return bands;
+}
+
+extern "C" int lr_linear_resid(const lr_linear_resid_t* d, int M, lr_stream_t stream) {
+  if (d == nullptr) return LR_E_NULL;
+  LR_REQUIRE_PTR(d->resid_in);
+  LR_REQUIRE_PTR(d->resid_out);
+  LR_REQUIRE_PTR(d->gain2);
+  LR_REQUIRE_PTR(d->out2);
+  const bool joint = d->joint != 0;
+  if (d->sums2 == nullptr) return LR_E_NULL;
+  if (!joint) {
+    LR_REQUIRE_PTR(d->gain1);
+    LR_REQUIRE_PTR(d->out1);
+    if (d->sums1 == nullptr) return LR_E_NULL;
+  }
+  if (M < 1) return LR_E_SHAPE;
+  if (M > LR_ROW_NORM_MAX_ROWS) return LR_E_UNSUPPORTED;
+  const bool w8 = d->scales1 != nullptr;
+  Proj pr[2] = {};
+  for (int i = 0; i < 2; ++i) {
+    int rc;
+    if (w8) {
+      const lr_projection_fp8_t q = {i ? d->x2 : d->x1, i ? d->ldx2 : d->ldx1, i ? d->w2 : d->w1, i ? d->scales2 : d->scales1, d->resid_out, d->D,
+                                     d->D, i ? d->K2 : d->K1, LR_EPI_NONE, nullptr};
+      rc = sb_fill_projection_fp8(q, pr[i]);
+    } else {
+      const lr_projection_t q = {i ? d->x2 : d->x1, i ? d->ldx2 : d->ldx1, i ? d->w2 : d->w1, d->resid_out, d->D, d->D, i ? d->K2 : d->K1,
+                                 LR_EPI_NONE, nullptr};
+      rc = sb_fill_projection(q, pr[i]);
+    }
+    if (rc != LR_OK) return rc;
+  }
+  if ((int64_t)M * d->D * 2 >= 0x7fffffff) return LR_E_UNSUPPORTED;
+  const int ncu = lr_num_cus();
+  if (ncu < 1) return LR_E_LAUNCH;
+  plan_resid(d->D, ncu, pr[0].rpw, pr[0].nwg);
+  const ResidNorm rn = {pr[1].x, pr[1].w, pr[1].scales, pr[1].ldx, pr[1].K, (const u16*)d->resid_in, (u16*)d->resid_out,
+                        (const u16*)(joint ? d->gain2 : d->gain1), (const u16*)d->gain2, (u16*)d->out1, (u16*)d->out2,
+                        d->sums1, d->sums2, joint};
+  hipStream_t s = (hipStream_t)stream;
+  if (pr[0].rpw > 16) return launch_resid_rows<2, 16>(pr[0], M, rn, s);
+  return pr[0].rpw > 8 ? launch_resid_rows<1, 16>(pr[0], M, rn, s) : launch_resid_rows<1, 8>(pr[0], M, rn, s);
+}
+
 #ifdef LR_BAND_PROFILE
 // Profile builds only (not declared in the public header): following launches of this file's kernels record, per
 // wave, the six wall-clock stamps of stream_band.h into `device_buffer` (NULL switches it off).  Returns the
@@ -157,16 +259,19 @@ extern "C" long long lr_band_profile(void* device_buffer, int workgroups) {
 
 // lr_linear_fp8_multi (gemv_fp8.hip) for 3 to 16 input rows: the same bands with e4m3 weights.
 namespace lr_detail {
-int stream_fp8_multi(const lr_projection_fp8_t* proj, int n_proj, int M, lr_stream_t stream) {
+int stream_fp8_multi(const lr_projection_fp8_t* proj, const lr_row_norm_t* norms, int n_proj, int M, lr_stream_t stream) {
   if (M < 1 || M > 16) return LR_E_UNSUPPORTED;
   Proj pr[2] = {};
   for (int i = 0; i < n_proj; ++i) {
-    const int rc = sb_fill_projection_fp8(proj[i], pr[i]);
+    int rc = sb_fill_projection_fp8(proj[i], pr[i]);
+    if (rc == LR_OK && norms) rc = sb_fill_norm(norms + i, pr[i]);
     if (rc != LR_OK) return rc;
   }
   const int ncu = lr_num_cus();
   if (ncu < 1) return LR_E_LAUNCH;
   const int units = pick_units_and_plan(pr, n_proj, M, ncu);
+  for (int i = 0; i < n_proj; ++i)
+    if (pr[i].fold_sums && pr[i].nwg < M) return LR_E_UNSUPPORTED;   // (a row per workgroup)
   hipStream_t s = (hipStream_t)stream;
   const int rc = M <= 8 ? launch_fp8<true>(pr[0], pr[1], M, units, s) : launch_fp8<false>(pr[0], pr[1], M, units, s);
   return rc != LR_OK ? rc : lr_launch_status();

@@ -30,12 +30,16 @@ _PROTOS = {
     "lr_linear_scratch": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_size_t,
                                   c_void_p]),
     "lr_linear_multi": (c_int, [c_void_p, c_int, c_int, c_void_p]),
+    "lr_linear_multi_normed": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p]),
+    "lr_linear_resid_sums": (c_int, [c_int]),
+    "lr_linear_resid": (c_int, [c_void_p, c_int, c_void_p]),
     "lr_linear_swiglu_out": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p,
                                      c_size_t, c_void_p]),
     "lr_linear_swiglu_out_scratch": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p,
                                              c_size_t, c_void_p, c_size_t, c_void_p]),
     "lr_linear_fp8_scratch_bytes": (c_size_t, [c_int, c_int, c_int]),
     "lr_linear_fp8_multi": (c_int, [c_void_p, c_int, c_int, c_void_p]),
+    "lr_linear_fp8_multi_normed": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p]),
     "lr_linear_fp8": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p,
                               c_size_t, c_void_p]),
     "lr_swiglu": (c_int, [c_void_p, c_int64, c_void_p, c_int, c_int, c_void_p]),
@@ -54,6 +58,11 @@ _PROTOS = {
                                       c_int, c_int, c_int, c_void_p, c_size_t, c_void_p, c_int, c_void_p]),
     "lr_attn_decode_beside_fp8": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int,
                                           c_int, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p, c_int, c_void_p]),
+    "lr_attn_decode_beside_normed": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
+                                             c_int, c_int, c_int, c_void_p, c_size_t, c_void_p, c_void_p, c_int, c_void_p]),
+    "lr_attn_decode_beside_fp8_normed": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int,
+                                                 c_int, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p, c_void_p, c_int,
+                                                 c_void_p]),
     "lr_attn_decode_static": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
                                       c_int, c_int, c_int, c_void_p]),
     "lr_attn_prefill": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
@@ -339,8 +348,84 @@ def linear_multi(*projections):
     EPI_SWIGLU -> w holds [up; gate] rows and out [M, N / 2] = silu(gate) * up; or, for the fused q/k/v
     projection of a decode step, (x, w, out, rope_kv_epilogue(...)): q rotated in out, k and v into the cache
     (lr_linear_multi)."""
+    projections, norms = _norms_of(projections)
     arr, M, _keep = _projection_array(projections)
-    _check(load().lr_linear_multi(ctypes.cast(arr, c_void_p), len(projections), M, _stream()), "lr_linear_multi")
+    _check(load().lr_linear_multi_normed(ctypes.cast(arr, c_void_p), norms, len(projections), M, _stream()), "lr_linear_multi_normed")
+
+
+ROW_NORM_MAX_ROWS = 16   # LR_ROW_NORM_MAX_ROWS of include/ladder_hip.h
+_ROW_NORM_MAX = 512      # LR_ROW_NORM_MAX
+
+
+class _RowNorm(ctypes.Structure):   # lr_row_norm_t
+    _fields_ = [("sums", c_void_p), ("count", c_int32), ("dim", c_int32), ("eps", c_float), ("fold_sums", c_void_p),
+                ("fold_total", c_void_p), ("fold_count", c_int32)]
+
+
+class Normed:
+    """Projection input whose rows have a norm's gain and are still to be divided by their root mean square, `sums` [M, count]
+    holding the parts of their sums of squares (linear_resid makes both): the projection divides its results."""
+
+    def __init__(self, x: torch.Tensor, sums: torch.Tensor, eps: float, fold=None):
+        """fold: (parts [M, count], total [M, 1]) of another norm's sums of squares, which the launch adds for a later one."""
+        for t in (sums, *(fold or ())):
+            assert t.dtype == torch.float32 and t.is_contiguous() and t.shape[0] == x.shape[0]
+        assert fold is None or fold[1].shape[1] == 1
+        self.x, self.sums, self.eps, self.fold = x, sums, eps, fold
+
+
+def _norms_of(projections):
+    """(the projections with plain inputs, lr_row_norm_t array or None)"""
+    if not any(isinstance(p[0], Normed) for p in projections):
+        return projections, None
+    norms = (_RowNorm * len(projections))()
+    plain = []
+    for i, (x, *rest) in enumerate(projections):
+        if isinstance(x, Normed):
+            norms[i] = _RowNorm(_dev(x.sums, torch.float32), x.sums.shape[1], x.x.shape[1], x.eps)
+            if x.fold is not None:
+                parts, total = x.fold
+                norms[i].fold_sums, norms[i].fold_total = _dev(parts, torch.float32), _dev(total, torch.float32)
+                norms[i].fold_count = parts.shape[1]
+            x = x.x
+        plain.append((x, *rest))
+    return tuple(plain), norms
+
+
+class _LinearResid(ctypes.Structure):   # lr_linear_resid_t
+    _fields_ = [(n, c_void_p) for n in ("x1", "w1", "scales1", "x2", "w2", "scales2")] + [("ldx1", c_int64), ("ldx2", c_int64)] + \
+               [(n, c_int32) for n in ("K1", "K2", "D")] + \
+               [(n, c_void_p) for n in ("resid_in", "resid_out", "gain1", "gain2", "out1", "out2", "sums1", "sums2")] + [("joint", c_int32)]
+
+
+def linear_resid_sums(dim: int) -> int:
+    """Values per row that linear_resid leaves of a sum of squares; 0: rows of this width are not served."""
+    n = int(load().lr_linear_resid_sums(dim))
+    return n if n <= _ROW_NORM_MAX else 0
+
+
+def linear_resid(first, second, resid, joint=False):
+    """resid[M, D] += x w^T of `first` and then of `second`, each (x, module, gain, out, sums); out =
+    the updated residual times the gain, sums [M, linear_resid_sums(D)] = parts of its sum of squares: together an input for
+    Normed (lr_linear_resid).  joint: resid += second's + first's, the sum rounded first, and `first` has no (gain, out, sums)."""
+    M, D = resid.shape
+    d = _LinearResid(joint=joint, D=D, resid_in=_dev(resid), resid_out=_dev(resid))
+    assert resid.is_contiguous()
+    for i, (x, lin, *rest) in enumerate((first, second), 1):
+        m, K, ldx = _rows_ld(x)
+        w, scales = lin.weight, getattr(lin, "scales", None)
+        assert m == M and tuple(w.shape) == (D, K) and w.is_contiguous() and w.is_cuda
+        assert w.dtype == (torch.bfloat16 if scales is None else torch.float8_e4m3fn)
+        args = [("x", _dev(x)), ("w", w.data_ptr()), ("scales", None if scales is None else _dev(scales)), ("ldx", ldx), ("K", K)]
+        assert bool(rest) != (joint and i == 1)
+        if rest:
+            gain, out, sums = rest
+            assert gain.numel() == D and tuple(out.shape) == (M, D) and out.is_contiguous()
+            assert tuple(sums.shape) == (M, linear_resid_sums(D)) and sums.is_contiguous()
+            args += [("gain", _dev(gain)), ("out", _dev(out)), ("sums", _dev(sums, torch.float32))]
+        for name, v in args:
+            setattr(d, name + str(i), v)
+    _check(load().lr_linear_resid(ctypes.byref(d), M, _stream()), "lr_linear_resid")
 
 
 def _projection_array(projections):
@@ -373,8 +458,10 @@ class _ProjectionFp8(ctypes.Structure):
 def linear_fp8_multi(*projections):
     """linear_multi for weight-only e4m3 projections of the same M <= 16 rows (lr_linear_fp8_multi).  Each projection
     is (x [M, K], w8 [N, K] float8_e4m3fn, scales [N], out, epilogue), epilogue as in linear_multi."""
+    projections, norms = _norms_of(projections)
     arr, M, _keep = _projection_fp8_array(projections)
-    _check(load().lr_linear_fp8_multi(ctypes.cast(arr, c_void_p), len(projections), M, _stream()), "lr_linear_fp8_multi")
+    _check(load().lr_linear_fp8_multi_normed(ctypes.cast(arr, c_void_p), norms, len(projections), M, _stream()),
+           "lr_linear_fp8_multi_normed")
 
 
 def attn_decode_beside_fp8(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, projection) -> bool:
@@ -384,10 +471,11 @@ def attn_decode_beside_fp8(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd,
     _, _, ldy = _rows_ld(y)
     Smax = k_cache.shape[2]
     assert pos.dtype == torch.int32 and pos.numel() == 1 and scratch.dtype == torch.float32
+    (projection,), norms = _norms_of((projection,))
     arr, M, _keep = _projection_fp8_array((projection,))
-    rc = load().lr_attn_decode_beside_fp8(_dev(q), ldq, _dev(k_cache), _dev(v_cache), pos.data_ptr(), _dev(y), ldy, B,
-                                          Hq, Hkv, hd, Smax, scratch.data_ptr(), scratch.numel() * 4,
-                                          ctypes.cast(arr, c_void_p), M, _stream())
+    rc = load().lr_attn_decode_beside_fp8_normed(_dev(q), ldq, _dev(k_cache), _dev(v_cache), pos.data_ptr(), _dev(y), ldy, B,
+                                                 Hq, Hkv, hd, Smax, scratch.data_ptr(), scratch.numel() * 4,
+                                                 ctypes.cast(arr, c_void_p), norms, M, _stream())
     if rc == E_UNSUPPORTED:
         return False
     _check(rc, "lr_attn_decode_beside_fp8")
@@ -581,10 +669,11 @@ def attn_decode_beside(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, pro
     _, _, ldy = _rows_ld(y)
     Smax = k_cache.shape[2]
     assert pos.dtype == torch.int32 and pos.numel() == 1 and scratch.dtype == torch.float32
+    (projection,), norms = _norms_of((projection,))
     arr, M, _keep = _projection_array((projection,))
-    rc = load().lr_attn_decode_beside(_dev(q), ldq, _dev(k_cache), _dev(v_cache), pos.data_ptr(), _dev(y), ldy, B, Hq,
-                                      Hkv, hd, Smax, scratch.data_ptr(), scratch.numel() * 4,
-                                      ctypes.cast(arr, c_void_p), M, _stream())
+    rc = load().lr_attn_decode_beside_normed(_dev(q), ldq, _dev(k_cache), _dev(v_cache), pos.data_ptr(), _dev(y), ldy, B, Hq,
+                                             Hkv, hd, Smax, scratch.data_ptr(), scratch.numel() * 4,
+                                             ctypes.cast(arr, c_void_p), norms, M, _stream())
     if rc == E_UNSUPPORTED:
         return False
     _check(rc, "lr_attn_decode_beside")

@@ -59,6 +59,11 @@ class Workspace:
                 cus = torch.cuda.get_device_properties(device).multi_processor_count if device.type == "cuda" else 256
                 n = min(n, cus * 25 // 32 << 15)
             self.sums_mlp = torch.empty(n, dtype=torch.uint8, device=device)
+        # decode batches whose output projections leave the next norms' inputs undivided, with parts of the sums of squares
+        self.resid_sums = _hip.linear_resid_sums(D) if S == 1 and 1 < B <= _hip.ROW_NORM_MAX_ROWS and device.type == "cuda" else 0
+        if self.resid_sums:
+            self.sq, self.sq2 = (torch.empty(rows, self.resid_sums, dtype=torch.float32, device=device) for _ in range(2))
+            self.sq2_total = torch.empty(rows, 1, dtype=torch.float32, device=device)
         if S == 1:
             n = _hip.attn_decode_scratch_bytes(B, cfg.n_head_local, hd, smax) // 4
             self.scratch = torch.empty(n, dtype=torch.float32, device=device)

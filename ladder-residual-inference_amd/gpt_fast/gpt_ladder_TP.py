@@ -130,7 +130,8 @@ class GPTLadder(GPTBase):
         updates and both norms of a block (lr_ladder_norms: the MLP's input does not contain the block's own
         attention output), then the attention chain (wqkv, RoPE + cache write, attention, wo) and the MLP chain
         (w1, SwiGLU, w2) -- one after the other, or on two streams where the reference overlaps an all-reduce with
-        the next module (gpt_ladder_TP.py:339-349)."""
+        the next module (gpt_ladder_TP.py:339-349).  Up to 16 rows the norms launch is only the first block's: from then on
+        the output projections update the residual and leave the next block its rows undivided (linear_resid)."""
         cfg = self.config
         eps = cfg.norm_eps
         main = side = None
@@ -161,9 +162,12 @@ class GPTLadder(GPTBase):
         # weight-only e4m3 projections, up to 16 rows: the same two launches per block (lr_linear_fp8_multi)
         multi8 = side is None and fp8 and ws.B <= 16
         beside8 = multi8   # (declined by the library for a single row, where the projections are no bands)
-        for blk in self.layers:
-            _hip.ladder_norms(ws.x, pending_a, pending_m, blk.attention_norm.weight, blk.ffn_norm.weight, ws.x, ws.xn,
-                              ws.xn2, eps)
+        xn, xn2 = ws.xn, ws.xn2
+        resid = ws.resid_sums and (multi or multi8)
+        for blk, after in zip(self.layers, [*self.layers[1:], None]):
+            if not isinstance(xn, _hip.Normed):
+                _hip.ladder_norms(ws.x, pending_a, pending_m, blk.attention_norm.weight, blk.ffn_norm.weight, ws.x, ws.xn,
+                                  ws.xn2, eps)
             if two_chains:
                 chain.wait_stream(cur)
                 with torch.cuda.stream(chain):
@@ -174,27 +178,29 @@ class GPTLadder(GPTBase):
                 kv = blk.attention.kv_cache
                 rope = _hip.rope_kv_epilogue(self.freqs_cis, pos, kv.k_cache, kv.v_cache, cfg.n_head_local,
                                              cfg.n_kv_local, cfg.head_dim)
-                up_gate = (ws.xn2, blk.feed_forward.w1.weight, ws.act, _hip.EPI_SWIGLU)
+                up_gate = (xn2, blk.feed_forward.w1.weight, ws.act, _hip.EPI_SWIGLU)
                 if beside:
                     # up to 16 rows the up/gate bands leave room for a second workgroup per CU: the attention's
                     # items run in the same launch and wait for the KV cache behind the weight stream
-                    _hip.linear_multi((ws.xn, blk.attention.wqkv.weight, ws.qkv, rope))
+                    _hip.linear_multi((xn, blk.attention.wqkv.weight, ws.qkv, rope))
                     beside = _hip.attn_decode_beside(ws.qkv, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B,
                                                      cfg.n_head_local, cfg.n_kv_local, cfg.head_dim, up_gate)
                     if not beside:
                         _hip.linear_multi(up_gate)
                         self._attention(ws, blk, pos, None, None, roped=True)
                 else:
-                    _hip.linear_multi((ws.xn, blk.attention.wqkv.weight, ws.qkv, rope), up_gate)
+                    _hip.linear_multi((xn, blk.attention.wqkv.weight, ws.qkv, rope), up_gate)
                     self._attention(ws, blk, pos, None, None, roped=True)
-                _hip.linear_multi((ws.y, blk.attention.wo.weight, ws.a, _hip.EPI_NONE),
-                                  (ws.act, blk.feed_forward.w2.weight, ws.m, _hip.EPI_NONE))
+                if not (resid and after):
+                    xn, xn2 = ws.xn, ws.xn2
+                    _hip.linear_multi((ws.y, blk.attention.wo.weight, ws.a, _hip.EPI_NONE),
+                                      (ws.act, blk.feed_forward.w2.weight, ws.m, _hip.EPI_NONE))
             elif multi8:
                 att, ff, kv = blk.attention, blk.feed_forward, blk.attention.kv_cache
                 rope = _hip.rope_kv_epilogue(self.freqs_cis, pos, kv.k_cache, kv.v_cache, cfg.n_head_local,
                                              cfg.n_kv_local, cfg.head_dim)
-                qkv8 = (ws.xn, att.wqkv.weight, att.wqkv.scales, ws.qkv, rope)
-                up_gate8 = (ws.xn2, ff.w1.weight, ff.w1.scales, ws.act, _hip.EPI_SWIGLU)
+                qkv8 = (xn, att.wqkv.weight, att.wqkv.scales, ws.qkv, rope)
+                up_gate8 = (xn2, ff.w1.weight, ff.w1.scales, ws.act, _hip.EPI_SWIGLU)
                 if beside8:
                     _hip.linear_fp8_multi(qkv8)
                     beside8 = _hip.attn_decode_beside_fp8(ws.qkv, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B,
@@ -205,8 +211,10 @@ class GPTLadder(GPTBase):
                 else:
                     _hip.linear_fp8_multi(qkv8, up_gate8)
                     self._attention(ws, blk, pos, None, None, roped=True)
-                _hip.linear_fp8_multi((ws.y, att.wo.weight, att.wo.scales, ws.a, _hip.EPI_NONE),
-                                      (ws.act, ff.w2.weight, ff.w2.scales, ws.m, _hip.EPI_NONE))
+                if not (resid and after):
+                    xn, xn2 = ws.xn, ws.xn2
+                    _hip.linear_fp8_multi((ws.y, att.wo.weight, att.wo.scales, ws.a, _hip.EPI_NONE),
+                                          (ws.act, ff.w2.weight, ff.w2.scales, ws.m, _hip.EPI_NONE))
             elif side is not None:
                 side.wait_stream(main)
                 with torch.cuda.stream(side):
@@ -217,6 +225,13 @@ class GPTLadder(GPTBase):
                 self._attention(ws, blk, pos, blk.attention.wqkv, ws.a)
                 self._mlp(ws, blk, ws.m, ws.xn2)
             pending_a, pending_m = ws.a, ws.m
+            if resid and after:
+                _hip.linear_resid((ws.y, blk.attention.wo, after.attention_norm.weight, ws.xn, ws.sq),
+                                  (ws.act, blk.feed_forward.w2, after.ffn_norm.weight, ws.xn2, ws.sq2), ws.x)
+                if beside or beside8:   # (up/gate has its own, larger launch: q/k/v's adds the parts of its sums of squares)
+                    xn, xn2 = _hip.Normed(ws.xn, ws.sq, eps, (ws.sq2, ws.sq2_total)), _hip.Normed(ws.xn2, ws.sq2_total, eps)
+                else:
+                    xn, xn2 = _hip.Normed(ws.xn, ws.sq, eps), _hip.Normed(ws.xn2, ws.sq2, eps)
         return pending_a, pending_m
 
     def _run_layers(self, ws: Workspace, pos: Tensor):

@@ -81,14 +81,15 @@ class GPTParallel(GPTBase):
         cfg = self.config
         Hq, Hkv, hd = cfg.n_head_local, cfg.n_kv_local, cfg.head_dim
         q = ws.qkv[:, :nqkv]
-        pending = None
-        for blk in self.layers:
+        pending, xn, xu = None, ws.xn, ws.xn
+        for blk, after in zip(self.layers, [*self.layers[1:], None]):
             att, kv = blk.attention, blk.attention.kv_cache
-            _hip.add_rmsnorm(ws.x, pending, None, blk.attention_norm.weight, None if pending is None else ws.x, ws.xn,
-                             cfg.norm_eps)
+            if xn is ws.xn:
+                _hip.add_rmsnorm(ws.x, pending, None, blk.attention_norm.weight, None if pending is None else ws.x, ws.xn,
+                                 cfg.norm_eps)
             w = att.wqkv1.weight
-            qkv = (ws.xn, w[:nqkv], q, _hip.rope_kv_epilogue(self.freqs_cis, pos, kv.k_cache, kv.v_cache, Hq, Hkv, hd))
-            up_gate = (ws.xn, w[nqkv:], ws.act, _hip.EPI_SWIGLU)
+            qkv = (xn, w[:nqkv], q, _hip.rope_kv_epilogue(self.freqs_cis, pos, kv.k_cache, kv.v_cache, Hq, Hkv, hd))
+            up_gate = (xu, w[nqkv:], ws.act, _hip.EPI_SWIGLU)
             if ws.B > self.band_rows_to:
                 _hip.linear_rope_kv(ws.xn, w[:nqkv], q, self.freqs_cis, pos, kv.k_cache, kv.v_cache, ws.B, 1, Hq, Hkv, hd, ws.sums)
                 _hip.linear_swiglu_out(ws.xn, w[nqkv:], ws.act, sums=ws.sums)
@@ -103,6 +104,14 @@ class GPTParallel(GPTBase):
             else:
                 _hip.linear_multi(qkv, up_gate)
                 _hip.attn_decode(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd)
+            if ws.resid_sums and after is not None and blk.keeps_residual:
+                # both sums go to the residual and the next norm's undivided rows come with parts of their sums of squares,
+                # which the q/k/v launch adds for up/gate
+                _hip.linear_resid((ws.y, att.wo), (ws.act, att.w2, after.attention_norm.weight, ws.xn, ws.sq2), ws.x, joint=True)
+                xn = _hip.Normed(ws.xn, ws.sq2, cfg.norm_eps, (ws.sq2, ws.sq2_total))
+                xu, pending = _hip.Normed(ws.xn, ws.sq2_total, cfg.norm_eps), None
+                continue
+            xn = xu = ws.xn
             if ws.B <= self.band_rows_to:
                 _hip.linear_multi((ws.y, att.wo.weight, ws.a, _hip.EPI_NONE), (ws.act, att.w2.weight, ws.m, _hip.EPI_NONE))
             _hip.add(ws.m, ws.a, ws.m)                               # w2(...) + wo(...)

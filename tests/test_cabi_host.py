@@ -415,3 +415,19 @@ def test_products_with_memory_for_partial_sums_refuse_what_the_ones_without_refu
     # the projection's buffer may be missing for up to 64 rows and for large grids, not in between
     for M, N in ((65, 48), (511, 1 << 16), (1536, 7936)):      # (186 tiles of 256 rows x 128 pairs)
         assert swiglu(M=M, N=N, ldy=N // 2) == E_NULL
+
+
+def test_linear_resid_refuses_what_it_cannot_serve(lib):
+    """Checked before anything is launched: missing parts, more rows than its bands hold, misaligned rows."""
+    from gpt_fast import _hip
+
+    def rc(M=4, **kw):
+        d = _hip._LinearResid(**{**dict(x1=256, w1=256, x2=256, w2=256, ldx1=64, ldx2=64, K1=64, K2=64, D=64, resid_in=256, resid_out=256,
+                                        gain1=256, gain2=256, out1=256, out2=256, sums1=256, sums2=256), **kw})
+        return lib.lr_linear_resid(ctypes.byref(d), M, None)
+
+    assert lib.lr_linear_resid(None, 4, None) == -1
+    for name in ("x1", "w1", "x2", "w2", "gain1", "gain2", "out1", "out2", "sums1", "sums2", "resid_in", "resid_out"):
+        assert rc(**{name: None}) == -1, name
+    assert rc(joint=1, gain2=None) == -1 and rc(M=0) == -3 and rc(M=17) == -4
+    assert rc(K1=60) == -2 and rc(ldx2=60) == -3 and rc(w1=250) == -2

@@ -1001,3 +1001,69 @@ def test_decode_batches_beyond_the_reach_of_the_gemm_stay_with_the_bands(hip):
     hip.rope_kv_write(want, table, False, pos, *(torch.empty_like(kc) for _ in range(2)), M, 1, 4, 1, 8)
     assert torch.equal(plain, want) and torch.equal(vc[:, 0, 3], want[:, 40:])
     hip.raise_on_device_error(plain.device)
+
+
+def quantised(w):
+    """(e4m3 bytes, scales, the values they stand for in float64)"""
+    scale = (w.float().abs().amax(1) / 448.0).clamp_min(2.0 ** -20).to(BF)
+    w8 = (w.float() / scale.float()[:, None]).clamp(-448, 448).to(torch.float8_e4m3fn)
+    return w8, scale
+
+
+# bands of 2, 8, 9 (with a ragged last one), 16 and 32 columns; K within a chunk, ragged and of many chunks; the first and the last
+# row counts of both input layouts
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("M,D,K1,K2", [(2, 264, 48, 1040), (8, 2048, 256, 272), (9, 2056, 1040, 48), (16, 4096, 512, 1552), (7, 8192, 1024, 3584),
+                                       (12, 8192, 272, 1024)])
+def test_linear_resid_and_the_projections_of_its_rows(hip, M, D, K1, K2, fp8):
+    """Output projections with the residual updates, then a projection of the undivided rows they leave, each against the
+    float64 product of what it was given: one bf16 step per rounding between input and result (sums of fp32 products are
+    far closer than that), and the sums of squares to fp32 accuracy."""
+    class Lin:
+        pass
+    dq = lambda l: l.weight.double() * l.scales.double()[:, None] if fp8 else l.weight.double()
+    lins = []
+    for i, K in enumerate((K1, K2)):
+        l = Lin()
+        l.weight = rnd(D, K, seed=120 + i, scale=K ** -0.5)
+        if fp8:
+            l.weight, l.scales = quantised(l.weight)
+        lins.append(l)
+    xs = [rnd(M, K, seed=122 + i) for i, K in enumerate((K1, K2))]
+    gains = [rnd(D, seed=124 + i) * 0.1 + 1 for i in range(2)]
+    resid0 = rnd(M, D, seed=126) * 4
+    n = hip.linear_resid_sums(D)
+    assert n == -(-D // (-(-D // 256)))
+    a, m = (x.double() @ dq(l).T for x, l in zip(xs, lins))
+    step = lambda t: 2.0 ** -8 * t.abs()          # half a bf16 step
+    w, eps = rnd(512, D, seed=127, scale=D ** -0.5), 1e-5
+
+    def project(x, sums, fold=None):
+        y = torch.full((M, 516), 5.0, dtype=BF, device=DEV)
+        hip.linear_multi((hip.Normed(x, sums, eps, fold), w, y[:, :512], hip.EPI_NONE))
+        rs = torch.rsqrt(sums.double().sum(1, keepdim=True) / D + eps)
+        want = x.double() @ w.double().T * rs
+        assert ((y[:, :512].double() - want).abs() <= 1.01 * step(want) + 1e-5).all() and (y[:, 512:] == 5.0).all()
+        return y
+
+    for joint in (False, True):
+        resid, outs = resid0.clone(), [torch.full((M, D), 7.0, dtype=BF, device=DEV) for _ in range(2)]
+        sums = [torch.full((M, n), 7.0, device=DEV) for _ in range(2)]
+        first = (xs[0], lins[0]) if joint else (xs[0], lins[0], gains[0], outs[0], sums[0])
+        hip.linear_resid(first, (xs[1], lins[1], gains[1], outs[1], sums[1]), resid, joint=joint)
+        r0, got = resid0.double(), resid.double()
+        r1 = r0 + a
+        want = r1 + m
+        bound = (2 if fp8 else 1) * (step(a) + step(m)) + step(r1) + step(a + m) + step(want)    # (rounded before a scale too)
+        assert ((got - want).abs() <= 1.05 * bound + 1e-4).all()
+        assert torch.equal(outs[1], (got * gains[1].double()).to(BF))
+        assert torch.allclose(sums[1].double().sum(1), got.square().sum(1), rtol=1e-5)
+        if not joint:    # what the first update leaves is not stored: its rows to the same bounds
+            assert ((outs[0].double() / gains[0].double() - r1).abs() <= 1.05 * (bound + step(r1)) + 1e-4).all()
+            assert torch.allclose(sums[0].double().sum(1), r1.square().sum(1), rtol=2e-2)
+        else:
+            assert (outs[0] == 7.0).all() and (sums[0] == 7.0).all()
+        total = torch.full((M, 1), 7.0, device=DEV)
+        y = project(outs[1], sums[1], (sums[1], total))
+        assert torch.allclose(total[:, 0].double(), sums[1].double().sum(1), rtol=1e-6)
+        assert (ulp_diff(project(outs[1], total), y) <= 1).all()
