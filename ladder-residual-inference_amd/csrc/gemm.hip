@@ -562,32 +562,26 @@ struct GemmPlan {
   int tile;        // index into GEMM_TILES; -1: no tile serves the shape
   int full, rem, splits;
 };
-// What it decides, measured (us, weights from HBM; rows, N x K: with all the memory it could use | without any):
-//   777 rows,  4096 x 14336   117 (64 tiles of 256 x 256 in 4 pieces)      | 110 (224 of 128 x 128)
-//   777 rows,  4096 x  4096    34 (224 tiles of 128 x 128)                 |  the same
-//   300 rows,  4096 x 14336    57 (48 tiles of 128 x 256 in 5)             | 102 (160 of 64 x 128)
-//   128 rows,  2048 x  8192    22 (32 tiles of 64 x 128 in 16)             |  55
-//   128 rows, 16384 x  2048    24 (256 pair tiles of 64 x 128)             |  the same
-//  2048 rows,  4096 x 14336   189 (128 tiles of 256 x 256 in 2)            | 198 (256 of 128 x 256)
-//  3002 rows, 28672 x  4096   564 (1280 pair tiles whole, 64 in 4)         | 577 (1344 whole)
-//    64 rows,  1280 x  8192    16 (10 tiles of 64 x 128 in 16)             |  55   (the bands of stream_band.h 24)
-//    64 rows,  7168 x  8192    34 (56 pair tiles of 64 x 128 in 4)         |  60   (bands 38)
-//    64 rows,  8192 x  3584    20 (64 tiles of 64 x 128 in 3)              |  29   (bands 24)
-//    64 rows, 28672 x  4096    53 (224 pair tiles of 64 x 128)             |  the same   (bands 78)
-//    64 rows,  4096 x 14336    34 (32 tiles of 64 x 128 in 7)              |  97   (in 6 pieces 32)
-// Where it errs: the first line (98 and 106 when the costs below were fitted) and the last.
 // A workgroup's time is nk * (ktile + busy * slope) + fixed, `busy` the workgroups per CU: the more CUs are at work, the
-// lower the clock and the more of them ask the L2s (256 x 256: 1.05 us per k-tile on a quarter of the chip, 1.41 on all of
-// it); `cold` in place of the slope where a single row tile reads every weight from HBM itself; `pair` where two share a CU.
-// The weights need their time on the way from HBM whatever the tiles.  Pieces cost a launch and their trip through memory.
+// lower the clock and the more of them ask the L2s; `cold` in place of the slope where a single row tile reads every weight
+// from HBM itself; `pair` where two share a CU, `pair_cold` while up to two row tiles share a weight: then both wait for HBM,
+// and a k-tile costs almost what two in turn do.  The weights need their time on the way from HBM whatever the tiles.
+// Pieces cost a launch, their trip through memory and the ramp of each.
+// The costs are fitted to 219 products (33 to 3002 rows of 14 weights between 1280 x 8192 and 128256 x 4096, every tile,
+// whole and in 2 to 16 pieces, weights from HBM): what the plan takes is 1.0 % above the best of all on average, and 23 % at
+// worst (192 rows, 3072 x 2048: 17.1 us, 13.9 in three pieces); fitted without `pair_cold` and the ramp, on fewer rows, it was
+// 3.8 % and 37 %.  Some of them, us, N x K, chosen before / now | the best there is:
+//    64 rows,  3072 x  2048   12.3 / 11.2 | 10.8        128 rows,  2048 x  8192   19.6 / 16.2 | 16.2
+//    64 rows, 11264 x  4096   31.1 / 25.4 | 25.4        128 rows,  3072 x  2048   17.2 / 13.0 | 12.8
+//   128 rows,  4096 x 14336   38.5 / 33.0 | 33.0        128 rows, 28672 x  4096   64.4 / 52.4 | 52.4 (pairs)
 struct GemmTileCost {
   int a16, bh, per_cu;
-  float ktile, slope, cold, pair, fixed;
+  float ktile, slope, cold, pair, pair_cold, fixed;
 };
-constexpr GemmTileCost GEMM_TILES[4] = {{4, 2, 1, 0.95f, 0.46f, 1.4f, 0.0f, 5.0f},
-                                         {2, 2, 1, 0.58f, 0.29f, 1.6f, 0.0f, 3.0f},
-                                         {2, 1, 2, 0.44f, 0.06f, 0.5f, 0.92f, 3.0f},
-                                         {1, 1, 2, 0.27f, 0.26f, 0.4f, 0.72f, 2.5f}};
+constexpr GemmTileCost GEMM_TILES[4] = {{4, 2, 1, 0.961f, 0.424f, 0.157f, 0.0f, 0.0f, 5.76f},
+                                         {2, 2, 1, 0.576f, 0.302f, 0.661f, 0.0f, 0.0f, 3.01f},
+                                         {2, 1, 2, 0.485f, 0.0676f, 0.284f, 0.955f, 2.39f, 2.72f},
+                                         {1, 1, 2, 0.266f, 0.235f, 0.293f, 0.988f, 0.846f, 2.88f}};
 constexpr size_t GEMM_SCRATCH = (size_t)64 << 20;   // pieces of one round of the largest tiles
 constexpr int GEMM_SCRATCH_FROM = 33;               // rows from which a projection that has memory for pieces is one of this file's
 
@@ -597,7 +591,7 @@ static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
   int cus = lr_num_cus();
   if (cus <= 0) cus = 256;
   const int nk = (K + 63) / 64;
-  const float weights_us = (float)N * (mode == GEMM_PAIR ? 2 : 1) * K * 2 / 5.5e6f;
+  const float weights_us = (float)N * (mode == GEMM_PAIR ? 2 : 1) * K * 2 / 5.96e6f;
   float best_us = 0;
   for (int c = 0; c < 4; ++c) {
     const GemmTileCost& t = GEMM_TILES[c];
@@ -607,7 +601,7 @@ static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
     const int left = (int)(tiles - rounds * slots);
     auto round_us = [&](int workgroups, int k) {
       const float busy = (float)workgroups / cus;
-      return k * (busy > 1.0f ? t.pair : t.ktile + busy * (M <= TM ? t.cold : t.slope));
+      return k * (busy > 1.0f ? (M <= 2 * TM ? t.pair_cold : t.pair) : t.ktile + busy * (M <= TM ? t.cold : t.slope));
     };
     auto consider = [&](float us, float more, const GemmPlan& p) {
       us = (us > weights_us ? us : weights_us) + more;
@@ -621,7 +615,7 @@ static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
     for (int s = 2; left && s <= 16 && 4 * s <= nk && left * s <= slots; ++s) {
       const size_t bytes = (size_t)left * s * (64 * t.a16) * (128 * t.bh) * sizeof(float);
       if (bytes > scratch) break;
-      consider(whole + round_us(left * s, (nk + s - 1) / s), fixed + 6.0f + bytes / 6.5e6f, GemmPlan{c, (int)tiles - left, left, s});
+      consider(whole + round_us(left * s, (nk + s - 1) / s), fixed + 4.56f + 0.0746f * s + bytes / 4.76e6f, GemmPlan{c, (int)tiles - left, left, s});
     }
   }
   return best;
