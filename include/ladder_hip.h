@@ -89,6 +89,11 @@ int lr_add_rmsnorm(const void* resid_in, const void* d1, const void* d2, const v
  * side by side, e.g. on two streams.  d1 / d2 may be NULL (the first block); resid_out may alias resid_in. */
 int lr_ladder_norms(const void* resid_in, const void* d1, const void* d2, const void* gain1, const void* gain2,
                     void* resid_out, void* normed1, void* normed2, int rows, int dim, float eps, lr_stream_t stream);
+/* The same; where pieces1 (pieces2) is not 0, d1 (d2) is fp32 [pieces][rows][dim], what lr_linear_pieces left: their sum, rounded
+ * to bf16, takes d1's (d2's) place. */
+int lr_ladder_norms_pieces(const void* resid_in, const void* d1, int pieces1, const void* d2, int pieces2, const void* gain1,
+                           const void* gain2, void* resid_out, void* normed1, void* normed2, int rows, int dim, float eps,
+                           lr_stream_t stream);
 
 /* y[m, n] = bf16( sum_k x[m, k] * w[n, k] )   x [M, K] (row stride ldx), w [N, K] dense,
  * y [M, N] (row stride ldy).  nn.Linear without bias: wqkv / wo (utils.py:191, 258), w1 / w2
@@ -121,6 +126,12 @@ typedef struct lr_linear_plan {
 int lr_linear_plan(int M, int N, int K, int pair, size_t scratch_bytes, lr_linear_plan_t* plan);
 int lr_linear_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, void* scratch,
                       size_t scratch_bytes, lr_stream_t stream);
+
+/* The sums of lr_linear_scratch's pieces before they are added, sums [pieces][M][N] fp32, for a launch that adds them itself
+ * (lr_ladder_norms_pieces); *pieces says how many.  LR_E_UNSUPPORTED, with nothing launched, where a product of this shape
+ * has tiles that are computed whole, up to 32 rows and for N % 4 != 0.  No counterpart in the reference. */
+int lr_linear_pieces(const void* x, int64_t ldx, const void* w, int M, int N, int K, void* sums, size_t sums_bytes, int32_t* pieces,
+                     lr_stream_t stream);
 
 /* lr_linear with the launch configuration of the GEMV given by the caller instead of chosen from
  * the shape: gemv_cfg = rows per wave * 100 + K-split * 10 + unroll, one of 144, 212, 222, 242, 244,
@@ -378,6 +389,28 @@ int lr_attn_decode_static(const void* q, int64_t ldq, const void* k_cache, const
  * rows, bit for bit. */
 int lr_attn_prefill(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos, void* y,
                     int64_t ldy, int B, int S, int Hq, int Hkv, int hd, int Smax, lr_stream_t stream);
+
+/* One block of a prompt in the all-ladder schedule (gpt_ladder_TP.py:312-358, M = B * S > 4 rows): lr_ladder_norms_pieces
+ * on the residual x and the outputs a and m of the block before, lr_linear_rope_kv of xn, lr_attn_prefill, lr_linear_swiglu_out
+ * of xn2, lr_linear with wo into a and with w2 into m, with products of one grid and partial sums left to the next block where
+ * that is faster.  The same arithmetic; the order of sums depends on the sizes.  Nothing is launched if a pointer or size is refused. */
+typedef struct lr_ladder_block {
+  int32_t B, S, dim, ffn;
+  float eps;
+  lr_rope_kv_t rope;   /* pos: int32 [S] */
+  void *x, *xn, *xn2;  /* [M, dim] */
+  void *qkv, *y;       /* [M, (n_head + 2 n_kv_head) head_dim], [M, n_head head_dim] */
+  void *act, *h;       /* [M, ffn], [M, 2 ffn] */
+  void *a, *m;         /* [M, dim] */
+  void *sums_a, *sums_m; /* sums_bytes each, both or neither: memory for partial sums, see lr_linear_scratch */
+  size_t sums_bytes;
+  const void *gain1, *gain2, *wqkv, *wo, *w1, *w2;
+  /* where the block before left its outputs, and then where this one does: 0 in a (m), n > 0 as n pieces in sums_a (sums_m),
+   * -1 (in only) there is none */
+  int32_t a_pieces, m_pieces;
+  int32_t finish; /* leave a and m themselves */
+} lr_ladder_block_t;
+int lr_ladder_block(lr_ladder_block_t* block, lr_stream_t stream);
 
 /* out[b] = argmax_v logits[b, v], lowest index on ties; logits [B, V] bf16 (row stride ldl),
  * out int32 [B].  Greedy stand-in for sample() (benchmark.py:73-77): torch.argmax(logits[:, -1]). */

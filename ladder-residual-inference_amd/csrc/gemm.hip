@@ -178,12 +178,13 @@ struct GemmGroup {
   int64_t xrows;           // rows of x
 };
 // Tiles [0, full) are computed whole; each of the `rem` tiles after them is cut along K into `splits` pieces, whose fp32
-// sums go to `part` in the order a wave holds them (k_gemm_sum adds them in order and finishes the tile).
+// sums go to `part` in the order a wave holds them (k_gemm_sum adds them in order and finishes the tile), or, in ROWS mode
+// (full == 0, N % 4 == 0), to part [splits][M][N] for a launch that needs whole rows anyway.
 struct GemmSplit {
   float* part;
   int full, rem, splits;
 };
-enum { GEMM_PLAIN, GEMM_PAIR, GEMM_ROPE };   // PAIR: w holds [up; gate] rows, N counts pairs, output silu(gate) * up
+enum { GEMM_PLAIN, GEMM_PAIR, GEMM_ROPE, GEMM_ROWS };   // ROWS: every tile is cut, the pieces stay, see GemmSplit; PAIR: w holds [up; gate] rows, N counts pairs, output silu(gate) * up
 
 template <int A16, int BH>
 struct GemmTile {
@@ -324,10 +325,10 @@ __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u1
 
 // KTAIL: K is not a multiple of the 64-element k-tile, so the last one needs a per-lane range check.  NT: weights are loaded
 // non-temporally.
-template <int A16, int BH, bool KTAIL, int MODE, bool GROUP, bool NT = false>
-__global__ __launch_bounds__(256, A16 * BH <= 2 ? 2 : 1) void k_gemm_dma(const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
-                                                                        u16* __restrict__ y, int64_t ldy, int M, int N, int K, int tm, int tn,
-                                                                        const GemmRope rp, const GemmSplit sp, const GemmGroup gp) {
+template <int A16, int BH, bool KTAIL, int MODE, bool GROUP, bool NT>
+__device__ __forceinline__ void gemm_tile(const int block, const int blocks, const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
+                                          u16* __restrict__ y, int64_t ldy, int M, int N, int K, int tm, int tn, const GemmRope& rp,
+                                          const GemmSplit& sp, const GemmGroup& gp) {
   using T = GemmTile<A16, BH>;
   constexpr int HA = T::HA, HB = T::HB, NA = T::NA, NB = T::NB, BOFF = 4 * HA;
   extern __shared__ __attribute__((aligned(1024))) u16 gsm[];
@@ -336,7 +337,7 @@ __global__ __launch_bounds__(256, A16 * BH <= 2 ? 2 : 1) void k_gemm_dma(const u
   int mt, nt, piece = -1, kt0 = 0, nk = (K + 63) / 64;
   int32_t* const entry = reinterpret_cast<int32_t*>(gsm + T::LDS / 2);   // (GROUP) the tile's entries
   if constexpr (GROUP) {
-    const int id = xcd_run(blockIdx.x, gridDim.x);   // a row tile's column tiles one after the other
+    const int id = xcd_run(block, blocks);   // a row tile's column tiles one after the other
     mt = id / tn;
     nt = id - mt * tn;
     if (mt >= gp.ntiles[0]) return;
@@ -347,7 +348,7 @@ __global__ __launch_bounds__(256, A16 * BH <= 2 ? 2 : 1) void k_gemm_dma(const u
     mt = 0;
     __syncthreads();
   } else {
-    int t = blockIdx.x;
+    int t = block;
     if (t < sp.full) {
       t = xcd_run(t, sp.full);
     } else {
@@ -510,7 +511,20 @@ __global__ __launch_bounds__(256, A16 * BH <= 2 ? 2 : 1) void k_gemm_dma(const u
   // way into LDS, nobody still reads it
   asm volatile("s_nop 15\n\ts_nop 15\n\ts_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   if constexpr (!GROUP) {
-    if (piece >= 0) {
+    if constexpr (MODE == GEMM_ROWS) {
+      float* const p = sp.part + (int64_t)(piece % sp.splits) * M * N;
+#pragma unroll
+      for (int a = 0; a < 2 * A16; ++a) {
+        const int m = m0 + a / A16 * 32 * A16 + wm * 16 * A16 + a % A16 * 16 + (lane & 15);
+#pragma unroll
+        for (int b = 0; b < 4 * BH; ++b) {
+          const int n = n0 + b / (2 * BH) * 64 * BH + wn * 32 * BH + b % (2 * BH) * 16 + (lane >> 4) * 4;
+          if (m < M && n < N) *reinterpret_cast<f32x4_t*>(p + (int64_t)m * N + n) = acc[a][b];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      return;
+    } else if (piece >= 0) {
       float* p = sp.part + (int64_t)piece * (T::TM * T::TN) + (int64_t)wave * (8 * A16 * BH * 256) + lane * 4;
 #pragma unroll
       for (int a = 0; a < 2 * A16; ++a) {
@@ -521,7 +535,39 @@ __global__ __launch_bounds__(256, A16 * BH <= 2 ? 2 : 1) void k_gemm_dma(const u
       return;
     }
   }
-  gemm_store<A16, BH, MODE, 2 * A16>(acc, gsm + wave * (T::EBYTES / 8), 0, wm, wn, m0, n0, y, ldy, M, N, rp, GROUP ? entry : nullptr);
+  if constexpr (MODE != GEMM_ROWS) gemm_store<A16, BH, MODE, 2 * A16>(acc, gsm + wave * (T::EBYTES / 8), 0, wm, wn, m0, n0, y, ldy, M, N, rp, GROUP ? entry : nullptr);
+}
+
+template <int A16, int BH, bool KTAIL, int MODE, bool GROUP, bool NT = false>
+__global__ __launch_bounds__(256, A16 * BH <= 2 ? 2 : 1) void k_gemm_dma(const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
+                                                                        u16* __restrict__ y, int64_t ldy, int M, int N, int K, int tm, int tn,
+                                                                        const GemmRope rp, const GemmSplit sp, const GemmGroup gp) {
+  gemm_tile<A16, BH, KTAIL, MODE, GROUP, NT>(blockIdx.x, gridDim.x, x, ldx, w, y, ldy, M, N, K, tm, tn, rp, sp, gp);
+}
+
+// Two products of as many rows in one grid, the first `n0` workgroups the first's.  A short prompt's products each leave most
+// of the chip idle or end with a ramp and a drain of their own; in a ladder block q/k/v and up/gate have their inputs at the
+// same time, and so have, behind the attention, wo and w2.
+struct GemmProduct {
+  const u16* x;
+  int64_t ldx;
+  const u16* w;
+  u16* y;
+  int64_t ldy;
+  int M, N, K, tm, tn;
+  GemmSplit sp;
+};
+template <int A16, int BH, int MODE0, int MODE1, bool NT>
+__global__ __launch_bounds__(256, A16 * BH <= 2 ? 2 : 1) void k_gemm_two(const GemmProduct a, const GemmProduct b, const int n0, const GemmRope rp) {
+  const bool second = (int)blockIdx.x >= n0;
+  if constexpr (MODE0 == MODE1) {
+    const GemmProduct p = second ? b : a;
+    gemm_tile<A16, BH, false, MODE0, false, NT>(blockIdx.x - (second ? n0 : 0), 0, p.x, p.ldx, p.w, p.y, p.ldy, p.M, p.N, p.K, p.tm, p.tn, rp, p.sp, GemmGroup{});
+  } else if (second) {
+    gemm_tile<A16, BH, false, MODE1, false, NT>(blockIdx.x - n0, 0, b.x, b.ldx, b.w, b.y, b.ldy, b.M, b.N, b.K, b.tm, b.tn, GemmRope{}, b.sp, GemmGroup{});
+  } else {
+    gemm_tile<A16, BH, false, MODE0, false, NT>(blockIdx.x, 0, a.x, a.ldx, a.w, a.y, a.ldy, a.M, a.N, a.K, a.tm, a.tn, rp, a.sp, GemmGroup{});
+  }
 }
 
 // The cut tiles: a workgroup adds the pieces of a 1 / (2 A16) part of one (16 rows per wave, four pieces' loads in flight
@@ -561,6 +607,7 @@ __global__ __launch_bounds__(256) void k_gemm_sum(u16* __restrict__ y, int64_t l
 struct GemmPlan {
   int tile;        // index into GEMM_TILES; -1: no tile serves the shape
   int full, rem, splits;
+  float us;        // what it should take
 };
 // A workgroup's time is nk * (ktile + busy * slope) + fixed, `busy` the workgroups per CU: the more CUs are at work, the
 // lower the clock and the more of them ask the L2s; `cold` in place of the slope where a single row tile reads every weight
@@ -568,9 +615,9 @@ struct GemmPlan {
 // and a k-tile costs almost what two in turn do.  The weights need their time on the way from HBM whatever the tiles.
 // Pieces cost a launch, their trip through memory and the ramp of each.
 // The costs are fitted to 219 products (33 to 3002 rows of 14 weights between 1280 x 8192 and 128256 x 4096, every tile,
-// whole and in 2 to 16 pieces, weights from HBM): what the plan takes is 1.0 % above the best of all on average, and 23 % at
-// worst (192 rows, 3072 x 2048: 17.1 us, 13.9 in three pieces); fitted without `pair_cold` and the ramp, on fewer rows, it was
-// 3.8 % and 37 %.  Some of them, us, N x K, chosen before / now | the best there is:
+// whole and in 2 to 16 pieces, weights from HBM) and to 90 more of up to 16384 rows, two plans of each: what the plan takes is
+// 1.1 % above the best of all on average, and 23 % at worst (192 rows, 3072 x 2048: 17.1 us, 13.9 in three pieces); fitted
+// without `pair_cold` and the ramp, on fewer rows, it was 3.8 % and 37 %.  Some of them, us, N x K, chosen before / now | the best there is:
 //    64 rows,  3072 x  2048   12.3 / 11.2 | 10.8        128 rows,  2048 x  8192   19.6 / 16.2 | 16.2
 //    64 rows, 11264 x  4096   31.1 / 25.4 | 25.4        128 rows,  3072 x  2048   17.2 / 13.0 | 12.8
 //   128 rows,  4096 x 14336   38.5 / 33.0 | 33.0        128 rows, 28672 x  4096   64.4 / 52.4 | 52.4 (pairs)
@@ -578,44 +625,49 @@ struct GemmTileCost {
   int a16, bh, per_cu;
   float ktile, slope, cold, pair, pair_cold, fixed;
 };
-constexpr GemmTileCost GEMM_TILES[4] = {{4, 2, 1, 0.961f, 0.424f, 0.157f, 0.0f, 0.0f, 5.76f},
-                                         {2, 2, 1, 0.576f, 0.302f, 0.661f, 0.0f, 0.0f, 3.01f},
-                                         {2, 1, 2, 0.485f, 0.0676f, 0.284f, 0.955f, 2.39f, 2.72f},
-                                         {1, 1, 2, 0.266f, 0.235f, 0.293f, 0.988f, 0.846f, 2.88f}};
+constexpr GemmTileCost GEMM_TILES[4] = {{4, 2, 1, 0.968f, 0.416f, 0.0848f, 0.0f, 0.0f, 5.94f},
+                                         {2, 2, 1, 0.576f, 0.304f, 0.658f, 0.0f, 0.0f, 3.05f},
+                                         {2, 1, 2, 0.486f, 0.0641f, 0.314f, 0.957f, 2.43f, 2.76f},
+                                         {1, 1, 2, 0.278f, 0.236f, 0.279f, 0.737f, 1.33f, 2.82f}};
 constexpr size_t GEMM_SCRATCH = (size_t)64 << 20;   // pieces of one round of the largest tiles
 constexpr int GEMM_SCRATCH_FROM = 33;               // rows from which a projection that has memory for pieces is one of this file's
 
+constexpr float GEMM_WEIGHT_BYTES_US = 5.98e6f, GEMM_SUM_US = 4.62f, GEMM_PIECE_US = 0.0884f, GEMM_PIECE_BYTES_US = 4.78e6f;
+
+// `workgroups` of k k-tiles each, at the same time
+static float gemm_round_us(const GemmTileCost& t, int M, int cus, int workgroups, int k) {
+  const float busy = (float)workgroups / cus;
+  const int TM = 64 * t.a16;
+  return k * (busy > 1.0f ? (M <= 2 * TM ? t.pair_cold : t.pair) : t.ktile + busy * (M <= TM ? t.cold : t.slope));
+}
+static int gemm_cus() {
+  const int cus = lr_num_cus();
+  return cus > 0 ? cus : 256;
+}
+
 static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
-  GemmPlan best{-1, 0, 0, 1};
+  GemmPlan best{-1, 0, 0, 1, 0.0f};
   if (M > 0x7fffffff - 256 || N > 0x7fffffff - 256 || K > 0x7fffffff - 256) return best;   // (row, column and k of the last tile are ints)
-  int cus = lr_num_cus();
-  if (cus <= 0) cus = 256;
-  const int nk = (K + 63) / 64;
-  const float weights_us = (float)N * (mode == GEMM_PAIR ? 2 : 1) * K * 2 / 5.96e6f;
-  float best_us = 0;
+  const int cus = gemm_cus(), nk = (K + 63) / 64;
+  const float weights_us = (float)N * (mode == GEMM_PAIR ? 2 : 1) * K * 2 / GEMM_WEIGHT_BYTES_US;
   for (int c = 0; c < 4; ++c) {
     const GemmTileCost& t = GEMM_TILES[c];
     const int TM = 64 * t.a16, TN = (mode == GEMM_PAIR ? 64 : 128) * t.bh, slots = cus * t.per_cu;
     const int64_t tiles = (int64_t)((M + TM - 1) / TM) * ((N + TN - 1) / TN), rounds = tiles / slots;
     if (tiles > 0x3fffffff) continue;
     const int left = (int)(tiles - rounds * slots);
-    auto round_us = [&](int workgroups, int k) {
-      const float busy = (float)workgroups / cus;
-      return k * (busy > 1.0f ? (M <= 2 * TM ? t.pair_cold : t.pair) : t.ktile + busy * (M <= TM ? t.cold : t.slope));
-    };
-    auto consider = [&](float us, float more, const GemmPlan& p) {
+    auto round_us = [&](int workgroups, int k) { return gemm_round_us(t, M, cus, workgroups, k); };
+    auto consider = [&](float us, float more, int whole, int cut, int pieces) {
       us = (us > weights_us ? us : weights_us) + more;
-      if (best.tile < 0 || us < best_us) {
-        best = p;
-        best_us = us;
-      }
+      if (best.tile < 0 || us < best.us) best = GemmPlan{c, whole, cut, pieces, us};
     };
     const float whole = rounds * round_us(slots, nk), fixed = (rounds + (left ? 1 : 0)) * t.fixed;
-    consider(whole + (left ? round_us(left, nk) : 0.0f), fixed, GemmPlan{c, (int)tiles, 0, 1});
+    consider(whole + (left ? round_us(left, nk) : 0.0f), fixed, (int)tiles, 0, 1);
     for (int s = 2; left && s <= 16 && 4 * s <= nk && left * s <= slots; ++s) {
       const size_t bytes = (size_t)left * s * (64 * t.a16) * (128 * t.bh) * sizeof(float);
       if (bytes > scratch) break;
-      consider(whole + round_us(left * s, (nk + s - 1) / s), fixed + 4.56f + 0.0746f * s + bytes / 4.76e6f, GemmPlan{c, (int)tiles - left, left, s});
+      consider(whole + round_us(left * s, (nk + s - 1) / s), fixed + GEMM_SUM_US + GEMM_PIECE_US * s + bytes / GEMM_PIECE_BYTES_US,
+               (int)tiles - left, left, s);
     }
   }
   return best;
@@ -631,7 +683,8 @@ static int gemm_run_as(const void* x, int64_t ldx, const void* w, void* y, int64
   const GemmSplit sp{(float*)scratch, p.full, p.rem, p.splits};
   k_gemm_dma<A16, BH, KTAIL, MODE, false, NT><<<dim3((unsigned)(p.full + p.rem * p.splits)), dim3(256), T::LDS, s>>>(
       (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, M, N, K, tm, tn, rp, sp, GemmGroup{});
-  if (p.rem) k_gemm_sum<A16, BH, MODE><<<dim3((unsigned)(p.rem * 2 * A16)), dim3(256), 0, s>>>((u16*)y, ldy, M, N, tm, tn, rp, sp);
+  if constexpr (MODE != GEMM_ROWS)
+    if (p.rem) k_gemm_sum<A16, BH, MODE><<<dim3((unsigned)(p.rem * 2 * A16)), dim3(256), 0, s>>>((u16*)y, ldy, M, N, tm, tn, rp, sp);
   return lr_launch_status();
 }
 template <int A16, int BH, bool KTAIL, bool NT = false>
@@ -639,6 +692,7 @@ static int gemm_run_mode(const void* x, int64_t ldx, const void* w, void* y, int
                          const GemmPlan& p, void* scratch, hipStream_t s) {
   if (mode == GEMM_PAIR) return gemm_run_as<A16, BH, KTAIL, GEMM_PAIR, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
   if (mode == GEMM_ROPE) return gemm_run_as<A16, BH, KTAIL, GEMM_ROPE, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+  if (mode == GEMM_ROWS) return gemm_run_as<A16, BH, KTAIL, GEMM_ROWS, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
   return gemm_run_as<A16, BH, KTAIL, GEMM_PLAIN, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
 }
 static int gemm_run(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, int mode, const GemmRope& rp,
@@ -670,6 +724,120 @@ static int gemm(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy,
   if (p.tile < 0) return LR_E_UNSUPPORTED;
   return gemm_run(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
 }
+
+// ---- two products of one grid, and products whose partial sums stay
+static GemmProduct gemm_product(int tile, int mode, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K) {
+  const GemmTileCost& t = GEMM_TILES[tile];
+  const int TM = 64 * t.a16, TN = (mode == GEMM_PAIR ? 64 : 128) * t.bh;
+  GemmProduct p = {(const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, M, N, K, (M + TM - 1) / TM, (N + TN - 1) / TN, GemmSplit{}};
+  p.sp.full = p.tm * p.tn;
+  p.sp.splits = 1;
+  return p;
+}
+template <int A16, int BH, int MODE0, int MODE1, bool NT>
+static int gemm_two_as(const GemmProduct& a, const GemmProduct& b, const GemmRope& rp, hipStream_t s) {
+  using T = GemmTile<A16, BH>;
+  static std::atomic<unsigned long long> raised{0};
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_two<A16, BH, MODE0, MODE1, NT>), T::LDS, raised)) return LR_E_LAUNCH;
+  const int n0 = a.sp.full + a.sp.rem * a.sp.splits, n1 = b.sp.full + b.sp.rem * b.sp.splits;
+  k_gemm_two<A16, BH, MODE0, MODE1, NT><<<dim3((unsigned)(n0 + n1)), dim3(256), T::LDS, s>>>(a, b, n0, rp);
+  return lr_launch_status();
+}
+template <int MODE0, int MODE1>
+static int gemm_two(int tile, const GemmProduct& a, const GemmProduct& b, const GemmRope& rp, hipStream_t s) {
+  if (tile == 0) return gemm_two_as<4, 2, MODE0, MODE1, false>(a, b, rp, s);
+  if (tile == 1) return gemm_two_as<2, 2, MODE0, MODE1, false>(a, b, rp, s);
+  if (tile == 2) return gemm_two_as<2, 1, MODE0, MODE1, false>(a, b, rp, s);
+  return a.M <= 64 ? gemm_two_as<1, 1, MODE0, MODE1, true>(a, b, rp, s) : gemm_two_as<1, 1, MODE0, MODE1, false>(a, b, rp, s);
+}
+
+namespace lr_detail {
+// The q/k/v projection of x0 (rotated and cached on its way out) and the up/gate projection of x1 (activated), M rows, in one
+// launch where that should take less than the two (the plan's costs decide); LR_E_UNSUPPORTED, nothing launched, otherwise.
+int gemm_inputs(const void* x0, const void* wqkv, void* qkv, int S, const lr_rope_kv_t* rope, const void* x1, const void* w1, void* act,
+                int I, int M, int K, size_t sums_bytes, hipStream_t s) {
+  const int N = (rope->n_head + 2 * rope->n_kv_head) * rope->head_dim, cus = gemm_cus(), nk = (K + 63) / 64;
+  if (K % 64 || !gemm_reaches(K, N, K, GEMM_ROPE) || !gemm_reaches(K, I, K, GEMM_PAIR)) return LR_E_UNSUPPORTED;
+  const GemmPlan p0 = gemm_plan(M, N, K, GEMM_ROPE, sums_bytes), p1 = gemm_plan(M, I, K, GEMM_PAIR, sums_bytes);
+  if (p0.tile < 0 || p1.tile < 0) return LR_E_UNSUPPORTED;
+  const float weights_us = ((float)N + 2.0f * I) * K * 2 / GEMM_WEIGHT_BYTES_US;
+  float best_us = p0.us + p1.us;
+  int best = -1;
+  for (int c = 0; c < 4; ++c) {
+    const GemmTileCost& t = GEMM_TILES[c];
+    const int TM = 64 * t.a16, slots = cus * t.per_cu;
+    const int64_t tiles = (int64_t)((M + TM - 1) / TM) * ((N + 128 * t.bh - 1) / (128 * t.bh) + (I + 64 * t.bh - 1) / (64 * t.bh));
+    // (of several rounds only the last one leaves room, and q/k/v goes cold before the attention reads it: 8 x 2048 tokens of
+    // the 8B model, in one grid 185.4 ms, apart 183.2)
+    if (tiles > slots) continue;
+    float us = gemm_round_us(t, M, cus, (int)tiles, nk);
+    us = (us > weights_us ? us : weights_us) + t.fixed;
+    if (us < best_us) {
+      best_us = us;
+      best = c;
+    }
+  }
+  if (best < 0) return LR_E_UNSUPPORTED;
+  const GemmRope rp{(const u16*)rope->table, rope->pos, (u16*)rope->k_cache, (u16*)rope->v_cache, rope->err, S, rope->n_head,
+                    rope->n_kv_head, rope->head_dim, rope->smax, rope->block_size};
+  return gemm_two<GEMM_ROPE, GEMM_PAIR>(best, gemm_product(best, GEMM_ROPE, x0, K, wqkv, qkv, N, M, N, K),
+                                        gemm_product(best, GEMM_PAIR, x1, K, w1, act, I, M, I, K), rp, s);
+}
+
+// x w^T as partial sums [pieces][M][N] in `sums`; LR_E_UNSUPPORTED, nothing launched, where a product of this shape has whole tiles
+int gemm_pieces(const void* x, int64_t ldx, const void* w, int M, int N, int K, void* sums, size_t sums_bytes, int* pieces, hipStream_t s) {
+  if (M < GEMM_SCRATCH_FROM || sums == nullptr || lr_misaligned(sums) || N % 4 || !gemm_reaches(ldx, N, K, GEMM_PLAIN)) return LR_E_UNSUPPORTED;
+  const GemmPlan p = gemm_plan(M, N, K, GEMM_PLAIN, sums_bytes);
+  if (p.tile < 0 || p.full || !p.rem) return LR_E_UNSUPPORTED;
+  *pieces = p.splits;   // (less memory than the plan's own pieces, which have their tiles' absent rows and columns)
+  return gemm_run(x, ldx, w, nullptr, 0, M, N, K, GEMM_ROWS, GemmRope{}, p, sums, s);
+}
+
+// Two such products of N columns each in one launch, pieces of about the same length, where that should take less than the two
+struct GemmOutputs {
+  int tile, s0, s1;   // tile -1: the two are faster
+};
+static GemmOutputs outputs_plan(int M, int N, int K0, int K1, size_t sums_bytes) {
+  GemmOutputs best{-1, 1, 1};
+  if (M < GEMM_SCRATCH_FROM || N % 4 || K0 % 64 || K1 % 64 || !gemm_reaches(K0, N, K0, GEMM_PLAIN) || !gemm_reaches(K1, N, K1, GEMM_PLAIN)) return best;
+  const GemmPlan p0 = gemm_plan(M, N, K0, GEMM_PLAIN, sums_bytes), p1 = gemm_plan(M, N, K1, GEMM_PLAIN, sums_bytes);
+  if (p0.tile < 0 || p1.tile < 0) return best;
+  const float weights_us = ((float)K0 + K1) * N * 2 / GEMM_WEIGHT_BYTES_US;
+  auto alone = [](const GemmPlan& p) { return p.us - (p.rem && !p.full ? GEMM_SUM_US : 0.0f); };   // (its sum would be the norms' too)
+  float best_us = alone(p0) + alone(p1);
+  const int cus = gemm_cus(), pairs0 = (K0 / 64 + 1) / 2, pairs1 = (K1 / 64 + 1) / 2;
+  const size_t row = (size_t)M * N * sizeof(float);
+  for (int c = 0; c < 4; ++c) {
+    const GemmTileCost& t = GEMM_TILES[c];
+    const int TM = 64 * t.a16, TN = 128 * t.bh, slots = cus * t.per_cu;
+    const int64_t tiles = (int64_t)((M + TM - 1) / TM) * ((N + TN - 1) / TN);
+    for (int s0 = 1; s0 <= 16 && 2 * s0 <= pairs0 + 1 && row * s0 <= sums_bytes; ++s0)
+      for (int s1 = 1; s1 <= 16 && 2 * s1 <= pairs1 + 1 && row * s1 <= sums_bytes && tiles * (s0 + s1) <= slots; ++s1) {
+        const int k0 = 2 * ((pairs0 + s0 - 1) / s0), k1 = 2 * ((pairs1 + s1 - 1) / s1);
+        float us = gemm_round_us(t, M, cus, (int)tiles * (s0 + s1), k0 > k1 ? k0 : k1);
+        us = (us > weights_us ? us : weights_us) + t.fixed + GEMM_PIECE_US * (s0 + s1) + row * (s0 + s1) / GEMM_PIECE_BYTES_US;
+        if (us < best_us) {
+          best_us = us;
+          best = GemmOutputs{c, s0, s1};
+        }
+      }
+  }
+  return best;
+}
+bool gemm_outputs_pay(int M, int N, int K0, int K1, size_t sums_bytes) { return outputs_plan(M, N, K0, K1, sums_bytes).tile >= 0; }
+int gemm_outputs(const void* x0, const void* w0, int K0, void* sums0, int* pieces0, const void* x1, const void* w1, int K1, void* sums1, int* pieces1,
+                 int M, int N, size_t sums_bytes, hipStream_t s) {
+  if (lr_misaligned(sums0) || lr_misaligned(sums1)) return LR_E_ALIGN;
+  const GemmOutputs p = outputs_plan(M, N, K0, K1, sums_bytes);
+  if (p.tile < 0) return LR_E_UNSUPPORTED;
+  GemmProduct a = gemm_product(p.tile, GEMM_ROWS, x0, K0, w0, nullptr, 0, M, N, K0), b = gemm_product(p.tile, GEMM_ROWS, x1, K1, w1, nullptr, 0, M, N, K1);
+  a.sp = GemmSplit{(float*)sums0, 0, a.sp.full, p.s0};
+  b.sp = GemmSplit{(float*)sums1, 0, b.sp.full, p.s1};
+  *pieces0 = p.s0;
+  *pieces1 = p.s1;
+  return gemm_two<GEMM_ROWS, GEMM_ROWS>(p.tile, a, b, GemmRope{}, s);
+}
+}  // namespace lr_detail
 
 // Grouped products (lr_moe): rows of several matrices' tiles, see GemmGroup; pair_off != 0: GEMM_PAIR (N counts pairs).
 // tile_rows: 128 or 256, the height the tile table was made for.
@@ -767,6 +935,17 @@ extern "C" int lr_linear_scratch(const void* x, int64_t ldx, const void* w, void
                                  size_t scratch_bytes, lr_stream_t stream) {
   LR_OPTIONAL_PTR(scratch);
   return linear_rows(x, ldx, w, y, ldy, M, N, K, 0, 0, scratch, scratch_bytes, (hipStream_t)stream);
+}
+
+extern "C" int lr_linear_pieces(const void* x, int64_t ldx, const void* w, int M, int N, int K, void* sums, size_t sums_bytes, int32_t* pieces,
+                                lr_stream_t stream) {
+  LR_REQUIRE_PTR(x);
+  LR_REQUIRE_PTR(w);
+  LR_REQUIRE_PTR(sums);
+  if (pieces == nullptr) return LR_E_NULL;
+  if (M <= 0 || N <= 0 || K <= 0 || ldx < K) return LR_E_SHAPE;
+  if (K % 8 || ldx % 8) return LR_E_ALIGN;
+  return lr_detail::gemm_pieces(x, ldx, w, M, N, K, sums, sums_bytes, pieces, (hipStream_t)stream);
 }
 
 // The fused q/k/v projection of M = B * S rows (S tokens per sequence, row b * S + s at position pos[s]) finished as

@@ -20,6 +20,8 @@ _PROTOS = {
     "lr_add": (c_int, [c_void_p, c_void_p, c_float, c_void_p, c_int64, c_void_p]),
     "lr_add_rmsnorm": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float,
                                c_void_p]),
+    "lr_ladder_norms_pieces": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
+                                       c_int, c_float, c_void_p]),
     "lr_ladder_norms": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,
                                 c_float, c_void_p]),
     "lr_linear": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int, c_void_p]),
@@ -29,6 +31,7 @@ _PROTOS = {
     "lr_linear_plan": (c_int, [c_int, c_int, c_int, c_int, c_size_t, c_void_p]),
     "lr_linear_scratch": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_size_t,
                                   c_void_p]),
+    "lr_linear_pieces": (c_int, [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p, c_void_p]),
     "lr_linear_multi": (c_int, [c_void_p, c_int, c_int, c_void_p]),
     "lr_linear_multi_normed": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p]),
     "lr_linear_resid_sums": (c_int, [c_int]),
@@ -67,6 +70,7 @@ _PROTOS = {
                                       c_int, c_int, c_int, c_void_p]),
     "lr_attn_prefill": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
                                 c_int, c_int, c_int, c_int, c_void_p]),
+    "lr_ladder_block": (c_int, [c_void_p, c_void_p]),
     "lr_argmax": (c_int, [c_void_p, c_int64, c_void_p, c_int, c_int, c_void_p]),
     "lr_stream_read": (c_int, [c_void_p, c_size_t, c_void_p, c_void_p]),
     "lr_sample_topk": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_float, c_int, c_void_p, c_int64,
@@ -228,16 +232,27 @@ def add_rmsnorm(resid_in, d1, d2, gain, resid_out, normed_out, eps: float):
     return normed_out
 
 
+class Pieces:
+    """A product [rows, dim] as partial sums: `sums` holds [count][rows][dim] fp32 (linear_pieces); ladder_norms adds them."""
+
+    def __init__(self, sums: torch.Tensor, count: int, rows: int, dim: int):
+        assert sums.is_contiguous() and sums.numel() * sums.element_size() >= count * rows * dim * 4
+        self.sums, self.count, self.rows, self.dim = sums, count, rows, dim
+
+
 def ladder_norms(resid_in, d1, d2, gain1, gain2, resid_out, normed1, normed2, eps: float):
-    """Both residual updates and both norms of a ladder block (lr_ladder_norms)."""
+    """Both residual updates and both norms of a ladder block (lr_ladder_norms); d1 and d2 may be Pieces."""
     dim = resid_in.shape[-1]
     rows = resid_in.numel() // dim
     for t in (resid_in, d1, d2, resid_out, normed1, normed2):
-        assert t is None or (t.is_contiguous() and t.numel() == rows * dim)
+        if isinstance(t, Pieces):
+            assert (t.rows, t.dim) == (rows, dim)
+        else:
+            assert t is None or (t.is_contiguous() and t.numel() == rows * dim)
     assert gain1.numel() == dim and gain2.numel() == dim
-    p = lambda t: None if t is None else _dev(t)
-    _check(load().lr_ladder_norms(_dev(resid_in), p(d1), p(d2), _dev(gain1), _dev(gain2), _dev(resid_out), _dev(normed1),
-                                  _dev(normed2), rows, dim, float(eps), _stream()), "lr_ladder_norms")
+    p = lambda t: (None, 0) if t is None else (_dev(t.sums, t.sums.dtype), t.count) if isinstance(t, Pieces) else (_dev(t), 0)
+    _check(load().lr_ladder_norms_pieces(_dev(resid_in), *p(d1), *p(d2), _dev(gain1), _dev(gain2), _dev(resid_out), _dev(normed1),
+                                         _dev(normed2), rows, dim, float(eps), _stream()), "lr_ladder_norms_pieces")
 
 
 # Rows of a decode step up to which the weight-streaming bands are the faster kernel for projections that could have
@@ -554,6 +569,53 @@ def linear_swiglu_out(x: torch.Tensor, w1: torch.Tensor, act: torch.Tensor, scra
     _check(load().lr_linear_swiglu_out_scratch(_dev(x), ldx, _dev(w1), _dev(act), ldy, M, N, K, sp, sb, *_scratch_args(sums),
                                                _stream()), "lr_linear_swiglu_out_scratch")
     return act
+
+
+def linear_pieces(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, scratch):
+    """linear(x, w, out, scratch=scratch), or its partial sums (Pieces in `scratch`, out untouched) where no tile is computed whole."""
+    M, xc, ldx = _rows_ld(x)
+    N, K = w.shape
+    assert w.is_contiguous() and xc == K and tuple(out.shape) == (M, N)
+    count = c_int32()
+    rc = E_UNSUPPORTED if scratch is None else \
+        load().lr_linear_pieces(_dev(x), ldx, _dev(w), M, N, K, *_scratch_args(scratch), ctypes.byref(count), _stream())
+    if rc == E_UNSUPPORTED:
+        return linear(x, w, out, scratch=scratch)
+    _check(rc, "lr_linear_pieces")
+    return Pieces(scratch, count.value, M, N)
+
+
+class _LadderBlock(ctypes.Structure):   # lr_ladder_block_t
+    _fields_ = [(n, c_int32) for n in ("B", "S", "dim", "ffn")] + [("eps", c_float), ("rope", _RopeKv)] + \
+               [(n, c_void_p) for n in ("x", "xn", "xn2", "qkv", "y", "act", "h", "a", "m", "sums_a", "sums_m")] + [("sums_bytes", c_size_t)] + \
+               [(n, c_void_p) for n in ("gain1", "gain2", "wqkv", "wo", "w1", "w2")] + \
+               [(n, c_int32) for n in ("a_pieces", "m_pieces", "finish")]
+
+
+def ladder_blocks(blocks, ws, table, pos, Hq, Hkv, hd, eps):
+    """The all-ladder schedule of a prompt, a call per block (lr_ladder_block): ws.x -> ws.a, ws.m, which the last block leaves
+    to be added.  `blocks`: (gain1, gain2, wqkv, wo, w1, w2, k_cache, v_cache) of each; ws: the model's activation buffers."""
+    rows, D = ws.x.shape
+    I, nqkv = ws.act.shape[1], (Hq + 2 * Hkv) * hd
+    for t, cols in ((ws.x, D), (ws.xn, D), (ws.xn2, D), (ws.qkv, nqkv), (ws.y, Hq * hd), (ws.act, I), (ws.h, 2 * I), (ws.a, D), (ws.m, D)):
+        assert t.is_contiguous() and tuple(t.shape) == (rows, cols)
+    d = _LadderBlock(B=ws.B, S=ws.S, dim=D, ffn=I, eps=eps, a_pieces=-1, m_pieces=-1)
+    for n in ("x", "xn", "xn2", "qkv", "y", "act", "h", "a", "m"):
+        setattr(d, n, _dev(getattr(ws, n)))
+    if ws.sums is not None:
+        assert ws.sums.is_contiguous() and ws.sums_mlp.is_contiguous()
+        d.sums_a, d.sums_m = _dev(ws.sums, torch.uint8), _dev(ws.sums_mlp, torch.uint8)
+        d.sums_bytes = min(ws.sums.numel(), ws.sums_mlp.numel())
+    shapes = ((D,), (D,), (nqkv, D), (D, Hq * hd), (2 * I, D), (D, I))
+    fn, stream, ref = load().lr_ladder_block, _stream(), ctypes.byref(d)
+    for i, (*weights, kc, vc) in enumerate(blocks):
+        for t, shape in zip(weights, shapes):
+            assert tuple(t.shape) == shape and t.is_contiguous()
+        d.gain1, d.gain2, d.wqkv, d.wo, d.w1, d.w2 = map(_dev, weights)
+        assert kc.shape[0] >= ws.B
+        d.rope = rope_kv_epilogue(table, pos, kc, vc, Hq, Hkv, hd, n_pos=ws.S)
+        d.finish = i == len(blocks) - 1
+        _check(fn(ref, stream), "lr_ladder_block")
 
 
 def module_linear(x: torch.Tensor, mod, out: torch.Tensor, scratch=None):

@@ -23,7 +23,7 @@ class Workspace:
     """Activation buffers for one (batch, seq) shape, all bf16 [rows, *]."""
 
     def __init__(self, cfg: ModelArgs, B: int, S: int, fused_width: int, device, dtype, smax: int, all_logits: bool,
-                 sums_bytes: int):
+                 sums_bytes: int, two_sums: bool = False):
         rows = B * S
         D, hd = cfg.dim, cfg.head_dim
         e = lambda *shape: torch.empty(*shape, dtype=dtype, device=device)
@@ -46,16 +46,17 @@ class Workspace:
         self.next_token = torch.empty(B, 1, dtype=torch.int32, device=device)
         self.next_token_valid_for = None   # set by a fused decode step that already chose the token
         self.scratch = None
-        # Partial sums of products, in a decode step two memories: the MLP's may run beside the attention's, and alternating
-        # ones are faster also one after the other (8B dense, 33 rows: 4.67 ms per step, 4.71 in one).  The MLP's of up to 64
+        # Partial sums of products: two memories where a prompt's blocks leave both outputs' to the next norms (two_sums), and
+        # in a decode step, where the MLP's may run beside the attention's, and alternating ones are faster also one after the
+        # other (8B dense, 33 rows: 4.67 ms per step, 4.71 in one).  The MLP's of up to 64
         # rows has room for the pieces of 25 of 32 compute units, 32 KiB each: beside the attention's products these keep
         # the rest (70B rank shard, 64 rows: 7.6 ms per step, 8.2 with as many pieces as pay for a product alone), and
         # alone more are no faster (w2 4096 x 14336 of 64 rows: 31.9 us in six pieces, 34.2 in seven).  More rows have
         # larger tiles and one chain (70B rank shard, 96 rows: 9.7 ms per step, 10.9 with room for as little).
         n = sums_bytes
         self.sums = self.sums_mlp = torch.empty(n, dtype=torch.uint8, device=device) if n else None
-        if n and S == 1:
-            if rows <= 64:
+        if n and (two_sums or S == 1):
+            if rows <= 64 and S == 1:
                 cus = torch.cuda.get_device_properties(device).multi_processor_count if device.type == "cuda" else 256
                 n = min(n, cus * 25 // 32 << 15)
             self.sums_mlp = torch.empty(n, dtype=torch.uint8, device=device)
@@ -129,6 +130,7 @@ class GPTBase(nn.Module):
         _hip.device_error_word(device)  # exists before any step is captured into a graph
 
     supported_dtypes = (torch.bfloat16,)
+    prompt_pieces = False   # a prompt's output projections leave partial sums to the next norms: memory for both
 
     def _check_caches(self, max_seq_length):
         cfg = self.config
@@ -178,7 +180,7 @@ class GPTBase(nn.Module):
 
     def _new_workspace(self, B: int, S: int):
         return Workspace(self.config, B, S, self._fused_width(), self.output.weight.device, self.norm.weight.dtype,
-                         self.max_seq_length, not self.last_logits_only, self._sums_bytes(B, S))
+                         self.max_seq_length, not self.last_logits_only, self._sums_bytes(B, S), self.prompt_pieces)
 
     def _products(self, B: int, S: int):
         """(rows, N, K, pair) of every bf16 projection of a (B, S) step, as linear_sums_bytes takes them."""
@@ -241,10 +243,11 @@ class GPTBase(nn.Module):
         in question; weight-only quantised ones have kernels of their own.)"""
         return ws.S == 1 and self.band_rows_from <= ws.B <= self.band_rows_to and not any(hasattr(m, "scales") for m in linears)
 
-    def _attention(self, ws: Workspace, blk, pos: Tensor, wqkv: nn.Module, out: Tensor, roped: bool = False):
+    def _attention(self, ws: Workspace, blk, pos: Tensor, wqkv: nn.Module, out: Tensor, roped: bool = False,
+                   pieces: bool = False):
         """ws.xn -> fused projection -> RoPE + cache write -> attention -> wo -> out (partial sum).
         wqkv None: ws.qkv already holds the projection (roped: rotated, with k and v already in the cache).
-        out None: stop at the attention output ws.y."""
+        out None: stop at the attention output ws.y.  Returns out, or with `pieces` its partial sums where there are any."""
         cfg = self.config
         B, S = ws.B, ws.S
         Hq, Hkv, hd = cfg.n_head_local, cfg.n_kv_local, cfg.head_dim
@@ -270,23 +273,29 @@ class GPTBase(nn.Module):
             return
         if bands:
             _hip.linear_multi((ws.y, blk.attention.wo.weight, out, _hip.EPI_NONE))
+        elif pieces:
+            return _hip.linear_pieces(ws.y, blk.attention.wo.weight, out, ws.sums)
         else:
             _hip.module_linear(ws.y, blk.attention.wo, out, ws.sums)
+        return out
 
-    def _mlp(self, ws: Workspace, blk, out: Tensor, xn: Optional[Tensor] = None):
+    def _mlp(self, ws: Workspace, blk, out: Tensor, xn: Optional[Tensor] = None, pieces: bool = False):
         ff = blk.feed_forward
         xin = ws.xn if xn is None else xn
         if self._decode_bands(ws, ff.w1, ff.w2):
             _hip.linear_multi((xin, ff.w1.weight, ws.act, _hip.EPI_SWIGLU))
             _hip.linear_multi((ws.act, ff.w2.weight, out, _hip.EPI_NONE))
-            return
+            return out
         if xin.shape[0] > 4 and not hasattr(ff.w1, "scales"):
             # the activation in the first projection's epilogue; up to 4 rows it is fused into w2's GEMV instead
             _hip.linear_swiglu_out(xin, ff.w1.weight, ws.act, ws.h, ws.sums_mlp)
+            if pieces:
+                return _hip.linear_pieces(ws.act, ff.w2.weight, out, ws.sums_mlp)
             _hip.module_linear(ws.act, ff.w2, out, ws.sums_mlp)
-            return
+            return out
         _hip.module_linear(xin, ff.w1, ws.h)
         _hip.module_linear_swiglu(ws.h, ff.w2, out, ws.act)
+        return out
 
     # -- greedy decoding helper ---------------------------------------------------------------------
     def greedy_next(self, logits: Tensor) -> Tensor:

@@ -431,3 +431,36 @@ def test_linear_resid_refuses_what_it_cannot_serve(lib):
         assert rc(**{name: None}) == -1, name
     assert rc(joint=1, gain2=None) == -1 and rc(M=0) == -3 and rc(M=17) == -4
     assert rc(K1=60) == -2 and rc(ldx2=60) == -3 and rc(w1=250) == -2
+
+
+def test_ladder_block_and_pieces_refuse_what_they_cannot_serve(lib):
+    """Checked before anything is launched."""
+    from gpt_fast import _hip
+
+    pointers = ("x", "xn", "xn2", "qkv", "y", "act", "h", "a", "m", "gain1", "gain2", "wqkv", "wo", "w1", "w2")
+    heads = dict(n_head=4, n_kv_head=2, head_dim=64, smax=64, block_size=64)
+
+    def rc(rope=None, **kw):
+        r = _hip._RopeKv(**{**dict(table=256, pos=256, k_cache=256, v_cache=256), **heads, **(rope or {})})
+        d = _hip._LadderBlock(**{**{n: 256 for n in pointers}, **dict(B=1, S=8, dim=64, ffn=64, eps=1e-5, rope=r, a_pieces=-1, m_pieces=-1), **kw})
+        return lib.lr_ladder_block(ctypes.byref(d), None)
+
+    assert lib.lr_ladder_block(None, None) == -1
+    for name in pointers:
+        assert rc(**{name: None}) == -1 and rc(**{name: 264}) == -2, name
+    for name in ("table", "pos", "k_cache", "v_cache"):
+        assert rc(rope={name: None}) == -1, name
+    for name in heads:
+        assert rc(rope={name: 0}) == -3, name
+    assert rc(rope=dict(n_head=5)) == -3 and rc(rope=dict(head_dim=60)) == -2
+    assert rc(S=4) == -4 and rc(S=0) == -3 and rc(dim=60) == -2 and rc(ffn=60) == -2 and rc(a_pieces=2) == -1 and rc(sums_a=8) == -2
+
+    n = ctypes.c_int32()
+    pieces = lambda x=256, ldx=64, w=256, M=64, N=64, K=64, sums=256, size=1 << 20, out=ctypes.byref(n): \
+        lib.lr_linear_pieces(x, ldx, w, M, N, K, sums, size, out, None)
+    for name in ("x", "w", "sums", "out"):
+        assert pieces(**{name: None}) == -1, name
+    assert pieces(K=60) == -2 and pieces(ldx=56) == -3 and pieces(N=0) == -3
+    assert pieces(M=32) == -4 and pieces(N=66) == -4 and pieces(size=64) == -4      # nothing is cut
+    norms = lambda d1=256, p1=0, d2=256, p2=0: lib.lr_ladder_norms_pieces(256, d1, p1, d2, p2, 256, 256, 256, 256, 256, 8, 60, 1e-5, None)
+    assert norms(p1=-1) == -3 and norms(d1=None, p1=2) == -1 and norms(d2=None, p2=2) == -1 and norms(p1=2, p2=3) == -2

@@ -495,6 +495,85 @@ def test_ladder_norms_equals_two_add_rmsnorm_calls(hip, rows, dim, first_block):
     assert_close_ulp(n2, O.rms_norm(r2, g2, 1e-5), max_ulp=2, max_frac=0.05, what="ladder_norms n2")
 
 
+@pytest.mark.parametrize("M,D,K1,K2", [(33, 264, 2056, 4096), (64, 8192, 1024, 3584), (128, 2048, 2048, 8192), (100, 4096, 520, 14336),
+                                       (300, 4104, 4096, 4104), (40, 16384, 8192, 512), (777, 2048, 256, 8192)])
+def test_ladder_norms_of_partial_sums(hip, M, D, K1, K2):
+    """Products left as partial sums and added by the norms: the bits of products finished first."""
+    x, g1, g2 = rnd(M, D, seed=55), rnd(D, seed=56), rnd(D, seed=57)
+    sums = [torch.empty(hip.linear_scratch_bytes(M), dtype=torch.uint8, device=DEV) for _ in range(2)]
+    whole, parts = [], []
+    for i, K in enumerate((K1, K2)):
+        xi, w = rnd(M, K, seed=58 + i), rnd(D, K, seed=60 + i, scale=K ** -0.5)
+        whole.append(hip.linear(xi, w, torch.empty(M, D, dtype=BF, device=DEV), scratch=sums[i]).clone())
+        plan = hip.linear_plan(M, D, K)
+        sums[i].fill_(255)                                       # (NaN, where a sum is not written)
+        parts.append(hip.linear_pieces(xi, w, torch.empty(M, D, dtype=BF, device=DEV), sums[i]))
+        assert isinstance(parts[-1], hip.Pieces) == (plan.cut > 0 and plan.whole == 0)
+    outs = []
+    for d1, d2 in (whole, parts):
+        r, n1, n2 = x.clone(), torch.empty_like(x), torch.empty_like(x)
+        hip.ladder_norms(r, d1, d2, g1, g2, r, n1, n2, 1e-5)
+        outs.append((r, n1, n2))
+    assert any(isinstance(p, hip.Pieces) for p in parts)
+    for got, want in zip(outs[1], outs[0]):
+        assert torch.equal(got, want)
+
+
+class BlockBuffers:
+    """The activation buffers of a model's workspace that ladder_blocks uses."""
+
+    def __init__(self, hip, B, S, D, I, Hq, Hkv, hd):
+        e = lambda c: torch.full((B * S, c), float("nan"), dtype=BF, device=DEV)
+        self.B, self.S = B, S
+        self.x, self.xn, self.xn2, self.a, self.m, self.y, self.act, self.h = (e(c) for c in (D, D, D, D, D, Hq * hd, I, 2 * I))
+        self.qkv = e((Hq + 2 * Hkv) * hd)
+        n = hip.linear_scratch_bytes(B * S)
+        self.sums, self.sums_mlp = (torch.empty(n, dtype=torch.uint8, device=DEV) if n else None for _ in range(2))
+
+
+# (rows without memory for sums; both pairs of products in a grid, in tiles of 64, 128 and 256 rows; none; K no whole k-tiles; several
+# sequences; a block of its own)
+@pytest.mark.parametrize("B,S,D,I,Hq,Hkv,hd,layers", [
+    (1, 5, 256, 512, 4, 2, 64, 3), (2, 17, 512, 1024, 4, 1, 128, 3), (1, 63, 2048, 8192, 32, 8, 64, 2), (1, 128, 2048, 8192, 32, 8, 64, 3),
+    (1, 130, 4096, 14336, 32, 8, 128, 2), (3, 100, 1032, 1096, 4, 2, 64, 3), (2, 256, 2048, 8192, 32, 8, 64, 2), (1, 1100, 1024, 3584, 8, 1, 128, 2),
+    (1, 128, 2048, 8192, 32, 8, 64, 1),
+])
+def test_ladder_blocks_of_a_prompt(hip, B, S, D, I, Hq, Hkv, hd, layers):
+    """Blocks in one call each against the calls they are made of.  Where only the order of fp32 sums differs, a rounded
+    intermediate moves by a step of bf16 (2^-8) at the most, and few do: a stream of such blocks stays within 2^-7 by norm."""
+    rows, Smax = B * S, S + 8
+    pos = torch.arange(S, dtype=torch.int32, device=DEV)
+    t = torch.outer(torch.arange(Smax, device=DEV).float(), 10000.0 ** (-torch.arange(0, hd, 2, device=DEV).float() / hd))
+    table = torch.stack([t.cos(), t.sin()], -1).to(BF).contiguous()
+    nqkv = (Hq + 2 * Hkv) * hd
+    weights = []
+    for i in range(layers):
+        w = lambda k, n, m: rnd(n, m, seed=200 + 10 * i + k, scale=m ** -0.5)
+        weights.append((1 + rnd(D, seed=208 + 10 * i, scale=0.1), 1 + rnd(D, seed=209 + 10 * i, scale=0.1), w(0, nqkv, D), w(1, D, Hq * hd),
+                        w(2, 2 * I, D), w(3, D, I)))
+    results = []
+    for native in (True, True, False):
+        ws = BlockBuffers(hip, B, S, D, I, Hq, Hkv, hd)
+        ws.x.copy_(rnd(rows, D, seed=199))
+        caches = [tuple(torch.zeros(B, Hkv, Smax, hd, dtype=BF, device=DEV) for _ in range(2)) for _ in range(layers)]
+        if native:
+            hip.ladder_blocks([(*w, *c) for w, c in zip(weights, caches)], ws, table, pos, Hq, Hkv, hd, 1e-5)
+        else:
+            a = m = None
+            for (g1, g2, wqkv, wo, w1, w2), (kc, vc) in zip(weights, caches):
+                hip.ladder_norms(ws.x, a, m, g1, g2, ws.x, ws.xn, ws.xn2, 1e-5)
+                hip.linear_rope_kv(ws.xn, wqkv, ws.qkv, table, pos, kc, vc, B, S, Hq, Hkv, hd)
+                hip.attn_prefill(ws.qkv, kc, vc, pos, ws.y, B, S, Hq, Hkv, hd)
+                hip.linear(ws.y, wo, ws.a)
+                hip.linear_swiglu_out(ws.xn2, w1, ws.act, ws.h)
+                hip.linear(ws.act, w2, ws.m)
+                a, m = ws.a, ws.m
+        results.append([ws.x, ws.a, ws.m, *(t for c in caches for t in c)])
+    for again, got, want in zip(*results):
+        assert torch.equal(again, got) and torch.isfinite(got).all()
+        assert (got.double() - want.double()).norm() <= 2.0 ** -7 * want.double().norm()
+
+
 @pytest.mark.parametrize("M", [1, 2, 7, 8])
 @pytest.mark.parametrize("N,K", [(5, 16), (1280, 4112), (2048, 528), (2056, 144), (4104, 2064)])
 def test_bands_of_few_rows_equal_the_bands_of_many(hip, M, N, K):
