@@ -393,7 +393,8 @@ int lr_attn_prefill(const void* q, int64_t ldq, const void* k_cache, const void*
 /* One block of a prompt in the all-ladder schedule (gpt_ladder_TP.py:312-358, M = B * S > 4 rows): lr_ladder_norms_pieces
  * on the residual x and the outputs a and m of the block before, lr_linear_rope_kv of xn, lr_attn_prefill, lr_linear_swiglu_out
  * of xn2, lr_linear with wo into a and with w2 into m, with products of one grid and partial sums left to the next block where
- * that is faster.  The same arithmetic; the order of sums depends on the sizes.  Nothing is launched if a pointer or size is refused. */
+ * that is faster.  The same arithmetic; the order of sums depends on the sizes.  Pointers, sizes and alignments are checked before
+ * anything is launched; a limit of one of those calls (lr_attn_prefill) is reported when its turn comes. */
 typedef struct lr_ladder_block {
   int32_t B, S, dim, ffn;
   float eps;

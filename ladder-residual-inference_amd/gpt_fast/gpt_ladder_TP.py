@@ -172,10 +172,9 @@ class GPTLadder(GPTBase):
             if two_chains:
                 chain.wait_stream(cur)
                 with torch.cuda.stream(chain):
-                    pending_m = self._mlp(ws, blk, ws.m, ws.xn2, pieces=after is not None)
-                pending_a = self._attention(ws, blk, pos, blk.attention.wqkv, ws.a, pieces=after is not None)
+                    self._mlp(ws, blk, ws.m, ws.xn2)
+                self._attention(ws, blk, pos, blk.attention.wqkv, ws.a)
                 cur.wait_stream(chain)
-                continue
             elif multi:
                 kv = blk.attention.kv_cache
                 rope = _hip.rope_kv_epilogue(self.freqs_cis, pos, kv.k_cache, kv.v_cache, cfg.n_head_local,
