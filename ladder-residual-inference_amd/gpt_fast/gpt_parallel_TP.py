@@ -75,9 +75,10 @@ class GPTParallel(GPTBase):
         """Decode step through the weight-streaming bands.  The rows of the fused input weight are two projections
         of the same input: [q | k | v], rotated and cached on the way out, and [up | gate], stored as silu(gate) * up
         -- the second independent of the attention, so up to 16 sequences its bands share the attention's launch
-        (lr_attn_decode_beside) and above that the q/k/v launch; wo and w2 share a launch; y + x is left to the next
-        block's norm launch (x + y: the same sum).  Six launches per block instead of nine.  Above 32 sequences each
-        projection is a product of its own, with partial sums."""
+        (lr_attn_decode_beside) and above that the q/k/v launch; wo and w2 share a launch.  Up to 16 sequences that launch
+        also updates the residual and leaves the next block its rows undivided (linear_resid): four launches per block
+        instead of nine; above, and in the last block, y + x is left to the next norm launch (x + y: the same sum), six.
+        Above 32 sequences each projection is a product of its own, with partial sums."""
         cfg = self.config
         Hq, Hkv, hd = cfg.n_head_local, cfg.n_kv_local, cfg.head_dim
         q = ws.qkv[:, :nqkv]
@@ -104,9 +105,9 @@ class GPTParallel(GPTBase):
             else:
                 _hip.linear_multi(qkv, up_gate)
                 _hip.attn_decode(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd)
-            if ws.resid_sums and after is not None and blk.keeps_residual:
+            if ws.resid_sums and ws.B <= self.band_rows_to and after is not None and blk.keeps_residual:
                 # both sums go to the residual and the next norm's undivided rows come with parts of their sums of squares,
-                # which the q/k/v launch adds for up/gate
+                # which the q/k/v launch adds for up/gate (bands only: the products above read normed rows)
                 _hip.linear_resid((ws.y, att.wo), (ws.act, att.w2, after.attention_norm.weight, ws.xn, ws.sq2), ws.x, joint=True)
                 xn = _hip.Normed(ws.xn, ws.sq2, cfg.norm_eps, (ws.sq2, ws.sq2_total))
                 xu, pending = _hip.Normed(ws.xn, ws.sq2_total, cfg.norm_eps), None

@@ -909,6 +909,27 @@ def test_variant_decode_on_the_bands_equals_the_single_projection_kernels(family
     assert rel_err(kb, kp) <= REL_TOL and rel_err(vb, vp) <= REL_TOL
 
 
+@pytest.mark.parametrize("B", [3, 16])
+@torch.no_grad()
+def test_parallel_batches_above_the_bands_do_not_leave_rows_undivided(B):
+    """Bands switched off for a batch that would end its blocks with undivided rows (linear_resid): each projection is then a
+    product of its own and reads normed rows.  The same tokens fed, another one in every row: logits and caches within the
+    tolerance of two summation orders."""
+    model = build("parallel", **TINY)
+    model.setup_caches(B, 32)
+    toks = torch.randint(0, 512, (B, 10), device=DEV, generator=torch.Generator(device=DEV).manual_seed(3))
+
+    def steps(rows_to):
+        model.band_rows_to = rows_to
+        out = [model(toks[:, t:t + 1], torch.tensor([t], device=DEV)).clone() for t in range(10)]
+        model.check_device_errors()
+        kv = model.layers[-1].attention.kv_cache
+        return out + [kv.k_cache[:B, :, :10].clone(), kv.v_cache[:B, :, :10].clone()]
+
+    for got, want in zip(steps(B - 1), steps(32)):
+        assert rel_err(got, want) <= REL_TOL
+
+
 def test_parallel_semi_compiled_nonzero_rank_drops_the_residual():
     """gpt_parallel_TP.py:197-199: in the semi-compiled model only rank 0 adds the residual."""
     kw = dict(TINY, n_layer=2, tp_world_size=2, tp_rank=1, semi_compiled_model=True)
