@@ -1,4 +1,4 @@
-"""Where the time of one launch of the weight-streaming band kernel (lr_linear_multi, decode batches) goes.
+"""Where the time of one launch of the weight-streaming band kernels (lr_linear_multi, lr_linear_resid, decode batches) goes.
 
     python build.py --profile-bands         # once, anywhere hipcc runs: gpt_fast/libladder_hip_bandprof.so
     python band_phases.py [--rows 8]
@@ -23,6 +23,7 @@ from gpt_fast import _hip  # noqa: E402
 NAMES = ["entry -> first requests made", "-> first chunk in LDS", "-> end of the K loop", "-> partial sums exchanged",
          "-> end (sum, epilogue, store)"]
 MAX_WG = 4096
+WAVES = 8   # a workgroup's share of the buffer; the kernels of lr_linear_multi have four and leave the rest zero
 
 
 def main():
@@ -40,7 +41,7 @@ def main():
     lib.lr_band_profile.argtypes = [ctypes.c_void_p, ctypes.c_int]
     dev = "cuda"
     nbytes = lib.lr_band_profile(None, MAX_WG)
-    assert nbytes > 0, nbytes
+    assert nbytes == MAX_WG * WAVES * 8 * 8, nbytes
     prof = torch.zeros(nbytes // 8, dtype=torch.int64, device=dev)
     g = torch.Generator(device=dev)
     g.manual_seed(0)
@@ -65,20 +66,28 @@ def main():
     def up_gate(M, D, I):
         return lambda: ((rnd(M, D), rnd(2 * I, D), out(M, I), _hip.EPI_SWIGLU),)
 
-    def run(tag, make, reps=6):
+    def resid(M, D, Q, I):
+        class Weight:
+            def __init__(self, n, k):
+                self.weight = rnd(n, k)
+        n = _hip.linear_resid_sums(D)
+        side = lambda k: (rnd(M, k), Weight(D, k), rnd(D), out(M, D), torch.empty(M, n, device=dev))
+        return lambda: (side(Q), side(I), rnd(M, D))
+
+    def run(tag, make, reps=6, launch=_hip.linear_multi):
         sets = [make() for _ in range(reps)]   # fresh weights per launch: nothing of them is in L2
         for st in sets[:-1]:
-            _hip.linear_multi(*st)
+            launch(*st)
         torch.cuda.synchronize()
         prof.zero_()
         torch.cuda.synchronize()
         assert lib.lr_band_profile(prof.data_ptr(), MAX_WG) > 0
-        _hip.linear_multi(*sets[-1])
+        launch(*sets[-1])
         torch.cuda.synchronize()
         lib.lr_band_profile(None, 0)
-        t = prof.view(-1, 4, 8).cpu().double() * 0.01   # [workgroup][wave][stamp], microseconds
+        t = prof.view(-1, WAVES, 8).cpu().double() * 0.01   # [workgroup][wave][stamp], microseconds
         nwg = int((t[:, 0, 0] != 0).sum().item())
-        t = t[:nwg]
+        t = t[:nwg, :int((t[0, :, 0] != 0).sum().item())]
         t0 = t[:, :, 0].min()
         w0 = t[:, 0, :]                                 # wave 0 of every workgroup
         print(f"--- {tag}: {nwg} workgroups; first entry to last end {(t[:, :, 5].max() - t0):.2f} us")
@@ -94,10 +103,14 @@ def main():
     M = args.rows
     run(f"70B TP8 shard, q/k/v (1280 x 8192, RoPE + cache epilogue), {M} rows", qkv(M, 8192, 8, 1, 128, 2304, 2048))
     run(f"70B TP8 shard, up/gate (7168 x 8192, SwiGLU epilogue), {M} rows", up_gate(M, 8192, 3584))
-    run(f"70B TP8 shard, wo (8192 x 1024) next to w2 (8192 x 3584), {M} rows", wo_w2(M, 8192, 1024, 3584))
+    if 1 < M <= _hip.ROW_NORM_MAX_ROWS:
+        run(f"70B TP8 shard, wo (8192 x 1024) and w2 (8192 x 3584) with the residual updates, {M} rows", resid(M, 8192, 1024, 3584),
+            launch=_hip.linear_resid)
+    run(f"70B TP8 shard, wo (8192 x 1024) next to w2 (8192 x 3584), {M} rows (to 16: the last layer's)", wo_w2(M, 8192, 1024, 3584))
     run("70B TP8 shard, wo next to w2, 64 rows", wo_w2(64, 8192, 1024, 3584))
     run("Ladder-8B, q/k/v (6144 x 4096), 16 rows", qkv(16, 4096, 32, 8, 128, 1280, 1024))
-    run("Ladder-8B, wo (4096 x 4096) next to w2 (4096 x 14336), 16 rows", wo_w2(16, 4096, 4096, 14336))
+    run("Ladder-8B, wo (4096 x 4096) and w2 (4096 x 14336) with the residual updates, 16 rows", resid(16, 4096, 4096, 14336),
+        launch=_hip.linear_resid)
 
 
 if __name__ == "__main__":

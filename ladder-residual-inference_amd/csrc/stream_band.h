@@ -23,12 +23,17 @@ constexpr int AUX_WEIGHTS = 2;        // weights: non-temporal (every line is us
 #ifdef LR_BAND_PROFILE
 // Profile builds only: when set (lr_band_profile, stream_gemm.hip), every wave of every band records 100 MHz
 // wall-clock stamps at six points -- 0 entry, 1 first requests made, 2 first chunk in LDS, 3 end of the K loop,
-// 4 partial sums exchanged (second barrier), 5 end -- at [(workgroup * NWV + wave) * 8 + point].
+// 4 partial sums exchanged (second barrier), 5 end -- at band_prof_at(workgroup, wave, point).
+constexpr int BAND_PROF_WAVES = 8;  // of the widest workgroups; narrower ones leave the rest as it was
+__host__ __device__ constexpr size_t band_prof_at(unsigned workgroup, int wave, int point) {
+  return ((size_t)workgroup * BAND_PROF_WAVES + wave) * 8 + point;
+}
+constexpr long long band_prof_bytes(unsigned workgroups) { return (long long)(band_prof_at(workgroups, 0, 0) * sizeof(unsigned long long)); }
 static __device__ unsigned long long* g_band_prof;
 static __device__ unsigned g_band_prof_wgs;  // workgroups the buffer has room for; the others record nothing
-#define LR_BAND_STAMP(k)                                                                              \
-  if (g_band_prof && blockIdx.x < g_band_prof_wgs && lane == 0)                                       \
-    g_band_prof[((size_t)blockIdx.x * NWV + wave) * 8 + (k)] = wall_clock64();
+#define LR_BAND_STAMP(k)                                                \
+  static_assert(NW <= BAND_PROF_WAVES, "a workgroup's stamps are its own"); \
+  if (g_band_prof && blockIdx.x < g_band_prof_wgs && lane == 0) g_band_prof[band_prof_at(blockIdx.x, wave, k)] = wall_clock64();
 #else
 #define LR_BAND_STAMP(k)
 #endif

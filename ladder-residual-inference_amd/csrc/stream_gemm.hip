@@ -253,7 +253,7 @@ extern "C" long long lr_band_profile(void* device_buffer, int workgroups) {
   if (hipMemcpyToSymbol(HIP_SYMBOL(g_band_prof), &ptr, sizeof(ptr)) != hipSuccess ||
       hipMemcpyToSymbol(HIP_SYMBOL(g_band_prof_wgs), &wgs, sizeof(wgs)) != hipSuccess)
     return LR_E_LAUNCH;
-  return (long long)workgroups * NWV * 8 * (long long)sizeof(unsigned long long);
+  return band_prof_bytes(wgs);
 }
 #endif
 

@@ -464,3 +464,22 @@ def test_ladder_block_and_pieces_refuse_what_they_cannot_serve(lib):
     assert pieces(M=32) == -4 and pieces(N=66) == -4 and pieces(size=64) == -4      # nothing is cut
     norms = lambda d1=256, p1=0, d2=256, p2=0: lib.lr_ladder_norms_pieces(256, d1, p1, d2, p2, 256, 256, 256, 256, 256, 8, 60, 1e-5, None)
     assert norms(p1=-1) == -3 and norms(d1=None, p1=2) == -1 and norms(d2=None, p2=2) == -1 and norms(p1=2, p2=3) == -2
+
+
+def test_a_profile_builds_stamps_stay_in_the_buffer_it_asks_for(tmp_path):
+    """Host part of the bands' sources, as a profile build compiles them: the last stamp of a workgroup of any width is its own, and
+    the buffer that lr_band_profile asks for ends behind the last one."""
+    import shutil
+    import subprocess
+
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    csrc = os.path.join(ROOT, "ladder-residual-inference_amd", "csrc")
+    src = tmp_path / "stamps.hip"
+    src.write_text(f'''#define LR_BAND_PROFILE
+#include "{csrc}/stream_gemm.hip"
+static_assert(band_prof_at(3, RN_WAVES - 1, 5) < band_prof_at(4, 0, 0) && band_prof_at(3, NWV - 1, 5) < band_prof_at(4, 0, 0), "");
+static_assert(band_prof_bytes(4) >= (long long)sizeof(unsigned long long) * (band_prof_at(3, RN_WAVES - 1, 5) + 1), "");
+''')
+    r = subprocess.run([hipcc, "--cuda-host-only", "-fsyntax-only", "-std=c++17", "-x", "hip", "--offload-arch=gfx950", str(src)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
