@@ -211,6 +211,28 @@ def wider(family):
     return build(family, **(dict(WIDER, **shard) if family == "desync" else WIDER))
 
 
+@pytest.mark.parametrize("B", [3, 8, 9, 16])
+@pytest.mark.parametrize("fp8", [False, True])
+@torch.no_grad()
+def test_ladder_decode_of_different_sequences_equals_each_alone(B, fp8):
+    """Steps that leave rows undivided by their root mean squares, another sequence (and so another root mean square) in every
+    row: each row's logits are those of the sequence decoded alone, within the tolerance of two summation orders."""
+    from gpt_fast.quantize import quantize_model_fp8
+
+    model = build("ladder", **TINY)
+    model.tok_embeddings.weight.mul_(torch.logspace(-2, 2, 512, base=2.0, device=DEV).to(BF)[:, None])
+    if fp8:
+        quantize_model_fp8(model)
+    model.setup_caches(B, 16)
+    toks = torch.randint(0, 512, (B, 6), device=DEV, generator=torch.Generator(device=DEV).manual_seed(9))
+    toks[:, 0] = torch.arange(B, device=DEV) * 511 // (B - 1)     # (from the smallest to the largest embeddings)
+    decode = lambda rows: torch.cat([model(rows[:, t:t + 1].contiguous(), torch.tensor([t], device=DEV)).clone() for t in range(6)], 1)
+    together = decode(toks)
+    assert model._ws[(B, 1, False)].resid_sums
+    for b in range(B):
+        assert rel_err(together[b], decode(toks[b:b + 1])[0]) <= REL_TOL, b
+
+
 @pytest.mark.parametrize("family", ["ladder", "dense", "desync", "parallel"])
 @pytest.mark.parametrize("B", [33, 40, 64, 70])
 def test_decode_batches_above_32_run_products_with_partial_sums(family, B):

@@ -1146,3 +1146,96 @@ def test_linear_resid_and_the_projections_of_its_rows(hip, M, D, K1, K2, fp8):
         y = project(outs[1], sums[1], (sums[1], total))
         assert torch.allclose(total[:, 0].double(), sums[1].double().sum(1), rtol=1e-6)
         assert (ulp_diff(project(outs[1], total), y) <= 1).all()
+
+
+def parts_of(x, count):
+    """Sums of squares of `count` runs of columns, [M, count] fp32."""
+    D = x.shape[1]
+    runs = torch.zeros(x.shape[0], count, dtype=torch.float64, device=DEV)
+    return runs.index_add_(1, torch.arange(D, device=DEV) * count // D, x.double().square()).float()
+
+
+def rotated(t, table, hd):
+    """Interleaved pairs of float64 heads [M, n] turned by table [hd / 2, 2]."""
+    v, c, s = t.view(t.shape[0], -1, hd // 2, 2), table[:, 0].double(), table[:, 1].double()
+    return torch.stack([v[..., 0] * c - v[..., 1] * s, v[..., 1] * c + v[..., 0] * s], -1).view_as(t)
+
+
+# both input layouts of a band (to 8 rows, from 9), the e4m3 ones too; sums as one part, several and the most there may be; K of
+# one chunk and of many, ragged bands
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("M,D,parts,parts2,Hq,Hkv,hd,I", [
+    (3, 272, 17, 5, 4, 2, 64, 72), (8, 1024, 128, 256, 8, 1, 128, 456), (9, 2048, 256, 300, 8, 2, 64, 200), (13, 528, 511, 512, 4, 2, 64, 1000),
+    (16, 8192, 256, 1, 8, 1, 128, 456), (16, 4096, 256, 256, 32, 8, 128, 1400)])
+def test_every_projection_of_undivided_rows(hip, M, D, parts, parts2, Hq, Hkv, hd, I, fp8):
+    """Rows whose root mean squares lie a factor of 64 apart, to be divided by the projection: q/k/v with the RoPE and cache
+    epilogue and up/gate with the activation, in one launch, alone, and beside the attention on the sums that the q/k/v
+    launch has added, each against float64.  A rounding moves a value by up to 2^-8 of it; fp32 sums are closer by far."""
+    eps, N, Smax, pos = 1e-5, (Hq + 2 * Hkv) * hd, 64, 37
+    spread = 2.0 ** ((torch.arange(M, device=DEV) * 5 % 7) - 3.0)
+    x, x2 = ((rnd(M, D, seed=300 + i).double() * s[:, None]).to(BF) for i, s in enumerate((spread, spread.flip(0))))
+    sums, sums2 = parts_of(x, parts), parts_of(x2, parts2)
+    w, w2 = rnd(N, D, seed=302, scale=D ** -0.5), rnd(2 * I, D, seed=303, scale=D ** -0.5)
+    table = O.rope_table(Smax, hd, 10000.0, BF).to(DEV)
+    p = torch.tensor([pos], dtype=torch.int32, device=DEV)
+    if fp8:
+        (w, sc), (w2, sc2) = quantised(w), quantised(w2)
+    step = lambda t: 2.0 ** -8 * t.abs()
+
+    def product(x, sums, w, scales):
+        """(x w^T of the divided rows, what its rounding and the fp32 sum may move it by)"""
+        rs = torch.rsqrt(sums.double().sum(1, keepdim=True) / D + eps)
+        f = 1.0 if scales is None else scales.double()
+        v = (x.double() @ w.double().T) * rs * f
+        return v, (1 if scales is None else 2) * step(v) + 2.0 ** -20 * (x.double().abs() @ w.double().abs().T) * rs * f
+
+    v, dv = product(x, sums, w, sc if fp8 else None)
+    n_qk, tab = (Hq + Hkv) * hd, table[pos].view(hd // 2, 2)
+    pair = lambda t: t.view(M, -1, 2).flip(-1).reshape(M, -1)
+    want_qk = rotated(v[:, :n_qk], tab, hd)
+    want = torch.cat([want_qk, v[:, n_qk:]], 1)
+    bound = torch.cat([dv[:, :n_qk] + pair(dv[:, :n_qk]) + step(want_qk), dv[:, n_qk:]], 1)
+    (u, g), (du, dg) = (t.split(I, 1) for t in product(x2, sums2, w2, sc2 if fp8 else None))
+    act = torch.nn.functional.silu(g)
+    want_act, bound_act = act * u, u.abs() * (1.1 * dg + step(act)) + (act.abs() + 1.1 * dg) * du + step(act * u)
+
+    def check(got, want, bound, what):
+        assert ((got.double() - want).abs() <= 1.05 * bound + 1e-6).all(), what
+
+    proj = lambda x, w, s, out, epi: (x, w, s, out, epi) if fp8 else (x, w, out, epi)
+    multi = hip.linear_fp8_multi if fp8 else hip.linear_multi
+    scales, scales2 = (sc, sc2) if fp8 else (None, None)
+    for form in ("one launch", "beside", "alone"):
+        qkv, out = torch.full((M, N), 5.0, dtype=BF, device=DEV), torch.full((M, I + 8), 5.0, dtype=BF, device=DEV)
+        kc, vc = (rnd(M, Hkv, Smax, hd, seed=304 + i) for i in range(2))
+        rope = hip.rope_kv_epilogue(table, p, kc, vc, Hq, Hkv, hd)
+        total = torch.full((M, 1), 7.0, device=DEV)
+        if form == "one launch":
+            multi(proj(hip.Normed(x, sums, eps), w, scales, qkv, rope), proj(hip.Normed(x2, sums2, eps), w2, scales2, out[:, :I], hip.EPI_SWIGLU))
+        else:
+            multi(proj(hip.Normed(x, sums, eps, (sums2, total)), w, scales, qkv, rope))
+            assert torch.allclose(total[:, 0].double(), sums2.double().sum(1), rtol=1e-6)
+            up_gate = proj(hip.Normed(x2, total, eps), w2, scales2, out[:, :I], hip.EPI_SWIGLU)
+            if form == "alone":
+                multi(up_gate)
+            else:
+                scratch = torch.zeros(hip.attn_decode_scratch_bytes(M, Hq, hd, Smax) // 4, dtype=torch.float32, device=DEV)
+                y, y1 = (torch.zeros(M, Hq * hd, dtype=BF, device=DEV) for _ in range(2))
+                beside = hip.attn_decode_beside_fp8 if fp8 else hip.attn_decode_beside
+                assert beside(qkv, kc, vc, p, y, scratch, M, Hq, Hkv, hd, up_gate)
+                hip.attn_decode(qkv, kc, vc, p, y1, scratch, M, Hq, Hkv, hd)
+                assert torch.equal(y, y1)
+        got = torch.cat([qkv[:, :Hq * hd], kc[:, :, pos].reshape(M, -1), vc[:, :, pos].reshape(M, -1)], 1)
+        check(got, want, bound, form + ": q, k, v")
+        check(out[:, :I], want_act, bound_act, form + ": activation")
+        assert (out[:, I:] == 5.0).all()
+    hip.raise_on_device_error(x.device)
+
+
+def test_undivided_rows_that_no_launch_serves_are_refused(hip):
+    """Sums for a later launch of more rows than the projection has bands: nothing is launched."""
+    x, y, sums, total = rnd(8, 64, seed=310), torch.full((8, 28), 5.0, dtype=BF, device=DEV), torch.ones(8, 2, device=DEV), torch.full((8, 1), 7.0, device=DEV)
+    with pytest.raises(hip.LadderHipError):
+        hip.linear_multi((hip.Normed(x, sums, 1e-5, (sums, total)), rnd(28, 64, seed=311), y, hip.EPI_NONE))
+    torch.cuda.synchronize()
+    assert (y == 5.0).all() and (total == 7.0).all()
