@@ -49,6 +49,8 @@ extern "C" int lr_ladder_block(lr_ladder_block_t* d, lr_stream_t stream) {
   if (rows64 < 5) return LR_E_UNSUPPORTED;   // (the activation is the second projection's there)
   if (D % 8 || I % 8 || hd % 8) return LR_E_ALIGN;
   if ((d->a_pieces > 0 || d->m_pieces > 0) && (d->sums_a == nullptr || d->sums_m == nullptr)) return LR_E_NULL;
+  for (const int n : {d->a_pieces, d->m_pieces})   // (as many as there is room for)
+    if (n > 0 && d->sums_bytes / sizeof(float) / (unsigned)D / (unsigned)n < (size_t)rows64) return LR_E_SHAPE;
   const int rows = (int)rows64, nqkv = (int)nqkv64, Dq = Hq * hd;
   const bool sums = d->sums_a != nullptr && d->sums_m != nullptr;
   const size_t bytes = sums ? d->sums_bytes : 0;

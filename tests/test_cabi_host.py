@@ -466,6 +466,20 @@ def test_ladder_block_and_pieces_refuse_what_they_cannot_serve(lib):
     assert norms(p1=-1) == -3 and norms(d1=None, p1=2) == -1 and norms(d2=None, p2=2) == -1 and norms(p1=2, p2=3) == -2
 
 
+def test_ladder_block_refuses_more_partial_sums_than_its_memory_holds(lib):
+    """What the block before left is read in whole pieces of rows x dim: a count that the memory cannot hold is a mistake of the
+    caller's, found before anything is launched."""
+    from gpt_fast import _hip
+
+    pointers = ("x", "xn", "xn2", "qkv", "y", "act", "h", "a", "m", "gain1", "gain2", "wqkv", "wo", "w1", "w2", "sums_a", "sums_m")
+    r = _hip._RopeKv(table=256, pos=256, k_cache=256, v_cache=256, n_head=4, n_kv_head=2, head_dim=64, smax=64, block_size=64)
+    for which in ("a_pieces", "m_pieces"):
+        for pieces, size in ((1, 40 * 64 * 4 - 1), (3, 40 * 64 * 4 * 3 - 1), (0x7fffffff, 1 << 26)):
+            d = _hip._LadderBlock(**{n: 256 for n in pointers}, B=1, S=40, dim=64, ffn=64, eps=1e-5, rope=r, sums_bytes=size,
+                                  **{**dict(a_pieces=-1, m_pieces=-1), which: pieces})
+            assert lib.lr_ladder_block(ctypes.byref(d), None) == -3, (which, pieces)
+
+
 def test_a_profile_builds_stamps_stay_in_the_buffer_it_asks_for(tmp_path):
     """Host part of the bands' sources, as a profile build compiles them: the last stamp of a workgroup of any width is its own, and
     the buffer that lr_band_profile asks for ends behind the last one."""
