@@ -602,7 +602,7 @@ def ladder_blocks(blocks, ws, table, pos, Hq, Hkv, hd, eps):
     d = _LadderBlock(B=ws.B, S=ws.S, dim=D, ffn=I, eps=eps, a_pieces=-1, m_pieces=-1)
     for n in ("x", "xn", "xn2", "qkv", "y", "act", "h", "a", "m"):
         setattr(d, n, _dev(getattr(ws, n)))
-    if ws.sums is not None:
+    if ws.sums is not ws.sums_mlp:   # (one memory for both outputs' pieces: none)
         assert ws.sums.is_contiguous() and ws.sums_mlp.is_contiguous()
         d.sums_a, d.sums_m = _dev(ws.sums, torch.uint8), _dev(ws.sums_mlp, torch.uint8)
         d.sums_bytes = min(ws.sums.numel(), ws.sums_mlp.numel())

@@ -130,7 +130,10 @@ class GPTBase(nn.Module):
         _hip.device_error_word(device)  # exists before any step is captured into a graph
 
     supported_dtypes = (torch.bfloat16,)
-    prompt_pieces = False   # a prompt's output projections leave partial sums to the next norms: memory for both
+
+    def _prompt_pieces(self) -> bool:
+        """Do a prompt's output projections leave partial sums to the next norms, which takes memory for both?"""
+        return False
 
     def _check_caches(self, max_seq_length):
         cfg = self.config
@@ -180,7 +183,7 @@ class GPTBase(nn.Module):
 
     def _new_workspace(self, B: int, S: int):
         return Workspace(self.config, B, S, self._fused_width(), self.output.weight.device, self.norm.weight.dtype,
-                         self.max_seq_length, not self.last_logits_only, self._sums_bytes(B, S), self.prompt_pieces)
+                         self.max_seq_length, not self.last_logits_only, self._sums_bytes(B, S), self._prompt_pieces())
 
     def _products(self, B: int, S: int):
         """(rows, N, K, pair) of every bf16 projection of a (B, S) step, as linear_sums_bytes takes them."""

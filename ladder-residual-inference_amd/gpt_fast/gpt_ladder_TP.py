@@ -61,7 +61,9 @@ class GPTLadder(GPTBase):
     # decode steps of batch <= 2 run as ONE persistent kernel (lr_ladder_decode_step) when the shape
     # is supported; set to False to force the per-op kernels
     use_fused_step = True
-    prompt_pieces = True
+
+    def _prompt_pieces(self):
+        return self.config.ladder_layers is None and not hasattr(self.layers[0].attention.wqkv, "scales")   # (lr_ladder_block's)
 
     def _make_block(self, config, layer_idx):
         return LadderTransformerBlock(config)

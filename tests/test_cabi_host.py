@@ -325,6 +325,21 @@ def test_a_model_without_bf16_projections_holds_no_memory_for_partial_sums(lib):
         assert model._new_workspace(B, S).sums is None
 
 
+def test_only_prompts_whose_blocks_keep_both_outputs_pieces_hold_memory_for_both(lib):
+    """lr_ladder_block's: all-ladder models on bf16 weights.  Others, with a bf16 head or whole, hold one piece of memory."""
+    import gpt_fast
+    from gpt_fast.quantize import quantize_model_fp8
+
+    apart = lambda model: (lambda ws: ws.sums is not None and ws.sums is not ws.sums_mlp)(model._new_workspace(1, 777))
+    assert apart(meta_model("ladder", "ladder-8b"))
+    quantised = quantize_model_fp8(meta_model("ladder", "ladder-8b"), include_output=False)
+    assert quantised._new_workspace(1, 777).sums is not None and not apart(quantised)
+    assert not apart(meta_model("dense", "ladder-8b"))
+    partial = meta_model("ladder", "ladder-8b")
+    partial.config.ladder_layers = [0, 1]
+    assert partial._new_workspace(1, 777).sums is not None and not apart(partial)
+
+
 @pytest.mark.parametrize("family,name", FAMILIES[:3])
 @pytest.mark.parametrize("B", [33, 64, 65, 96])
 def test_partial_sums_of_the_mlp_are_limited_where_that_was_measured(lib, family, name, B):
