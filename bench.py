@@ -66,7 +66,7 @@ TRAFFIC_BYTES_PER_LAUNCH = {
 }
 # HBM bytes of a whole decode step through the per-op kernels (all its launches), from the same kind of counter runs
 STEP_TRAFFIC_BYTES = {
-    ("gpt_ladder:ladder-70b-tp8", 8, 2048): 18.62e9,     # 1.03 x algorithmic
+    ("gpt_ladder:ladder-70b-tp8", 8, 2048): 18.60e9,     # 1.03 x algorithmic
     ("gpt_ladder:ladder-70b-tp8", 64, 2048): 27.52e9,    # 1.21 x algorithmic
 }
 

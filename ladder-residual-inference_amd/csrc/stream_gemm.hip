@@ -154,8 +154,9 @@ extern "C" int lr_linear_residual_tanh(const void* x, int64_t ldx, const void* w
 // and its share of their sums of squares, and the next projections divide their results by the rows' root mean squares
 // (stream_band: has_norm).  Bound: HBM, like the bands it replaces, whose two workgroups of four waves per CU become one of
 // eight: chunks of the first weight, then of the second, are dealt round the waves.  Measured, us per launch under a
-// profiler: 8192 x (1024 | 3584) e4m3 of 5 rows 10.7 -> 11.8 and q/k/v 7.0 -> 7.9, for a norm launch of 4.7; a step, us: 70B
-// rank shard, 8 rows 4617 -> 4403, e4m3 5 rows 3450 -> 3257; 8B 16 rows 3576 -> 3560; 8B parallel blocks, 6 rows 3220 -> 3114.
+// profiler (70B rank shard, 8 rows): 8192 x (1024 | 3584) 17.0 -> 17.9 and q/k/v 8.6 -> 9.1, e4m3 11.8 -> 12.7 and 7.9 -> 9.0,
+// for a norm launch of 4.8; a step, us: 70B rank shard, 8 rows 4617 -> 4403, e4m3 5 rows 3450 -> 3257; 8B 16 rows 3576 -> 3560;
+// 8B parallel blocks, 6 rows 3220 -> 3114.
 // Not for 17 rows and more (the 32-row band fills the register file with four waves), nor where the norm stands between a
 // block's attention and its MLP: up/gate then has several bands per CU, each of which would add all the parts (12 rows of 8B
 // desync blocks 3755 -> 3772), and rounding the rows once instead of twice moves near-ties of two-row batches.
