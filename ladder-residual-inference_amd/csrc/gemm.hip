@@ -609,36 +609,51 @@ struct GemmPlan {
   int full, rem, splits;
   float us;        // what it should take
 };
-// A workgroup's time is nk * (ktile + busy * slope) + fixed, `busy` the workgroups per CU: the more CUs are at work, the
-// lower the clock and the more of them ask the L2s; `cold` in place of the slope where a single row tile reads every weight
-// from HBM itself; `pair` where two share a CU, `pair_cold` while up to two row tiles share a weight: then both wait for HBM,
-// and a k-tile costs almost what two in turn do.  The weights need their time on the way from HBM whatever the tiles.
-// Pieces cost a launch, their trip through memory and the ramp of each.
-// The costs are fitted to 219 products (33 to 3002 rows of 14 weights between 1280 x 8192 and 128256 x 4096, every tile,
-// whole and in 2 to 16 pieces, weights from HBM) and to 90 more of up to 16384 rows, two plans of each: what the plan takes is
-// 1.1 % above the best of all on average, and 23 % at worst (192 rows, 3072 x 2048: 17.1 us, 13.9 in three pieces); fitted
-// without `pair_cold` and the ramp, on fewer rows, it was 3.8 % and 37 %.  Some of them, us, N x K, chosen before / now | the best there is:
-//    64 rows,  3072 x  2048   12.3 / 11.2 | 10.8        128 rows,  2048 x  8192   19.6 / 16.2 | 16.2
-//    64 rows, 11264 x  4096   31.1 / 25.4 | 25.4        128 rows,  3072 x  2048   17.2 / 13.0 | 12.8
-//   128 rows,  4096 x 14336   38.5 / 33.0 | 33.0        128 rows, 28672 x  4096   64.4 / 52.4 | 52.4 (pairs)
+// A round of workgroups takes k * (ktile + busy * slope), `busy` the workgroups per CU: the more CUs are at work, the lower
+// the clock and the more of them ask the L2s.  Two to a CU take `pair` per k-tile.  A single row tile reads every weight from
+// HBM itself, which is `cold` (`pair_cold`) in their place; with two row tiles GEMM_TWO of the way to it is left, with more
+// none (128 x 128, two to a CU: 1.25 | 0.93 | 0.87 us per k-tile).  `fixed` is the ramp and drain of a round, `store` what the
+// outputs of a whole tile per CU add to it; weights and outputs need their time from and to HBM whatever the tiles.  Pieces
+// cost a launch, their trip through memory and the round trips of whoever adds them.
+// The costs are fitted to 1296 products, 33 to 16384 rows of the 37 weights of the model families, with 64 MiB for pieces, 6.5 and
+// none (2700 choices, of each the tiles and pieces that could be near the best, weights from HBM).  What the plan takes is 0.8 % above
+// the best of them on average and 22 % at worst; with the costs of the fit before (219 products of up to 3002 rows, 90 of more) 1.2 and
+// 25 %, with those before that 2.2 and 38 %.  Some products in us, N x K, with the first costs / the second / now | the best there is:
+//   128 rows,  2048 x  2048  12.4 / 10.4 / 10.4 | 10.1         200 rows,  8192 x   512   6.0 /  7.2 /  6.0 |  6.0
+//   128 rows,  3072 x  2048  17.2 / 13.3 / 13.3 | 13.0         900 rows,  2048 x    16   4.2 /  5.1 /  4.2 |  4.2
+//   128 rows,  4096 x 14336  38.3 / 32.8 / 32.8 | 32.8        1501 rows,  7168 x  8192 153.9 / 168.2 / 153.9 | 153.9 (pairs)
+//   128 rows, 28672 x  4096  65.8 / 54.8 / 54.8 | 54.8 (pairs)  2100 rows, 4608 x 4096  79.2 / 82.3 / 79.2 | 77.2
+// and where it loses most: 129 rows, 16032 x 8192 65.9 / 78.8 / 77.1 | 65.9; 5000 rows, 2048 x 5120 95.5 / 95.5 / 109.6 | 95.5; 192 rows,
+// 3072 x 2048 17.1 in all three | 14.0; 1100 rows, 8192 x 512 19.9 in all three | 16.4.
 struct GemmTileCost {
   int a16, bh, per_cu;
-  float ktile, slope, cold, pair, pair_cold, fixed;
+  float ktile, slope, cold, pair, pair_cold, fixed, store;
 };
-constexpr GemmTileCost GEMM_TILES[4] = {{4, 2, 1, 0.968f, 0.416f, 0.0848f, 0.0f, 0.0f, 5.94f},
-                                         {2, 2, 1, 0.576f, 0.304f, 0.658f, 0.0f, 0.0f, 3.05f},
-                                         {2, 1, 2, 0.486f, 0.0641f, 0.314f, 0.957f, 2.43f, 2.76f},
-                                         {1, 1, 2, 0.278f, 0.236f, 0.279f, 0.737f, 1.33f, 2.82f}};
+constexpr GemmTileCost GEMM_TILES[4] = {{4, 2, 1, 1.2f, 0.0f, 0.0f, 0.0f, 0.0f, 4.35f, 4.43f},
+                                         {2, 2, 1, 0.684f, 0.108f, 0.552f, 0.0f, 0.0f, 2.85f, 1.47f},
+                                         {2, 1, 2, 0.504f, 0.0f, 0.262f, 0.874f, 1.25f, 3.18f, 0.166f},
+                                         {1, 1, 2, 0.302f, 0.201f, 0.284f, 0.737f, 1.19f, 3.24f, 0.0f}};
 constexpr size_t GEMM_SCRATCH = (size_t)64 << 20;   // pieces of one round of the largest tiles
 constexpr int GEMM_SCRATCH_FROM = 33;               // rows from which a projection that has memory for pieces is one of this file's
 
-constexpr float GEMM_WEIGHT_BYTES_US = 5.98e6f, GEMM_SUM_US = 4.62f, GEMM_PIECE_US = 0.0884f, GEMM_PIECE_BYTES_US = 4.78e6f;
+constexpr float GEMM_WEIGHT_BYTES_US = 5.73e6f, GEMM_OUTPUT_BYTES_US = 6.98e6f, GEMM_SUM_US = 4.92f, GEMM_TRIP_US = 0.267f, GEMM_PIECE_BYTES_US = 3.83e6f,
+                GEMM_TWO = 0.157f, GEMM_NORM_PIECE_US = 0.15f;
 
 // `workgroups` of k k-tiles each, at the same time
 static float gemm_round_us(const GemmTileCost& t, int M, int cus, int workgroups, int k) {
   const float busy = (float)workgroups / cus;
   const int TM = 64 * t.a16;
-  return k * (busy > 1.0f ? (M <= 2 * TM ? t.pair_cold : t.pair) : t.ktile + busy * (M <= TM ? t.cold : t.slope));
+  const float own = M <= TM ? 1.0f : M <= 2 * TM ? GEMM_TWO : 0.0f;   // how much a weight is one row tile's own
+  return k * (busy > 1.0f ? t.pair + (t.pair_cold - t.pair) * own : t.ktile + busy * (t.slope + (t.cold - t.slope) * own));
+}
+// N outputs per row, of as many weight rows or twice as many
+static float gemm_bytes_us(int M, int N, int K, int mode) {
+  return (mode == GEMM_PAIR ? 2.0f : 1.0f) * N * K * 2 / GEMM_WEIGHT_BYTES_US + (float)M * N * 2 / GEMM_OUTPUT_BYTES_US;
+}
+// Round trips to memory of whoever adds the pieces: the first piece and four more, then four at a time.
+static int gemm_trips(int pieces) { return (pieces + 2) / 4; }
+static float gemm_store_us(const GemmTileCost& t, int64_t tiles, int cus, int mode) {
+  return t.store * (mode == GEMM_PAIR ? 0.5f : 1.0f) * tiles / cus;
 }
 static int gemm_cus() {
   const int cus = lr_num_cus();
@@ -649,7 +664,7 @@ static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
   GemmPlan best{-1, 0, 0, 1, 0.0f};
   if (M > 0x7fffffff - 256 || N > 0x7fffffff - 256 || K > 0x7fffffff - 256) return best;   // (row, column and k of the last tile are ints)
   const int cus = gemm_cus(), nk = (K + 63) / 64;
-  const float weights_us = (float)N * (mode == GEMM_PAIR ? 2 : 1) * K * 2 / GEMM_WEIGHT_BYTES_US;
+  const float bytes_us = gemm_bytes_us(M, N, K, mode);
   for (int c = 0; c < 4; ++c) {
     const GemmTileCost& t = GEMM_TILES[c];
     const int TM = 64 * t.a16, TN = (mode == GEMM_PAIR ? 64 : 128) * t.bh, slots = cus * t.per_cu;
@@ -658,7 +673,7 @@ static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
     const int left = (int)(tiles - rounds * slots);
     auto round_us = [&](int workgroups, int k) { return gemm_round_us(t, M, cus, workgroups, k); };
     auto consider = [&](float us, float more, int whole, int cut, int pieces) {
-      us = (us > weights_us ? us : weights_us) + more;
+      us = (us > bytes_us ? us : bytes_us) + more + gemm_store_us(t, whole, cus, mode);
       if (best.tile < 0 || us < best.us) best = GemmPlan{c, whole, cut, pieces, us};
     };
     const float whole = rounds * round_us(slots, nk), fixed = (rounds + (left ? 1 : 0)) * t.fixed;
@@ -666,7 +681,7 @@ static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
     for (int s = 2; left && s <= 16 && 4 * s <= nk && left * s <= slots; ++s) {
       const size_t bytes = (size_t)left * s * (64 * t.a16) * (128 * t.bh) * sizeof(float);
       if (bytes > scratch) break;
-      consider(whole + round_us(left * s, (nk + s - 1) / s), fixed + GEMM_SUM_US + GEMM_PIECE_US * s + bytes / GEMM_PIECE_BYTES_US,
+      consider(whole + round_us(left * s, (nk + s - 1) / s), fixed + GEMM_SUM_US + gemm_trips(s) * GEMM_TRIP_US + bytes / GEMM_PIECE_BYTES_US,
                (int)tiles - left, left, s);
     }
   }
@@ -760,18 +775,18 @@ int gemm_inputs(const void* x0, const void* wqkv, void* qkv, int S, const lr_rop
   if (K % 64 || !gemm_reaches(K, N, K, GEMM_ROPE) || !gemm_reaches(K, I, K, GEMM_PAIR)) return LR_E_UNSUPPORTED;
   const GemmPlan p0 = gemm_plan(M, N, K, GEMM_ROPE, sums_bytes), p1 = gemm_plan(M, I, K, GEMM_PAIR, sums_bytes);
   if (p0.tile < 0 || p1.tile < 0) return LR_E_UNSUPPORTED;
-  const float weights_us = ((float)N + 2.0f * I) * K * 2 / GEMM_WEIGHT_BYTES_US;
+  const float bytes_us = gemm_bytes_us(M, N, K, GEMM_ROPE) + gemm_bytes_us(M, I, K, GEMM_PAIR);
   float best_us = p0.us + p1.us;
   int best = -1;
   for (int c = 0; c < 4; ++c) {
     const GemmTileCost& t = GEMM_TILES[c];
     const int TM = 64 * t.a16, slots = cus * t.per_cu;
-    const int64_t tiles = (int64_t)((M + TM - 1) / TM) * ((N + 128 * t.bh - 1) / (128 * t.bh) + (I + 64 * t.bh - 1) / (64 * t.bh));
+    const int64_t tm = (M - 1) / TM + 1, tiles0 = tm * ((N - 1) / (128 * t.bh) + 1), tiles1 = tm * ((I - 1) / (64 * t.bh) + 1), tiles = tiles0 + tiles1;
     // (of several rounds only the last one leaves room, and q/k/v goes cold before the attention reads it: 8 x 2048 tokens of
     // the 8B model, in one grid 185.4 ms, apart 183.2)
     if (tiles > slots) continue;
     float us = gemm_round_us(t, M, cus, (int)tiles, nk);
-    us = (us > weights_us ? us : weights_us) + t.fixed;
+    us = (us > bytes_us ? us : bytes_us) + t.fixed + gemm_store_us(t, tiles0, cus, GEMM_ROPE) + gemm_store_us(t, tiles1, cus, GEMM_PAIR);
     if (us < best_us) {
       best_us = us;
       best = c;
@@ -793,7 +808,9 @@ int gemm_pieces(const void* x, int64_t ldx, const void* w, int M, int N, int K, 
   return gemm_run(x, ldx, w, nullptr, 0, M, N, K, GEMM_ROWS, GemmRope{}, p, sums, s);
 }
 
-// Two such products of N columns each in one launch, pieces of about the same length, where that should take less than the two
+// Two such products of N columns each in one launch, pieces of about the same length, where that should take less than the two.
+// (GEMM_NORM_PIECE_US: the norms add a row per workgroup, slower than k_gemm_sum.  With it 128 rows of the 1B model keep eight pieces in tiles of 64
+// rows, a prompt 1059 us; ten in tiles of 128, 1063.)
 struct GemmOutputs {
   int tile, s0, s1;   // tile -1: the two are faster
 };
@@ -802,7 +819,7 @@ static GemmOutputs outputs_plan(int M, int N, int K0, int K1, size_t sums_bytes)
   if (M < GEMM_SCRATCH_FROM || N % 4 || K0 % 64 || K1 % 64 || !gemm_reaches(K0, N, K0, GEMM_PLAIN) || !gemm_reaches(K1, N, K1, GEMM_PLAIN)) return best;
   const GemmPlan p0 = gemm_plan(M, N, K0, GEMM_PLAIN, sums_bytes), p1 = gemm_plan(M, N, K1, GEMM_PLAIN, sums_bytes);
   if (p0.tile < 0 || p1.tile < 0) return best;
-  const float weights_us = ((float)K0 + K1) * N * 2 / GEMM_WEIGHT_BYTES_US;
+  const float bytes_us = gemm_bytes_us(M, N, K0, GEMM_ROWS) + gemm_bytes_us(M, N, K1, GEMM_ROWS);
   auto alone = [](const GemmPlan& p) { return p.us - (p.rem && !p.full ? GEMM_SUM_US : 0.0f); };   // (its sum would be the norms' too)
   float best_us = alone(p0) + alone(p1);
   const int cus = gemm_cus(), pairs0 = (K0 / 64 + 1) / 2, pairs1 = (K1 / 64 + 1) / 2;
@@ -815,7 +832,7 @@ static GemmOutputs outputs_plan(int M, int N, int K0, int K1, size_t sums_bytes)
       for (int s1 = 1; s1 <= 16 && 2 * s1 <= pairs1 + 1 && row * s1 <= sums_bytes && tiles * (s0 + s1) <= slots; ++s1) {
         const int k0 = 2 * ((pairs0 + s0 - 1) / s0), k1 = 2 * ((pairs1 + s1 - 1) / s1);
         float us = gemm_round_us(t, M, cus, (int)tiles * (s0 + s1), k0 > k1 ? k0 : k1);
-        us = (us > weights_us ? us : weights_us) + t.fixed + GEMM_PIECE_US * (s0 + s1) + row * (s0 + s1) / GEMM_PIECE_BYTES_US;
+        us = (us > bytes_us ? us : bytes_us) + t.fixed + (gemm_trips(s0) + gemm_trips(s1)) * GEMM_TRIP_US + row * (s0 + s1) / GEMM_PIECE_BYTES_US + (s0 + s1) * GEMM_NORM_PIECE_US;
         if (us < best_us) {
           best_us = us;
           best = GemmOutputs{c, s0, s1};

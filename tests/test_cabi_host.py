@@ -315,6 +315,43 @@ def test_memory_for_partial_sums_is_what_the_products_of_a_step_can_use(lib, fam
             assert held <= 16 << 20
 
 
+# Products of models' weights in us, by tile (rows, columns) and pieces of K, measured one after the other with weights from HBM: the
+# choice that costs fitted to fewer of them made, and the ones near the best.
+MEASURED_PRODUCTS = [
+    # M, N, K, pair, MiB for pieces
+    (1700, 1024, 16, False, 64, {(128, 128, 1): 5.1, (64, 128, 1): 4.2}),
+    (900, 2048, 16, False, 0, {(128, 128, 1): 5.1, (64, 128, 1): 4.2}),
+    (200, 8192, 512, False, 64, {(128, 128, 1): 7.2, (64, 128, 1): 6.0}),
+    (512, 4096, 512, False, 64, {(128, 128, 1): 7.3, (64, 128, 1): 6.3}),
+    (129, 4096, 22528, False, 64, {(256, 256, 12): 61.4, (128, 256, 8): 54.4, (128, 128, 4): 54.2}),
+    (1501, 7168, 8192, True, 64, {(256, 256, 1): 168.2, (128, 256, 3): 153.9}),
+    (257, 2048, 12288, False, 64, {(128, 256, 10): 30.2, (128, 128, 5): 27.8}),
+    (4100, 8192, 1024, False, 64, {(256, 256, 1): 81.6, (256, 256, 4): 76.7}),
+    (1315, 2048, 5120, False, 64, {(128, 256, 2): 44.5, (128, 128, 1): 41.8}),
+    (3002, 7168, 8192, True, 0, {(256, 256, 1): 338.9, (128, 256, 1): 303.1}),
+    (2630, 6160, 2048, False, 0, {(128, 256, 1): 80.8, (128, 128, 1): 72.7}),
+    (6004, 4096, 4096, True, 0, {(256, 256, 1): 188.6, (128, 256, 1): 170.6}),
+    (9205, 2048, 8192, False, 0, {(128, 256, 1): 288.1, (128, 128, 1): 263.0}),
+    (520, 28672, 4096, True, 0, {(128, 256, 1): 162.7, (128, 128, 1): 151.5}),
+    # and what those costs had won over the ones before
+    (128, 2048, 2048, False, 64, {(64, 128, 8): 12.4, (64, 128, 4): 10.4, (64, 128, 3): 10.1}),
+    (900, 2048, 2048, False, 64, {(128, 128, 1): 15.3, (64, 128, 1): 12.8}),
+    (128, 3072, 2048, False, 64, {(64, 128, 1): 17.2, (64, 128, 4): 13.3, (64, 128, 5): 13.0}),
+    (128, 4096, 14336, False, 64, {(64, 128, 8): 38.3, (128, 128, 8): 32.8}),
+    (128, 28672, 4096, True, 64, {(64, 128, 1): 65.8, (128, 128, 1): 54.8}),
+    (9205, 2560, 2048, False, 64, {(256, 256, 2): 94.4, (128, 256, 1): 87.9}),
+]
+
+
+@pytest.mark.parametrize("M,N,K,pair,mib,times", MEASURED_PRODUCTS)
+def test_the_plan_takes_no_tiles_that_measured_slower(lib, M, N, K, pair, mib, times):
+    """Within 3 % of the fastest, the difference that two runs of one product may show."""
+    from gpt_fast import _hip
+
+    plan = _hip.linear_plan(M, N, K, pair, mib << 20)
+    assert times[(plan.tile_rows, plan.tile_cols, plan.pieces)] <= 1.03 * min(times.values())
+
+
 def test_a_model_without_bf16_projections_holds_no_memory_for_partial_sums(lib):
     from gpt_fast.quantize import quantize_model_fp8
 
