@@ -574,6 +574,30 @@ def test_ladder_blocks_of_a_prompt(hip, B, S, D, I, Hq, Hkv, hd, layers):
         assert (got.double() - want.double()).norm() <= 2.0 ** -7 * want.double().norm()
 
 
+# (no product cut: 256 bytes; other tiles and pieces than with all the memory there may be; as many)
+@pytest.mark.parametrize("rows,D,I,Hq,Hkv,hd", [(40, 1024, 3584, 8, 1, 128), (448, 2048, 8192, 32, 8, 64), (128, 2048, 8192, 32, 8, 64), (600, 2048, 8192, 32, 8, 64)])
+def test_ladder_blocks_with_the_memory_that_a_model_gives_them(hip, rows, D, I, Hq, Hkv, hd):
+    """A model's memory for partial sums is sized for its products one by one: fewer pieces may fit than with the most there
+    may be, and no more is touched.  Only the order of fp32 sums differs: within 2^-7 by norm."""
+    pos, N = torch.arange(rows, dtype=torch.int32, device=DEV), (Hq + 2 * Hkv) * hd
+    table = O.rope_table(rows, hd, 10000.0, BF).to(DEV)
+    w = lambda k, n, m: rnd(n, m, seed=220 + k, scale=m ** -0.5)
+    weights = (1 + rnd(D, seed=228, scale=0.1), 1 + rnd(D, seed=229, scale=0.1), w(0, N, D), w(1, D, Hq * hd), w(2, 2 * I, D), w(3, D, I))
+    sized = hip.linear_sums_bytes([(rows, N, D, False), (rows, D, Hq * hd, False), (rows, 2 * I, D, True), (rows, D, I, False)])
+    results = []
+    for nbytes in (hip.linear_scratch_bytes(rows), sized):
+        ws = BlockBuffers(hip, 1, rows, D, I, Hq, Hkv, hd)
+        held = [torch.full((nbytes + 4096,), 85, dtype=torch.uint8, device=DEV) for _ in range(2)]
+        ws.sums, ws.sums_mlp = (h[:nbytes] for h in held)
+        ws.x.copy_(rnd(rows, D, seed=219))
+        caches = [[torch.zeros(1, Hkv, rows, hd, dtype=BF, device=DEV) for _ in range(2)] for _ in range(3)]
+        hip.ladder_blocks([(*weights, *c) for c in caches], ws, table, pos, Hq, Hkv, hd, 1e-5)
+        assert all((h[nbytes:] == 85).all() for h in held)
+        results.append([ws.x, ws.a, ws.m, *(t for c in caches for t in c)])
+    for got, want in zip(*results):
+        assert torch.isfinite(got).all() and (got.double() - want.double()).norm() <= 2.0 ** -7 * want.double().norm()
+
+
 @pytest.mark.parametrize("M", [1, 2, 7, 8])
 @pytest.mark.parametrize("N,K", [(5, 16), (1280, 4112), (2048, 528), (2056, 144), (4104, 2064)])
 def test_bands_of_few_rows_equal_the_bands_of_many(hip, M, N, K):
