@@ -485,6 +485,35 @@ def test_linear_resid_refuses_what_it_cannot_serve(lib):
     assert rc(K1=60) == -2 and rc(ldx2=60) == -3 and rc(w1=250) == -2
 
 
+@pytest.mark.parametrize("entry", ["linear_multi", "linear_fp8_multi", "attn_decode_beside", "attn_decode_beside_fp8"])
+def test_undivided_rows_are_refused_where_they_cannot_be_served(lib, entry):
+    """Checked before anything is launched: sums of another width than the rows, more parts or rows than a launch holds, a total
+    with no place to go."""
+    from gpt_fast import _hip
+
+    fp8 = "fp8" in entry
+    q = (_hip._ProjectionFp8 if fp8 else _hip._Projection)()
+    q.x, q.ldx, q.y, q.ldy, q.N, q.K, q.epilogue = 256, 64, 256, 64, 64, 64, _hip.EPI_NONE
+    if fp8:
+        q.w8, q.scales = 256, 256
+    else:
+        q.w = 256
+
+    def rc(M=4, **kw):
+        norm = _hip._RowNorm(**{**dict(sums=256, count=2, dim=64, eps=1e-5), **kw})
+        p, n = ctypes.cast(ctypes.byref(q), ctypes.c_void_p), ctypes.byref(norm)
+        if "beside" in entry:
+            return getattr(lib, f"lr_{entry}_normed")(256, 256, 256, 256, 256, 256, 256, M, 2, 1, 64, 64, 256, 1 << 20, p, n, M, None)
+        return getattr(lib, f"lr_{entry}_normed")(p, n, 1, M, None)
+
+    assert rc(count=0) == -3 and rc(dim=72) == -3 and rc(count=513) == -4 and rc(sums=264) == -2
+    assert rc(fold_sums=256, fold_count=2) == -1 and rc(fold_sums=264, fold_total=256, fold_count=2) == -2
+    assert rc(fold_sums=256, fold_total=256, fold_count=0) == -3 and rc(fold_sums=256, fold_total=256, fold_count=513) == -4
+    assert rc(M=17) == -4
+    if fp8:
+        assert rc(M=1) == -4      # (one row: the matrix-vector kernel)
+
+
 def test_ladder_block_and_pieces_refuse_what_they_cannot_serve(lib):
     """Checked before anything is launched."""
     from gpt_fast import _hip
