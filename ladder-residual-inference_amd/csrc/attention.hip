@@ -23,32 +23,38 @@ extern "C" size_t lr_attn_decode_scratch_bytes(int B, int Hq, int hd, int Smax) 
   return (size_t)B * Hq * attn_nsplit_cap(Smax) * (hd + 2) * sizeof(float);
 }
 
-template <int HD, int G>
+template <int HD, int G, int GROUPS>
 __global__ __launch_bounds__(256) void k_attn_decode_partial(const u16* __restrict__ q, int64_t ldq,
                                                              const u16* __restrict__ kc, const u16* __restrict__ vc,
                                                              const int32_t* __restrict__ pos_ptr,
                                                              float* __restrict__ o_part, float* __restrict__ ml_part,
                                                              int Hkv, int Smax, int nsplit, int chunk_max) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
-  attn_partial_item<HD, G, true>(q, ldq, kc, vc, pos_ptr, o_part, ml_part, Hkv, Smax, nsplit, chunk_max, blockIdx.x,
+  attn_partial_item<HD, G, GROUPS>(q, ldq, kc, vc, pos_ptr, o_part, ml_part, Hkv, Smax, nsplit, chunk_max, blockIdx.x,
                            blockIdx.y, blockIdx.z, smem);
 }
 
-template <int HD, int G>
-static int launch_decode(const u16* q, int64_t ldq, const u16* kc, const u16* vc, const int32_t* pos, u16* y,
-                         int64_t ldy, int B, int Hkv, int Smax, float* scratch, hipStream_t s) {
+template <int HD, int G, int GROUPS>
+static int launch_decode_as(const u16* q, int64_t ldq, const u16* kc, const u16* vc, const int32_t* pos, u16* y,
+                            int64_t ldy, int B, int Hkv, int Smax, int nsplit, int chunk_max, float* scratch, hipStream_t s) {
   const int Hq = Hkv * G;
-  const int nsplit = attn_pick_nsplit(B, Hkv, Smax);
-  const int chunk_max = ((Smax + nsplit - 1) / nsplit + 3) & ~3;
   float* o_part = scratch;
   float* ml_part = scratch + (size_t)B * Hq * nsplit * HD;
   const size_t lds = (size_t)attn_item_lds_floats<HD, G>(chunk_max) * sizeof(float);
   static std::atomic<unsigned long long> lds_raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_attn_decode_partial<HD, G>), lds, lds_raised)) return LR_E_LAUNCH;
-  k_attn_decode_partial<HD, G><<<dim3(nsplit, Hkv, B), dim3(256), lds, s>>>(q, ldq, kc, vc, pos, o_part, ml_part, Hkv,
-                                                                            Smax, nsplit, chunk_max);
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_attn_decode_partial<HD, G, GROUPS>), lds, lds_raised)) return LR_E_LAUNCH;
+  k_attn_decode_partial<HD, G, GROUPS><<<dim3(nsplit, Hkv, B), dim3(256), lds, s>>>(q, ldq, kc, vc, pos, o_part, ml_part, Hkv,
+                                                                                    Smax, nsplit, chunk_max);
   launch_attn_combine<HD>(o_part, ml_part, y, ldy, Hq, B, nsplit, s);
   return lr_launch_status();
+}
+template <int HD, int G>
+static int launch_decode(const u16* q, int64_t ldq, const u16* kc, const u16* vc, const int32_t* pos, u16* y,
+                         int64_t ldy, int B, int Hkv, int Smax, float* scratch, hipStream_t s) {
+  const int nsplit = attn_pick_nsplit(B, Hkv, Smax);
+  const int chunk_max = ((Smax + nsplit - 1) / nsplit + 3) & ~3;
+  return attn_two_groups(chunk_max) ? launch_decode_as<HD, G, 2>(q, ldq, kc, vc, pos, y, ldy, B, Hkv, Smax, nsplit, chunk_max, scratch, s)
+                                    : launch_decode_as<HD, G, 4>(q, ldq, kc, vc, pos, y, ldy, B, Hkv, Smax, nsplit, chunk_max, scratch, s);
 }
 
 extern "C" int lr_attn_decode(const void* q, int64_t ldq, const void* k_cache, const void* v_cache,

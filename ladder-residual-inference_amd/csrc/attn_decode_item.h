@@ -5,6 +5,7 @@
 //      A chunk never exceeds ATT_CHUNK keys: the item then requests all of its K and V rows at once.
 constexpr int ATT_CHUNK = 256;
 constexpr int ATT_NCU = 256;  // CUs of the MI355X
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
 
 static inline int attn_nsplit_cap(int Smax) {
   const int by_len = (Smax + ATT_CHUNK - 1) / ATT_CHUNK;
@@ -39,50 +40,54 @@ static inline int attn_pick_nsplit(int B, int Hkv, int Smax) {
 // LDS row length of the score buffer: whole 16-key tiles, plus 4 so that the 16 heads a tile's scores are
 // written for do not share a bank
 __host__ __device__ constexpr int attn_sc_ld(int chunk_max) { return ((chunk_max + 15) & ~15) + 4; }
+// and of the softmax weights', in bf16 elements: whole 64-key groups, plus 16 bytes for the same reason
+__host__ __device__ constexpr int attn_p_ld(int chunk_max) { return ((chunk_max + 63) & ~63) + 8; }
 
 // One (split, kv head, sequence) item of the split-KV decode attention, by 256 lanes (4 waves): scores,
-// softmax statistics and the un-normalised P.V of keys [k0, k1) (at most ATT_CHUNK) for all G q heads of
+// softmax statistics and the un-normalised P.V of keys [k0, k1) (at most 64 GROUPS <= ATT_CHUNK) for all G q heads of
 // the kv head.  `smem`: attn_item_lds_floats<HD, G>(chunk_max) floats of LDS.  (A kv head with more q heads than
 // an instantiation takes can be served as kv_share groups of G: every head's result is the same either way.)
 //
-// Every K and V row of the chunk is requested before anything else -- whole rows, 1 KiB contiguous per
-// wave instruction, up to 32 KiB per wave in flight -- so the item costs one memory round trip.  Scores
-// run on the matrix cores: a 16-key tile of K takes a trip through a wave-private piece of LDS (written
-// row-major as loaded, read back as v_mfma_f32_16x16x32_bf16 A fragments, rows padded by 16 bytes), the
-// q heads are the B operand (loaded straight into fragment layout, heads beyond G are zero columns).
-// Softmax statistics and P.V stay in fp32 on the vector units: a lane owns 8 output elements of one key
-// group, so the inner loop has no cross-lane traffic.
+// Bound: memory latency and the instructions behind it.  Every K and V row of the chunk is requested before anything else
+// -- whole rows, 1 KiB contiguous per wave instruction, up to 32 KiB per wave in flight, buffer loads whose offset lies
+// outside the buffer for what is not wanted (a branch per load makes the compiler wait for everything in flight in the
+// middle of the sequence) -- so the item costs one memory round trip.  Scores run on the matrix cores: a 16-key tile of K
+// takes a trip through a wave-private piece of LDS (written row-major as loaded, read back as v_mfma_f32_16x16x32_bf16 A
+// fragments, rows padded by 16 bytes), the q heads are the B operand (loaded straight into fragment layout, heads beyond G
+// are zero columns).  P.V too: V lies in LDS as it came, 64 keys at a time, and is read transposed
+// (ds_read_b64_tr_b16) as A fragments, a wave multiplies HD / 4 of the dimensions by all keys, and a softmax weight enters as
+// three bf16 summands, which hold all 24 bits of it: the products are those of fp32 weights.
+// (P.V on the vector units, lanes owning 8 dimensions of one key in four and the four waves' sums met in LDS, was 14 KB of code
+// passed through once, which every launch fetches anew: 6.7 us from the last row's arrival to the stored result for 8 heads of
+// 65 keys beside a weight stream, now 2.5 us in 4 KB.  64 sequences of the 70B rank shard, ms per step: 7.45 -> 7.05.  The
+// chunk results' error against 64 bits is 1.6e-7 of their norm, as it was.)
 template <int HD, int G>
 __host__ __device__ constexpr int attn_item_lds_floats(int chunk_max) {
-  return (4 * G * HD > 32 * (HD + 8) ? 4 * G * HD : 32 * (HD + 8)) + G * attn_sc_ld(chunk_max) + 2 * G + 4;
+  return 32 * (HD + 8) + G * attn_sc_ld(chunk_max) + (3 * G * attn_p_ld(chunk_max) + 1) / 2 + 2 * G + 4;
 }
+// GROUPS of 64 keys that an item's registers hold: two, or ATT_CHUNK / 64
+static inline bool attn_two_groups(int chunk_max) { return chunk_max <= 128; }
 
-// EAGER: every request is a buffer load whose offset lies outside the buffer for what is not wanted (it reads as
-// zero), q first.  Written as `wanted ? load : 0` each load sits in a branch of its own, and the copy that merges
-// one of them with its zero makes the compiler wait for everything in flight in the middle of the sequence: two
-// memory round trips per item instead of one (70B shard, 64 sequences: 9.83 -> 9.43 ms per step; 8B, 16 sequences:
-// 3.63 -> 3.57).  With short chunks beside a weight stream (8 sequences of the 70B shard: one tile of four per wave
-// holds keys) the branches are the better neighbour (5.05 against 5.11 ms): the caller chooses.
-template <int HD, int G, bool EAGER = false>
+template <int HD, int G, int GROUPS>
 __device__ __forceinline__ void attn_partial_item(const u16* __restrict__ q, int64_t ldq, const u16* __restrict__ kc,
                                                   const u16* __restrict__ vc, const int32_t* __restrict__ pos_ptr,
                                                   float* __restrict__ o_part, float* __restrict__ ml_part, int Hkv,
                                                   int Smax, int nsplit, int chunk_max, int split, int kvh, int b,
                                                   float* __restrict__ smem, int kv_share = 1) {
   static_assert(G <= 16, "the q heads of a kv head are the 16 columns of one matrix-core tile");
+  static_assert(GROUPS * 64 <= ATT_CHUNK, "");
   constexpr int LPK = HD / 8;    // lanes that share one key row (8 elements each)
   constexpr int KPW = 64 / LPK;  // keys per wave instruction
   constexpr int NI = 16 / KPW;   // instructions per 16-key tile
   constexpr int KS = HD / 32;    // matrix-core k-steps per row
-  constexpr int TPW = ATT_CHUNK / 64;  // tiles per wave
-  constexpr int LROW = HD + 8;   // LDS row length of the K piece, in elements
-  constexpr int REGION = 4 * G * HD > 32 * LROW ? 4 * G * HD : 32 * LROW;
-  float* ored = smem;                         // [4][G][HD]   (after the scores)
-  u16* kpiece = reinterpret_cast<u16*>(smem);  // [4 waves][16][LROW] bf16 (during the scores)
-  float* sc = smem + REGION;                  // [G][ldsc]
-  const int ldsc = attn_sc_ld(chunk_max);
-  float* s_m = sc + G * ldsc;                 // [G]
-  float* s_l = s_m + G;                       // [G]
+  constexpr int LROW = HD + 8;   // LDS row length of the K and V pieces, in elements
+  constexpr int DT = HD / 64;    // 16-dimension tiles of a wave
+  u16* const piece = reinterpret_cast<u16*>(smem);  // [4 waves][16][LROW] of K (during the scores), then [64][LROW] of V
+  float* const sc = smem + 32 * LROW;               // [G][ldsc]
+  const int ldsc = attn_sc_ld(chunk_max), ldp = attn_p_ld(chunk_max);
+  float* const s_m = sc + G * ldsc;                 // [G]
+  float* const s_l = s_m + G;                       // [G]
+  u16* const sp = reinterpret_cast<u16*>(s_l + G + (4 - 2 * G % 4) % 4);  // [3][G][ldp] the weights' summands
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int Hq = Hkv * G;
@@ -91,16 +96,18 @@ __device__ __forceinline__ void attn_partial_item(const u16* __restrict__ q, int
   const int chunk = (nkeys + nsplit - 1) / nsplit;
   const int k0 = split * chunk;
   const int k1 = k0 + chunk < nkeys ? k0 + chunk : nkeys;
-  const int n = k1 - k0;  // <= chunk_max <= ATT_CHUNK by construction
+  const int n = k1 - k0;  // <= chunk_max <= 64 GROUPS by construction
 
   float* o_out = o_part + (((int64_t)b * Hq + kvh * G) * nsplit + split) * HD;  // + g * nsplit * HD
   float* ml_out = ml_part + (((int64_t)b * Hq + kvh * G) * nsplit + split) * 2;  // + g * nsplit * 2
+  // four consecutive outputs of head g; a head's statistics
+  auto put = [&](int g, int d, const f32x4_t& v) { *reinterpret_cast<f32x4_t*>(o_out + g * nsplit * HD + d) = v; };
+  auto put_ml = [&](int g, float m, float l) {
+    *reinterpret_cast<f32x2_t*>(ml_out + g * nsplit * 2) = f32x2_t{m, l};
+  };
   if (n <= 0) {
-    for (int i = tid; i < G * HD; i += 256) o_out[(int64_t)(i / HD) * nsplit * HD + (i % HD)] = 0.0f;
-    if (tid < G) {
-      ml_out[(int64_t)tid * nsplit * 2] = -INFINITY;
-      ml_out[(int64_t)tid * nsplit * 2 + 1] = 0.0f;
-    }
+    for (int i = tid * 4; i < G * HD; i += 1024) put(i / HD, i % HD, f32x4_t{0.0f, 0.0f, 0.0f, 0.0f});
+    if (tid < G) put_ml(tid, -INFINITY, 0.0f);
     return;
   }
 
@@ -112,71 +119,42 @@ __device__ __forceinline__ void attn_partial_item(const u16* __restrict__ q, int
   // wave w owns the 16-key tiles w, w + 4, ...; instruction i of a tile covers keys i * KPW .. + KPW
   // q as B fragments: column = head lane % 16, k-step ks holds elements ks * 32 + (lane / 16) * 8 .. + 8
   const int l16 = lane & 15, l4 = lane >> 4;
-  uint4 kr[TPW][NI], vr[TPW][NI];
+  u32x4_t kr[GROUPS][NI], vr[GROUPS][NI];
   bf16x8_t qf[KS];
-  if constexpr (EAGER) {
+  {
     constexpr int OOB_ = (int)0x80000000;
     const __amdgpu_buffer_rsrc_t kres = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(kbase), 0, 0x7fffffff, 0x00020000);
     const __amdgpu_buffer_rsrc_t vres = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(vbase), 0, 0x7fffffff, 0x00020000);
     const __amdgpu_buffer_rsrc_t qres = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<u16*>(q + (int64_t)b * ldq + (int64_t)kvh * G * HD), 0, 0x7fffffff, 0x00020000);
-    auto bld = [](const __amdgpu_buffer_rsrc_t& r, int off) {
-      const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
-      return make_uint4(v.x, v.y, v.z, v.w);
-    };
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const uint4 v = bld(qres, l16 < G ? (l16 * HD + ks * 32 + l4 * 8) * 2 : OOB_);
-      const u32x4_t vv = {v.x, v.y, v.z, v.w};
-      qf[ks] = __builtin_bit_cast(bf16x8_t, vv);
-    }
+    for (int ks = 0; ks < KS; ++ks)
+      qf[ks] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(qres, l16 < G ? (l16 * HD + ks * 32 + l4 * 8) * 2 : OOB_, 0, 0));
+    int off[GROUPS][NI];
 #pragma unroll
-    for (int j = 0; j < TPW; ++j)
+    for (int j = 0; j < GROUPS; ++j)
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
         const int key = k0 + (j * 4 + wave) * 16 + i * KPW + kl;
-        kr[j][i] = bld(kres, key < k1 ? (key * HD + dl) * 2 : OOB_);
+        off[j][i] = key < k1 ? (key * HD + dl) * 2 : OOB_;
+        kr[j][i] = __builtin_amdgcn_raw_buffer_load_b128(kres, off[j][i], 0, 0);
       }
 #pragma unroll
-    for (int j = 0; j < TPW; ++j)
+    for (int j = 0; j < GROUPS; ++j)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int key = k0 + (j * 4 + wave) * 16 + i * KPW + kl;
-        vr[j][i] = bld(vres, key < k1 ? (key * HD + dl) * 2 : OOB_);
-      }
-  } else {
-#pragma unroll
-    for (int j = 0; j < TPW; ++j)
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int key = k0 + (j * 4 + wave) * 16 + i * KPW + kl;
-        kr[j][i] = key < k1 ? ld16(kbase + (int64_t)key * HD + dl) : make_uint4(0, 0, 0, 0);
-      }
-#pragma unroll
-    for (int j = 0; j < TPW; ++j)
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int key = k0 + (j * 4 + wave) * 16 + i * KPW + kl;
-        vr[j][i] = key < k1 ? ld16(vbase + (int64_t)key * HD + dl) : make_uint4(0, 0, 0, 0);
-      }
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const uint4 v = l16 < G ? ld16(q + (int64_t)b * ldq + (kvh * G + l16) * HD + ks * 32 + l4 * 8) : make_uint4(0, 0, 0, 0);
-      const u32x4_t vv = {v.x, v.y, v.z, v.w};
-      qf[ks] = __builtin_bit_cast(bf16x8_t, vv);
-    }
+      for (int i = 0; i < NI; ++i) vr[j][i] = __builtin_amdgcn_raw_buffer_load_b128(vres, off[j][i], 0, 0);
   }
 
   // ---- scores: S[key][head] = sum_d K[key][d] q[head][d] on the matrix cores
   {
-    u16* my = kpiece + wave * 16 * LROW;
+    u16* my = piece + wave * 16 * LROW;
 #pragma unroll
-    for (int j = 0; j < TPW; ++j) {
+    for (int j = 0; j < GROUPS; ++j) {
       const int t16 = (j * 4 + wave) * 16;  // first key of the tile, relative to k0
       if (t16 < n) {  // uniform
         asm volatile("" ::: "memory");
 #pragma unroll
-        for (int i = 0; i < NI; ++i) st16(my + (i * KPW + kl) * LROW + dl, kr[j][i]);
+        for (int i = 0; i < NI; ++i) *reinterpret_cast<u32x4_t*>(my + (i * KPW + kl) * LROW + dl) = kr[j][i];
         asm volatile("" ::: "memory");
         f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -193,76 +171,85 @@ __device__ __forceinline__ void attn_partial_item(const u16* __restrict__ q, int
     }
   }
   __syncthreads();
+  auto store_v = [&](int j) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) *reinterpret_cast<u32x4_t*>(piece + (wave * 16 + i * KPW + kl) * LROW + dl) = vr[j][i];
+  };
+  store_v(0);
 
-  // ---- softmax statistics per head; sc becomes exp(s - max)
+  // ---- softmax statistics per head; the weights exp(s - max) as sums of three bf16 numbers, zero from key n on
   for (int g = wave; g < G; g += 4) {
-    float m = -INFINITY;
-    for (int i = lane; i < n; i += 64) m = fmaxf(m, sc[g * ldsc + i]);
+    float v[GROUPS], m = -INFINITY, l = 0.0f;
+#pragma unroll
+    for (int t = 0; t < GROUPS; ++t) {
+      v[t] = t * 64 + lane < n ? sc[g * ldsc + t * 64 + lane] : -INFINITY;
+      m = fmaxf(m, v[t]);
+    }
     m = wave_max(m);
-    float l = 0.0f;
-    for (int i = lane; i < n; i += 64) {
-      const float p = expf(sc[g * ldsc + i] - m);
-      sc[g * ldsc + i] = p;
-      l += p;
+#pragma unroll
+    for (int t = 0; t < GROUPS; ++t) {
+      if (t * 64 < n) {  // uniform
+        const float p = t * 64 + lane < n ? expf(v[t] - m) : 0.0f;
+        l += p;
+        const float p0 = round_bf(p), p1 = round_bf(p - p0);
+        u16* const at = sp + g * ldp + t * 64 + lane;
+        at[0] = f_to_bf(p0);
+        at[G * ldp] = f_to_bf(p1);
+        at[2 * G * ldp] = f_to_bf(p - p0 - p1);
+      }
     }
     l = wave_sum(l);
     if (lane == 0) { s_m[g] = m; s_l[g] = l; }
   }
   __syncthreads();
 
-  // ---- P.V
-  {
-    float acc[G][8];
+  // ---- P.V: O^T[dim][head] = sum_key V[key][dim] p[head][key]; a wave has DT tiles of 16 dimensions.  Three sums, of the
+  // weights' leading parts in even and in odd steps and of what is left of them: few roundings at the size of the result, short chains.
+  f32x4_t acc[DT][3];
 #pragma unroll
-    for (int g = 0; g < G; ++g)
+  for (int d = 0; d < DT; ++d)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc[g][j] = 0.0f;
+    for (int c = 0; c < 3; ++c) acc[d][c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  const int ph = l16 < G ? l16 : 0;   // (the columns beyond G are not stored)
 #pragma unroll
-    for (int j = 0; j < TPW; ++j) {
-      const int t16 = (j * 4 + wave) * 16;
-      if (t16 < n) {  // uniform
+  for (int j = 0; j < GROUPS; ++j) {
+    if (j * 64 < n) {  // uniform
+      if (j > 0) {
+        __syncthreads();
+        store_v(j);
+        __syncthreads();
+      }
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-          const int kk = t16 + i * KPW + kl;  // relative to k0
-          if (kk < n) {
-            float vf[8];
-            unpack8(vr[j][i], vf);
+      for (int ks = 0; ks < 2; ++ks) {
+        bf16x8_t pf[3];
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-              const float p = sc[g * ldsc + kk];
+        for (int w = 0; w < 3; ++w) pf[w] = *reinterpret_cast<const bf16x8_t*>(sp + (w * G + ph) * ldp + j * 64 + ks * 32 + l4 * 8);
 #pragma unroll
-              for (int e = 0; e < 8; ++e) acc[g][e] = fmaf(p, vf[e], acc[g][e]);
-            }
+        for (int d = 0; d < DT; ++d) {
+          // 16 lanes read 4 rows of 16 dimensions, a lane 4 of one row, and receive the 4 keys of one dimension each
+          const u16* const at = piece + (ks * 32 + l4 * 8 + (l16 >> 2)) * LROW + wave * (HD / 4) + d * 16 + (l16 & 3) * 4;
+          const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(at));
+          const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(at + 4 * LROW));
+          const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+          for (int w = 2; w >= 0; --w) {
+            f32x4_t& to = acc[d][w ? 2 : ks];
+            to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[w], to, 0, 0, 0);
           }
         }
       }
     }
-    // fold the KPW key groups of the wave, then the four waves through LDS (fixed order)
+  }
+  if (l16 < G) {
 #pragma unroll
-    for (int g = 0; g < G; ++g)
+    for (int d = 0; d < DT; ++d) {
+      f32x4_t o = acc[d][0] + acc[d][1];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float v = acc[g][j];
-#pragma unroll
-        for (int o = LPK; o < 64; o <<= 1) v += __shfl_xor(v, o, LR_WAVE);
-        acc[g][j] = v;
-      }
-    if (kl == 0) {
-#pragma unroll
-      for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) ored[(wave * G + g) * HD + dl + j] = acc[g][j];
+      for (int e = 0; e < 4; ++e) o[e] = fabsf(acc[d][2][e]) < INFINITY ? o[e] + acc[d][2][e] : o[e];   // (an infinite V: its weight's parts may be zero or negative)
+      put(l16, wave * (HD / 4) + d * 16 + l4 * 4, o);
     }
   }
-  __syncthreads();
-  for (int i = tid; i < G * HD; i += 256) {
-    const float v = (ored[i] + ored[G * HD + i]) + (ored[2 * G * HD + i] + ored[3 * G * HD + i]);
-    o_out[(int64_t)(i / HD) * nsplit * HD + (i % HD)] = v;
-  }
-  if (tid < G) {
-    ml_out[(int64_t)tid * nsplit * 2] = s_m[tid];
-    ml_out[(int64_t)tid * nsplit * 2 + 1] = s_l[tid];
-  }
+  if (tid < G) put_ml(tid, s_m[tid], s_l[tid]);
 }
 
 // ---- merge of the chunk results: y = sum_s w_s o_s with w_s = exp(m_s - max) / sum_s' exp(m_s' - max) l_s'

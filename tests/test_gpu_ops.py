@@ -777,6 +777,32 @@ def test_attn_decode(hip, B, Hq, Hkv, hd, Smax, pos):
     assert_close_ulp(y, want, max_frac=0.03, what="attn_decode")
 
 
+@pytest.mark.parametrize("hd,Hq,Smax", [(128, 8, 64), (128, 16, 128), (64, 4, 129), (128, 2, 256), (64, 1, 2176)])
+@pytest.mark.parametrize("pos", [0, 14, 15, 16, 63, 64, 65, 128, 200, 2175])
+def test_attn_decode_chunk_edges_and_infinite_values(hip, hd, Hq, Smax, pos):
+    """Positions at the edges of the 16-key tiles and 64-key groups, in chunks of two and of four groups; an infinite value comes
+    through as the sum of positive weights times it, and stays in its dimension."""
+    B, Hkv, pos = 3, 1, min(pos, Smax - 1)
+    q, kc, vc = rnd(B, Hq * hd, seed=24), rnd(B, Hkv, Smax, hd, seed=25), rnd(B, Hkv, Smax, hd, seed=26)
+    kc[:, :, pos + 1:] = 7.0
+    vc[:, :, pos + 1:] = float("nan")
+    p = torch.tensor([pos], dtype=torch.int32, device=DEV)
+    scratch = torch.empty(hip.attn_decode_scratch_bytes(B, Hq, hd, Smax) // 4, dtype=torch.float32, device=DEV)
+    mask = (torch.arange(Smax, device=DEV) <= pos).view(1, Smax)
+
+    def want():
+        v = vc.masked_fill(~mask.view(1, 1, Smax, 1), 0.0)
+        return O.sdpa_math(q.view(B, 1, Hq, hd).transpose(1, 2), kc, v, mask).transpose(1, 2).reshape(B, Hq * hd)
+    y = hip.attn_decode(q, kc, vc, p, torch.empty(B, Hq * hd, dtype=BF, device=DEV), scratch, B, Hq, Hkv, hd)
+    assert_close_ulp(y, want(), max_frac=0.03, what="attn_decode")
+    vc[1, 0, pos // 2, 5] = float("inf")
+    vc[2, 0, pos, 9] = float("-inf")
+    y, finite = hip.attn_decode(q, kc, vc, p, torch.empty_like(y), scratch, B, Hq, Hkv, hd), y
+    y, finite = y.view(B, Hq, hd), finite.view(B, Hq, hd).clone()
+    finite[1, :, 5], finite[2, :, 9] = float("inf"), float("-inf")
+    assert torch.equal(y, finite)
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,hd,Smax,pos,D,I,epi_swiglu", [
     (8, 8, 1, 128, 2176, 2100, 1024, 456, True),     # the 70B rank shard's heads at batch 8
     (16, 32, 8, 128, 1100, 1024, 512, 1000, True),   # Ladder-8B's heads at batch 16
