@@ -265,6 +265,12 @@ int lr_attn_decode_beside_normed(const void* q, int64_t ldq, const void* k_cache
                                  void* y, int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch,
                                  size_t scratch_bytes, const lr_projection_t* projection, const lr_row_norm_t* norm, int M,
                                  lr_stream_t stream);
+/* The same with the attention's chunk results merged inside the launch instead of in a second one: the same bits.  `tickets`: 32 * B * Hq uint32 on the device, zero before the first call and left zero
+ * by every call (calls that may overlap have their own); NULL: two launches.  norm may be NULL. */
+int lr_attn_decode_beside_merged(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos,
+                                 void* y, int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch,
+                                 size_t scratch_bytes, const lr_projection_t* projection, const lr_row_norm_t* norm,
+                                 void* tickets, int M, lr_stream_t stream);
 
 /* Weight-only fp8 linear:  y[m, n] = bf16( bf16( sum_k x[m, k] * w8[n, k] ) * scales[n] ).
  * w8 [N, K] dense float8 e4m3 (OCP "e4m3fn": bias 7, no infinities, max 448), one byte per weight;
@@ -318,6 +324,10 @@ int lr_attn_decode_beside_fp8_normed(const void* q, int64_t ldq, const void* k_c
                                      const int32_t* pos, void* y, int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax,
                                      void* scratch, size_t scratch_bytes, const lr_projection_fp8_t* projection,
                                      const lr_row_norm_t* norm, int M, lr_stream_t stream);
+int lr_attn_decode_beside_fp8_merged(const void* q, int64_t ldq, const void* k_cache, const void* v_cache,
+                                     const int32_t* pos, void* y, int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax,
+                                     void* scratch, size_t scratch_bytes, const lr_projection_fp8_t* projection,
+                                     const lr_row_norm_t* norm, void* tickets, int M, lr_stream_t stream);
 
 /* out[r, i] = bf16( bf16(silu(h[r, I + i])) * h[r, i] ),  h [rows, 2I] = [u | g] (row stride ldh).
  * F.silu(g) * u after chunk(2), utils.py:147-148 and :386. */

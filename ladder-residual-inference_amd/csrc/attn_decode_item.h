@@ -43,6 +43,9 @@ __host__ __device__ constexpr int attn_sc_ld(int chunk_max) { return ((chunk_max
 // and of the softmax weights', in bf16 elements: whole 64-key groups, plus 16 bytes for the same reason
 __host__ __device__ constexpr int attn_p_ld(int chunk_max) { return ((chunk_max + 63) & ~63) + 8; }
 
+// What other XCDs are to see or have written: past this XCD's L2 (bit 0 sc0, bit 4 sc1 of a raw buffer operation).
+constexpr int ATT_AUX_COHERENT = 17;
+
 // One (split, kv head, sequence) item of the split-KV decode attention, by 256 lanes (4 waves): scores,
 // softmax statistics and the un-normalised P.V of keys [k0, k1) (at most 64 GROUPS <= ATT_CHUNK) for all G q heads of
 // the kv head.  `smem`: attn_item_lds_floats<HD, G>(chunk_max) floats of LDS.  (A kv head with more q heads than
@@ -68,7 +71,8 @@ __host__ __device__ constexpr int attn_item_lds_floats(int chunk_max) {
 // GROUPS of 64 keys that an item's registers hold: two, or ATT_CHUNK / 64
 static inline bool attn_two_groups(int chunk_max) { return chunk_max <= 128; }
 
-template <int HD, int G, int GROUPS>
+// THROUGH: the results are written through to the memory side (sc0 sc1), where attn_merge_wave reads them.
+template <int HD, int G, int GROUPS, bool THROUGH = false>
 __device__ __forceinline__ void attn_partial_item(const u16* __restrict__ q, int64_t ldq, const u16* __restrict__ kc,
                                                   const u16* __restrict__ vc, const int32_t* __restrict__ pos_ptr,
                                                   float* __restrict__ o_part, float* __restrict__ ml_part, int Hkv,
@@ -100,10 +104,18 @@ __device__ __forceinline__ void attn_partial_item(const u16* __restrict__ q, int
 
   float* o_out = o_part + (((int64_t)b * Hq + kvh * G) * nsplit + split) * HD;  // + g * nsplit * HD
   float* ml_out = ml_part + (((int64_t)b * Hq + kvh * G) * nsplit + split) * 2;  // + g * nsplit * 2
+  const __amdgpu_buffer_rsrc_t ores = __builtin_amdgcn_make_buffer_rsrc(o_out, 0, ((G - 1) * nsplit + 1) * HD * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t mres = __builtin_amdgcn_make_buffer_rsrc(ml_out, 0, ((G - 1) * nsplit + 1) * 8, 0x00020000);
   // four consecutive outputs of head g; a head's statistics
-  auto put = [&](int g, int d, const f32x4_t& v) { *reinterpret_cast<f32x4_t*>(o_out + g * nsplit * HD + d) = v; };
+  auto put = [&](int g, int d, const f32x4_t& v) {
+    const int at = g * nsplit * HD + d;
+    if constexpr (THROUGH) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), ores, at * 4, 0, ATT_AUX_COHERENT);
+    else *reinterpret_cast<f32x4_t*>(o_out + at) = v;
+  };
   auto put_ml = [&](int g, float m, float l) {
-    *reinterpret_cast<f32x2_t*>(ml_out + g * nsplit * 2) = f32x2_t{m, l};
+    const f32x2_t v = {m, l};
+    if constexpr (THROUGH) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, v), mres, g * nsplit * 8, 0, ATT_AUX_COHERENT);
+    else *reinterpret_cast<f32x2_t*>(ml_out + g * nsplit * 2) = v;
   };
   if (n <= 0) {
     for (int i = tid * 4; i < G * HD; i += 1024) put(i / HD, i % HD, f32x4_t{0.0f, 0.0f, 0.0f, 0.0f});
@@ -308,6 +320,61 @@ __global__ __launch_bounds__(HD) void k_attn_decode_combine_once(const float* __
     }
   }
   y[(int64_t)b * ldy + h * HD + d] = f_to_bf(L > 0.0f ? o / L : 0.0f);
+}
+
+// The same inside the launch of the items, by waves of workgroups that stand behind them in the grid: whoever runs has seen all
+// items start, and an item waits for nobody, so the wait below ends (it is bounded all the same).  An item counts its
+// kv head's ticket up when the memory side has acknowledged its results (attn_item_done), and a wave reads them from there
+// (sc0 sc1): 64 outputs, all of up to 64 chunks' in one round trip.  The last of a kv head's waves sets the ticket back to zero.
+constexpr int ATT_MERGE_MAX = 64;   // chunks
+constexpr int ATT_TICKET = 32;      // words from one kv head's ticket to the next: 128 bytes
+__device__ __forceinline__ void attn_item_done(u32* ticket) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) (void)__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// `wave`: which 64 of the outputs [B][Hq * HD].  A merge in a launch of its own is 4.7 us per block
+// and step; here it ends before the weight stream does (70B rank shard, 8 rows: chunks stored at 6 us of 23, merged at 20).
+// What did not do: all of a head's outputs by whoever stores its last chunk (131 KB of 32 chunks through one CU beside its part of the
+// stream: the launch 2.5 us longer); tickets in one cache line, polled without a pause (the polls queue before the items' counts: e4m3,
+// 5 rows, the whole stream 12 -> 17 us).
+template <int HD, int G>
+__device__ __forceinline__ void attn_merge_wave(const float* __restrict__ o_part, const float* __restrict__ ml_part, u32* tickets, u16* __restrict__ y,
+                                                int64_t ldy, int Hkv, int nsplit, int wave) {
+  const int lane = threadIdx.x & 63, Hq = Hkv * G;
+  const int head = wave / (HD / 64), b = head / Hq, h = head - b * Hq, d = wave % (HD / 64) * 64 + lane;   // (head: of all sequences)
+  u32* const ticket = tickets + head / G * ATT_TICKET;
+  for (int i = 0; __hip_atomic_load(ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < (u32)nsplit && i < 1 << 16; ++i) __builtin_amdgcn_s_sleep(40);
+  asm volatile("" ::: "memory");
+  const __amdgpu_buffer_rsrc_t ores = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(o_part + (int64_t)head * nsplit * HD), 0, nsplit * HD * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t mres = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(ml_part + (int64_t)head * nsplit * 2), 0, nsplit * 8, 0x00020000);
+  // (a chunk beyond the last lies outside the resource and reads as zero)
+  const u32x2_t mlv = __builtin_amdgcn_raw_buffer_load_b64(mres, lane * 8, 0, ATT_AUX_COHERENT);
+  constexpr int NB = 32;
+  float ov[NB], o = 0.0f, L = 0.0f, w_lane = 0.0f, l_lane = 0.0f;
+  for (int s0 = 0; s0 < nsplit; s0 += NB) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) ov[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ores, ((s0 + j) * HD + d) * 4, 0, ATT_AUX_COHERENT));
+    if (s0 == 0) {
+      const float ms = lane < nsplit ? __uint_as_float(mlv.x) : -INFINITY;
+      l_lane = __uint_as_float(mlv.y);
+      const float M = wave_max(ms);
+      w_lane = ms == -INFINITY ? 0.0f : expf(ms - M);  // an empty chunk: (-inf, 0, 0)
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+      if (s0 + j < nsplit) {  // uniform
+        const float wgt = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w_lane), s0 + j));
+        L = fmaf(wgt, __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(l_lane), s0 + j)), L);
+        o = fmaf(wgt, ov[j], o);
+      }
+  }
+  y[(int64_t)b * ldy + h * HD + d] = f_to_bf(L > 0.0f ? o / L : 0.0f);
+  if (lane == 0) {
+    const u32 last = (u32)(nsplit + G * (HD / 64) - 1);
+    if (__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == last)
+      __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
 
 template <int HD>

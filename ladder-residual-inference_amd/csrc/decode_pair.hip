@@ -9,10 +9,9 @@
 // two workgroups share a CU and the attention disappears behind the weight stream.
 //
 // Both halves are the device functions their own kernels use (attn_partial_item, stream_band), so
-// the results are bit-identical to lr_attn_decode followed by lr_linear_multi.  The merge of the
-// attention's chunks stays a launch of its own: done inside this one by whoever stores the last
-// chunk of a kv head (chunk results written through to the memory side, one ticket per kv head),
-// it became the tail of the grid instead of hiding in it (0.4 ms per step slower at batch 8 and 16).
+// the results are bit-identical to lr_attn_decode followed by lr_linear_multi.  With a ticket per kv head
+// the chunks are merged here too, by workgroups at the end of the grid (attn_merge_wave), also beside the
+// weight stream; without, in a launch of their own.
 //
 // lr_attn_decode_beside_fp8: the same grid with the e4m3 variant of the band (weight-only quantised models,
 // 2 to 16 rows).
@@ -32,58 +31,74 @@ struct AttnItems {
   int Hkv, Smax, nsplit, chunk_max;  // Hkv: groups of G q heads (kv_share of them per head of the cache)
   int kv_share;
   int n_items;  // nsplit * Hkv * B: the first workgroups of the grid
+  // MERGE: the workgroups behind the bands merge the chunks into y
+  u32* tickets;  // [B * Hkv], zero
+  u16* y;
+  int64_t ldy;
+  int merge_waves, waves_per_wg;  // of 64 outputs; of them in a workgroup
 };
 
 constexpr int PAIR_MT = 16, PAIR_UNITS = 2;
 
 // X8: at most 8 input rows in fragment layout, requested as far ahead as the weights (see stream_band)
 // GROUPS: keys of an attention item, in 64s (see attn_partial_item)
-template <int HD, int G, bool W8, bool XL, int GROUPS, bool X8>
+template <int HD, int G, bool W8, bool XL, int GROUPS, bool X8, bool MERGE>
 __global__ __launch_bounds__(256, XL ? 0 : 2) void k_attn_beside_band(const AttnItems a, const Proj p, const int M) {
   extern __shared__ __attribute__((aligned(16))) unsigned char pair_smem[];
   const int wg = blockIdx.x;
   if (wg < a.n_items) {
     const int split = wg % a.nsplit, rest = wg / a.nsplit;
-    attn_partial_item<HD, G, GROUPS>(a.q, a.ldq, a.kc, a.vc, a.pos, a.o_part, a.ml_part, a.Hkv, a.Smax, a.nsplit,
-                             a.chunk_max, split, rest % a.Hkv, rest / a.Hkv, reinterpret_cast<float*>(pair_smem),
-                             a.kv_share);
+    float* const smem = reinterpret_cast<float*>(pair_smem);
+    attn_partial_item<HD, G, GROUPS, MERGE>(a.q, a.ldq, a.kc, a.vc, a.pos, a.o_part, a.ml_part, a.Hkv, a.Smax, a.nsplit,
+                                           a.chunk_max, split, rest % a.Hkv, rest / a.Hkv, smem, a.kv_share);
+    if constexpr (MERGE) attn_item_done(a.tickets + rest * ATT_TICKET);
+  } else if (MERGE && wg >= a.n_items + p.nwg) {
+    const int wave = threadIdx.x >> 6, m = (wg - a.n_items - p.nwg) * a.waves_per_wg + wave;
+    if (wave < a.waves_per_wg && m < a.merge_waves)
+      attn_merge_wave<HD, G>(a.o_part, a.ml_part, a.tickets, a.y, a.ldy, a.Hkv, a.nsplit, __builtin_amdgcn_readfirstlane(m));
   } else {
     stream_band<PAIR_MT, PAIR_UNITS, W8, XL, false, false, NWV, 16, X8, X8>(p, M, wg - a.n_items, reinterpret_cast<u16*>(pair_smem));
   }
 }
 
-template <int HD, int G, bool W8, bool XL, int GROUPS, bool X8 = !W8 && !XL>
-static int launch_pair_as(const AttnItems& a, const Proj& p, int M, u16* y, int64_t ldy, int B, hipStream_t s) {
-  const int Hq = a.Hkv * G;
+template <int HD, int G, bool W8, bool XL, int GROUPS, bool X8, bool MERGE>
+static int launch_pair_merge(const AttnItems& a, const Proj& p, int M, int B, hipStream_t s) {
+  const int mergers = MERGE ? (a.merge_waves + a.waves_per_wg - 1) / a.waves_per_wg : 0;
   const size_t lds_att = (size_t)attn_item_lds_floats<HD, G>(a.chunk_max) * sizeof(float);
   const size_t lds_band = stream_band_lds_bytes<PAIR_MT, PAIR_UNITS, W8, XL>() + stream_band_norm_bytes(p, M);
   const size_t lds = lds_att > lds_band ? lds_att : lds_band;
   static std::atomic<unsigned long long> lds_raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_attn_beside_band<HD, G, W8, XL, GROUPS, X8>), lds, lds_raised)) return LR_E_LAUNCH;
-  k_attn_beside_band<HD, G, W8, XL, GROUPS, X8><<<dim3((unsigned)(a.n_items + p.nwg)), dim3(256), lds, s>>>(a, p, M);
-  launch_attn_combine<HD>(a.o_part, a.ml_part, y, ldy, Hq, B, a.nsplit, s);
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_attn_beside_band<HD, G, W8, XL, GROUPS, X8, MERGE>), lds, lds_raised)) return LR_E_LAUNCH;
+  k_attn_beside_band<HD, G, W8, XL, GROUPS, X8, MERGE><<<dim3((unsigned)(a.n_items + p.nwg + mergers)), dim3(256), lds, s>>>(a, p, M);
+  if (!MERGE) launch_attn_combine<HD>(a.o_part, a.ml_part, a.y, a.ldy, a.Hkv * G, B, a.nsplit, s);
   return lr_launch_status();
+}
+template <int HD, int G, bool W8, bool XL, int GROUPS, bool X8 = !W8 && !XL>
+static int launch_pair_as(const AttnItems& a, const Proj& p, int M, int B, hipStream_t s) {
+  return a.tickets ? launch_pair_merge<HD, G, W8, XL, GROUPS, X8, true>(a, p, M, B, s)
+                   : launch_pair_merge<HD, G, W8, XL, GROUPS, X8, false>(a, p, M, B, s);
 }
 
 // (the band's inputs in whole lines or in fragment layout: the choice lr_linear_multi makes for the same rows)
 template <int HD, int G, bool W8>
-static int launch_pair(const AttnItems& a, const Proj& p, int M, u16* y, int64_t ldy, int B, hipStream_t s) {
+static int launch_pair(const AttnItems& a, const Proj& p, int M, int B, hipStream_t s) {
   const bool two = attn_two_groups(a.chunk_max);
   if (!W8 && M >= XLDS_M16_FROM)
-    return two ? launch_pair_as<HD, G, false, true, 2>(a, p, M, y, ldy, B, s)
-               : launch_pair_as<HD, G, false, true, 4>(a, p, M, y, ldy, B, s);
+    return two ? launch_pair_as<HD, G, false, true, 2>(a, p, M, B, s)
+               : launch_pair_as<HD, G, false, true, 4>(a, p, M, B, s);
   if (W8 && M <= 8)
-    return two ? launch_pair_as<HD, G, W8, false, 2, true>(a, p, M, y, ldy, B, s)
-               : launch_pair_as<HD, G, W8, false, 4, true>(a, p, M, y, ldy, B, s);
-  return two ? launch_pair_as<HD, G, W8, false, 2>(a, p, M, y, ldy, B, s)
-             : launch_pair_as<HD, G, W8, false, 4>(a, p, M, y, ldy, B, s);
+    return two ? launch_pair_as<HD, G, W8, false, 2, true>(a, p, M, B, s)
+               : launch_pair_as<HD, G, W8, false, 4, true>(a, p, M, B, s);
+  return two ? launch_pair_as<HD, G, W8, false, 2>(a, p, M, B, s)
+             : launch_pair_as<HD, G, W8, false, 4>(a, p, M, B, s);
 }
 
 // shared body of the two entry points; `fill` turns the caller's projection into a Proj
 template <bool W8, class Projection, class Fill>
 static int beside(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos, void* y,
                   int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch, size_t scratch_bytes,
-                  const Projection* proj, const lr_row_norm_t* norm, int M, int m_min, lr_stream_t stream, Fill fill) {
+                  const Projection* proj, const lr_row_norm_t* norm, void* tickets, int M, int m_min, lr_stream_t stream,
+                  Fill fill) {
   LR_REQUIRE_PTR(q);
   LR_REQUIRE_PTR(k_cache);
   LR_REQUIRE_PTR(v_cache);
@@ -95,6 +110,7 @@ static int beside(const void* q, int64_t ldq, const void* k_cache, const void* v
   if (ldq < (int64_t)Hq * hd || ldy < (int64_t)Hq * hd || B > 65535) return LR_E_SHAPE;
   if (ldq % 8 || ldy % 8) return LR_E_ALIGN;
   if (scratch_bytes < lr_attn_decode_scratch_bytes(B, Hq, hd, Smax)) return LR_E_SHAPE;
+  if (((uintptr_t)tickets & 3) != 0) return LR_E_ALIGN;
   // the projection must not touch the cache the attention reads, and only the 16-row band shares a CU
   if (proj->epilogue == LR_EPI_ROPE_KV || M > PAIR_MT || M < m_min) return LR_E_UNSUPPORTED;
   Proj p;
@@ -118,14 +134,18 @@ static int beside(const void* q, int64_t ldq, const void* k_cache, const void* v
   a.ml_part = a.o_part + (size_t)B * Hq * a.nsplit * hd;
   if ((int64_t)a.nsplit * a.Hkv * B > 0x3fffffff) return LR_E_UNSUPPORTED;
   a.n_items = a.nsplit * a.Hkv * B;
+  a.y = (u16*)y; a.ldy = ldy;
+  a.tickets = a.nsplit <= ATT_MERGE_MAX ? (u32*)tickets : nullptr;   // (more chunks: a launch of their own)
   if (!((hd == 128 || hd == 64) && (G == 1 || G == 2 || G == 4 || G == 8))) return LR_E_UNSUPPORTED;
   const int ncu = lr_num_cus();
   if (ncu < 1) return LR_E_LAUNCH;
   plan(p, M, p.pair_off ? 16 : 16 * PAIR_UNITS, ncu);
+  a.merge_waves = B * Hq * (hd / 64);
+  a.waves_per_wg = a.merge_waves > 2 * ncu ? 4 : a.merge_waves > ncu ? 2 : 1;   // (spread over the CUs, whose bands are to end together)
   if (p.fold_sums && p.nwg < M) return LR_E_UNSUPPORTED;   // (a row per workgroup)
   hipStream_t s = (hipStream_t)stream;
 #define LR_PAIR(HDV, GV) \
-  if (hd == HDV && G == GV) return launch_pair<HDV, GV, W8>(a, p, M, (u16*)y, ldy, B, s);
+  if (hd == HDV && G == GV) return launch_pair<HDV, GV, W8>(a, p, M, B, s);
   LR_PAIR(128, 1) LR_PAIR(128, 2) LR_PAIR(128, 4) LR_PAIR(128, 8)
   LR_PAIR(64, 1) LR_PAIR(64, 2) LR_PAIR(64, 4) LR_PAIR(64, 8)
 #undef LR_PAIR
@@ -134,36 +154,53 @@ static int beside(const void* q, int64_t ldq, const void* k_cache, const void* v
 
 }  // namespace
 
+extern "C" int lr_attn_decode_beside_merged(const void* q, int64_t ldq, const void* k_cache, const void* v_cache,
+                                            const int32_t* pos, void* y, int64_t ldy, int B, int Hq, int Hkv, int hd,
+                                            int Smax, void* scratch, size_t scratch_bytes, const lr_projection_t* proj,
+                                            const lr_row_norm_t* norm, void* tickets, int M, lr_stream_t stream) {
+  return beside<false>(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj, norm, tickets, M, 1,
+                       stream, sb_fill_projection);
+}
+
 extern "C" int lr_attn_decode_beside_normed(const void* q, int64_t ldq, const void* k_cache, const void* v_cache,
                                             const int32_t* pos, void* y, int64_t ldy, int B, int Hq, int Hkv, int hd,
                                             int Smax, void* scratch, size_t scratch_bytes, const lr_projection_t* proj,
                                             const lr_row_norm_t* norm, int M, lr_stream_t stream) {
-  return beside<false>(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj, norm, M, 1,
-                       stream, sb_fill_projection);
+  return lr_attn_decode_beside_merged(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj,
+                                      norm, nullptr, M, stream);
 }
 
 extern "C" int lr_attn_decode_beside(const void* q, int64_t ldq, const void* k_cache, const void* v_cache,
                                      const int32_t* pos, void* y, int64_t ldy, int B, int Hq, int Hkv, int hd,
                                      int Smax, void* scratch, size_t scratch_bytes, const lr_projection_t* proj,
                                      int M, lr_stream_t stream) {
-  return lr_attn_decode_beside_normed(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj,
-                                      nullptr, M, stream);
+  return lr_attn_decode_beside_merged(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj,
+                                      nullptr, nullptr, M, stream);
 }
 
 // (for one row lr_linear_fp8_multi uses the matrix-vector kernel, which has no band to put beside the attention)
+extern "C" int lr_attn_decode_beside_fp8_merged(const void* q, int64_t ldq, const void* k_cache, const void* v_cache,
+                                                const int32_t* pos, void* y, int64_t ldy, int B, int Hq, int Hkv, int hd,
+                                                int Smax, void* scratch, size_t scratch_bytes,
+                                                const lr_projection_fp8_t* proj, const lr_row_norm_t* norm, void* tickets,
+                                                int M, lr_stream_t stream) {
+  return beside<true>(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj, norm, tickets, M,
+                      LR_FP8_GEMV_MAX_M + 1, stream, sb_fill_projection_fp8);
+}
+
 extern "C" int lr_attn_decode_beside_fp8_normed(const void* q, int64_t ldq, const void* k_cache, const void* v_cache,
                                                 const int32_t* pos, void* y, int64_t ldy, int B, int Hq, int Hkv, int hd,
                                                 int Smax, void* scratch, size_t scratch_bytes,
                                                 const lr_projection_fp8_t* proj, const lr_row_norm_t* norm, int M,
                                                 lr_stream_t stream) {
-  return beside<true>(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj, norm, M,
-                      LR_FP8_GEMV_MAX_M + 1, stream, sb_fill_projection_fp8);
+  return lr_attn_decode_beside_fp8_merged(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj,
+                                          norm, nullptr, M, stream);
 }
 
 extern "C" int lr_attn_decode_beside_fp8(const void* q, int64_t ldq, const void* k_cache, const void* v_cache,
                                          const int32_t* pos, void* y, int64_t ldy, int B, int Hq, int Hkv, int hd,
                                          int Smax, void* scratch, size_t scratch_bytes,
                                          const lr_projection_fp8_t* proj, int M, lr_stream_t stream) {
-  return lr_attn_decode_beside_fp8_normed(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj,
-                                          nullptr, M, stream);
+  return lr_attn_decode_beside_fp8_merged(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, proj,
+                                          nullptr, nullptr, M, stream);
 }

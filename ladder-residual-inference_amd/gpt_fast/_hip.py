@@ -66,6 +66,12 @@ _PROTOS = {
     "lr_attn_decode_beside_fp8_normed": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int,
                                                  c_int, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p, c_void_p, c_int,
                                                  c_void_p]),
+    "lr_attn_decode_beside_merged": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
+                                             c_int, c_int, c_int, c_void_p, c_size_t, c_void_p, c_void_p, c_void_p, c_int,
+                                             c_void_p]),
+    "lr_attn_decode_beside_fp8_merged": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int,
+                                                 c_int, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p, c_void_p, c_void_p,
+                                                 c_int, c_void_p]),
     "lr_attn_decode_static": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
                                       c_int, c_int, c_int, c_void_p]),
     "lr_attn_prefill": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
@@ -479,18 +485,26 @@ def linear_fp8_multi(*projections):
            "lr_linear_fp8_multi_normed")
 
 
-def attn_decode_beside_fp8(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, projection) -> bool:
+def _tickets(t, n):
+    if t is None:
+        return None
+    assert t.is_cuda and t.dtype == torch.int32 and t.is_contiguous() and t.numel() >= n, (t.shape, n)
+    return t.data_ptr()
+
+
+def attn_decode_beside_fp8(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, projection, tickets=None) -> bool:
     """attn_decode and linear_fp8_multi(projection) in one launch (lr_attn_decode_beside_fp8); False, with nothing
-    launched, when the library has no such kernel for the shape (a single row among them)."""
+    launched, when the library has no such kernel for the shape (a single row among them).  tickets: as in
+    attn_decode_beside."""
     _, _, ldq = _rows_ld(q)
     _, _, ldy = _rows_ld(y)
     Smax = k_cache.shape[2]
     assert pos.dtype == torch.int32 and pos.numel() == 1 and scratch.dtype == torch.float32
     (projection,), norms = _norms_of((projection,))
     arr, M, _keep = _projection_fp8_array((projection,))
-    rc = load().lr_attn_decode_beside_fp8_normed(_dev(q), ldq, _dev(k_cache), _dev(v_cache), pos.data_ptr(), _dev(y), ldy, B,
+    rc = load().lr_attn_decode_beside_fp8_merged(_dev(q), ldq, _dev(k_cache), _dev(v_cache), pos.data_ptr(), _dev(y), ldy, B,
                                                  Hq, Hkv, hd, Smax, scratch.data_ptr(), scratch.numel() * 4,
-                                                 ctypes.cast(arr, c_void_p), norms, M, _stream())
+                                                 ctypes.cast(arr, c_void_p), norms, _tickets(tickets, 32 * B * Hq), M, _stream())
     if rc == E_UNSUPPORTED:
         return False
     _check(rc, "lr_attn_decode_beside_fp8")
@@ -726,18 +740,19 @@ def attn_decode(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd):
     return y
 
 
-def attn_decode_beside(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, projection) -> bool:
+def attn_decode_beside(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, projection, tickets=None) -> bool:
     """attn_decode and linear_multi(projection) in one launch (lr_attn_decode_beside); the two must not depend
-    on each other.  False, with nothing launched, when the library has no such kernel for the shape."""
+    on each other.  False, with nothing launched, when the library has no such kernel for the shape.  tickets: 32 B Hq
+    int32, zero and left zero (None: the chunk results are merged by a launch of their own)."""
     _, _, ldq = _rows_ld(q)
     _, _, ldy = _rows_ld(y)
     Smax = k_cache.shape[2]
     assert pos.dtype == torch.int32 and pos.numel() == 1 and scratch.dtype == torch.float32
     (projection,), norms = _norms_of((projection,))
     arr, M, _keep = _projection_array((projection,))
-    rc = load().lr_attn_decode_beside_normed(_dev(q), ldq, _dev(k_cache), _dev(v_cache), pos.data_ptr(), _dev(y), ldy, B, Hq,
+    rc = load().lr_attn_decode_beside_merged(_dev(q), ldq, _dev(k_cache), _dev(v_cache), pos.data_ptr(), _dev(y), ldy, B, Hq,
                                              Hkv, hd, Smax, scratch.data_ptr(), scratch.numel() * 4,
-                                             ctypes.cast(arr, c_void_p), norms, M, _stream())
+                                             ctypes.cast(arr, c_void_p), norms, _tickets(tickets, 32 * B * Hq), M, _stream())
     if rc == E_UNSUPPORTED:
         return False
     _check(rc, "lr_attn_decode_beside")

@@ -68,6 +68,9 @@ class Workspace:
         if S == 1:
             n = _hip.attn_decode_scratch_bytes(B, cfg.n_head_local, hd, smax) // 4
             self.scratch = torch.empty(n, dtype=torch.float32, device=device)
+            # attn_decode_beside's (none where they would be zero only once a graph that is being captured is replayed)
+            capturing = device.type == "cuda" and torch.cuda.is_current_stream_capturing()
+            self.tickets = None if capturing else torch.zeros(32 * B * cfg.n_head_local, dtype=torch.int32, device=device)
 
 
 class GPTBase(nn.Module):

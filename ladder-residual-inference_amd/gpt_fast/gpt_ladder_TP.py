@@ -187,7 +187,7 @@ class GPTLadder(GPTBase):
                     # items run in the same launch and wait for the KV cache behind the weight stream
                     _hip.linear_multi((xn, blk.attention.wqkv.weight, ws.qkv, rope))
                     beside = _hip.attn_decode_beside(ws.qkv, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B,
-                                                     cfg.n_head_local, cfg.n_kv_local, cfg.head_dim, up_gate)
+                                                     cfg.n_head_local, cfg.n_kv_local, cfg.head_dim, up_gate, ws.tickets)
                     if not beside:
                         _hip.linear_multi(up_gate)
                         self._attention(ws, blk, pos, None, None, roped=True)
@@ -207,7 +207,7 @@ class GPTLadder(GPTBase):
                 if beside8:
                     _hip.linear_fp8_multi(qkv8)
                     beside8 = _hip.attn_decode_beside_fp8(ws.qkv, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B,
-                                                          cfg.n_head_local, cfg.n_kv_local, cfg.head_dim, up_gate8)
+                                                          cfg.n_head_local, cfg.n_kv_local, cfg.head_dim, up_gate8, ws.tickets)
                     if not beside8:
                         _hip.linear_fp8_multi(up_gate8)
                         self._attention(ws, blk, pos, None, None, roped=True)

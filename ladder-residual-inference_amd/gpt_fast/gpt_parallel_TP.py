@@ -99,7 +99,8 @@ class GPTParallel(GPTBase):
                 _hip.linear(ws.act, att.w2.weight, ws.m, scratch=ws.sums)
             elif ws.B <= 16:
                 _hip.linear_multi(qkv)
-                if not _hip.attn_decode_beside(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd, up_gate):
+                if not _hip.attn_decode_beside(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd, up_gate,
+                                               ws.tickets):
                     _hip.linear_multi(up_gate)
                     _hip.attn_decode(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd)
             else:

@@ -863,6 +863,41 @@ def test_attn_decode_beside_fp8_equals_the_two_calls(hip, B, Hq, Hkv, hd, Smax, 
     assert bool((o1 == 5.0).all()) and bool((y1 == 5.0).all())
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("B,Hq,Hkv,hd,Smax,pos", [
+    (8, 8, 1, 128, 2176, 2100),      # 32 chunks, the whole first round trip
+    (3, 4, 4, 64, 4096, 4095),       # more than 32 chunks: two round trips; one q head per kv head
+    (2, 8, 1, 128, 4096, 40),        # 64 chunks, most of them without a key
+    (16, 32, 8, 128, 1100, 1024),    # few chunks, several kv heads
+    (5, 16, 1, 128, 520, 400),       # 16 q heads as two groups of 8
+    (4, 8, 2, 64, 40, 0),            # one chunk, one key
+    (2, 8, 1, 128, 20000, 19000),    # more chunks than the merge inside the launch takes: a launch of its own
+])
+def test_attn_decode_merged_beside_a_projection_equals_the_two_launches(hip, fp8, B, Hq, Hkv, hd, Smax, pos):
+    """The chunks merged by whoever stores a kv head's last one: the bits of the merge in a launch of its own, launch after
+    launch, with scratch of NaN (nothing is read that this call has not written), and the tickets zero again."""
+    D, I = 272, 72
+    q = rnd(B, (Hq + 2 * Hkv) * hd, seed=50)
+    p = torch.tensor([pos], dtype=torch.int32, device=DEV)
+    x = rnd(B, D, seed=53)
+    w = rnd(2 * I, D, seed=54, scale=0.05, dtype=torch.float32)
+    if fp8:
+        proj, beside, alone = (x, *O.quantize_fp8_rowwise(w, BF)), hip.attn_decode_beside_fp8, hip.linear_fp8_multi
+    else:
+        proj, beside, alone = (x, w.to(BF)), hip.attn_decode_beside, hip.linear_multi
+    tickets = torch.zeros(32 * B * Hq, dtype=torch.int32, device=DEV)
+    scratch = torch.empty(hip.attn_decode_scratch_bytes(B, Hq, hd, Smax) // 4, dtype=torch.float32, device=DEV)
+    for seed in range(4):
+        kc, vc = rnd(B, Hkv, Smax, hd, seed=60 + seed), rnd(B, Hkv, Smax, hd, seed=80 + seed)
+        y, out = torch.zeros(2, B, Hq * hd, dtype=BF, device=DEV), torch.zeros(2, B, I, dtype=BF, device=DEV)
+        hip.attn_decode(q, kc, vc, p, y[0], scratch, B, Hq, Hkv, hd)
+        alone((*proj, out[0], hip.EPI_SWIGLU))
+        scratch.fill_(float("nan"))
+        assert beside(q, kc, vc, p, y[1], scratch, B, Hq, Hkv, hd, (*proj, out[1], hip.EPI_SWIGLU), tickets)
+        assert torch.equal(y[1], y[0]) and torch.equal(out[1], out[0]) and bool(y[0].any())
+        assert not bool(tickets.any())
+
+
 def test_attn_decode_beside_declines_what_it_has_no_kernel_for(hip):
     """More than 16 rows, 32 q heads per kv head, or a projection that writes the cache: False, nothing launched."""
     def run(B, Hq, Hkv, epi=None):
