@@ -131,8 +131,8 @@ __global__ __launch_bounds__(256) void k_gemm(const u16* __restrict__ x, int64_t
 }
 
 // ---------------------------------------------------------------------------------------------
-// The GEMM of prompts and of decode batches above 32.  A workgroup of four waves (2 x 2) multiplies a tile of 64 A16 input
-// rows x 128 BH weight rows: 256 x 256, 128 x 256, 128 x 128 or 64 x 128 (gemm_plan picks).  Bound: the matrix cores, at the
+// The GEMM of prompts and of decode batches above 32.  A workgroup of four waves (2 x 2) multiplies a tile of 32 A input
+// rows x 128 BH weight rows: 160 to 256 rows in steps of 32, or 128, by 256; 64, 128, 160 or 192 by 128 (gemm_plan picks).  Bound: the matrix cores, at the
 // clock the chip's power allows, from a few hundred rows on (16384 x 4096 x 14336, one counter run: 1302 us = 1.48 PFLOP/s,
 // matrix cores busy 79 % of the cycles at 1.78 GHz); the weights' HBM traffic below.
 //
@@ -142,7 +142,12 @@ __global__ __launch_bounds__(256) void k_gemm(const u16* __restrict__ x, int64_t
 // from and again by the address a fragment is read at: conflict-free for the 16-row fragments of
 // v_mfma_f32_16x16x32_bf16.
 //
-// A k-tile is 64 elements; its operand rows come in two halves each (A: input rows, B: weight rows) and the tile's four
+// What a tile of fewer rows costs is what the L2s give a CU, about 65 GB/s: (m + n) * 128 bytes per k-tile, 1.0 us at 256 x 256 where the
+// matrix cores need 1.1 to 1.2, 0.5 at 128 x 128 where they need 0.3.  So tiles from 160 rows on are as good per row as the largest, and rows
+// that are no multiple of 256 want them: 777 rows are four tiles of 224 (measured below, at GEMM_TILES).
+//
+// A k-tile is 64 elements; its operand rows come in two halves each (A: input rows, B: weight rows; the first half of the input
+// rows has a group of 16 per wave more where A is odd) and the tile's four
 // quarter products follow one another in four phases, (A0 B0) (A0 B1) (A1 B1) (A1 B0).  Every phase reads ONE half from
 // LDS into registers for a later phase and requests the half of two k-tiles ahead into the LDS slot that the phase before
 // it emptied: a request has seven phases to land, a slot is read in exactly one phase, and one barrier per phase orders
@@ -186,16 +191,23 @@ struct GemmSplit {
 };
 enum { GEMM_PLAIN, GEMM_PAIR, GEMM_ROPE, GEMM_ROWS };   // ROWS: every tile is cut, the pieces stay, see GemmSplit; PAIR: w holds [up; gate] rows, N counts pairs, output silu(gate) * up
 
-template <int A16, int BH>
+template <int A, int BH>
 struct GemmTile {
-  static constexpr int TM = 64 * A16, TN = 128 * BH;
-  static constexpr int HA = 4096 * A16, HB = 8192 * BH;   // bytes of half an operand's k-tile
-  static constexpr int NA = A16, NB = 2 * BH;         // DMA instructions of a wave for it
-  static constexpr int RING = 4 * (HA + HB);
+  static constexpr int TM = 32 * A, TN = 128 * BH;
+  static constexpr int A0 = (A + 1) / 2, A1 = A / 2;     // 16-row groups of a wave in either half of the input rows
+  static constexpr int NB = 2 * BH;                      // DMA instructions of a wave for half a k-tile of weights (of input rows: A0, A1)
+  static constexpr int HB = 8192 * BH;                   // its bytes
+  static constexpr int ABYTES = 4096 * A;                // and those of a k-tile of input rows
+  static constexpr int RING = 2 * ABYTES + 4 * HB;
   static constexpr int EPITCH = 64 * BH + 8;             // row pitch of a wave's output piece (plain), in elements
-  static constexpr int EBYTES = 4 * 32 * A16 * EPITCH * 2;
+  static constexpr int EBYTES = 4 * 16 * A * EPITCH * 2;
   static constexpr int LDS = RING > EBYTES ? RING : EBYTES;
+  // tile row at which 16-row group g of the waves `wm` begins
+  static __device__ __forceinline__ int group_row(int g, int wm) { return g < A0 ? wm * 16 * A0 + g * 16 : 32 * A0 + wm * 16 * A1 + (g - A0) * 16; }
 };
+
+// workgroups of a tile that share a CU (LDS and registers: 160 KB, 256 registers per lane)
+constexpr int GEMM_PER_CU(int A, int BH) { return A * BH <= 5 ? 2 : 1; }
 
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
 // One wave instruction: 64 x 16 bytes from memory to LDS at `lds` + 16 * lane.  M0, which holds `lds`, is an operand: the
@@ -232,7 +244,7 @@ __device__ __forceinline__ void gemm_tile_at(int t, int tm, int tn, int& mt, int
 // of weight rows, the others of its second.  Stored from there an instruction would touch 32 bytes in each of 16 rows: they
 // take one trip through LDS (`eb`, a piece of the wave's own) and leave as whole rows.  `row0`: first of the wave's row
 // groups here, m = tile row of group g is row_of(g).
-template <int A16, int BH, int MODE, int R16>
+template <int A, int BH, int MODE, int R16>
 __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u16* eb, int g0, int wm, int wn, int m0, int n0, u16* __restrict__ y,
                                            int64_t ldy, int M, int N, const GemmRope& rp, const int32_t* entry) {
   int lane = threadIdx.x & 63;   // (laundered: the addresses below are not formed before the k loop and kept through it)
@@ -256,10 +268,7 @@ __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u1
   constexpr int LPR = HC / 8, RPI = 64 / LPR;         // lanes per row, rows per instruction
   const int cl = (lane % LPR) * 8;
   const bool vec_ok = (ldy & 7) == 0;
-  auto row_of = [&](int ml) {
-    const int g = g0 + (ml >> 4);
-    return m0 + (g / (A16)) * 32 * A16 + wm * 16 * A16 + (g % (A16)) * 16 + (ml & 15);
-  };
+  auto row_of = [&](int ml) { return m0 + GemmTile<A, BH>::group_row(g0 + (ml >> 4), wm) + (ml & 15); };
   auto store_row = [&](int m, int n, const uint4& v) {
     if (m >= M) return;
     if (entry != nullptr) m = entry[m];
@@ -280,11 +289,12 @@ __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u1
       // (head_dim % 8 == 0).  Positions of several rows first, then their table entries, then the arithmetic: two memory
       // round trips per RB rows (row by row the position and the entry it selects are a chain of two loads per row, and
       // the output pass of a tile took three times as long).
-      constexpr int RB = R16 * 16 / RPI < 8 ? R16 * 16 / RPI : 8;
+      constexpr int RI = R16 * 16 / RPI, RB = RI <= 8 ? RI : RI % 8 == 0 ? 8 : RI / 2;   // (10, 12 and 14 in two halves)
+      static_assert(RI % RB == 0 && RB <= 8, "");
       const int nq = rp.Hq * rp.hd, nkv = rp.Hkv * rp.hd;
       const int sect = n < nq ? 0 : (n < nq + nkv ? 1 : 2), cc = n - (sect == 0 ? 0 : (sect == 1 ? nq : nq + nkv));
       const int hh = cc / rp.hd, dd = cc - hh * rp.hd;
-      for (int i0 = 0; i0 < R16 * 16 / RPI; i0 += RB) {
+      for (int i0 = 0; i0 < RI; i0 += RB) {
         int ps[RB], bb[RB];
 #pragma unroll
         for (int i = 0; i < RB; ++i) {
@@ -325,12 +335,12 @@ __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u1
 
 // KTAIL: K is not a multiple of the 64-element k-tile, so the last one needs a per-lane range check.  NT: weights are loaded
 // non-temporally.
-template <int A16, int BH, bool KTAIL, int MODE, bool GROUP, bool NT>
+template <int A, int BH, bool KTAIL, int MODE, bool GROUP, bool NT>
 __device__ __forceinline__ void gemm_tile(const int block, const int blocks, const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
                                           u16* __restrict__ y, int64_t ldy, int M, int N, int K, int tm, int tn, const GemmRope& rp,
                                           const GemmSplit& sp, const GemmGroup& gp) {
-  using T = GemmTile<A16, BH>;
-  constexpr int HA = T::HA, HB = T::HB, NA = T::NA, NB = T::NB, BOFF = 4 * HA;
+  using T = GemmTile<A, BH>;
+  constexpr int A0 = T::A0, A1 = T::A1, HB = T::HB, NB = T::NB, BOFF = 2 * T::ABYTES;
   extern __shared__ __attribute__((aligned(1024))) u16 gsm[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
@@ -371,12 +381,12 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
   constexpr int OUT = (int)0x80000000;
   const int klen = K - kt0 * 64;
   const int chunk = ((lane & 7) ^ (lane >> 3)) * 8;      // (row % 8 == lane / 8)
-  int xo[2][NA], wo[2][NB];
+  int xo[2][A0], wo[2][NB];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      const int r = h * 32 * A16 + (wave * NA + i) * 8 + (lane >> 3);
+    for (int i = 0; i < (h ? A1 : A0); ++i) {
+      const int r = h * 32 * A0 + (wave * (h ? A1 : A0) + i) * 8 + (lane >> 3);
       const int row = GROUP ? entry[r] / gp.xdiv : r;
       xo[h][i] = m0 + r < M ? (int)((int64_t)row * ldx * 2) + chunk * 2 : OUT;
     }
@@ -401,27 +411,28 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
     if (KTAIL) voff = t * 64 + chunk < klen ? voff : OUT;
     dma16<decltype(ONCE)::value>(r, voff, in ? t * 128 : 0, lds);
   };
-  auto dma_a = [&](int t, int par, int h, int i) { request(std::false_type{}, xb, xbytes, xo[h][i], t, lds0 + (par * 2 + h) * HA + (wave * NA + i) * 1024); };
+  auto dma_a = [&](int t, int par, int h, int i) { request(std::false_type{}, xb, xbytes, xo[h][i], t, lds0 + par * T::ABYTES + h * 4096 * A0 + (wave * (h ? A1 : A0) + i) * 1024); };
   auto dma_b = [&](int t, int par, int h, int i) { request(std::bool_constant<NT>{}, wb, wbytes, wo[h][i], t, lds0 + BOFF + (par * 2 + h) * HB + (wave * NB + i) * 1024); };
 
-  f32x4_t acc[2 * A16][4 * BH];
+  f32x4_t acc[A][4 * BH];
 #pragma unroll
-  for (int a = 0; a < 2 * A16; ++a)
+  for (int a = 0; a < A; ++a)
 #pragma unroll
     for (int b = 0; b < 4 * BH; ++b)
 #pragma unroll
       for (int v = 0; v < 4; ++v) acc[a][b][v] = 0.0f;
-  bf16x8_t af[2][A16][2], bf[2][2 * BH][2];
+  bf16x8_t af[2][A0][2], bf[2][2 * BH][2];
   const char* const smb = reinterpret_cast<const char*>(gsm);
-  int fa[2], fb[2];
+  int fa[2][2], fb[2];
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
     const int c = ((4 * ks + (lane >> 4)) ^ (lane & 7)) * 16;
-    fa[ks] = (wm * 16 * A16 + (lane & 15)) * 128 + c;
+    fa[0][ks] = (wm * 16 * A0 + (lane & 15)) * 128 + c;
+    fa[1][ks] = (wm * 16 * A1 + (lane & 15)) * 128 + c;
     fb[ks] = (wn * 32 * BH + (lane & 15)) * 128 + c + BOFF;
   }
   auto read_a = [&](int par, int h, int t, int ks) {
-    af[h][t][ks] = *reinterpret_cast<const bf16x8_t*>(smb + fa[ks] + (par * 2 + h) * HA + t * 2048);
+    af[h][t][ks] = *reinterpret_cast<const bf16x8_t*>(smb + fa[h][ks] + par * T::ABYTES + h * 4096 * A0 + t * 2048);
   };
   auto read_b = [&](int set, int par, int h, int t, int ks) {
     bf[set][t][ks] = *reinterpret_cast<const bf16x8_t*>(smb + fb[ks] + (par * 2 + h) * HB + t * 2048);
@@ -434,27 +445,27 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
 #pragma unroll
-    for (int i = 0; i < NA; ++i) dma_a(t, t, 0, i);
+    for (int i = 0; i < A0; ++i) dma_a(t, t, 0, i);
 #pragma unroll
     for (int i = 0; i < NB; ++i) dma_b(t, t, 0, i);
 #pragma unroll
     for (int i = 0; i < NB; ++i) dma_b(t, t, 1, i);
 #pragma unroll
-    for (int i = 0; i < NA; ++i) dma_a(t, t, 1, i);
+    for (int i = 0; i < A1; ++i) dma_a(t, t, 1, i);
   }
-  wait_requests_and_lds<3 * NA + 3 * NB>();
+  wait_requests_and_lds<A0 + 2 * A1 + 3 * NB>();
   barrier();
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-    for (int t = 0; t < A16; ++t) read_a(0, 0, t, ks);
+    for (int t = 0; t < A0; ++t) read_a(0, 0, t, ks);
 #pragma unroll
     for (int t = 0; t < 2 * BH; ++t) read_b(0, 0, 0, t, ks);
   }
-  wait_requests_and_lds<3 * NA + 3 * NB>();
+  wait_requests_and_lds<A0 + 2 * A1 + 3 * NB>();
   barrier();
 #pragma unroll
-  for (int i = 0; i < NA; ++i) dma_a(2, 0, 0, i);
+  for (int i = 0; i < A0; ++i) dma_a(2, 0, 0, i);
 
   // Phase P of k-tile t (even: PAR 0).  Reads B1 of this tile, A1 of this tile, A0 of the next, B0 of the next; requests
   // B0, B1, A1 of tile t + 2 and A0 of tile t + 3.
@@ -462,21 +473,21 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
     constexpr int PAR = decltype(PAR_)::value, P = decltype(P_)::value;
     constexpr int ah = P >> 1, bh = (P == 1 || P == 2), set = bh ^ PAR;
     // requests younger than the slot read here: those of the six phases since
-    wait_requests_and_lds<(P == 0 ? 4 * NA + 2 * NB : P == 2 ? 2 * NA + 4 * NB : 3 * NA + 3 * NB)>();
+    wait_requests_and_lds<(P == 0 ? 2 * A + 2 * NB : P == 1 ? A + A0 + 3 * NB : P == 2 ? A + 4 * NB : A + A1 + 3 * NB)>();
     barrier();
-    constexpr int J = 4 * A16 * BH, RD = (P == 1 || P == 2) ? 2 * A16 : 4 * BH, RQ = (P == 2 || P == 3) ? NA : NB;
+    constexpr int AH = ah ? A1 : A0, J = 4 * AH * BH, RD = P == 1 ? 2 * A1 : P == 2 ? 2 * A0 : 4 * BH, RQ = P == 2 ? A1 : P == 3 ? A0 : NB;
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-      const int tb = j % (2 * BH), ta = j / (2 * BH) % (A16), ks = j / (2 * A16 * BH);
+      const int tb = j % (2 * BH), ta = j / (2 * BH) % AH, ks = j / (2 * AH * BH);
       asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
-                   : "+a"(acc[ah * A16 + ta][bh * 2 * BH + tb])
+                   : "+a"(acc[ah * A0 + ta][bh * 2 * BH + tb])
                    : "v"(bf[set][tb][ks]), "v"(af[ah][ta][ks]));
       if (j < J / 2) {
 #pragma unroll
         for (int e = j * RD / (J / 2); e < (j + 1) * RD / (J / 2); ++e) {
           if (P == 0) read_b(1 ^ PAR, PAR, 1, e % (2 * BH), e / (2 * BH));
-          if (P == 1) read_a(PAR, 1, e % (A16), e / (A16));
-          if (P == 2) read_a(PAR ^ 1, 0, e % (A16), e / (A16));
+          if (P == 1) read_a(PAR, 1, e % A1, e / A1);
+          if (P == 2) read_a(PAR ^ 1, 0, e % A0, e / A0);
           if (P == 3) read_b(1 ^ PAR, PAR ^ 1, 0, e % (2 * BH), e / (2 * BH));
         }
       } else {
@@ -514,8 +525,8 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
     if constexpr (MODE == GEMM_ROWS) {
       float* const p = sp.part + (int64_t)(piece % sp.splits) * M * N;
 #pragma unroll
-      for (int a = 0; a < 2 * A16; ++a) {
-        const int m = m0 + a / A16 * 32 * A16 + wm * 16 * A16 + a % A16 * 16 + (lane & 15);
+      for (int a = 0; a < A; ++a) {
+        const int m = m0 + T::group_row(a, wm) + (lane & 15);
 #pragma unroll
         for (int b = 0; b < 4 * BH; ++b) {
           const int n = n0 + b / (2 * BH) * 64 * BH + wn * 32 * BH + b % (2 * BH) * 16 + (lane >> 4) * 4;
@@ -525,9 +536,9 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
       }
       return;
     } else if (piece >= 0) {
-      float* p = sp.part + (int64_t)piece * (T::TM * T::TN) + (int64_t)wave * (8 * A16 * BH * 256) + lane * 4;
+      float* p = sp.part + (int64_t)piece * (T::TM * T::TN) + (int64_t)wave * (4 * A * BH * 256) + lane * 4;
 #pragma unroll
-      for (int a = 0; a < 2 * A16; ++a) {
+      for (int a = 0; a < A; ++a) {
 #pragma unroll
         for (int b = 0; b < 4 * BH; ++b) *reinterpret_cast<f32x4_t*>(p + (a * 4 * BH + b) * 256) = acc[a][b];
         __builtin_amdgcn_sched_barrier(0);
@@ -535,14 +546,14 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
       return;
     }
   }
-  if constexpr (MODE != GEMM_ROWS) gemm_store<A16, BH, MODE, 2 * A16>(acc, gsm + wave * (T::EBYTES / 8), 0, wm, wn, m0, n0, y, ldy, M, N, rp, GROUP ? entry : nullptr);
+  if constexpr (MODE != GEMM_ROWS) gemm_store<A, BH, MODE, A>(acc, gsm + wave * (T::EBYTES / 8), 0, wm, wn, m0, n0, y, ldy, M, N, rp, GROUP ? entry : nullptr);
 }
 
-template <int A16, int BH, bool KTAIL, int MODE, bool GROUP, bool NT = false>
-__global__ __launch_bounds__(256, A16 * BH <= 2 ? 2 : 1) void k_gemm_dma(const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
+template <int A, int BH, bool KTAIL, int MODE, bool GROUP, bool NT = false>
+__global__ __launch_bounds__(256, GEMM_PER_CU(A, BH)) void k_gemm_dma(const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
                                                                         u16* __restrict__ y, int64_t ldy, int M, int N, int K, int tm, int tn,
                                                                         const GemmRope rp, const GemmSplit sp, const GemmGroup gp) {
-  gemm_tile<A16, BH, KTAIL, MODE, GROUP, NT>(blockIdx.x, gridDim.x, x, ldx, w, y, ldy, M, N, K, tm, tn, rp, sp, gp);
+  gemm_tile<A, BH, KTAIL, MODE, GROUP, NT>(blockIdx.x, gridDim.x, x, ldx, w, y, ldy, M, N, K, tm, tn, rp, sp, gp);
 }
 
 // Two products of as many rows in one grid, the first `n0` workgroups the first's.  A short prompt's products each leave most
@@ -557,33 +568,33 @@ struct GemmProduct {
   int M, N, K, tm, tn;
   GemmSplit sp;
 };
-template <int A16, int BH, int MODE0, int MODE1, bool NT>
-__global__ __launch_bounds__(256, A16 * BH <= 2 ? 2 : 1) void k_gemm_two(const GemmProduct a, const GemmProduct b, const int n0, const GemmRope rp) {
+template <int A, int BH, int MODE0, int MODE1, bool NT>
+__global__ __launch_bounds__(256, GEMM_PER_CU(A, BH)) void k_gemm_two(const GemmProduct a, const GemmProduct b, const int n0, const GemmRope rp) {
   const bool second = (int)blockIdx.x >= n0;
   if constexpr (MODE0 == MODE1) {
     const GemmProduct p = second ? b : a;
-    gemm_tile<A16, BH, false, MODE0, false, NT>(blockIdx.x - (second ? n0 : 0), 0, p.x, p.ldx, p.w, p.y, p.ldy, p.M, p.N, p.K, p.tm, p.tn, rp, p.sp, GemmGroup{});
+    gemm_tile<A, BH, false, MODE0, false, NT>(blockIdx.x - (second ? n0 : 0), 0, p.x, p.ldx, p.w, p.y, p.ldy, p.M, p.N, p.K, p.tm, p.tn, rp, p.sp, GemmGroup{});
   } else if (second) {
-    gemm_tile<A16, BH, false, MODE1, false, NT>(blockIdx.x - n0, 0, b.x, b.ldx, b.w, b.y, b.ldy, b.M, b.N, b.K, b.tm, b.tn, GemmRope{}, b.sp, GemmGroup{});
+    gemm_tile<A, BH, false, MODE1, false, NT>(blockIdx.x - n0, 0, b.x, b.ldx, b.w, b.y, b.ldy, b.M, b.N, b.K, b.tm, b.tn, GemmRope{}, b.sp, GemmGroup{});
   } else {
-    gemm_tile<A16, BH, false, MODE0, false, NT>(blockIdx.x, 0, a.x, a.ldx, a.w, a.y, a.ldy, a.M, a.N, a.K, a.tm, a.tn, rp, a.sp, GemmGroup{});
+    gemm_tile<A, BH, false, MODE0, false, NT>(blockIdx.x, 0, a.x, a.ldx, a.w, a.y, a.ldy, a.M, a.N, a.K, a.tm, a.tn, rp, a.sp, GemmGroup{});
   }
 }
 
-// The cut tiles: a workgroup adds the pieces of a 1 / (2 A16) part of one (16 rows per wave, four pieces' loads in flight
+// The cut tiles: a workgroup adds the pieces of a 1 / A part of one (16 rows per wave, four pieces' loads in flight
 // together, summed in order) and finishes it.  Bound: memory, mostly the last-level cache: the pieces were just written.
-template <int A16, int BH, int MODE>
+template <int A, int BH, int MODE>
 __global__ __launch_bounds__(256) void k_gemm_sum(u16* __restrict__ y, int64_t ldy, int M, int N, int tm, int tn, const GemmRope rp, const GemmSplit sp) {
-  using T = GemmTile<A16, BH>;
+  using T = GemmTile<A, BH>;
   __shared__ __attribute__((aligned(16))) u16 sm[4 * 16 * T::EPITCH];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int rt = blockIdx.x / (2 * A16), g0 = blockIdx.x - rt * 2 * A16;
+  const int rt = blockIdx.x / A, g0 = blockIdx.x - rt * A;
   int mt, nt;
   gemm_tile_at(sp.full + rt, tm, tn, mt, nt);
   const int m0 = mt * T::TM, n0 = nt * (MODE == GEMM_PAIR ? T::TN / 2 : T::TN);
-  if (m0 + (g0 / (A16)) * 32 * A16 + (g0 % (A16)) * 16 >= M) return;   // (its lowest row; no barrier follows)
+  if (m0 + T::group_row(g0, 0) >= M) return;   // (its lowest row; no barrier follows)
   constexpr int C = 4 * BH, STEP = T::TM * T::TN;
-  const float* p = sp.part + (int64_t)rt * sp.splits * STEP + ((int64_t)wave * 2 * A16 + g0) * (C * 256) + lane * 4;
+  const float* p = sp.part + (int64_t)rt * sp.splits * STEP + ((int64_t)wave * A + g0) * (C * 256) + lane * 4;
   f32x4_t acc[1][C], v[4][C];
 #pragma unroll
   for (int b = 0; b < C; ++b) acc[0][b] = *reinterpret_cast<const f32x4_t*>(p + b * 256);
@@ -600,7 +611,7 @@ __global__ __launch_bounds__(256) void k_gemm_sum(u16* __restrict__ y, int64_t l
         for (int b = 0; b < C; ++b) acc[0][b] += v[i][b];
       }
   }
-  gemm_store<A16, BH, MODE, 1>(acc, sm + wave * (16 * T::EPITCH), g0, wave >> 1, wave & 1, m0, n0, y, ldy, M, N, rp, nullptr);
+  gemm_store<A, BH, MODE, 1>(acc, sm + wave * (16 * T::EPITCH), g0, wave >> 1, wave & 1, m0, n0, y, ldy, M, N, rp, nullptr);
 }
 
 // ---- which tile, and which tiles are cut along K
@@ -623,16 +634,29 @@ struct GemmPlan {
 //   128 rows,  3072 x  2048  17.2 / 13.3 / 13.3 | 13.0         900 rows,  2048 x    16   4.2 /  5.1 /  4.2 |  4.2
 //   128 rows,  4096 x 14336  38.3 / 32.8 / 32.8 | 32.8        1501 rows,  7168 x  8192 153.9 / 168.2 / 153.9 | 153.9 (pairs)
 //   128 rows, 28672 x  4096  65.8 / 54.8 / 54.8 | 54.8 (pairs)  2100 rows, 4608 x 4096  79.2 / 82.3 / 79.2 | 77.2
-// and where it loses most: 129 rows, 16032 x 8192 65.9 / 78.8 / 77.1 | 65.9; 5000 rows, 2048 x 5120 95.5 / 95.5 / 109.6 | 95.5; 192 rows,
+// Tiles of 160, 192 and 224 rows came later; their costs are fitted to 1457 products of 131 to 4096 rows of 31 weights, with 64 MiB for pieces
+// and none, the first four tiles' as they were.  The products took 5.3 % less on average, 11 of 2914 choices more than 3 % more (257 rows,
+// 2048 x 8192 21.6 -> 24.4), and the plan is 0.9 % above the best choice.  us, with four tiles / now:
+//   300 rows, 28672 x 4096 100.3 / 74.0 (pairs)   450 rows,  7168 x 8192  69.4 / 58.7 (pairs)   777 rows, 28672 x 4096 197.2 / 176.9 (pairs)
+//   777 rows,  6144 x 4096  55.7 / 44.1           777 rows,  4096 x 14336 94.7 / 89.4          1501 rows,  7168 x 8192 162.5 / 138.4 (pairs)
+//  1100 rows,  4096 x 4096  52.1 / 41.0          9205 rows,  2048 x 8192 278.1 / 227.4 (no memory)
+// Up to 128 rows they would hold rows that are not there, and K of no whole k-tiles is left to the first four: neither is looked at.
+// Where the first four lose most: 129 rows, 16032 x 8192 65.9 / 78.8 / 77.1 | 65.9; 5000 rows, 2048 x 5120 95.5 / 95.5 / 109.6 | 95.5; 192 rows,
 // 3072 x 2048 17.1 in all three | 14.0; 1100 rows, 8192 x 512 19.9 in all three | 16.4.
 struct GemmTileCost {
-  int a16, bh, per_cu;
+  int a, bh, per_cu;
   float ktile, slope, cold, pair, pair_cold, fixed, store;
 };
-constexpr GemmTileCost GEMM_TILES[4] = {{4, 2, 1, 1.2f, 0.0f, 0.0f, 0.0f, 0.0f, 4.35f, 4.43f},
-                                         {2, 2, 1, 0.684f, 0.108f, 0.552f, 0.0f, 0.0f, 2.85f, 1.47f},
-                                         {2, 1, 2, 0.504f, 0.0f, 0.262f, 0.874f, 1.25f, 3.18f, 0.166f},
-                                         {1, 1, 2, 0.302f, 0.201f, 0.284f, 0.737f, 1.19f, 3.24f, 0.0f}};
+constexpr int GEMM_NTILES = 9, GEMM_TILES_ANY = 4;   // the first four take any K and any number of rows, see gemm_plan
+constexpr GemmTileCost GEMM_TILES[GEMM_NTILES] = {{8, 2, 1, 1.2f, 0.0f, 0.0f, 0.0f, 0.0f, 4.35f, 4.43f},
+                                                  {4, 2, 1, 0.684f, 0.108f, 0.552f, 0.0f, 0.0f, 2.85f, 1.47f},
+                                                  {4, 1, 2, 0.504f, 0.0f, 0.262f, 0.874f, 1.25f, 3.18f, 0.166f},
+                                                  {2, 1, 2, 0.302f, 0.201f, 0.284f, 0.737f, 1.19f, 3.24f, 0.0f},
+                                                  {7, 2, 1, 1.098f, 0.0394f, 0.0f, 0.0f, 0.0f, 6.28f, 2.11f},
+                                                  {6, 2, 1, 0.953f, 0.0412f, 0.119f, 0.0f, 0.0f, 6.24f, 1.61f},
+                                                  {5, 2, 1, 0.668f, 0.2935f, 0.581f, 0.0f, 0.0f, 3.12f, 5.41f},
+                                                  {5, 1, 2, 0.553f, 0.0159f, 0.173f, 1.103f, 4.77f, 3.88f, 0.0077f},
+                                                  {6, 1, 1, 0.617f, 0.0f, 0.0944f, 0.0f, 0.0f, 4.28f, 0.0f}};
 constexpr size_t GEMM_SCRATCH = (size_t)64 << 20;   // pieces of one round of the largest tiles
 constexpr int GEMM_SCRATCH_FROM = 33;               // rows from which a projection that has memory for pieces is one of this file's
 
@@ -642,7 +666,7 @@ constexpr float GEMM_WEIGHT_BYTES_US = 5.73e6f, GEMM_OUTPUT_BYTES_US = 6.98e6f, 
 // `workgroups` of k k-tiles each, at the same time
 static float gemm_round_us(const GemmTileCost& t, int M, int cus, int workgroups, int k) {
   const float busy = (float)workgroups / cus;
-  const int TM = 64 * t.a16;
+  const int TM = 32 * t.a;
   const float own = M <= TM ? 1.0f : M <= 2 * TM ? GEMM_TWO : 0.0f;   // how much a weight is one row tile's own
   return k * (busy > 1.0f ? t.pair + (t.pair_cold - t.pair) * own : t.ktile + busy * (t.slope + (t.cold - t.slope) * own));
 }
@@ -665,9 +689,9 @@ static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
   if (M > 0x7fffffff - 256 || N > 0x7fffffff - 256 || K > 0x7fffffff - 256) return best;   // (row, column and k of the last tile are ints)
   const int cus = gemm_cus(), nk = (K + 63) / 64;
   const float bytes_us = gemm_bytes_us(M, N, K, mode);
-  for (int c = 0; c < 4; ++c) {
+  for (int c = 0; c < (M > 128 && K % 64 == 0 ? GEMM_NTILES : GEMM_TILES_ANY); ++c) {
     const GemmTileCost& t = GEMM_TILES[c];
-    const int TM = 64 * t.a16, TN = (mode == GEMM_PAIR ? 64 : 128) * t.bh, slots = cus * t.per_cu;
+    const int TM = 32 * t.a, TN = (mode == GEMM_PAIR ? 64 : 128) * t.bh, slots = cus * t.per_cu;
     const int64_t tiles = (int64_t)((M + TM - 1) / TM) * ((N + TN - 1) / TN), rounds = tiles / slots;
     if (tiles > 0x3fffffff) continue;
     const int left = (int)(tiles - rounds * slots);
@@ -679,7 +703,7 @@ static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
     const float whole = rounds * round_us(slots, nk), fixed = (rounds + (left ? 1 : 0)) * t.fixed;
     consider(whole + (left ? round_us(left, nk) : 0.0f), fixed, (int)tiles, 0, 1);
     for (int s = 2; left && s <= 16 && 4 * s <= nk && left * s <= slots; ++s) {
-      const size_t bytes = (size_t)left * s * (64 * t.a16) * (128 * t.bh) * sizeof(float);
+      const size_t bytes = (size_t)left * s * (32 * t.a) * (128 * t.bh) * sizeof(float);
       if (bytes > scratch) break;
       consider(whole + round_us(left * s, (nk + s - 1) / s), fixed + GEMM_SUM_US + gemm_trips(s) * GEMM_TRIP_US + bytes / GEMM_PIECE_BYTES_US,
                (int)tiles - left, left, s);
@@ -688,45 +712,50 @@ static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
   return best;
 }
 
-template <int A16, int BH, bool KTAIL, int MODE, bool NT = false>
+template <int A, int BH, bool KTAIL, int MODE, bool NT = false>
 static int gemm_run_as(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, const GemmRope& rp,
                        const GemmPlan& p, void* scratch, hipStream_t s) {
-  using T = GemmTile<A16, BH>;
+  using T = GemmTile<A, BH>;
   static std::atomic<unsigned long long> raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_dma<A16, BH, KTAIL, MODE, false, NT>), T::LDS, raised)) return LR_E_LAUNCH;
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_dma<A, BH, KTAIL, MODE, false, NT>), T::LDS, raised)) return LR_E_LAUNCH;
   const int gn = MODE == GEMM_PAIR ? T::TN / 2 : T::TN, tm = (M + T::TM - 1) / T::TM, tn = (N + gn - 1) / gn;
   const GemmSplit sp{(float*)scratch, p.full, p.rem, p.splits};
-  k_gemm_dma<A16, BH, KTAIL, MODE, false, NT><<<dim3((unsigned)(p.full + p.rem * p.splits)), dim3(256), T::LDS, s>>>(
+  k_gemm_dma<A, BH, KTAIL, MODE, false, NT><<<dim3((unsigned)(p.full + p.rem * p.splits)), dim3(256), T::LDS, s>>>(
       (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, M, N, K, tm, tn, rp, sp, GemmGroup{});
   if constexpr (MODE != GEMM_ROWS)
-    if (p.rem) k_gemm_sum<A16, BH, MODE><<<dim3((unsigned)(p.rem * 2 * A16)), dim3(256), 0, s>>>((u16*)y, ldy, M, N, tm, tn, rp, sp);
+    if (p.rem) k_gemm_sum<A, BH, MODE><<<dim3((unsigned)(p.rem * A)), dim3(256), 0, s>>>((u16*)y, ldy, M, N, tm, tn, rp, sp);
   return lr_launch_status();
 }
-template <int A16, int BH, bool KTAIL, bool NT = false>
+template <int A, int BH, bool KTAIL, bool NT = false>
 static int gemm_run_mode(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, int mode, const GemmRope& rp,
                          const GemmPlan& p, void* scratch, hipStream_t s) {
-  if (mode == GEMM_PAIR) return gemm_run_as<A16, BH, KTAIL, GEMM_PAIR, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
-  if (mode == GEMM_ROPE) return gemm_run_as<A16, BH, KTAIL, GEMM_ROPE, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
-  if (mode == GEMM_ROWS) return gemm_run_as<A16, BH, KTAIL, GEMM_ROWS, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
-  return gemm_run_as<A16, BH, KTAIL, GEMM_PLAIN, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+  if (mode == GEMM_PAIR) return gemm_run_as<A, BH, KTAIL, GEMM_PAIR, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+  if (mode == GEMM_ROPE) return gemm_run_as<A, BH, KTAIL, GEMM_ROPE, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+  if (mode == GEMM_ROWS) return gemm_run_as<A, BH, KTAIL, GEMM_ROWS, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+  return gemm_run_as<A, BH, KTAIL, GEMM_PLAIN, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
 }
 static int gemm_run(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, int mode, const GemmRope& rp,
                     const GemmPlan& p, void* scratch, hipStream_t s) {
   const bool kt = K % 64 != 0;
   if (p.tile == 0)
+    return kt ? gemm_run_mode<8, 2, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
+              : gemm_run_mode<8, 2, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+  if (p.tile == 1)
     return kt ? gemm_run_mode<4, 2, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
               : gemm_run_mode<4, 2, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
-  if (p.tile == 1)
-    return kt ? gemm_run_mode<2, 2, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
-              : gemm_run_mode<2, 2, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
   if (p.tile == 2)
-    return kt ? gemm_run_mode<2, 1, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
-              : gemm_run_mode<2, 1, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+    return kt ? gemm_run_mode<4, 1, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
+              : gemm_run_mode<4, 1, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+  if (p.tile == 4) return gemm_run_mode<7, 2, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+  if (p.tile == 5) return gemm_run_mode<6, 2, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+  if (p.tile == 6) return gemm_run_mode<5, 2, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+  if (p.tile == 7) return gemm_run_mode<5, 1, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+  if (p.tile == 8) return gemm_run_mode<6, 1, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
   if (M <= 64)   // every weight is used once: non-temporal (28672 x 4096 at 64 rows 50.0 -> 46.7 us, 16032 x 8192 61.9 -> 57.5)
-    return kt ? gemm_run_mode<1, 1, true, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
-              : gemm_run_mode<1, 1, false, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
-  return kt ? gemm_run_mode<1, 1, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
-            : gemm_run_mode<1, 1, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+    return kt ? gemm_run_mode<2, 1, true, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
+              : gemm_run_mode<2, 1, false, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+  return kt ? gemm_run_mode<2, 1, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
+            : gemm_run_mode<2, 1, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
 }
 // whether a tile's rows lie within the 2 GiB that an offset of a request reaches (N: pairs in PAIR mode)
 static bool gemm_reaches(int64_t ldx, int N, int K, int mode) {
@@ -743,27 +772,27 @@ static int gemm(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy,
 // ---- two products of one grid, and products whose partial sums stay
 static GemmProduct gemm_product(int tile, int mode, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K) {
   const GemmTileCost& t = GEMM_TILES[tile];
-  const int TM = 64 * t.a16, TN = (mode == GEMM_PAIR ? 64 : 128) * t.bh;
+  const int TM = 32 * t.a, TN = (mode == GEMM_PAIR ? 64 : 128) * t.bh;
   GemmProduct p = {(const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, M, N, K, (M + TM - 1) / TM, (N + TN - 1) / TN, GemmSplit{}};
   p.sp.full = p.tm * p.tn;
   p.sp.splits = 1;
   return p;
 }
-template <int A16, int BH, int MODE0, int MODE1, bool NT>
+template <int A, int BH, int MODE0, int MODE1, bool NT>
 static int gemm_two_as(const GemmProduct& a, const GemmProduct& b, const GemmRope& rp, hipStream_t s) {
-  using T = GemmTile<A16, BH>;
+  using T = GemmTile<A, BH>;
   static std::atomic<unsigned long long> raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_two<A16, BH, MODE0, MODE1, NT>), T::LDS, raised)) return LR_E_LAUNCH;
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_two<A, BH, MODE0, MODE1, NT>), T::LDS, raised)) return LR_E_LAUNCH;
   const int n0 = a.sp.full + a.sp.rem * a.sp.splits, n1 = b.sp.full + b.sp.rem * b.sp.splits;
-  k_gemm_two<A16, BH, MODE0, MODE1, NT><<<dim3((unsigned)(n0 + n1)), dim3(256), T::LDS, s>>>(a, b, n0, rp);
+  k_gemm_two<A, BH, MODE0, MODE1, NT><<<dim3((unsigned)(n0 + n1)), dim3(256), T::LDS, s>>>(a, b, n0, rp);
   return lr_launch_status();
 }
 template <int MODE0, int MODE1>
 static int gemm_two(int tile, const GemmProduct& a, const GemmProduct& b, const GemmRope& rp, hipStream_t s) {
-  if (tile == 0) return gemm_two_as<4, 2, MODE0, MODE1, false>(a, b, rp, s);
-  if (tile == 1) return gemm_two_as<2, 2, MODE0, MODE1, false>(a, b, rp, s);
-  if (tile == 2) return gemm_two_as<2, 1, MODE0, MODE1, false>(a, b, rp, s);
-  return a.M <= 64 ? gemm_two_as<1, 1, MODE0, MODE1, true>(a, b, rp, s) : gemm_two_as<1, 1, MODE0, MODE1, false>(a, b, rp, s);
+  if (tile == 0) return gemm_two_as<8, 2, MODE0, MODE1, false>(a, b, rp, s);
+  if (tile == 1) return gemm_two_as<4, 2, MODE0, MODE1, false>(a, b, rp, s);
+  if (tile == 2) return gemm_two_as<4, 1, MODE0, MODE1, false>(a, b, rp, s);
+  return a.M <= 64 ? gemm_two_as<2, 1, MODE0, MODE1, true>(a, b, rp, s) : gemm_two_as<2, 1, MODE0, MODE1, false>(a, b, rp, s);
 }
 
 namespace lr_detail {
@@ -778,9 +807,9 @@ int gemm_inputs(const void* x0, const void* wqkv, void* qkv, int S, const lr_rop
   const float bytes_us = gemm_bytes_us(M, N, K, GEMM_ROPE) + gemm_bytes_us(M, I, K, GEMM_PAIR);
   float best_us = p0.us + p1.us;
   int best = -1;
-  for (int c = 0; c < 4; ++c) {
+  for (int c = 0; c < GEMM_TILES_ANY; ++c) {
     const GemmTileCost& t = GEMM_TILES[c];
-    const int TM = 64 * t.a16, slots = cus * t.per_cu;
+    const int TM = 32 * t.a, slots = cus * t.per_cu;
     const int64_t tm = (M - 1) / TM + 1, tiles0 = tm * ((N - 1) / (128 * t.bh) + 1), tiles1 = tm * ((I - 1) / (64 * t.bh) + 1), tiles = tiles0 + tiles1;
     // (of several rounds only the last one leaves room, and q/k/v goes cold before the attention reads it: 8 x 2048 tokens of
     // the 8B model, in one grid 185.4 ms, apart 183.2)
@@ -824,9 +853,9 @@ static GemmOutputs outputs_plan(int M, int N, int K0, int K1, size_t sums_bytes)
   float best_us = alone(p0) + alone(p1);
   const int cus = gemm_cus(), pairs0 = (K0 / 64 + 1) / 2, pairs1 = (K1 / 64 + 1) / 2;
   const size_t row = (size_t)M * N * sizeof(float);
-  for (int c = 0; c < 4; ++c) {
+  for (int c = 0; c < GEMM_TILES_ANY; ++c) {
     const GemmTileCost& t = GEMM_TILES[c];
-    const int TM = 64 * t.a16, TN = 128 * t.bh, slots = cus * t.per_cu;
+    const int TM = 32 * t.a, TN = 128 * t.bh, slots = cus * t.per_cu;
     const int64_t tiles = (int64_t)((M + TM - 1) / TM) * ((N + TN - 1) / TN);
     for (int s0 = 1; s0 <= 16 && 2 * s0 <= pairs0 + 1 && row * s0 <= sums_bytes; ++s0)
       for (int s1 = 1; s1 <= 16 && 2 * s1 <= pairs1 + 1 && row * s1 <= sums_bytes && tiles * (s0 + s1) <= slots; ++s1) {
@@ -859,15 +888,15 @@ int gemm_outputs(const void* x0, const void* w0, int K0, void* sums0, int* piece
 // Grouped products (lr_moe): rows of several matrices' tiles, see GemmGroup; pair_off != 0: GEMM_PAIR (N counts pairs).
 // tile_rows: 128 or 256, the height the tile table was made for.
 namespace lr_detail {
-template <int A16, int BH, bool KTAIL, int MODE>
+template <int A, int BH, bool KTAIL, int MODE>
 static int gemm_grouped_as(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int N, int K, const GemmGroup& gp, int max_tiles,
                            hipStream_t s) {
-  using T = GemmTile<A16, BH>;
+  using T = GemmTile<A, BH>;
   constexpr size_t lds = T::LDS + T::TM * sizeof(int32_t);
   static std::atomic<unsigned long long> raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_dma<A16, BH, KTAIL, MODE, true>), lds, raised)) return LR_E_LAUNCH;
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_dma<A, BH, KTAIL, MODE, true>), lds, raised)) return LR_E_LAUNCH;
   const int gn = MODE == GEMM_PAIR ? T::TN / 2 : T::TN, tn = (N + gn - 1) / gn;
-  k_gemm_dma<A16, BH, KTAIL, MODE, true><<<dim3((unsigned)(max_tiles * tn)), dim3(256), lds, s>>>(
+  k_gemm_dma<A, BH, KTAIL, MODE, true><<<dim3((unsigned)(max_tiles * tn)), dim3(256), lds, s>>>(
       (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, T::TM, N, K, max_tiles, tn, GemmRope{}, GemmSplit{}, gp);
   return lr_launch_status();
 }
@@ -878,16 +907,16 @@ int gemm_grouped(const void* x, int64_t ldx, int64_t xrows, const void* w, void*
   const bool kt = K % 64 != 0;
   if (tile_rows == 128) {
     if (pair_off)
-      return kt ? gemm_grouped_as<2, 1, true, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
-                : gemm_grouped_as<2, 1, false, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
-    return kt ? gemm_grouped_as<2, 1, true, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
-              : gemm_grouped_as<2, 1, false, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
+      return kt ? gemm_grouped_as<4, 1, true, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
+                : gemm_grouped_as<4, 1, false, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
+    return kt ? gemm_grouped_as<4, 1, true, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
+              : gemm_grouped_as<4, 1, false, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
   }
   if (pair_off)
-    return kt ? gemm_grouped_as<4, 2, true, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
-              : gemm_grouped_as<4, 2, false, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
-  return kt ? gemm_grouped_as<4, 2, true, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
-            : gemm_grouped_as<4, 2, false, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
+    return kt ? gemm_grouped_as<8, 2, true, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
+              : gemm_grouped_as<8, 2, false, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
+  return kt ? gemm_grouped_as<8, 2, true, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
+            : gemm_grouped_as<8, 2, false, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
 }
 }  // namespace lr_detail
 
@@ -939,7 +968,7 @@ extern "C" int lr_linear_plan(int M, int N, int K, int pair, size_t scratch_byte
   if (K % 8) return LR_E_ALIGN;
   const GemmPlan p = gemm_plan(M, pair ? N / 2 : N, K, pair ? GEMM_PAIR : GEMM_PLAIN, scratch_bytes);
   if (p.tile < 0) return LR_E_UNSUPPORTED;
-  plan->tile_rows = 64 * GEMM_TILES[p.tile].a16;
+  plan->tile_rows = 32 * GEMM_TILES[p.tile].a;
   plan->tile_cols = 128 * GEMM_TILES[p.tile].bh;
   plan->whole = p.full;
   plan->cut = p.rem;

@@ -1090,6 +1090,37 @@ def test_linear_rope_kv_of_every_tile_whole_and_cut(hip, tile, kind, B, S, Hq, H
     check_rope_kv(hip, B, S, Hq, Hkv, hd, K, hip.linear_scratch_bytes(M) if with_sums else 0)
 
 
+# the tiles between (above 128 rows, whole k-tiles): halves of the rows that differ by a 16-row group per wave, last tiles of a few rows
+@pytest.mark.parametrize("tile,kind,M,N,K", [
+    ((160, 128), "whole", 650, 11017, 64), ((160, 128), "cut", 129, 3023, 2560), ((160, 256), "whole", 902, 8349, 1088),
+    ((160, 256), "cut", 131, 10909, 3328), ((192, 128), "whole", 513, 8514, 256), ((192, 128), "cut", 164, 2809, 5184),
+    ((192, 256), "whole", 1123, 8527, 192), ((192, 256), "cut", 169, 11013, 5056), ((192, 256), "mixed", 5166, 4666, 3968),
+    ((224, 256), "whole", 1025, 10942, 192), ((224, 256), "cut", 193, 11270, 4928), ((224, 256), "mixed", 1293, 11992, 2176),
+])
+def test_linear_of_the_tiles_between(hip, tile, kind, M, N, K):
+    test_linear_of_every_tile_whole_and_cut(hip, tile, kind, M, N, K)
+
+
+@pytest.mark.parametrize("tile,kind,M,I,K", [
+    ((160, 128), "whole", 652, 5480, 64), ((160, 128), "cut", 130, 1440, 2560), ((160, 256), "whole", 791, 4680, 384),
+    ((160, 256), "cut", 259, 2696, 3456), ((192, 128), "whole", 514, 4904, 384), ((192, 128), "cut", 168, 1392, 5184),
+    ((192, 256), "whole", 802, 5760, 320), ((192, 256), "cut", 170, 5464, 5760), ((224, 256), "whole", 1031, 5416, 896),
+    ((224, 256), "cut", 193, 5488, 5056), ((224, 256), "mixed", 1314, 5960, 2368),
+])
+def test_linear_swiglu_out_of_the_tiles_between(hip, tile, kind, M, I, K):
+    test_linear_swiglu_out_of_every_tile_whole_and_cut(hip, tile, kind, M, I, K)
+
+
+@pytest.mark.parametrize("tile,kind,B,S,Hq,Hkv,hd,K", [
+    ((160, 128), "whole", 2, 651, 357, 7, 16, 64), ((160, 128), "cut", 3, 45, 368, 2, 8, 2816), ((160, 256), "whole", 4, 388, 308, 4, 16, 1088),
+    ((160, 256), "cut", 2, 134, 85, 1, 64, 3328), ((192, 128), "whole", 2, 322, 96, 6, 64, 256), ((192, 128), "cut", 3, 54, 520, 8, 8, 3584),
+    ((192, 256), "whole", 3, 540, 732, 6, 8, 192), ((192, 256), "cut", 2, 282, 91, 7, 64, 5760), ((224, 256), "whole", 4, 645, 579, 1, 8, 256),
+    ((224, 256), "cut", 2, 328, 54, 6, 64, 5696),
+])
+def test_linear_rope_kv_of_the_tiles_between(hip, tile, kind, B, S, Hq, Hkv, hd, K):
+    test_linear_rope_kv_of_every_tile_whole_and_cut(hip, tile, kind, B, S, Hq, Hkv, hd, K)
+
+
 @pytest.mark.parametrize("M,I,K", [(40, 1000, 2056), (128, 512, 4096), (300, 1000, 4104), (777, 2048, 4096)])
 def test_linear_swiglu_out_pieces(hip, M, I, K):
     """[up; gate] pairs in cut tiles: the activation after the sums are complete."""
