@@ -133,6 +133,11 @@ int lr_linear_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_
 int lr_linear_pieces(const void* x, int64_t ldx, const void* w, int M, int N, int K, void* sums, size_t sums_bytes, int32_t* pieces,
                      lr_stream_t stream);
 
+/* Two such products of dense rows, x0 [M, K0] w0 [N, K0]^T and x1 [M, K1] w1 [N, K1]^T, in one launch: pieces of about the same
+ * length, sums_bytes of memory for either.  LR_E_UNSUPPORTED, with nothing launched, where two launches are the faster way. */
+int lr_linear_pieces_two(const void* x0, const void* w0, int K0, void* sums0, int32_t* pieces0, const void* x1, const void* w1, int K1,
+                         void* sums1, int32_t* pieces1, int M, int N, size_t sums_bytes, lr_stream_t stream);
+
 /* lr_linear with the launch configuration of the GEMV given by the caller instead of chosen from
  * the shape: gemv_cfg = rows per wave * 100 + K-split * 10 + unroll, one of 144, 212, 222, 242, 244,
  * 412, 422, 442 (anything else: 242; 0: the shape heuristic, i.e. lr_linear).  A non-zero gemv_cfg
@@ -271,6 +276,15 @@ int lr_attn_decode_beside_merged(const void* q, int64_t ldq, const void* k_cache
                                  void* y, int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch,
                                  size_t scratch_bytes, const lr_projection_t* projection, const lr_row_norm_t* norm,
                                  void* tickets, int M, lr_stream_t stream);
+
+/* lr_attn_decode and, in the same grid, lr_linear_swiglu_out_scratch of 33 to 64 rows: act [M, N / 2] = silu(gate) * up for w [N, K] =
+ * [up; gate] rows, its partial sums in `sums`.  The two must be independent of each other.  Same bits as the two calls.  `tickets` as
+ * in lr_attn_decode_beside_merged, not NULL.  LR_E_UNSUPPORTED (nothing launched): other numbers of rows, K % 64 != 0, more than 64 key
+ * chunks, q heads per kv head other than 1, 2, 4, 8, 16, and products that the plan gives other tiles. */
+int lr_attn_decode_beside_product(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos, void* y,
+                                  int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch, size_t scratch_bytes,
+                                  void* tickets, const void* x, int64_t ldx, const void* w, void* act, int64_t ld_act, int M, int N,
+                                  int K, void* sums, size_t sums_bytes, lr_stream_t stream);
 
 /* Weight-only fp8 linear:  y[m, n] = bf16( bf16( sum_k x[m, k] * w8[n, k] ) * scales[n] ).
  * w8 [N, K] dense float8 e4m3 (OCP "e4m3fn": bias 7, no infinities, max 448), one byte per weight;

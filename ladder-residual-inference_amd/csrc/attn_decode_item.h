@@ -1,5 +1,6 @@
 #pragma once
 #include "lr_common.h"
+#include <type_traits>
 
 // ---- how the valid keys are cut into chunks (one workgroup item per chunk, kv head and sequence).
 //      A chunk never exceeds ATT_CHUNK keys: the item then requests all of its K and V rows at once.
@@ -60,9 +61,9 @@ constexpr int ATT_AUX_COHERENT = 17;
 // are zero columns).  P.V too: V lies in LDS as it came, 64 keys at a time, and is read transposed
 // (ds_read_b64_tr_b16) as A fragments, a wave multiplies HD / 4 of the dimensions by all keys, and a softmax weight enters as
 // three bf16 summands, which hold all 24 bits of it: the products are those of fp32 weights.
-// (P.V on the vector units, lanes owning 8 dimensions of one key in four and the four waves' sums met in LDS, was 14 KB of code
-// passed through once, which every launch fetches anew: 6.7 us from the last row's arrival to the stored result for 8 heads of
-// 65 keys beside a weight stream, now 2.5 us in 4 KB.  64 sequences of the 70B rank shard, ms per step: 7.45 -> 7.05.  The
+// (P.V on the vector units, lanes owning 8 dimensions of one key in four and the four waves' sums met in LDS, was a thousand
+// vector instructions one behind the other, at 4 to 8 cycles each: 6.7 us from the last row's arrival to the stored result for 8
+// heads of 65 keys beside a weight stream, now 2.5 us.  64 sequences of the 70B rank shard, ms per step: 7.45 -> 7.05.  The
 // chunk results' error against 64 bits is 1.6e-7 of their norm, as it was.)
 template <int HD, int G>
 __host__ __device__ constexpr int attn_item_lds_floats(int chunk_max) {
@@ -142,19 +143,25 @@ __device__ __forceinline__ void attn_partial_item(const u16* __restrict__ q, int
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
       qf[ks] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(qres, l16 < G ? (l16 * HD + ks * 32 + l4 * 8) * 2 : OOB_, 0, 0));
-    int off[GROUPS][NI];
+    // (non-temporal: a row is read once per step, and what it would push out of the L2 are the inputs of the projection beside it --
+    // unless two groups of heads share it.  70B rank shard, us per step: 64 rows 6826 -> 6744, 8 rows 4383 -> 4331, 8B 16 rows 3469 -> 3442)
+    auto load = [&](auto AUX) {
+      int off[GROUPS][NI];
 #pragma unroll
-    for (int j = 0; j < GROUPS; ++j)
+      for (int j = 0; j < GROUPS; ++j)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int key = k0 + (j * 4 + wave) * 16 + i * KPW + kl;
-        off[j][i] = key < k1 ? (key * HD + dl) * 2 : OOB_;
-        kr[j][i] = __builtin_amdgcn_raw_buffer_load_b128(kres, off[j][i], 0, 0);
-      }
+        for (int i = 0; i < NI; ++i) {
+          const int key = k0 + (j * 4 + wave) * 16 + i * KPW + kl;
+          off[j][i] = key < k1 ? (key * HD + dl) * 2 : OOB_;
+          kr[j][i] = __builtin_amdgcn_raw_buffer_load_b128(kres, off[j][i], 0, decltype(AUX)::value);
+        }
 #pragma unroll
-    for (int j = 0; j < GROUPS; ++j)
+      for (int j = 0; j < GROUPS; ++j)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) vr[j][i] = __builtin_amdgcn_raw_buffer_load_b128(vres, off[j][i], 0, 0);
+        for (int i = 0; i < NI; ++i) vr[j][i] = __builtin_amdgcn_raw_buffer_load_b128(vres, off[j][i], 0, decltype(AUX)::value);
+    };
+    if (kv_share == 1) load(std::integral_constant<int, 2>{});
+    else load(std::integral_constant<int, 0>{});
   }
 
   // ---- scores: S[key][head] = sum_d K[key][d] q[head][d] on the matrix cores
@@ -383,4 +390,79 @@ static inline void launch_attn_combine(const float* o_part, const float* ml_part
   if (nsplit <= 32) k_attn_decode_combine_once<HD, 1><<<dim3(Hq, B), dim3(HD), 0, s>>>(o_part, ml_part, y, ldy, Hq, nsplit);
   else if (nsplit <= 64) k_attn_decode_combine_once<HD, 2><<<dim3(Hq, B), dim3(HD), 0, s>>>(o_part, ml_part, y, ldy, Hq, nsplit);
   else k_attn_decode_combine<HD><<<dim3(Hq, B), dim3(HD), 0, s>>>(o_part, ml_part, y, ldy, Hq, nsplit);
+}
+
+// ---- the items, and the waves that merge them, as the workgroups of a grid that holds a projection too (decode_pair.hip, gemm.hip)
+struct AttnItems {
+  const u16* q;
+  int64_t ldq;
+  const u16* kc;
+  const u16* vc;
+  const int32_t* pos;
+  float* o_part;
+  float* ml_part;
+  int Hkv, Smax, nsplit, chunk_max;  // Hkv: groups of G q heads (kv_share of them per head of the cache)
+  int kv_share;
+  int n_items;  // nsplit * Hkv * B workgroups
+  // with tickets: the chunks are merged into y by workgroups of their own
+  u32* tickets;  // [B * Hkv * ATT_TICKET], zero
+  u16* y;
+  int64_t ldy;
+  int merge_waves, waves_per_wg;  // of 64 outputs; of them in a workgroup
+
+  int mergers() const { return tickets ? (merge_waves + waves_per_wg - 1) / waves_per_wg : 0; }
+};
+// item `wg` of n_items; merging workgroup `wg` of mergers(), behind all items in the grid
+template <int HD, int G, int GROUPS, bool MERGE>
+__device__ __forceinline__ void attn_item(const AttnItems& a, int wg, float* smem) {
+  const int split = wg % a.nsplit, rest = wg / a.nsplit;
+  attn_partial_item<HD, G, GROUPS, MERGE>(a.q, a.ldq, a.kc, a.vc, a.pos, a.o_part, a.ml_part, a.Hkv, a.Smax, a.nsplit,
+                                          a.chunk_max, split, rest % a.Hkv, rest / a.Hkv, smem, a.kv_share);
+  if constexpr (MERGE) attn_item_done(a.tickets + rest * ATT_TICKET);
+}
+template <int HD, int G>
+__device__ __forceinline__ void attn_merge(const AttnItems& a, int wg) {
+  const int wave = threadIdx.x >> 6, m = wg * a.waves_per_wg + wave;
+  if (wave < a.waves_per_wg && m < a.merge_waves)
+    attn_merge_wave<HD, G>(a.o_part, a.ml_part, a.tickets, a.y, a.ldy, a.Hkv, a.nsplit, __builtin_amdgcn_readfirstlane(m));
+}
+// Checks lr_attn_decode's arguments and fills `a`; G: q heads of an item.
+static inline int attn_fill_items(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos, void* y, int64_t ldy,
+                                  int B, int Hq, int Hkv, int hd, int Smax, void* scratch, size_t scratch_bytes, void* tickets, AttnItems& a,
+                                  int& G) {
+  LR_REQUIRE_PTR(q);
+  LR_REQUIRE_PTR(k_cache);
+  LR_REQUIRE_PTR(v_cache);
+  LR_REQUIRE_PTR(y);
+  LR_REQUIRE_PTR(scratch);
+  if (pos == nullptr) return LR_E_NULL;
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || hd <= 0 || Smax <= 0 || Hq % Hkv) return LR_E_SHAPE;
+  if ((int64_t)Smax * hd * 2 >= 0x7fffffff) return LR_E_UNSUPPORTED;  // the rows of one (sequence, head) are addressed with 32-bit offsets
+  if (ldq < (int64_t)Hq * hd || ldy < (int64_t)Hq * hd || B > 65535) return LR_E_SHAPE;
+  if (ldq % 8 || ldy % 8) return LR_E_ALIGN;
+  if (scratch_bytes < lr_attn_decode_scratch_bytes(B, Hq, hd, Smax)) return LR_E_SHAPE;
+  if (((uintptr_t)tickets & 3) != 0) return LR_E_ALIGN;
+  a = AttnItems{};
+  G = Hq / Hkv;
+  a.kv_share = 1;
+  a.q = (const u16*)q; a.ldq = ldq; a.kc = (const u16*)k_cache; a.vc = (const u16*)v_cache; a.pos = pos;
+  a.Smax = Smax;
+  a.nsplit = attn_pick_nsplit(B, Hkv, Smax);  // the chunks of lr_attn_decode
+  if (G == 16) {
+    // 16 q heads per kv head need the whole register file (one workgroup per CU): two groups of 8 instead
+    G = 8;
+    a.kv_share = 2;
+  }
+  a.Hkv = Hkv * a.kv_share;
+  a.chunk_max = ((Smax + a.nsplit - 1) / a.nsplit + 3) & ~3;
+  a.o_part = (float*)scratch;
+  a.ml_part = a.o_part + (size_t)B * Hq * a.nsplit * hd;
+  if ((int64_t)a.nsplit * a.Hkv * B > 0x3fffffff) return LR_E_UNSUPPORTED;
+  a.n_items = a.nsplit * a.Hkv * B;
+  a.y = (u16*)y; a.ldy = ldy;
+  a.tickets = a.nsplit <= ATT_MERGE_MAX ? (u32*)tickets : nullptr;   // (more chunks: a launch of their own)
+  if (!((hd == 128 || hd == 64) && (G == 1 || G == 2 || G == 4 || G == 8))) return LR_E_UNSUPPORTED;
+  a.merge_waves = B * Hq * (hd / 64);
+  a.waves_per_wg = a.merge_waves > 2 * ATT_NCU ? 4 : a.merge_waves > ATT_NCU ? 2 : 1;   // (spread over the CUs, whose parts of a projection are to end together)
+  return LR_OK;
 }

@@ -20,24 +20,6 @@
 
 namespace {
 
-struct AttnItems {
-  const u16* q;
-  int64_t ldq;
-  const u16* kc;
-  const u16* vc;
-  const int32_t* pos;
-  float* o_part;
-  float* ml_part;
-  int Hkv, Smax, nsplit, chunk_max;  // Hkv: groups of G q heads (kv_share of them per head of the cache)
-  int kv_share;
-  int n_items;  // nsplit * Hkv * B: the first workgroups of the grid
-  // MERGE: the workgroups behind the bands merge the chunks into y
-  u32* tickets;  // [B * Hkv], zero
-  u16* y;
-  int64_t ldy;
-  int merge_waves, waves_per_wg;  // of 64 outputs; of them in a workgroup
-};
-
 constexpr int PAIR_MT = 16, PAIR_UNITS = 2;
 
 // X8: at most 8 input rows in fragment layout, requested as far ahead as the weights (see stream_band)
@@ -47,15 +29,9 @@ __global__ __launch_bounds__(256, XL ? 0 : 2) void k_attn_beside_band(const Attn
   extern __shared__ __attribute__((aligned(16))) unsigned char pair_smem[];
   const int wg = blockIdx.x;
   if (wg < a.n_items) {
-    const int split = wg % a.nsplit, rest = wg / a.nsplit;
-    float* const smem = reinterpret_cast<float*>(pair_smem);
-    attn_partial_item<HD, G, GROUPS, MERGE>(a.q, a.ldq, a.kc, a.vc, a.pos, a.o_part, a.ml_part, a.Hkv, a.Smax, a.nsplit,
-                                           a.chunk_max, split, rest % a.Hkv, rest / a.Hkv, smem, a.kv_share);
-    if constexpr (MERGE) attn_item_done(a.tickets + rest * ATT_TICKET);
+    attn_item<HD, G, GROUPS, MERGE>(a, wg, reinterpret_cast<float*>(pair_smem));
   } else if (MERGE && wg >= a.n_items + p.nwg) {
-    const int wave = threadIdx.x >> 6, m = (wg - a.n_items - p.nwg) * a.waves_per_wg + wave;
-    if (wave < a.waves_per_wg && m < a.merge_waves)
-      attn_merge_wave<HD, G>(a.o_part, a.ml_part, a.tickets, a.y, a.ldy, a.Hkv, a.nsplit, __builtin_amdgcn_readfirstlane(m));
+    attn_merge<HD, G>(a, wg - a.n_items - p.nwg);
   } else {
     stream_band<PAIR_MT, PAIR_UNITS, W8, XL, false, false, NWV, 16, X8, X8>(p, M, wg - a.n_items, reinterpret_cast<u16*>(pair_smem));
   }
@@ -63,13 +39,12 @@ __global__ __launch_bounds__(256, XL ? 0 : 2) void k_attn_beside_band(const Attn
 
 template <int HD, int G, bool W8, bool XL, int GROUPS, bool X8, bool MERGE>
 static int launch_pair_merge(const AttnItems& a, const Proj& p, int M, int B, hipStream_t s) {
-  const int mergers = MERGE ? (a.merge_waves + a.waves_per_wg - 1) / a.waves_per_wg : 0;
   const size_t lds_att = (size_t)attn_item_lds_floats<HD, G>(a.chunk_max) * sizeof(float);
   const size_t lds_band = stream_band_lds_bytes<PAIR_MT, PAIR_UNITS, W8, XL>() + stream_band_norm_bytes(p, M);
   const size_t lds = lds_att > lds_band ? lds_att : lds_band;
   static std::atomic<unsigned long long> lds_raised{0};
   if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_attn_beside_band<HD, G, W8, XL, GROUPS, X8, MERGE>), lds, lds_raised)) return LR_E_LAUNCH;
-  k_attn_beside_band<HD, G, W8, XL, GROUPS, X8, MERGE><<<dim3((unsigned)(a.n_items + p.nwg + mergers)), dim3(256), lds, s>>>(a, p, M);
+  k_attn_beside_band<HD, G, W8, XL, GROUPS, X8, MERGE><<<dim3((unsigned)(a.n_items + p.nwg + a.mergers())), dim3(256), lds, s>>>(a, p, M);
   if (!MERGE) launch_attn_combine<HD>(a.o_part, a.ml_part, a.y, a.ldy, a.Hkv * G, B, a.nsplit, s);
   return lr_launch_status();
 }
@@ -99,49 +74,22 @@ static int beside(const void* q, int64_t ldq, const void* k_cache, const void* v
                   int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch, size_t scratch_bytes,
                   const Projection* proj, const lr_row_norm_t* norm, void* tickets, int M, int m_min, lr_stream_t stream,
                   Fill fill) {
-  LR_REQUIRE_PTR(q);
-  LR_REQUIRE_PTR(k_cache);
-  LR_REQUIRE_PTR(v_cache);
-  LR_REQUIRE_PTR(y);
-  LR_REQUIRE_PTR(scratch);
-  if (pos == nullptr || proj == nullptr) return LR_E_NULL;
-  if (B <= 0 || Hq <= 0 || Hkv <= 0 || hd <= 0 || Smax <= 0 || Hq % Hkv || M < 1) return LR_E_SHAPE;
-  if ((int64_t)Smax * hd * 2 >= 0x7fffffff) return LR_E_UNSUPPORTED;  // the rows of one (sequence, head) are addressed with 32-bit offsets
-  if (ldq < (int64_t)Hq * hd || ldy < (int64_t)Hq * hd || B > 65535) return LR_E_SHAPE;
-  if (ldq % 8 || ldy % 8) return LR_E_ALIGN;
-  if (scratch_bytes < lr_attn_decode_scratch_bytes(B, Hq, hd, Smax)) return LR_E_SHAPE;
-  if (((uintptr_t)tickets & 3) != 0) return LR_E_ALIGN;
+  AttnItems a;
+  int G;
+  const int arc = attn_fill_items(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, tickets, a, G);
+  if (arc != LR_OK && arc != LR_E_UNSUPPORTED) return arc;
+  if (proj == nullptr) return LR_E_NULL;
+  if (M < 1) return LR_E_SHAPE;
+  if (arc != LR_OK) return arc;
   // the projection must not touch the cache the attention reads, and only the 16-row band shares a CU
   if (proj->epilogue == LR_EPI_ROPE_KV || M > PAIR_MT || M < m_min) return LR_E_UNSUPPORTED;
   Proj p;
   int rc = fill(*proj, p);
   if (rc == LR_OK) rc = sb_fill_norm(norm, p);
   if (rc != LR_OK) return rc;
-  int G = Hq / Hkv;
-  AttnItems a;
-  a.kv_share = 1;
-  a.q = (const u16*)q; a.ldq = ldq; a.kc = (const u16*)k_cache; a.vc = (const u16*)v_cache; a.pos = pos;
-  a.Smax = Smax;
-  a.nsplit = attn_pick_nsplit(B, Hkv, Smax);  // the chunks of lr_attn_decode
-  if (G == 16) {
-    // 16 q heads per kv head need the whole register file (one workgroup per CU): two groups of 8 instead
-    G = 8;
-    a.kv_share = 2;
-  }
-  a.Hkv = Hkv * a.kv_share;
-  a.chunk_max = ((Smax + a.nsplit - 1) / a.nsplit + 3) & ~3;
-  a.o_part = (float*)scratch;
-  a.ml_part = a.o_part + (size_t)B * Hq * a.nsplit * hd;
-  if ((int64_t)a.nsplit * a.Hkv * B > 0x3fffffff) return LR_E_UNSUPPORTED;
-  a.n_items = a.nsplit * a.Hkv * B;
-  a.y = (u16*)y; a.ldy = ldy;
-  a.tickets = a.nsplit <= ATT_MERGE_MAX ? (u32*)tickets : nullptr;   // (more chunks: a launch of their own)
-  if (!((hd == 128 || hd == 64) && (G == 1 || G == 2 || G == 4 || G == 8))) return LR_E_UNSUPPORTED;
   const int ncu = lr_num_cus();
   if (ncu < 1) return LR_E_LAUNCH;
   plan(p, M, p.pair_off ? 16 : 16 * PAIR_UNITS, ncu);
-  a.merge_waves = B * Hq * (hd / 64);
-  a.waves_per_wg = a.merge_waves > 2 * ncu ? 4 : a.merge_waves > ncu ? 2 : 1;   // (spread over the CUs, whose bands are to end together)
   if (p.fold_sums && p.nwg < M) return LR_E_UNSUPPORTED;   // (a row per workgroup)
   hipStream_t s = (hipStream_t)stream;
 #define LR_PAIR(HDV, GV) \

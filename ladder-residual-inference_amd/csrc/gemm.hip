@@ -9,6 +9,7 @@
 // bytes (stride 144 B keeps ds_read_b128 of 16 consecutive rows on distinct banks) -> 128-bit LDS
 // reads that deliver exactly the 8 consecutive k an MFMA lane feeds.  LDS is double-buffered and
 // the global loads of tile t+1 are in flight while tile t is multiplied.
+#include "attn_decode_item.h"
 #include "lr_common.h"
 #include <type_traits>
 
@@ -239,13 +240,39 @@ __device__ __forceinline__ void gemm_tile_at(int t, int tm, int tn, int& mt, int
   mt = band * 4 + r - nt * h;
 }
 
-// The outputs of R16 groups of 16 rows of a wave's part of a tile.  The products are W-tile x X-tile^T: a lane of
+// Eight columns of an output row, from column n on.
+__device__ __forceinline__ void gemm_put(u16* __restrict__ y, int64_t ldy, int N, int m, int n, const uint4& v) {
+  if ((ldy & 7) == 0 && n + 7 < N) {
+    st16(y + (int64_t)m * ldy + n, v);
+  } else {
+    const u32 q[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (n + e < N) y[(int64_t)m * ldy + n + e] = (u16)(q[e >> 1] >> ((e & 1) * 16));
+  }
+}
+// The section (q, k, v), head and dimension of column n.
+__device__ __forceinline__ void gemm_rope_at(const GemmRope& rp, int n, int& sect, int& hh, int& dd) {
+  const int nq = rp.Hq * rp.hd, nkv = rp.Hkv * rp.hd;
+  sect = n < nq ? 0 : (n < nq + nkv ? 1 : 2);
+  const int cc = n - (sect == 0 ? 0 : (sect == 1 ? nq : nq + nkv));
+  hh = cc / rp.hd;
+  dd = cc - hh * rp.hd;
+}
+// What k_rope_kv_write would do to eight columns of sequence b's row at position ps, with their table entries tv; what is stored.
+__device__ __forceinline__ uint4 gemm_rope(const GemmRope& rp, int sect, int hh, int dd, int b, int ps, const uint4& v, const uint4& tv) {
+  const uint4 r = sect < 2 ? rope8(v, tv) : v;
+  if (sect == 0) return r;
+  st16((sect == 1 ? rp.k_cache : rp.v_cache) + (((int64_t)b * rp.Hkv + hh) * rp.Smax + ps) * rp.hd + dd, r);
+  return v;
+}
+
+// The outputs of a wave's part of a tile.  The products are W-tile x X-tile^T: a lane of
 // acc[a][b] holds four consecutive columns 4 (lane / 16) .. of row lane % 16; b < 2 BH are columns of the tile's first half
 // of weight rows, the others of its second.  Stored from there an instruction would touch 32 bytes in each of 16 rows: they
-// take one trip through LDS (`eb`, a piece of the wave's own) and leave as whole rows.  `row0`: first of the wave's row
-// groups here, m = tile row of group g is row_of(g).
-template <int A, int BH, int MODE, int R16>
-__device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u16* eb, int g0, int wm, int wn, int m0, int n0, u16* __restrict__ y,
+// take one trip through LDS (`eb`, a piece of the wave's own) and leave as whole rows.
+template <int A, int BH, int MODE>
+__device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[A][4 * BH], u16* eb, int wm, int wn, int m0, int n0, u16* __restrict__ y,
                                            int64_t ldy, int M, int N, const GemmRope& rp, const int32_t* entry) {
   int lane = threadIdx.x & 63;   // (laundered: the addresses below are not formed before the k loop and kept through it)
   asm volatile("" : "+v"(lane));
@@ -253,7 +280,7 @@ __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u1
   constexpr int HC = 32 * BH;                        // a wave's columns in one half
   constexpr int EP = (P ? HC : 2 * HC) + 8;
 #pragma unroll
-  for (int a = 0; a < R16; ++a) {
+  for (int a = 0; a < A; ++a) {
     const int ml = a * 16 + (lane & 15);
 #pragma unroll
     for (int b = 0; b < (P ? 2 * BH : 4 * BH); ++b) {
@@ -267,19 +294,10 @@ __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u1
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // a wave reads back only what it wrote itself
   constexpr int LPR = HC / 8, RPI = 64 / LPR;         // lanes per row, rows per instruction
   const int cl = (lane % LPR) * 8;
-  const bool vec_ok = (ldy & 7) == 0;
-  auto row_of = [&](int ml) { return m0 + GemmTile<A, BH>::group_row(g0 + (ml >> 4), wm) + (ml & 15); };
+  auto row_of = [&](int ml) { return m0 + GemmTile<A, BH>::group_row(ml >> 4, wm) + (ml & 15); };
   auto store_row = [&](int m, int n, const uint4& v) {
     if (m >= M) return;
-    if (entry != nullptr) m = entry[m];
-    if (vec_ok && n + 7 < N) {
-      st16(y + (int64_t)m * ldy + n, v);
-    } else {
-      const u32 q[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (n + e < N) y[(int64_t)m * ldy + n + e] = (u16)(q[e >> 1] >> ((e & 1) * 16));
-    }
+    gemm_put(y, ldy, N, entry != nullptr ? entry[m] : m, n, v);
   };
 #pragma unroll
   for (int hb = 0; hb < (P ? 1 : 2); ++hb) {
@@ -289,11 +307,10 @@ __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u1
       // (head_dim % 8 == 0).  Positions of several rows first, then their table entries, then the arithmetic: two memory
       // round trips per RB rows (row by row the position and the entry it selects are a chain of two loads per row, and
       // the output pass of a tile took three times as long).
-      constexpr int RI = R16 * 16 / RPI, RB = RI <= 8 ? RI : RI % 8 == 0 ? 8 : RI / 2;   // (10, 12 and 14 in two halves)
+      constexpr int RI = A * 16 / RPI, RB = RI <= 8 ? RI : RI % 8 == 0 ? 8 : RI / 2;   // (10, 12 and 14 in two halves)
       static_assert(RI % RB == 0 && RB <= 8, "");
-      const int nq = rp.Hq * rp.hd, nkv = rp.Hkv * rp.hd;
-      const int sect = n < nq ? 0 : (n < nq + nkv ? 1 : 2), cc = n - (sect == 0 ? 0 : (sect == 1 ? nq : nq + nkv));
-      const int hh = cc / rp.hd, dd = cc - hh * rp.hd;
+      int sect, hh, dd;
+      gemm_rope_at(rp, n, sect, hh, dd);
       for (int i0 = 0; i0 < RI; i0 += RB) {
         int ps[RB], bb[RB];
 #pragma unroll
@@ -314,9 +331,7 @@ __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u1
           const int ml = (i0 + i) * RPI + lane / LPR, m = row_of(ml);
           uint4 v = *reinterpret_cast<const uint4*>(&eb[ml * EP + hb * HC + cl]);
           if (ok[i]) {
-            const uint4 r = sect < 2 ? rope8(v, tv[i]) : v;
-            if (sect == 0) v = r;
-            else st16((sect == 1 ? rp.k_cache : rp.v_cache) + (((int64_t)bb[i] * rp.Hkv + hh) * rp.Smax + ps[i]) * rp.hd + dd, r);
+            v = gemm_rope(rp, sect, hh, dd, bb[i], ps[i], v, tv[i]);
           } else if (m < M && n == 0 && rp.err) {
             *rp.err = LR_DEV_POS_RANGE;
           }
@@ -325,7 +340,7 @@ __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[R16][4 * BH], u1
       }
     } else {
 #pragma unroll 4
-      for (int r0 = 0; r0 < R16 * 16; r0 += RPI) {
+      for (int r0 = 0; r0 < A * 16; r0 += RPI) {
         const int ml = r0 + lane / LPR;
         store_row(row_of(ml), n, *reinterpret_cast<const uint4*>(&eb[ml * EP + hb * HC + cl]));
       }
@@ -546,7 +561,7 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
       return;
     }
   }
-  if constexpr (MODE != GEMM_ROWS) gemm_store<A, BH, MODE, A>(acc, gsm + wave * (T::EBYTES / 8), 0, wm, wn, m0, n0, y, ldy, M, N, rp, GROUP ? entry : nullptr);
+  if constexpr (MODE != GEMM_ROWS) gemm_store<A, BH, MODE>(acc, gsm + wave * (T::EBYTES / 8), wm, wn, m0, n0, y, ldy, M, N, rp, GROUP ? entry : nullptr);
 }
 
 template <int A, int BH, bool KTAIL, int MODE, bool GROUP, bool NT = false>
@@ -581,37 +596,84 @@ __global__ __launch_bounds__(256, GEMM_PER_CU(A, BH)) void k_gemm_two(const Gemm
   }
 }
 
-// The cut tiles: a workgroup adds the pieces of a 1 / A part of one (16 rows per wave, four pieces' loads in flight
-// together, summed in order) and finishes it.  Bound: memory, mostly the last-level cache: the pieces were just written.
+// The attention of a decode step of 33 to 64 sequences and the block's up/gate product, which do not depend on each other in a ladder
+// or a parallel block, in one grid: an attention item (attn_decode_item.h) for every CU, the product's tiles, the other items, the
+// waves that merge them.  Bound: HBM; apart, the attention's items leave the memory idle between their rows' arrival and the next
+// item's request, and the product's workgroups at their ramp and drain.  us per step of the 70B rank shard at 64 rows: the two chains of
+// a block on two branches of the graph 7125, in this grid 6825 (all items behind the tiles 6935, all in front 7059; the plan's three
+// pieces of K, with four 7340), of it per block 38 here, where the product alone takes 28 and the attention alone 16 and 4.
+template <int HD, int G, int GROUPS>
+__global__ __launch_bounds__(256, 2) void k_attn_beside_gemm(const AttnItems a, const GemmProduct p, const int n_gemm) {
+  extern __shared__ __attribute__((aligned(1024))) u16 gsm[];
+  const int first = a.n_items < ATT_NCU ? a.n_items : ATT_NCU, tile = (int)blockIdx.x - first, wg = tile < 0 ? (int)blockIdx.x : (int)blockIdx.x - n_gemm;
+  if (tile >= 0 && tile < n_gemm)
+    gemm_tile<2, 1, false, GEMM_PAIR, false, true>(tile, 0, p.x, p.ldx, p.w, p.y, p.ldy, p.M, p.N, p.K, p.tm, p.tn, GemmRope{}, p.sp, GemmGroup{});
+  else if (wg < a.n_items)
+    attn_item<HD, G, GROUPS, true>(a, wg, reinterpret_cast<float*>(gsm));
+  else
+    attn_merge<HD, G>(a, wg - a.n_items);
+}
+
+// The cut tiles: a workgroup adds the pieces of 16 rows of a wave's part of one and finishes them.  Bound: memory, mostly the
+// last-level cache, since the pieces were just written; of small products the round trips: so a wave takes a quarter of the
+// columns, up to eight pieces' loads in flight together, summed in order, and a lane finishes eight columns of one row.  (A
+// wave for all columns and four pieces at a time, us: q/k/v of the 70B rank shard at 64 rows, 16 pieces, 7.1 -> @@, up/gate 4.7 -> @@.)
 template <int A, int BH, int MODE>
 __global__ __launch_bounds__(256) void k_gemm_sum(u16* __restrict__ y, int64_t ldy, int M, int N, int tm, int tn, const GemmRope rp, const GemmSplit sp) {
   using T = GemmTile<A, BH>;
-  __shared__ __attribute__((aligned(16))) u16 sm[4 * 16 * T::EPITCH];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int rt = blockIdx.x / A, g0 = blockIdx.x - rt * A;
+  constexpr bool P = MODE == GEMM_PAIR;
+  constexpr int HC = 32 * BH, EP = (P ? HC : 2 * HC) + 8;
+  __shared__ __attribute__((aligned(16))) u16 eb[16 * EP];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int part = blockIdx.x & 3, wm = part >> 1, wn = part & 1;
+  const int rt = blockIdx.x / (4 * A), g = blockIdx.x / 4 - rt * A;
   int mt, nt;
   gemm_tile_at(sp.full + rt, tm, tn, mt, nt);
-  const int m0 = mt * T::TM, n0 = nt * (MODE == GEMM_PAIR ? T::TN / 2 : T::TN);
-  if (m0 + T::group_row(g0, 0) >= M) return;   // (its lowest row; no barrier follows)
-  constexpr int C = 4 * BH, STEP = T::TM * T::TN;
-  const float* p = sp.part + (int64_t)rt * sp.splits * STEP + ((int64_t)wave * A + g0) * (C * 256) + lane * 4;
-  f32x4_t acc[1][C], v[4][C];
+  const int m0 = mt * T::TM + T::group_row(g, wm), n0 = nt * (P ? T::TN / 2 : T::TN) + wn * HC;
+  if (m0 >= M) return;   // uniform
+  constexpr int C = 4 * BH, STEP = T::TM * T::TN, UNITS = P ? 2 * BH : C;   // a unit: sixteen columns, or as many pairs
+  const float* const p = sp.part + (int64_t)rt * sp.splits * STEP + ((int64_t)part * A + g) * (C * 256) + lane * 4;
+  for (int u = wave; u < UNITS; u += 4) {
+    constexpr int NF = P ? 2 : 1, NP = 8;
+    f32x4_t acc[NF], v[NP][NF];
 #pragma unroll
-  for (int b = 0; b < C; ++b) acc[0][b] = *reinterpret_cast<const f32x4_t*>(p + b * 256);
-  for (int s = 1; s < sp.splits; s += 4) {
+    for (int f = 0; f < NF; ++f) acc[f] = *reinterpret_cast<const f32x4_t*>(p + (u + f * 2 * BH) * 256);
+    for (int s = 1; s < sp.splits; s += NP) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < NP; ++i)
 #pragma unroll
-      for (int b = 0; b < C; ++b)
-        v[i][b] = *reinterpret_cast<const f32x4_t*>(p + (int64_t)(s + i < sp.splits ? s + i : 0) * STEP + b * 256);
+        for (int f = 0; f < NF; ++f)
+          v[i][f] = *reinterpret_cast<const f32x4_t*>(p + (int64_t)(s + i < sp.splits ? s + i : 0) * STEP + (u + f * 2 * BH) * 256);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (s + i < sp.splits) {
+      for (int i = 0; i < NP; ++i)
+        if (s + i < sp.splits) {
 #pragma unroll
-        for (int b = 0; b < C; ++b) acc[0][b] += v[i][b];
-      }
+          for (int f = 0; f < NF; ++f) acc[f] += v[i][f];
+        }
+    }
+    float o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = P ? swiglu_bf(round_bf(acc[0][e]), round_bf(acc[NF - 1][e])) : acc[0][e];
+    *reinterpret_cast<uint2*>(&eb[(lane & 15) * EP + u * 16 + (lane >> 4) * 4]) = make_uint2(pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]));
   }
-  gemm_store<A, BH, MODE, 1>(acc, sm + wave * (16 * T::EPITCH), g0, wave >> 1, wave & 1, m0, n0, y, ldy, M, N, rp, nullptr);
+  __syncthreads();
+  constexpr int LPR = HC / 8, LANES = 16 * LPR * (P ? 1 : 2);   // of a row's half
+  static_assert(LANES <= 256, "");
+  if (tid >= LANES) return;
+  const int hb = tid / (16 * LPR), r = tid / LPR % 16, cl = tid % LPR * 8;
+  const int m = m0 + r, n = n0 + hb * 64 * BH + cl;
+  if (m >= M) return;
+  uint4 v = *reinterpret_cast<const uint4*>(&eb[r * EP + hb * HC + cl]);
+  if constexpr (MODE == GEMM_ROPE) {
+    int sect, hh, dd;
+    gemm_rope_at(rp, n, sect, hh, dd);
+    const int b = m / rp.S, ps = rp.pos[m - b * rp.S];
+    if (n < N && ps >= 0 && ps < rp.Smax && ps < rp.block_size)
+      v = gemm_rope(rp, sect, hh, dd, b, ps, v, sect < 2 ? ld16(rp.table + (int64_t)ps * rp.hd + dd) : make_uint4(0, 0, 0, 0));
+    else if (n == 0 && rp.err)
+      *rp.err = LR_DEV_POS_RANGE;
+  }
+  gemm_put(y, ldy, N, m, n, v);
 }
 
 // ---- which tile, and which tiles are cut along K
@@ -723,7 +785,7 @@ static int gemm_run_as(const void* x, int64_t ldx, const void* w, void* y, int64
   k_gemm_dma<A, BH, KTAIL, MODE, false, NT><<<dim3((unsigned)(p.full + p.rem * p.splits)), dim3(256), T::LDS, s>>>(
       (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, M, N, K, tm, tn, rp, sp, GemmGroup{});
   if constexpr (MODE != GEMM_ROWS)
-    if (p.rem) k_gemm_sum<A, BH, MODE><<<dim3((unsigned)(p.rem * A)), dim3(256), 0, s>>>((u16*)y, ldy, M, N, tm, tn, rp, sp);
+    if (p.rem) k_gemm_sum<A, BH, MODE><<<dim3((unsigned)(p.rem * A * 4)), dim3(256), 0, s>>>((u16*)y, ldy, M, N, tm, tn, rp, sp);
   return lr_launch_status();
 }
 template <int A, int BH, bool KTAIL, bool NT = false>
@@ -826,6 +888,34 @@ int gemm_inputs(const void* x0, const void* wqkv, void* qkv, int S, const lr_rop
                     rope->n_kv_head, rope->head_dim, rope->smax, rope->block_size};
   return gemm_two<GEMM_ROPE, GEMM_PAIR>(best, gemm_product(best, GEMM_ROPE, x0, K, wqkv, qkv, N, M, N, K),
                                         gemm_product(best, GEMM_PAIR, x1, K, w1, act, I, M, I, K), rp, s);
+}
+
+template <int HD, int G, int GROUPS>
+static int attn_beside_gemm(const AttnItems& a, const GemmProduct& p, hipStream_t s) {
+  const size_t att = (size_t)attn_item_lds_floats<HD, G>(a.chunk_max) * sizeof(float), lds = att > GemmTile<2, 1>::LDS ? att : GemmTile<2, 1>::LDS;
+  static std::atomic<unsigned long long> raised{0};
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_attn_beside_gemm<HD, G, GROUPS>), lds, raised)) return LR_E_LAUNCH;
+  const int n = p.sp.full + p.sp.rem * p.sp.splits;
+  k_attn_beside_gemm<HD, G, GROUPS><<<dim3((unsigned)(n + a.n_items + a.mergers())), dim3(256), lds, s>>>(a, p, n);
+  if (p.sp.rem)
+    k_gemm_sum<2, 1, GEMM_PAIR><<<dim3((unsigned)(p.sp.rem * 2 * 4)), dim3(256), 0, s>>>(p.y, p.ldy, p.M, p.N, p.tm, p.tn, GemmRope{}, p.sp);
+  return lr_launch_status();
+}
+// lr_attn_decode_beside_product, arguments checked; LR_E_UNSUPPORTED, nothing launched, where the product is none of 64-row tiles
+int gemm_beside_attention(const AttnItems& a, int hd, int G, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int I, int K,
+                          void* sums, size_t sums_bytes, hipStream_t s) {
+  if (M < GEMM_SCRATCH_FROM || M > 64 || K % 64 || !gemm_reaches(ldx, I, K, GEMM_PAIR)) return LR_E_UNSUPPORTED;
+  const GemmPlan plan = gemm_plan(M, I, K, GEMM_PAIR, sums_bytes);
+  if (plan.tile != 3) return LR_E_UNSUPPORTED;
+  GemmProduct p = gemm_product(3, GEMM_PAIR, x, ldx, w, y, ldy, M, I, K);
+  p.sp = GemmSplit{(float*)sums, plan.full, plan.rem, plan.splits};
+  const bool two = attn_two_groups(a.chunk_max);
+#define LR_PRODUCT(HDV, GV) \
+  if (hd == HDV && G == GV) return two ? attn_beside_gemm<HDV, GV, 2>(a, p, s) : attn_beside_gemm<HDV, GV, 4>(a, p, s);
+  LR_PRODUCT(128, 1) LR_PRODUCT(128, 2) LR_PRODUCT(128, 4) LR_PRODUCT(128, 8)
+  LR_PRODUCT(64, 1) LR_PRODUCT(64, 2) LR_PRODUCT(64, 4) LR_PRODUCT(64, 8)
+#undef LR_PRODUCT
+  return LR_E_UNSUPPORTED;
 }
 
 // x w^T as partial sums [pieces][M][N] in `sums`; LR_E_UNSUPPORTED, nothing launched, where a product of this shape has whole tiles
@@ -1067,4 +1157,37 @@ extern "C" int lr_linear_swiglu_out_scratch(const void* x, int64_t ldx, const vo
 extern "C" int lr_linear_swiglu_out(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K,
                                     void* scratch, size_t scratch_bytes, lr_stream_t stream) {
   return lr_linear_swiglu_out_scratch(x, ldx, w, y, ldy, M, N, K, scratch, scratch_bytes, nullptr, 0, stream);
+}
+
+extern "C" int lr_attn_decode_beside_product(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos, void* y,
+                                             int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch, size_t scratch_bytes,
+                                             void* tickets, const void* x, int64_t ldx, const void* w, void* act, int64_t ld_act, int M, int N,
+                                             int K, void* sums, size_t sums_bytes, lr_stream_t stream) {
+  AttnItems a;
+  int G;
+  const int rc = attn_fill_items(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, tickets, a, G);
+  if (rc != LR_OK && rc != LR_E_UNSUPPORTED) return rc;
+  LR_REQUIRE_PTR(x);
+  LR_REQUIRE_PTR(w);
+  LR_REQUIRE_PTR(act);
+  LR_OPTIONAL_PTR(sums);
+  if (tickets == nullptr) return LR_E_NULL;
+  if (M <= 0 || N <= 0 || K <= 0 || N % 2 || ldx < K || ld_act < N / 2) return LR_E_SHAPE;
+  if (K % 8 || ldx % 8) return LR_E_ALIGN;
+  if (rc != LR_OK || a.tickets == nullptr) return LR_E_UNSUPPORTED;
+  return lr_detail::gemm_beside_attention(a, hd, G, x, ldx, w, act, ld_act, M, N / 2, K, sums, sums ? sums_bytes : 0, (hipStream_t)stream);
+}
+
+extern "C" int lr_linear_pieces_two(const void* x0, const void* w0, int K0, void* sums0, int32_t* pieces0, const void* x1, const void* w1, int K1,
+                                    void* sums1, int32_t* pieces1, int M, int N, size_t sums_bytes, lr_stream_t stream) {
+  LR_REQUIRE_PTR(x0);
+  LR_REQUIRE_PTR(w0);
+  LR_REQUIRE_PTR(sums0);
+  LR_REQUIRE_PTR(x1);
+  LR_REQUIRE_PTR(w1);
+  LR_REQUIRE_PTR(sums1);
+  if (pieces0 == nullptr || pieces1 == nullptr) return LR_E_NULL;
+  if (M <= 0 || N <= 0 || K0 <= 0 || K1 <= 0) return LR_E_SHAPE;
+  if (K0 % 8 || K1 % 8) return LR_E_ALIGN;
+  return lr_detail::gemm_outputs(x0, w0, K0, sums0, pieces0, x1, w1, K1, sums1, pieces1, M, N, sums_bytes, (hipStream_t)stream);
 }

@@ -72,6 +72,11 @@ _PROTOS = {
     "lr_attn_decode_beside_fp8_merged": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int,
                                                  c_int, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p, c_void_p, c_void_p,
                                                  c_int, c_void_p]),
+    "lr_attn_decode_beside_product": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
+                                              c_int, c_int, c_int, c_void_p, c_size_t, c_void_p, c_void_p, c_int64, c_void_p,
+                                              c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]),
+    "lr_linear_pieces_two": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
+                                     c_int, c_int, c_size_t, c_void_p]),
     "lr_attn_decode_static": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
                                       c_int, c_int, c_int, c_void_p]),
     "lr_attn_prefill": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
@@ -601,6 +606,21 @@ def linear_pieces(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, scratch):
     return Pieces(scratch, count.value, M, N)
 
 
+def linear_pieces_two(x0, w0, out0, sums0, x1, w1, out1, sums1):
+    """linear_pieces(x0, w0, out0, sums0) and linear_pieces(x1, w1, out1, sums1), in one launch where that is the faster way
+    (lr_linear_pieces_two)."""
+    (M, K0), (N, K1) = x0.shape, w1.shape
+    assert sums0 is not sums1 and all(t.is_contiguous() for t in (x0, w0, x1, w1)) and x1.shape == (M, K1) and w0.shape == (N, K0)
+    n0, n1 = c_int32(), c_int32()
+    (p0, b0), (p1, b1) = _scratch_args(sums0), _scratch_args(sums1)
+    rc = load().lr_linear_pieces_two(_dev(x0), _dev(w0), K0, p0, ctypes.byref(n0), _dev(x1), _dev(w1), K1, p1, ctypes.byref(n1), M, N,
+                                     min(b0, b1), _stream())
+    if rc == E_UNSUPPORTED:
+        return linear_pieces(x0, w0, out0, sums0), linear_pieces(x1, w1, out1, sums1)
+    _check(rc, "lr_linear_pieces_two")
+    return Pieces(sums0, n0.value, M, N), Pieces(sums1, n1.value, M, N)
+
+
 class _LadderBlock(ctypes.Structure):   # lr_ladder_block_t
     _fields_ = [(n, c_int32) for n in ("B", "S", "dim", "ffn")] + [("eps", c_float), ("rope", _RopeKv)] + \
                [(n, c_void_p) for n in ("x", "xn", "xn2", "qkv", "y", "act", "h", "a", "m", "sums_a", "sums_m")] + [("sums_bytes", c_size_t)] + \
@@ -756,6 +776,26 @@ def attn_decode_beside(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, pro
     if rc == E_UNSUPPORTED:
         return False
     _check(rc, "lr_attn_decode_beside")
+    return True
+
+
+def attn_decode_beside_product(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, tickets, x, w1, act, sums) -> bool:
+    """attn_decode and linear_swiglu_out(x, w1, act, sums=sums) of 33 to 64 rows in one grid; the two must not depend on each
+    other.  False, with nothing launched, when the library has no such kernel for the shape.  tickets: as in attn_decode_beside."""
+    _, _, ldq = _rows_ld(q)
+    _, _, ldy = _rows_ld(y)
+    M, K, ldx = _rows_ld(x)
+    N, Kw = w1.shape
+    Mo, Io, ld_act = _rows_ld(act)
+    assert pos.dtype == torch.int32 and pos.numel() == 1 and scratch.dtype == torch.float32
+    assert w1.is_contiguous() and Kw == K and N % 2 == 0 and (Mo, Io) == (M, N // 2), (x.shape, w1.shape, act.shape)
+    rc = load().lr_attn_decode_beside_product(_dev(q), ldq, _dev(k_cache), _dev(v_cache), pos.data_ptr(), _dev(y), ldy, B, Hq, Hkv,
+                                              hd, k_cache.shape[2], scratch.data_ptr(), scratch.numel() * 4,
+                                              _tickets(tickets, 32 * B * Hq), _dev(x), ldx, _dev(w1), _dev(act), ld_act, M, N, K,
+                                              *_scratch_args(sums), _stream())
+    if rc == E_UNSUPPORTED:
+        return False
+    _check(rc, "lr_attn_decode_beside_product")
     return True
 
 

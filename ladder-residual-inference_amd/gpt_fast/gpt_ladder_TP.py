@@ -157,6 +157,8 @@ class GPTLadder(GPTBase):
         # 70B rank shard, batch 64: 7.6 ms per step, one after the other 10.0 (in bands 9.45 and 9.96); at batch 32 nothing
         # moves (7.35 / 7.31, in bands), below that the attention shares the up/gate launch instead
         two_chains = multi and not beside and ws.B >= self.two_chains_from
+        # up to 64 rows the attention shares a launch with the up/gate product instead, wo one with w2 whose partial sums go to the norms
+        products = two_chains and ws.B <= 64 and ws.tickets is not None and ws.sums is not None and ws.sums is not ws.sums_mlp
         if two_chains:
             cur = torch.cuda.current_stream()
             chain = getattr(self, "_chain_stream", None)
@@ -171,7 +173,22 @@ class GPTLadder(GPTBase):
             if not isinstance(xn, _hip.Normed):
                 _hip.ladder_norms(ws.x, pending_a, pending_m, blk.attention_norm.weight, blk.ffn_norm.weight, ws.x, ws.xn,
                                   ws.xn2, eps)
-            if two_chains:
+            if products:
+                att, ff, kv = blk.attention, blk.feed_forward, blk.attention.kv_cache
+                heads = cfg.n_head_local, cfg.n_kv_local, cfg.head_dim
+                _hip.linear_rope_kv(ws.xn, att.wqkv.weight, ws.qkv, self.freqs_cis, pos, kv.k_cache, kv.v_cache, ws.B, 1, *heads, ws.sums)
+                products = _hip.attn_decode_beside_product(ws.qkv, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, *heads, ws.tickets,
+                                                           ws.xn2, ff.w1.weight, ws.act, ws.sums)
+                if not products:
+                    self._attention(ws, blk, pos, None, ws.a, roped=True)
+                    self._mlp(ws, blk, ws.m, ws.xn2)
+                elif after:
+                    pending_a, pending_m = _hip.linear_pieces_two(ws.y, att.wo.weight, ws.a, ws.sums, ws.act, ff.w2.weight, ws.m, ws.sums_mlp)
+                    continue
+                else:
+                    _hip.linear(ws.y, att.wo.weight, ws.a, scratch=ws.sums)
+                    _hip.linear(ws.act, ff.w2.weight, ws.m, scratch=ws.sums_mlp)
+            elif two_chains:
                 chain.wait_stream(cur)
                 with torch.cuda.stream(chain):
                     self._mlp(ws, blk, ws.m, ws.xn2)

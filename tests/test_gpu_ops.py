@@ -898,6 +898,66 @@ def test_attn_decode_merged_beside_a_projection_equals_the_two_launches(hip, fp8
         assert not bool(tickets.any())
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,hd,Smax,pos,K,I", [
+    (64, 8, 1, 128, 2176, 2100, 2048, 456),      # chunks of four groups of keys, a product in pieces
+    (33, 8, 2, 64, 640, 300, 1024, 17),          # one row more than the bands', one pair of a tile's 64
+    (64, 16, 1, 128, 128, 5, 64, 24000),         # 16 q heads as two groups of 8; whole tiles, more than the chip has CUs
+    (40, 4, 4, 64, 200, 199, 4096, 1000),        # one q head per kv head
+])
+def test_attn_decode_beside_a_product_equals_the_two_calls(hip, B, Hq, Hkv, hd, Smax, pos, K, I):
+    """Tiles, attention items and their merge in one grid: the bits of lr_attn_decode and lr_linear_swiglu_out, launch after launch,
+    the tickets zero again."""
+    q, x = rnd(B, (Hq + 2 * Hkv) * hd, seed=50), rnd(B, K, seed=53)
+    w = rnd(2 * I, K, seed=54, scale=K ** -0.5)
+    p = torch.tensor([pos], dtype=torch.int32, device=DEV)
+    tickets = torch.zeros(32 * B * Hq, dtype=torch.int32, device=DEV)
+    scratch = torch.empty(hip.attn_decode_scratch_bytes(B, Hq, hd, Smax) // 4, dtype=torch.float32, device=DEV)
+    sums = torch.empty(hip.linear_scratch_bytes(B), dtype=torch.uint8, device=DEV)
+    for seed in range(3):
+        kc, vc = rnd(B, Hkv, Smax, hd, seed=60 + seed), rnd(B, Hkv, Smax, hd, seed=80 + seed)
+        y = torch.zeros(2, B, Hq * hd, dtype=BF, device=DEV)
+        act = [torch.full((B, I + 3), 5.0, dtype=BF, device=DEV) for _ in range(2)]
+        hip.attn_decode(q, kc, vc, p, y[0], scratch, B, Hq, Hkv, hd)
+        hip.linear_swiglu_out(x, w, act[0][:, :I], sums=sums)
+        scratch.fill_(float("nan"))
+        sums.fill_(255)
+        assert hip.attn_decode_beside_product(q, kc, vc, p, y[1], scratch, B, Hq, Hkv, hd, tickets, x, w, act[1][:, :I], sums)
+        assert torch.equal(y[1], y[0]) and torch.equal(act[1], act[0]) and bool(y[0].any())
+        assert not bool(tickets.any())
+
+
+def test_attn_decode_beside_a_product_declines_what_it_has_no_kernel_for(hip):
+    """Rows that the bands or larger tiles serve, K of no whole k-tiles, more key chunks than a wave merges: False, nothing launched."""
+    def run(B, K=4096, Smax=64, Hq=8):
+        hd, I = 64, 64
+        kc, vc = rnd(B, 1, Smax, hd, seed=56), rnd(B, 1, Smax, hd, seed=57)
+        y, act = torch.full((B, Hq * hd), 5.0, dtype=BF, device=DEV), torch.full((B, I), 5.0, dtype=BF, device=DEV)
+        scratch = torch.zeros(hip.attn_decode_scratch_bytes(B, Hq, hd, Smax) // 4, dtype=torch.float32, device=DEV)
+        ok = hip.attn_decode_beside_product(rnd(B, Hq * hd, seed=55), kc, vc, torch.tensor([3], dtype=torch.int32, device=DEV), y, scratch, B, Hq, 1,
+                                            hd, torch.zeros(32 * B * Hq, dtype=torch.int32, device=DEV), rnd(B, K, seed=58), rnd(2 * I, K, seed=59),
+                                            act, None)
+        return ok, bool((y == 5.0).all()) and bool((act == 5.0).all())
+    assert run(33)[0] is True
+    for kw in (dict(B=32), dict(B=65), dict(B=33, K=4104), dict(B=33, Smax=17000), dict(B=33, Hq=3)):
+        assert run(**kw) == (False, True), kw
+
+
+@pytest.mark.parametrize("M,N,K0,K1", [(64, 8192, 1024, 3584), (33, 264, 2048, 4096), (128, 2048, 2048, 8192), (64, 2048, 64, 64)])
+def test_linear_pieces_two(hip, M, N, K0, K1):
+    """Two products' partial sums of one grid: their totals, in fp32, against float64."""
+    x, w = [rnd(M, K, seed=90 + K % 7) for K in (K0, K1)], [rnd(N, K, seed=91 + K % 7, scale=K ** -0.5) for K in (K0, K1)]
+    sums = [torch.full((hip.linear_scratch_bytes(M),), 255, dtype=torch.uint8, device=DEV) for _ in range(2)]
+    out = [torch.zeros(M, N, dtype=BF, device=DEV) for _ in range(2)]
+    parts = hip.linear_pieces_two(x[0], w[0], out[0], sums[0], x[1], w[1], out[1], sums[1])
+    for i, p in enumerate(parts):
+        want = x[i].double() @ w[i].double().T
+        if isinstance(p, hip.Pieces):
+            got = sums[i].view(torch.float32)[:p.count * M * N].view(p.count, M, N).double().sum(0)
+            assert ((got - want).abs() <= 1e-5 * want.abs().max()).all()
+        else:
+            assert_close_ulp(p, want.to(BF))
+
+
 def test_attn_decode_beside_declines_what_it_has_no_kernel_for(hip):
     """More than 16 rows, 32 q heads per kv head, or a projection that writes the cache: False, nothing launched."""
     def run(B, Hq, Hkv, epi=None):
