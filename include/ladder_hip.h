@@ -134,7 +134,8 @@ int lr_linear_pieces(const void* x, int64_t ldx, const void* w, int M, int N, in
                      lr_stream_t stream);
 
 /* Two such products of dense rows, x0 [M, K0] w0 [N, K0]^T and x1 [M, K1] w1 [N, K1]^T, in one launch: pieces of about the same
- * length, sums_bytes of memory for either.  LR_E_UNSUPPORTED, with nothing launched, where two launches are the faster way. */
+ * length, sums_bytes of memory for either, from 17 rows on.  LR_E_UNSUPPORTED, with nothing launched, where two launches are the faster
+ * way. */
 int lr_linear_pieces_two(const void* x0, const void* w0, int K0, void* sums0, int32_t* pieces0, const void* x1, const void* w1, int K1,
                          void* sums1, int32_t* pieces1, int M, int N, size_t sums_bytes, lr_stream_t stream);
 
@@ -277,9 +278,9 @@ int lr_attn_decode_beside_merged(const void* q, int64_t ldq, const void* k_cache
                                  size_t scratch_bytes, const lr_projection_t* projection, const lr_row_norm_t* norm,
                                  void* tickets, int M, lr_stream_t stream);
 
-/* lr_attn_decode and, in the same grid, lr_linear_swiglu_out_scratch of 33 to 64 rows: act [M, N / 2] = silu(gate) * up for w [N, K] =
+/* lr_attn_decode and, in the same grid, lr_linear_swiglu_out_scratch of 17 to 64 rows: act [M, N / 2] = silu(gate) * up for w [N, K] =
  * [up; gate] rows, its partial sums in `sums`.  The two must be independent of each other.  Same bits as the two calls.  `tickets` as
- * in lr_attn_decode_beside_merged, not NULL.  LR_E_UNSUPPORTED (nothing launched): other numbers of rows, K % 64 != 0, more than 64 key
+ * in lr_attn_decode_beside_merged, not NULL; up to 32 rows the product is the GEMM's here and the bands' there.  LR_E_UNSUPPORTED (nothing launched): other numbers of rows, K % 64 != 0, more than 64 key
  * chunks, q heads per kv head other than 1, 2, 4, 8, 16, and products that the plan gives other tiles. */
 int lr_attn_decode_beside_product(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos, void* y,
                                   int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch, size_t scratch_bytes,

@@ -262,9 +262,10 @@ __device__ __forceinline__ void attn_partial_item(const u16* __restrict__ q, int
   if (l16 < G) {
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
-      f32x4_t o = acc[d][0] + acc[d][1];
+      f32x4_t o = acc[d][1];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = fabsf(acc[d][2][e]) < INFINITY ? o[e] + acc[d][2][e] : o[e];   // (an infinite V: its weight's parts may be zero or negative)
+      for (int e = 0; e < 4; ++e)   // the small ones first (an infinite V: its weight's parts may be zero or negative)
+        o[e] = acc[d][0][e] + (fabsf(acc[d][2][e]) < INFINITY ? o[e] + acc[d][2][e] : o[e]);
       put(l16, wave * (HD / 4) + d * 16 + l4 * 4, o);
     }
   }

@@ -596,7 +596,7 @@ __global__ __launch_bounds__(256, GEMM_PER_CU(A, BH)) void k_gemm_two(const Gemm
   }
 }
 
-// The attention of a decode step of 33 to 64 sequences and the block's up/gate product, which do not depend on each other in a ladder
+// The attention of a decode step of 17 to 64 sequences and the block's up/gate product, which do not depend on each other in a ladder
 // or a parallel block, in one grid: an attention item (attn_decode_item.h) for every CU, the product's tiles, the other items, the
 // waves that merge them.  Bound: HBM; apart, the attention's items leave the memory idle between their rows' arrival and the next
 // item's request, and the product's workgroups at their ramp and drain.  us per step of the 70B rank shard at 64 rows: the two chains of
@@ -617,7 +617,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_beside_gemm(const AttnItems a, 
 // The cut tiles: a workgroup adds the pieces of 16 rows of a wave's part of one and finishes them.  Bound: memory, mostly the
 // last-level cache, since the pieces were just written; of small products the round trips: so a wave takes a quarter of the
 // columns, up to eight pieces' loads in flight together, summed in order, and a lane finishes eight columns of one row.  (A
-// wave for all columns and four pieces at a time, us: q/k/v of the 70B rank shard at 64 rows, 16 pieces, 7.1 -> @@, up/gate 4.7 -> @@.)
+// wave for all columns and four pieces at a time, us: q/k/v of the 70B rank shard at 64 rows, 16 pieces, 7.1 -> 4.9, up/gate 4.7 -> 4.9.)
 template <int A, int BH, int MODE>
 __global__ __launch_bounds__(256) void k_gemm_sum(u16* __restrict__ y, int64_t ldy, int M, int N, int tm, int tn, const GemmRope rp, const GemmSplit sp) {
   using T = GemmTile<A, BH>;
@@ -721,6 +721,11 @@ constexpr GemmTileCost GEMM_TILES[GEMM_NTILES] = {{8, 2, 1, 1.2f, 0.0f, 0.0f, 0.
                                                   {6, 1, 1, 0.617f, 0.0f, 0.0944f, 0.0f, 0.0f, 4.28f, 0.0f}};
 constexpr size_t GEMM_SCRATCH = (size_t)64 << 20;   // pieces of one round of the largest tiles
 constexpr int GEMM_SCRATCH_FROM = 33;               // rows from which a projection that has memory for pieces is one of this file's
+// and from which the two grids of a decode step are, that hold a product beside the attention or another product: below, the
+// bands of 16 rows leave room for the attention; those of 32 do not, and read their inputs at half the rate (us per step, up/gate, wo
+// and w2 in bands / in these grids, q/k/v in bands: 70B rank shard, 17 rows 6565 / 5240, 32 rows 7020 / 5780; 8B, 17 rows 4190 / 3680,
+// 32 rows 4530 / 3780; 1B, 24 rows at 1900 tokens 1371 / 1101)
+constexpr int GEMM_BESIDE_FROM = 17;
 
 constexpr float GEMM_WEIGHT_BYTES_US = 5.73e6f, GEMM_OUTPUT_BYTES_US = 6.98e6f, GEMM_SUM_US = 4.92f, GEMM_TRIP_US = 0.267f, GEMM_PIECE_BYTES_US = 3.83e6f,
                 GEMM_TWO = 0.157f, GEMM_NORM_PIECE_US = 0.15f;
@@ -904,7 +909,7 @@ static int attn_beside_gemm(const AttnItems& a, const GemmProduct& p, hipStream_
 // lr_attn_decode_beside_product, arguments checked; LR_E_UNSUPPORTED, nothing launched, where the product is none of 64-row tiles
 int gemm_beside_attention(const AttnItems& a, int hd, int G, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int I, int K,
                           void* sums, size_t sums_bytes, hipStream_t s) {
-  if (M < GEMM_SCRATCH_FROM || M > 64 || K % 64 || !gemm_reaches(ldx, I, K, GEMM_PAIR)) return LR_E_UNSUPPORTED;
+  if (M < GEMM_BESIDE_FROM || M > 64 || K % 64 || !gemm_reaches(ldx, I, K, GEMM_PAIR)) return LR_E_UNSUPPORTED;
   const GemmPlan plan = gemm_plan(M, I, K, GEMM_PAIR, sums_bytes);
   if (plan.tile != 3) return LR_E_UNSUPPORTED;
   GemmProduct p = gemm_product(3, GEMM_PAIR, x, ldx, w, y, ldy, M, I, K);
@@ -935,7 +940,7 @@ struct GemmOutputs {
 };
 static GemmOutputs outputs_plan(int M, int N, int K0, int K1, size_t sums_bytes) {
   GemmOutputs best{-1, 1, 1};
-  if (M < GEMM_SCRATCH_FROM || N % 4 || K0 % 64 || K1 % 64 || !gemm_reaches(K0, N, K0, GEMM_PLAIN) || !gemm_reaches(K1, N, K1, GEMM_PLAIN)) return best;
+  if (N % 4 || K0 % 64 || K1 % 64 || !gemm_reaches(K0, N, K0, GEMM_PLAIN) || !gemm_reaches(K1, N, K1, GEMM_PLAIN)) return best;
   const GemmPlan p0 = gemm_plan(M, N, K0, GEMM_PLAIN, sums_bytes), p1 = gemm_plan(M, N, K1, GEMM_PLAIN, sums_bytes);
   if (p0.tile < 0 || p1.tile < 0) return best;
   const float bytes_us = gemm_bytes_us(M, N, K0, GEMM_ROWS) + gemm_bytes_us(M, N, K1, GEMM_ROWS);
@@ -960,10 +965,13 @@ static GemmOutputs outputs_plan(int M, int N, int K0, int K1, size_t sums_bytes)
   }
   return best;
 }
-bool gemm_outputs_pay(int M, int N, int K0, int K1, size_t sums_bytes) { return outputs_plan(M, N, K0, K1, sums_bytes).tile >= 0; }
+bool gemm_outputs_pay(int M, int N, int K0, int K1, size_t sums_bytes) {
+  return M >= GEMM_SCRATCH_FROM && outputs_plan(M, N, K0, K1, sums_bytes).tile >= 0;
+}
 int gemm_outputs(const void* x0, const void* w0, int K0, void* sums0, int* pieces0, const void* x1, const void* w1, int K1, void* sums1, int* pieces1,
                  int M, int N, size_t sums_bytes, hipStream_t s) {
   if (lr_misaligned(sums0) || lr_misaligned(sums1)) return LR_E_ALIGN;
+  if (M < GEMM_BESIDE_FROM) return LR_E_UNSUPPORTED;
   const GemmOutputs p = outputs_plan(M, N, K0, K1, sums_bytes);
   if (p.tile < 0) return LR_E_UNSUPPORTED;
   GemmProduct a = gemm_product(p.tile, GEMM_ROWS, x0, K0, w0, nullptr, 0, M, N, K0), b = gemm_product(p.tile, GEMM_ROWS, x1, K1, w1, nullptr, 0, M, N, K1);

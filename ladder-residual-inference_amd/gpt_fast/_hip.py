@@ -780,7 +780,7 @@ def attn_decode_beside(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, pro
 
 
 def attn_decode_beside_product(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, tickets, x, w1, act, sums) -> bool:
-    """attn_decode and linear_swiglu_out(x, w1, act, sums=sums) of 33 to 64 rows in one grid; the two must not depend on each
+    """attn_decode and linear_swiglu_out(x, w1, act, sums=sums) of 17 to 64 rows in one grid; the two must not depend on each
     other.  False, with nothing launched, when the library has no such kernel for the shape.  tickets: as in attn_decode_beside."""
     _, _, ldq = _rows_ld(q)
     _, _, ldy = _rows_ld(y)

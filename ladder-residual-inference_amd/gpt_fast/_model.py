@@ -70,6 +70,9 @@ class Workspace:
             self.scratch = torch.empty(n, dtype=torch.float32, device=device)
             # attn_decode_beside's (none where they would be zero only once a graph that is being captured is replayed)
             capturing = device.type == "cuda" and torch.cuda.is_current_stream_capturing()
+            # memory for the partial sums of the products that 17 to 32 sequences have beside each other
+            n = 200 << 15 if two_sums and 16 < rows <= _hip.BANDS_TO else 0
+            self.pair_sums = [torch.empty(n, dtype=torch.uint8, device=device) for _ in range(2)] if n else None
             self.tickets = None if capturing else torch.zeros(32 * B * cfg.n_head_local, dtype=torch.int32, device=device)
 
 

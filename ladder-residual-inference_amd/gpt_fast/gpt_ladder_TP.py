@@ -157,8 +157,10 @@ class GPTLadder(GPTBase):
         # 70B rank shard, batch 64: 7.6 ms per step, one after the other 10.0 (in bands 9.45 and 9.96); at batch 32 nothing
         # moves (7.35 / 7.31, in bands), below that the attention shares the up/gate launch instead
         two_chains = multi and not beside and ws.B >= self.two_chains_from
-        # up to 64 rows the attention shares a launch with the up/gate product instead, wo one with w2 whose partial sums go to the norms
-        products = two_chains and ws.B <= 64 and ws.tickets is not None and ws.sums is not None and ws.sums is not ws.sums_mlp
+        # from 17 rows on (q/k/v in bands up to 32) the attention shares a launch with the up/gate product instead, and wo one with w2 whose
+        # partial sums go to the norms
+        pair = ws.pair_sums or (ws.sums, ws.sums_mlp)
+        products = (two_chains or ws.pair_sums is not None) and ws.tickets is not None and pair[0] is not None and pair[0] is not pair[1]
         if two_chains:
             cur = torch.cuda.current_stream()
             chain = getattr(self, "_chain_stream", None)
@@ -176,14 +178,18 @@ class GPTLadder(GPTBase):
             if products:
                 att, ff, kv = blk.attention, blk.feed_forward, blk.attention.kv_cache
                 heads = cfg.n_head_local, cfg.n_kv_local, cfg.head_dim
-                _hip.linear_rope_kv(ws.xn, att.wqkv.weight, ws.qkv, self.freqs_cis, pos, kv.k_cache, kv.v_cache, ws.B, 1, *heads, ws.sums)
+                if ws.sums is None:
+                    rope = _hip.rope_kv_epilogue(self.freqs_cis, pos, kv.k_cache, kv.v_cache, *heads)
+                    _hip.linear_multi((ws.xn, att.wqkv.weight, ws.qkv, rope))
+                else:
+                    _hip.linear_rope_kv(ws.xn, att.wqkv.weight, ws.qkv, self.freqs_cis, pos, kv.k_cache, kv.v_cache, ws.B, 1, *heads, ws.sums)
                 products = _hip.attn_decode_beside_product(ws.qkv, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, *heads, ws.tickets,
-                                                           ws.xn2, ff.w1.weight, ws.act, ws.sums)
+                                                           ws.xn2, ff.w1.weight, ws.act, pair[0])
                 if not products:
                     self._attention(ws, blk, pos, None, ws.a, roped=True)
                     self._mlp(ws, blk, ws.m, ws.xn2)
                 elif after:
-                    pending_a, pending_m = _hip.linear_pieces_two(ws.y, att.wo.weight, ws.a, ws.sums, ws.act, ff.w2.weight, ws.m, ws.sums_mlp)
+                    pending_a, pending_m = _hip.linear_pieces_two(ws.y, att.wo.weight, ws.a, pair[0], ws.act, ff.w2.weight, ws.m, pair[1])
                     continue
                 else:
                     _hip.linear(ws.y, att.wo.weight, ws.a, scratch=ws.sums)

@@ -233,6 +233,39 @@ def test_ladder_decode_of_different_sequences_equals_each_alone(B, fp8):
         assert rel_err(together[b], decode(toks[b:b + 1])[0]) <= REL_TOL, b
 
 
+@pytest.mark.parametrize("B,fp8", [(17, False), (32, False), (33, False), (64, False)])
+@torch.no_grad()
+def test_ladder_decode_of_many_different_sequences_equals_each_alone(B, fp8, monkeypatch):
+    """17 to 64 rows, the attention beside the up/gate product and wo beside w2, or e4m3 bands of up to 16 rows at a time: another
+    sequence in every row, each row's logits those of the sequence decoded alone, replays equal to eager steps."""
+    from gpt_fast import _hip
+    from gpt_fast.quantize import quantize_model_fp8
+
+    model = build("ladder", **dict(WIDER, dim=1024, intermediate_size=8192))
+    if fp8:
+        quantize_model_fp8(model)
+    model.setup_caches(B, 16)
+    beside, launches = _hip.attn_decode_beside_product, []
+    monkeypatch.setattr(_hip, "attn_decode_beside_product", lambda *a: (launches.append(beside(*a)), launches[-1])[1])
+    toks = torch.randint(0, 512, (B, 6), device=DEV, generator=torch.Generator(device=DEV).manual_seed(9))
+    pos = torch.zeros(1, dtype=torch.int32, device=DEV)
+    decode = lambda rows: torch.cat([model(rows[:, t:t + 1].contiguous(), torch.tensor([t], device=DEV)).clone() for t in range(6)], 1)
+    together = decode(toks)
+    assert fp8 or (launches and all(launches))
+    for b in range(0, B, 5):
+        assert rel_err(together[b], decode(toks[b:b + 1])[0]) <= REL_TOL, b
+    decode(toks)
+    idx = toks[:, 5:].contiguous()
+    pos.fill_(5)
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+        out = model(idx, pos)
+    for _ in range(4):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[:, 0], together[:, 5])
+
+
 @pytest.mark.parametrize("family", ["ladder", "dense", "desync", "parallel"])
 @pytest.mark.parametrize("B", [33, 40, 64, 70])
 def test_decode_batches_above_32_run_products_with_partial_sums(family, B):

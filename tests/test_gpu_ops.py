@@ -926,6 +926,25 @@ def test_attn_decode_beside_a_product_equals_the_two_calls(hip, B, Hq, Hkv, hd, 
         assert not bool(tickets.any())
 
 
+@pytest.mark.parametrize("B,K,I", [(17, 64, 8192), (32, 8192, 456), (20, 4096, 1000)])
+def test_attn_decode_beside_a_product_of_up_to_32_rows(hip, B, K, I):
+    """Rows that lr_linear_swiglu_out gives the bands: lr_attn_decode's bits, and the activation of the float64 product (up, gate and
+    silu(gate) are each rounded: one step of any of them is at most 2^-7 of the result)."""
+    Hq, Hkv, hd, Smax, pos = 8, 1, 128, 600, 555
+    q, x, w = rnd(B, (Hq + 2 * Hkv) * hd, seed=50), rnd(B, K, seed=53), rnd(2 * I, K, seed=54, scale=K ** -0.5)
+    kc, vc = rnd(B, Hkv, Smax, hd, seed=60), rnd(B, Hkv, Smax, hd, seed=80)
+    p, tickets = torch.tensor([pos], dtype=torch.int32, device=DEV), torch.zeros(32 * B * Hq, dtype=torch.int32, device=DEV)
+    scratch = torch.empty(hip.attn_decode_scratch_bytes(B, Hq, hd, Smax) // 4, dtype=torch.float32, device=DEV)
+    y, act = torch.zeros(2, B, Hq * hd, dtype=BF, device=DEV), torch.empty(B, I, dtype=BF, device=DEV)
+    hip.attn_decode(q, kc, vc, p, y[0], scratch, B, Hq, Hkv, hd)
+    sums = torch.empty(200 << 15, dtype=torch.uint8, device=DEV)
+    assert hip.attn_decode_beside_product(q, kc, vc, p, y[1], scratch, B, Hq, Hkv, hd, tickets, x, w, act, sums)
+    assert torch.equal(y[0], y[1])
+    u, g = (x.double() @ w.double().T).to(BF).float().chunk(2, 1)
+    want = ((g / (1 + torch.exp(-g))).to(BF).float() * u).to(BF).float()
+    assert ((act.float() - want).abs() <= 2.0 ** -7 * 3 * want.abs() + 2.0 ** -12).all()
+
+
 def test_attn_decode_beside_a_product_declines_what_it_has_no_kernel_for(hip):
     """Rows that the bands or larger tiles serve, K of no whole k-tiles, more key chunks than a wave merges: False, nothing launched."""
     def run(B, K=4096, Smax=64, Hq=8):
@@ -938,15 +957,16 @@ def test_attn_decode_beside_a_product_declines_what_it_has_no_kernel_for(hip):
                                             act, None)
         return ok, bool((y == 5.0).all()) and bool((act == 5.0).all())
     assert run(33)[0] is True
-    for kw in (dict(B=32), dict(B=65), dict(B=33, K=4104), dict(B=33, Smax=17000), dict(B=33, Hq=3)):
+    for kw in (dict(B=16), dict(B=65), dict(B=33, K=4104), dict(B=33, Smax=17000), dict(B=33, Hq=3)):
         assert run(**kw) == (False, True), kw
 
 
-@pytest.mark.parametrize("M,N,K0,K1", [(64, 8192, 1024, 3584), (33, 264, 2048, 4096), (128, 2048, 2048, 8192), (64, 2048, 64, 64)])
+@pytest.mark.parametrize("M,N,K0,K1", [(64, 8192, 1024, 3584), (33, 264, 2048, 4096), (128, 2048, 2048, 8192), (64, 2048, 64, 64),
+                                       (17, 8192, 1024, 3584), (16, 264, 2048, 4096)])
 def test_linear_pieces_two(hip, M, N, K0, K1):
     """Two products' partial sums of one grid: their totals, in fp32, against float64."""
     x, w = [rnd(M, K, seed=90 + K % 7) for K in (K0, K1)], [rnd(N, K, seed=91 + K % 7, scale=K ** -0.5) for K in (K0, K1)]
-    sums = [torch.full((hip.linear_scratch_bytes(M),), 255, dtype=torch.uint8, device=DEV) for _ in range(2)]
+    sums = [torch.full((max(hip.linear_scratch_bytes(M), 200 << 15),), 255, dtype=torch.uint8, device=DEV) for _ in range(2)]
     out = [torch.zeros(M, N, dtype=BF, device=DEV) for _ in range(2)]
     parts = hip.linear_pieces_two(x[0], w[0], out[0], sums[0], x[1], w[1], out[1], sums[1])
     for i, p in enumerate(parts):
