@@ -365,6 +365,18 @@ extern "C" int lr_linear_fp8(const void* x, int64_t ldx, const void* w8, const v
   }
   LR_REQUIRE_PTR(scratch);
   if (scratch_bytes < lr_linear_fp8_scratch_bytes(M, N, K)) return LR_E_SHAPE;
+  if (M <= LR_FP8_PASSES_TO && !lr_misaligned(scales) && ldy % 8 == 0) {   // (a pass begins at a row of its own)
+    // the bands again, in passes of up to 16 rows: four reads of the bytes are fewer than the expansion's read, write and read of
+    // twice as many (us per step expanded / in passes: 70B rank shard, 17 rows 13100 / 6280, 64 rows 16090 / 14230; 8B, 24 rows 9206 / 5087)
+    int rc = LR_OK;
+    for (int r0 = 0, left = (M + 15) / 16; rc == LR_OK && left; --left) {
+      const int rows = (M - r0 + left - 1) / left;
+      const lr_projection_fp8_t one = {xp + (int64_t)r0 * ldx, ldx, w8, scales, yp + (int64_t)r0 * ldy, ldy, N, K, LR_EPI_NONE, nullptr};
+      rc = lr_detail::stream_fp8_multi(&one, nullptr, 1, rows, stream);
+      r0 += rows;
+    }
+    if (rc != LR_E_UNSUPPORTED) return rc;
+  }
   const int64_t n16 = (int64_t)N * K / 16;
   const int grid = (int)((n16 + 255) / 256 < 65535 ? (n16 + 255) / 256 : 65535);
   k_fp8_to_bf16<<<dim3(grid), dim3(256), 0, s>>>(wp, (u16*)scratch, n16);

@@ -169,6 +169,9 @@ class GPTLadder(GPTBase):
         # weight-only e4m3 projections, up to 16 rows: the same two launches per block (lr_linear_fp8_multi)
         multi8 = side is None and fp8 and ws.B <= 16
         beside8 = multi8   # (declined by the library for a single row, where the projections are no bands)
+        # and beyond, the bands' launches for up to 16 rows at a time
+        n = -(-ws.B // 16)
+        parts = [slice(i * ws.B // n, (i + 1) * ws.B // n) for i in range(n)] if side is None and fp8 and 1 < n <= 4 else None
         xn, xn2 = ws.xn, ws.xn2
         resid = ws.resid_sums and (multi or multi8)
         for blk, after in zip(self.layers, [*self.layers[1:], None]):
@@ -241,6 +244,17 @@ class GPTLadder(GPTBase):
                     xn, xn2 = ws.xn, ws.xn2
                     _hip.linear_fp8_multi((ws.y, att.wo.weight, att.wo.scales, ws.a, _hip.EPI_NONE),
                                           (ws.act, ff.w2.weight, ff.w2.scales, ws.m, _hip.EPI_NONE))
+            elif parts:
+                att, ff, kv = blk.attention, blk.feed_forward, blk.attention.kv_cache
+                for r in parts:
+                    rope = _hip.rope_kv_epilogue(self.freqs_cis, pos, kv.k_cache[r], kv.v_cache[r], cfg.n_head_local, cfg.n_kv_local,
+                                                 cfg.head_dim)
+                    _hip.linear_fp8_multi((ws.xn[r], att.wqkv.weight, att.wqkv.scales, ws.qkv[r], rope),
+                                          (ws.xn2[r], ff.w1.weight, ff.w1.scales, ws.act[r], _hip.EPI_SWIGLU))
+                self._attention(ws, blk, pos, None, None, roped=True)
+                for r in parts:
+                    _hip.linear_fp8_multi((ws.y[r], att.wo.weight, att.wo.scales, ws.a[r], _hip.EPI_NONE),
+                                          (ws.act[r], ff.w2.weight, ff.w2.scales, ws.m[r], _hip.EPI_NONE))
             elif side is not None:
                 side.wait_stream(main)
                 with torch.cuda.stream(side):

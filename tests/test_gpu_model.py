@@ -233,7 +233,7 @@ def test_ladder_decode_of_different_sequences_equals_each_alone(B, fp8):
         assert rel_err(together[b], decode(toks[b:b + 1])[0]) <= REL_TOL, b
 
 
-@pytest.mark.parametrize("B,fp8", [(17, False), (32, False), (33, False), (64, False)])
+@pytest.mark.parametrize("B,fp8", [(17, False), (32, False), (33, False), (64, False), (17, True), (40, True), (64, True)])
 @torch.no_grad()
 def test_ladder_decode_of_many_different_sequences_equals_each_alone(B, fp8, monkeypatch):
     """17 to 64 rows, the attention beside the up/gate product and wo beside w2, or e4m3 bands of up to 16 rows at a time: another
