@@ -1073,6 +1073,34 @@ def test_argmax_lowest_index_on_ties(hip):
     assert torch.equal(out[:2], lg3[:, -1, :1003].argmax(-1, keepdim=True).to(torch.int32))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("V", [1, 7, 8, 9, 1003, 8191, 8192, 8200, 65536, 65543, 128256])
+def test_argmax_at_the_edges_of_its_groups(hip, V, dtype):
+    """Whole and partial groups of 8 and rounds of 8192 and 65536 columns; ties, signed zeros, infinities, NaNs (never
+    chosen) and rows without a value above the lowest one."""
+    g = torch.Generator().manual_seed(V)
+    lg = (torch.randint(-40, 40, (9, V), generator=g) / 8).to(dtype)   # (many equal values)
+    lg[1] = -0.0
+    lg[1, V // 2:] = 0.0
+    lg[2] = float("-inf")
+    lg[3] = float("nan")
+    lg[4, ::2] = float("nan")
+    lg[5, V // 3:] = float("inf")
+    lg[6] = float("-inf")
+    lg[6, : V // 2] = float("nan")
+    lg[7, V - 1] = 9.0
+    lg[8, :] = -3.0e38
+    want = torch.argmax(torch.where(lg.isnan(), float("-inf"), lg.double()), -1)
+    want = torch.where(lg.isnan().all(-1), 0, want)
+    want[6] = min(V // 2, V - 1)
+    ld = (V + 15) // 8 * 8
+    padded = torch.full((9, ld), 1e9, dtype=dtype, device=DEV)      # (columns beyond V are not the row's)
+    padded[:, :V] = lg.to(DEV)
+    out = torch.full((9, 1), -7, dtype=torch.int32, device=DEV)
+    hip.argmax(padded[:, :V], out)
+    assert out.flatten().tolist() == want.tolist()
+
+
 def test_torch_argmax_itself_returns_first_maximum_on_this_device():
     """The oracle's greedy() relies on it."""
     lg = torch.zeros(1, 16032, dtype=BF, device=DEV)
