@@ -160,7 +160,7 @@ class GPTLadder(GPTBase):
         # from 17 rows on (q/k/v in bands up to 32) the attention shares a launch with the up/gate product instead, and wo one with w2 whose
         # partial sums go to the norms
         pair = ws.pair_sums or (ws.sums, ws.sums_mlp)
-        products = (two_chains or ws.pair_sums is not None) and ws.tickets is not None and pair[0] is not None and pair[0] is not pair[1]
+        products = multi and (two_chains or ws.pair_sums is not None) and ws.tickets is not None and pair[0] is not None and pair[0] is not pair[1]
         if two_chains:
             cur = torch.cuda.current_stream()
             chain = getattr(self, "_chain_stream", None)

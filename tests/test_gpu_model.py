@@ -266,6 +266,33 @@ def test_ladder_decode_of_many_different_sequences_equals_each_alone(B, fp8, mon
         assert torch.equal(out[:, 0], together[:, 5])
 
 
+@pytest.mark.parametrize("B", [17, 32, 40])
+@torch.no_grad()
+def test_a_step_of_many_rows_follows_what_the_model_has_become(B, monkeypatch):
+    """Buffers are kept from step to step: a model that is quantised, or told to overlap its modules, between two steps takes
+    the route that a model takes which never was anything else."""
+    from gpt_fast import _hip
+    from gpt_fast.quantize import quantize_model_fp8
+
+    launches = []
+    beside = _hip.attn_decode_beside_product
+    monkeypatch.setattr(_hip, "attn_decode_beside_product", lambda *a: (launches.append(beside(*a)), launches[-1])[1])
+    toks = torch.randint(0, 512, (B, 1), device=DEV, generator=torch.Generator(device=DEV).manual_seed(4))
+    pos = torch.zeros(1, dtype=torch.int32, device=DEV)
+    fresh, model = (build("ladder", **dict(WIDER, dim=1024, intermediate_size=8192)) for _ in range(2))
+    for m in (fresh, model):
+        m.setup_caches(B, 16)
+    plain = model(toks, pos).clone()
+    assert launches and all(launches)
+    launches.clear()
+    model.overlap_modules = True
+    assert rel_err(model(toks, pos), plain) <= REL_TOL and not launches
+    model.overlap_modules = False
+    quantize_model_fp8(model)
+    quantize_model_fp8(fresh)
+    assert torch.equal(model(toks, pos), fresh(toks, pos)) and not launches
+
+
 @pytest.mark.parametrize("family", ["ladder", "dense", "desync", "parallel"])
 @pytest.mark.parametrize("B", [33, 40, 64, 70])
 def test_decode_batches_above_32_run_products_with_partial_sums(family, B):
