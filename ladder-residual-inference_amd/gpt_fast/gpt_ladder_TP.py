@@ -65,6 +65,9 @@ class GPTLadder(GPTBase):
     def _prompt_pieces(self):
         return self.config.ladder_layers is None and not hasattr(self.layers[0].attention.wqkv, "scales")   # (lr_ladder_block's)
 
+    def _pair_sums(self):
+        return 2 if self._prompt_pieces() else 0
+
     def _make_block(self, config, layer_idx):
         return LadderTransformerBlock(config)
 
@@ -160,7 +163,7 @@ class GPTLadder(GPTBase):
         # from 17 rows on (q/k/v in bands up to 32) the attention shares a launch with the up/gate product instead, and wo one with w2 whose
         # partial sums go to the norms
         pair = ws.pair_sums or (ws.sums, ws.sums_mlp)
-        products = multi and (two_chains or ws.pair_sums is not None) and ws.tickets is not None and pair[0] is not None and pair[0] is not pair[1]
+        products = multi and (two_chains or ws.pair_sums) and ws.tickets is not None and pair[0] is not None and pair[0] is not pair[1]
         if two_chains:
             cur = torch.cuda.current_stream()
             chain = getattr(self, "_chain_stream", None)

@@ -44,6 +44,9 @@ class GPTParallel(GPTBase):
     def _fused_width(self) -> int:
         return super()._fused_width() + 2 * self.config.ffn_local
 
+    def _pair_sums(self):
+        return 0 if hasattr(self.layers[0].attention.wqkv1, "scales") else 1
+
     def _products(self, B, S):
         nqkv = GPTBase._fused_width(self)
         for rows, N, K, pair in super()._products(B, S):
@@ -74,15 +77,17 @@ class GPTParallel(GPTBase):
     def _run_layers_decode(self, ws: Workspace, pos: Tensor, nqkv: int):
         """Decode step through the weight-streaming bands.  The rows of the fused input weight are two projections
         of the same input: [q | k | v], rotated and cached on the way out, and [up | gate], stored as silu(gate) * up
-        -- the second independent of the attention, so up to 16 sequences its bands share the attention's launch
-        (lr_attn_decode_beside) and above that the q/k/v launch; wo and w2 share a launch.  Up to 16 sequences that launch
-        also updates the residual and leaves the next block its rows undivided (linear_resid): four launches per block
-        instead of nine; above, and in the last block, y + x is left to the next norm launch (x + y: the same sum), six.
-        Above 32 sequences each projection is a product of its own, with partial sums."""
+        -- the second independent of the attention, whose launch it shares: up to 16 sequences as bands (lr_attn_decode_beside),
+        above that as a product with partial sums (lr_attn_decode_beside_product; 8B, us per step, bands and an attention of its
+        own before it: 20 sequences 4330 -> 4020, 32 4810 -> 4520; 48 4640 -> 4140).  wo and w2 share a launch.  Up to 16
+        sequences that launch also updates the residual and leaves the next block its rows undivided (linear_resid): three
+        launches per block instead of nine; above, and in the last block, y + x is left to the next norm launch (x + y: the same
+        sum), six.  Above 32 sequences q/k/v, wo and w2 too are products of their own, with partial sums."""
         cfg = self.config
         Hq, Hkv, hd = cfg.n_head_local, cfg.n_kv_local, cfg.head_dim
         q = ws.qkv[:, :nqkv]
         pending, xn, xu = None, ws.xn, ws.xn
+        products = ws.tickets is not None   # from 17 sequences on, where the library has the grid for the shape
         for blk, after in zip(self.layers, [*self.layers[1:], None]):
             att, kv = blk.attention, blk.attention.kv_cache
             if xn is ws.xn:
@@ -93,14 +98,24 @@ class GPTParallel(GPTBase):
             up_gate = (xu, w[nqkv:], ws.act, _hip.EPI_SWIGLU)
             if ws.B > self.band_rows_to:
                 _hip.linear_rope_kv(ws.xn, w[:nqkv], q, self.freqs_cis, pos, kv.k_cache, kv.v_cache, ws.B, 1, Hq, Hkv, hd, ws.sums)
-                _hip.linear_swiglu_out(ws.xn, w[nqkv:], ws.act, sums=ws.sums)
-                _hip.attn_decode(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd)
+                products = products and _hip.attn_decode_beside_product(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd,
+                                                                        ws.tickets, ws.xn, w[nqkv:], ws.act, ws.sums)
+                if not products:
+                    _hip.linear_swiglu_out(ws.xn, w[nqkv:], ws.act, sums=ws.sums)
+                    _hip.attn_decode(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd)
                 _hip.linear(ws.y, att.wo.weight, ws.a, scratch=ws.sums)
                 _hip.linear(ws.act, att.w2.weight, ws.m, scratch=ws.sums)
             elif ws.B <= 16:
                 _hip.linear_multi(qkv)
                 if not _hip.attn_decode_beside(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd, up_gate,
                                                ws.tickets):
+                    _hip.linear_multi(up_gate)
+                    _hip.attn_decode(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd)
+            elif ws.pair_sums and products:
+                _hip.linear_multi(qkv)
+                products = _hip.attn_decode_beside_product(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd, ws.tickets,
+                                                           ws.xn, w[nqkv:], ws.act, ws.pair_sums[0])
+                if not products:
                     _hip.linear_multi(up_gate)
                     _hip.attn_decode(q, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, Hq, Hkv, hd)
             else:

@@ -266,6 +266,37 @@ def test_ladder_decode_of_many_different_sequences_equals_each_alone(B, fp8, mon
         assert torch.equal(out[:, 0], together[:, 5])
 
 
+@pytest.mark.parametrize("B", [17, 32, 33, 64])
+@pytest.mark.parametrize("declined", [False, True])
+@torch.no_grad()
+def test_parallel_decode_of_many_different_sequences_equals_each_alone(B, declined, monkeypatch):
+    """17 to 64 rows, the attention beside the up/gate product (or, where the library declines, after it): another sequence in
+    every row, each row's logits those of the sequence decoded alone, replays equal to eager steps."""
+    from gpt_fast import _hip
+
+    model = build("parallel", **dict(WIDER, dim=1024, intermediate_size=8192))
+    model.setup_caches(B, 16)
+    beside, launches = _hip.attn_decode_beside_product, []
+    monkeypatch.setattr(_hip, "attn_decode_beside_product", lambda *a: (launches.append(not declined and beside(*a)), launches[-1])[1])
+    toks = torch.randint(0, 512, (B, 6), device=DEV, generator=torch.Generator(device=DEV).manual_seed(9))
+    pos = torch.zeros(1, dtype=torch.int32, device=DEV)
+    decode = lambda rows: torch.cat([model(rows[:, t:t + 1].contiguous(), torch.tensor([t], device=DEV)).clone() for t in range(6)], 1)
+    together = decode(toks)
+    assert launches and (declined or all(launches))
+    for b in range(0, B, 5):
+        assert rel_err(together[b], decode(toks[b:b + 1])[0]) <= REL_TOL, b
+    decode(toks)
+    idx = toks[:, 5:].contiguous()
+    pos.fill_(5)
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+        out = model(idx, pos)
+    for _ in range(4):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[:, 0], together[:, 5])
+
+
 @pytest.mark.parametrize("B", [17, 32, 40])
 @torch.no_grad()
 def test_a_step_of_many_rows_follows_what_the_model_has_become(B, monkeypatch):
