@@ -5,7 +5,9 @@
 // A wave owns R rows; KSPLIT waves of the workgroup share a row group and split K between them.
 // Partial sums are combined by a wave64 butterfly and then, across the KSPLIT waves, through LDS
 // in a fixed order -- no atomics, so results are bit-reproducible run to run.
-// x (a few KiB) is re-read by every wave and lives in L1/L2.
+// x (a few KiB) is re-read by every wave and lives in L1/L2; the weights, used once, take no room there (non-temporal
+// loads).  us of one row, ordinary / non-temporal loads: 128256 x 2048 87.6 / 78.2 (6.7 TB/s), 128256 x 4096 174.4 / 153.8
+// (6.8), 28672 x 4096 39.7 / 36.2, 4096 x 14336 21.6 / 19.5, 6144 x 4096 10.4 / 9.6; two rows of 128256 x 4096 166 / 148.
 #include "lr_common.h"
 
 constexpr int GEMV_WPB = 4;  // waves per workgroup
@@ -82,7 +84,7 @@ __global__ __launch_bounds__(GEMV_WPB * 64) void k_gemv(const u16* __restrict__ 
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int r = 0; r < R; ++r) wv[u][r] = ld16(wrow[r] + k + u * KSTEP);
+      for (int r = 0; r < R; ++r) wv[u][r] = ld16_once(wrow[r] + k + u * KSTEP);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       uint4 xp[M];
@@ -94,7 +96,7 @@ __global__ __launch_bounds__(GEMV_WPB * 64) void k_gemv(const u16* __restrict__ 
   for (; k < K; k += KSTEP) {
     uint4 wv[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) wv[r] = ld16(wrow[r] + k);
+    for (int r = 0; r < R; ++r) wv[r] = ld16_once(wrow[r] + k);
     uint4 xp[M];
     load_x<M, SWIGLU>(x, ldx, K, k, m_real, xp);
     mac8<M, R>(wv, xp, acc);

@@ -44,6 +44,11 @@ __device__ __forceinline__ u32 pack_bf2(float lo, float hi) {
 __device__ __forceinline__ float round_bf(float f) { return bf_to_f(f_to_bf(f)); }
 
 __device__ __forceinline__ uint4 ld16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
+// The same for what a launch reads once (non-temporal: it takes no room in the caches).
+__device__ __forceinline__ uint4 ld16_once(const void* p) {
+  const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
 // The same through pointers the compiler cannot trace back to a kernel argument (read from a table, chosen between
 // two sources): stated to be global memory.  A generic ("flat") access could also target LDS, so it counts as an
 // LDS operation as well, may complete out of order, and while one is pending every wait the compiler inserts
