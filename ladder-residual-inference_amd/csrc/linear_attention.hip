@@ -494,7 +494,7 @@ __global__ __launch_bounds__(256) void k_gla_log_decay(const T* __restrict__ low
 }
 
 // ---------------------------------------------------------------------------------------------- decode
-template <typename T, int V>
+template <typename T, int V, bool ONCE>
 __global__ __launch_bounds__(1024) void k_linear_attention_step(const LinAttn a) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int bh = blockIdx.x, b = bh / a.H, h = bh - b * a.H, tid = threadIdx.x, nt = blockDim.x;
@@ -516,8 +516,9 @@ __global__ __launch_bounds__(1024) void k_linear_attention_step(const LinAttn a)
       const int c = r + u * nrow;
       const float* src = st + (on && c < dk ? c * dv : 0);
       if constexpr (V == 4) {
-        const float4 t = *reinterpret_cast<const float4*>(src);
-        s[u][0] = t.x; s[u][1] = t.y; s[u][2] = t.z; s[u][3] = t.w;
+        const f32x4_t t = ld_state4<ONCE>(src);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[u][j] = t[j];
       } else {
         s[u][0] = *src;
       }
@@ -725,9 +726,12 @@ int step(const LinAttn& a, hipStream_t s) {
   nt = nt < 64 ? 64 : (nt > 1024 ? 1024 : nt);
   const size_t lds = sizeof(float) * ((size_t)3 * a.dk + (size_t)(nt / nq) * a.dv + 4);
   if (v == 4) {
-    k_linear_attention_step<T, 4><<<dim3(a.B * a.H), dim3(nt), lds, s>>>(a);
+    if ((size_t)a.B * a.H * a.dk * a.dv * sizeof(float) > STATE_CACHED_MAX)
+      k_linear_attention_step<T, 4, true><<<dim3(a.B * a.H), dim3(nt), lds, s>>>(a);
+    else
+      k_linear_attention_step<T, 4, false><<<dim3(a.B * a.H), dim3(nt), lds, s>>>(a);
   } else {
-    k_linear_attention_step<T, 1><<<dim3(a.B * a.H), dim3(nt), lds, s>>>(a);
+    k_linear_attention_step<T, 1, false><<<dim3(a.B * a.H), dim3(nt), lds, s>>>(a);
   }
   return lr_launch_status();
 }

@@ -44,6 +44,15 @@ __device__ __forceinline__ u32 pack_bf2(float lo, float hi) {
 __device__ __forceinline__ float round_bf(float f) { return bf_to_f(f_to_bf(f)); }
 
 __device__ __forceinline__ uint4 ld16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
+// Recurrent states of up to this many bytes per layer are found in the caches by the next token's step; larger ones are not, and are
+// read without taking room there (non-temporal).  us per step, ordinary / non-temporal: Lasivik 8B (2 MiB per sequence) 1 sequence
+// 3208 / 3231, 2 3540 / 3554, 4 3680 / 3635, 16 4196 / 4135, 64 6158 / 6070; Lasivik 1B 2 sequences (2 MiB) 920 / 930; Gepolix 8B 6 sequences
+// (12 MiB) 3816 / 3777, 16 4713 / 4610, 64 8300 / 8255; Gepolix 1B 16 sequences (16 MiB) 1163 / 1122.
+constexpr size_t STATE_CACHED_MAX = (size_t)6 << 20;
+template <bool ONCE>
+__device__ __forceinline__ f32x4_t ld_state4(const float* p) {
+  return ONCE ? __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(p)) : *reinterpret_cast<const f32x4_t*>(p);
+}
 // The same for what a launch reads once (non-temporal: it takes no room in the caches).
 __device__ __forceinline__ uint4 ld16_once(const void* p) {
   const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));

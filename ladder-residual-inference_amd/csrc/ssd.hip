@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256) void k_ssd_walk(const Ssd a) {
 
 // ---------------------------------------------------------------------------------------------- one token
 // 256 threads: four columns each, the rows of S side by side.  Everything from memory is asked for before anything is used.
-template <typename T, int TAPS>
+template <typename T, int TAPS, bool ONCE = false>
 __global__ __launch_bounds__(256) void k_ssd_step(const Ssd a) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int bh = blockIdx.x, b = bh / a.H, h = bh - b * a.H, hpg = a.H / a.G, g = h / hpg, tid = threadIdx.x;
@@ -232,7 +232,8 @@ __global__ __launch_bounds__(256) void k_ssd_step(const Ssd a) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int n = r + u * nrow;
-      s[u] = *reinterpret_cast<const float4*>(st + (on && n < N ? (int64_t)n * P : 0));
+      const f32x4_t t = ld_state4<ONCE>(st + (on && n < N ? (int64_t)n * P : 0));
+      s[u] = make_float4(t[0], t[1], t[2], t[3]);
     }
   };
   load(r0);
@@ -849,7 +850,9 @@ extern "C" int lr_ssd_step(const lr_ssd_t* d, const void* conv_w, const void* co
   const size_t lds = sizeof(float) * ((size_t)a.P + 2 * a.N + (256 / (a.P / 4)) * a.P);
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid(a.B * a.H), blk(256);
+  const size_t state_bytes = sizeof(float) * (size_t)a.B * a.H * a.N * a.P;
   if (d->dtype == LR_F32) k_ssd_step<float, 0><<<grid, blk, lds, s>>>(a);
+  else if (taps == 4 && state_bytes > STATE_CACHED_MAX) k_ssd_step<u16, 4, true><<<grid, blk, lds, s>>>(a);
   else if (taps == 4) k_ssd_step<u16, 4><<<grid, blk, lds, s>>>(a);
   else k_ssd_step<u16, 0><<<grid, blk, lds, s>>>(a);
   return lr_launch_status();

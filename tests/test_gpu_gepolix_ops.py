@@ -209,6 +209,27 @@ def test_ssd_step_with_its_convolution(hip, dtype, H, G, N, P, taps):
     close(c.state, S, dtype, scale=1.0 if dtype == F32 else 0.1)
 
 
+@pytest.mark.parametrize("B", [3, 4])
+def test_ssd_step_reads_states_of_any_size_alike(hip, B):
+    """2 MiB of state per sequence: at most 6 MiB and more are read in different ways, with the bits of a sequence alone."""
+    H, G, N, P, taps = 64, 1, 128, 64, 4
+    c = Ssm(B, 1, H, G, N, P, BF)
+    Cc = c.u.shape[-1]
+    w, b = rnd(Cc, taps, seed=8, dtype=BF), rnd(Cc, seed=9, dtype=BF)
+    state, ring = rnd(B, H, N, P, seed=10), rnd(B, taps, Cc, seed=11, dtype=BF)
+
+    def step(rows):
+        S, R = state[rows].clone(), ring[rows].clone()
+        n = S.shape[0]
+        rest, y = c.rest[rows].reshape(n, -1).contiguous(), torch.empty(n, H * P, dtype=BF, device=DEV)
+        hip.ssd_step(rest[:, :H * P], c.u[rows].reshape(n, -1).contiguous(), rest[:, H * P:], w, b, R, *c.heads, at_pos(9, 1), S, y, n, H, G)
+        return S, R, y
+
+    together = step(slice(0, B))
+    for i in range(B):
+        assert all(torch.equal(a[i], t[0]) for a, t in zip(together, step(slice(i, i + 1))))
+
+
 @pytest.mark.parametrize("dtype", [F32, BF])
 @pytest.mark.parametrize("heads,P,PP,parts", [(4, 16, 16, 1), (4, 16, 16, 4), (4, 9, 16, 3), (6, 24, 32, 2), (64, 64, 64, 8), (3, 7, 16, 7)])
 def test_parts_norm(hip, dtype, heads, P, PP, parts):

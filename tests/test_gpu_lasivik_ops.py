@@ -223,6 +223,26 @@ def test_linear_attention_sizes(hip, H, dk, dv, gated, dtype):
     close(c.state[:2], S, F32 if dtype == F32 else BF, "state", 4)
 
 
+@pytest.mark.parametrize("B", [3, 4])
+@pytest.mark.parametrize("gated", [True, False])
+def test_linear_attention_step_reads_states_of_any_size_alike(hip, B, gated):
+    """2 MiB of state per sequence: at most 6 MiB and more are read in different ways, with the bits of a sequence alone."""
+    H, dk, dv = 16, 128, 256
+    c = LinearCase(B, 1, H, dk, dv, gated, BF, decay=[0.5 + 0.03 * h for h in range(H)])
+    state = rnd(B, H, dk, dv, seed=10)
+
+    def step(rows):
+        S = state[rows].clone()
+        y = torch.empty(S.shape[0], H * dv, dtype=BF, device=DEV)
+        hip.linear_attention(c.proj[rows].contiguous(), y, S, torch.tensor([9], dtype=torch.int32, device=DEV), S.shape[0], 1, H, dk, dv, 1e-5,
+                             **c.kw)
+        return S, y
+
+    together = step(slice(0, B))
+    for i in range(B):
+        assert all(torch.equal(a[i], t[0]) for a, t in zip(together, step(slice(i, i + 1))))
+
+
 @pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("cuts", [[1], [2], [15], [16], [17], [2, 3, 12, 16, 1, 1, 17, 2], [31, 33, 32, 1, 63], [130, 200, 2]])
 def test_linear_attention_portions(hip, cuts, gated):
