@@ -1,4 +1,5 @@
-// Matrix-core bf16 GEMMs for prefill, decode batches above 64 rows, and from 33 rows on where there is memory for partial sums:
+// Matrix-core bf16 GEMMs for prefill, decode batches above 64 rows, and from 33 rows on where there is memory for partial sums
+// (from 17 in the grids that a decode step's blocks share, lr_attn_decode_beside_product and lr_linear_pieces_two):
 //   y[m, n] = bf16( sum_k x[m, k] * w[n, k] ),  fp32 accumulation.
 // k_gemm_dma (below) is the one that matters; k_gemm here serves an input that is activated on its way in, and rows longer
 // than the 2 GiB offsets of k_gemm_dma's requests reach.

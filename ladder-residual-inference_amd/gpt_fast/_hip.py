@@ -593,7 +593,7 @@ def linear_swiglu_out(x: torch.Tensor, w1: torch.Tensor, act: torch.Tensor, scra
 def linear_pieces(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, scratch):
     """linear(x, w, out, scratch=scratch), or its partial sums (Pieces in `scratch`, out untouched) where no tile is computed whole.
     For blocks that a caller puts together itself: the models' prompts leave pieces inside lr_ladder_block, and their decode steps
-    add them in launches of their own (w2's sums then run beside the attention: 70B rank shard, 64 rows: 7611 us per step, 7718 with them left to the norms)."""
+    take both output products' together (linear_pieces_two)."""
     M, xc, ldx = _rows_ld(x)
     N, K = w.shape
     assert w.is_contiguous() and xc == K and tuple(out.shape) == (M, N)

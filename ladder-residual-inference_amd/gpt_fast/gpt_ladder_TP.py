@@ -137,7 +137,9 @@ class GPTLadder(GPTBase):
         attention output), then the attention chain (wqkv, RoPE + cache write, attention, wo) and the MLP chain
         (w1, SwiGLU, w2) -- one after the other, or on two streams where the reference overlaps an all-reduce with
         the next module (gpt_ladder_TP.py:339-349).  Up to 16 rows the norms launch is only the first block's: from then on
-        the output projections update the residual and leave the next block its rows undivided (linear_resid)."""
+        the output projections update the residual and leave the next block its rows undivided (linear_resid).  17 to 64
+        rows on bf16 weights share a grid between the attention and the up/gate product, and leave both outputs' partial
+        sums to the norms; on e4m3 weights they are passes of up to 16 rows."""
         cfg = self.config
         eps = cfg.norm_eps
         main = side = None
@@ -155,13 +157,14 @@ class GPTLadder(GPTBase):
         fp8 = hasattr(self.layers[0].attention.wqkv, "scales")
         multi = side is None and ws.B <= 64 and not fp8
         beside = multi and ws.B <= 16
-        # Above 32 rows the projections are products with partial sums, whose launches leave room: the MLP chain (up/gate,
-        # w2) runs as a second branch of the captured graph beside the attention chain (q/k/v, attention, wo) --
-        # 70B rank shard, batch 64: 7.6 ms per step, one after the other 10.0 (in bands 9.45 and 9.96); at batch 32 nothing
-        # moves (7.35 / 7.31, in bands), below that the attention shares the up/gate launch instead
+        # Above 32 rows the projections are products with partial sums, whose launches leave room.  Where the attention cannot share
+        # a grid with the up/gate product (below), the MLP chain (up/gate, w2) runs as a second branch of the captured graph beside
+        # the attention chain (q/k/v, attention, wo) -- 70B rank shard, batch 64: 7.6 ms per step, one after the other 10.0; up to 32
+        # rows, in bands, nothing moves (batch 32 7.35 / 7.31)
         two_chains = multi and not beside and ws.B >= self.two_chains_from
-        # from 17 rows on (q/k/v in bands up to 32) the attention shares a launch with the up/gate product instead, and wo one with w2 whose
-        # partial sums go to the norms
+        # from 17 rows on (q/k/v in bands up to 32) the attention shares a grid with the up/gate product, and wo one with w2, both with
+        # their partial sums left to the norms -- 70B rank shard, 64 rows at 2048 tokens: 6.59 ms per step, on two branches 7.13; 32
+        # rows at 1000 tokens 5.78, in bands 7.02
         pair = ws.pair_sums or (ws.sums, ws.sums_mlp)
         products = multi and (two_chains or ws.pair_sums) and ws.tickets is not None and pair[0] is not None and pair[0] is not pair[1]
         if two_chains:
