@@ -46,8 +46,8 @@ __device__ __forceinline__ float round_bf(float f) { return bf_to_f(f_to_bf(f));
 __device__ __forceinline__ uint4 ld16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
 // Recurrent states of up to this many bytes per layer are found in the caches by the next token's step; larger ones are not, and are
 // read without taking room there (non-temporal).  us per step, ordinary / non-temporal: Lasivik 8B (2 MiB per sequence) 1 sequence
-// 3208 / 3231, 2 3540 / 3554, 4 3680 / 3635, 16 4196 / 4135, 64 6158 / 6070; Lasivik 1B 2 sequences (2 MiB) 920 / 930; Gepolix 8B 6 sequences
-// (12 MiB) 3816 / 3777, 16 4713 / 4610, 64 8300 / 8255; Gepolix 1B 16 sequences (16 MiB) 1163 / 1122.
+// 3208 / 3231, 2 3540 / 3554, 4 3680 / 3635, 16 4196 / 4135, 64 6158 / 6070; Lasivik 1B 2 sequences (2 MiB) 920 / 930; Gepolix 8B (4 MiB per
+// sequence) 6 sequences 3816 / 3777, 16 4713 / 4610, 64 8300 / 8255; Gepolix 1B (2 MiB) 16 sequences 1163 / 1122.
 constexpr size_t STATE_CACHED_MAX = (size_t)6 << 20;
 template <bool ONCE>
 __device__ __forceinline__ f32x4_t ld_state4(const float* p) {
