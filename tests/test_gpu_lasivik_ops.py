@@ -45,6 +45,28 @@ def close(got, want, dtype, what="", scale=1.0):
 d64 = lambda t: t.detach().cpu().to(F64)
 
 
+# ------------------------------------------------------------------------------------------------ projections
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("N,K", [(256, 256), (264, 256), (256, 264), (4608, 256), (6152, 256), (1003, 40)])
+def test_projections_of_few_rows_by_either_kernel(hip, rows, N, K, monkeypatch):
+    """On both sides of the lines between the matrix-vector kernel and the bands (N = K and N = 6 rows K), strided outputs."""
+    from gpt_fast.mixers import project
+
+    calls = []
+    multi = hip.linear_multi
+    monkeypatch.setattr(hip, "linear_multi", lambda *a: (calls.append(1), multi(*a))[1])
+    lin = torch.nn.Linear(K, N, bias=False, dtype=BF, device=DEV)
+    lin.weight.data.copy_(rnd(N, K, seed=1).to(BF))
+    x = rnd(rows, K, seed=2, dtype=BF)
+    out = torch.full((rows, N + 13 - N % 8 + 8), float("nan"), dtype=BF, device=DEV)[:, :(N + 7) // 8 * 8]
+    with torch.no_grad():
+        project(x, lin, out[:, :N])
+    close(out[:, :N], d64(x) @ d64(lin.weight).T, BF)
+    assert torch.isnan(out[:, N:].float()).all()
+    assert bool(calls) == (rows > 1 and not (rows == 2 and N > K or rows <= 4 and N > 6 * rows * K))
+
+
 # ------------------------------------------------------------------------------------------------ residual stream
 
 @pytest.mark.parametrize("dtype", [F32, BF])
