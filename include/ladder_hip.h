@@ -271,8 +271,10 @@ int lr_attn_decode_beside_normed(const void* q, int64_t ldq, const void* k_cache
                                  void* y, int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch,
                                  size_t scratch_bytes, const lr_projection_t* projection, const lr_row_norm_t* norm, int M,
                                  lr_stream_t stream);
-/* The same with the attention's chunk results merged inside the launch instead of in a second one: the same bits.  `tickets`: 32 * B * Hq uint32 on the device, zero before the first call and left zero
- * by every call (calls that may overlap have their own); NULL: two launches.  norm may be NULL. */
+/* The same with the attention's chunk results merged inside the launch instead of in a second one: the same bits.  `tickets`: 32 * B * Hq
+ * uint32 on the device, zero before the first call (calls that may overlap have their own); NULL: two launches.  norm may be NULL.
+ * Of every 32 words the first is zero again after a call.  The second may be set by the caller: n > 0 has the merging waves look n - 1 times for
+ * the chunks before they hand their part over to the workgroup that stores the last one (0: about a millisecond's worth); the third counts the parts handed over. */
 int lr_attn_decode_beside_merged(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos,
                                  void* y, int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch,
                                  size_t scratch_bytes, const lr_projection_t* projection, const lr_row_norm_t* norm,

@@ -330,30 +330,40 @@ __global__ __launch_bounds__(HD) void k_attn_decode_combine_once(const float* __
   y[(int64_t)b * ldy + h * HD + d] = f_to_bf(L > 0.0f ? o / L : 0.0f);
 }
 
-// The same inside the launch of the items, by waves of workgroups that stand behind them in the grid: whoever runs has seen all
-// items start, and an item waits for nobody, so the wait below ends (it is bounded all the same).  An item counts its
-// kv head's ticket up when the memory side has acknowledged its results (attn_item_done), and a wave reads them from there
-// (sc0 sc1): 64 outputs, all of up to 64 chunks' in one round trip.  The last of a kv head's waves sets the ticket back to zero.
+// The same inside the launch of the items, by waves of workgroups that stand behind them in the grid.  An item counts its
+// kv head's chunks up when the memory side has acknowledged its results (attn_item_done), and a wave reads them from there
+// (sc0 sc1): 64 outputs, all of up to 64 chunks' in one round trip.
+//
+// A wave waits for the chunks, an item for nobody.  Workgroups are dealt to the XCDs in turn and every XCD starts its own in
+// order: a wave that runs has seen the items of its XCD start, those of another may still stand behind a projection's workgroups there,
+// or behind the waiting waves of a second grid whose items stand behind this one's.  So a wave that has looked ATT_MERGE_LOOKS times
+// (about a millisecond, where 20 us are usual) hands its part over and ends; the item that stores the last chunk merges what was handed over.  One
+// word decides which of the two it is, whatever the order: bits 0 to 7 chunks stored, 8 to 15 parts merged, 16 to 31 parts handed
+// over.  A wave that sets its bit sees in the same operation whether all chunks are there -- then the last item has gone by, and
+// the part is still its own; the last item sees in its own the bits set before it.  Whoever merges a kv head's last part sets the word to zero: nobody
+// looks at it any more.
 constexpr int ATT_MERGE_MAX = 64;   // chunks
-constexpr int ATT_TICKET = 32;      // words from one kv head's ticket to the next: 128 bytes
-__device__ __forceinline__ void attn_item_done(u32* ticket) {
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  if (threadIdx.x == 0) (void)__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+constexpr int ATT_TICKET = 32;      // words from one kv head's to the next: 128 bytes
+constexpr u32 ATT_MERGE_LOOKS = 512;
+// the other words of a kv head's: [1] n > 0: n - 1 looks instead; [2] parts handed over so far
+__device__ __forceinline__ u32 attn_look(u32* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// one lane adds; the value before, in every lane
+__device__ __forceinline__ u32 attn_count(u32* p, u32 n) {
+  u32 was = 0;
+  if ((threadIdx.x & 63) == 0) was = __hip_atomic_fetch_add(p, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return __builtin_amdgcn_readfirstlane(was);
 }
-// `wave`: which 64 of the outputs [B][Hq * HD].  A merge in a launch of its own is 4.7 us per block
+
+// `part`: which 64 of the outputs [B][Hq * HD].  A merge in a launch of its own is 4.7 us per block
 // and step; here it ends before the weight stream does (70B rank shard, 8 rows: chunks stored at 6 us of 23, merged at 20).
 // What did not do: all of a head's outputs by whoever stores its last chunk (131 KB of 32 chunks through one CU beside its part of the
 // stream: the launch 2.5 us longer); tickets in one cache line, polled without a pause (the polls queue before the items' counts: e4m3,
 // 5 rows, the whole stream 12 -> 17 us).
-template <int HD, int G>
-__device__ __forceinline__ void attn_merge_wave(const float* __restrict__ o_part, const float* __restrict__ ml_part, u32* tickets, u16* __restrict__ y,
-                                                int64_t ldy, int Hkv, int nsplit, int wave) {
-  const int lane = threadIdx.x & 63, Hq = Hkv * G;
-  const int head = wave / (HD / 64), b = head / Hq, h = head - b * Hq, d = wave % (HD / 64) * 64 + lane;   // (head: of all sequences)
-  u32* const ticket = tickets + head / G * ATT_TICKET;
-  for (int i = 0; __hip_atomic_load(ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < (u32)nsplit && i < 1 << 16; ++i) __builtin_amdgcn_s_sleep(40);
-  asm volatile("" ::: "memory");
+template <int HD>
+__device__ __forceinline__ void attn_merge_part(const float* __restrict__ o_part, const float* __restrict__ ml_part, u16* __restrict__ y, int64_t ldy,
+                                                int Hq, int nsplit, int part) {
+  const int lane = threadIdx.x & 63;
+  const int head = part / (HD / 64), b = head / Hq, h = head - b * Hq, d = part % (HD / 64) * 64 + lane;   // (head: of all sequences)
   const __amdgpu_buffer_rsrc_t ores = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(o_part + (int64_t)head * nsplit * HD), 0, nsplit * HD * 4, 0x00020000);
   const __amdgpu_buffer_rsrc_t mres = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(ml_part + (int64_t)head * nsplit * 2), 0, nsplit * 8, 0x00020000);
   // (a chunk beyond the last lies outside the resource and reads as zero)
@@ -378,11 +388,50 @@ __device__ __forceinline__ void attn_merge_wave(const float* __restrict__ o_part
       }
   }
   y[(int64_t)b * ldy + h * HD + d] = f_to_bf(L > 0.0f ? o / L : 0.0f);
-  if (lane == 0) {
-    const u32 last = (u32)(nsplit + G * (HD / 64) - 1);
-    if (__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == last)
-      __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <int HD, int G>
+__device__ __forceinline__ void attn_merged(u32* ticket, u32 parts) {
+  if ((attn_count(ticket, parts << 8) >> 8 & 255) + parts == G * (HD / 64) && (threadIdx.x & 63) == 0)
+    __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <int HD, int G>
+__device__ __forceinline__ void attn_merge_wave(const float* __restrict__ o_part, const float* __restrict__ ml_part, u32* tickets, u16* __restrict__ y,
+                                                int64_t ldy, int Hkv, int nsplit, int part) {
+  constexpr int PARTS = G * (HD / 64);
+  static_assert(PARTS <= 16 && ATT_MERGE_MAX < 256, "fields of a ticket");
+  u32* const ticket = tickets + part / PARTS * ATT_TICKET;
+  const u32 limit = attn_look(ticket + 1), looks = limit ? limit - 1 : ATT_MERGE_LOOKS;
+  u32 seen = attn_look(ticket);
+  for (u32 i = 0; (seen & 255) < (u32)nsplit && i < looks; ++i) {
+    __builtin_amdgcn_s_sleep(40);
+    seen = attn_look(ticket);
   }
+  if ((seen & 255) < (u32)nsplit) {
+    if ((threadIdx.x & 63) == 0) seen = __hip_atomic_fetch_or(ticket, 1u << (16 + part % PARTS), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((__builtin_amdgcn_readfirstlane(seen) & 255) < (u32)nsplit) {
+      attn_count(ticket + 2, 1);
+      return;
+    }
+  }
+  asm volatile("" ::: "memory");
+  attn_merge_part<HD>(o_part, ml_part, y, ldy, Hkv * G, nsplit, part);
+  attn_merged<HD, G>(ticket, 1);
+}
+// The end of an item of kv head `group` of all sequences'.
+template <int HD, int G>
+__device__ __forceinline__ void attn_item_done(const float* __restrict__ o_part, const float* __restrict__ ml_part, u32* tickets, u16* __restrict__ y,
+                                               int64_t ldy, int Hkv, int nsplit, int group) {
+  constexpr int PARTS = G * (HD / 64);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  u32* const ticket = tickets + group * ATT_TICKET;
+  const u32 was = attn_count(ticket, 1), handed = was >> 16;
+  if ((was & 255) + 1 < (u32)nsplit || handed == 0) return;
+  asm volatile("" ::: "memory");
+  for (int i = 0; i < PARTS; ++i)
+    if (handed >> i & 1) attn_merge_part<HD>(o_part, ml_part, y, ldy, Hkv * G, nsplit, group * PARTS + i);
+  attn_merged<HD, G>(ticket, __builtin_popcount(handed));
 }
 
 template <int HD>
@@ -419,7 +468,7 @@ __device__ __forceinline__ void attn_item(const AttnItems& a, int wg, float* sme
   const int split = wg % a.nsplit, rest = wg / a.nsplit;
   attn_partial_item<HD, G, GROUPS, MERGE>(a.q, a.ldq, a.kc, a.vc, a.pos, a.o_part, a.ml_part, a.Hkv, a.Smax, a.nsplit,
                                           a.chunk_max, split, rest % a.Hkv, rest / a.Hkv, smem, a.kv_share);
-  if constexpr (MERGE) attn_item_done(a.tickets + rest * ATT_TICKET);
+  if constexpr (MERGE) attn_item_done<HD, G>(a.o_part, a.ml_part, a.tickets, a.y, a.ldy, a.Hkv, a.nsplit, rest);
 }
 template <int HD, int G>
 __device__ __forceinline__ void attn_merge(const AttnItems& a, int wg) {

@@ -763,7 +763,7 @@ def attn_decode(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd):
 def attn_decode_beside(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, projection, tickets=None) -> bool:
     """attn_decode and linear_multi(projection) in one launch (lr_attn_decode_beside); the two must not depend
     on each other.  False, with nothing launched, when the library has no such kernel for the shape.  tickets: 32 B Hq
-    int32, zero and left zero (None: the chunk results are merged by a launch of their own)."""
+    int32, zero before the first call and no overlapping call's (None: the chunk results are merged by a launch of their own)."""
     _, _, ldq = _rows_ld(q)
     _, _, ldy = _rows_ld(y)
     Smax = k_cache.shape[2]

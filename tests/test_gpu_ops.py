@@ -863,6 +863,7 @@ def test_attn_decode_beside_fp8_equals_the_two_calls(hip, B, Hq, Hkv, hd, Smax, 
     assert bool((o1 == 5.0).all()) and bool((y1 == 5.0).all())
 
 
+@pytest.mark.parametrize("looks", [0, 1, 3])   # the library's own number; a merging wave that does not wait at all; one that looks twice
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("B,Hq,Hkv,hd,Smax,pos", [
     (8, 8, 1, 128, 2176, 2100),      # 32 chunks, the whole first round trip
@@ -873,9 +874,10 @@ def test_attn_decode_beside_fp8_equals_the_two_calls(hip, B, Hq, Hkv, hd, Smax, 
     (4, 8, 2, 64, 40, 0),            # one chunk, one key
     (2, 8, 1, 128, 20000, 19000),    # more chunks than the merge inside the launch takes: a launch of its own
 ])
-def test_attn_decode_merged_beside_a_projection_equals_the_two_launches(hip, fp8, B, Hq, Hkv, hd, Smax, pos):
-    """The chunks merged by whoever stores a kv head's last one: the bits of the merge in a launch of its own, launch after
-    launch, with scratch of NaN (nothing is read that this call has not written), and the tickets zero again."""
+def test_attn_decode_merged_beside_a_projection_equals_the_two_launches(hip, looks, fp8, B, Hq, Hkv, hd, Smax, pos):
+    """The chunks merged by waves at the end of the grid, or, where these do not wait for them, by the item that stores a kv head's
+    last one: the bits of the merge in a launch of its own, launch after launch, with scratch of NaN (nothing is read that this
+    call has not written), and the tickets zero again."""
     D, I = 272, 72
     q = rnd(B, (Hq + 2 * Hkv) * hd, seed=50)
     p = torch.tensor([pos], dtype=torch.int32, device=DEV)
@@ -885,7 +887,8 @@ def test_attn_decode_merged_beside_a_projection_equals_the_two_launches(hip, fp8
         proj, beside, alone = (x, *O.quantize_fp8_rowwise(w, BF)), hip.attn_decode_beside_fp8, hip.linear_fp8_multi
     else:
         proj, beside, alone = (x, w.to(BF)), hip.attn_decode_beside, hip.linear_multi
-    tickets = torch.zeros(32 * B * Hq, dtype=torch.int32, device=DEV)
+    tickets = torch.zeros(B * Hq, 32, dtype=torch.int32, device=DEV)
+    tickets[:, 1] = looks
     scratch = torch.empty(hip.attn_decode_scratch_bytes(B, Hq, hd, Smax) // 4, dtype=torch.float32, device=DEV)
     for seed in range(4):
         kc, vc = rnd(B, Hkv, Smax, hd, seed=60 + seed), rnd(B, Hkv, Smax, hd, seed=80 + seed)
@@ -895,22 +898,25 @@ def test_attn_decode_merged_beside_a_projection_equals_the_two_launches(hip, fp8
         scratch.fill_(float("nan"))
         assert beside(q, kc, vc, p, y[1], scratch, B, Hq, Hkv, hd, (*proj, out[1], hip.EPI_SWIGLU), tickets)
         assert torch.equal(y[1], y[0]) and torch.equal(out[1], out[0]) and bool(y[0].any())
-        assert not bool(tickets.any())
+        assert not bool(tickets[:, 0].any())
+    assert looks != 1 or Smax == 20000 or bool(tickets[:, 2].any())   # (an item takes microseconds: some waves were earlier)
 
 
+@pytest.mark.parametrize("looks", [0, 1, 3])
 @pytest.mark.parametrize("B,Hq,Hkv,hd,Smax,pos,K,I", [
     (64, 8, 1, 128, 2176, 2100, 2048, 456),      # chunks of four groups of keys, a product in pieces
     (33, 8, 2, 64, 640, 300, 1024, 17),          # one row more than the bands', one pair of a tile's 64
     (64, 16, 1, 128, 128, 5, 64, 24000),         # 16 q heads as two groups of 8; whole tiles, more than the chip has CUs
     (40, 4, 4, 64, 200, 199, 4096, 1000),        # one q head per kv head
 ])
-def test_attn_decode_beside_a_product_equals_the_two_calls(hip, B, Hq, Hkv, hd, Smax, pos, K, I):
-    """Tiles, attention items and their merge in one grid: the bits of lr_attn_decode and lr_linear_swiglu_out, launch after launch,
-    the tickets zero again."""
+def test_attn_decode_beside_a_product_equals_the_two_calls(hip, looks, B, Hq, Hkv, hd, Smax, pos, K, I):
+    """Tiles, attention items and their merge in one grid, with and without a wait for the items: the bits of lr_attn_decode and
+    lr_linear_swiglu_out, launch after launch, the tickets zero again."""
     q, x = rnd(B, (Hq + 2 * Hkv) * hd, seed=50), rnd(B, K, seed=53)
     w = rnd(2 * I, K, seed=54, scale=K ** -0.5)
     p = torch.tensor([pos], dtype=torch.int32, device=DEV)
-    tickets = torch.zeros(32 * B * Hq, dtype=torch.int32, device=DEV)
+    tickets = torch.zeros(B * Hq, 32, dtype=torch.int32, device=DEV)
+    tickets[:, 1] = looks
     scratch = torch.empty(hip.attn_decode_scratch_bytes(B, Hq, hd, Smax) // 4, dtype=torch.float32, device=DEV)
     sums = torch.empty(hip.linear_scratch_bytes(B), dtype=torch.uint8, device=DEV)
     for seed in range(3):
@@ -923,7 +929,7 @@ def test_attn_decode_beside_a_product_equals_the_two_calls(hip, B, Hq, Hkv, hd, 
         sums.fill_(255)
         assert hip.attn_decode_beside_product(q, kc, vc, p, y[1], scratch, B, Hq, Hkv, hd, tickets, x, w, act[1][:, :I], sums)
         assert torch.equal(y[1], y[0]) and torch.equal(act[1], act[0]) and bool(y[0].any())
-        assert not bool(tickets.any())
+        assert not bool(tickets[:, 0].any())
 
 
 @pytest.mark.parametrize("B,K,I", [(17, 64, 8192), (32, 8192, 456), (20, 4096, 1000)])
