@@ -911,7 +911,14 @@ static int attn_beside_gemm(const AttnItems& a, const GemmProduct& p, hipStream_
 int gemm_beside_attention(const AttnItems& a, int hd, int G, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int I, int K,
                           void* sums, size_t sums_bytes, hipStream_t s) {
   if (M < GEMM_BESIDE_FROM || M > 64 || K % 64 || !gemm_reaches(ldx, I, K, GEMM_PAIR)) return LR_E_UNSUPPORTED;
-  const GemmPlan plan = gemm_plan(M, I, K, GEMM_PAIR, sums_bytes);
+  GemmPlan plan = gemm_plan(M, I, K, GEMM_PAIR, sums_bytes);
+  // Of two numbers of pieces that take a product alone as long the smaller: what it leaves is the attention's (70B rank shard, 17 to 24 rows,
+  // three pieces or four, a product alone 30.9 us: 24 layers 1629 to 1677 and 1662 to 1711 us).
+  for (const float best = plan.us; plan.tile == 3 && plan.rem;) {
+    const GemmPlan fewer = gemm_plan(M, I, K, GEMM_PAIR, (size_t)plan.rem * plan.splits * GemmTile<2, 1>::TM * GemmTile<2, 1>::TN * sizeof(float) - 1);
+    if (fewer.tile != 3 || fewer.us > 1.003f * best) break;
+    plan = fewer;
+  }
   if (plan.tile != 3) return LR_E_UNSUPPORTED;
   GemmProduct p = gemm_product(3, GEMM_PAIR, x, ldx, w, y, ldy, M, I, K);
   p.sp = GemmSplit{(float*)sums, plan.full, plan.rem, plan.splits};
@@ -965,6 +972,11 @@ static GemmOutputs outputs_plan(int M, int N, int K0, int K1, size_t sums_bytes)
       }
   }
   return best;
+}
+// Bytes for either of the two with which the plan is that of all the memory it could ask for; 0: two launches.
+static size_t outputs_bytes(int M, int N, int K0, int K1) {
+  const GemmOutputs p = M < GEMM_BESIDE_FROM ? GemmOutputs{-1, 1, 1} : outputs_plan(M, N, K0, K1, GEMM_SCRATCH);
+  return p.tile < 0 ? 0 : (size_t)M * N * sizeof(float) * (p.s0 > p.s1 ? p.s0 : p.s1);
 }
 bool gemm_outputs_pay(int M, int N, int K0, int K1, size_t sums_bytes) {
   return M >= GEMM_SCRATCH_FROM && outputs_plan(M, N, K0, K1, sums_bytes).tile >= 0;
@@ -1185,6 +1197,10 @@ extern "C" int lr_attn_decode_beside_product(const void* q, int64_t ldq, const v
   if (K % 8 || ldx % 8) return LR_E_ALIGN;
   if (rc != LR_OK || a.tickets == nullptr) return LR_E_UNSUPPORTED;
   return lr_detail::gemm_beside_attention(a, hd, G, x, ldx, w, act, ld_act, M, N / 2, K, sums, sums ? sums_bytes : 0, (hipStream_t)stream);
+}
+
+extern "C" size_t lr_linear_pieces_two_bytes(int M, int N, int K0, int K1) {
+  return M <= 0 || N <= 0 || K0 <= 0 || K1 <= 0 || K0 % 8 || K1 % 8 ? 0 : lr_detail::outputs_bytes(M, N, K0, K1);
 }
 
 extern "C" int lr_linear_pieces_two(const void* x0, const void* w0, int K0, void* sums0, int32_t* pieces0, const void* x1, const void* w1, int K1,

@@ -75,6 +75,7 @@ _PROTOS = {
     "lr_attn_decode_beside_product": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
                                               c_int, c_int, c_int, c_void_p, c_size_t, c_void_p, c_void_p, c_int64, c_void_p,
                                               c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]),
+    "lr_linear_pieces_two_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
     "lr_linear_pieces_two": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                                      c_int, c_int, c_size_t, c_void_p]),
     "lr_attn_decode_static": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
@@ -619,6 +620,15 @@ def linear_pieces_two(x0, w0, out0, sums0, x1, w1, out1, sums1):
         return linear_pieces(x0, w0, out0, sums0), linear_pieces(x1, w1, out1, sums1)
     _check(rc, "lr_linear_pieces_two")
     return Pieces(sums0, n0.value, M, N), Pieces(sums1, n1.value, M, N)
+
+
+def linear_pieces_two_bytes(M, N, K0, K1) -> int:
+    return int(load().lr_linear_pieces_two_bytes(M, N, K0, K1))
+
+
+def beside_product_bytes(M, N, K) -> int:
+    """Bytes beyond which attn_decode_beside_product's plan for w1 [N, K] does not change."""
+    return linear_plan(M, N, K, True, linear_scratch_bytes(BANDS_TO + 1)).sums_bytes if K % 64 == 0 else 0
 
 
 class _LadderBlock(ctypes.Structure):   # lr_ladder_block_t

@@ -23,7 +23,7 @@ class Workspace:
     """Activation buffers for one (batch, seq) shape, all bf16 [rows, *]."""
 
     def __init__(self, cfg: ModelArgs, B: int, S: int, fused_width: int, device, dtype, smax: int, all_logits: bool,
-                 sums_bytes: int, two_sums: bool = False, pair_sums: int = 0):
+                 sums_bytes: int, two_sums: bool = False, pair_bytes: tuple = ()):
         rows = B * S
         D, hd = cfg.dim, cfg.head_dim
         e = lambda *shape: torch.empty(*shape, dtype=dtype, device=device)
@@ -70,9 +70,11 @@ class Workspace:
             self.scratch = torch.empty(n, dtype=torch.float32, device=device)
             # attn_decode_beside's (none where they would be zero only once a graph that is being captured is replayed)
             capturing = device.type == "cuda" and torch.cuda.is_current_stream_capturing()
-            # memory for the partial sums of the products that 17 to 32 sequences have beside each other or beside the attention
-            n = pair_sums if 16 < rows <= _hip.BANDS_TO else 0
-            self.pair_sums = [torch.empty(200 << 15, dtype=torch.uint8, device=device) for _ in range(n)]
+            # memory for the partial sums of the products that 17 to 64 sequences have beside each other or beside the attention: what is
+            # here already where that is enough
+            have = (self.sums, self.sums_mlp) if self.sums is not self.sums_mlp else (self.sums, None)
+            self.pair_sums = [m if m is not None and m.numel() >= n else torch.empty(max(n, 256), dtype=torch.uint8, device=device)
+                              for m, n in zip(have, pair_bytes)]
             self.tickets = None if capturing else torch.zeros(32 * B * cfg.n_head_local, dtype=torch.int32, device=device)
 
 
@@ -141,9 +143,9 @@ class GPTBase(nn.Module):
         """Do a prompt's output projections leave partial sums to the next norms, which takes memory for both?"""
         return False
 
-    def _pair_sums(self) -> int:
-        """Memories for partial sums that a decode step of 17 to 32 sequences holds (Workspace.pair_sums)."""
-        return 0
+    def _pair_bytes(self, B: int) -> tuple:
+        """Bytes of the memories for partial sums that the shared grids of a decode step of B sequences take (Workspace.pair_sums)."""
+        return ()
 
     def _check_caches(self, max_seq_length):
         cfg = self.config
@@ -193,7 +195,8 @@ class GPTBase(nn.Module):
 
     def _new_workspace(self, B: int, S: int):
         return Workspace(self.config, B, S, self._fused_width(), self.output.weight.device, self.norm.weight.dtype,
-                         self.max_seq_length, not self.last_logits_only, self._sums_bytes(B, S), self._prompt_pieces(), self._pair_sums())
+                         self.max_seq_length, not self.last_logits_only, self._sums_bytes(B, S), self._prompt_pieces(),
+                         self._pair_bytes(B) if S == 1 and 16 < B <= 64 else ())
 
     def _products(self, B: int, S: int):
         """(rows, N, K, pair) of every bf16 projection of a (B, S) step, as linear_sums_bytes takes them."""

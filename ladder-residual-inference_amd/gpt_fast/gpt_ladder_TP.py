@@ -65,8 +65,12 @@ class GPTLadder(GPTBase):
     def _prompt_pieces(self):
         return self.config.ladder_layers is None and not hasattr(self.layers[0].attention.wqkv, "scales")   # (lr_ladder_block's)
 
-    def _pair_sums(self):
-        return 2 if self._prompt_pieces() else 0
+    def _pair_bytes(self, B):
+        if not self._prompt_pieces():
+            return ()
+        c = self.config
+        outputs = _hip.linear_pieces_two_bytes(B, c.dim, c.n_head_local * c.head_dim, c.ffn_local)
+        return max(outputs, _hip.beside_product_bytes(B, 2 * c.ffn_local, c.dim)), outputs
 
     def _make_block(self, config, layer_idx):
         return LadderTransformerBlock(config)
@@ -165,8 +169,8 @@ class GPTLadder(GPTBase):
         # from 17 rows on (q/k/v in bands up to 32) the attention shares a grid with the up/gate product, and wo one with w2, both with
         # their partial sums left to the norms -- 70B rank shard, 64 rows at 2048 tokens: 6.59 ms per step, on two branches 7.13; 32
         # rows at 1000 tokens 5.78, in bands 7.02
-        pair = ws.pair_sums or (ws.sums, ws.sums_mlp)
-        products = multi and (two_chains or ws.pair_sums) and ws.tickets is not None and pair[0] is not None and pair[0] is not pair[1]
+        pair = ws.pair_sums
+        products = multi and pair and (two_chains or ws.sums is None) and ws.tickets is not None
         if two_chains:
             cur = torch.cuda.current_stream()
             chain = getattr(self, "_chain_stream", None)

@@ -44,8 +44,10 @@ class GPTParallel(GPTBase):
     def _fused_width(self) -> int:
         return super()._fused_width() + 2 * self.config.ffn_local
 
-    def _pair_sums(self):
-        return 0 if hasattr(self.layers[0].attention.wqkv1, "scales") else 1
+    def _pair_bytes(self, B):
+        if B > _hip.BANDS_TO or hasattr(self.layers[0].attention.wqkv1, "scales"):
+            return ()
+        return (_hip.beside_product_bytes(B, 2 * self.config.ffn_local, self.config.dim),)
 
     def _products(self, B, S):
         nqkv = GPTBase._fused_width(self)

@@ -387,6 +387,27 @@ def test_partial_sums_of_the_mlp_are_limited_where_that_was_measured(lib, family
     assert ws.sums_mlp.numel() == (min(ws.sums.numel(), 200 << 15) if B <= 64 else ws.sums.numel())
 
 
+@pytest.mark.parametrize("family", ["ladder", "parallel"])
+@pytest.mark.parametrize("name", ["ladder-1b", "ladder-8b", "ladder-70b-tp8", "ladder-405b-tp8"])
+@pytest.mark.parametrize("B", [16, 17, 32, 33, 64, 65])
+def test_shared_grids_of_a_decode_step_hold_the_memory_that_their_products_can_use(lib, family, name, B):
+    """The up/gate product beside the attention, and in a ladder block wo beside w2: divided as with all the memory they could ask for."""
+    from gpt_fast import _hip
+
+    model = meta_model(family, name)
+    c, ws = model.config, model._new_workspace(B, 1)
+    if B in (16, 65) or (family, B > 32) == ("parallel", True):
+        assert ws.pair_sums == []
+        return
+    held = [t.numel() for t in ws.pair_sums]
+    up = (B, 2 * c.ffn_local, c.dim, True)
+    assert bytes(_hip.linear_plan(*up, scratch_bytes=held[0])) == bytes(_hip.linear_plan(*up, scratch_bytes=64 << 20))
+    if family == "ladder":
+        two = lib.lr_linear_pieces_two_bytes(B, c.dim, c.n_head_local * c.head_dim, c.ffn_local)
+        assert len(held) == 2 and ws.pair_sums[0] is not ws.pair_sums[1] and 0 < two <= min(held)
+    assert max(held) <= 16 << 20
+
+
 def test_swiglu_projection_of_many_rows_refuses_what_its_two_calls_refuse(lib):
     """More than 64 rows on a small grid are specified as lr_linear into `scratch` and lr_swiglu: scratch of the projection's
     size, multiples of 8 columns, and no more rows than lr_swiglu takes -- with memory for partial sums or without."""
