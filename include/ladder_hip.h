@@ -134,7 +134,7 @@ int lr_linear_pieces(const void* x, int64_t ldx, const void* w, int M, int N, in
                      lr_stream_t stream);
 
 /* Two such products of dense rows, x0 [M, K0] w0 [N, K0]^T and x1 [M, K1] w1 [N, K1]^T, in one launch: pieces of about the same
- * length, sums_bytes of memory for either, from 17 rows on.  LR_E_UNSUPPORTED, with nothing launched, where two launches are the faster
+ * length, sums_bytes of memory for either (LR_E_SHAPE: of which some is both's), from 17 rows on.  LR_E_UNSUPPORTED, with nothing launched, where two launches are the faster
  * way.  lr_linear_pieces_two_bytes: the sums_bytes beyond which nothing changes; 0: two launches whatever the memory. */
 size_t lr_linear_pieces_two_bytes(int M, int N, int K0, int K1);
 int lr_linear_pieces_two(const void* x0, const void* w0, int K0, void* sums0, int32_t* pieces0, const void* x1, const void* w1, int K1,

@@ -1214,5 +1214,7 @@ extern "C" int lr_linear_pieces_two(const void* x0, const void* w0, int K0, void
   if (pieces0 == nullptr || pieces1 == nullptr) return LR_E_NULL;
   if (M <= 0 || N <= 0 || K0 <= 0 || K1 <= 0) return LR_E_SHAPE;
   if (K0 % 8 || K1 % 8) return LR_E_ALIGN;
+  const uintptr_t s0 = (uintptr_t)sums0, s1 = (uintptr_t)sums1;
+  if ((s0 > s1 ? s0 - s1 : s1 - s0) < sums_bytes) return LR_E_SHAPE;   // (both are written at the same time)
   return lr_detail::gemm_outputs(x0, w0, K0, sums0, pieces0, x1, w1, K1, sums1, pieces1, M, N, sums_bytes, (hipStream_t)stream);
 }

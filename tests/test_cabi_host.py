@@ -569,6 +569,61 @@ def test_ladder_block_and_pieces_refuse_what_they_cannot_serve(lib):
     assert norms(p1=-1) == -3 and norms(d1=None, p1=2) == -1 and norms(d2=None, p2=2) == -1 and norms(p1=2, p2=3) == -2
 
 
+def test_two_products_of_one_launch_refuse_what_they_cannot_serve(lib):
+    """Memory that both would write among it; what two launches serve is declined."""
+    n0, n1 = ctypes.c_int32(), ctypes.c_int32()
+
+    def two(x0=256, w0=256, K0=1024, sums0=1 << 30, n0=ctypes.byref(n0), x1=256, w1=256, K1=1024, sums1=2 << 30, n1=ctypes.byref(n1), M=64, N=64,
+            size=1 << 20):
+        return lib.lr_linear_pieces_two(x0, w0, K0, sums0, n0, x1, w1, K1, sums1, n1, M, N, size, None)
+
+    for name in ("x0", "w0", "sums0", "n0", "x1", "w1", "sums1", "n1"):
+        assert two(**{name: None}) == -1, name
+    for name in ("x0", "w0", "sums0", "x1", "w1", "sums1"):
+        assert two(**{name: 264}) == -2, name
+    for name in ("M", "N", "K0", "K1"):
+        assert two(**{name: 0}) == -3, name
+    assert two(K0=1028) == -2 and two(K1=1028) == -2
+    assert two(sums1=1 << 30) == -3 and two(sums1=(1 << 30) + (1 << 20) - 256) == -3 and two(sums1=(1 << 30) - 256) == -3
+    assert two(M=16) == -4 and two(N=66) == -4 and two(K0=1032) == -4 and two(size=0) == -4
+    assert lib.lr_linear_pieces_two_bytes(16, 64, 1024, 1024) == 0 == lib.lr_linear_pieces_two_bytes(64, 66, 1024, 1024)
+    assert lib.lr_linear_pieces_two_bytes(64, 0, 1024, 1024) == 0 == lib.lr_linear_pieces_two_bytes(64, 64, 1028, 1024)
+
+
+@pytest.mark.parametrize("entry", ["beside_merged", "beside_fp8_merged", "beside_product"])
+def test_attention_in_a_shared_launch_refuses_what_its_own_launch_refuses(lib, entry):
+    """lr_attn_decode's arguments and the tickets; what is not for these grids is declined."""
+    from gpt_fast import _hip
+
+    proj = _hip._ProjectionFp8 if "fp8" in entry else _hip._Projection
+    p = proj(**{**{"w8" if "fp8" in entry else "w": 256}, **dict(x=256, y=256, ldx=64, ldy=64, N=64, K=64, epilogue=0), **(dict(scales=256) if "fp8" in entry else {})})
+
+    def rc(q=256, ldq=1024, k=256, v=256, pos=256, y=256, ldy=1024, B=32, Hq=8, Hkv=1, hd=128, Smax=64, scratch=256, n=1 << 24, tickets=256, M=16,
+           K=64):
+        a = q, ldq, k, v, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, n
+        if entry == "beside_product":
+            return lib.lr_attn_decode_beside_product(*a, tickets, 256, 64, 256, 256, 64, 2 * M, 128, K, 256, 1 << 20, None)
+        return getattr(lib, "lr_attn_decode_" + entry)(*a, ctypes.cast(ctypes.byref(p), ctypes.c_void_p), None, tickets, M, None)
+
+    for name in ("q", "k", "v", "y", "scratch", "pos"):
+        assert rc(**{name: None}) == -1, name
+    for name in ("q", "k", "v", "y", "scratch"):
+        assert rc(**{name: 264}) == -2, name
+    for name in ("B", "Hq", "Hkv", "hd", "Smax", "M"):
+        assert rc(**{name: 0}) == -3, name
+    assert rc(ldq=1016) == -3 and rc(ldy=1016) == -3 and rc(ldq=1028) == -2 and rc(ldy=1028) == -2 and rc(Hkv=3) == -3 and rc(n=16) == -3
+    assert rc(B=65536) == -3 and rc(tickets=258) == -2
+    assert rc(M=33) == -4 and rc(Hq=3, Hkv=1) == -4 and rc(hd=96) == -4
+    if entry == "beside_product":
+        assert rc(tickets=None) == -1 and rc(K=4) == -2 and rc(K=72, M=16) == -3 and rc(Smax=17000, n=1 << 30) == -4 and rc(M=8) == -4
+        assert lib.lr_attn_decode_beside_product(256, 1024, 256, 256, 256, 256, 1024, 32, 8, 1, 128, 64, 256, 1 << 24, 256, 256, 64, 256, 256, 63, 32,
+                                                 128, 64, 256, 1 << 20, None) == -3      # rows of the activation
+        return
+    assert rc(M=17) == -4
+    null = getattr(lib, "lr_attn_decode_" + entry)(256, 1024, 256, 256, 256, 256, 1024, 4, 8, 1, 128, 64, 256, 1 << 24, None, None, 256, 4, None)
+    assert null == -1
+
+
 def test_ladder_block_refuses_more_partial_sums_than_its_memory_holds(lib):
     """What the block before left is read in whole pieces of rows x dim: a count that the memory cannot hold is a mistake of the
     caller's, found before anything is launched."""
