@@ -331,6 +331,20 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, act_swiglu: bool
 _FP8_SCRATCH = {}
 
 
+def _fp8_scratch(device, need: int) -> torch.Tensor:
+    """Memory for the expanded weights of one linear_fp8: a buffer per (device, stream) that grows to the largest matrix seen -- calls on
+    one stream are ordered and share it, calls on two (a block's attention and MLP chains with overlap_modules) expand
+    different matrices at once.  While a graph is captured it is the graph's own, from its pool: a buffer kept here would be
+    given back when a later call grows it, and the graph go on writing to where it was."""
+    if device.type == "cuda" and torch.cuda.is_current_stream_capturing():
+        return torch.empty(need, dtype=torch.uint8, device=device)
+    key = (device, _stream())
+    t = _FP8_SCRATCH.get(key)
+    if t is None or t.numel() < need:
+        t = _FP8_SCRATCH[key] = torch.empty(need, dtype=torch.uint8, device=device)
+    return t
+
+
 class _RopeKv(ctypes.Structure):   # lr_rope_kv_t
     _fields_ = [("table", c_void_p), ("pos", c_void_p), ("k_cache", c_void_p), ("v_cache", c_void_p), ("err", c_void_p),
                 ("n_head", c_int32), ("n_kv_head", c_int32), ("head_dim", c_int32), ("smax", c_int32),
@@ -541,8 +555,7 @@ def _projection_fp8_array(projections):
 
 def linear_fp8(x: torch.Tensor, w8: torch.Tensor, scales: torch.Tensor, out: torch.Tensor):
     """out[M, N] = (x[M, K] @ w8[N, K]^T rounded to bf16) * scales[N]: weight-only e4m3 linear.  For M > 16 the
-    expanded weights go through a per-device scratch buffer that grows to the largest matrix seen (allocated
-    here, outside the library; allocate it before capturing a graph by running the shape once)."""
+    expanded weights go through scratch memory (_fp8_scratch)."""
     M, K, ldx = _rows_ld(x)
     N, Kw = w8.shape
     assert w8.dtype == torch.float8_e4m3fn and w8.is_contiguous() and Kw == K and w8.is_cuda
@@ -551,14 +564,7 @@ def linear_fp8(x: torch.Tensor, w8: torch.Tensor, scales: torch.Tensor, out: tor
     assert (Mo, No) == (M, N), (out.shape, M, N)
     lib = load()
     need = int(lib.lr_linear_fp8_scratch_bytes(M, N, K))
-    scratch = None
-    if need:
-        # one expansion buffer per (device, stream): calls on one stream are ordered and share it; calls on two
-        # streams (a block's attention and MLP chains with overlap_modules) expand different matrices at once
-        key = (x.device, _stream())
-        scratch = _FP8_SCRATCH.get(key)
-        if scratch is None or scratch.numel() < need:
-            scratch = _FP8_SCRATCH[key] = torch.empty(need, dtype=torch.uint8, device=x.device)
+    scratch = _fp8_scratch(x.device, need) if need else None
     _check(lib.lr_linear_fp8(_dev(x), ldx, w8.data_ptr(), _dev(scales), _dev(out), ldy, M, N, K,
                              None if scratch is None else scratch.data_ptr(), need, _stream()), "lr_linear_fp8")
     return out

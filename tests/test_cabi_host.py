@@ -624,6 +624,29 @@ def test_attention_in_a_shared_launch_refuses_what_its_own_launch_refuses(lib, e
     assert null == -1
 
 
+def test_expanded_weights_of_a_graph_are_in_memory_of_its_own(lib, monkeypatch):
+    """Of calls on one stream the eager ones share a buffer that grows; what is captured neither takes nor leaves one there."""
+    from types import SimpleNamespace
+
+    from gpt_fast import _hip
+
+    made, capturing = [], [False]
+    monkeypatch.setattr(_hip, "_FP8_SCRATCH", {})
+    monkeypatch.setattr(_hip, "_stream", lambda: 7)
+    monkeypatch.setattr(_hip.torch, "empty", lambda n, **kw: made.append(n) or SimpleNamespace(numel=lambda: n))
+    monkeypatch.setattr(_hip.torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    dev = torch.device("cuda", 0)
+    a = _hip._fp8_scratch(dev, 100)
+    assert _hip._fp8_scratch(dev, 50) is a
+    capturing[0] = True
+    g = [_hip._fp8_scratch(dev, n) for n in (50, 50, 200)]
+    assert a not in g and g[0] is not g[1] and list(_hip._FP8_SCRATCH.values()) == [a]
+    capturing[0] = False
+    assert _hip._fp8_scratch(dev, 100) is a
+    b = _hip._fp8_scratch(dev, 200)
+    assert b not in g and made == [100, 50, 50, 200, 200] and _hip._fp8_scratch(dev, 200) is b
+
+
 def test_ladder_block_refuses_more_partial_sums_than_its_memory_holds(lib):
     """What the block before left is read in whole pieces of rows x dim: a count that the memory cannot hold is a mistake of the
     caller's, found before anything is launched."""

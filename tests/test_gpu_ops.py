@@ -666,6 +666,32 @@ def test_linear_fp8(hip, M, N, K):
     assert_close_ulp(y, exact, max_ulp=2, max_frac=0.4, what="fp8 linear vs fp64")
 
 
+def test_linear_fp8_in_graphs_captured_one_after_the_other(hip):
+    """A later graph's larger matrix, and memory given back in between, leave the earlier graphs' expanded weights where they were."""
+    M = 80
+    x = {K: rnd(M, K, seed=42) for K in (64, 2048)}
+    cases = [O.quantize_fp8_rowwise(rnd(N, K, seed=43, scale=0.02, dtype=torch.float32), BF) for N, K in ((64, 64), (256, 2048), (4096, 2048))]
+    want = [torch.empty(M, w8.shape[0], dtype=BF, device=DEV) for w8, _ in cases]
+    eager = lambda: [hip.linear_fp8(x[w8.shape[1]], w8, sc, y) for (w8, sc), y in zip(cases, want)]
+    eager()
+    graphs = []
+    for upto in (1, 2, 3):
+        ys = [torch.zeros(M, w8.shape[0], dtype=BF, device=DEV) for w8, _ in cases[:upto]]
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            for (w8, sc), y in zip(cases, ys):
+                hip.linear_fp8(x[w8.shape[1]], w8, sc, y)
+        graphs.append((g, ys))
+        torch.cuda.empty_cache()
+    for _ in range(3):
+        eager()
+        for g, ys in graphs:
+            for y in ys:
+                y.fill_(3.0)
+            g.replay()
+            assert all(torch.equal(y, w) for y, w in zip(ys, want))
+
+
 @pytest.mark.parametrize("M,D,Hq,Hkv,hd,I", [(1, 8192, 8, 1, 128, 3584), (8, 8192, 8, 1, 128, 3584), (3, 4096, 32, 8, 128, 1000),
                                              (5, 2048, 4, 2, 64, 72), (2, 1040, 2, 2, 64, 17), (4, 64, 1, 1, 8, 8),
                                              (16, 4096, 32, 8, 128, 14336), (13, 528, 4, 4, 64, 33)])
