@@ -299,7 +299,7 @@ int lr_attn_decode_beside_product(const void* q, int64_t ldq, const void* k_cach
  * (the reference ships no quantiser and no quantised layer, so parity at this boundary is pinned by
  * the formula only).  M <= 16 (decode) streams the fp8 weights once: half the HBM bytes of lr_linear
  * (one row: matrix-vector kernel; 2 to 16 rows: the matrix-core bands of lr_linear_fp8_multi).
- * 17 to 64 rows with ldy % 8 == 0 are passes of up to 16 rows.  Else (prefill) M > 16 expands the weights
+ * 17 to 64 rows with ldy % 8 == 0 are passes of up to 16 rows where N and K are large enough.  Else (prefill) M > 16 expands the weights
  * to bf16 into `scratch` (lr_linear_fp8_scratch_bytes(M, N, K) bytes, 16-byte aligned; asked for whatever
  * the route), runs lr_linear on them and scales the columns; scratch may be NULL for M <= 16. */
 size_t lr_linear_fp8_scratch_bytes(int M, int N, int K);

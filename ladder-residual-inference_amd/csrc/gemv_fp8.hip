@@ -8,9 +8,9 @@
 // F.linear(x, w.to(bf16)) * scales.  Partial sums meet in a fixed order: bit-reproducible.
 //
 // From 2 to 16 input rows (decode batches) the projections run as matrix-core bands that expand the
-// weights on their way through LDS (stream_band.h, W8), 17 to 64 in passes of up to 16 rows.  For more
-// (prefill) the weights are expanded to bf16 in a caller-provided scratch buffer and the bf16 matrix-core
-// GEMM runs on that, followed by the per-column scaling.
+// weights on their way through LDS (stream_band.h, W8), 17 to 64 in passes of up to 16 rows where those pay
+// (passes_pay).  For more (prefill) the weights are expanded to bf16 in a caller-provided scratch buffer and
+// the bf16 matrix-core GEMM runs on that, followed by the per-column scaling.
 //
 // Weights are used once and take no room in the caches (non-temporal loads).  us of one row, ordinary /
 // non-temporal loads: 128256 x 4096 81.9 / 79.5, 28672 x 4096 20.3 / 19.7, two projections' kernel with one
@@ -330,6 +330,18 @@ __global__ __launch_bounds__(256) void k_scale_cols(u16* __restrict__ y, int64_t
     row[n] = f_to_bf(bf_to_f(row[n]) * bf_to_f(scales[n]));
 }
 
+// 17 to 64 rows in passes of up to 16 through the bands, or expanded.  Four reads of the bytes are fewer than the expansion's read,
+// write and read of twice as many, but a pass takes 4 us at least and has every CU read its input rows, which few columns do not pay for.
+// us of one product, expanded / in passes, at N x K (weights from memory):
+//   32 rows  2048 x 512  9.0 / 9.1   2048 x 1024 11.6 / 11.2   1024 x 8192 21.1 / 21.4   2048 x 14336 41.8 / 35.1   28672 x 4096 112 / 67
+//   48 rows  2048 x 1024 15.0 / 16.7   2048 x 2048 17.9 / 17.8   1024 x 4096 21.6 / 22.1   4096 x 4096 32.3 / 24.8   128256 x 4096 589 / 362
+//   64 rows  8192 x 1024 23.6 / 26.3   16384 x 1024 42.1 / 39.3   2048 x 8192 40.2 / 44.4   4096 x 14336 74.1 / 77.1   6144 x 4096 41.1 / 38.7
+static bool passes_pay(int M, int N, int K) {
+  const int64_t weights = (int64_t)N * K;
+  if (M <= 48) return M > 16 && N >= 2048 && weights >= (M <= 32 ? 1 << 21 : 1 << 22);
+  return M <= 64 && N >= 6144 && weights >= 1 << 24;
+}
+
 }  // namespace
 
 namespace lr_detail {
@@ -369,9 +381,7 @@ extern "C" int lr_linear_fp8(const void* x, int64_t ldx, const void* w8, const v
   }
   LR_REQUIRE_PTR(scratch);
   if (scratch_bytes < lr_linear_fp8_scratch_bytes(M, N, K)) return LR_E_SHAPE;
-  if (M <= LR_FP8_PASSES_TO && !lr_misaligned(scales) && ldy % 8 == 0) {   // (a pass begins at a row of its own)
-    // the bands again, in passes of up to 16 rows: four reads of the bytes are fewer than the expansion's read, write and read of
-    // twice as many (us per step expanded / in passes: 70B rank shard, 17 rows 13100 / 6280, 64 rows 16090 / 14230; 8B, 24 rows 9206 / 5087)
+  if (passes_pay(M, N, K) && !lr_misaligned(scales) && ldy % 8 == 0) {   // (a pass begins at a row of its own)
     int rc = LR_OK;
     for (int r0 = 0, left = (M + 15) / 16; rc == LR_OK && left; --left) {
       const int rows = (M - r0 + left - 1) / left;

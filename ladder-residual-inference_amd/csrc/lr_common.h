@@ -15,9 +15,6 @@
 // input rows the matrix-vector kernel, above it the matrix-core bands.  Measured on the 70B rank shard, ms per
 // step, kernel / bands: 1 row 3.66 / 3.77, 2 rows 4.40 / 3.77, 4 rows 5.22 / 3.96, 8 rows 8.13 / 4.19.
 constexpr int LR_FP8_GEMV_MAX_M = 1;
-// Rows up to which a projection with e4m3 weights is done in passes of the 16-row bands; above, the weights are expanded to bf16 for
-// the GEMM.
-constexpr int LR_FP8_PASSES_TO = 64;
 
 typedef uint16_t u16;
 typedef uint32_t u32;

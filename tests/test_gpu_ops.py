@@ -648,11 +648,11 @@ def test_linear_fp8_decodes_every_e4m3_value_exactly(hip):
                                  (1001, 528), (24, 64)])
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 16, 17, 300])
 def test_linear_fp8(hip, M, N, K):
-    """Decode (one row: matrix-vector kernel; 2 to 16 rows: matrix-core bands; fp8 weights streamed once) and prefill
-    (M > 16: expanded to bf16 in scratch + matrix-core GEMM + column scaling) against the oracle's
-    F.linear(x, w8.to(bf16)) * scales."""
+    """Decode (one row: matrix-vector kernel; 2 to 16 rows: matrix-core bands; fp8 weights streamed once; 17 rows: two passes
+    of them, or as a prompt) and prefill (expanded to bf16 in scratch + matrix-core GEMM + column scaling) against the
+    oracle's F.linear(x, w8.to(bf16)) * scales."""
     if M == 300 and N * K > 30e6:
-        M = 64
+        M = 65
     x = rnd(M, K, seed=40)
     w8, scales = O.quantize_fp8_rowwise(rnd(N, K, seed=41, scale=0.02, dtype=torch.float32), BF)
     y = torch.empty(M, N, dtype=BF, device=DEV)
@@ -664,6 +664,36 @@ def test_linear_fp8(hip, M, N, K):
     exact = ((x.double() @ w8.double().T) * scales.double()).to(BF)
     # (the single rounding of the exact product differs from the two roundings of the scheme at about a quarter of the elements, by one step)
     assert_close_ulp(y, exact, max_ulp=2, max_frac=0.4, what="fp8 linear vs fp64")
+
+
+@pytest.mark.parametrize("N,K,passes_to", [
+    (2048, 1024, 32), (2040, 1040, 16), (2048, 1008, 16),    # columns and weights from which two passes are taken
+    (2048, 2048, 48), (4096, 1008, 32),                      # and three
+    (6144, 2736, 64), (6136, 2752, 48), (6144, 2720, 48),    # and four
+    (7168, 8192, 64)])
+@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64, 65])
+def test_linear_fp8_of_17_to_64_rows(hip, M, N, K, passes_to):
+    """In passes of equal parts through the bands, the bits of linear_fp8_multi, or expanded, those of linear and the scaling; either
+    against float64 (two roundings, as in test_linear_fp8)."""
+    x = rnd(M, K, seed=40)
+    w8, sc = O.quantize_fp8_rowwise(rnd(N, K, seed=41, scale=0.02, dtype=torch.float32), BF)
+    y, want = torch.full((M, N + 8), 3.0, dtype=BF, device=DEV), torch.empty(M, N, dtype=BF, device=DEV)
+    hip.linear_fp8(x, w8, sc, y[:, :N])
+    if M <= passes_to:
+        n, at = -(-M // 16), 0
+        for left in range(n, 0, -1):
+            rows = -(-(M - at) // left)
+            hip.linear_fp8_multi((x[at:at + rows], w8, sc, want[at:at + rows], hip.EPI_NONE))
+            at += rows
+    else:
+        hip.linear(x, w8.to(BF), want)
+        want = (want.float() * sc.float()).to(BF)
+    assert torch.equal(y[:, :N], want) and bool((y[:, N:] == 3.0).all())
+    exact = ((x.double() @ w8.double().T) * sc.double()).to(BF)
+    assert_close_ulp(y[:, :N].contiguous(), exact, max_ulp=2, max_frac=0.4, what="fp8 linear vs fp64")
+    odd = torch.empty(M, N + 1, dtype=BF, device=DEV)     # rows that begin anywhere: expanded
+    hip.linear_fp8(x, w8, sc, odd[:, :N])
+    assert_close_ulp(odd[:, :N].contiguous(), exact, max_ulp=2, max_frac=0.4, what="fp8 linear vs fp64")
 
 
 def test_linear_fp8_in_graphs_captured_one_after_the_other(hip):
