@@ -191,15 +191,19 @@ def test_tiny_ladder_per_op_decode_modes(B, mode):
     check(stats)
 
 
-def test_tiny_ladder_mlp_chain_as_a_parallel_graph_branch():
-    """Above 16 sequences the MLP chain can run beside the attention chain as a second branch of the captured graph, up to
-    32 in bands: same tokens and logits as the oracle, replays equal to eager.  (The default, from 33 sequences on and without
-    bands: test_decode_batches_above_32_run_products_with_partial_sums.)"""
+def test_tiny_ladder_mlp_chain_as_a_parallel_graph_branch(monkeypatch):
+    """Above 16 sequences the MLP chain can run beside the attention chain as a second branch of the captured graph, where the
+    attention cannot share a grid with the up/gate product, up to 32 in bands: same tokens and logits as the oracle, replays
+    equal to eager.  (Without bands: test_ladder_decode_where_no_shared_grid_serves_equals_each_alone.)"""
+    from gpt_fast import _hip
+
     model = build("ladder", **dict(TINY, dim=512, n_head=8, n_local_heads=2, intermediate_size=640))
     model.two_chains_from = 17
+    monkeypatch.setattr(_hip, "attn_decode_beside_product", lambda *a: False)
     stats = run_parity(model, "ladder", B=20, T=20, new=12, fused=False)
     print(stats)
     check(stats)
+    assert hasattr(model, "_chain_stream")
 
 
 WIDER = dict(TINY, dim=512, n_head=8, n_local_heads=2, intermediate_size=2560)   # K long enough to be cut
@@ -252,6 +256,40 @@ def test_ladder_decode_of_many_different_sequences_equals_each_alone(B, fp8, mon
     decode = lambda rows: torch.cat([model(rows[:, t:t + 1].contiguous(), torch.tensor([t], device=DEV)).clone() for t in range(6)], 1)
     together = decode(toks)
     assert fp8 or (launches and all(launches))
+    for b in range(0, B, 5):
+        assert rel_err(together[b], decode(toks[b:b + 1])[0]) <= REL_TOL, b
+    decode(toks)
+    idx = toks[:, 5:].contiguous()
+    pos.fill_(5)
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+        out = model(idx, pos)
+    for _ in range(4):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[:, 0], together[:, 5])
+
+
+@pytest.mark.parametrize("why", ["declined", "tickets"])
+@pytest.mark.parametrize("B,chains", [(20, False), (32, True), (33, True), (64, True)])
+@torch.no_grad()
+def test_ladder_decode_where_no_shared_grid_serves_equals_each_alone(B, chains, why, monkeypatch):
+    """The library declines the first block's, or the workspace has no tickets: bands, and from 33 rows on products on two branches
+    of the graph (32: told to be).  Each row's logits those of the sequence decoded alone, replays equal to eager steps."""
+    from gpt_fast import _hip
+
+    model = build("ladder", **dict(WIDER, dim=1024, intermediate_size=8192))
+    model.two_chains_from = min(model.two_chains_from, 32)
+    model.setup_caches(B, 16)
+    launches = []
+    monkeypatch.setattr(_hip, "attn_decode_beside_product", lambda *a: bool(launches.append(a)))
+    if why == "tickets":
+        model._workspace(B, 1).tickets = None
+    toks = torch.randint(0, 512, (B, 6), device=DEV, generator=torch.Generator(device=DEV).manual_seed(9))
+    pos = torch.zeros(1, dtype=torch.int32, device=DEV)
+    decode = lambda rows: torch.cat([model(rows[:, t:t + 1].contiguous(), torch.tensor([t], device=DEV)).clone() for t in range(6)], 1)
+    together = decode(toks)
+    assert len(launches) == (6 if why == "declined" else 0) and hasattr(model, "_chain_stream") == chains
     for b in range(0, B, 5):
         assert rel_err(together[b], decode(toks[b:b + 1])[0]) <= REL_TOL, b
     decode(toks)
@@ -327,8 +365,8 @@ def test_a_step_of_many_rows_follows_what_the_model_has_become(B, monkeypatch):
 @pytest.mark.parametrize("family", ["ladder", "dense", "desync", "parallel"])
 @pytest.mark.parametrize("B", [33, 40, 64, 70])
 def test_decode_batches_above_32_run_products_with_partial_sums(family, B):
-    """Their default route (the ladder's up to 64 with the MLP chain as a second branch of the captured graph): the oracle's
-    tokens and logits, replays equal to eager steps."""
+    """Their default route (the ladder's up to 64 with the attention beside up/gate in one grid and wo beside w2 in another, the
+    parallel block's with the first of them): the oracle's tokens and logits, replays equal to eager steps."""
     from gpt_fast import _hip
 
     model = wider(family)

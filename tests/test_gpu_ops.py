@@ -1023,16 +1023,24 @@ def test_attn_decode_beside_a_product_declines_what_it_has_no_kernel_for(hip):
         assert run(**kw) == (False, True), kw
 
 
-@pytest.mark.parametrize("M,N,K0,K1", [(64, 8192, 1024, 3584), (33, 264, 2048, 4096), (128, 2048, 2048, 8192), (64, 2048, 64, 64),
-                                       (17, 8192, 1024, 3584), (16, 264, 2048, 4096)])
-def test_linear_pieces_two(hip, M, N, K0, K1):
-    """Two products' partial sums of one grid: their totals, in fp32, against float64."""
+@pytest.mark.parametrize("M,N,K0,K1,joint", [(64, 8192, 1024, 3584, True), (33, 264, 2048, 4096, True), (128, 2048, 2048, 8192, True),
+                                             (64, 2048, 64, 64, True), (17, 8192, 1024, 3584, True), (32, 260, 4096, 64, True),
+                                             (64, 16384, 2048, 6656, True),
+                                             (16, 264, 2048, 4096, False), (33, 264, 2056, 4096, False)])   # (few rows; no whole k-tiles)
+def test_linear_pieces_two(hip, monkeypatch, M, N, K0, K1, joint):
+    """Two products' partial sums of one grid, or of two where the library declines: their totals, in fp32, against float64."""
     x, w = [rnd(M, K, seed=90 + K % 7) for K in (K0, K1)], [rnd(N, K, seed=91 + K % 7, scale=K ** -0.5) for K in (K0, K1)]
-    sums = [torch.full((max(hip.linear_scratch_bytes(M), 200 << 15),), 255, dtype=torch.uint8, device=DEV) for _ in range(2)]
+    n = hip.linear_pieces_two_bytes(M, N, K0, K1)
+    assert (n > 0) == joint
+    sums = [torch.full((max(hip.linear_scratch_bytes(M), n, 256),), 255, dtype=torch.uint8, device=DEV) for _ in range(2)]
     out = [torch.zeros(M, N, dtype=BF, device=DEV) for _ in range(2)]
+    apart, single = [], hip.linear_pieces
+    monkeypatch.setattr(hip, "linear_pieces", lambda *a: (apart.append(a), single(*a))[1])
     parts = hip.linear_pieces_two(x[0], w[0], out[0], sums[0], x[1], w[1], out[1], sums[1])
+    assert len(apart) == (0 if joint else 2)
     for i, p in enumerate(parts):
         want = x[i].double() @ w[i].double().T
+        assert not joint or isinstance(p, hip.Pieces) and p.count * M * N * 4 <= n and not bool(out[i].any())
         if isinstance(p, hip.Pieces):
             got = sums[i].view(torch.float32)[:p.count * M * N].view(p.count, M, N).double().sum(0)
             assert ((got - want).abs() <= 1e-5 * want.abs().max()).all()
