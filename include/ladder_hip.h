@@ -281,10 +281,12 @@ int lr_attn_decode_beside_merged(const void* q, int64_t ldq, const void* k_cache
                                  size_t scratch_bytes, const lr_projection_t* projection, const lr_row_norm_t* norm,
                                  void* tickets, int M, lr_stream_t stream);
 
-/* lr_attn_decode and, in the same grid, lr_linear_swiglu_out_scratch of 17 to 64 rows: act [M, N / 2] = silu(gate) * up for w [N, K] =
- * [up; gate] rows, its partial sums in `sums`.  The two must be independent of each other.  Same bits as the two calls.  `tickets` as
- * in lr_attn_decode_beside_merged, not NULL; up to 32 rows the product is the GEMM's here and the bands' there.  LR_E_UNSUPPORTED (nothing launched): other numbers of rows, K % 64 != 0, more than 64 key
- * chunks, q heads per kv head other than 1, 2, 4, 8, 16, and products that the plan gives other tiles. */
+/* lr_attn_decode and, in the same grid, the product of lr_linear_swiglu_out_scratch for 17 to 64 rows: act [M, N / 2] = silu(gate) * up for
+ * w [N, K] = [up; gate] rows, its partial sums in `sums`.  The two must be independent of each other.  y has lr_attn_decode's bits;
+ * act those of lr_linear_swiglu_out_scratch from 33 rows on where both cut the product into as many pieces (here fewer where that costs the
+ * same), and at 17 to 32 rows, which are the bands' there, the same sums in another order.  `tickets` as in lr_attn_decode_beside_merged, not
+ * NULL.  LR_E_UNSUPPORTED (nothing launched): other numbers of rows, K % 64 != 0, more than 64 key chunks, q heads per kv head other than
+ * 1, 2, 4, 8, 16, and products that the plan gives other tiles. */
 int lr_attn_decode_beside_product(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos, void* y,
                                   int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch, size_t scratch_bytes,
                                   void* tickets, const void* x, int64_t ldx, const void* w, void* act, int64_t ld_act, int M, int N,

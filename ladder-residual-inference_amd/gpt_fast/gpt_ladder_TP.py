@@ -153,7 +153,7 @@ class GPTLadder(GPTBase):
             if side is None or side.device != main.device:
                 side = self._side_stream = torch.cuda.Stream(device=main.device)
         pending_a = pending_m = None
-        # decode batches of up to 32 rows on bf16 weights: the block's two input projections share one launch of
+        # decode batches of up to 32 rows on bf16 weights (from 17 on where no shared grid serves): the block's two input projections share one launch of
         # the weight-streaming kernel (q/k/v -- rotated and cached on the way out -- next to up/gate, which stores
         # silu(gate) * up directly), and so do its two output projections (wo next to w2).  Also below 5 rows,
         # where single projections go to the matrix-vector kernel: five or six launches per block instead of nine

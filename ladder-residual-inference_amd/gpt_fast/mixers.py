@@ -57,7 +57,9 @@ def project(x: Tensor, lin: nn.Linear, out: Tensor, sums: Optional[Tensor] = Non
     Two rows of weights with more rows than columns, and up to four of a head's, are the matrix-vector kernel's: a band's start and end
     weigh more there than arithmetic per row.  us, matrix-vector / bands, two rows: 128256 x 4096 150 / 185, 34816 x 4096 43.3 / 47.1, 10240 x
     4096 16.1 / 18.0, 5120 x 2048 5.6 / 6.9, but 4096 x 18432 26.2 / 26.1, 2048 x 8192 8.4 / 7.9; three rows: 128256 x 4096 173 / 184, 34816 x
-    4096 50.3 / 47.4; four: 128256 x 4096 180 / 184, 10240 x 4096 19.1 / 17.1."""
+    4096 50.3 / 47.4; four: 128256 x 4096 180 / 184, 10240 x 4096 19.1 / 17.1.  6: between the widest of these models' other projections (34816 x
+    4096, 2.8 columns' worth per row, the bands') and their heads (from 7.8 on); of widths between and beyond, 24576 to 262144 x 1024 to 4096,
+    it is the faster one where the rule takes it (24576 x 1024, three rows 13.2 / 15.4; 262144 x 4096, four rows, 378 / 372, is not)."""
     rows, (N, K) = x.shape[0], lin.weight.shape
     few = rows == 2 and N > K or rows <= 4 and N > 6 * rows * K
     if x.dtype == torch.bfloat16 and not few and 2 <= rows <= (64 if sums is None else _hip.BANDS_TO):
