@@ -516,24 +516,24 @@ __global__ __launch_bounds__(1024) void k_argmax(const T* __restrict__ logits, i
                                                  int32_t* __restrict__ out, int V) {
   __shared__ float sv[2][16];
   __shared__ int si[2][16];
-  constexpr int AHEAD = 8, STEP = 1024 * 8;
+  constexpr u32 AHEAD = 8, STEP = 1024 * 8;   // (columns are counted unsigned: a step beyond the last one may pass 2^31)
   const T* row = logits + (int64_t)blockIdx.x * ldl;
   float bv = -INFINITY;
   int bi = 0x7fffffff;
-  const int V8 = V & ~7, at = threadIdx.x * 8;
+  const u32 V8 = V & ~7, at = threadIdx.x * 8;
   decltype(logits8_load(row)) best = {};   // the group that bv is from
-  for (int c0 = 0; c0 < V8; c0 += AHEAD * STEP) {
+  for (u32 c0 = 0; c0 < V8; c0 += AHEAD * STEP) {
     decltype(logits8_load(row)) raw[AHEAD];
 #pragma unroll
-    for (int a = 0; a < AHEAD; ++a)
+    for (u32 a = 0; a < AHEAD; ++a)
       if (a == 0 || c0 + a * STEP < V8) {   // (uniform; a lane beyond the end looks at the first group again)
-        const int c = c0 + a * STEP + at;
+        const u32 c = c0 + a * STEP + at;
         raw[a] = logits8_load(row + (c < V8 ? c : 0));
       }
 #pragma unroll
-    for (int a = 0; a < AHEAD; ++a)
+    for (u32 a = 0; a < AHEAD; ++a)
       if (a == 0 || c0 + a * STEP < V8) {
-        const int c = c0 + a * STEP + at;
+        const u32 c = c0 + a * STEP + at;
         float f[8], m = -INFINITY;
         logits8(raw[a], f);
 #pragma unroll
@@ -549,10 +549,10 @@ __global__ __launch_bounds__(1024) void k_argmax(const T* __restrict__ logits, i
     for (int i = 6; i >= 0; --i) j = f[i] == bv ? i : j;
     bi += j;
   }
-  if ((int)threadIdx.x < V - V8) amax_merge(bv, bi, logit1(row + V8 + threadIdx.x), V8 + threadIdx.x);
+  if (threadIdx.x < V - V8) amax_merge(bv, bi, logit1(row + V8 + threadIdx.x), V8 + threadIdx.x);
   amax_workgroup(bv, bi, sv[0], si[0]);
   if (bv == -INFINITY) {   // nothing above the lowest value: the first column that has it
-    for (int c = threadIdx.x; c < V; c += 1024) amax_merge(bv, bi, logit1(row + c), c);
+    for (u32 c = threadIdx.x; c < (u32)V; c += 1024) amax_merge(bv, bi, logit1(row + c), c);
     amax_workgroup(bv, bi, sv[1], si[1]);
   }
   if (threadIdx.x == 0) out[blockIdx.x] = bi == 0x7fffffff ? 0 : bi;

@@ -1171,6 +1171,20 @@ def test_argmax_at_the_edges_of_its_groups(hip, V, dtype):
     assert out.flatten().tolist() == want.tolist()
 
 
+def test_argmax_of_a_row_as_long_as_its_index_reaches(hip):
+    """Columns whose steps pass 2^31: the last one, in the ragged end, the last of the groups of eight, one in the middle; none at all."""
+    V = 2 ** 31 - 9
+    lg, out = torch.full((1, V + 1), -1.0, dtype=BF, device=DEV), torch.empty(1, dtype=torch.int32, device=DEV)
+    for at in (V - 1, V - 8, V // 2):
+        lg[0, at] = 1.0
+        hip.argmax(lg[:, :V], out)
+        assert out.item() == at
+        lg[0, at] = float("-inf")
+    lg.fill_(float("-inf"))
+    hip.argmax(lg[:, :V], out)
+    assert out.item() == 0
+
+
 def test_torch_argmax_itself_returns_first_maximum_on_this_device():
     """The oracle's greedy() relies on it."""
     lg = torch.zeros(1, 16032, dtype=BF, device=DEV)
