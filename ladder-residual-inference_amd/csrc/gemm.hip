@@ -698,8 +698,10 @@ struct GemmPlan {
 //   128 rows,  4096 x 14336  38.3 / 32.8 / 32.8 | 32.8        1501 rows,  7168 x  8192 153.9 / 168.2 / 153.9 | 153.9 (pairs)
 //   128 rows, 28672 x  4096  65.8 / 54.8 / 54.8 | 54.8 (pairs)  2100 rows, 4608 x 4096  79.2 / 82.3 / 79.2 | 77.2
 // Tiles of 160, 192 and 224 rows came later; their costs are fitted to 1457 products of 131 to 4096 rows of 31 weights, with 64 MiB for pieces
-// and none, the first four tiles' as they were.  The products took 5.3 % less on average, 11 of 2914 choices more than 3 % more (257 rows,
-// 2048 x 8192 21.6 -> 24.4), and the plan is 0.9 % above the best choice.  us, with four tiles / now:
+// and none, the first four tiles' as they were.  160 x 128 is cut into eight pieces at most: of a single row tile more were the slower choice
+// (131 to 160 rows: 1280 x 8192 15.5 -> 16.5 us, 2048 x 5120 16.2 -> 17.9).  The products take 4.7 % less on average, 12 of 2898 choices
+// more than 2 % more (777 rows, 2048 x 8192 36.8 -> 40.7, 2200 rows, 6144 x 2048 49.4 -> 53.0, 4096 rows, 6144 x 4096 without memory 158 -> 167,
+// else less than 5 %; costs that spare these lose as much elsewhere), and the plan is 0.8 % above the best choice.  us, with four tiles / now:
 //   300 rows, 28672 x 4096 100.3 / 74.0 (pairs)   450 rows,  7168 x 8192  69.4 / 58.7 (pairs)   777 rows, 28672 x 4096 197.2 / 176.9 (pairs)
 //   777 rows,  6144 x 4096  55.7 / 44.1           777 rows,  4096 x 14336 94.7 / 89.4          1501 rows,  7168 x 8192 162.5 / 138.4 (pairs)
 //  1100 rows,  4096 x 4096  52.1 / 41.0          9205 rows,  2048 x 8192 278.1 / 227.4 (no memory)
@@ -707,19 +709,19 @@ struct GemmPlan {
 // Where the first four lose most: 129 rows, 16032 x 8192 65.9 / 78.8 / 77.1 | 65.9; 5000 rows, 2048 x 5120 95.5 / 95.5 / 109.6 | 95.5; 192 rows,
 // 3072 x 2048 17.1 in all three | 14.0; 1100 rows, 8192 x 512 19.9 in all three | 16.4.
 struct GemmTileCost {
-  int a, bh, per_cu;
+  int a, bh, per_cu, pieces;   // (pieces: at most)
   float ktile, slope, cold, pair, pair_cold, fixed, store;
 };
 constexpr int GEMM_NTILES = 9, GEMM_TILES_ANY = 4;   // the first four take any K and any number of rows, see gemm_plan
-constexpr GemmTileCost GEMM_TILES[GEMM_NTILES] = {{8, 2, 1, 1.2f, 0.0f, 0.0f, 0.0f, 0.0f, 4.35f, 4.43f},
-                                                  {4, 2, 1, 0.684f, 0.108f, 0.552f, 0.0f, 0.0f, 2.85f, 1.47f},
-                                                  {4, 1, 2, 0.504f, 0.0f, 0.262f, 0.874f, 1.25f, 3.18f, 0.166f},
-                                                  {2, 1, 2, 0.302f, 0.201f, 0.284f, 0.737f, 1.19f, 3.24f, 0.0f},
-                                                  {7, 2, 1, 1.098f, 0.0394f, 0.0f, 0.0f, 0.0f, 6.28f, 2.11f},
-                                                  {6, 2, 1, 0.953f, 0.0412f, 0.119f, 0.0f, 0.0f, 6.24f, 1.61f},
-                                                  {5, 2, 1, 0.668f, 0.2935f, 0.581f, 0.0f, 0.0f, 3.12f, 5.41f},
-                                                  {5, 1, 2, 0.553f, 0.0159f, 0.173f, 1.103f, 4.77f, 3.88f, 0.0077f},
-                                                  {6, 1, 1, 0.617f, 0.0f, 0.0944f, 0.0f, 0.0f, 4.28f, 0.0f}};
+constexpr GemmTileCost GEMM_TILES[GEMM_NTILES] = {{8, 2, 1, 16, 1.2f, 0.0f, 0.0f, 0.0f, 0.0f, 4.35f, 4.43f},
+                                                  {4, 2, 1, 16, 0.684f, 0.108f, 0.552f, 0.0f, 0.0f, 2.85f, 1.47f},
+                                                  {4, 1, 2, 16, 0.504f, 0.0f, 0.262f, 0.874f, 1.25f, 3.18f, 0.166f},
+                                                  {2, 1, 2, 16, 0.302f, 0.201f, 0.284f, 0.737f, 1.19f, 3.24f, 0.0f},
+                                                  {7, 2, 1, 16, 1.098f, 0.0394f, 0.0f, 0.0f, 0.0f, 6.28f, 2.11f},
+                                                  {6, 2, 1, 16, 0.953f, 0.0412f, 0.119f, 0.0f, 0.0f, 6.24f, 1.61f},
+                                                  {5, 2, 1, 16, 0.668f, 0.2935f, 0.581f, 0.0f, 0.0f, 3.12f, 5.41f},
+                                                  {5, 1, 2, 8, 0.553f, 0.0159f, 0.173f, 1.103f, 4.77f, 3.88f, 0.0077f},
+                                                  {6, 1, 1, 16, 0.617f, 0.0f, 0.0944f, 0.0f, 0.0f, 4.28f, 0.0f}};
 constexpr size_t GEMM_SCRATCH = (size_t)64 << 20;   // pieces of one round of the largest tiles
 constexpr int GEMM_SCRATCH_FROM = 33;               // rows from which a projection that has memory for pieces is one of this file's
 // and from which the two grids of a decode step are, that hold a product beside the attention or another product: below, the
@@ -742,7 +744,9 @@ static float gemm_round_us(const GemmTileCost& t, int M, int cus, int workgroups
 static float gemm_bytes_us(int M, int N, int K, int mode) {
   return (mode == GEMM_PAIR ? 2.0f : 1.0f) * N * K * 2 / GEMM_WEIGHT_BYTES_US + (float)M * N * 2 / GEMM_OUTPUT_BYTES_US;
 }
-// Round trips to memory of whoever adds the pieces: the first piece and four more, then four at a time.
+// What more pieces cost whoever adds them, beside their bytes: a step for every four, as the norms take them.  (k_gemm_sum takes eight at a
+// time; measured again with it, 1740 products are nearest their best with these steps and 4.92 us: 1.1 % above it from 129 rows on; steps of
+// eight, of one or none, 3.5 to 5.3 us and other rates: 1.1 to 2.6 %.)
 static int gemm_trips(int pieces) { return (pieces + 2) / 4; }
 static float gemm_store_us(const GemmTileCost& t, int64_t tiles, int cus, int mode) {
   return t.store * (mode == GEMM_PAIR ? 0.5f : 1.0f) * tiles / cus;
@@ -770,7 +774,7 @@ static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
     };
     const float whole = rounds * round_us(slots, nk), fixed = (rounds + (left ? 1 : 0)) * t.fixed;
     consider(whole + (left ? round_us(left, nk) : 0.0f), fixed, (int)tiles, 0, 1);
-    for (int s = 2; left && s <= 16 && 4 * s <= nk && left * s <= slots; ++s) {
+    for (int s = 2; left && s <= t.pieces && 4 * s <= nk && left * s <= slots; ++s) {
       const size_t bytes = (size_t)left * s * (32 * t.a) * (128 * t.bh) * sizeof(float);
       if (bytes > scratch) break;
       consider(whole + round_us(left * s, (nk + s - 1) / s), fixed + GEMM_SUM_US + gemm_trips(s) * GEMM_TRIP_US + bytes / GEMM_PIECE_BYTES_US,

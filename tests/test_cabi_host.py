@@ -340,6 +340,9 @@ MEASURED_PRODUCTS = [
     (128, 3072, 2048, False, 64, {(64, 128, 1): 17.2, (64, 128, 4): 13.3, (64, 128, 5): 13.0}),
     (128, 4096, 14336, False, 64, {(64, 128, 8): 38.3, (128, 128, 8): 32.8}),
     (128, 28672, 4096, True, 64, {(64, 128, 1): 65.8, (128, 128, 1): 54.8}),
+    (136, 1280, 8192, False, 64, {(64, 128, 8): 15.5, (160, 128, 16): 16.5}),
+    (145, 2048, 5120, False, 64, {(64, 128, 5): 16.2, (160, 128, 10): 17.9}),
+    (160, 2048, 10240, False, 64, {(128, 128, 8): 19.8, (160, 128, 16): 20.8}),
     (9205, 2560, 2048, False, 64, {(256, 256, 2): 95.6, (128, 256, 1): 85.9, (192, 256, 1): 80.2}),
 ]
 
