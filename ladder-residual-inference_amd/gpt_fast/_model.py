@@ -47,8 +47,8 @@ class Workspace:
         self.next_token_valid_for = None   # set by a fused decode step that already chose the token
         self.scratch = None
         # Partial sums of products: two memories where a prompt's blocks leave both outputs' to the next norms (two_sums), and
-        # in a decode step, where the MLP's may run beside the attention's, and alternating ones are faster also one after the
-        # other (8B dense, 33 rows: 4.67 ms per step, 4.71 in one).  The MLP's of up to 64
+        # in a decode step, where the MLP's may run beside the attention's (a ladder's two branches, where no shared grid serves), and
+        # alternating ones are faster also one after the other (8B dense, 33 rows: 4.67 ms per step, 4.71 in one).  The MLP's of up to 64
         # rows has room for the pieces of 25 of 32 compute units, 32 KiB each: beside the attention's products these keep
         # the rest (70B rank shard, 64 rows: 7.6 ms per step, 8.2 with as many pieces as pay for a product alone), and
         # alone more are no faster (w2 4096 x 14336 of 64 rows: 31.9 us in six pieces, 34.2 in seven).  More rows have
