@@ -257,15 +257,29 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
 #pragma unroll
     for (int mt = 0; mt < MTILES; ++mt) acc[u][mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-  // chunk ci of this wave starts at k0 = (ci * NWV + wave) * KCW; what lies beyond K reads as zero (no
-  // branch around a load: the number of loads in flight is fixed, so the waits between chunks are exact).
-  // (Every band walks K from 0, so the whole grid asks for the same 4 KiB window of its rows at the same time.
-  // Starting band b `b % chunks` chunks in, wrapping around, spreads that over the DRAM channels: 16-row bands
-  // 1.5 % faster per step, 64-row bands 8 % slower -- their inputs come from L2, which likes the common window.
-  // Not kept: the order of a sum would then depend on how the rows are cut into bands.)
+  // Which chunk of K is the wave's ci-th: bf16 bands are read in a slice of K per wave, one chunk behind the other.  (The waves'
+  // chunks in turn, g = ci KW + wave, as it was and as e4m3 bands and the two matrices of RN still are: a wave then skips three
+  // chunks of every row.  us, 8 rows, in turn / in slices: 128256 x 4096 194 / 157, 16384 x 2048 15.9 / 14.7, 6144 x 4096 12.4 / 11.7,
+  // 4096 x 14336 22.2 / 20.9; of RN, 8192 x (1024 | 3584) 18.4 / 19.6.)
+  // All workgroups walk K from the same end, over rows that lie a multiple of 4 KiB apart: the four waves' places should differ
+  // there too, or all of the grid asks for the same 1 KiB in four of the DRAM's interleaving.  Slices of whole 4 KiB (K 8192) begin
+  // at four different quarters and wrap around: 7168 x 8192 22.4 in turn, 26.3 in slices, 21.2 so, 16032 x 8192 54.7 / 51.5 / 42.7.
+  // What lies beyond K or the wave's last chunk reads as zero (no branch around a load: the number of loads in flight is fixed, so
+  // the waits between chunks are exact).  The order of a sum is a matter of K alone, not of how the rows are cut into bands.
+  const int nck = nck1 + (RN ? (rn.K2 + KCW - 1) / KCW : 0);
+  constexpr bool SLICES = !RN && !W8;
+  const int kper = (nck + KW - 1) / KW, kfirst = SLICES ? kwave * kper : kwave;
+  const int nch = kfirst >= nck ? 0 : SLICES ? (nck - kfirst < kper ? nck - kfirst : kper) : (nck - kfirst + KW - 1) / KW;  // chunks of this wave
+  constexpr int CHUNKS_4K = 4096 / (KCW * WB), QUARTER = CHUNKS_4K / 4;
+  const int kturn = SLICES && kper % CHUNKS_4K == 0 && nch == kper ? kwave * QUARTER % CHUNKS_4K : 0;
+  auto chunk_at = [&](int ci) {
+    if (!SLICES) return ci * KW + kfirst;
+    const int c = ci + kturn;
+    return ci < nch ? kfirst + (c < nch ? c : c - nch) : nck;
+  };
   auto issue_w = [&](int ci, u32x4_t (&dst)[NLD]) {
     if constexpr (RN) {
-      const int g = ci * KW + kwave;
+      const int g = chunk_at(ci);
       const bool second = g >= nck1;
       const int k0 = (second ? g - nck1 : g) * KCW, Kx = second ? rn.K2 : K;
       const __amdgpu_buffer_rsrc_t res = __builtin_amdgcn_make_buffer_rsrc(
@@ -277,7 +291,7 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
         dst[i] = __builtin_amdgcn_raw_buffer_load_b128(res, at | beyond(4 * i + l4, nrows), (k0 + 4 * i * Kx) * WB, AUX_WEIGHTS);
       return;
     }
-    const int k0 = (ci * KW + kwave) * KCW;
+    const int k0 = chunk_at(ci) * KCW;
     const bool kok = k0 + l16 * (16 / WB) < K;
 #pragma unroll
     for (int i = 0; i < NLD; ++i)
@@ -285,7 +299,7 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
   };
   auto issue_x = [&](int ci, u32x4_t (&dst)[MTILES][X8 ? KS / 2 : KS]) {
     if constexpr (RN) {
-      const int g = ci * KW + kwave;
+      const int g = chunk_at(ci);
       const bool second = g >= nck1;
       const int k0 = (second ? g - nck1 : g) * KCW, Kx = second ? rn.K2 : K;
       const __amdgpu_buffer_rsrc_t res =
@@ -300,7 +314,7 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
       }
       return;
     }
-    const int k0 = (ci * KW + kwave) * KCW;
+    const int k0 = chunk_at(ci) * KCW;
     if constexpr (XLDS) {
       const bool kok = k0 + l16 * 8 < K;
 #pragma unroll
@@ -324,8 +338,6 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
     }
   };
 
-  const int nck = nck1 + (RN ? (rn.K2 + KCW - 1) / KCW : 0);
-  const int nch = kwave < nck ? (nck - kwave + KW - 1) / KW : 0;  // chunks of this wave
   // (the fences keep the requests in this order: the wait for chunk 0 counts the requests made after it, and the
   // scheduler, left alone, asks for chunk 0 last -- the loop then waited for all but the last 8 requests at the top
   // of every round of NS chunks)
@@ -419,7 +431,7 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
     for (int s = 0; s < NS; ++s) {
       const int ci = c0 + s;
       if constexpr (RN) {
-        if (in_first && ci * KW + kwave >= nck1) {
+        if (in_first && chunk_at(ci) >= nck1) {
           in_first = false;
 #pragma unroll
           for (int u = 0; u < UNITS; ++u)

@@ -618,6 +618,16 @@ def test_bands_of_few_rows_equal_the_bands_of_many(hip, M, N, K):
         assert torch.equal(few, many[:M])
 
 
+@pytest.mark.parametrize("M", [3, 24, 60])
+@pytest.mark.parametrize("K", [8, 120, 136, 520, 8064, 8072, 8192, 8200, 16384, 16512])
+def test_bands_in_slices_of_k(hip, M, K):
+    """Each wave's slice of K: fewer chunks than waves, a last wave with fewer or none, slices of whole 4 KiB (which wrap around)."""
+    x, w = rnd(M, K, seed=94), rnd(40, K, seed=95, scale=0.02)
+    y = torch.empty(M, 40, dtype=BF, device=DEV)
+    hip.linear_multi((x, w, y, hip.EPI_NONE))
+    assert_close_ulp(y, linear_ref(x, w), what=f"slices M={M} K={K}")
+
+
 @pytest.mark.parametrize("rows,dim", [(2, 4096), (2, 4104), (257, 8192), (3, 8200), (1, 16376)])
 def test_norms_at_the_edges_of_the_lanes_per_row(hip, rows, dim):
     """256 lanes up to 4096 columns, 1024 above; the last columns leave most lanes of the last turn idle."""
