@@ -144,7 +144,7 @@ __global__ __launch_bounds__(256) void k_gemm(const u16* __restrict__ x, int64_t
 // from and again by the address a fragment is read at: conflict-free for the 16-row fragments of
 // v_mfma_f32_16x16x32_bf16.
 //
-// What a tile of fewer rows costs is what the L2s give a CU, about 65 GB/s: (m + n) * 128 bytes per k-tile, 1.0 us at 256 x 256 where the
+// What a tile of fewer rows costs is what a CU draws, about 65 GB/s while part of it comes from HBM (from L2 alone 127): (m + n) * 128 bytes per k-tile, 1.0 us at 256 x 256 where the
 // matrix cores need 1.1 to 1.2, 0.5 at 128 x 128 where they need 0.3.  So tiles from 160 rows on are as good per row as the largest, and rows
 // that are no multiple of 256 want them: 777 rows are four tiles of 224 (measured below, at GEMM_TILES).
 //
@@ -166,7 +166,18 @@ __global__ __launch_bounds__(256) void k_gemm(const u16* __restrict__ x, int64_t
 // instructions took 1337 us for the last: twice the accumulator traffic per product, at a power-limited clock.  The matrix
 // instruction is assembler text because its accumulator has to be one register block in and out: left to the compiler,
 // 180 accumulator moves per two k-tiles (1.15 PFLOP/s).
+//
+// A ring of three k-tiles, for up to 64 rows and, as a tile of its own (GEMM_LONG), 128 x 128 of up to 128: what bounds these is the
+// weights' way from HBM, and a CU has at most some 48 KiB of requests on their way whoever waits for them, so a ring of two, of
+// which a k-tile and a half are, asks for too little; four are no faster (7168 x 8192, 64 rows, four pieces: two 31.0 us, three 27.4,
+// four 27.6).  And all workgroups walk K from the same end, over rows that lie a multiple of 4 KiB apart: at any time they ask for
+// one place of the DRAM's interleaving.  With a long ring column tile nt begins at k-tile GEMM_TURN * nt and goes round (a stream of
+// such operands without products, 128 rows, 7168 x 8192: ring of two 33.3 us, turned 30.9, ring of four 27.2, turned 23.3).  Not with
+// several row tiles, which share the rows and the weights in L2 while they go in step.  us before / now: 64 rows, 28672 x 4096 (pairs)
+// 47.5 / 39.9, 6144 x 4096 31.4 / 30.1 without pieces; 128 rows, 16032 x 8192 66.5 / 56.7, 28672 x 4096 (pairs) 54.7 / 50.6, 7168 x
+// 8192 (pairs) 36.0 / 32.3.
 // ---------------------------------------------------------------------------------------------
+constexpr int GEMM_RING = 3, GEMM_TURN = 5;
 struct GemmRope {   // the projection is the fused q/k/v projection of a prefill: see lr_linear_rope_kv
   const u16* table;
   const int32_t* pos;
@@ -193,14 +204,15 @@ struct GemmSplit {
 };
 enum { GEMM_PLAIN, GEMM_PAIR, GEMM_ROPE, GEMM_ROWS };   // ROWS: every tile is cut, the pieces stay, see GemmSplit; PAIR: w holds [up; gate] rows, N counts pairs, output silu(gate) * up
 
-template <int A, int BH>
+template <int A, int BH, int R = 2>
 struct GemmTile {
   static constexpr int TM = 32 * A, TN = 128 * BH;
   static constexpr int A0 = (A + 1) / 2, A1 = A / 2;     // 16-row groups of a wave in either half of the input rows
   static constexpr int NB = 2 * BH;                      // DMA instructions of a wave for half a k-tile of weights (of input rows: A0, A1)
   static constexpr int HB = 8192 * BH;                   // its bytes
   static constexpr int ABYTES = 4096 * A;                // and those of a k-tile of input rows
-  static constexpr int RING = 2 * ABYTES + 4 * HB;
+  static constexpr int SLOT = ABYTES + 2 * HB;           // a k-tile
+  static constexpr int RING = R * SLOT;
   static constexpr int EPITCH = 64 * BH + 8;             // row pitch of a wave's output piece (plain), in elements
   static constexpr int EBYTES = 4 * 16 * A * EPITCH * 2;
   static constexpr int LDS = RING > EBYTES ? RING : EBYTES;
@@ -351,12 +363,16 @@ __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[A][4 * BH], u16*
 
 // KTAIL: K is not a multiple of the 64-element k-tile, so the last one needs a per-lane range check.  NT: weights are loaded
 // non-temporally.
-template <int A, int BH, bool KTAIL, int MODE, bool GROUP, bool NT>
+template <int A, int BH, bool KTAIL, int MODE, bool GROUP, bool NT, int R = 2>
 __device__ __forceinline__ void gemm_tile(const int block, const int blocks, const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
                                           u16* __restrict__ y, int64_t ldy, int M, int N, int K, int tm, int tn, const GemmRope& rp,
                                           const GemmSplit& sp, const GemmGroup& gp) {
-  using T = GemmTile<A, BH>;
-  constexpr int A0 = T::A0, A1 = T::A1, HB = T::HB, NB = T::NB, BOFF = 2 * T::ABYTES;
+  using T = GemmTile<A, BH, R>;
+  // Where k-tile t lies in LDS: of a ring of two by its parity, a constant; else a slot is input rows and weight rows together, at
+  // an offset that goes round with the loop.
+  constexpr bool LONG = R > 2;
+  constexpr int A0 = T::A0, A1 = T::A1, HB = T::HB, NB = T::NB, BOFF = LONG ? T::ABYTES : 2 * T::ABYTES;
+  constexpr int APAR = LONG ? 0 : T::ABYTES, BPAR = LONG ? 0 : 2 * HB;
   extern __shared__ __attribute__((aligned(1024))) u16 gsm[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
@@ -417,8 +433,10 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
   const int64_t xlast = GROUP ? gp.xrows - 1 : (M - m0 < T::TM ? M - m0 : T::TM) - 1;
   const int64_t wlast = MODE == GEMM_PAIR ? N + (int64_t)(N - n0 < T::TN / 2 ? N - n0 : T::TN / 2) - 1 : (N - n0 < T::TN ? N - n0 : T::TN) - 1;
   const int xbytes = (int)((xlast * ldx + klen) * 2), wbytes = (int)((wlast * K + klen) * 2);   // (below 2 GiB: gemm_reaches)
+  const int turn = LONG ? (int)((unsigned)(nt * GEMM_TURN) % (unsigned)nk) : 0;   // the k-tile that is multiplied first
   auto request = [&](auto ONCE, const u16* base, int bytes, int voff, int t, u32 lds) {
     const bool in = t < nk;
+    if (LONG) t = t + turn < nk ? t + turn : t + turn - nk;
     i32x4_t r;
     r.x = (int)(u32)(unsigned long long)base;
     r.y = (int)(u32)((unsigned long long)base >> 32) & 0xffff;
@@ -427,8 +445,12 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
     if (KTAIL) voff = t * 64 + chunk < klen ? voff : OUT;
     dma16<decltype(ONCE)::value>(r, voff, in ? t * 128 : 0, lds);
   };
-  auto dma_a = [&](int t, int par, int h, int i) { request(std::false_type{}, xb, xbytes, xo[h][i], t, lds0 + par * T::ABYTES + h * 4096 * A0 + (wave * (h ? A1 : A0) + i) * 1024); };
-  auto dma_b = [&](int t, int par, int h, int i) { request(std::bool_constant<NT>{}, wb, wbytes, wo[h][i], t, lds0 + BOFF + (par * 2 + h) * HB + (wave * NB + i) * 1024); };
+  auto dma_a = [&](int t, int par, int slot, int h, int i) {
+    request(std::false_type{}, xb, xbytes, xo[h][i], t, lds0 + slot + par * APAR + h * 4096 * A0 + (wave * (h ? A1 : A0) + i) * 1024);
+  };
+  auto dma_b = [&](int t, int par, int slot, int h, int i) {
+    request(std::bool_constant<NT>{}, wb, wbytes, wo[h][i], t, lds0 + slot + BOFF + par * BPAR + h * HB + (wave * NB + i) * 1024);
+  };
 
   f32x4_t acc[A][4 * BH];
 #pragma unroll
@@ -447,49 +469,51 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
     fa[1][ks] = (wm * 16 * A1 + (lane & 15)) * 128 + c;
     fb[ks] = (wn * 32 * BH + (lane & 15)) * 128 + c + BOFF;
   }
-  auto read_a = [&](int par, int h, int t, int ks) {
-    af[h][t][ks] = *reinterpret_cast<const bf16x8_t*>(smb + fa[h][ks] + par * T::ABYTES + h * 4096 * A0 + t * 2048);
+  auto read_a = [&](int par, int slot, int h, int t, int ks) {
+    af[h][t][ks] = *reinterpret_cast<const bf16x8_t*>(smb + (fa[h][ks] + slot) + par * APAR + h * 4096 * A0 + t * 2048);
   };
-  auto read_b = [&](int set, int par, int h, int t, int ks) {
-    bf[set][t][ks] = *reinterpret_cast<const bf16x8_t*>(smb + fb[ks] + (par * 2 + h) * HB + t * 2048);
+  auto read_b = [&](int set, int par, int slot, int h, int t, int ks) {
+    bf[set][t][ks] = *reinterpret_cast<const bf16x8_t*>(smb + (fb[ks] + slot) + par * BPAR + h * HB + t * 2048);
   };
   auto barrier = [&] {
     asm volatile("s_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
 
+  constexpr int AHEAD = (R - 2) * (A + 2 * NB);   // requests of a wave beyond those of two k-tiles
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
+  for (int t = 0; t < R; ++t) {
+    const int par = t & 1, slot = LONG ? t * T::SLOT : 0;
 #pragma unroll
-    for (int i = 0; i < A0; ++i) dma_a(t, t, 0, i);
+    for (int i = 0; i < A0; ++i) dma_a(t, par, slot, 0, i);
 #pragma unroll
-    for (int i = 0; i < NB; ++i) dma_b(t, t, 0, i);
+    for (int i = 0; i < NB; ++i) dma_b(t, par, slot, 0, i);
 #pragma unroll
-    for (int i = 0; i < NB; ++i) dma_b(t, t, 1, i);
+    for (int i = 0; i < NB; ++i) dma_b(t, par, slot, 1, i);
 #pragma unroll
-    for (int i = 0; i < A1; ++i) dma_a(t, t, 1, i);
+    for (int i = 0; i < A1; ++i) dma_a(t, par, slot, 1, i);
   }
-  wait_requests_and_lds<A0 + 2 * A1 + 3 * NB>();
+  wait_requests_and_lds<AHEAD + A0 + 2 * A1 + 3 * NB>();
   barrier();
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-    for (int t = 0; t < A0; ++t) read_a(0, 0, t, ks);
+    for (int t = 0; t < A0; ++t) read_a(0, 0, 0, t, ks);
 #pragma unroll
-    for (int t = 0; t < 2 * BH; ++t) read_b(0, 0, 0, t, ks);
+    for (int t = 0; t < 2 * BH; ++t) read_b(0, 0, 0, 0, t, ks);
   }
-  wait_requests_and_lds<A0 + 2 * A1 + 3 * NB>();
+  wait_requests_and_lds<AHEAD + A0 + 2 * A1 + 3 * NB>();
   barrier();
 #pragma unroll
-  for (int i = 0; i < A0; ++i) dma_a(2, 0, 0, i);
+  for (int i = 0; i < A0; ++i) dma_a(R, 0, 0, 0, i);
 
   // Phase P of k-tile t (even: PAR 0).  Reads B1 of this tile, A1 of this tile, A0 of the next, B0 of the next; requests
-  // B0, B1, A1 of tile t + 2 and A0 of tile t + 3.
-  auto phase = [&](auto PAR_, auto P_, int t) {
+  // B0, B1, A1 of tile t + R and A0 of tile t + 1 + R.  `here`, `next`: the slots of this tile and the next.
+  auto phase = [&](auto PAR_, auto P_, int t, int here, int next) {
     constexpr int PAR = decltype(PAR_)::value, P = decltype(P_)::value;
     constexpr int ah = P >> 1, bh = (P == 1 || P == 2), set = bh ^ PAR;
     // requests younger than the slot read here: those of the six phases since
-    wait_requests_and_lds<(P == 0 ? 2 * A + 2 * NB : P == 1 ? A + A0 + 3 * NB : P == 2 ? A + 4 * NB : A + A1 + 3 * NB)>();
+    wait_requests_and_lds<AHEAD + (P == 0 ? 2 * A + 2 * NB : P == 1 ? A + A0 + 3 * NB : P == 2 ? A + 4 * NB : A + A1 + 3 * NB)>();
     barrier();
     constexpr int AH = ah ? A1 : A0, J = 4 * AH * BH, RD = P == 1 ? 2 * A1 : P == 2 ? 2 * A0 : 4 * BH, RQ = P == 2 ? A1 : P == 3 ? A0 : NB;
 #pragma unroll
@@ -501,18 +525,18 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
       if (j < J / 2) {
 #pragma unroll
         for (int e = j * RD / (J / 2); e < (j + 1) * RD / (J / 2); ++e) {
-          if (P == 0) read_b(1 ^ PAR, PAR, 1, e % (2 * BH), e / (2 * BH));
-          if (P == 1) read_a(PAR, 1, e % A1, e / A1);
-          if (P == 2) read_a(PAR ^ 1, 0, e % A0, e / A0);
-          if (P == 3) read_b(1 ^ PAR, PAR ^ 1, 0, e % (2 * BH), e / (2 * BH));
+          if (P == 0) read_b(1 ^ PAR, PAR, here, 1, e % (2 * BH), e / (2 * BH));
+          if (P == 1) read_a(PAR, here, 1, e % A1, e / A1);
+          if (P == 2) read_a(PAR ^ 1, next, 0, e % A0, e / A0);
+          if (P == 3) read_b(1 ^ PAR, PAR ^ 1, next, 0, e % (2 * BH), e / (2 * BH));
         }
       } else {
 #pragma unroll
         for (int e = (j - J / 2) * RQ / (J / 2); e < (j + 1 - J / 2) * RQ / (J / 2); ++e) {
-          if (P == 0) dma_b(t + 2, PAR, 0, e);
-          if (P == 1) dma_b(t + 2, PAR, 1, e);
-          if (P == 2) dma_a(t + 2, PAR, 1, e);
-          if (P == 3) dma_a(t + 3, PAR ^ 1, 0, e);
+          if (P == 0) dma_b(t + R, PAR, here, 0, e);
+          if (P == 1) dma_b(t + R, PAR, here, 1, e);
+          if (P == 2) dma_a(t + R, PAR, here, 1, e);
+          if (P == 3) dma_a(t + 1 + R, PAR ^ 1, next, 0, e);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -523,15 +547,19 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
     std::integral_constant<int, 1> c1;
     std::integral_constant<int, 2> c2;
     std::integral_constant<int, 3> c3;
+    int s0 = 0;
+    auto after = [](int slot) { return !LONG ? 0 : slot + T::SLOT < T::RING ? slot + T::SLOT : 0; };
     for (int t = 0; t < nk; t += 2) {   // (an odd number of k-tiles ends with one of zeros)
-      phase(c0, c0, t);
-      phase(c0, c1, t);
-      phase(c0, c2, t);
-      phase(c0, c3, t);
-      phase(c1, c0, t + 1);
-      phase(c1, c1, t + 1);
-      phase(c1, c2, t + 1);
-      phase(c1, c3, t + 1);
+      const int s1 = after(s0), s2 = after(s1);
+      phase(c0, c0, t, s0, s1);
+      phase(c0, c1, t, s0, s1);
+      phase(c0, c2, t, s0, s1);
+      phase(c0, c3, t, s0, s1);
+      phase(c1, c0, t + 1, s1, s2);
+      phase(c1, c1, t + 1, s1, s2);
+      phase(c1, c2, t + 1, s1, s2);
+      phase(c1, c3, t + 1, s1, s2);
+      s0 = s2;
     }
   }
   // the last matrix instructions' results can be read (they are assembler text: the wait states are ours), nothing is on its
@@ -565,11 +593,11 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
   if constexpr (MODE != GEMM_ROWS) gemm_store<A, BH, MODE>(acc, gsm + wave * (T::EBYTES / 8), wm, wn, m0, n0, y, ldy, M, N, rp, GROUP ? entry : nullptr);
 }
 
-template <int A, int BH, bool KTAIL, int MODE, bool GROUP, bool NT = false>
-__global__ __launch_bounds__(256, GEMM_PER_CU(A, BH)) void k_gemm_dma(const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
+template <int A, int BH, bool KTAIL, int MODE, bool GROUP, bool NT = false, int R = 2>
+__global__ __launch_bounds__(256, R > 2 && A > 2 ? 1 : GEMM_PER_CU(A, BH)) void k_gemm_dma(const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
                                                                         u16* __restrict__ y, int64_t ldy, int M, int N, int K, int tm, int tn,
                                                                         const GemmRope rp, const GemmSplit sp, const GemmGroup gp) {
-  gemm_tile<A, BH, KTAIL, MODE, GROUP, NT>(blockIdx.x, gridDim.x, x, ldx, w, y, ldy, M, N, K, tm, tn, rp, sp, gp);
+  gemm_tile<A, BH, KTAIL, MODE, GROUP, NT, R>(blockIdx.x, gridDim.x, x, ldx, w, y, ldy, M, N, K, tm, tn, rp, sp, gp);
 }
 
 // Two products of as many rows in one grid, the first `n0` workgroups the first's.  A short prompt's products each leave most
@@ -584,16 +612,16 @@ struct GemmProduct {
   int M, N, K, tm, tn;
   GemmSplit sp;
 };
-template <int A, int BH, int MODE0, int MODE1, bool NT>
+template <int A, int BH, int MODE0, int MODE1, bool NT, int R>
 __global__ __launch_bounds__(256, GEMM_PER_CU(A, BH)) void k_gemm_two(const GemmProduct a, const GemmProduct b, const int n0, const GemmRope rp) {
   const bool second = (int)blockIdx.x >= n0;
   if constexpr (MODE0 == MODE1) {
     const GemmProduct p = second ? b : a;
-    gemm_tile<A, BH, false, MODE0, false, NT>(blockIdx.x - (second ? n0 : 0), 0, p.x, p.ldx, p.w, p.y, p.ldy, p.M, p.N, p.K, p.tm, p.tn, rp, p.sp, GemmGroup{});
+    gemm_tile<A, BH, false, MODE0, false, NT, R>(blockIdx.x - (second ? n0 : 0), 0, p.x, p.ldx, p.w, p.y, p.ldy, p.M, p.N, p.K, p.tm, p.tn, rp, p.sp, GemmGroup{});
   } else if (second) {
-    gemm_tile<A, BH, false, MODE1, false, NT>(blockIdx.x - n0, 0, b.x, b.ldx, b.w, b.y, b.ldy, b.M, b.N, b.K, b.tm, b.tn, GemmRope{}, b.sp, GemmGroup{});
+    gemm_tile<A, BH, false, MODE1, false, NT, R>(blockIdx.x - n0, 0, b.x, b.ldx, b.w, b.y, b.ldy, b.M, b.N, b.K, b.tm, b.tn, GemmRope{}, b.sp, GemmGroup{});
   } else {
-    gemm_tile<A, BH, false, MODE0, false, NT>(blockIdx.x, 0, a.x, a.ldx, a.w, a.y, a.ldy, a.M, a.N, a.K, a.tm, a.tn, rp, a.sp, GemmGroup{});
+    gemm_tile<A, BH, false, MODE0, false, NT, R>(blockIdx.x, 0, a.x, a.ldx, a.w, a.y, a.ldy, a.M, a.N, a.K, a.tm, a.tn, rp, a.sp, GemmGroup{});
   }
 }
 
@@ -603,12 +631,17 @@ __global__ __launch_bounds__(256, GEMM_PER_CU(A, BH)) void k_gemm_two(const Gemm
 // item's request, and the product's workgroups at their ramp and drain.  us per step of the 70B rank shard at 64 rows: the two chains of
 // a block on two branches of the graph 7125, in this grid 6825 (all items behind the tiles 6935, all in front 7059; the plan's three
 // pieces of K, with four 7340), of it per block 38 here, where the product alone takes 28 and the attention alone 16 and 4.
+// An item for every CU, and of more than two rounds one round more, so that a round is left for the CUs whose tiles are done (70B rank
+// shard, 2048 tokens, 64 rows, 768 items: 256 in front 6523 us per step, 512 6296, all 6282; 40 rows, 520 items: 256 5856, 512 5892).
+__device__ __forceinline__ int attn_items_in_front(int items) {
+  return items < ATT_NCU ? items : items <= 2 * ATT_NCU ? ATT_NCU : items - ATT_NCU < 2 * ATT_NCU ? items - ATT_NCU : 2 * ATT_NCU;
+}
 template <int HD, int G, int GROUPS>
 __global__ __launch_bounds__(256, 2) void k_attn_beside_gemm(const AttnItems a, const GemmProduct p, const int n_gemm) {
   extern __shared__ __attribute__((aligned(1024))) u16 gsm[];
-  const int first = a.n_items < ATT_NCU ? a.n_items : ATT_NCU, tile = (int)blockIdx.x - first, wg = tile < 0 ? (int)blockIdx.x : (int)blockIdx.x - n_gemm;
+  const int first = attn_items_in_front(a.n_items), tile = (int)blockIdx.x - first, wg = tile < 0 ? (int)blockIdx.x : (int)blockIdx.x - n_gemm;
   if (tile >= 0 && tile < n_gemm)
-    gemm_tile<2, 1, false, GEMM_PAIR, false, true>(tile, 0, p.x, p.ldx, p.w, p.y, p.ldy, p.M, p.N, p.K, p.tm, p.tn, GemmRope{}, p.sp, GemmGroup{});
+    gemm_tile<2, 1, false, GEMM_PAIR, false, true, GEMM_RING>(tile, 0, p.x, p.ldx, p.w, p.y, p.ldy, p.M, p.N, p.K, p.tm, p.tn, GemmRope{}, p.sp, GemmGroup{});
   else if (wg < a.n_items)
     attn_item<HD, G, GROUPS, true>(a, wg, reinterpret_cast<float*>(gsm));
   else
@@ -712,7 +745,8 @@ struct GemmTileCost {
   int a, bh, per_cu, pieces;   // (pieces: at most)
   float ktile, slope, cold, pair, pair_cold, fixed, store;
 };
-constexpr int GEMM_NTILES = 9, GEMM_TILES_ANY = 4;   // the first four take any K and any number of rows, see gemm_plan
+constexpr int GEMM_NTILES = 10, GEMM_TILES_ANY = 4;   // the first four take any K and any number of rows, see gemm_plan
+constexpr int GEMM_ROWS64 = 3, GEMM_LONG = 9;
 constexpr GemmTileCost GEMM_TILES[GEMM_NTILES] = {{8, 2, 1, 16, 1.2f, 0.0f, 0.0f, 0.0f, 0.0f, 4.35f, 4.43f},
                                                   {4, 2, 1, 16, 0.684f, 0.108f, 0.552f, 0.0f, 0.0f, 2.85f, 1.47f},
                                                   {4, 1, 2, 16, 0.504f, 0.0f, 0.262f, 0.874f, 1.25f, 3.18f, 0.166f},
@@ -721,7 +755,18 @@ constexpr GemmTileCost GEMM_TILES[GEMM_NTILES] = {{8, 2, 1, 16, 1.2f, 0.0f, 0.0f
                                                   {6, 2, 1, 16, 0.953f, 0.0412f, 0.119f, 0.0f, 0.0f, 6.24f, 1.61f},
                                                   {5, 2, 1, 16, 0.668f, 0.2935f, 0.581f, 0.0f, 0.0f, 3.12f, 5.41f},
                                                   {5, 1, 2, 8, 0.553f, 0.0159f, 0.173f, 1.103f, 4.77f, 3.88f, 0.0077f},
-                                                  {6, 1, 1, 16, 0.617f, 0.0f, 0.0944f, 0.0f, 0.0f, 4.28f, 0.0f}};
+                                                  {6, 1, 1, 16, 0.617f, 0.0f, 0.0944f, 0.0f, 0.0f, 4.28f, 0.0f},
+                                                  {4, 1, 1, 16, 0.407f, 0.0508f, 0.206f, 0.0f, 0.0f, 5.0f, 0.101f}};
+// The long rings' costs are fitted to 25 weights of the model families: 17 to 64 rows (92 products; what the plan takes is 0.6 % above the
+// best of the pieces, 6 % at worst; with the ring of two's costs 1.7 and 17 %) and, beside 64 x 128 and 128 x 128, 65 to 128 (66; 0.7 and 6 %).
+constexpr GemmTileCost GEMM_FEW_COST = {2, 1, 2, 16, 0.353f, 0.201f, 0.281f, 0.737f, 1.19f, 3.17f, 0.0f};
+static const GemmTileCost& gemm_cost(int tile, int M) { return tile == GEMM_ROWS64 && M <= 64 ? GEMM_FEW_COST : GEMM_TILES[tile]; }
+// whether a tile serves the product
+static bool gemm_takes(int tile, int M, int K) {
+  if (tile < GEMM_TILES_ANY) return true;
+  if (tile == GEMM_LONG) return M > 64 && M <= 128 && K % 64 == 0;
+  return M > 128 && K % 64 == 0;
+}
 constexpr size_t GEMM_SCRATCH = (size_t)64 << 20;   // pieces of one round of the largest tiles
 constexpr int GEMM_SCRATCH_FROM = 33;               // rows from which a projection that has memory for pieces is one of this file's
 // and from which the two grids of a decode step are, that hold a product beside the attention or another product: below, the
@@ -761,8 +806,9 @@ static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
   if (M > 0x7fffffff - 256 || N > 0x7fffffff - 256 || K > 0x7fffffff - 256) return best;   // (row, column and k of the last tile are ints)
   const int cus = gemm_cus(), nk = (K + 63) / 64;
   const float bytes_us = gemm_bytes_us(M, N, K, mode);
-  for (int c = 0; c < (M > 128 && K % 64 == 0 ? GEMM_NTILES : GEMM_TILES_ANY); ++c) {
-    const GemmTileCost& t = GEMM_TILES[c];
+  for (int c = 0; c < GEMM_NTILES; ++c) {
+    if (!gemm_takes(c, M, K)) continue;
+    const GemmTileCost& t = gemm_cost(c, M);
     const int TM = 32 * t.a, TN = (mode == GEMM_PAIR ? 64 : 128) * t.bh, slots = cus * t.per_cu;
     const int64_t tiles = (int64_t)((M + TM - 1) / TM) * ((N + TN - 1) / TN), rounds = tiles / slots;
     if (tiles > 0x3fffffff) continue;
@@ -784,27 +830,27 @@ static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
   return best;
 }
 
-template <int A, int BH, bool KTAIL, int MODE, bool NT = false>
+template <int A, int BH, bool KTAIL, int MODE, bool NT = false, int R = 2>
 static int gemm_run_as(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, const GemmRope& rp,
                        const GemmPlan& p, void* scratch, hipStream_t s) {
-  using T = GemmTile<A, BH>;
+  using T = GemmTile<A, BH, R>;
   static std::atomic<unsigned long long> raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_dma<A, BH, KTAIL, MODE, false, NT>), T::LDS, raised)) return LR_E_LAUNCH;
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_dma<A, BH, KTAIL, MODE, false, NT, R>), T::LDS, raised)) return LR_E_LAUNCH;
   const int gn = MODE == GEMM_PAIR ? T::TN / 2 : T::TN, tm = (M + T::TM - 1) / T::TM, tn = (N + gn - 1) / gn;
   const GemmSplit sp{(float*)scratch, p.full, p.rem, p.splits};
-  k_gemm_dma<A, BH, KTAIL, MODE, false, NT><<<dim3((unsigned)(p.full + p.rem * p.splits)), dim3(256), T::LDS, s>>>(
+  k_gemm_dma<A, BH, KTAIL, MODE, false, NT, R><<<dim3((unsigned)(p.full + p.rem * p.splits)), dim3(256), T::LDS, s>>>(
       (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, M, N, K, tm, tn, rp, sp, GemmGroup{});
   if constexpr (MODE != GEMM_ROWS)
     if (p.rem) k_gemm_sum<A, BH, MODE><<<dim3((unsigned)(p.rem * A * 4)), dim3(256), 0, s>>>((u16*)y, ldy, M, N, tm, tn, rp, sp);
   return lr_launch_status();
 }
-template <int A, int BH, bool KTAIL, bool NT = false>
+template <int A, int BH, bool KTAIL, bool NT = false, int R = 2>
 static int gemm_run_mode(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, int mode, const GemmRope& rp,
                          const GemmPlan& p, void* scratch, hipStream_t s) {
-  if (mode == GEMM_PAIR) return gemm_run_as<A, BH, KTAIL, GEMM_PAIR, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
-  if (mode == GEMM_ROPE) return gemm_run_as<A, BH, KTAIL, GEMM_ROPE, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
-  if (mode == GEMM_ROWS) return gemm_run_as<A, BH, KTAIL, GEMM_ROWS, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
-  return gemm_run_as<A, BH, KTAIL, GEMM_PLAIN, NT>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+  if (mode == GEMM_PAIR) return gemm_run_as<A, BH, KTAIL, GEMM_PAIR, NT, R>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+  if (mode == GEMM_ROPE) return gemm_run_as<A, BH, KTAIL, GEMM_ROPE, NT, R>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+  if (mode == GEMM_ROWS) return gemm_run_as<A, BH, KTAIL, GEMM_ROWS, NT, R>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
+  return gemm_run_as<A, BH, KTAIL, GEMM_PLAIN, NT, R>(x, ldx, w, y, ldy, M, N, K, rp, p, scratch, s);
 }
 static int gemm_run(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, int mode, const GemmRope& rp,
                     const GemmPlan& p, void* scratch, hipStream_t s) {
@@ -823,9 +869,10 @@ static int gemm_run(const void* x, int64_t ldx, const void* w, void* y, int64_t 
   if (p.tile == 6) return gemm_run_mode<5, 2, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
   if (p.tile == 7) return gemm_run_mode<5, 1, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
   if (p.tile == 8) return gemm_run_mode<6, 1, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+  if (p.tile == GEMM_LONG) return gemm_run_mode<4, 1, false, false, GEMM_RING>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
   if (M <= 64)   // every weight is used once: non-temporal (28672 x 4096 at 64 rows 50.0 -> 46.7 us, 16032 x 8192 61.9 -> 57.5)
-    return kt ? gemm_run_mode<2, 1, true, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
-              : gemm_run_mode<2, 1, false, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
+    return kt ? gemm_run_mode<2, 1, true, true, GEMM_RING>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
+              : gemm_run_mode<2, 1, false, true, GEMM_RING>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
   return kt ? gemm_run_mode<2, 1, true>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s)
             : gemm_run_mode<2, 1, false>(x, ldx, w, y, ldy, M, N, K, mode, rp, p, scratch, s);
 }
@@ -850,13 +897,13 @@ static GemmProduct gemm_product(int tile, int mode, const void* x, int64_t ldx, 
   p.sp.splits = 1;
   return p;
 }
-template <int A, int BH, int MODE0, int MODE1, bool NT>
+template <int A, int BH, int MODE0, int MODE1, bool NT, int R = 2>
 static int gemm_two_as(const GemmProduct& a, const GemmProduct& b, const GemmRope& rp, hipStream_t s) {
-  using T = GemmTile<A, BH>;
+  using T = GemmTile<A, BH, R>;
   static std::atomic<unsigned long long> raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_two<A, BH, MODE0, MODE1, NT>), T::LDS, raised)) return LR_E_LAUNCH;
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_two<A, BH, MODE0, MODE1, NT, R>), T::LDS, raised)) return LR_E_LAUNCH;
   const int n0 = a.sp.full + a.sp.rem * a.sp.splits, n1 = b.sp.full + b.sp.rem * b.sp.splits;
-  k_gemm_two<A, BH, MODE0, MODE1, NT><<<dim3((unsigned)(n0 + n1)), dim3(256), T::LDS, s>>>(a, b, n0, rp);
+  k_gemm_two<A, BH, MODE0, MODE1, NT, R><<<dim3((unsigned)(n0 + n1)), dim3(256), T::LDS, s>>>(a, b, n0, rp);
   return lr_launch_status();
 }
 template <int MODE0, int MODE1>
@@ -864,7 +911,7 @@ static int gemm_two(int tile, const GemmProduct& a, const GemmProduct& b, const 
   if (tile == 0) return gemm_two_as<8, 2, MODE0, MODE1, false>(a, b, rp, s);
   if (tile == 1) return gemm_two_as<4, 2, MODE0, MODE1, false>(a, b, rp, s);
   if (tile == 2) return gemm_two_as<4, 1, MODE0, MODE1, false>(a, b, rp, s);
-  return a.M <= 64 ? gemm_two_as<2, 1, MODE0, MODE1, true>(a, b, rp, s) : gemm_two_as<2, 1, MODE0, MODE1, false>(a, b, rp, s);
+  return a.M <= 64 ? gemm_two_as<2, 1, MODE0, MODE1, true, GEMM_RING>(a, b, rp, s) : gemm_two_as<2, 1, MODE0, MODE1, false>(a, b, rp, s);
 }
 
 namespace lr_detail {
@@ -880,7 +927,7 @@ int gemm_inputs(const void* x0, const void* wqkv, void* qkv, int S, const lr_rop
   float best_us = p0.us + p1.us;
   int best = -1;
   for (int c = 0; c < GEMM_TILES_ANY; ++c) {
-    const GemmTileCost& t = GEMM_TILES[c];
+    const GemmTileCost& t = gemm_cost(c, M);
     const int TM = 32 * t.a, slots = cus * t.per_cu;
     const int64_t tm = (M - 1) / TM + 1, tiles0 = tm * ((N - 1) / (128 * t.bh) + 1), tiles1 = tm * ((I - 1) / (64 * t.bh) + 1), tiles = tiles0 + tiles1;
     // (of several rounds only the last one leaves room, and q/k/v goes cold before the attention reads it: 8 x 2048 tokens of
@@ -902,7 +949,7 @@ int gemm_inputs(const void* x0, const void* wqkv, void* qkv, int S, const lr_rop
 
 template <int HD, int G, int GROUPS>
 static int attn_beside_gemm(const AttnItems& a, const GemmProduct& p, hipStream_t s) {
-  const size_t att = (size_t)attn_item_lds_floats<HD, G>(a.chunk_max) * sizeof(float), lds = att > GemmTile<2, 1>::LDS ? att : GemmTile<2, 1>::LDS;
+  const size_t att = (size_t)attn_item_lds_floats<HD, G>(a.chunk_max) * sizeof(float), lds = att > GemmTile<2, 1, GEMM_RING>::LDS ? att : GemmTile<2, 1, GEMM_RING>::LDS;
   static std::atomic<unsigned long long> raised{0};
   if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_attn_beside_gemm<HD, G, GROUPS>), lds, raised)) return LR_E_LAUNCH;
   const int n = p.sp.full + p.sp.rem * p.sp.splits;
@@ -918,13 +965,13 @@ int gemm_beside_attention(const AttnItems& a, int hd, int G, const void* x, int6
   GemmPlan plan = gemm_plan(M, I, K, GEMM_PAIR, sums_bytes);
   // Of two numbers of pieces that take a product alone as long the smaller: what it leaves is the attention's (70B rank shard, 17 to 24 rows,
   // three pieces or four, a product alone 30.9 us: 24 layers 1629 to 1677 and 1662 to 1711 us).
-  for (const float best = plan.us; plan.tile == 3 && plan.rem;) {
+  for (const float best = plan.us; plan.tile == GEMM_ROWS64 && plan.rem;) {
     const GemmPlan fewer = gemm_plan(M, I, K, GEMM_PAIR, (size_t)plan.rem * plan.splits * GemmTile<2, 1>::TM * GemmTile<2, 1>::TN * sizeof(float) - 1);
-    if (fewer.tile != 3 || fewer.us > 1.003f * best) break;
+    if (fewer.tile != GEMM_ROWS64 || fewer.us > 1.003f * best) break;
     plan = fewer;
   }
-  if (plan.tile != 3) return LR_E_UNSUPPORTED;
-  GemmProduct p = gemm_product(3, GEMM_PAIR, x, ldx, w, y, ldy, M, I, K);
+  if (plan.tile != GEMM_ROWS64) return LR_E_UNSUPPORTED;
+  GemmProduct p = gemm_product(GEMM_ROWS64, GEMM_PAIR, x, ldx, w, y, ldy, M, I, K);
   p.sp = GemmSplit{(float*)sums, plan.full, plan.rem, plan.splits};
   const bool two = attn_two_groups(a.chunk_max);
 #define LR_PRODUCT(HDV, GV) \
@@ -961,7 +1008,7 @@ static GemmOutputs outputs_plan(int M, int N, int K0, int K1, size_t sums_bytes)
   const int cus = gemm_cus(), pairs0 = (K0 / 64 + 1) / 2, pairs1 = (K1 / 64 + 1) / 2;
   const size_t row = (size_t)M * N * sizeof(float);
   for (int c = 0; c < GEMM_TILES_ANY; ++c) {
-    const GemmTileCost& t = GEMM_TILES[c];
+    const GemmTileCost& t = gemm_cost(c, M);
     const int TM = 32 * t.a, TN = 128 * t.bh, slots = cus * t.per_cu;
     const int64_t tiles = (int64_t)((M + TM - 1) / TM) * ((N + TN - 1) / TN);
     for (int s0 = 1; s0 <= 16 && 2 * s0 <= pairs0 + 1 && row * s0 <= sums_bytes; ++s0)

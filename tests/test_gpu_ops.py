@@ -628,6 +628,20 @@ def test_bands_in_slices_of_k(hip, M, K):
     assert_close_ulp(y, linear_ref(x, w), what=f"slices M={M} K={K}")
 
 
+@pytest.mark.parametrize("M,N,K", [(33, 200, 64), (64, 136, 128), (40, 1030, 192), (64, 2000, 832), (48, 264, 8192), (64, 4096, 4160),
+                                   (65, 200, 4096), (96, 264, 8192), (128, 1030, 8192), (127, 4104, 2112), (129, 200, 4160)])
+@pytest.mark.parametrize("memory", [0, 8 << 20])
+def test_products_in_long_rings(hip, M, N, K, memory):
+    """Rings of three k-tiles: fewer k-tiles than slots, odd numbers of them, every column tile's own first k-tile, cut along K or not,
+    rows on both sides of where they are used; columns beyond the last stay."""
+    x, w = rnd(M, K, seed=96), rnd(N, K, seed=97, scale=0.02)
+    scratch = torch.full((memory or 256,), 85, dtype=torch.uint8, device=DEV)
+    y = torch.full((M, N + 8), 3.0, dtype=BF, device=DEV)
+    hip.linear(x, w, y[:, :N], scratch=scratch)
+    assert_close_ulp(y[:, :N].contiguous(), linear_ref(x, w), what=f"long ring M={M} N={N} K={K}")
+    assert bool((y[:, N:] == 3.0).all())
+
+
 @pytest.mark.parametrize("rows,dim", [(2, 4096), (2, 4104), (257, 8192), (3, 8200), (1, 16376)])
 def test_norms_at_the_edges_of_the_lanes_per_row(hip, rows, dim):
     """256 lanes up to 4096 columns, 1024 above; the last columns leave most lanes of the last turn idle."""
