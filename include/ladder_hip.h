@@ -292,6 +292,24 @@ int lr_attn_decode_beside_product(const void* q, int64_t ldq, const void* k_cach
                                   void* tickets, const void* x, int64_t ldx, const void* w, void* act, int64_t ld_act, int M, int N,
                                   int K, void* sums, size_t sums_bytes, lr_stream_t stream);
 
+/* The products of a decode step of 17 to 64 rows on weight-only e4m3 weights (scales: one bf16 per weight row), K % 128 == 0; LR_E_UNSUPPORTED,
+ * nothing launched, for anything else.  A row's sum is scaled in fp32 and rounded once (lr_linear_fp8 rounds it before the scale, too).
+ * lr_linear_fp8_product: y = x (w8 scales)^T; rope not NULL: the q/k/v projection of M sequences' next token, rotated and cached as
+ * lr_linear_rope_kv does.  lr_linear_fp8_product_bytes: the sums_bytes beyond which nothing changes for it or, pair != 0, for w8 of [up; gate] rows
+ * in lr_attn_decode_beside_product_fp8; 0: none are used, or no such product.
+ * lr_attn_decode_beside_product_fp8, lr_linear_fp8_pieces_two and its _bytes (0: not served): as the bf16 ones. */
+size_t lr_linear_fp8_product_bytes(int M, int N, int K, int pair);
+int lr_linear_fp8_product(const void* x, int64_t ldx, const void* w8, const void* scales, void* y, int64_t ldy, int M, int N, int K,
+                          const lr_rope_kv_t* rope, void* sums, size_t sums_bytes, lr_stream_t stream);
+int lr_attn_decode_beside_product_fp8(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos, void* y,
+                                      int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch, size_t scratch_bytes, void* tickets,
+                                      const void* x, int64_t ldx, const void* w8, const void* scales, void* act, int64_t ld_act, int M, int N,
+                                      int K, void* sums, size_t sums_bytes, lr_stream_t stream);
+size_t lr_linear_fp8_pieces_two_bytes(int M, int N, int K0, int K1);
+int lr_linear_fp8_pieces_two(const void* x0, const void* w0, const void* scales0, int K0, void* sums0, int32_t* pieces0, const void* x1,
+                             const void* w1, const void* scales1, int K1, void* sums1, int32_t* pieces1, int M, int N, size_t sums_bytes,
+                             lr_stream_t stream);
+
 /* Weight-only fp8 linear:  y[m, n] = bf16( bf16( sum_k x[m, k] * w8[n, k] ) * scales[n] ).
  * w8 [N, K] dense float8 e4m3 (OCP "e4m3fn": bias 7, no infinities, max 448), one byte per weight;
  * scales [N] bf16, one per output row; x, y bf16 as in lr_linear.  K % 16 == 0.

@@ -201,16 +201,19 @@ struct GemmGroup {
 struct GemmSplit {
   float* part;
   int full, rem, splits;
+  const u16* scales;   // of e4m3 weights, one per weight row
 };
 enum { GEMM_PLAIN, GEMM_PAIR, GEMM_ROPE, GEMM_ROWS };   // ROWS: every tile is cut, the pieces stay, see GemmSplit; PAIR: w holds [up; gate] rows, N counts pairs, output silu(gate) * up
 
-template <int A, int BH, int R = 2>
+template <int A, int BH, int R = 2, bool W8 = false>
 struct GemmTile {
+  static constexpr int KT = W8 ? 128 : 64;               // k elements of a k-tile: 128 bytes of a weight row
+  static constexpr int NA = KT / 64;                     // 64-element parts of its input rows
   static constexpr int TM = 32 * A, TN = 128 * BH;
   static constexpr int A0 = (A + 1) / 2, A1 = A / 2;     // 16-row groups of a wave in either half of the input rows
   static constexpr int NB = 2 * BH;                      // DMA instructions of a wave for half a k-tile of weights (of input rows: A0, A1)
   static constexpr int HB = 8192 * BH;                   // its bytes
-  static constexpr int ABYTES = 4096 * A;                // and those of a k-tile of input rows
+  static constexpr int ABYTES = 4096 * A * NA;           // and those of a k-tile of input rows
   static constexpr int SLOT = ABYTES + 2 * HB;           // a k-tile
   static constexpr int RING = R * SLOT;
   static constexpr int EPITCH = 64 * BH + 8;             // row pitch of a wave's output piece (plain), in elements
@@ -233,6 +236,12 @@ __device__ __forceinline__ void dma16(const i32x4_t& rsrc, int voff, int soff, u
     asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"{m0}"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
   else
     asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+}
+// the low (HI == false) or high two e4m3 values of a dword as a packed bf16 pair (exact)
+template <bool HI>
+__device__ __forceinline__ u32 gemm_fp8_pair(u32 v) {
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(u32, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 1.0f, HI));
 }
 template <int N>
 __device__ __forceinline__ void wait_requests_and_lds() {
@@ -363,20 +372,28 @@ __device__ __forceinline__ void gemm_store(const f32x4_t (&acc)[A][4 * BH], u16*
 
 // KTAIL: K is not a multiple of the 64-element k-tile, so the last one needs a per-lane range check.  NT: weights are loaded
 // non-temporally.
-template <int A, int BH, bool KTAIL, int MODE, bool GROUP, bool NT, int R = 2>
+// W8: e4m3 weights with a bf16 scale per row, K % 128 == 0.  A k-tile is 128 elements: as many bytes of a weight row as of 64 in bf16 and
+// two parts of the input rows.  A lane takes sixteen consecutive k of its row in one LDS read, expands them on their way into the
+// matrix instructions (exactly: e4m3 is a subset of bf16) and multiplies them by the input's same sixteen, eight and eight; the sums are
+// scaled as they are, in fp32, before anything else sees them.  The ring holds two k-tiles, 64 KiB, so that two workgroups share a CU.
+// Bound: what a CU draws, of which the input rows are half (58 GB/s: 0.55 us per k-tile), below HBM's rate.  us, 64 rows, in passes of 16
+// through the bands / here: 14336 x 4096 pairs 160 / 26.2, 8B decode step 10154 / 3505; 70B rank shard 14067 / 4843, 17 rows 6298 / 4120.
+template <int A, int BH, bool KTAIL, int MODE, bool GROUP, bool NT, int R = 2, bool W8 = false>
 __device__ __forceinline__ void gemm_tile(const int block, const int blocks, const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
                                           u16* __restrict__ y, int64_t ldy, int M, int N, int K, int tm, int tn, const GemmRope& rp,
                                           const GemmSplit& sp, const GemmGroup& gp) {
-  using T = GemmTile<A, BH, R>;
+  using T = GemmTile<A, BH, R, W8>;
+  static_assert(!W8 || (!KTAIL && !GROUP), "");
   // Where k-tile t lies in LDS: of a ring of two by its parity, a constant; else a slot is input rows and weight rows together, at
   // an offset that goes round with the loop.
-  constexpr bool LONG = R > 2;
+  constexpr bool LONG = R > 2 || W8;
+  constexpr int KT = T::KT, NA = T::NA, KS = KT / 32, WB = W8 ? 1 : 2;   // (KS: k-steps; WB: bytes per weight)
   constexpr int A0 = T::A0, A1 = T::A1, HB = T::HB, NB = T::NB, BOFF = LONG ? T::ABYTES : 2 * T::ABYTES;
   constexpr int APAR = LONG ? 0 : T::ABYTES, BPAR = LONG ? 0 : 2 * HB;
   extern __shared__ __attribute__((aligned(1024))) u16 gsm[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
-  int mt, nt, piece = -1, kt0 = 0, nk = (K + 63) / 64;
+  int mt, nt, piece = -1, kt0 = 0, nk = (K + KT - 1) / KT;
   int32_t* const entry = reinterpret_cast<int32_t*>(gsm + T::LDS / 2);   // (GROUP) the tile's entries
   if constexpr (GROUP) {
     const int id = xcd_run(block, blocks);   // a row tile's column tiles one after the other
@@ -408,10 +425,10 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
   // Requests.  Instruction i of a wave's share of a half covers the half's rows (wave * n + i) * 8 + lane / 8, a lane 16
   // bytes of one.  Operand rows are read through buffer resources that hold the tile's rows and no more; a row beyond M or N
   // has an offset outside the resource and reads as zero.
-  const u16* const xb = x + (int64_t)m0 * ldx + kt0 * 64;
-  const u16* const wb = w + (int64_t)n0 * K + kt0 * 64;
+  const u16* const xb = x + (int64_t)m0 * ldx + kt0 * KT;
+  const u16* const wb = reinterpret_cast<const u16*>(reinterpret_cast<const char*>(w) + ((int64_t)n0 * K + kt0 * KT) * WB);
   constexpr int OUT = (int)0x80000000;
-  const int klen = K - kt0 * 64;
+  const int klen = K - kt0 * KT;
   const int chunk = ((lane & 7) ^ (lane >> 3)) * 8;      // (row % 8 == lane / 8)
   int xo[2][A0], wo[2][NB];
 #pragma unroll
@@ -425,16 +442,16 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
       const int r = (wave * NB + i) * 8 + (lane >> 3);
-      if (MODE == GEMM_PAIR) wo[h][i] = n0 + r < N ? (int)((int64_t)(h * N + r) * K * 2) + chunk * 2 : OUT;   // (half 0 up, half 1 gate)
-      else wo[h][i] = n0 + h * 64 * BH + r < N ? (int)((int64_t)(h * 64 * BH + r) * K * 2) + chunk * 2 : OUT;
+      if (MODE == GEMM_PAIR) wo[h][i] = n0 + r < N ? (int)((int64_t)(h * N + r) * K * WB) + chunk * 2 : OUT;   // (half 0 up, half 1 gate)
+      else wo[h][i] = n0 + h * 64 * BH + r < N ? (int)((int64_t)(h * 64 * BH + r) * K * WB) + chunk * 2 : OUT;
     }
   }
   const u32 lds0 = __builtin_amdgcn_readfirstlane((u32)(uintptr_t)(__attribute__((address_space(3))) u16*)gsm);
   const int64_t xlast = GROUP ? gp.xrows - 1 : (M - m0 < T::TM ? M - m0 : T::TM) - 1;
   const int64_t wlast = MODE == GEMM_PAIR ? N + (int64_t)(N - n0 < T::TN / 2 ? N - n0 : T::TN / 2) - 1 : (N - n0 < T::TN ? N - n0 : T::TN) - 1;
-  const int xbytes = (int)((xlast * ldx + klen) * 2), wbytes = (int)((wlast * K + klen) * 2);   // (below 2 GiB: gemm_reaches)
+  const int xbytes = (int)((xlast * ldx + klen) * 2), wbytes = (int)((wlast * K + klen) * WB);   // (below 2 GiB: gemm_reaches)
   const int turn = LONG ? (int)((unsigned)(nt * GEMM_TURN) % (unsigned)nk) : 0;   // the k-tile that is multiplied first
-  auto request = [&](auto ONCE, const u16* base, int bytes, int voff, int t, u32 lds) {
+  auto request = [&](auto ONCE, const u16* base, int bytes, int voff, int t, int per, int part, u32 lds) {   // (per: bytes of a row in a k-tile)
     const bool in = t < nk;
     if (LONG) t = t + turn < nk ? t + turn : t + turn - nk;
     i32x4_t r;
@@ -443,13 +460,15 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
     r.z = in ? bytes : 0;
     r.w = 0x00020000;
     if (KTAIL) voff = t * 64 + chunk < klen ? voff : OUT;
-    dma16<decltype(ONCE)::value>(r, voff, in ? t * 128 : 0, lds);
+    dma16<decltype(ONCE)::value>(r, voff, in ? t * per + part * 128 : 0, lds);
   };
-  auto dma_a = [&](int t, int par, int slot, int h, int i) {
-    request(std::false_type{}, xb, xbytes, xo[h][i], t, lds0 + slot + par * APAR + h * 4096 * A0 + (wave * (h ? A1 : A0) + i) * 1024);
+  auto dma_a = [&](int t, int par, int slot, int h, int e) {   // part e % NA of the wave's e / NA-th rows
+    const int i = e / NA, part = e % NA;
+    request(std::false_type{}, xb, xbytes, xo[h][i], t, 2 * KT, part,
+            lds0 + slot + par * APAR + part * 4096 * A + h * 4096 * A0 + (wave * (h ? A1 : A0) + i) * 1024);
   };
   auto dma_b = [&](int t, int par, int slot, int h, int i) {
-    request(std::bool_constant<NT>{}, wb, wbytes, wo[h][i], t, lds0 + slot + BOFF + par * BPAR + h * HB + (wave * NB + i) * 1024);
+    request(std::bool_constant<NT>{}, wb, wbytes, wo[h][i], t, 128, 0, lds0 + slot + BOFF + par * BPAR + h * HB + (wave * NB + i) * 1024);
   };
 
   f32x4_t acc[A][4 * BH];
@@ -459,69 +478,103 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
     for (int b = 0; b < 4 * BH; ++b)
 #pragma unroll
       for (int v = 0; v < 4; ++v) acc[a][b][v] = 0.0f;
-  bf16x8_t af[2][A0][2], bf[2][2 * BH][2];
+  bf16x8_t af[2][A0][KS], bf[2][2 * BH][KS];
+  u32x4_t raw[2 * BH][2];   // (W8) half a k-tile's weights as they are: sixteen consecutive k of a lane's row, twice
   const char* const smb = reinterpret_cast<const char*>(gsm);
   int fa[2][2], fb[2];
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
     const int c = ((4 * ks + (lane >> 4)) ^ (lane & 7)) * 16;
-    fa[0][ks] = (wm * 16 * A0 + (lane & 15)) * 128 + c;
-    fa[1][ks] = (wm * 16 * A1 + (lane & 15)) * 128 + c;
+    const int ca = W8 ? ((2 * (lane >> 4) + ks) ^ (lane & 7)) * 16 : c;   // (W8: the k of the lane's weights, eight and eight)
+    fa[0][ks] = (wm * 16 * A0 + (lane & 15)) * 128 + ca;
+    fa[1][ks] = (wm * 16 * A1 + (lane & 15)) * 128 + ca;
     fb[ks] = (wn * 32 * BH + (lane & 15)) * 128 + c + BOFF;
   }
   auto read_a = [&](int par, int slot, int h, int t, int ks) {
-    af[h][t][ks] = *reinterpret_cast<const bf16x8_t*>(smb + (fa[h][ks] + slot) + par * APAR + h * 4096 * A0 + t * 2048);
+    af[h][t][ks] = *reinterpret_cast<const bf16x8_t*>(smb + (fa[h][ks & 1] + slot) + par * APAR + (ks >> 1) * 4096 * A + h * 4096 * A0 + t * 2048);
   };
-  auto read_b = [&](int set, int par, int slot, int h, int t, int ks) {
-    bf[set][t][ks] = *reinterpret_cast<const bf16x8_t*>(smb + (fb[ks] + slot) + par * BPAR + h * HB + t * 2048);
+  auto read_b = [&](int set, int par, int slot, int h, int t, int ks) {   // (W8: ks half the k-steps)
+    const char* const at = smb + (fb[ks] + slot) + par * BPAR + h * HB + t * 2048;
+    if constexpr (W8) raw[t][ks] = *reinterpret_cast<const u32x4_t*>(at);
+    else bf[set][t][ks] = *reinterpret_cast<const bf16x8_t*>(at);
+  };
+  auto expand = [&](int half) {   // what read_b has read, as bf16 (exactly)
+#pragma unroll
+    for (int t = 0; t < 2 * BH; ++t)
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const u32 lo = raw[t][ks >> 1][2 * (ks & 1)], hi = raw[t][ks >> 1][2 * (ks & 1) + 1];
+        const u32x4_t v = {gemm_fp8_pair<false>(lo), gemm_fp8_pair<true>(lo), gemm_fp8_pair<false>(hi), gemm_fp8_pair<true>(hi)};
+        if constexpr (W8) bf[half][t][ks] = __builtin_bit_cast(bf16x8_t, v);
+      }
   };
   auto barrier = [&] {
     asm volatile("s_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  constexpr int AHEAD = (R - 2) * (A + 2 * NB);   // requests of a wave beyond those of two k-tiles
+  constexpr int QA0 = NA * A0, QA1 = NA * A1, QA = QA0 + QA1, AHEAD = (R - 2) * (QA + 2 * NB);   // requests of a wave; those beyond two k-tiles'
+  // the scales of the lane's columns, ahead of the requests that are counted
+  float scale[2 * BH * 2][4];
+  if constexpr (W8) {
+#pragma unroll
+    for (int b = 0; b < 4 * BH; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int half = b / (2 * BH), c = n0 + (MODE == GEMM_PAIR ? 0 : half * 64 * BH) + wn * 32 * BH + b % (2 * BH) * 16 + (lane >> 4) * 4 + e;
+        scale[b][e] = bf_to_f(sp.scales[c < N ? c + (MODE == GEMM_PAIR ? half * N : 0) : 0]);
+      }
+    asm volatile("" ::: "memory");
+  }
 #pragma unroll
   for (int t = 0; t < R; ++t) {
     const int par = t & 1, slot = LONG ? t * T::SLOT : 0;
 #pragma unroll
-    for (int i = 0; i < A0; ++i) dma_a(t, par, slot, 0, i);
+    for (int i = 0; i < QA0; ++i) dma_a(t, par, slot, 0, i);
 #pragma unroll
     for (int i = 0; i < NB; ++i) dma_b(t, par, slot, 0, i);
 #pragma unroll
     for (int i = 0; i < NB; ++i) dma_b(t, par, slot, 1, i);
 #pragma unroll
-    for (int i = 0; i < A1; ++i) dma_a(t, par, slot, 1, i);
+    for (int i = 0; i < QA1; ++i) dma_a(t, par, slot, 1, i);
   }
-  wait_requests_and_lds<AHEAD + A0 + 2 * A1 + 3 * NB>();
+  wait_requests_and_lds<AHEAD + QA0 + 2 * QA1 + 3 * NB>();
   barrier();
 #pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
+  for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
     for (int t = 0; t < A0; ++t) read_a(0, 0, 0, t, ks);
 #pragma unroll
-    for (int t = 0; t < 2 * BH; ++t) read_b(0, 0, 0, 0, t, ks);
+    for (int t = 0; t < 2 * BH; ++t)
+      if (ks < 2) read_b(0, 0, 0, 0, t, ks);
   }
-  wait_requests_and_lds<AHEAD + A0 + 2 * A1 + 3 * NB>();
+  wait_requests_and_lds<AHEAD + QA0 + 2 * QA1 + 3 * NB>();
   barrier();
 #pragma unroll
-  for (int i = 0; i < A0; ++i) dma_a(R, 0, 0, 0, i);
+  for (int i = 0; i < QA0; ++i) dma_a(R, 0, 0, 0, i);
 
   // Phase P of k-tile t (even: PAR 0).  Reads B1 of this tile, A1 of this tile, A0 of the next, B0 of the next; requests
   // B0, B1, A1 of tile t + R and A0 of tile t + 1 + R.  `here`, `next`: the slots of this tile and the next.
   auto phase = [&](auto PAR_, auto P_, int t, int here, int next) {
     constexpr int PAR = decltype(PAR_)::value, P = decltype(P_)::value;
-    constexpr int ah = P >> 1, bh = (P == 1 || P == 2), set = bh ^ PAR;
+    constexpr int ah = P >> 1, bh = (P == 1 || P == 2), set = W8 ? bh : bh ^ PAR;
     // requests younger than the slot read here: those of the six phases since
-    wait_requests_and_lds<AHEAD + (P == 0 ? 2 * A + 2 * NB : P == 1 ? A + A0 + 3 * NB : P == 2 ? A + 4 * NB : A + A1 + 3 * NB)>();
+    wait_requests_and_lds<AHEAD + (P == 0 ? 2 * QA + 2 * NB : P == 1 ? QA + QA0 + 3 * NB : P == 2 ? QA + 4 * NB : QA + QA1 + 3 * NB)>();
     barrier();
-    constexpr int AH = ah ? A1 : A0, J = 4 * AH * BH, RD = P == 1 ? 2 * A1 : P == 2 ? 2 * A0 : 4 * BH, RQ = P == 2 ? A1 : P == 3 ? A0 : NB;
+    constexpr int AH = ah ? A1 : A0, J = 2 * KS * AH * BH, RD = P == 1 ? KS * A1 : P == 2 ? KS * A0 : 4 * BH, RQ = P == 2 ? QA1 : P == 3 ? QA0 : NB;
+    if constexpr (W8 && P < 2) {
+      expand(P);
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int j = 0; j < J; ++j) {
       const int tb = j % (2 * BH), ta = j / (2 * BH) % AH, ks = j / (2 * AH * BH);
-      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
-                   : "+a"(acc[ah * A0 + ta][bh * 2 * BH + tb])
-                   : "v"(bf[set][tb][ks]), "v"(af[ah][ta][ks]));
+      if constexpr (W8)   // (behind vector instructions that write its operand: the compiler sees to the wait states)
+        acc[ah * A0 + ta][bh * 2 * BH + tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[set][tb][ks], af[ah][ta][ks], acc[ah * A0 + ta][bh * 2 * BH + tb], 0, 0, 0);
+      else
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+                     : "+a"(acc[ah * A0 + ta][bh * 2 * BH + tb])
+                     : "v"(bf[set][tb][ks]), "v"(af[ah][ta][ks]));
       if (j < J / 2) {
 #pragma unroll
         for (int e = j * RD / (J / 2); e < (j + 1) * RD / (J / 2); ++e) {
@@ -565,6 +618,13 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
   // the last matrix instructions' results can be read (they are assembler text: the wait states are ours), nothing is on its
   // way into LDS, nobody still reads it
   asm volatile("s_nop 15\n\ts_nop 15\n\ts_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if constexpr (W8)
+#pragma unroll
+    for (int a = 0; a < A; ++a)
+#pragma unroll
+      for (int b = 0; b < 4 * BH; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[a][b][e] *= scale[b][e];
   if constexpr (!GROUP) {
     if constexpr (MODE == GEMM_ROWS) {
       float* const p = sp.part + (int64_t)(piece % sp.splits) * M * N;
@@ -593,11 +653,11 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
   if constexpr (MODE != GEMM_ROWS) gemm_store<A, BH, MODE>(acc, gsm + wave * (T::EBYTES / 8), wm, wn, m0, n0, y, ldy, M, N, rp, GROUP ? entry : nullptr);
 }
 
-template <int A, int BH, bool KTAIL, int MODE, bool GROUP, bool NT = false, int R = 2>
+template <int A, int BH, bool KTAIL, int MODE, bool GROUP, bool NT = false, int R = 2, bool W8 = false>
 __global__ __launch_bounds__(256, R > 2 && A > 2 ? 1 : GEMM_PER_CU(A, BH)) void k_gemm_dma(const u16* __restrict__ x, int64_t ldx, const u16* __restrict__ w,
                                                                         u16* __restrict__ y, int64_t ldy, int M, int N, int K, int tm, int tn,
                                                                         const GemmRope rp, const GemmSplit sp, const GemmGroup gp) {
-  gemm_tile<A, BH, KTAIL, MODE, GROUP, NT, R>(blockIdx.x, gridDim.x, x, ldx, w, y, ldy, M, N, K, tm, tn, rp, sp, gp);
+  gemm_tile<A, BH, KTAIL, MODE, GROUP, NT, R, W8>(blockIdx.x, gridDim.x, x, ldx, w, y, ldy, M, N, K, tm, tn, rp, sp, gp);
 }
 
 // Two products of as many rows in one grid, the first `n0` workgroups the first's.  A short prompt's products each leave most
@@ -612,16 +672,16 @@ struct GemmProduct {
   int M, N, K, tm, tn;
   GemmSplit sp;
 };
-template <int A, int BH, int MODE0, int MODE1, bool NT, int R>
+template <int A, int BH, int MODE0, int MODE1, bool NT, int R, bool W8>
 __global__ __launch_bounds__(256, GEMM_PER_CU(A, BH)) void k_gemm_two(const GemmProduct a, const GemmProduct b, const int n0, const GemmRope rp) {
   const bool second = (int)blockIdx.x >= n0;
   if constexpr (MODE0 == MODE1) {
     const GemmProduct p = second ? b : a;
-    gemm_tile<A, BH, false, MODE0, false, NT, R>(blockIdx.x - (second ? n0 : 0), 0, p.x, p.ldx, p.w, p.y, p.ldy, p.M, p.N, p.K, p.tm, p.tn, rp, p.sp, GemmGroup{});
+    gemm_tile<A, BH, false, MODE0, false, NT, R, W8>(blockIdx.x - (second ? n0 : 0), 0, p.x, p.ldx, p.w, p.y, p.ldy, p.M, p.N, p.K, p.tm, p.tn, rp, p.sp, GemmGroup{});
   } else if (second) {
-    gemm_tile<A, BH, false, MODE1, false, NT, R>(blockIdx.x - n0, 0, b.x, b.ldx, b.w, b.y, b.ldy, b.M, b.N, b.K, b.tm, b.tn, GemmRope{}, b.sp, GemmGroup{});
+    gemm_tile<A, BH, false, MODE1, false, NT, R, W8>(blockIdx.x - n0, 0, b.x, b.ldx, b.w, b.y, b.ldy, b.M, b.N, b.K, b.tm, b.tn, GemmRope{}, b.sp, GemmGroup{});
   } else {
-    gemm_tile<A, BH, false, MODE0, false, NT, R>(blockIdx.x, 0, a.x, a.ldx, a.w, a.y, a.ldy, a.M, a.N, a.K, a.tm, a.tn, rp, a.sp, GemmGroup{});
+    gemm_tile<A, BH, false, MODE0, false, NT, R, W8>(blockIdx.x, 0, a.x, a.ldx, a.w, a.y, a.ldy, a.M, a.N, a.K, a.tm, a.tn, rp, a.sp, GemmGroup{});
   }
 }
 
@@ -636,12 +696,12 @@ __global__ __launch_bounds__(256, GEMM_PER_CU(A, BH)) void k_gemm_two(const Gemm
 __device__ __forceinline__ int attn_items_in_front(int items) {
   return items < ATT_NCU ? items : items <= 2 * ATT_NCU ? ATT_NCU : items - ATT_NCU < 2 * ATT_NCU ? items - ATT_NCU : 2 * ATT_NCU;
 }
-template <int HD, int G, int GROUPS>
+template <int HD, int G, int GROUPS, bool W8>
 __global__ __launch_bounds__(256, 2) void k_attn_beside_gemm(const AttnItems a, const GemmProduct p, const int n_gemm) {
   extern __shared__ __attribute__((aligned(1024))) u16 gsm[];
   const int first = attn_items_in_front(a.n_items), tile = (int)blockIdx.x - first, wg = tile < 0 ? (int)blockIdx.x : (int)blockIdx.x - n_gemm;
   if (tile >= 0 && tile < n_gemm)
-    gemm_tile<2, 1, false, GEMM_PAIR, false, true, GEMM_RING>(tile, 0, p.x, p.ldx, p.w, p.y, p.ldy, p.M, p.N, p.K, p.tm, p.tn, GemmRope{}, p.sp, GemmGroup{});
+    gemm_tile<2, 1, false, GEMM_PAIR, false, true, W8 ? 2 : GEMM_RING, W8>(tile, 0, p.x, p.ldx, p.w, p.y, p.ldy, p.M, p.N, p.K, p.tm, p.tn, GemmRope{}, p.sp, GemmGroup{});
   else if (wg < a.n_items)
     attn_item<HD, G, GROUPS, true>(a, wg, reinterpret_cast<float*>(gsm));
   else
@@ -760,6 +820,7 @@ constexpr GemmTileCost GEMM_TILES[GEMM_NTILES] = {{8, 2, 1, 16, 1.2f, 0.0f, 0.0f
 // The long rings' costs are fitted to 25 weights of the model families: 17 to 64 rows (92 products; what the plan takes is 0.6 % above the
 // best of the pieces, 6 % at worst; with the ring of two's costs 1.7 and 17 %) and, beside 64 x 128 and 128 x 128, 65 to 128 (66; 0.7 and 6 %).
 constexpr GemmTileCost GEMM_FEW_COST = {2, 1, 2, 16, 0.353f, 0.201f, 0.281f, 0.737f, 1.19f, 3.17f, 0.0f};
+constexpr GemmTileCost GEMM_FEW8_COST = {2, 1, 2, 16, 0.547f, 0.201f, 0.242f, 0.8f, 1.405f, 1.78f, 0.0f};   // (64 products of 17 weights: 0.7 % above the best pieces)
 static const GemmTileCost& gemm_cost(int tile, int M) { return tile == GEMM_ROWS64 && M <= 64 ? GEMM_FEW_COST : GEMM_TILES[tile]; }
 // whether a tile serves the product
 static bool gemm_takes(int tile, int M, int K) {
@@ -801,44 +862,51 @@ static int gemm_cus() {
   return cus > 0 ? cus : 256;
 }
 
+// the best of tile c's ways to compute a product of nk k-tiles, if it is better than `best`
+static void gemm_consider(const GemmTileCost& t, int c, int M, int N, int nk, int mode, float bytes_us, size_t scratch, GemmPlan& best) {
+  const int cus = gemm_cus(), TM = 32 * t.a, TN = (mode == GEMM_PAIR ? 64 : 128) * t.bh, slots = cus * t.per_cu;
+  const int64_t tiles = (int64_t)((M + TM - 1) / TM) * ((N + TN - 1) / TN), rounds = tiles / slots;
+  if (tiles > 0x3fffffff) return;
+  const int left = (int)(tiles - rounds * slots);
+  auto round_us = [&](int workgroups, int k) { return gemm_round_us(t, M, cus, workgroups, k); };
+  auto consider = [&](float us, float more, int whole, int cut, int pieces) {
+    us = (us > bytes_us ? us : bytes_us) + more + gemm_store_us(t, whole, cus, mode);
+    if (best.tile < 0 || us < best.us) best = GemmPlan{c, whole, cut, pieces, us};
+  };
+  const float whole = rounds * round_us(slots, nk), fixed = (rounds + (left ? 1 : 0)) * t.fixed;
+  consider(whole + (left ? round_us(left, nk) : 0.0f), fixed, (int)tiles, 0, 1);
+  for (int s = 2; left && s <= t.pieces && 4 * s <= nk && left * s <= slots; ++s) {
+    const size_t bytes = (size_t)left * s * (32 * t.a) * (128 * t.bh) * sizeof(float);
+    if (bytes > scratch) break;
+    consider(whole + round_us(left * s, (nk + s - 1) / s), fixed + GEMM_SUM_US + gemm_trips(s) * GEMM_TRIP_US + bytes / GEMM_PIECE_BYTES_US,
+             (int)tiles - left, left, s);
+  }
+}
 static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
   GemmPlan best{-1, 0, 0, 1, 0.0f};
   if (M > 0x7fffffff - 256 || N > 0x7fffffff - 256 || K > 0x7fffffff - 256) return best;   // (row, column and k of the last tile are ints)
-  const int cus = gemm_cus(), nk = (K + 63) / 64;
   const float bytes_us = gemm_bytes_us(M, N, K, mode);
-  for (int c = 0; c < GEMM_NTILES; ++c) {
-    if (!gemm_takes(c, M, K)) continue;
-    const GemmTileCost& t = gemm_cost(c, M);
-    const int TM = 32 * t.a, TN = (mode == GEMM_PAIR ? 64 : 128) * t.bh, slots = cus * t.per_cu;
-    const int64_t tiles = (int64_t)((M + TM - 1) / TM) * ((N + TN - 1) / TN), rounds = tiles / slots;
-    if (tiles > 0x3fffffff) continue;
-    const int left = (int)(tiles - rounds * slots);
-    auto round_us = [&](int workgroups, int k) { return gemm_round_us(t, M, cus, workgroups, k); };
-    auto consider = [&](float us, float more, int whole, int cut, int pieces) {
-      us = (us > bytes_us ? us : bytes_us) + more + gemm_store_us(t, whole, cus, mode);
-      if (best.tile < 0 || us < best.us) best = GemmPlan{c, whole, cut, pieces, us};
-    };
-    const float whole = rounds * round_us(slots, nk), fixed = (rounds + (left ? 1 : 0)) * t.fixed;
-    consider(whole + (left ? round_us(left, nk) : 0.0f), fixed, (int)tiles, 0, 1);
-    for (int s = 2; left && s <= t.pieces && 4 * s <= nk && left * s <= slots; ++s) {
-      const size_t bytes = (size_t)left * s * (32 * t.a) * (128 * t.bh) * sizeof(float);
-      if (bytes > scratch) break;
-      consider(whole + round_us(left * s, (nk + s - 1) / s), fixed + GEMM_SUM_US + gemm_trips(s) * GEMM_TRIP_US + bytes / GEMM_PIECE_BYTES_US,
-               (int)tiles - left, left, s);
-    }
-  }
+  for (int c = 0; c < GEMM_NTILES; ++c)
+    if (gemm_takes(c, M, K)) gemm_consider(gemm_cost(c, M), c, M, N, (K + 63) / 64, mode, bytes_us, scratch, best);
+  return best;
+}
+// The same for e4m3 weights (K % 128 == 0): tiles of 64 x 128, k-tiles of 128.
+static GemmPlan gemm_plan8(int M, int N, int K, int mode, size_t scratch) {
+  GemmPlan best{-1, 0, 0, 1, 0.0f};
+  if (M < GEMM_BESIDE_FROM || M > 64 || K % 128 || N > 0x7fffffff - 256) return best;
+  gemm_consider(GEMM_FEW8_COST, GEMM_ROWS64, M, N, K / 128, mode, gemm_bytes_us(M, N, K / 2, mode), scratch, best);
   return best;
 }
 
-template <int A, int BH, bool KTAIL, int MODE, bool NT = false, int R = 2>
+template <int A, int BH, bool KTAIL, int MODE, bool NT = false, int R = 2, bool W8 = false>
 static int gemm_run_as(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, const GemmRope& rp,
-                       const GemmPlan& p, void* scratch, hipStream_t s) {
-  using T = GemmTile<A, BH, R>;
+                       const GemmPlan& p, void* scratch, hipStream_t s, const void* scales = nullptr) {
+  using T = GemmTile<A, BH, R, W8>;
   static std::atomic<unsigned long long> raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_dma<A, BH, KTAIL, MODE, false, NT, R>), T::LDS, raised)) return LR_E_LAUNCH;
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_dma<A, BH, KTAIL, MODE, false, NT, R, W8>), T::LDS, raised)) return LR_E_LAUNCH;
   const int gn = MODE == GEMM_PAIR ? T::TN / 2 : T::TN, tm = (M + T::TM - 1) / T::TM, tn = (N + gn - 1) / gn;
-  const GemmSplit sp{(float*)scratch, p.full, p.rem, p.splits};
-  k_gemm_dma<A, BH, KTAIL, MODE, false, NT, R><<<dim3((unsigned)(p.full + p.rem * p.splits)), dim3(256), T::LDS, s>>>(
+  const GemmSplit sp{(float*)scratch, p.full, p.rem, p.splits, (const u16*)scales};
+  k_gemm_dma<A, BH, KTAIL, MODE, false, NT, R, W8><<<dim3((unsigned)(p.full + p.rem * p.splits)), dim3(256), T::LDS, s>>>(
       (const u16*)x, ldx, (const u16*)w, (u16*)y, ldy, M, N, K, tm, tn, rp, sp, GemmGroup{});
   if constexpr (MODE != GEMM_ROWS)
     if (p.rem) k_gemm_sum<A, BH, MODE><<<dim3((unsigned)(p.rem * A * 4)), dim3(256), 0, s>>>((u16*)y, ldy, M, N, tm, tn, rp, sp);
@@ -897,13 +965,13 @@ static GemmProduct gemm_product(int tile, int mode, const void* x, int64_t ldx, 
   p.sp.splits = 1;
   return p;
 }
-template <int A, int BH, int MODE0, int MODE1, bool NT, int R = 2>
+template <int A, int BH, int MODE0, int MODE1, bool NT, int R = 2, bool W8 = false>
 static int gemm_two_as(const GemmProduct& a, const GemmProduct& b, const GemmRope& rp, hipStream_t s) {
-  using T = GemmTile<A, BH, R>;
+  using T = GemmTile<A, BH, R, W8>;
   static std::atomic<unsigned long long> raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_two<A, BH, MODE0, MODE1, NT, R>), T::LDS, raised)) return LR_E_LAUNCH;
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_gemm_two<A, BH, MODE0, MODE1, NT, R, W8>), T::LDS, raised)) return LR_E_LAUNCH;
   const int n0 = a.sp.full + a.sp.rem * a.sp.splits, n1 = b.sp.full + b.sp.rem * b.sp.splits;
-  k_gemm_two<A, BH, MODE0, MODE1, NT, R><<<dim3((unsigned)(n0 + n1)), dim3(256), T::LDS, s>>>(a, b, n0, rp);
+  k_gemm_two<A, BH, MODE0, MODE1, NT, R, W8><<<dim3((unsigned)(n0 + n1)), dim3(256), T::LDS, s>>>(a, b, n0, rp);
   return lr_launch_status();
 }
 template <int MODE0, int MODE1>
@@ -947,35 +1015,39 @@ int gemm_inputs(const void* x0, const void* wqkv, void* qkv, int S, const lr_rop
                                         gemm_product(best, GEMM_PAIR, x1, K, w1, act, I, M, I, K), rp, s);
 }
 
-template <int HD, int G, int GROUPS>
+template <int HD, int G, int GROUPS, bool W8>
 static int attn_beside_gemm(const AttnItems& a, const GemmProduct& p, hipStream_t s) {
-  const size_t att = (size_t)attn_item_lds_floats<HD, G>(a.chunk_max) * sizeof(float), lds = att > GemmTile<2, 1, GEMM_RING>::LDS ? att : GemmTile<2, 1, GEMM_RING>::LDS;
+  using T = GemmTile<2, 1, W8 ? 2 : GEMM_RING, W8>;
+  const size_t att = (size_t)attn_item_lds_floats<HD, G>(a.chunk_max) * sizeof(float), lds = att > T::LDS ? att : T::LDS;
   static std::atomic<unsigned long long> raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_attn_beside_gemm<HD, G, GROUPS>), lds, raised)) return LR_E_LAUNCH;
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_attn_beside_gemm<HD, G, GROUPS, W8>), lds, raised)) return LR_E_LAUNCH;
   const int n = p.sp.full + p.sp.rem * p.sp.splits;
-  k_attn_beside_gemm<HD, G, GROUPS><<<dim3((unsigned)(n + a.n_items + a.mergers())), dim3(256), lds, s>>>(a, p, n);
+  k_attn_beside_gemm<HD, G, GROUPS, W8><<<dim3((unsigned)(n + a.n_items + a.mergers())), dim3(256), lds, s>>>(a, p, n);
   if (p.sp.rem)
     k_gemm_sum<2, 1, GEMM_PAIR><<<dim3((unsigned)(p.sp.rem * 2 * 4)), dim3(256), 0, s>>>(p.y, p.ldy, p.M, p.N, p.tm, p.tn, GemmRope{}, p.sp);
   return lr_launch_status();
 }
-// lr_attn_decode_beside_product, arguments checked; LR_E_UNSUPPORTED, nothing launched, where the product is none of 64-row tiles
-int gemm_beside_attention(const AttnItems& a, int hd, int G, const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int I, int K,
-                          void* sums, size_t sums_bytes, hipStream_t s) {
-  if (M < GEMM_BESIDE_FROM || M > 64 || K % 64 || !gemm_reaches(ldx, I, K, GEMM_PAIR)) return LR_E_UNSUPPORTED;
-  GemmPlan plan = gemm_plan(M, I, K, GEMM_PAIR, sums_bytes);
+// lr_attn_decode_beside_product, arguments checked; LR_E_UNSUPPORTED, nothing launched, where the product is none of 64-row tiles.
+// scales: of e4m3 weights.
+template <bool W8>
+int gemm_beside_attention(const AttnItems& a, int hd, int G, const void* x, int64_t ldx, const void* w, const void* scales, void* y, int64_t ldy,
+                          int M, int I, int K, void* sums, size_t sums_bytes, hipStream_t s) {
+  if (M < GEMM_BESIDE_FROM || M > 64 || K % (W8 ? 128 : 64) || !gemm_reaches(ldx, I, K, GEMM_PAIR)) return LR_E_UNSUPPORTED;
+  auto planned = [&](size_t bytes) { return W8 ? gemm_plan8(M, I, K, GEMM_PAIR, bytes) : gemm_plan(M, I, K, GEMM_PAIR, bytes); };
+  GemmPlan plan = planned(sums_bytes);
   // Of two numbers of pieces that take a product alone as long the smaller: what it leaves is the attention's (70B rank shard, 17 to 24 rows,
   // three pieces or four, a product alone 30.9 us: 24 layers 1629 to 1677 and 1662 to 1711 us).
   for (const float best = plan.us; plan.tile == GEMM_ROWS64 && plan.rem;) {
-    const GemmPlan fewer = gemm_plan(M, I, K, GEMM_PAIR, (size_t)plan.rem * plan.splits * GemmTile<2, 1>::TM * GemmTile<2, 1>::TN * sizeof(float) - 1);
+    const GemmPlan fewer = planned((size_t)plan.rem * plan.splits * GemmTile<2, 1>::TM * GemmTile<2, 1>::TN * sizeof(float) - 1);
     if (fewer.tile != GEMM_ROWS64 || fewer.us > 1.003f * best) break;
     plan = fewer;
   }
   if (plan.tile != GEMM_ROWS64) return LR_E_UNSUPPORTED;
   GemmProduct p = gemm_product(GEMM_ROWS64, GEMM_PAIR, x, ldx, w, y, ldy, M, I, K);
-  p.sp = GemmSplit{(float*)sums, plan.full, plan.rem, plan.splits};
+  p.sp = GemmSplit{(float*)sums, plan.full, plan.rem, plan.splits, (const u16*)scales};
   const bool two = attn_two_groups(a.chunk_max);
 #define LR_PRODUCT(HDV, GV) \
-  if (hd == HDV && G == GV) return two ? attn_beside_gemm<HDV, GV, 2>(a, p, s) : attn_beside_gemm<HDV, GV, 4>(a, p, s);
+  if (hd == HDV && G == GV) return two ? attn_beside_gemm<HDV, GV, 2, W8>(a, p, s) : attn_beside_gemm<HDV, GV, 4, W8>(a, p, s);
   LR_PRODUCT(128, 1) LR_PRODUCT(128, 2) LR_PRODUCT(128, 4) LR_PRODUCT(128, 8)
   LR_PRODUCT(64, 1) LR_PRODUCT(64, 2) LR_PRODUCT(64, 4) LR_PRODUCT(64, 8)
 #undef LR_PRODUCT
@@ -997,18 +1069,21 @@ int gemm_pieces(const void* x, int64_t ldx, const void* w, int M, int N, int K, 
 struct GemmOutputs {
   int tile, s0, s1;   // tile -1: the two are faster
 };
+template <bool W8 = false>
 static GemmOutputs outputs_plan(int M, int N, int K0, int K1, size_t sums_bytes) {
+  constexpr int KT = W8 ? 128 : 64;
   GemmOutputs best{-1, 1, 1};
-  if (N % 4 || K0 % 64 || K1 % 64 || !gemm_reaches(K0, N, K0, GEMM_PLAIN) || !gemm_reaches(K1, N, K1, GEMM_PLAIN)) return best;
-  const GemmPlan p0 = gemm_plan(M, N, K0, GEMM_PLAIN, sums_bytes), p1 = gemm_plan(M, N, K1, GEMM_PLAIN, sums_bytes);
+  if (N % 4 || K0 % KT || K1 % KT || !gemm_reaches(K0, N, K0, GEMM_PLAIN) || !gemm_reaches(K1, N, K1, GEMM_PLAIN)) return best;
+  auto planned = [&](int K) { return W8 ? gemm_plan8(M, N, K, GEMM_PLAIN, sums_bytes) : gemm_plan(M, N, K, GEMM_PLAIN, sums_bytes); };
+  const GemmPlan p0 = planned(K0), p1 = planned(K1);
   if (p0.tile < 0 || p1.tile < 0) return best;
-  const float bytes_us = gemm_bytes_us(M, N, K0, GEMM_ROWS) + gemm_bytes_us(M, N, K1, GEMM_ROWS);
+  const float bytes_us = gemm_bytes_us(M, N, W8 ? K0 / 2 : K0, GEMM_ROWS) + gemm_bytes_us(M, N, W8 ? K1 / 2 : K1, GEMM_ROWS);
   auto alone = [](const GemmPlan& p) { return p.us - (p.rem && !p.full ? GEMM_SUM_US : 0.0f); };   // (its sum would be the norms' too)
-  float best_us = alone(p0) + alone(p1);
-  const int cus = gemm_cus(), pairs0 = (K0 / 64 + 1) / 2, pairs1 = (K1 / 64 + 1) / 2;
+  float best_us = W8 ? 1e30f : alone(p0) + alone(p1);   // (e4m3: there is no other way to leave pieces)
+  const int cus = gemm_cus(), pairs0 = (K0 / KT + 1) / 2, pairs1 = (K1 / KT + 1) / 2;
   const size_t row = (size_t)M * N * sizeof(float);
-  for (int c = 0; c < GEMM_TILES_ANY; ++c) {
-    const GemmTileCost& t = gemm_cost(c, M);
+  for (int c = W8 ? GEMM_ROWS64 : 0; c < GEMM_TILES_ANY; ++c) {
+    const GemmTileCost& t = W8 ? GEMM_FEW8_COST : gemm_cost(c, M);
     const int TM = 32 * t.a, TN = 128 * t.bh, slots = cus * t.per_cu;
     const int64_t tiles = (int64_t)((M + TM - 1) / TM) * ((N + TN - 1) / TN);
     for (int s0 = 1; s0 <= 16 && 2 * s0 <= pairs0 + 1 && row * s0 <= sums_bytes; ++s0)
@@ -1025,18 +1100,19 @@ static GemmOutputs outputs_plan(int M, int N, int K0, int K1, size_t sums_bytes)
   return best;
 }
 // Bytes for either of the two with which the plan is that of all the memory it could ask for; 0: two launches.
+template <bool W8>
 static size_t outputs_bytes(int M, int N, int K0, int K1) {
-  const GemmOutputs p = M < GEMM_BESIDE_FROM ? GemmOutputs{-1, 1, 1} : outputs_plan(M, N, K0, K1, GEMM_SCRATCH);
+  const GemmOutputs p = M < GEMM_BESIDE_FROM ? GemmOutputs{-1, 1, 1} : outputs_plan<W8>(M, N, K0, K1, GEMM_SCRATCH);
   return p.tile < 0 ? 0 : (size_t)M * N * sizeof(float) * (p.s0 > p.s1 ? p.s0 : p.s1);
 }
 bool gemm_outputs_pay(int M, int N, int K0, int K1, size_t sums_bytes) {
-  return M >= GEMM_SCRATCH_FROM && outputs_plan(M, N, K0, K1, sums_bytes).tile >= 0;
+  return M >= GEMM_SCRATCH_FROM && outputs_plan<>(M, N, K0, K1, sums_bytes).tile >= 0;
 }
 int gemm_outputs(const void* x0, const void* w0, int K0, void* sums0, int* pieces0, const void* x1, const void* w1, int K1, void* sums1, int* pieces1,
                  int M, int N, size_t sums_bytes, hipStream_t s) {
   if (lr_misaligned(sums0) || lr_misaligned(sums1)) return LR_E_ALIGN;
   if (M < GEMM_BESIDE_FROM) return LR_E_UNSUPPORTED;
-  const GemmOutputs p = outputs_plan(M, N, K0, K1, sums_bytes);
+  const GemmOutputs p = outputs_plan<>(M, N, K0, K1, sums_bytes);
   if (p.tile < 0) return LR_E_UNSUPPORTED;
   GemmProduct a = gemm_product(p.tile, GEMM_ROWS, x0, K0, w0, nullptr, 0, M, N, K0), b = gemm_product(p.tile, GEMM_ROWS, x1, K1, w1, nullptr, 0, M, N, K1);
   a.sp = GemmSplit{(float*)sums0, 0, a.sp.full, p.s0};
@@ -1044,6 +1120,19 @@ int gemm_outputs(const void* x0, const void* w0, int K0, void* sums0, int* piece
   *pieces0 = p.s0;
   *pieces1 = p.s1;
   return gemm_two<GEMM_ROWS, GEMM_ROWS>(p.tile, a, b, GemmRope{}, s);
+}
+// The same of e4m3 weights; there is no other way to leave their pieces.
+static int gemm_outputs8(const void* x0, const void* w0, const void* scales0, int K0, void* sums0, int* pieces0, const void* x1, const void* w1,
+                         const void* scales1, int K1, void* sums1, int* pieces1, int M, int N, size_t sums_bytes, hipStream_t s) {
+  if (lr_misaligned(sums0) || lr_misaligned(sums1)) return LR_E_ALIGN;
+  const GemmOutputs p = outputs_plan<true>(M, N, K0, K1, sums_bytes);
+  if (p.tile < 0) return LR_E_UNSUPPORTED;
+  GemmProduct a = gemm_product(GEMM_ROWS64, GEMM_ROWS, x0, K0, w0, nullptr, 0, M, N, K0), b = gemm_product(GEMM_ROWS64, GEMM_ROWS, x1, K1, w1, nullptr, 0, M, N, K1);
+  a.sp = GemmSplit{(float*)sums0, 0, a.sp.full, p.s0, (const u16*)scales0};
+  b.sp = GemmSplit{(float*)sums1, 0, b.sp.full, p.s1, (const u16*)scales1};
+  *pieces0 = p.s0;
+  *pieces1 = p.s1;
+  return gemm_two_as<2, 1, GEMM_ROWS, GEMM_ROWS, true, 2, true>(a, b, GemmRope{}, s);
 }
 }  // namespace lr_detail
 
@@ -1231,10 +1320,10 @@ extern "C" int lr_linear_swiglu_out(const void* x, int64_t ldx, const void* w, v
   return lr_linear_swiglu_out_scratch(x, ldx, w, y, ldy, M, N, K, scratch, scratch_bytes, nullptr, 0, stream);
 }
 
-extern "C" int lr_attn_decode_beside_product(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos, void* y,
-                                             int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch, size_t scratch_bytes,
-                                             void* tickets, const void* x, int64_t ldx, const void* w, void* act, int64_t ld_act, int M, int N,
-                                             int K, void* sums, size_t sums_bytes, lr_stream_t stream) {
+static int beside_product(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos, void* y, int64_t ldy, int B,
+                          int Hq, int Hkv, int hd, int Smax, void* scratch, size_t scratch_bytes, void* tickets, const void* x, int64_t ldx,
+                          const void* w, const void* scales, void* act, int64_t ld_act, int M, int N, int K, void* sums, size_t sums_bytes,
+                          lr_stream_t stream) {
   AttnItems a;
   int G;
   const int rc = attn_fill_items(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, tickets, a, G);
@@ -1247,11 +1336,87 @@ extern "C" int lr_attn_decode_beside_product(const void* q, int64_t ldq, const v
   if (M <= 0 || N <= 0 || K <= 0 || N % 2 || ldx < K || ld_act < N / 2) return LR_E_SHAPE;
   if (K % 8 || ldx % 8) return LR_E_ALIGN;
   if (rc != LR_OK || a.tickets == nullptr) return LR_E_UNSUPPORTED;
-  return lr_detail::gemm_beside_attention(a, hd, G, x, ldx, w, act, ld_act, M, N / 2, K, sums, sums ? sums_bytes : 0, (hipStream_t)stream);
+  auto run = scales ? &lr_detail::gemm_beside_attention<true> : &lr_detail::gemm_beside_attention<false>;
+  return run(a, hd, G, x, ldx, w, scales, act, ld_act, M, N / 2, K, sums, sums ? sums_bytes : 0, (hipStream_t)stream);
+}
+
+extern "C" int lr_attn_decode_beside_product(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos, void* y,
+                                             int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch, size_t scratch_bytes,
+                                             void* tickets, const void* x, int64_t ldx, const void* w, void* act, int64_t ld_act, int M, int N,
+                                             int K, void* sums, size_t sums_bytes, lr_stream_t stream) {
+  return beside_product(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, tickets, x, ldx, w, nullptr, act,
+                        ld_act, M, N, K, sums, sums_bytes, stream);
+}
+
+extern "C" int lr_attn_decode_beside_product_fp8(const void* q, int64_t ldq, const void* k_cache, const void* v_cache, const int32_t* pos, void* y,
+                                                 int64_t ldy, int B, int Hq, int Hkv, int hd, int Smax, void* scratch, size_t scratch_bytes,
+                                                 void* tickets, const void* x, int64_t ldx, const void* w8, const void* scales, void* act,
+                                                 int64_t ld_act, int M, int N, int K, void* sums, size_t sums_bytes, lr_stream_t stream) {
+  if (scales == nullptr) return LR_E_NULL;
+  return beside_product(q, ldq, k_cache, v_cache, pos, y, ldy, B, Hq, Hkv, hd, Smax, scratch, scratch_bytes, tickets, x, ldx, w8, scales, act,
+                        ld_act, M, N, K, sums, sums_bytes, stream);
+}
+
+extern "C" size_t lr_linear_fp8_product_bytes(int M, int N, int K, int pair) {
+  if (M <= 0 || N <= 0 || K <= 0 || (pair && N % 2)) return 0;
+  const GemmPlan p = gemm_plan8(M, pair ? N / 2 : N, K, pair ? GEMM_PAIR : GEMM_PLAIN, GEMM_SCRATCH);
+  return p.tile < 0 ? 0 : (size_t)p.rem * (p.rem ? p.splits : 0) * GemmTile<2, 1>::TM * GemmTile<2, 1>::TN * sizeof(float);
+}
+
+extern "C" int lr_linear_fp8_product(const void* x, int64_t ldx, const void* w8, const void* scales, void* y, int64_t ldy, int M, int N, int K,
+                                     const lr_rope_kv_t* rope, void* sums, size_t sums_bytes, lr_stream_t stream) {
+  LR_REQUIRE_PTR(x);
+  LR_REQUIRE_PTR(w8);
+  LR_REQUIRE_PTR(y);
+  LR_OPTIONAL_PTR(sums);
+  if (scales == nullptr) return LR_E_NULL;
+  if (M <= 0 || N <= 0 || K <= 0 || ldx < K || ldy < N) return LR_E_SHAPE;
+  if (K % 16 || ldx % 8) return LR_E_ALIGN;
+  GemmRope rp{};
+  if (rope) {
+    if (rope->pos == nullptr) return LR_E_NULL;
+    LR_REQUIRE_PTR(rope->table);
+    LR_REQUIRE_PTR(rope->k_cache);
+    LR_REQUIRE_PTR(rope->v_cache);
+    if (rope->n_head <= 0 || rope->n_kv_head <= 0 || rope->head_dim <= 0 || rope->smax <= 0 || rope->block_size <= 0 ||
+        (int64_t)(rope->n_head + 2 * (int64_t)rope->n_kv_head) * rope->head_dim != N)
+      return LR_E_SHAPE;
+    if (ldy % 8 || rope->head_dim % 8) return LR_E_ALIGN;
+    rp = GemmRope{(const u16*)rope->table, rope->pos, (u16*)rope->k_cache, (u16*)rope->v_cache, rope->err, 1, rope->n_head,
+                  rope->n_kv_head, rope->head_dim, rope->smax, rope->block_size};
+  }
+  if (!gemm_reaches(ldx, N, K, GEMM_PLAIN)) return LR_E_UNSUPPORTED;
+  const int mode = rope ? GEMM_ROPE : GEMM_PLAIN;
+  const GemmPlan p = gemm_plan8(M, N, K, mode, sums ? sums_bytes : 0);
+  if (p.tile < 0) return LR_E_UNSUPPORTED;
+  hipStream_t s = (hipStream_t)stream;
+  return rope ? gemm_run_as<2, 1, false, GEMM_ROPE, true, 2, true>(x, ldx, w8, y, ldy, M, N, K, rp, p, sums, s, scales)
+              : gemm_run_as<2, 1, false, GEMM_PLAIN, true, 2, true>(x, ldx, w8, y, ldy, M, N, K, rp, p, sums, s, scales);
+}
+
+extern "C" size_t lr_linear_fp8_pieces_two_bytes(int M, int N, int K0, int K1) {
+  return M <= 0 || N <= 0 || K0 <= 0 || K1 <= 0 ? 0 : lr_detail::outputs_bytes<true>(M, N, K0, K1);
+}
+
+extern "C" int lr_linear_fp8_pieces_two(const void* x0, const void* w0, const void* scales0, int K0, void* sums0, int32_t* pieces0, const void* x1,
+                                        const void* w1, const void* scales1, int K1, void* sums1, int32_t* pieces1, int M, int N,
+                                        size_t sums_bytes, lr_stream_t stream) {
+  LR_REQUIRE_PTR(x0);
+  LR_REQUIRE_PTR(w0);
+  LR_REQUIRE_PTR(sums0);
+  LR_REQUIRE_PTR(x1);
+  LR_REQUIRE_PTR(w1);
+  LR_REQUIRE_PTR(sums1);
+  if (scales0 == nullptr || scales1 == nullptr || pieces0 == nullptr || pieces1 == nullptr) return LR_E_NULL;
+  if (M <= 0 || N <= 0 || K0 <= 0 || K1 <= 0) return LR_E_SHAPE;
+  if (K0 % 16 || K1 % 16) return LR_E_ALIGN;
+  const uintptr_t s0 = (uintptr_t)sums0, s1 = (uintptr_t)sums1;
+  if ((s0 > s1 ? s0 - s1 : s1 - s0) < sums_bytes) return LR_E_SHAPE;   // (both are written at the same time)
+  return lr_detail::gemm_outputs8(x0, w0, scales0, K0, sums0, pieces0, x1, w1, scales1, K1, sums1, pieces1, M, N, sums_bytes, (hipStream_t)stream);
 }
 
 extern "C" size_t lr_linear_pieces_two_bytes(int M, int N, int K0, int K1) {
-  return M <= 0 || N <= 0 || K0 <= 0 || K1 <= 0 || K0 % 8 || K1 % 8 ? 0 : lr_detail::outputs_bytes(M, N, K0, K1);
+  return M <= 0 || N <= 0 || K0 <= 0 || K1 <= 0 || K0 % 8 || K1 % 8 ? 0 : lr_detail::outputs_bytes<false>(M, N, K0, K1);
 }
 
 extern "C" int lr_linear_pieces_two(const void* x0, const void* w0, int K0, void* sums0, int32_t* pieces0, const void* x1, const void* w1, int K1,

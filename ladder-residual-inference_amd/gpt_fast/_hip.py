@@ -75,6 +75,15 @@ _PROTOS = {
     "lr_attn_decode_beside_product": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
                                               c_int, c_int, c_int, c_void_p, c_size_t, c_void_p, c_void_p, c_int64, c_void_p,
                                               c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]),
+    "lr_attn_decode_beside_product_fp8": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
+                                                  c_int, c_int, c_int, c_void_p, c_size_t, c_void_p, c_void_p, c_int64, c_void_p, c_void_p,
+                                                  c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p]),
+    "lr_linear_fp8_product_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
+    "lr_linear_fp8_product": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_void_p,
+                                      c_size_t, c_void_p]),
+    "lr_linear_fp8_pieces_two_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
+    "lr_linear_fp8_pieces_two": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
+                                         c_void_p, c_void_p, c_int, c_int, c_size_t, c_void_p]),
     "lr_linear_pieces_two_bytes": (c_size_t, [c_int, c_int, c_int, c_int]),
     "lr_linear_pieces_two": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                                      c_int, c_int, c_size_t, c_void_p]),
@@ -798,6 +807,17 @@ def attn_decode_beside(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, pro
 def attn_decode_beside_product(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, tickets, x, w1, act, sums) -> bool:
     """attn_decode and linear_swiglu_out(x, w1, act, sums=sums) of 17 to 64 rows in one grid; the two must not depend on each
     other.  False, with nothing launched, when the library has no such kernel for the shape.  tickets: as in attn_decode_beside."""
+    return _beside_product("lr_attn_decode_beside_product", q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, tickets, x, w1, (_dev(w1),),
+                           act, sums)
+
+
+def attn_decode_beside_product_fp8(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, tickets, x, w1, act, sums) -> bool:
+    """The same for a weight-only e4m3 module w1 (lr_attn_decode_beside_product_fp8)."""
+    return _beside_product("lr_attn_decode_beside_product_fp8", q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, tickets, x, w1.weight,
+                           _fp8_args(w1.weight, w1.scales), act, sums)
+
+
+def _beside_product(name, q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv, hd, tickets, x, w1, weights, act, sums) -> bool:
     _, _, ldq = _rows_ld(q)
     _, _, ldy = _rows_ld(y)
     M, K, ldx = _rows_ld(x)
@@ -805,14 +825,57 @@ def attn_decode_beside_product(q, k_cache, v_cache, pos, y, scratch, B, Hq, Hkv,
     Mo, Io, ld_act = _rows_ld(act)
     assert pos.dtype == torch.int32 and pos.numel() == 1 and scratch.dtype == torch.float32
     assert w1.is_contiguous() and Kw == K and N % 2 == 0 and (Mo, Io) == (M, N // 2), (x.shape, w1.shape, act.shape)
-    rc = load().lr_attn_decode_beside_product(_dev(q), ldq, _dev(k_cache), _dev(v_cache), pos.data_ptr(), _dev(y), ldy, B, Hq, Hkv,
-                                              hd, k_cache.shape[2], scratch.data_ptr(), scratch.numel() * 4,
-                                              _tickets(tickets, 32 * B * Hq), _dev(x), ldx, _dev(w1), _dev(act), ld_act, M, N, K,
-                                              *_scratch_args(sums), _stream())
+    rc = getattr(load(), name)(_dev(q), ldq, _dev(k_cache), _dev(v_cache), pos.data_ptr(), _dev(y), ldy, B, Hq, Hkv, hd, k_cache.shape[2],
+                               scratch.data_ptr(), scratch.numel() * 4, _tickets(tickets, 32 * B * Hq), _dev(x), ldx, *weights, _dev(act),
+                               ld_act, M, N, K, *_scratch_args(sums), _stream())
     if rc == E_UNSUPPORTED:
         return False
-    _check(rc, "lr_attn_decode_beside_product")
+    _check(rc, name)
     return True
+
+
+def _fp8_args(w8, scales):
+    assert w8.dtype == torch.float8_e4m3fn and w8.is_contiguous() and w8.is_cuda
+    assert scales.dtype == torch.bfloat16 and scales.numel() == w8.shape[0] and scales.is_contiguous()
+    return w8.data_ptr(), _dev(scales)
+
+
+def linear_fp8_product(x, lin, out, sums, rope=None) -> bool:
+    """out = x @ (lin.weight * lin.scales)^T of 17 to 64 rows in cut tiles (lr_linear_fp8_product); rope (rope_kv_epilogue): rotated and
+    cached on its way out.  False, with nothing launched, for other shapes."""
+    M, K, ldx = _rows_ld(x)
+    N, Kw = lin.weight.shape
+    Mo, No, ldy = _rows_ld(out)
+    assert Kw == K and (Mo, No) == (M, N)
+    rc = load().lr_linear_fp8_product(_dev(x), ldx, *_fp8_args(lin.weight, lin.scales), _dev(out), ldy, M, N, K,
+                                      None if rope is None else ctypes.byref(rope), *_scratch_args(sums), _stream())
+    if rc == E_UNSUPPORTED:
+        return False
+    _check(rc, "lr_linear_fp8_product")
+    return True
+
+
+def linear_fp8_product_bytes(M, N, K, pair=False) -> int:
+    return int(load().lr_linear_fp8_product_bytes(M, N, K, int(pair)))
+
+
+def linear_fp8_pieces_two(x0, lin0, sums0, x1, lin1, sums1):
+    """Both products' partial sums (Pieces) of 17 to 64 rows, in one launch (lr_linear_fp8_pieces_two); None, with nothing launched, for
+    shapes it does not serve."""
+    (M, K0), (N, K1) = x0.shape, lin1.weight.shape
+    assert sums0 is not sums1 and x0.is_contiguous() and x1.is_contiguous() and x1.shape == (M, K1) and lin0.weight.shape == (N, K0)
+    n0, n1 = c_int32(), c_int32()
+    (p0, b0), (p1, b1) = _scratch_args(sums0), _scratch_args(sums1)
+    rc = load().lr_linear_fp8_pieces_two(_dev(x0), *_fp8_args(lin0.weight, lin0.scales), K0, p0, ctypes.byref(n0), _dev(x1),
+                                         *_fp8_args(lin1.weight, lin1.scales), K1, p1, ctypes.byref(n1), M, N, min(b0, b1), _stream())
+    if rc == E_UNSUPPORTED:
+        return None
+    _check(rc, "lr_linear_fp8_pieces_two")
+    return Pieces(sums0, n0.value, M, N), Pieces(sums1, n1.value, M, N)
+
+
+def linear_fp8_pieces_two_bytes(M, N, K0, K1) -> int:
+    return int(load().lr_linear_fp8_pieces_two_bytes(M, N, K0, K1))
 
 
 ATTN_DECODE_STATIC_MAX_BYTES = 32 << 20   # LR_ATTN_DECODE_STATIC_MAX_BYTES of include/ladder_hip.h

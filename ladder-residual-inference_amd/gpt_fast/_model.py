@@ -231,11 +231,14 @@ class GPTBase(nn.Module):
             last = lambda t, out: None if t is None else _hip.embed(t.view(B * S, -1), ws.last_rows, out)
             _hip.add_rmsnorm(last(ws.x, ws.xl), last(final_d1, ws.d1l), last(final_d2, ws.d2l), self.norm.weight, None,
                              ws.xnl, cfg.norm_eps)
-            _hip.module_linear(ws.xnl, self.output, ws.logits.view(B, -1), ws.sums)
+            self._linear(ws, ws.xnl, self.output, ws.logits.view(B, -1))
         else:
             _hip.add_rmsnorm(ws.x, final_d1, final_d2, self.norm.weight, None, ws.xn, cfg.norm_eps)
-            _hip.module_linear(ws.xn, self.output, ws.logits.view(B * S, -1), ws.sums)
+            self._linear(ws, ws.xn, self.output, ws.logits.view(B * S, -1))
         return ws.logits
+
+    def _linear(self, ws: Workspace, x: Tensor, lin: nn.Module, out: Tensor):
+        _hip.module_linear(x, lin, out, ws.sums)
 
     def _run_layers(self, ws: Workspace, pos: Tensor):
         """Runs all blocks on ws.x; returns up to two tensors still to be added to ws.x before the

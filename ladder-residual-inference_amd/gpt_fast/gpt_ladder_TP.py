@@ -66,11 +66,21 @@ class GPTLadder(GPTBase):
         return self.config.ladder_layers is None and not hasattr(self.layers[0].attention.wqkv, "scales")   # (lr_ladder_block's)
 
     def _pair_bytes(self, B):
+        c = self.config
+        if c.ladder_layers is None and hasattr(self.layers[0].attention.wqkv, "scales"):
+            outputs = _hip.linear_fp8_pieces_two_bytes(B, c.dim, c.n_head_local * c.head_dim, c.ffn_local)
+            if not outputs or not self._all_fp8():
+                return ()
+            return max(outputs, _hip.linear_fp8_product_bytes(B, 2 * c.ffn_local, c.dim, pair=True),
+                       _hip.linear_fp8_product_bytes(B, self._fused_width(), c.dim),
+                       _hip.linear_fp8_product_bytes(B, c.output_rows, c.dim)), outputs
         if not self._prompt_pieces():
             return ()
-        c = self.config
         outputs = _hip.linear_pieces_two_bytes(B, c.dim, c.n_head_local * c.head_dim, c.ffn_local)
         return max(outputs, _hip.beside_product_bytes(B, 2 * c.ffn_local, c.dim)), outputs
+
+    def _all_fp8(self):
+        return all(hasattr(m, "scales") for b in self.layers for m in (b.attention.wqkv, b.attention.wo, b.feed_forward.w1, b.feed_forward.w2))
 
     def _make_block(self, config, layer_idx):
         return LadderTransformerBlock(config)
@@ -142,8 +152,8 @@ class GPTLadder(GPTBase):
         (w1, SwiGLU, w2) -- one after the other, or on two streams where the reference overlaps an all-reduce with
         the next module (gpt_ladder_TP.py:339-349).  Up to 16 rows the norms launch is only the first block's: from then on
         the output projections update the residual and leave the next block its rows undivided (linear_resid).  17 to 64
-        rows on bf16 weights share a grid between the attention and the up/gate product, and leave both outputs' partial
-        sums to the norms; on e4m3 weights they are passes of up to 16 rows."""
+        rows share a grid between the attention and the up/gate product, and leave both outputs' partial sums to the norms; e4m3
+        weights that those products do not serve (inner dimensions in 128s) are passes of up to 16 rows."""
         cfg = self.config
         eps = cfg.norm_eps
         main = side = None
@@ -171,6 +181,8 @@ class GPTLadder(GPTBase):
         # rows at 1000 tokens 5.78, in bands 7.02
         pair = ws.pair_sums
         products = multi and pair and (two_chains or ws.sums is None) and ws.tickets is not None
+        # the same on e4m3 weights, q/k/v a product of its own at any of these numbers of rows
+        products8 = side is None and fp8 and pair and ws.tickets is not None
         if two_chains:
             cur = torch.cuda.current_stream()
             chain = getattr(self, "_chain_stream", None)
@@ -207,6 +219,13 @@ class GPTLadder(GPTBase):
                 else:
                     _hip.linear(ws.y, att.wo.weight, ws.a, scratch=ws.sums)
                     _hip.linear(ws.act, ff.w2.weight, ws.m, scratch=ws.sums_mlp)
+            elif products8 and (products8 := self._block_products8(ws, blk, pos)):
+                two = _hip.linear_fp8_pieces_two(ws.y, blk.attention.wo, pair[0], ws.act, blk.feed_forward.w2, pair[1]) if after else None
+                if two:
+                    pending_a, pending_m = two
+                    continue
+                self._linear(ws, ws.y, blk.attention.wo, ws.a)
+                self._linear(ws, ws.act, blk.feed_forward.w2, ws.m)
             elif two_chains:
                 chain.wait_stream(cur)
                 with torch.cuda.stream(chain):
@@ -283,6 +302,21 @@ class GPTLadder(GPTBase):
                 else:
                     xn, xn2 = _hip.Normed(ws.xn, ws.sq, eps), _hip.Normed(ws.xn2, ws.sq2, eps)
         return pending_a, pending_m
+
+    def _linear(self, ws: Workspace, x: Tensor, lin, out: Tensor):
+        # (e4m3, 17 to 64 rows: the head 16032 x 8192 of 64 rows in one product instead of four passes)
+        if not (ws.S == 1 and hasattr(lin, "scales") and ws.pair_sums and _hip.linear_fp8_product(x, lin, out, ws.pair_sums[0])):
+            super()._linear(ws, x, lin, out)
+
+    def _block_products8(self, ws: Workspace, blk, pos: Tensor) -> bool:
+        """q/k/v, then the attention in one grid with up/gate, all as e4m3 products of 17 to 64 rows: ws.xn, ws.xn2 -> ws.y, ws.act.
+        False, with ws.qkv and the caches rewritten at most, where the library has no such grid."""
+        cfg, att, ff, kv = self.config, blk.attention, blk.feed_forward, blk.attention.kv_cache
+        heads = cfg.n_head_local, cfg.n_kv_local, cfg.head_dim
+        rope = _hip.rope_kv_epilogue(self.freqs_cis, pos, kv.k_cache, kv.v_cache, *heads)
+        return (_hip.linear_fp8_product(ws.xn, att.wqkv, ws.qkv, ws.pair_sums[0], rope)
+                and _hip.attn_decode_beside_product_fp8(ws.qkv, kv.k_cache, kv.v_cache, pos, ws.y, ws.scratch, ws.B, *heads, ws.tickets,
+                                                        ws.xn2, ff.w1, ws.act, ws.pair_sums[0]))
 
     def _run_layers(self, ws: Workspace, pos: Tensor):
         cfg = self.config

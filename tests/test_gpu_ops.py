@@ -651,6 +651,78 @@ def test_norms_at_the_edges_of_the_lanes_per_row(hip, rows, dim):
 
 # ------------------------------------------------------------------------------------ weight-only fp8 linear
 
+class Fp8Linear:
+    def __init__(self, N, K, seed):
+        self.weight, self.scales = rnd(N, K, seed=seed, scale=20.0).to(torch.float8_e4m3fn), rnd(N, seed=seed + 1).abs() * 1e-3
+
+    def of(self, x):
+        return (x.double() @ self.weight.double().T) * self.scales.double()
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 130, 128), (33, 264, 256), (64, 1030, 384), (40, 128, 640), (64, 1280, 8192), (20, 2048, 4096)])
+@pytest.mark.parametrize("memory", [0, 8 << 20])
+def test_linear_fp8_product(hip, M, N, K, memory):
+    """17 to 64 rows of e4m3 weights in tiles: fewer k-tiles than the ring holds, odd numbers of them, ragged columns, cut along K or not."""
+    x, lin = rnd(M, K, seed=110), Fp8Linear(N, K, 111)
+    y = torch.full((M, N + 8), 3.0, dtype=BF, device=DEV)
+    sums = torch.full((memory or 256,), 255, dtype=torch.uint8, device=DEV)
+    assert hip.linear_fp8_product(x, lin, y[:, :N], sums)
+    assert_close_ulp(y[:, :N].contiguous(), lin.of(x).to(BF), what=f"e4m3 product M={M} N={N} K={K}")
+    assert bool((y[:, N:] == 3.0).all())
+
+
+def test_linear_fp8_product_serves_17_to_64_rows_of_whole_k_tiles(hip):
+    for M, K in ((16, 256), (65, 256), (32, 192)):
+        assert not hip.linear_fp8_product(rnd(M, K), Fp8Linear(64, K, 1), torch.empty(M, 64, dtype=BF, device=DEV), None)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,hd,D,memory", [(17, 8, 1, 128, 512, 8 << 20), (64, 4, 2, 64, 4096, 8 << 20), (33, 8, 2, 128, 256, 0)])
+def test_linear_fp8_product_rotates_and_caches(hip, B, Hq, Hkv, hd, D, memory):
+    """What the plain product followed by lr_rope_kv_write leaves, and no other cache slot touched."""
+    Smax, block, pos_value = 48, 64, 37
+    N = (Hq + 2 * Hkv) * hd
+    x, lin, table = rnd(B, D, seed=40), Fp8Linear(N, D, 41), O.rope_table(block, hd, 10000.0, BF).to(DEV)
+    pos = torch.tensor([pos_value], dtype=torch.int32, device=DEV)
+    kc, vc = ([rnd(B, Hkv, Smax, hd, seed=s) for _ in range(2)] for s in (42, 43))
+    q = torch.empty(2, B, N, dtype=BF, device=DEV)
+    sums = torch.empty(memory or 256, dtype=torch.uint8, device=DEV)
+    assert hip.linear_fp8_product(x, lin, q[0], sums)
+    hip.rope_kv_write(q[0], table, False, pos, kc[0], vc[0], B, 1, Hq, Hkv, hd)
+    assert hip.linear_fp8_product(x, lin, q[1], sums, hip.rope_kv_epilogue(table, pos, kc[1], vc[1], Hq, Hkv, hd))
+    assert torch.equal(q[0], q[1]) and torch.equal(kc[0], kc[1]) and torch.equal(vc[0], vc[1])
+
+
+@pytest.mark.parametrize("B,K,I", [(17, 128, 8192), (64, 8192, 456), (40, 4096, 1000)])
+def test_attn_decode_beside_an_fp8_product(hip, B, K, I):
+    """lr_attn_decode's bits, and the activation of the float64 product (up, gate and silu(gate) are each rounded: one step of any of them
+    is at most 2^-7 of the result)."""
+    Hq, Hkv, hd, Smax, pos = 8, 1, 128, 600, 555
+    q, x, lin = rnd(B, (Hq + 2 * Hkv) * hd, seed=50), rnd(B, K, seed=53), Fp8Linear(2 * I, K, 54)
+    kc, vc = rnd(B, Hkv, Smax, hd, seed=60), rnd(B, Hkv, Smax, hd, seed=80)
+    p, tickets = torch.tensor([pos], dtype=torch.int32, device=DEV), torch.zeros(32 * B * Hq, dtype=torch.int32, device=DEV)
+    scratch = torch.empty(hip.attn_decode_scratch_bytes(B, Hq, hd, Smax) // 4, dtype=torch.float32, device=DEV)
+    y, act = torch.zeros(2, B, Hq * hd, dtype=BF, device=DEV), torch.empty(B, I, dtype=BF, device=DEV)
+    hip.attn_decode(q, kc, vc, p, y[0], scratch, B, Hq, Hkv, hd)
+    sums = torch.empty(max(hip.linear_fp8_product_bytes(B, 2 * I, K, True), 256), dtype=torch.uint8, device=DEV)
+    assert hip.attn_decode_beside_product_fp8(q, kc, vc, p, y[1], scratch, B, Hq, Hkv, hd, tickets, x, lin, act, sums)
+    assert torch.equal(y[0], y[1])
+    u, g = lin.of(x).to(BF).float().chunk(2, 1)
+    want = ((g / (1 + torch.exp(-g))).to(BF).float() * u).to(BF).float()
+    assert ((act.float() - want).abs() <= 2.0 ** -7 * want.abs() + 1e-6 * want.abs().max()).all()
+
+
+@pytest.mark.parametrize("M,D,K0,K1", [(17, 256, 128, 384), (64, 8192, 1024, 3584), (33, 4096, 4096, 14336)])
+def test_fp8_pieces_of_two_products(hip, M, D, K0, K1):
+    """Their sums, added in fp32, against the float64 products."""
+    x, lins = [rnd(M, K, seed=120 + K) for K in (K0, K1)], [Fp8Linear(D, K, 130 + K) for K in (K0, K1)]
+    n = hip.linear_fp8_pieces_two_bytes(M, D, K0, K1)
+    sums = [torch.full((n,), 255, dtype=torch.uint8, device=DEV) for _ in range(2)]
+    for x_, lin, p in zip(x, lins, hip.linear_fp8_pieces_two(x[0], lins[0], sums[0], x[1], lins[1], sums[1])):
+        got = p.sums.view(torch.float32)[:p.count * M * D].view(p.count, M, D).double().sum(0)
+        want = lin.of(x_)
+        assert (got - want).abs().max() <= 2e-6 * want.abs().max() * x_.shape[1] ** 0.5
+
+
 def test_linear_fp8_decodes_every_e4m3_value_exactly(hip):
     """All 254 finite byte patterns of float8_e4m3fn (normals, denormals, both zeros) through the kernel's
     conversion: with one-hot inputs and unit scales the output IS the stored value."""
