@@ -689,6 +689,18 @@ int lr_linear_residual_tanh(const void* x, int64_t ldx, const void* w, int M, in
                             const float* expert_weights, int top, const void* alpha, const void* gain, const void* bias,
                             void* x_compute, lr_stream_t stream);
 
+/* A post-norm sublayer's output projection of up to LR_ROW_NORM_MAX_ROWS rows, with the residual update behind it and what the norm
+ * after that needs (lr_residual_rmsnorm in the launches on either side of it):  with X = resid, or where `before` is given
+ * X = resid / sqrt(mean(resid^2) + before->eps) * (gain_offset + gain_before), before->sums holding the parts of resid's sums of squares,
+ *     resid [M, N] = scale * X + x w^T (fp32),   x_compute [M, N] = bf16(resid * (gain_offset + gain)),
+ *     sums [M, lr_linear_residual_rms_sums(N)] = parts of the new resid's sums of squares:
+ * x_compute and sums are an input of lr_linear_multi_normed, resid, sums and gain what the next call takes as resid, `before` and
+ * gain_before.  `sums` must not be before->sums, whose dim is N.  lr_linear_residual_rms_sums: 0 where rows of N are not served. */
+int lr_linear_residual_rms_sums(int N);
+int lr_linear_residual_rms(const void* x, int64_t ldx, const void* w, int M, int N, int K, float* resid, float scale,
+                           const lr_row_norm_t* before, const void* gain_before, const void* gain, float gain_offset,
+                           void* x_compute, float* sums, lr_stream_t stream);
+
 /* Causal convolution per channel and silu over S consecutive tokens per sequence: out[t, c] =
  * silu(bias[c] + sum_j w[c, j] u[t - (taps - 1) + j, c]).  u [B*S, C] (row stride ldu), w [C, taps] (the last column is the
  * current token's), out [B*S, C] (row stride ldo; not u).  ring [Bmax, taps, C] holds a sequence's last inputs, a token's at

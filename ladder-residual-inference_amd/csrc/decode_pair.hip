@@ -33,7 +33,7 @@ __global__ __launch_bounds__(256, XL ? 0 : 2) void k_attn_beside_band(const Attn
   } else if (MERGE && wg >= a.n_items + p.nwg) {
     attn_merge<HD, G>(a, wg - a.n_items - p.nwg);
   } else {
-    stream_band<PAIR_MT, PAIR_UNITS, W8, XL, false, false, NWV, 16, X8, X8>(p, M, wg - a.n_items, reinterpret_cast<u16*>(pair_smem));
+    stream_band<PAIR_MT, PAIR_UNITS, W8, XL, false, RESID_NONE, NWV, 16, X8, X8>(p, M, wg - a.n_items, reinterpret_cast<u16*>(pair_smem));
   }
 }
 

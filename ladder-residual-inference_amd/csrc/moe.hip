@@ -157,7 +157,7 @@ __global__ __launch_bounds__(NWV * 64, MT == 16 ? 2 : 0) void k_project_route(co
   }
   const bool second = id >= p0.nwg;
   const Proj p = second ? p1 : p0;
-  stream_band<MT, 2, false, XL, false, false, NWV, 16, MT == 16, MT == 16 && !XL>(p, M, second ? id - p0.nwg : id, sg_smem);
+  stream_band<MT, 2, false, XL, false, RESID_NONE, NWV, 16, MT == 16, MT == 16 && !XL>(p, M, second ? id - p0.nwg : id, sg_smem);
 }
 
 // the shared expert's activations times their gate, four values per thread
@@ -325,7 +325,7 @@ __global__ __launch_bounds__(NWV * 64, 2) void k_expert_band(Proj p, const int64
   p.w += e * wstride;
   for (int i = 0; i < m; i += BAND_ENTRIES) {
     if (i) __syncthreads();
-    stream_band<16, UNITS, false, false, true, false, KW, 16, false>(p, min(BAND_ENTRIES, m - i), blockIdx.x, sg_smem, list + i, xdiv);
+    stream_band<16, UNITS, false, false, true, RESID_NONE, KW, 16, false>(p, min(BAND_ENTRIES, m - i), blockIdx.x, sg_smem, list + i, xdiv);
   }
 }
 

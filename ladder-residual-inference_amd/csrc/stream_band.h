@@ -116,15 +116,22 @@ __device__ __forceinline__ void band_dma16(const void* base, int bytes, int voff
 // 256 bytes, now 256 elements of K, which are expanded to bf16 (exactly: e4m3 is a subset of bf16) on their way
 // into the LDS piece; the sum is rounded to bf16, multiplied by the row's scale and rounded again, as
 // F.linear(x, w.to(bf16)) * scales does, before the epilogue sees it.
-// RESID: nothing is stored to y; the sums, and a token's experts' weighted rows if there are any, are added to the fp32 residual,
-// whose scaled tanh (lr_residual_tanh) goes out as the next layer's input.
+// RESID: nothing is stored to y.  TANH: the sums, and a token's experts' weighted rows if there are any, are added to the fp32 residual,
+// whose scaled tanh (lr_residual_tanh) goes out as the next layer's input.  RMS: they are added to the scaled fp32 residual, which is
+// brought up to date first where it lacks the norm of the sublayer before (lr_linear_residual_rms).
 struct BandResidual {
   float* x;                              // [M, N]
   u16* xc;                               // [M, N]
   const u16 *alpha, *gain, *bias, *eo;   // eo [M * top, N] or nullptr
   const float* ew;                       // [M, top]
   int top;
+  // RMS: x <- scale * x + sums, x divided by its rows' root mean square and times offset + before ahead of that if before != nullptr (the
+  // rows' sums of squares are the projection's norm_sums); xc = x times offset + gain, squares [M][bands] its rows' sums of squares
+  float scale, offset;
+  const u16* before;
+  float* squares;
 };
+enum { RESID_NONE, RESID_TANH, RESID_RMS };
 // KW: waves that share a band's K, all of them or 1: then every wave has a band of its own (`band_` counts groups of NWV).
 // DEEP: the inputs are requested as far ahead as the weights.  Loads come back in the order of their requests, so a wait
 // for inputs that were asked for one chunk ago is a wait for nearly all the weights asked for before them; with both in
@@ -137,13 +144,13 @@ struct BandResidual {
 // 7168 x 8192 22.4 -> 21.9, 8192 x (1024 | 3584) 16.9 -> 16.3; 16 rows (DEEP alone) 4096 x 14336 25.1 -> 23.8; e4m3, 5 rows:
 // 1280 x 8192 7.80 -> 6.32, 8192 x (1024 | 3584) 11.9 -> 10.8, up/gate 14.2 -> 13.6.  The sums keep their order.
 // GATHER: input row m is row rows[m] / xdiv of x, output row m is row rows[m] of y (`rows`: M of them, in LDS).
-template <int MT, int UNITS, bool W8 = false, bool XL = (MT >= XLDS_MIN_MT), bool GATHER = false, bool RESID = false, int KW = NWV,
+template <int MT, int UNITS, bool W8 = false, bool XL = (MT >= XLDS_MIN_MT), bool GATHER = false, int RESID = RESID_NONE, int KW = NWV,
           int UROWS = 16, bool DEEP = true, bool X8 = false, int NW = NWV, bool RN = false>
 __device__ __forceinline__ void stream_band(const Proj& p, const int M, const int band_, u16* sg_smem,
                                             const int32_t* rows = nullptr, const int xdiv = 1, const BandResidual rs = {},
                                             const ResidNorm& rn = {}) {
   static_assert(!W8 || MT == 16, "the e4m3 path is built for up to 16 input rows");
-  const bool has_norm = MT == 16 && KW == NW && !GATHER && !RESID && !RN && p.norm_sums != nullptr;
+  const bool has_norm = MT == 16 && KW == NW && !GATHER && RESID != RESID_TANH && !RN && p.norm_sums != nullptr;
   constexpr int KCW = W8 ? 256 : 128;  // k elements per chunk
   constexpr int LRW = KCW + 8;         // LDS row length in elements
   constexpr int WB = W8 ? 1 : 2;       // bytes per weight
@@ -385,6 +392,25 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
     }
     asm volatile("" ::: "memory");
   }
+  // (RMS) the lane's outputs' residuals and gains
+  constexpr int RMS_ROWS = 16 * UNITS;
+  static_assert(RESID != RESID_RMS || (MT == 16 && KW == NWV && NW == NWV), "UNITS outputs per lane");
+  u32 rms_x[UNITS];
+  u16 rms_before[UNITS], rms_gain[UNITS];
+  if constexpr (RESID == RESID_RMS) {
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(rs.x, 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(rs.before), 0, rs.before ? N * 2 : 0, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(rs.gain), 0, N * 2, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < UNITS; ++i) {
+      const int o = tid + i * NW * 64, r = o % RMS_ROWS, m = o / RMS_ROWS;
+      const bool ok = r < nrows && m < M;
+      rms_x[i] = __builtin_amdgcn_raw_buffer_load_b32(rx, ok ? (m * N + n0 + r) * 4 : OOB, 0, 0);
+      rms_before[i] = __builtin_amdgcn_raw_buffer_load_b16(rb, ok ? (n0 + r) * 2 : OOB, 0, 0);
+      rms_gain[i] = __builtin_amdgcn_raw_buffer_load_b16(rg, ok ? (n0 + r) * 2 : OOB, 0, 0);
+    }
+    asm volatile("" ::: "memory");
+  }
   f32x4_t acc1[UNITS][MTILES];   // (RN) the first pair's sums, once the wave has its last chunk of it
   bool in_first = true;
   issue_x(0, xr[0]);
@@ -586,6 +612,28 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
     LR_BAND_STAMP(5)
     return;
   }
+  if constexpr (RESID == RESID_RMS) {
+#pragma unroll
+    for (int i = 0; i < UNITS; ++i) {
+      const int o = tid + i * NW * 64, r = o % RMS_ROWS, m = o / RMS_ROWS;
+      const int ln = ((r & 15) >> 2) * 16 + m, e = r & 3, u = r >> 4;
+      const bool ok = r < nrows && m < M;
+      float s0 = 0.0f, v = __builtin_bit_cast(float, rms_x[i]);
+#pragma unroll
+      for (int wv = 0; wv < NW; ++wv) s0 += red[wv * WSTRIDE + (u * 4 + e) * 64 + ln];
+      if (rs.before) v = normed(v, m) * (rs.offset + bf_to_f(rms_before[i]));
+      v = ok ? fmaf(rs.scale, v, s0) : 0.0f;
+      float sq = row_sum(v * v);
+      if (UNITS == 2) sq += __shfl_xor(sq, 16, LR_WAVE);
+      if (ok) {
+        rs.x[(int64_t)m * N + n0 + r] = v;
+        rs.xc[(int64_t)m * N + n0 + r] = f_to_bf(v * (rs.offset + bf_to_f(rms_gain[i])));
+        if (r == 0) rs.squares[m * p.nwg + band] = sq;
+      }
+    }
+    LR_BAND_STAMP(5)
+    return;
+  }
   const int rows_out = pair_off ? 16 : 16 * UNITS;
   if (rope_table != nullptr) {
     // The fused q/k/v projection of a decode step (one token per sequence: input row m is sequence m):
@@ -641,7 +689,7 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
     float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll
     for (int wv = 0; wv < KW; ++wv) s0 += red[(KW == 1 ? wave : wv) * WSTRIDE + ((u * MTILES + mt) * 4 + e) * 64 + ln];
-    if constexpr (RESID) {
+    if constexpr (RESID == RESID_TANH) {
       const int n = n0 + r;
       const int64_t at = (int64_t)m * N + n;
       float v = rs.x[at] + s0;

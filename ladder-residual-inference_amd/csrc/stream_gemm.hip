@@ -29,7 +29,7 @@ __global__ __launch_bounds__(NWV * 64, MT == 16 ? 2 : 0) void k_stream_gemm(cons
   extern __shared__ __attribute__((aligned(16))) u16 sg_smem[];
   const bool second = (int)blockIdx.x >= p0.nwg;
   const Proj p = second ? p1 : p0;
-  stream_band<MT, UNITS, W8, XL, false, false, NWV, UROWS, DEEP, X8>(p, M, second ? (int)blockIdx.x - p0.nwg : (int)blockIdx.x, sg_smem);
+  stream_band<MT, UNITS, W8, XL, false, RESID_NONE, NWV, UROWS, DEEP, X8>(p, M, second ? (int)blockIdx.x - p0.nwg : (int)blockIdx.x, sg_smem);
 }
 
 template <int MT, int UNITS, bool W8 = false, bool XL = (MT >= XLDS_MIN_MT), int UROWS = 16, bool X8 = (MT == 16 && !XL && !W8), bool DEEP = (MT == 16)>
@@ -103,7 +103,7 @@ namespace {
 template <int MT, int UNITS, bool XL>
 __global__ __launch_bounds__(NWV * 64, MT == 16 ? 2 : 0) void k_stream_residual(const Proj p, const int M, const BandResidual rs) {
   extern __shared__ __attribute__((aligned(16))) u16 sg_smem[];
-  stream_band<MT, UNITS, false, XL, false, true, NWV, 16, MT == 16, MT == 16 && !XL>(p, M, blockIdx.x, sg_smem, nullptr, 1, rs);
+  stream_band<MT, UNITS, false, XL, false, RESID_TANH, NWV, 16, MT == 16, MT == 16 && !XL>(p, M, blockIdx.x, sg_smem, nullptr, 1, rs);
 }
 
 template <int MT, int UNITS, bool XL>
@@ -147,6 +147,74 @@ extern "C" int lr_linear_residual_tanh(const void* x, int64_t ldx, const void* w
   return M >= XLDS_M16_FROM ? launch_residual<16, true>(pr[0], M, units, rs, s) : launch_residual<16, false>(pr[0], M, units, rs, s);
 }
 
+// ---- a post-norm sublayer's output projection with the residual update and what its norm needs (lr_linear_residual_rms)
+//
+// Such a norm is a launch between a projection into the residual and the next one out of it.  Here the band that owns a column adds
+// to the residual there, and leaves the column with its gain and its share of the rows' sums of squares: the projections that follow
+// divide their results (has_norm), and the next sublayer's residual update divides what it reads.  Up to 16 rows, like those.
+// Bound: HBM, as the bands without; a launch of 5 us less per sublayer, some of it given back by bands that add the parts first.
+// Decode steps, us, before / now: Lasivik 8B 8 rows at 1792 tokens 3693 / 3474, 3 rows 3522 / 3297, 16 rows 4129 / 3985; 1B 3 rows 888 / 819,
+// 8 rows 1001 / 941, 16 rows 1080 / 1043 (in part by the bands' slices of K, see stream_band).
+namespace {
+
+template <int UNITS, bool XL, int UROWS>
+__global__ __launch_bounds__(NWV * 64, 2) void k_stream_rms(const Proj p, const int M, const BandResidual rs) {
+  extern __shared__ __attribute__((aligned(16))) u16 sg_smem[];
+  stream_band<16, UNITS, false, XL, false, RESID_RMS, NWV, UROWS, true, !XL>(p, M, blockIdx.x, sg_smem, nullptr, 1, rs);
+}
+
+template <int UNITS, bool XL, int UROWS = 16>
+int launch_rms(const Proj& p, int M, const BandResidual& rs, hipStream_t s) {
+  const size_t lds = stream_band_lds_bytes<16, UNITS, false, XL>() + stream_band_norm_bytes(p, M);
+  static std::atomic<unsigned long long> raised{0};
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_stream_rms<UNITS, XL, UROWS>), lds, raised)) return LR_E_LAUNCH;
+  k_stream_rms<UNITS, XL, UROWS><<<dim3((unsigned)p.nwg), dim3(NWV * 64), lds, s>>>(p, M, rs);
+  return lr_launch_status();
+}
+
+}  // namespace
+
+extern "C" int lr_linear_residual_rms_sums(int N) {
+  const int ncu = lr_num_cus();
+  if (N <= 0 || ncu < 1) return 0;
+  Proj p{};
+  p.N = N;
+  pick_units_and_plan(&p, 1, 16, ncu);
+  return p.nwg <= LR_ROW_NORM_MAX ? p.nwg : 0;
+}
+
+extern "C" int lr_linear_residual_rms(const void* x, int64_t ldx, const void* w, int M, int N, int K, float* resid, float scale,
+                                      const lr_row_norm_t* before, const void* gain_before, const void* gain, float gain_offset,
+                                      void* x_compute, float* sums, lr_stream_t stream) {
+  LR_REQUIRE_PTR(resid);
+  LR_REQUIRE_PTR(gain);
+  LR_REQUIRE_PTR(x_compute);
+  LR_OPTIONAL_PTR(gain_before);
+  if (sums == nullptr || (before && (before->sums == nullptr || gain_before == nullptr))) return LR_E_NULL;
+  if (before && (before->dim != N || before->fold_sums || before->sums == sums)) return LR_E_SHAPE;   // (the sums are read while others are written)
+  if (M < 1) return LR_E_SHAPE;
+  const lr_projection_t q = {x, ldx, w, x_compute, N, N, K, LR_EPI_NONE, nullptr};
+  Proj p{};
+  int rc = sb_fill_projection(q, p);
+  if (rc != LR_OK) return rc;
+  if (M > LR_ROW_NORM_MAX_ROWS || lr_linear_residual_rms_sums(N) == 0 || (int64_t)M * N * 4 >= 0x7fffffff) return LR_E_UNSUPPORTED;
+  if (before) {
+    lr_row_norm_t of_input = *before;
+    of_input.dim = K;   // (checked against N above: the sums are the residual's)
+    rc = sb_fill_norm(&of_input, p);
+    if (rc != LR_OK) return rc;
+    p.norm_dim = N;
+  }
+  const int units = pick_units_and_plan(&p, 1, M, lr_num_cus());
+  BandResidual rs{};
+  rs.x = resid; rs.xc = (u16*)x_compute; rs.gain = (const u16*)gain; rs.scale = scale; rs.offset = gain_offset;
+  rs.before = before ? (const u16*)gain_before : nullptr; rs.squares = sums;
+  hipStream_t s = (hipStream_t)stream;
+  if (M >= XLDS_M16_FROM) return units == 2 ? launch_rms<2, true>(p, M, rs, s) : launch_rms<1, true>(p, M, rs, s);
+  if (units == 2) return launch_rms<2, false>(p, M, rs, s);
+  return p.rpw <= 8 ? launch_rms<1, false, 8>(p, M, rs, s) : launch_rms<1, false>(p, M, rs, s);
+}
+
 // ---- a layer's output projections with the residual updates and what the next norms need of the rows (lr_linear_resid)
 //
 // A norm between two projections is a launch that moves next to nothing and waits for everything.  Here the workgroup that
@@ -167,7 +235,7 @@ constexpr int RN_WAVES = 8;
 template <int UNITS, bool W8, bool XL, int UROWS, bool X8>
 __global__ __launch_bounds__(RN_WAVES * 64) void k_stream_resid(const Proj p, const int M, const ResidNorm rn) {
   extern __shared__ __attribute__((aligned(16))) u16 sg_smem[];
-  stream_band<16, UNITS, W8, XL, false, false, RN_WAVES, UROWS, !(XL && UNITS == 2), X8, RN_WAVES, true>(p, M, blockIdx.x, sg_smem, nullptr, 1, BandResidual{}, rn);
+  stream_band<16, UNITS, W8, XL, false, RESID_NONE, RN_WAVES, UROWS, !(XL && UNITS == 2), X8, RN_WAVES, true>(p, M, blockIdx.x, sg_smem, nullptr, 1, BandResidual{}, rn);
 }
 
 template <int UNITS, bool W8, bool XL, int UROWS, bool X8>

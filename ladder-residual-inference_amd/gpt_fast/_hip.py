@@ -123,6 +123,9 @@ _PROTOS = {
     "lr_latent_attention": (c_int, [c_void_p, c_void_p]),
     "lr_residual_tanh": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                  c_int, c_int, c_int, c_void_p]),
+    "lr_linear_residual_rms_sums": (c_int, [c_int]),
+    "lr_linear_residual_rms": (c_int, [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_void_p, c_float, c_void_p, c_void_p, c_void_p,
+                                       c_float, c_void_p, c_void_p, c_void_p]),
     "lr_linear_residual_tanh": (c_int, [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_void_p,
                                         c_void_p, c_void_p, c_void_p, c_void_p]),
     "lr_causal_conv": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int,
@@ -978,6 +981,29 @@ def residual_rmsnorm(x, alpha: float, d, gain, x_out, x_compute, eps: float, wid
                                       float(gain_offset), _opt(x_out, torch.float32), _opt(x_compute, gain.dtype), rows, dim,
                                       dim if width is None else width, float(eps), _DTYPES[gain.dtype], _stream()),
            "lr_residual_rmsnorm")
+
+
+def linear_residual_rms_sums(dim: int) -> int:
+    """Values per row that linear_residual_rms leaves of a sum of squares; 0: rows of this width are not served."""
+    return int(load().lr_linear_residual_rms_sums(dim))
+
+
+def linear_residual_rms(y, w, x, alpha: float, before, gain, gain_offset: float, x_compute, sums):
+    """x = alpha * X + y w^T in place (fp32 [M <= 16, dim]), X = x or, with before = (sums, gain, eps), rms_norm(x) * (gain_offset +
+    gain); x_compute and `sums` [M, linear_residual_rms_sums(dim)] together a Normed's (lr_linear_residual_rms).  bf16."""
+    M, K, ldy = _rows_ld(y)
+    N, Kw = w.shape
+    assert w.is_contiguous() and Kw == K and tuple(x.shape) == tuple(x_compute.shape) == (M, N) and x.is_contiguous()
+    assert x_compute.is_contiguous() and gain.numel() == N and gain.is_contiguous()
+    assert sums.shape == (M, linear_residual_rms_sums(N)) and sums.is_contiguous()
+    norm, gain_before = None, None
+    if before is not None:
+        parts, gain_before, eps = before
+        assert parts.shape[0] == M and parts.is_contiguous() and parts.dtype == torch.float32 and gain_before.numel() == N
+        norm = ctypes.byref(_RowNorm(_dev(parts, torch.float32), parts.shape[1], N, eps))
+    _check(load().lr_linear_residual_rms(_dev(y), ldy, _dev(w), M, N, K, _dev(x, torch.float32), float(alpha), norm,
+                                         _opt(gain_before, torch.bfloat16), _dev(gain), float(gain_offset), _dev(x_compute),
+                                         _dev(sums, torch.float32), _stream()), "lr_linear_residual_rms")
 
 
 def logit_cap(logits, scale: float, cap: float):

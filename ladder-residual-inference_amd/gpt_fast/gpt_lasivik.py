@@ -34,6 +34,12 @@ class LasivikWorkspace(HybridWorkspace):
             key = (m.y_cols, m.args.heads * m.args.vdim)
             if key not in self._y:
                 self._y[key] = torch.zeros(rows, m.y_cols, dtype=dtype, device=device)
+        # the parts of the rows' sums of squares behind a mixer and behind a feed-forward, see _run_layers_decode
+        self.sq = None
+        if S == 1 and model.norms_in_projections_from <= B <= _hip.ROW_NORM_MAX_ROWS and dtype == torch.bfloat16 and device.type == "cuda" \
+                and model.config.width == model.config.dim:
+            n = _hip.linear_residual_rms_sums(model.config.dim)
+            self.sq = tuple(e(rows, n, dt=torch.float32) for _ in range(2)) if n else None
 
     def y_of(self, cols: int, used: int) -> Tensor:
         return self._y[(cols, used)]
@@ -68,7 +74,35 @@ class GPTLasivik(GPTHybrid):
         """x <- norm(alpha x + d), in fp32 and in the compute type."""
         _hip.residual_rmsnorm(ws.x, alpha, d, norm.weight, ws.x, ws.xc, norm.eps, self.config.width, gain_offset=1.0)
 
+    # Decode batches from which a norm is part of the projections on either side of it (two rows' wide projections are the
+    # matrix-vector kernel's, see project)
+    norms_in_projections_from = 3
+
+    def _run_layers_decode(self, ws, pos):
+        """Decode step of up to 16 rows: an output projection updates the residual and leaves the rows with the norm's gain and their
+        sums of squares, by which the next projection divides (linear_residual_rms)."""
+        alpha, x, last = self.config.residual_scale, ws.xc, None    # last: (sums, gain, eps), what ws.x still lacks
+
+        def add(y, lin, norm):
+            sq = ws.sq[last is not None and last[0] is ws.sq[0]]    # (one pair of parts is read while the other is written)
+            _hip.linear_residual_rms(y, lin.weight, ws.x, alpha, last, norm.weight, 1.0, ws.xc, sq)
+            return _hip.Normed(ws.xc, sq, norm.eps), (sq, norm.weight, norm.eps)
+
+        for blk in self.layers:
+            m, ff = blk.mixer, blk.feed_forward
+            y = m._y(ws)
+            m.mix(ws, pos, project(x, m.in_proj, ws.proj[:, :m.proj_cols], ws.sums), y)
+            x, last = add(y, m.out_proj, blk.mixer_norm)
+            if ff is not None:
+                act = ws.ffn(ff.w2.in_features)[1]
+                _hip.linear_multi((x, ff.w1.weight, act, _hip.EPI_SWIGLU))
+                x, last = add(act, ff.w2, blk.ffn_norm)
+        _hip.residual_rmsnorm(ws.x, 1.0, None, last[1], ws.x, ws.xc, last[2], self.config.width, gain_offset=1.0)
+        return None, None
+
     def _run_layers(self, ws, pos):
+        if ws.sq is not None:
+            return self._run_layers_decode(ws, pos)
         alpha = self.config.residual_scale
         for blk in self.layers:
             blk.mixer.run(ws, pos)

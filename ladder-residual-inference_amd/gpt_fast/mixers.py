@@ -60,6 +60,9 @@ def project(x: Tensor, lin: nn.Linear, out: Tensor, sums: Optional[Tensor] = Non
     4096 50.3 / 47.4; four: 128256 x 4096 180 / 184, 10240 x 4096 19.1 / 17.1.  6: between the widest of these models' other projections (34816 x
     4096, 2.8 columns' worth per row, the bands') and their heads (from 7.8 on); of widths between and beyond, 24576 to 262144 x 1024 to 4096,
     it is the faster one where the rule takes it (24576 x 1024, three rows 13.2 / 15.4; 262144 x 4096, four rows, 378 / 372, is not)."""
+    if isinstance(x, _hip.Normed):      # (the bands divide)
+        _hip.linear_multi((x, lin.weight, out, _hip.EPI_NONE))
+        return out
     rows, (N, K) = x.shape[0], lin.weight.shape
     few = rows == 2 and N > K or rows <= 4 and N > 6 * rows * K
     if x.dtype == torch.bfloat16 and not few and 2 <= rows <= (64 if sums is None else _hip.BANDS_TO):

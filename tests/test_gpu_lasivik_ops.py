@@ -120,6 +120,33 @@ def test_a_row_of_residual_rmsnorm_does_not_depend_on_the_number_of_rows(hip, dt
         assert torch.equal(xo, outs[0][1][:rows]) and torch.equal(xc, outs[0][2][:rows])
 
 
+@pytest.mark.parametrize("M", [1, 3, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(72, 200), (1032, 136), (2048, 2048), (4096, 1000), (4104, 520), (8200, 264)])
+def test_linear_residual_rms_and_the_projections_of_its_rows(hip, M, N, K):
+    """Two sublayers' residual updates and a projection of each one's undivided rows, each against float64 of what it was given: fp32 sums
+    and residuals, one bf16 step (2^-8 relative, half of it from rounding) per stored row and result."""
+    y, w = [rnd(M, K + 8, seed=i, dtype=BF)[:, :K] for i in range(2)], [(rnd(N, K, seed=2 + i) / K ** 0.5).to(BF) for i in range(2)]
+    gain = [rnd(N, seed=4 + i, dtype=BF) * 0.1 for i in range(2)]
+    n, eps, alpha = hip.linear_residual_rms_sums(N), 1e-5, 2.8
+    assert 0 < n <= 512
+    x, out = rnd(M, N, seed=6), torch.full((M, N), float("nan"), dtype=BF, device=DEV)
+    sums, before = [torch.full((M, n), float("nan"), device=DEV) for _ in range(2)], None
+    up = (rnd(512, N, seed=7) / N ** 0.5).to(BF)
+    for i in range(2):
+        X = d64(x)
+        if before is not None:
+            X = X / (X.square().mean(1, keepdim=True) + eps).sqrt() * (1 + d64(gain[0]))
+        want = alpha * X + d64(y[i]) @ d64(w[i]).T
+        hip.linear_residual_rms(y[i], w[i], x, alpha, before, gain[i], 1.0, out, sums[i])
+        close(x, want, F32)
+        close(out, want * (1 + d64(gain[i])), BF)
+        assert torch.allclose(sums[i].double().sum(1).cpu(), d64(x).square().sum(1).cpu(), rtol=1e-5)
+        got = torch.full((M, 512), float("nan"), dtype=BF, device=DEV)
+        hip.linear_multi((hip.Normed(out, sums[i], eps), up, got, hip.EPI_NONE))
+        close(got, d64(out) / (d64(x).square().mean(1, keepdim=True) + eps).sqrt() @ d64(up).T, BF)
+        before = (sums[i], gain[i], eps)
+
+
 @pytest.mark.parametrize("dtype", [F32, BF])
 def test_logit_cap(hip, dtype):
     l = rnd(5, 104, seed=4, dtype=dtype) * 30
