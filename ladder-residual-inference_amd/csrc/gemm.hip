@@ -673,7 +673,7 @@ struct GemmProduct {
   GemmSplit sp;
 };
 template <int A, int BH, int MODE0, int MODE1, bool NT, int R, bool W8>
-__global__ __launch_bounds__(256, GEMM_PER_CU(A, BH)) void k_gemm_two(const GemmProduct a, const GemmProduct b, const int n0, const GemmRope rp) {
+__global__ __launch_bounds__(256, R > 2 && A > 2 ? 1 : GEMM_PER_CU(A, BH)) void k_gemm_two(const GemmProduct a, const GemmProduct b, const int n0, const GemmRope rp) {
   const bool second = (int)blockIdx.x >= n0;
   if constexpr (MODE0 == MODE1) {
     const GemmProduct p = second ? b : a;
@@ -828,6 +828,10 @@ static bool gemm_takes(int tile, int M, int K) {
   if (tile == GEMM_LONG) return M > 64 && M <= 128 && K % 64 == 0;
   return M > 128 && K % 64 == 0;
 }
+// and the two input projections of a block in one grid (K % 64 == 0): q/k/v beside up/gate of 1B, 128 rows, ring of two 29.5 us, of three 28.2
+// (a prompt of 128 tokens 1041 us -> 1019, of 70 935 -> 913).  Its output projections, cut so that every CU has a workgroup, are 64 x 128 there
+// in 17.0 us and would be 18.0 with the long ring: they keep the first four.
+static bool gemm_shares(int tile, int M, int K) { return (tile < GEMM_TILES_ANY || tile == GEMM_LONG) && gemm_takes(tile, M, K); }
 constexpr size_t GEMM_SCRATCH = (size_t)64 << 20;   // pieces of one round of the largest tiles
 constexpr int GEMM_SCRATCH_FROM = 33;               // rows from which a projection that has memory for pieces is one of this file's
 // and from which the two grids of a decode step are, that hold a product beside the attention or another product: below, the
@@ -979,6 +983,7 @@ static int gemm_two(int tile, const GemmProduct& a, const GemmProduct& b, const 
   if (tile == 0) return gemm_two_as<8, 2, MODE0, MODE1, false>(a, b, rp, s);
   if (tile == 1) return gemm_two_as<4, 2, MODE0, MODE1, false>(a, b, rp, s);
   if (tile == 2) return gemm_two_as<4, 1, MODE0, MODE1, false>(a, b, rp, s);
+  if (tile == GEMM_LONG) return gemm_two_as<4, 1, MODE0, MODE1, false, GEMM_RING>(a, b, rp, s);
   return a.M <= 64 ? gemm_two_as<2, 1, MODE0, MODE1, true, GEMM_RING>(a, b, rp, s) : gemm_two_as<2, 1, MODE0, MODE1, false>(a, b, rp, s);
 }
 
@@ -994,7 +999,8 @@ int gemm_inputs(const void* x0, const void* wqkv, void* qkv, int S, const lr_rop
   const float bytes_us = gemm_bytes_us(M, N, K, GEMM_ROPE) + gemm_bytes_us(M, I, K, GEMM_PAIR);
   float best_us = p0.us + p1.us;
   int best = -1;
-  for (int c = 0; c < GEMM_TILES_ANY; ++c) {
+  for (int c = 0; c < GEMM_NTILES; ++c) {
+    if (!gemm_shares(c, M, K)) continue;
     const GemmTileCost& t = gemm_cost(c, M);
     const int TM = 32 * t.a, slots = cus * t.per_cu;
     const int64_t tm = (M - 1) / TM + 1, tiles0 = tm * ((N - 1) / (128 * t.bh) + 1), tiles1 = tm * ((I - 1) / (64 * t.bh) + 1), tiles = tiles0 + tiles1;

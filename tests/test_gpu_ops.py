@@ -536,7 +536,7 @@ class BlockBuffers:
 @pytest.mark.parametrize("B,S,D,I,Hq,Hkv,hd,layers", [
     (1, 5, 256, 512, 4, 2, 64, 3), (2, 17, 512, 1024, 4, 1, 128, 3), (1, 63, 2048, 8192, 32, 8, 64, 2), (1, 128, 2048, 8192, 32, 8, 64, 3),
     (1, 130, 4096, 14336, 32, 8, 128, 2), (3, 100, 1032, 1096, 4, 2, 64, 3), (2, 256, 2048, 8192, 32, 8, 64, 2), (1, 1100, 1024, 3584, 8, 1, 128, 2),
-    (1, 128, 2048, 8192, 32, 8, 64, 1),
+    (1, 128, 2048, 8192, 32, 8, 64, 1), (1, 65, 2048, 8192, 32, 8, 64, 2), (2, 49, 2048, 8192, 32, 8, 64, 2),
 ])
 def test_ladder_blocks_of_a_prompt(hip, B, S, D, I, Hq, Hkv, hd, layers):
     """Blocks in one call each against the calls they are made of.  Where only the order of fp32 sums differs, a rounded
