@@ -263,22 +263,52 @@ struct WindowKeys {
   float scale;
 };
 
+// Keys come 64 at a time, K and V as they lie, by loads straight into LDS (a row of HD elements is 16-byte pieces; which piece lands
+// where is XOR-ed with the key, see key_swizzle and value_swizzle, so that the fragment reads below meet no bank twice), one portion
+// ahead of the products: one barrier per 64 keys.  V^T fragments are read across the rows (ds_read_b64_tr_b16).
+// KSP 2: a grid that leaves CUs without a second workgroup has eight waves in a workgroup, the second four the second 32 keys of every portion
+// for the same queries; their results are merged at the end.  From 512 queries on, where that pays for the merge (8 heads of 128, one
+// sequence, us: 2048 tokens 51.0 -> 45.5, 777 of 32 heads 23.8 -> 23.1, 256 of 32 heads of 64 8.3 -> 8.6).
+// KEYS 32: 32 at a time and with fewer registers, so that three workgroups share a CU where the grid has as many (8 x 2048 tokens, 32 heads of
+// 128: 399 us, three to a CU 375; two to a CU 408; 328 workgroups 38.6, so 42.9 to 46.2), and for short prompts, which have less to wait for.
+// Bound: matrix instructions 48 % of a SIMD's cycles, vector instructions 46 % (exponentials at a quarter of the rate, splitting P), which hardly
+// run at the same time, in another wave or between the matrix instructions of the same one (written so, it took as long).  No bank
+// conflicts.  Before (32 keys in one LDS buffer through registers, V transposed on its way in, two barriers) / now, us: 32 heads of 128,
+// 8 kv heads: 8 x 2048 tokens 503 / 400 (550 / 690 TFLOP/s of products), 4096 229 / 196, 1300 47.4 / 39.6, 777 29.6 / 23.8, 300 13.9 / 12.9, 100
+// 8.2 / 8.5; of 64: 4 x 4096 497 / 423, 512 15.4 / 12.4, 128 6.8 / 6.4.
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
+constexpr int PREFILL_PARTS_FROM = 512;   // queries, see above
+template <int HD, int KSP, int KEYS>
+struct PrefillLds {
+  static constexpr int TILE = KEYS * HD * 2, STAGE = 2 * TILE;   // a portion's keys or values; both
+  static constexpr int MERGE = KSP == 2 ? 4 * (HD / 2 + 2) * 64 * 4 : 0;
+  static constexpr int KMAX = 2 * STAGE > MERGE ? 2 * STAGE : MERGE, BYTES = KMAX + 32;   // (KMAX: an int of each of up to eight waves)
+};
+// the place among a row's pieces is the piece's number XOR this: 16 lanes reading one piece of 16 consecutive keys, and 16 reading four
+// neighbouring pieces (32 dimensions) of four keys, touch every bank once
+template <int HD>
+__device__ __forceinline__ int key_swizzle(int key) { return HD == 128 ? key & 15 : (key >> 1) & 7; }
+template <int HD>
+__device__ __forceinline__ int value_swizzle(int key) { return HD == 128 ? (key & 3) << 2 : ((key >> 1) & 1) << 2; }
+
 // WIN (lr_window_attention): a sliding window, the score scale as an argument, and the kv heads' keys and values side by
 // side as rows of a matrix, in the order lr_latent_window gives them; head sizes up to HD.
-template <int HD, int NWH, bool WIN = false>
-__global__ __launch_bounds__(256) void k_attn_prefill_mfma(const u16* __restrict__ q, int64_t ldq,
-                                                           const u16* __restrict__ kc, const u16* __restrict__ vc,
-                                                           const int32_t* __restrict__ pos, u16* __restrict__ y,
-                                                           int64_t ldy, int S, int Hq, int Hkv, int Smax,
-                                                           const WindowKeys w = {}) {
+template <int HD, int NWH, int KSP, int KEYS, bool WIN>
+__global__ __launch_bounds__(256 * KSP, KEYS == 32 ? 3 : 2) void k_attn_prefill_mfma(const u16* __restrict__ q, int64_t ldq,
+                                                                    const u16* __restrict__ kc, const u16* __restrict__ vc,
+                                                                    const int32_t* __restrict__ pos, u16* __restrict__ y,
+                                                                    int64_t ldy, int S, int Hq, int Hkv, int Smax,
+                                                                    const WindowKeys w = {}) {
   constexpr int NWQ = 4 / NWH;            // query tiles per workgroup
   constexpr int KS = HD / 16;             // k-steps of the score product
   constexpr int DT = HD / 32;             // 32-row tiles of O^T
-  constexpr int KROW = HD + 8;            // K tile row length in elements (16 B pad: conflict-free 128-bit reads)
-  constexpr int VROW = 32 + 4;            // V^T tile row length in elements (8 B pad)
-  __shared__ __attribute__((aligned(16))) u16 ks[32 * KROW];
-  __shared__ __attribute__((aligned(16))) u16 vt[HD * VROW];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  using L = PrefillLds<HD, KSP, KEYS>;
+  constexpr int NS = KEYS / 32 / KSP;             // 32-key tiles of a portion that a wave takes
+  constexpr int NW = 4 * KSP, RB = HD * 2, PIECES = RB / 16;
+  constexpr int RPL = 1024 / RB, LOADS = KEYS / RPL / NW;   // rows per load instruction, a wave's loads of K or V per portion
+  extern __shared__ __attribute__((aligned(1024))) unsigned char prefill_lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), part = KSP == 2 ? wave >> 2 : 0, w4 = wave & 3;
   const int col = lane & 31, half = lane >> 5;
   const int G = Hq / Hkv;
   const int hgroups = G / NWH;                       // workgroups per kv head along heads
@@ -287,17 +317,24 @@ __global__ __launch_bounds__(256) void k_attn_prefill_mfma(const u16* __restrict
   // that the workgroups that share the K / V rows of one (sequence, kv head) -- the query blocks, neighbours in that
   // order -- meet in one L2.  Inside, the query blocks go from the last (the longest history) to the first.
   const int gx = (S + 32 * NWQ - 1) / (32 * NWQ), gy = Hq / NWH;
-  int wg;
+  int bx, by, b;
   {
-    const int n = gridDim.x, xcd = blockIdx.x % 8, idx = blockIdx.x / 8;
-    const int base = n / 8, rem = n % 8;
-    wg = xcd * base + (xcd < rem ? xcd : rem) + idx;
+    const int n = gridDim.x, xcd = blockIdx.x % 8, idx = blockIdx.x / 8, columns = n / gx;
+    int column;   // a head group of a sequence
+    if (columns % 8 == 0) {
+      column = xcd * (columns / 8) + idx % (columns / 8);   // (all columns' longest first: 8 x 2048 tokens 414 us -> 399)
+      bx = gx - 1 - idx / (columns / 8);
+    } else {
+      const int wg = xcd * (n / 8) + (xcd < n % 8 ? xcd : n % 8) + idx;
+      column = wg / gx;
+      bx = gx - 1 - wg % gx;
+    }
+    by = column % gy;
+    b = column / gy;
   }
-  const int bx = gx - 1 - wg % gx, by = (wg / gx) % gy;
-  const int b = wg / (gx * gy);
   const int kvh = by / hgroups;
-  const int head = kvh * G + (by % hgroups) * NWH + (wave % NWH);
-  const int s = (bx * NWQ + wave / NWH) * 32 + col;  // this lane's query
+  const int head = kvh * G + (by % hgroups) * NWH + (w4 % NWH);
+  const int s = (bx * NWQ + w4 / NWH) * 32 + col;  // this lane's query
   const bool valid = s < S;
   int p = valid ? pos[s] : -1;
   if constexpr (WIN) {
@@ -306,22 +343,22 @@ __global__ __launch_bounds__(256) void k_attn_prefill_mfma(const u16* __restrict
   } else {
     p = p >= Smax ? Smax - 1 : p;
   }
-  // keys needed by anybody in the workgroup
+  // the last key of this wave's queries, and keys needed by anybody in the workgroup
   int kmax = p;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     const int t = __shfl_xor(kmax, o, LR_WAVE);
     kmax = t > kmax ? t : kmax;
   }
-  __shared__ int s_kmax[4];
+  const int pmax = __builtin_amdgcn_readfirstlane(kmax);
+  int* const s_kmax = reinterpret_cast<int*>(prefill_lds + L::KMAX);
   if (lane == 0) s_kmax[wave] = kmax;
   __syncthreads();
   kmax = max(max(s_kmax[0], s_kmax[1]), max(s_kmax[2], s_kmax[3]));
-  const int nkeys = kmax + 1;
-  // (WIN) the last key of this wave's queries, and the first tile anybody in the workgroup sees
-  int pmax = 0, t_first = 0;
+  const int nkeys = __builtin_amdgcn_readfirstlane(kmax + 1);
+  // (WIN) the first portion anybody in the workgroup sees
+  int t_first = 0;
   if constexpr (WIN) {
-    pmax = __builtin_amdgcn_readfirstlane(s_kmax[wave]);
     int lo = 0x7fffffff;
 #pragma unroll
     for (int t = 0; t < NWQ; ++t) {
@@ -329,7 +366,7 @@ __global__ __launch_bounds__(256) void k_attn_prefill_mfma(const u16* __restrict
       if (s_lo < S) lo = min(lo, pos[s_lo] - lr_window_base(pos[0], w.window, w.n_keys, Smax));
     }
     lo = lo - w.window + 1;
-    t_first = lo > 0 ? lo & ~31 : 0;
+    t_first = __builtin_amdgcn_readfirstlane(lo > 0 ? lo & ~31 : 0);
   }
 
   // Q as B operands: k-step ks_ holds elements 16 ks_ + 8 half .. + 8 of this lane's query
@@ -342,6 +379,9 @@ __global__ __launch_bounds__(256) void k_attn_prefill_mfma(const u16* __restrict
       const uint4 t = valid && 16 * i + 8 * half < dq ? ld16(qrow + 16 * i + 8 * half) : make_uint4(0, 0, 0, 0);
       qb[i] = u32x4_t{t.x, t.y, t.z, t.w};
     }
+    // (waited for here: inside the loop the compiler's wait for them would be one for the next portion)
+#pragma unroll
+    for (int i = 0; i < KS; ++i) asm volatile("" : "+v"(qb[i]));
   }
   f32x16_t o[DT];
 #pragma unroll
@@ -363,122 +403,159 @@ __global__ __launch_bounds__(256) void k_attn_prefill_mfma(const u16* __restrict
   const u16* kbase = WIN ? kc + (int64_t)b * w.n_keys * w.ld + kvh * w.dk : kc + ((int64_t)b * Hkv + kvh) * Smax * HD;
   const u16* vbase = WIN ? vc + (int64_t)b * w.n_keys * w.ld + kvh * w.dv : vc + ((int64_t)b * Hkv + kvh) * Smax * HD;
 
-  // Staging: a thread owns one 8-element slice of TWO neighbouring keys (key pair kp, slice dch), so
-  // that V^T can be written as whole dwords (two keys of one dimension).  The pair index is XOR-ed
-  // with 4 * (dch / 4): slices 32 dimensions apart would otherwise fall on the same LDS banks (row
-  // stride 18 dwords, 8 rows per slice).  The next tile's loads are in flight during the products.
-  const int dch = tid % (HD / 8), kp = tid / (HD / 8);
-  const bool stager = kp < 16;
-  const int kps = kp ^ ((dch >> 2) * 4);
-  // (buffer loads: a key beyond the needed range, or a thread without a staging slot, asks with an offset outside
-  // the resource and gets zeros -- no branch around a load)
-  u32x4_t gk[2], gv[2];
-  const __amdgpu_buffer_rsrc_t kres = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(kbase), 0, 0x7fffffff, 0x00020000);
-  const __amdgpu_buffer_rsrc_t vres = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(vbase), 0, 0x7fffffff, 0x00020000);
-  const int stage_off = stager ? (2 * kp * krow + dch * 8) * 2 : (int)0x80000000;  // bytes, first key of the pair
-  const bool k_has = !WIN || dch * 8 < w.dk, v_has = !WIN || dch * 8 < w.dv;
-  auto stage_load = [&](int t0) {
+  // Loads: instruction i of a wave covers rows (i NW + wave) RPL .. of a portion, a lane the piece that belongs to its place.  (A key
+  // beyond the needed ones, or a piece beyond the head's, is asked for outside the resource and comes as zeros.)
+  constexpr int OUT = (int)0x80000000;
+  const int lrow = lane / PIECES, place = lane % PIECES;
+  const int kpiece = place ^ key_swizzle<HD>(wave * RPL + lrow), vpiece = place ^ value_swizzle<HD>(lrow);
+  static_assert(NW * RPL % 16 == 0 && RPL % 4 == 0, "a lane's piece is the same for all of a wave's loads");
+  const int kvoff = !WIN || kpiece * 8 < w.dk ? lrow * krow * 2 + kpiece * 16 : OUT;
+  const int vvoff = !WIN || vpiece * 8 < w.dv ? lrow * krow * 2 + vpiece * 16 : OUT;
+  auto resource = [](const u16* at) {
+    return i32x4_t{(int)(u32)(unsigned long long)at, (int)(u32)((unsigned long long)at >> 32) & 0xffff, 0x7fffffff, 0x00020000};
+  };
+  const i32x4_t kres = resource(kbase), vres = resource(vbase);
+  const u32 lds0 = __builtin_amdgcn_readfirstlane((u32)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)prefill_lds);
+  auto load16 = [](const i32x4_t& res, int voff, int soff, u32 lds) {
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(voff), "s"(res), "s"(soff) : "memory");
+  };
+  auto stage = [&](int t0, int buf) {
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const int off = (stager && t0 + 2 * kp + e < nkeys) ? stage_off + (t0 + e) * krow * 2 : (int)0x80000000;
-      gk[e] = __builtin_amdgcn_raw_buffer_load_b128(kres, k_has ? off : (int)0x80000000, 0, 0);
-      gv[e] = __builtin_amdgcn_raw_buffer_load_b128(vres, v_has ? off : (int)0x80000000, 0, 0);
+    for (int i = 0; i < LOADS; ++i) {
+      const int first = (i * NW + wave) * RPL;
+      const bool ok = t0 + first + lrow < nkeys;
+      const int soff = t0 + first < nkeys ? (t0 + first) * krow * 2 : 0;
+      const u32 at = lds0 + buf * L::STAGE + (i * NW + wave) * 1024;
+      load16(kres, ok ? kvoff : OUT, soff, at);
+      load16(vres, ok ? vvoff : OUT, soff, at + L::TILE);
     }
   };
-  stage_load(t_first);
-  u32* vt32 = reinterpret_cast<u32*>(vt);
-  for (int t0 = t_first; t0 < nkeys; t0 += 32) {
-    __syncthreads();
-    // ---- 32 keys into LDS: K row-major, V transposed ([d][key], two keys per dword)
-    if (stager) {
+  // where this lane reads: the K fragments of key `col` of its tile (k-step i: XOR 32 i), and 4 dimensions of key (lane % 16) / 4
+  // of the four keys whose values 16 lanes exchange (32-row tile d of O^T: see below)
+  const int kat = (part * 32 + col) * RB + ((half ^ key_swizzle<HD>(col)) * 16);
+  const int vkey = (lane & 15) >> 2;
+  int vat[DT];
 #pragma unroll
-      for (int e = 0; e < 2; ++e) *reinterpret_cast<u32x4_t*>(&ks[(2 * kp + e) * KROW + dch * 8]) = gk[e];
-      const u32 a4[4] = {gv[0][0], gv[0][1], gv[0][2], gv[0][3]}, b4[4] = {gv[1][0], gv[1][1], gv[1][2], gv[1][3]};
+  for (int d = 0; d < DT; ++d) {
+    const int piece = 4 * d + ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1);
+    vat[d] = L::TILE + (part * 32 + 4 * half + vkey) * RB + (piece ^ value_swizzle<HD>(vkey)) * 16 + (lane & 1) * 8;
+  }
+  if (t_first < nkeys) stage(t_first, 0);
+  int buf = 0;
+  for (int t0 = t_first; t0 < nkeys; t0 += KEYS, buf ^= 1) {
+    // this portion has arrived, for all waves, and nobody reads the one before any more
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (t0 + KEYS < nkeys) stage(t0 + KEYS, buf ^ 1);
+    const int tk = t0 + part * 32;
+    if (tk > pmax || (WIN && tk + 32 * NS - 1 <= pmin - w.window)) continue;   // nothing here for this wave's queries
+    const unsigned char* const at = prefill_lds + buf * L::STAGE;
+    // ---- S^T tiles: rows = keys, columns = queries
+    f32x16_t sacc[NS];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        vt32[(dch * 8 + 2 * j) * (VROW / 2) + kps] = (a4[j] & 0xffffu) | (b4[j] << 16);
-        vt32[(dch * 8 + 2 * j + 1) * (VROW / 2) + kps] = (a4[j] >> 16) | (b4[j] & 0xffff0000u);
-      }
-    }
-    __syncthreads();
-    stage_load(t0 + 32);
-    if (WIN && (t0 > pmax || t0 + 31 <= pmin - w.window)) continue;   // nothing here for this wave's queries
-    // ---- S^T tile: rows = keys, columns = queries
-    f32x16_t sacc;
+    for (int n = 0; n < NS; ++n)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) sacc[v] = 0.0f;
+      for (int v = 0; v < 16; ++v) sacc[n][v] = 0.0f;
+    u32x4_t ka[KS][NS];   // (all on their way before the first product)
 #pragma unroll
-    for (int i = 0; i < KS; ++i) {
-      const uint4 t = *reinterpret_cast<const uint4*>(&ks[col * KROW + 16 * i + 8 * half]);
-      const u32x4_t ka = {t.x, t.y, t.z, t.w};
-      sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, ka), __builtin_bit_cast(bf16x8_t, qb[i]),
-                                                     sacc, 0, 0, 0);
-    }
-    // element v is key t0 + (v / 4) * 8 + half * 4 + v % 4 for query `col`; only a tile that reaches past the
+    for (int i = 0; i < KS; ++i)
+#pragma unroll
+      for (int n = 0; n < NS; ++n) ka[i][n] = *reinterpret_cast<const u32x4_t*>(at + (kat ^ (32 * i)) + n * 32 * RB);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < KS; ++i)
+#pragma unroll
+      for (int n = 0; n < NS; ++n)
+        sacc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, ka[i][n]), __builtin_bit_cast(bf16x8_t, qb[i]),
+                                                          sacc[n], 0, 0, 0);
+    // element v of tile n is key tk + 32 n + (v / 4) * 8 + half * 4 + v % 4 for query `col`; only a portion that reaches past the
     // smallest position of the wave's queries has anything to mask
-    if (t0 + 31 > pmin || (WIN && t0 <= pmax - w.window)) {
+    if (tk + 32 * NS - 1 > pmin || (WIN && tk <= pmax - w.window)) {
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int key = t0 + (v / 4) * 8 + half * 4 + (v % 4);
-        sacc[v] = key <= p && (!WIN || key > p - w.window) ? sacc[v] : -INFINITY;
-      }
+      for (int n = 0; n < NS; ++n)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int key = tk + 32 * n + (v / 4) * 8 + half * 4 + (v % 4);
+          sacc[n][v] = key <= p && (!WIN || key > p - w.window) ? sacc[n][v] : -INFINITY;
+        }
     }
-    float tmax = max_med3(sacc[0], sacc[1]);
+    float tmax = max_med3(sacc[0][0], sacc[0][1]);
 #pragma unroll
-    for (int v = 2; v < 16; ++v) tmax = max_med3(tmax, sacc[v]);
+    for (int v = 2; v < 16 * NS; ++v) tmax = max_med3(tmax, sacc[v / 16][v % 16]);
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32, LR_WAVE));
-    // The reference point m of the exponentials follows the running maximum lazily: it moves only when a tile's
+    // The reference point m of the exponentials follows the running maximum lazily: it moves only when a portion's
     // maximum exceeds it by more than PREFILL_TAU2 / c2, so the weights stay below 2^PREFILL_TAU2 (harmless in fp32,
-    // and hi + lo keeps their relative precision) and the accumulators are rescaled on few tiles instead of on
-    // most (with 32 queries per wave, some running maximum moves in the majority of tiles).
+    // and hi + lo keeps their relative precision) and the accumulators are rescaled on few portions instead of on
+    // most (with 32 queries per wave, some running maximum moves in the majority of them).
     const bool grow = tmax > m + tau_raw;  // m = -inf: any finite maximum
     const float mn = grow ? tmax : m;
     const float corr = grow ? exp2_hw((m - mn) * c2) : 1.0f;  // m = -inf -> 0
     const float nmc = mn == -INFINITY ? 0.0f : -mn * c2;     // nothing seen yet: every score is -inf, weight 0
     m = mn;
     l *= corr;
-    u32x4_t phi[2], plo[2];
-#pragma unroll
-    for (int h2 = 0; h2 < 2; ++h2)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float a0 = exp2_hw(fmaf(sacc[8 * h2 + 2 * j], c2, nmc));  // masked -> 0
-        const float a1 = exp2_hw(fmaf(sacc[8 * h2 + 2 * j + 1], c2, nmc));
-        l += a0 + a1;
-        const u32 hi = pack_bf2(a0, a1);
-        phi[h2][j] = hi;
-        plo[h2][j] = pack_bf2(a0 - __uint_as_float(hi << 16), a1 - __uint_as_float(hi & 0xffff0000u));
-      }
-    // ---- O^T += V^T P^T ; k-step h2 covers keys 16 h2 + {0..3, 8..11} + 4 half, in the order of sacc
-    const bool rescale = __any(grow);
-    if (rescale) {
+    if (__any(grow)) {
 #pragma unroll
       for (int d = 0; d < DT; ++d)
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[d][v] *= corr;
     }
-    // (consecutive matrix instructions go to different accumulators: one that adds to the result of the instruction
-    // right before it has to wait for that result)
 #pragma unroll
-    for (int h2 = 0; h2 < 2; ++h2) {
-      // keys 16 h2 + 4 half + {0..3} and + 8 + {0..3}; rows of tile d were stored with pairs XOR 4 d
-      u32x4_t va[DT];
+    for (int n = 0; n < NS; ++n) {
+      u32x4_t phi[2], plo[2];
 #pragma unroll
-      for (int d = 0; d < DT; ++d) {
-        const u16* vr = &vt[(d * 32 + col) * VROW];
-        const uint2 v0 = *reinterpret_cast<const uint2*>(vr + ((16 * h2 + 4 * half) ^ (8 * d)));
-        const uint2 v1 = *reinterpret_cast<const uint2*>(vr + ((16 * h2 + 8 + 4 * half) ^ (8 * d)));
-        va[d] = u32x4_t{v0.x, v0.y, v1.x, v1.y};
+      for (int h2 = 0; h2 < 2; ++h2)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float a0 = exp2_hw(fmaf(sacc[n][8 * h2 + 2 * j], c2, nmc));  // masked -> 0
+          const float a1 = exp2_hw(fmaf(sacc[n][8 * h2 + 2 * j + 1], c2, nmc));
+          l += a0 + a1;
+          const u32 hi = pack_bf2(a0, a1);
+          phi[h2][j] = hi;
+          plo[h2][j] = pack_bf2(a0 - __uint_as_float(hi << 16), a1 - __uint_as_float(hi & 0xffff0000u));
+        }
+      // ---- O^T += V^T P^T ; k-step h2 covers keys 16 h2 + {0..3, 8..11} + 4 half of the tile, in the order of sacc
+      // (consecutive matrix instructions go to different accumulators: one that adds to the result of the instruction
+      // right before it has to wait for that result)
+#pragma unroll
+      for (int h2 = 0; h2 < 2; ++h2) {
+        bf16x8_t va[DT];
+#pragma unroll
+        for (int d = 0; d < DT; ++d) {
+          // 16 lanes read 4 keys of 16 dimensions, a lane 4 of one key, and receive the 4 keys of one dimension each
+          const unsigned char* const v0 = at + vat[d] + (n * 32 + 16 * h2) * RB;
+          const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(v0));
+          const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(v0 + 8 * RB));
+          va[d] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[d], __builtin_bit_cast(bf16x8_t, phi[h2]), o[d], 0, 0, 0);
+#pragma unroll
+        for (int d = 0; d < DT; ++d)
+          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[d], __builtin_bit_cast(bf16x8_t, plo[h2]), o[d], 0, 0, 0);
       }
-#pragma unroll
-      for (int d = 0; d < DT; ++d)
-        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, va[d]),
-                                                       __builtin_bit_cast(bf16x8_t, phi[h2]), o[d], 0, 0, 0);
-#pragma unroll
-      for (int d = 0; d < DT; ++d)
-        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, va[d]),
-                                                       __builtin_bit_cast(bf16x8_t, plo[h2]), o[d], 0, 0, 0);
     }
+  }
+  if constexpr (KSP == 2) {
+    // the second four waves' results to the first four, which saw the other keys of the same queries
+    __syncthreads();
+    float* const mine = reinterpret_cast<float*>(prefill_lds) + w4 * (HD / 2 + 2) * 64 + lane;
+    if (part) {
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) mine[(d * 16 + v) * 64] = o[d][v];
+      mine[(HD / 2) * 64] = m;
+      mine[(HD / 2 + 1) * 64] = l;
+    }
+    __syncthreads();
+    if (part) return;
+    const float m1 = mine[(HD / 2) * 64], mn = fmaxf(m, m1);
+    const float f0 = m == -INFINITY ? 0.0f : exp2_hw((m - mn) * c2), f1 = m1 == -INFINITY ? 0.0f : exp2_hw((m1 - mn) * c2);
+    l = l * f0 + mine[(HD / 2 + 1) * 64] * f1;
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) o[d][v] = fmaf(mine[(d * 16 + v) * 64], f1, o[d][v] * f0);
   }
   l += __shfl_xor(l, 32, LR_WAVE);
   if (valid) {
@@ -498,21 +575,33 @@ __global__ __launch_bounds__(256) void k_attn_prefill_mfma(const u16* __restrict
   }
 }
 
-template <int HD>
-static int launch_prefill_mfma(const u16* q, int64_t ldq, const u16* kc, const u16* vc, const int32_t* pos, u16* y,
-                               int64_t ldy, int B, int S, int Hq, int Hkv, int Smax, hipStream_t s) {
-  const int G = Hq / Hkv;
-  if (G % 4 == 0) {
-    k_attn_prefill_mfma<HD, 4><<<dim3((unsigned)((int64_t)((S + 31) / 32) * (Hq / 4) * B)), dim3(256), 0, s>>>(
-        q, ldq, kc, vc, pos, y, ldy, S, Hq, Hkv, Smax);
-  } else if (G % 2 == 0) {
-    k_attn_prefill_mfma<HD, 2><<<dim3((unsigned)((int64_t)((S + 63) / 64) * (Hq / 2) * B)), dim3(256), 0, s>>>(
-        q, ldq, kc, vc, pos, y, ldy, S, Hq, Hkv, Smax);
-  } else {
-    k_attn_prefill_mfma<HD, 1><<<dim3((unsigned)((int64_t)((S + 127) / 128) * Hq * B)), dim3(256), 0, s>>>(
-        q, ldq, kc, vc, pos, y, ldy, S, Hq, Hkv, Smax);
-  }
+template <int HD, int NWH, int KSP, int KEYS, bool WIN>
+static int launch_prefill_as(unsigned workgroups, const u16* q, int64_t ldq, const u16* kc, const u16* vc, const int32_t* pos, u16* y, int64_t ldy,
+                             int S, int Hq, int Hkv, int Smax, const WindowKeys& w, hipStream_t s) {
+  constexpr size_t lds = PrefillLds<HD, KSP, KEYS>::BYTES;
+  static std::atomic<unsigned long long> raised{0};
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_attn_prefill_mfma<HD, NWH, KSP, KEYS, WIN>), lds, raised)) return LR_E_LAUNCH;
+  k_attn_prefill_mfma<HD, NWH, KSP, KEYS, WIN><<<dim3(workgroups), dim3(256 * KSP), lds, s>>>(q, ldq, kc, vc, pos, y, ldy, S, Hq, Hkv, Smax, w);
   return lr_launch_status();
+}
+template <int HD, int NWH, bool WIN>
+static int launch_prefill_heads(const u16* q, int64_t ldq, const u16* kc, const u16* vc, const int32_t* pos, u16* y, int64_t ldy, int B, int S,
+                                int Hq, int Hkv, int Smax, const WindowKeys& w, hipStream_t s) {
+  constexpr int queries = 32 * (4 / NWH);
+  const int64_t n = (int64_t)((S + queries - 1) / queries) * (Hq / NWH) * B;
+  const int cus = lr_num_cus();
+  auto run = n <= cus && S >= PREFILL_PARTS_FROM ? &launch_prefill_as<HD, NWH, 2, 64, WIN>
+             : HD == 128 && (n > 2 * cus || S <= 128) ? &launch_prefill_as<HD, NWH, 1, 32, WIN> : &launch_prefill_as<HD, NWH, 1, 64, WIN>;
+  return run((unsigned)n, q, ldq, kc, vc, pos, y, ldy, S, Hq, Hkv, Smax, w, s);
+}
+// NWH heads of a kv head in a workgroup: as many of four as divide its share
+template <int HD, bool WIN>
+static int launch_prefill_mfma(const u16* q, int64_t ldq, const u16* kc, const u16* vc, const int32_t* pos, u16* y, int64_t ldy, int B, int S,
+                               int Hq, int Hkv, int Smax, const WindowKeys& w, hipStream_t s) {
+  const int G = Hq / Hkv;
+  if (G % 4 == 0) return launch_prefill_heads<HD, 4, WIN>(q, ldq, kc, vc, pos, y, ldy, B, S, Hq, Hkv, Smax, w, s);
+  if (G % 2 == 0) return launch_prefill_heads<HD, 2, WIN>(q, ldq, kc, vc, pos, y, ldy, B, S, Hq, Hkv, Smax, w, s);
+  return launch_prefill_heads<HD, 1, WIN>(q, ldq, kc, vc, pos, y, ldy, B, S, Hq, Hkv, Smax, w, s);
 }
 
 extern "C" int lr_attn_prefill(const void* q, int64_t ldq, const void* k_cache, const void* v_cache,
@@ -534,11 +623,11 @@ extern "C" int lr_attn_prefill(const void* q, int64_t ldq, const void* k_cache, 
     // (and its grid is one-dimensional, at most (S / 32) * Hq * B workgroups of 256 lanes: 2^32 lanes is the limit)
     if ((hd == 128 || hd == 64) && (int64_t)((S + 31) / 32) * Hq * B >= (1 << 24)) return LR_E_UNSUPPORTED;
     if (hd == 128)
-      return launch_prefill_mfma<128>((const u16*)q, ldq, (const u16*)k_cache, (const u16*)v_cache, pos, (u16*)y, ldy,
-                                      B, S, Hq, Hkv, Smax, s);
+      return launch_prefill_mfma<128, false>((const u16*)q, ldq, (const u16*)k_cache, (const u16*)v_cache, pos, (u16*)y, ldy,
+                                             B, S, Hq, Hkv, Smax, {}, s);
     if (hd == 64)
-      return launch_prefill_mfma<64>((const u16*)q, ldq, (const u16*)k_cache, (const u16*)v_cache, pos, (u16*)y, ldy, B,
-                                     S, Hq, Hkv, Smax, s);
+      return launch_prefill_mfma<64, false>((const u16*)q, ldq, (const u16*)k_cache, (const u16*)v_cache, pos, (u16*)y, ldy, B,
+                                            S, Hq, Hkv, Smax, {}, s);
   }
   if (hd == 128)
     k_attn_prefill<128><<<grid, dim3(64), 0, s>>>((const u16*)q, ldq, (const u16*)k_cache, (const u16*)v_cache, pos,
@@ -561,20 +650,9 @@ int window_attention_mfma(const lr_window_attention_t* d, lr_stream_t stream) {
   if ((int64_t)(d->n_keys + 64) * d->ldk * 2 >= 0x7fffffff || (int64_t)((d->S + 31) / 32) * d->H * d->B >= (1 << 24))
     return LR_E_UNSUPPORTED;
   const WindowKeys w = {d->window, d->n_keys, (int)d->ldk, d->dk, d->dv, d->scale};
-  const int G = d->kv_heads > 0 ? d->kv_heads : d->H, share = d->H / G;
-  hipStream_t s = (hipStream_t)stream;
-#define LR_WIN(HD, NWH)                                                                                                \
-  k_attn_prefill_mfma<HD, NWH, true>                                                                                   \
-      <<<dim3((unsigned)((int64_t)((d->S + 32 * (4 / NWH) - 1) / (32 * (4 / NWH))) * (d->H / NWH) * d->B)), dim3(256), 0, s>>>( \
-          (const u16*)d->q, d->ldq, (const u16*)d->k, (const u16*)d->v, d->pos, (u16*)d->y, d->ldy, d->S, d->H, G, d->Smax, w)
-#define LR_WIN_HD(HD)                    \
-  if (share % 4 == 0) LR_WIN(HD, 4);     \
-  else if (share % 2 == 0) LR_WIN(HD, 2); \
-  else LR_WIN(HD, 1)
-  if (hd <= 64) { LR_WIN_HD(64); }
-  else { LR_WIN_HD(128); }
-#undef LR_WIN_HD
-#undef LR_WIN
-  return lr_launch_status();
+  const int G = d->kv_heads > 0 ? d->kv_heads : d->H;
+  auto run = hd <= 64 ? &launch_prefill_mfma<64, true> : &launch_prefill_mfma<128, true>;
+  return run((const u16*)d->q, d->ldq, (const u16*)d->k, (const u16*)d->v, d->pos, (u16*)d->y, d->ldy, d->B, d->S, d->H, G, d->Smax, w,
+             (hipStream_t)stream);
 }
 }  // namespace lr_detail

@@ -1187,6 +1187,25 @@ def test_attn_prefill(hip, B, S, Hq, Hkv, hd, Smax, start):
     assert_close_ulp(y, want, max_frac=0.03, what="attn_prefill")
 
 
+# (portions of 32 and of 64 keys, with and without a last half, and each wave half of them; workgroups of one, two and four heads, in
+# columns that are a multiple of eight and that are not)
+@pytest.mark.parametrize("B,S,Hq,Hkv,hd,start", [
+    (1, 16, 4, 1, 128, 0), (2, 33, 8, 2, 128, 31), (1, 128, 6, 3, 128, 64), (1, 129, 32, 8, 128, 0), (3, 161, 2, 2, 128, 95), (1, 511, 8, 2, 128, 1),
+    (1, 512, 8, 1, 128, 0), (1, 545, 6, 3, 128, 63), (2, 600, 2, 2, 128, 200), (8, 520, 32, 8, 128, 0), (5, 610, 28, 7, 128, 17),
+    (1, 17, 4, 1, 64, 0), (1, 130, 6, 3, 64, 33), (1, 512, 32, 8, 64, 0), (1, 577, 2, 2, 64, 64), (8, 530, 32, 8, 64, 3)])
+def test_attn_prefill_portions_of_keys(hip, B, S, Hq, Hkv, hd, start):
+    """Nothing beyond the last position is used, whatever lies there."""
+    n = start + S
+    q, kc, vc = rnd(B, S, Hq * hd, seed=31), rnd(B, Hkv, n + 70, hd, seed=32), rnd(B, Hkv, n + 70, hd, seed=33)
+    kc[:, :, n:], vc[:, :, n:] = float("nan"), float("nan")
+    pos = torch.arange(start, n, dtype=torch.int32, device=DEV)
+    y = torch.full((B, S, Hq * hd), float("nan"), dtype=BF, device=DEV)
+    hip.attn_prefill(q, kc, vc, pos, y, B, S, Hq, Hkv, hd)
+    mask = torch.arange(n, device=DEV).view(1, n) <= pos.view(S, 1)
+    want = O.sdpa_math(q.view(B, S, Hq, hd).transpose(1, 2), kc[:, :, :n].contiguous(), vc[:, :, :n].contiguous(), mask)
+    assert_close_ulp(y, want.transpose(1, 2).reshape(B, S, Hq * hd), max_frac=0.03, what="attn_prefill, portions")
+
+
 @pytest.mark.parametrize("qscale", [4.0, 12.0])
 def test_attn_prefill_large_scores(hip, qscale):
     """Scores with a standard deviation of 4 and 12: the running maximum of a query jumps by more than the kernel lets
