@@ -396,10 +396,11 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
   int mt, nt, piece = -1, kt0 = 0, nk = (K + KT - 1) / KT;
   int32_t* const entry = reinterpret_cast<int32_t*>(gsm + T::LDS / 2);   // (GROUP) the tile's entries
   if constexpr (GROUP) {
-    const int id = xcd_run(block, blocks);   // a row tile's column tiles one after the other
+    const int tiles = gp.ntiles[0] * tn;   // (of the grid's: there may be fewer, and each XCD has its share of those there are)
+    if (block >= tiles) return;
+    const int id = xcd_run(block, tiles);   // a row tile's column tiles one after the other
     mt = id / tn;
     nt = id - mt * tn;
-    if (mt >= gp.ntiles[0]) return;
     const int32_t* tile = gp.tiles + 3 * mt;
     w += tile[0] * gp.wstride;
     M = tile[2];
@@ -1143,8 +1144,37 @@ static int gemm_outputs8(const void* x0, const void* w0, const void* scales0, in
 }  // namespace lr_detail
 
 // Grouped products (lr_moe): rows of several matrices' tiles, see GemmGroup; pair_off != 0: GEMM_PAIR (N counts pairs).
-// tile_rows: 128 or 256, the height the tile table was made for.
+// tile_rows: the height the tile table was made for (grouped_rows): 128 or 160 (K % 64 == 0) with 128 columns, the latter's pairs with
+// 256 where that leaves no half of a tile without columns, or 256 x 256.
+static int grouped_pairs_bh(int tile_rows, int I) { return tile_rows == 128 || (tile_rows == 160 && (I + 63) / 64 % 2) ? 1 : 2; }
+// what one of the two takes whose row tiles are `tiles` of `rows` rows of an expert
+static float grouped_us(int a, int bh, float tiles, int rows, int N, int K, int mode) {
+  const GemmTileCost* t = nullptr;
+  for (const GemmTileCost& c : GEMM_TILES)
+    if (t == nullptr && c.a == a && c.bh == bh) t = &c;
+  const int cus = gemm_cus(), gn = (mode == GEMM_PAIR ? 64 : 128) * bh, nk = (K + 63) / 64;
+  const float workgroups = tiles * ((N + gn - 1) / gn), slots = (float)cus * t->per_cu, rounds = floorf(workgroups / slots), left = workgroups - rounds * slots;
+  float us = rounds * (gemm_round_us(*t, rows, cus, (int)slots, nk) + t->fixed);
+  if (left > 0.0f) us += gemm_round_us(*t, rows, cus, (int)left, nk) + t->fixed;
+  return us + t->store * (mode == GEMM_PAIR ? 0.5f : 1.0f) * workgroups / cus;
+}
 namespace lr_detail {
+// Height of the tiles for n rows of `experts` that are taken: what the costs of GEMM_TILES give both products, an expert ending in half a
+// tile on average.  The factors are fitted to 47 mixtures of 8 to 64 experts, 500 to 16384 tokens, even and skewed choices, where the
+// height taken is then 1.1 % above the best (13 % at worst; without them 2.2 and 17 %; 256 wherever an expert has as many rows and 128
+// below, as it was, 6.7 and 29 %).  us of the whole mixture, before / now (the empty tiles' place included, see gemm_tile): 32 experts,
+// 6 chosen, 384 x 4096: 500 tokens 145 / 111, 2500 309 / 198, 3002 316 / 258, 6000 512 / 421, 8192 582 / 582; 16 experts, 4 chosen, 448 x 2048:
+// 1000 63 / 53, 5000 181 / 141, 16384 477 / 438.
+int grouped_rows(int64_t n, int experts, int I, int D) {
+  const float rows = (float)n / experts;
+  auto us = [&](int h) {
+    const float tiles = (float)n / h + 0.5f * experts;
+    const int r = rows < 1.0f ? 1 : (int)rows, a = h / 32;
+    return grouped_us(a, grouped_pairs_bh(h, I), tiles, r, I, D, GEMM_PAIR) + grouped_us(a, h == 256 ? 2 : 1, tiles, r, D, I, GEMM_PLAIN);
+  };
+  const float u128 = 1.1f * us(128), u160 = I % 64 || D % 64 ? 1e30f : 0.95f * us(160), u256 = us(256);
+  return u160 < u128 && u160 < u256 ? 160 : u128 < u256 ? 128 : 256;
+}
 template <int A, int BH, bool KTAIL, int MODE>
 static int gemm_grouped_as(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int N, int K, const GemmGroup& gp, int max_tiles,
                            hipStream_t s) {
@@ -1162,6 +1192,12 @@ int gemm_grouped(const void* x, int64_t ldx, int64_t xrows, const void* w, void*
   if (xrows * ldx * 2 >= 0x7fffffff || ((int64_t)pair_off + 256) * K * 2 >= 0x7fffffff) return LR_E_UNSUPPORTED;
   const GemmGroup gp = {tiles, ntiles, entries, xdiv, wstride, xrows};
   const bool kt = K % 64 != 0;
+  if (tile_rows == 160) {
+    if (kt) return LR_E_UNSUPPORTED;
+    if (!pair_off) return gemm_grouped_as<5, 1, false, GEMM_PLAIN>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
+    return grouped_pairs_bh(tile_rows, N) == 1 ? gemm_grouped_as<5, 1, false, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)
+                                               : gemm_grouped_as<5, 2, false, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s);
+  }
   if (tile_rows == 128) {
     if (pair_off)
       return kt ? gemm_grouped_as<4, 1, true, GEMM_PAIR>(x, ldx, w, y, ldy, N, K, gp, max_tiles, s)

@@ -21,6 +21,7 @@ int gemm_grouped(const void* x, int64_t ldx, int64_t xrows, const void* w, void*
 int linear_f32_grouped(const float* x, int64_t ldx, const float* w, float* y, int64_t ldy, int N, int K, const int32_t* tiles,
                        const int32_t* ntiles, const int32_t* entries, int xdiv, int max_tiles, hipStream_t s);                   // residual.hip
 int linear_f32_grouped_rows();
+int grouped_rows(int64_t n, int experts, int I, int D);
 }  // namespace lr_detail
 
 namespace {
@@ -343,11 +344,11 @@ int launch_band(const Proj& p, int64_t wstride, const int32_t* experts, int n, i
 constexpr int BAND_ROWS = 64, BAND_LIST = 4096;      // tokens and entries up to which the bands are taken
 bool by_bands(int rows, int top, int dtype) { return dtype == LR_BF16 && rows <= BAND_ROWS && (int64_t)rows * top <= BAND_LIST; }
 
-// Height of the grouped tiles: 256 rows where experts fill them and there are tiles for most CUs.
+// Height of the grouped tiles
 int tile_rows(int rows, int E, int top, int I, int D, int dtype) {
   if (dtype == LR_F32) return lr_detail::linear_f32_grouped_rows();
-  const int64_t n = (int64_t)rows * top, e = n < E ? n : E, tall = n / 256 + e / 2;
-  return n >= 256 * e && tall * ((I + 127) / 128) >= 160 && tall * ((D + 255) / 256) >= 160 ? 256 : 128;
+  const int64_t n = (int64_t)rows * top;
+  return lr_detail::grouped_rows(n, n < E ? (int)n : E, I, D);
 }
 int max_tiles(int rows, int E, int top, int height) {
   const int64_t n = (int64_t)rows * top, e = n < E ? n : E;

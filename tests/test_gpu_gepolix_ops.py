@@ -407,6 +407,19 @@ def test_mixture_of_many_tokens(hip):
             m.check(x, act, before)
 
 
+# (tiles of 160 rows, pairs in 256 columns and, an odd number of 64s, in 128; of 256; of 128: see grouped_rows of gemm.hip)
+@pytest.mark.parametrize("rows,D,I,E,top", [(3002, 1024, 384, 32, 6), (1500, 1024, 192, 8, 4), (1100, 512, 448, 16, 4), (2500, 4096, 384, 32, 6),
+                                            (2000, 2056, 520, 8, 4), (3002, 512, 384, 32, 6)])
+@pytest.mark.parametrize("spread", [0.0, 6.0])
+def test_mixture_in_grouped_tiles(hip, rows, D, I, E, top, spread):
+    """Choices spread evenly, and unevenly enough for experts without a token: fewer tiles than the grid holds."""
+    m = Mix(D, I, E, top, 0, BF, seed=rows)
+    m.bias += torch.linspace(-spread, spread, E, device=DEV).to(BF)
+    x = rnd(rows, D, seed=3, dtype=BF)
+    hip.moe(m.desc(hip, x))
+    m.check(x)
+
+
 @pytest.mark.parametrize("rows", [3, 70])
 def test_every_token_chooses_the_same_experts_and_equals_go_to_the_lower(hip, rows):
     m = Mix(64, 32, 9, 3, 0, BF)
