@@ -79,6 +79,9 @@ int lr_add(const void* a, const void* b, float b_div, void* out, int64_t n, lr_s
  * (utils.py:68-74).  d1, d2, resid_out may be NULL; resid_out may alias resid_in.  dim <= 16384. */
 int lr_add_rmsnorm(const void* resid_in, const void* d1, const void* d2, const void* gain, void* resid_out,
                    void* normed_out, int rows, int dim, float eps, lr_stream_t stream);
+/* pieces1 > 0: d1 is the partial sums [pieces1][rows][dim] fp32 that lr_linear_pieces left; what a product with its sum would have given. */
+int lr_add_rmsnorm_pieces(const void* resid_in, const void* d1, int pieces1, const void* d2, const void* gain, void* resid_out,
+                          void* normed_out, int rows, int dim, float eps, lr_stream_t stream);
 
 /* Both residual updates and both RMSNorms of one ladder block in one launch:
  *     r1 = bf16(resid_in + d1),  normed1 = norm(r1) * gain1      (gpt_ladder_TP.py:326-337)

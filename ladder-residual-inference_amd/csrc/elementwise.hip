@@ -80,8 +80,32 @@ __device__ __forceinline__ float norm_sum(const float* red) {
 // loses at 2048 (2.34 -> 2.48): those rows keep the order of their sums.
 static int norm_lanes(int dim) { return dim <= 4096 ? 256 : 1024; }
 
-template <int T>
-__global__ __launch_bounds__(T) void k_add_rmsnorm(const u16* __restrict__ rin, const u16* __restrict__ d1,
+// Eight columns of a product's partial sums [pieces][rows][dim] (`step` elements apart), added in the order in which k_gemm_sum adds
+// them and rounded as its output is
+__device__ __forceinline__ uint4 sum_pieces8(const float* __restrict__ p, int pieces, int64_t step) {
+  f32x4_t lo = *reinterpret_cast<const f32x4_t*>(p), hi = *reinterpret_cast<const f32x4_t*>(p + 4);
+  for (int s = 1; s < pieces; s += 4) {
+    f32x4_t l[4], h[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float* const q = p + (s + i < pieces ? s + i : 0) * step;
+      l[i] = *reinterpret_cast<const f32x4_t*>(q);
+      h[i] = *reinterpret_cast<const f32x4_t*>(q + 4);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (s + i < pieces) {
+        lo += l[i];
+        hi += h[i];
+      }
+  }
+  return make_uint4(pack_bf2(lo[0], lo[1]), pack_bf2(lo[2], lo[3]), pack_bf2(hi[0], hi[1]), pack_bf2(hi[2], hi[3]));
+}
+// PIECES: d1 is such partial sums.  A product's sum then costs neither a launch nor its rounded rows' trip through memory.  us, dense 8B blocks,
+// two sums of 5 to 9 us per block in launches of their own / here: 48 sequences at 300 tokens 4417 / 4246, prompts of 90 tokens 4707 / 4513, of
+// 777, where w2's alone is in pieces, 12105 / 11915 (190 of it the attention's); desync 40 sequences at 1000 4927 / 4691.
+template <int T, bool PIECES>
+__global__ __launch_bounds__(T) void k_add_rmsnorm(const u16* __restrict__ rin, const void* __restrict__ d1, int pieces1,
                                                      const u16* __restrict__ d2, const u16* __restrict__ gain,
                                                      u16* rout, u16* __restrict__ nout, int dim, float eps) {
   __shared__ float red[T / 64];
@@ -98,7 +122,8 @@ __global__ __launch_bounds__(T) void k_add_rmsnorm(const u16* __restrict__ rin, 
     if (it * T * 8 >= dim) break;  // uniform
     const int c = c0 < dim ? c0 : 0;
     qr[it] = ld16(rin + base + c);
-    q1[it] = d1 ? ld16(d1 + base + c) : make_uint4(0, 0, 0, 0);
+    if (PIECES) q1[it] = sum_pieces8(static_cast<const float*>(d1) + base + c, pieces1, (int64_t)gridDim.x * dim);
+    else q1[it] = d1 ? ld16(static_cast<const u16*>(d1) + base + c) : make_uint4(0, 0, 0, 0);
     q2[it] = d2 ? ld16(d2 + base + c) : make_uint4(0, 0, 0, 0);
     qg[it] = ld16(gain + c);
   }
@@ -160,22 +185,32 @@ __global__ __launch_bounds__(T) void k_add_rmsnorm(const u16* __restrict__ rin, 
 
 extern "C" int lr_add_rmsnorm(const void* resid_in, const void* d1, const void* d2, const void* gain, void* resid_out,
                               void* normed_out, int rows, int dim, float eps, lr_stream_t stream) {
+  return lr_add_rmsnorm_pieces(resid_in, d1, 0, d2, gain, resid_out, normed_out, rows, dim, eps, stream);
+}
+
+extern "C" int lr_add_rmsnorm_pieces(const void* resid_in, const void* d1, int pieces1, const void* d2, const void* gain, void* resid_out,
+                                     void* normed_out, int rows, int dim, float eps, lr_stream_t stream) {
   LR_REQUIRE_PTR(resid_in);
   LR_REQUIRE_PTR(gain);
   LR_REQUIRE_PTR(normed_out);
   LR_OPTIONAL_PTR(d1);
   LR_OPTIONAL_PTR(d2);
   LR_OPTIONAL_PTR(resid_out);
-  if (rows <= 0 || dim <= 0) return LR_E_SHAPE;
+  if (rows <= 0 || dim <= 0 || pieces1 < 0) return LR_E_SHAPE;
+  if (pieces1 && d1 == nullptr) return LR_E_NULL;
   if (dim % 8) return LR_E_ALIGN;
   if (dim > NORM_MAX_DIM) return LR_E_UNSUPPORTED;
-  auto launch = [&](auto T) {
+  auto launch = [&](auto T, auto P) {
     constexpr int lanes = decltype(T)::value;
-    k_add_rmsnorm<lanes><<<dim3(rows), dim3(lanes), 0, (hipStream_t)stream>>>(
-        (const u16*)resid_in, (const u16*)d1, (const u16*)d2, (const u16*)gain, (u16*)resid_out, (u16*)normed_out, dim, eps);
+    k_add_rmsnorm<lanes, decltype(P)::value><<<dim3(rows), dim3(lanes), 0, (hipStream_t)stream>>>(
+        (const u16*)resid_in, d1, pieces1, (const u16*)d2, (const u16*)gain, (u16*)resid_out, (u16*)normed_out, dim, eps);
   };
-  if (norm_lanes(dim) == 1024) launch(std::integral_constant<int, 1024>{});
-  else launch(std::integral_constant<int, 256>{});
+  auto pick = [&](auto T) {
+    if (pieces1) launch(T, std::true_type{});
+    else launch(T, std::false_type{});
+  };
+  if (norm_lanes(dim) == 1024) pick(std::integral_constant<int, 1024>{});
+  else pick(std::integral_constant<int, 256>{});
   return lr_launch_status();
 }
 
@@ -184,29 +219,8 @@ extern "C" int lr_add_rmsnorm(const void* resid_in, const void* d1, const void* 
 // In the ladder schedule the MLP's input does not contain the attention output of the same block, so
 // both residual updates and both norms of a block can be done before either module runs.
 //
-// PIECES: d1 (d2), where pieces1 (pieces2) is not 0, is the partial sums [pieces][rows][dim] that a product left
-// (lr_linear_pieces): added here in the order in which k_gemm_sum adds them and rounded as its output is, so the bits are the
-// same; a product's sum then costs neither a launch nor its rounded rows' trip through memory.  128 rows of 2048, eight and
-// four pieces: 5.2 us for the launch, 5.0 + 5.0 + 3.8 for the three.
-__device__ __forceinline__ uint4 sum_pieces8(const float* __restrict__ p, int pieces, int64_t step) {
-  f32x4_t lo = *reinterpret_cast<const f32x4_t*>(p), hi = *reinterpret_cast<const f32x4_t*>(p + 4);
-  for (int s = 1; s < pieces; s += 4) {
-    f32x4_t l[4], h[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float* const q = p + (s + i < pieces ? s + i : 0) * step;
-      l[i] = *reinterpret_cast<const f32x4_t*>(q);
-      h[i] = *reinterpret_cast<const f32x4_t*>(q + 4);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (s + i < pieces) {
-        lo += l[i];
-        hi += h[i];
-      }
-  }
-  return make_uint4(pack_bf2(lo[0], lo[1]), pack_bf2(lo[2], lo[3]), pack_bf2(hi[0], hi[1]), pack_bf2(hi[2], hi[3]));
-}
+// PIECES: d1 (d2), where pieces1 (pieces2) is not 0, is the partial sums that a product left (lr_linear_pieces), see sum_pieces8.
+// 128 rows of 2048, eight and four pieces: 5.2 us for the launch, 5.0 + 5.0 + 3.8 for the three.
 template <int T, bool PIECES>
 __global__ __launch_bounds__(T) void k_ladder_norms(const u16* __restrict__ rin, const void* __restrict__ d1,
                                                       const void* __restrict__ d2, int pieces1, int pieces2,

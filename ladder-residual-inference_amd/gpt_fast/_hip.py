@@ -18,6 +18,7 @@ _PROTOS = {
     "lr_error_string": (c_char_p, [c_int]),
     "lr_embed": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_int64, c_int, c_int, c_void_p]),
     "lr_add": (c_int, [c_void_p, c_void_p, c_float, c_void_p, c_int64, c_void_p]),
+    "lr_add_rmsnorm_pieces": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float, c_void_p]),
     "lr_add_rmsnorm": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_float,
                                c_void_p]),
     "lr_ladder_norms_pieces": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
@@ -245,19 +246,25 @@ def add(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor, b_div: float = 1.0)
 
 
 def add_rmsnorm(resid_in, d1, d2, gain, resid_out, normed_out, eps: float):
+    """d1 may be Pieces."""
     dim = resid_in.shape[-1]
     rows = resid_in.numel() // dim
-    for t in (resid_in, d1, d2, resid_out, normed_out):
+    for t in (resid_in, None if isinstance(d1, Pieces) else d1, d2, resid_out, normed_out):
         assert t is None or (t.is_contiguous() and t.numel() == rows * dim)
     assert gain.numel() == dim
     p = lambda t: None if t is None else _dev(t)
-    _check(load().lr_add_rmsnorm(_dev(resid_in), p(d1), p(d2), _dev(gain), p(resid_out), _dev(normed_out), rows, dim,
-                                 float(eps), _stream()), "lr_add_rmsnorm")
+    if isinstance(d1, Pieces):
+        assert (d1.rows, d1.dim) == (rows, dim)
+        _check(load().lr_add_rmsnorm_pieces(_dev(resid_in), _dev(d1.sums, d1.sums.dtype), d1.count, p(d2), _dev(gain), p(resid_out),
+                                            _dev(normed_out), rows, dim, float(eps), _stream()), "lr_add_rmsnorm_pieces")
+    else:
+        _check(load().lr_add_rmsnorm(_dev(resid_in), p(d1), p(d2), _dev(gain), p(resid_out), _dev(normed_out), rows, dim,
+                                     float(eps), _stream()), "lr_add_rmsnorm")
     return normed_out
 
 
 class Pieces:
-    """A product [rows, dim] as partial sums: `sums` holds [count][rows][dim] fp32 (linear_pieces); ladder_norms adds them."""
+    """A product [rows, dim] as partial sums: `sums` holds [count][rows][dim] fp32 (linear_pieces); the norms add them."""
 
     def __init__(self, sums: torch.Tensor, count: int, rows: int, dim: int):
         assert sums.is_contiguous() and sums.numel() * sums.element_size() >= count * rows * dim * 4
@@ -611,8 +618,8 @@ def linear_swiglu_out(x: torch.Tensor, w1: torch.Tensor, act: torch.Tensor, scra
 
 def linear_pieces(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, scratch):
     """linear(x, w, out, scratch=scratch), or its partial sums (Pieces in `scratch`, out untouched) where no tile is computed whole.
-    For blocks that a caller puts together itself: the models' prompts leave pieces inside lr_ladder_block, and their decode steps
-    take both output products' together (linear_pieces_two)."""
+    (The ladder's prompts leave pieces inside lr_ladder_block, and its decode steps take both output products' together,
+    linear_pieces_two.)"""
     M, xc, ldx = _rows_ld(x)
     N, K = w.shape
     assert w.is_contiguous() and xc == K and tuple(out.shape) == (M, N)
@@ -688,6 +695,13 @@ def module_linear(x: torch.Tensor, mod, out: torch.Tensor, scratch=None):
     if scales is not None:
         return linear_fp8(x, mod.weight, scales, out)
     return linear(x, mod.weight, out, scratch=scratch)
+
+
+def module_linear_pieces(x: torch.Tensor, mod, out: torch.Tensor, scratch=None):
+    """module_linear, or its partial sums (linear_pieces)."""
+    if getattr(mod, "scales", None) is not None:
+        return linear_fp8(x, mod.weight, mod.scales, out)
+    return linear_pieces(x, mod.weight, out, scratch)
 
 
 def module_linear_swiglu(h: torch.Tensor, mod, out: torch.Tensor, act: torch.Tensor = None, scratch=None):

@@ -262,8 +262,9 @@ class GPTBase(nn.Module):
         in question; weight-only quantised ones have kernels of their own.)"""
         return ws.S == 1 and self.band_rows_from <= ws.B <= self.band_rows_to and not any(hasattr(m, "scales") for m in linears)
 
-    def _attention(self, ws: Workspace, blk, pos: Tensor, wqkv: nn.Module, out: Tensor, roped: bool = False):
-        """ws.xn -> fused projection -> RoPE + cache write -> attention -> wo -> out (partial sum).
+    def _attention(self, ws: Workspace, blk, pos: Tensor, wqkv: nn.Module, out: Tensor, roped: bool = False, pieces: bool = False):
+        """ws.xn -> fused projection -> RoPE + cache write -> attention -> wo -> out (partial sum), returned.
+        pieces: wo's partial sums instead where that is all there is of it (for add_rmsnorm, ahead of any other product).
         wqkv None: ws.qkv already holds the projection (roped: rotated, with k and v already in the cache).
         out None: stop at the attention output ws.y."""
         cfg = self.config
@@ -288,26 +289,27 @@ class GPTBase(nn.Module):
         else:
             _hip.attn_prefill(ws.qkv, kc, vc, pos, ws.y, B, S, Hq, Hkv, hd)
         if out is None:
-            return
+            return None
         if bands:
             _hip.linear_multi((ws.y, blk.attention.wo.weight, out, _hip.EPI_NONE))
-        else:
-            _hip.module_linear(ws.y, blk.attention.wo, out, ws.sums)
+            return out
+        return (_hip.module_linear_pieces if pieces else _hip.module_linear)(ws.y, blk.attention.wo, out, ws.sums)
 
-    def _mlp(self, ws: Workspace, blk, out: Tensor, xn: Optional[Tensor] = None):
+    def _mlp(self, ws: Workspace, blk, out: Tensor, xn: Optional[Tensor] = None, pieces: bool = False):
+        """Returns out, or w2's partial sums as _attention does."""
         ff = blk.feed_forward
         xin = ws.xn if xn is None else xn
         if self._decode_bands(ws, ff.w1, ff.w2):
             _hip.linear_multi((xin, ff.w1.weight, ws.act, _hip.EPI_SWIGLU))
             _hip.linear_multi((ws.act, ff.w2.weight, out, _hip.EPI_NONE))
-            return
+            return out
         if xin.shape[0] > 4 and not hasattr(ff.w1, "scales"):
             # the activation in the first projection's epilogue; up to 4 rows it is fused into w2's GEMV instead
             _hip.linear_swiglu_out(xin, ff.w1.weight, ws.act, ws.h, ws.sums_mlp)
-            _hip.module_linear(ws.act, ff.w2, out, ws.sums_mlp)
-            return
+            return (_hip.module_linear_pieces if pieces else _hip.module_linear)(ws.act, ff.w2, out, ws.sums_mlp)
         _hip.module_linear(xin, ff.w1, ws.h)
         _hip.module_linear_swiglu(ws.h, ff.w2, out, ws.act)
+        return out
 
     # -- greedy decoding helper ---------------------------------------------------------------------
     def greedy_next(self, logits: Tensor) -> Tensor:

@@ -47,13 +47,12 @@ class GPTDense(GPTBase):
     def _run_layers(self, ws: Workspace, pos: Tensor):
         eps = self.config.norm_eps
         pending = None  # module output not yet added to the stream
-        for blk in self.layers:
+        for blk, after in zip(self.layers, [*self.layers[1:], None]):
             if blk.keeps_residual:
                 _hip.add_rmsnorm(ws.x, pending, None, blk.attention_norm.weight, ws.x, ws.xn, eps)
-                self._attention(ws, blk, pos, blk.attention.wqkv, ws.a)
-                _hip.add_rmsnorm(ws.x, ws.a, None, blk.ffn_norm.weight, ws.x, ws.xn, eps)
-                self._mlp(ws, blk, ws.m)
-                pending = ws.m
+                a = self._attention(ws, blk, pos, blk.attention.wqkv, ws.a, pieces=True)
+                _hip.add_rmsnorm(ws.x, a, None, blk.ffn_norm.weight, ws.x, ws.xn, eps)
+                pending = self._mlp(ws, blk, ws.m, pieces=after is not None and after.keeps_residual)
             else:  # the stream is replaced by the module output
                 src = ws.x if pending is None else pending
                 _hip.add_rmsnorm(src, None, None, blk.attention_norm.weight, None, ws.xn, eps)

@@ -60,18 +60,18 @@ class GPTDesync(GPTBase):
         eps = self.config.norm_eps
         tp = float(self.config.tp_world_size)
         pending = None   # a module output whose residual is not divided: its add rides in the next norm launch
-        for blk in self.layers:
+        for blk, after in zip(self.layers, [*self.layers[1:], None]):
             _hip.add_rmsnorm(ws.x, pending, None, blk.attention_norm.weight, None if pending is None else ws.x, ws.xn,
                              eps)
-            self._attention(ws, blk, pos, blk.attention.wqkv, ws.a)
-            pending = ws.a
-            if blk.do_attention_all_reduce and tp != 1.0:
+            divided = blk.do_attention_all_reduce and tp != 1.0
+            pending = self._attention(ws, blk, pos, blk.attention.wqkv, ws.a, pieces=not divided)
+            if divided:
                 _hip.add(ws.a, ws.x, ws.x, tp)
                 pending = None
             _hip.add_rmsnorm(ws.x, pending, None, blk.ffn_norm.weight, None if pending is None else ws.x, ws.xn, eps)
-            self._mlp(ws, blk, ws.m)
-            pending = ws.m
-            if blk.do_mlp_all_reduce and tp != 1.0:
+            divided = blk.do_mlp_all_reduce and tp != 1.0
+            pending = self._mlp(ws, blk, ws.m, pieces=not divided and after is not None)
+            if divided:
                 _hip.add(ws.m, ws.x, ws.x, tp)
                 pending = None
         return pending, None

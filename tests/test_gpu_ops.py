@@ -598,6 +598,25 @@ def test_ladder_blocks_with_the_memory_that_a_model_gives_them(hip, rows, D, I, 
         assert torch.isfinite(got).all() and (got.double() - want.double()).norm() <= 2.0 ** -7 * want.double().norm()
 
 
+@pytest.mark.parametrize("rows,dim,K", [(33, 1024, 8192), (64, 4096, 14336), (65, 2048, 8192), (130, 4096, 4096), (777, 4096, 14336), (48, 8192, 3584)])
+@pytest.mark.parametrize("more", [False, True])
+def test_add_rmsnorm_of_partial_sums(hip, rows, dim, K, more):
+    """The bits of the product with its sum, then the norm."""
+    x, w, gain = rnd(rows, K, seed=240), rnd(dim, K, seed=241, scale=K ** -0.5), 1 + rnd(dim, seed=242, scale=0.1)
+    resid, d2 = rnd(rows, dim, seed=243), rnd(rows, dim, seed=244) if more else None
+    sums = torch.empty(hip.linear_scratch_bytes(rows), dtype=torch.uint8, device=DEV)
+    results = []
+    for leave in (True, False):
+        out = torch.empty(rows, dim, dtype=BF, device=DEV)
+        d1 = (hip.linear_pieces if leave else hip.linear)(x, w, out, scratch=sums)
+        assert isinstance(d1, hip.Pieces) == leave
+        r, n = torch.empty_like(resid), torch.empty_like(resid)
+        hip.add_rmsnorm(resid, d1, d2, gain, r, n, 1e-5)
+        results.append((r, n))
+    for got, want in zip(*results):
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("M", [1, 2, 7, 8])
 @pytest.mark.parametrize("N,K", [(5, 16), (1280, 4112), (2048, 528), (2056, 144), (4104, 2064)])
 def test_bands_of_few_rows_equal_the_bands_of_many(hip, M, N, K):
