@@ -555,7 +555,7 @@ __global__ __launch_bounds__(256 * KSP, KEYS == 32 ? 3 : 2) void k_attn_prefill_
 #pragma unroll
     for (int d = 0; d < DT; ++d)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) o[d][v] = fmaf(mine[(d * 16 + v) * 64], f1, o[d][v] * f0);
+      for (int v = 0; v < 16; ++v) o[d][v] = fmaf(o[d][v], f0, mine[(d * 16 + v) * 64] * f1);
   }
   l += __shfl_xor(l, 32, LR_WAVE);
   if (valid) {
