@@ -53,7 +53,7 @@ class GPTParallel(GPTBase):
         nqkv = GPTBase._fused_width(self)
         for rows, N, K, pair in super()._products(B, S):
             yield rows, N, K, pair
-            if S == 1 and N == self._fused_width():   # (the decode step's two parts of the fused weight)
+            if N == self._fused_width():   # (its two parts)
                 yield rows, nqkv, K, False
                 yield rows, N - nqkv, K, True
 
@@ -61,9 +61,11 @@ class GPTParallel(GPTBase):
         cfg = self.config
         nqkv = (cfg.n_head_local + 2 * cfg.n_kv_local) * cfg.head_dim
         att0 = self.layers[0].attention
-        if (ws.S == 1 and self.band_rows_from <= ws.B <= 64
-                and not any(hasattr(m, "scales") for m in (att0.wqkv1, att0.wo, att0.w2))):
-            return self._run_layers_decode(ws, pos, nqkv)
+        if not any(hasattr(m, "scales") for m in (att0.wqkv1, att0.wo, att0.w2)):
+            if ws.S == 1 and self.band_rows_from <= ws.B <= 64:
+                return self._run_layers_decode(ws, pos, nqkv)
+            if 4 < ws.rows <= self.parts_to or ws.rows >= self.parts_from:
+                return self._run_layers_prompt(ws, pos, nqkv)
         for blk in self.layers:
             att = blk.attention
             _hip.add_rmsnorm(ws.x, None, None, blk.attention_norm.weight, None, ws.xn, cfg.norm_eps)
@@ -75,6 +77,33 @@ class GPTParallel(GPTBase):
             else:
                 ws.x.copy_(ws.m)
         return None, None
+
+    # Rows of a prompt up to which, and from which on, the fused input weight is two products: few rows are launches, many are passes over
+    # the products' rows; in between one product leaves less of the last round of tiles empty (8B, us per prompt, one / two: 30 tokens
+    # 4391 / 4288, 50 4414 / 3797, 100 4986 / 4479, 150 5381 / 5165, 190 5462 / 5592, 400 7718 / 7878, 666 10134 / 10330, 4 x 2000 92032 / 89111, of which
+    # the attention's own gain is 1750; 220 to 300 and 600 to 2300 no difference but the attention's)
+    parts_to, parts_from = 160, 4096
+
+    def _run_layers_prompt(self, ws: Workspace, pos: Tensor, nqkv: int):
+        """Prompts (and decode batches above 64): the rows of the fused input weight as two products, whose output passes rotate and cache, and
+        apply the activation; y + x with the next norm.  Eight launches for the eleven of one product and passes over its rows."""
+        cfg = self.config
+        Hq, Hkv, hd = cfg.n_head_local, cfg.n_kv_local, cfg.head_dim
+        pending = None
+        for blk in self.layers:
+            att, kv = blk.attention, blk.attention.kv_cache
+            _hip.add_rmsnorm(ws.x, pending, None, blk.attention_norm.weight, None if pending is None else ws.x, ws.xn, cfg.norm_eps)
+            w = att.wqkv1.weight
+            _hip.linear_rope_kv(ws.xn, w[:nqkv], ws.qkv[:, :nqkv], self.freqs_cis, pos, kv.k_cache, kv.v_cache, ws.B, ws.S, Hq, Hkv, hd, ws.sums)
+            self._attention(ws, blk, pos, None, ws.a, roped=True)
+            _hip.linear_swiglu_out(ws.xn, w[nqkv:], ws.act, ws.h, ws.sums)
+            _hip.linear(ws.act, att.w2.weight, ws.m, scratch=ws.sums)
+            _hip.add(ws.m, ws.a, ws.m)                               # w2(...) + wo(...)
+            pending = ws.m
+            if not blk.keeps_residual:
+                ws.x.copy_(ws.m)
+                pending = None
+        return pending, None
 
     def _run_layers_decode(self, ws: Workspace, pos: Tensor, nqkv: int):
         """Decode step through the weight-streaming bands.  The rows of the fused input weight are two projections

@@ -1015,6 +1015,32 @@ def test_variants_on_70b_shard_shape_at_full_depth(family, B):
     check(stats)
 
 
+@pytest.mark.parametrize("B,S", [(1, 5), (2, 17), (1, 60), (4, 40), (5, 33)])
+@pytest.mark.parametrize("semi", [False, True])
+@torch.no_grad()
+def test_parallel_prompts_by_one_product_or_two(B, S, semi, monkeypatch):
+    """The fused input weight as two products with their output passes against one product and passes over its rows: rounded sums of
+    another order differ by a step of bf16 (2^-8) here and there, a stream of three such blocks by 2^-6 by norm."""
+    from gpt_fast import _hip
+
+    model = build("parallel", **dict(TINY, tp_world_size=2, tp_rank=1, semi_compiled_model=semi))
+    model.setup_caches(B, 64)
+    toks = torch.randint(0, 512, (B, S), device=DEV, generator=torch.Generator(device=DEV).manual_seed(4))
+    passes, rope = [], _hip.rope_kv_write
+    monkeypatch.setattr(_hip, "rope_kv_write", lambda *a: (passes.append(a), rope(*a))[1])
+    results = []
+    for parts_to in (model.parts_to, 0):
+        model.parts_to = parts_to
+        passes.clear()
+        out = model(toks, torch.arange(S, device=DEV)).clone()
+        model.check_device_errors()
+        kv = model.layers[-1].attention.kv_cache
+        results.append((out, kv.k_cache[:, :, :S].clone(), kv.v_cache[:, :, :S].clone()))
+        assert bool(passes) == (B * S > parts_to)
+    for got, want in zip(*results):
+        assert torch.isfinite(got).all() and (got.double() - want.double()).norm() <= 2.0 ** -6 * want.double().norm()
+
+
 @pytest.mark.parametrize("family", ["dense", "desync", "parallel"])
 @pytest.mark.parametrize("B", [3, 20])
 @pytest.mark.parametrize("semi", [False, True])
