@@ -100,9 +100,9 @@ def test_a_batch_gives_every_sequence_what_it_gets_alone(case, dtype):
 
 
 @pytest.mark.parametrize("case", ["mixed", "plain", "large"])
-@pytest.mark.parametrize("batch", [2, 3, 16, 17])
+@pytest.mark.parametrize("batch", [1, 2, 3, 16, 17])
 def test_decode_batches_with_norms_in_the_projections(case, batch, monkeypatch):
-    """3 to 16 rows ("plain": also behind a layer without a feed-forward) and the batches next to them: every sequence as alone."""
+    """2 to 16 rows ("plain": also behind a layer without a feed-forward) and the batches next to them: every sequence as alone."""
     from gpt_fast import _hip
     from test_gpu_gepolix_model import each, replays_equal_eager
 
@@ -113,7 +113,7 @@ def test_decode_batches_with_norms_in_the_projections(case, batch, monkeypatch):
     rows = [C.tokens(cfg, 40, seed=i) for i in range(batch)]
     got = s.feed(rows, [31] + [1] * 9)
     sublayers = sum(1 + (layer["mlp"] is not None) for layer in cfg["layers"])
-    assert len(launches) == (9 * sublayers if 3 <= batch <= 16 else 0)
+    assert len(launches) == (9 * sublayers if 2 <= batch <= 16 else 0)
     for r, g in list(zip(rows, got))[::4]:   # (single positions: see test_decode_batches_above_32_run_products)
         off = each(g, s.want(r))
         assert off.median() < TOL[BF] / 2 and (off < TOL[BF]).double().mean() >= 0.9
