@@ -75,8 +75,8 @@ class GPTLasivik(GPTHybrid):
         _hip.residual_rmsnorm(ws.x, alpha, d, norm.weight, ws.x, ws.xc, norm.eps, self.config.width, gain_offset=1.0)
 
     # Decode batches from which a norm is part of the projections on either side of it.  (Two rows' wide projections, which are the
-    # matrix-vector kernel's otherwise, see project, take 2 us longer in bands and the two norms of a layer 10: 8B at 1000 tokens, with norms of
-    # their own 3495 us per step, without 3253.  One row is the matrix-vector kernel's throughout.)
+    # matrix-vector kernel's otherwise, see project, take 2 us longer in bands and the two norms of a layer 10: 4 % of an 8B step at 1000
+    # tokens, 2 % of a 1B one.  One row is the matrix-vector kernel's throughout.)
     norms_in_projections_from = 2
 
     def _run_layers_decode(self, ws, pos):
