@@ -590,8 +590,10 @@ static int launch_prefill_heads(const u16* q, int64_t ldq, const u16* kc, const 
   constexpr int queries = 32 * (4 / NWH);
   const int64_t n = (int64_t)((S + queries - 1) / queries) * (Hq / NWH) * B;
   const int cus = lr_num_cus();
-  auto run = n <= cus && S >= PREFILL_PARTS_FROM ? &launch_prefill_as<HD, NWH, 2, 64, WIN>
-             : HD == 128 && (n > 2 * cus || S <= 128) ? &launch_prefill_as<HD, NWH, 1, 32, WIN> : &launch_prefill_as<HD, NWH, 1, 64, WIN>;
+  auto run = &launch_prefill_as<HD, NWH, 1, 64, WIN>;
+  if constexpr (HD == 128)
+    if (n > 2 * cus || S <= 128) run = &launch_prefill_as<HD, NWH, 1, 32, WIN>;
+  if (n <= cus && S >= PREFILL_PARTS_FROM) run = &launch_prefill_as<HD, NWH, 2, 64, WIN>;
   return run((unsigned)n, q, ldq, kc, vc, pos, y, ldy, S, Hq, Hkv, Smax, w, s);
 }
 // NWH heads of a kv head in a workgroup: as many of four as divide its share
