@@ -11,8 +11,8 @@
 //
 // A workgroup (4 waves, one per SIMD, so each has the whole register budget) owns a band of up to
 // 32 weight rows -- the number of rows is chosen so that every CU gets the same share -- and its
-// waves split K in 128-element chunks (wave w takes chunks w, w + 4, ...: together they read 1 KiB
-// contiguous per row and round).  Each wave keeps 4 chunks of weights (32 KiB) in flight in
+// waves walk K in 128-element chunks, a slice of K each (stream_band; e4m3 bands and lr_linear_resid's deal
+// the chunks round the waves).  Each wave keeps 4 chunks of weights (32 KiB) in flight in
 // registers, 128 KiB per CU.  The input rows come from L2 straight into B-fragment layout.  The waves' partial sums
 // meet in LDS and are added in a fixed order.
 //
