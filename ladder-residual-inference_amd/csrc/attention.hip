@@ -267,17 +267,26 @@ struct WindowKeys {
 // where is XOR-ed with the key, see key_swizzle and value_swizzle, so that the fragment reads below meet no bank twice), one portion
 // ahead of the products: one barrier per 64 keys.  V^T fragments are read across the rows (ds_read_b64_tr_b16).
 // KSP 2: a grid that leaves CUs without a second workgroup has eight waves in a workgroup, the second four the second 32 keys of every portion
-// for the same queries; their results are merged at the end.  From 512 queries on, where that pays for the merge (8 heads of 128, one
-// sequence, us: 2048 tokens 51.0 -> 45.5, 777 of 32 heads 23.8 -> 23.1, 256 of 32 heads of 64 8.3 -> 8.6).
-// KEYS 32: 32 at a time and with fewer registers, so that three workgroups share a CU where the grid has as many (8 x 2048 tokens, 32 heads of
-// 128: 399 us, three to a CU 375; two to a CU 408; 328 workgroups 38.6, so 42.9 to 46.2), and for short prompts, which have less to wait for.
+// for the same queries; their results are merged at the end.  From 512 keys on, where that pays for the merge (us, four waves / eight: 32 heads
+// of 128, 512 tokens 17.5 / 17.3, 777 23.3 / 22.4; 16 heads, 1500 tokens, window of 1024 30.7 / 28.1, of 128 10.9 / 11.7).  Keys, as far as
+// the host knows them: those of the call itself or of its window.  (A portion of 32 to 256 tokens at position 3000 would be 10 to 15 %
+// faster with eight waves, 32 tokens of 32 heads 72 / 62, but at position 0, where it is 6.5 / 8.2, looks the same to the host.)
+// KEYS 32: 32 at a time and with fewer registers, so that three workgroups share a CU where the grid has as many (64 / 32: 32 heads, 8 kv heads of
+// 128, 8 x 2048 tokens 401 / 397, 4 x 777 44.2 / 41.8, 4 x 1024 62.5 / 63.1, 4 x 1300 93.0 / 96.5; 2 x 1500 of window 128 27.2 / 25.0),
+// and for the 33 to 96 queries of two heads to a workgroup, whose first 32 have no use for the second 32 keys (28 heads, 14 kv heads, 64 tokens
+// 7.5 / 6.9).
+// HALF: a last portion of up to 32 keys is computed as such.  Short prompts are one (us without / with: 32 heads, 8 kv heads of 64, 32 tokens 5.31 /
+// 4.73, 100 tokens 6.29 / 5.78; of 128, 16 tokens 6.28 / 5.71, 32 tokens 7.02 / 6.49), and narrow windows have few others (1500 tokens, window of 128
+// 11.1 / 10.1).  Heads of 64: up to 128 keys, the loop is slower beside a second copy of its body (32 tokens at position 3000 47.5 / 51.0).
+// Heads of 64 keep to the 128 registers that let four workgroups share a CU (40 heads, 20 kv heads, 3000 tokens, window of 128: three to a CU
+// 22.6 us, four 19.0).
 // Bound: matrix instructions 48 % of a SIMD's cycles, vector instructions 46 % (exponentials at a quarter of the rate, splitting P), which hardly
 // run at the same time, in another wave or between the matrix instructions of the same one (written so, it took as long).  No bank
 // conflicts.  Before (32 keys in one LDS buffer through registers, V transposed on its way in, two barriers) / now, us: 32 heads of 128,
-// 8 kv heads: 8 x 2048 tokens 503 / 400 (550 / 690 TFLOP/s of products), 4096 229 / 196, 1300 47.4 / 39.6, 777 29.6 / 23.8, 300 13.9 / 12.9, 100
-// 8.2 / 8.5; of 64: 4 x 4096 497 / 423, 512 15.4 / 12.4, 128 6.8 / 6.4.
+// 8 kv heads: 8 x 2048 tokens 460 / 396 (598 / 694 TFLOP/s of products), 4 x 1300 112 / 96, 2 x 1000 50.8 / 35.9, 777 28.4 / 22.4, 300 14.0 / 12.3,
+// 100 8.2 / 8.0, 32 6.3 / 6.5, 16 5.6 / 5.7; of 64: 4 x 1024 59.9 / 40.1, 512 15.1 / 11.8, 100 6.3 / 5.8, 32 4.8 / 4.7.
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
-constexpr int PREFILL_PARTS_FROM = 512;   // queries, see above
+constexpr int PREFILL_PARTS_FROM = 512, PREFILL_HALF_TO = 128;   // keys that are seen, see above
 template <int HD, int KSP, int KEYS>
 struct PrefillLds {
   static constexpr int TILE = KEYS * HD * 2, STAGE = 2 * TILE;   // a portion's keys or values; both
@@ -293,8 +302,8 @@ __device__ __forceinline__ int value_swizzle(int key) { return HD == 128 ? (key 
 
 // WIN (lr_window_attention): a sliding window, the score scale as an argument, and the kv heads' keys and values side by
 // side as rows of a matrix, in the order lr_latent_window gives them; head sizes up to HD.
-template <int HD, int NWH, int KSP, int KEYS, bool WIN>
-__global__ __launch_bounds__(256 * KSP, KEYS == 32 ? 3 : 2) void k_attn_prefill_mfma(const u16* __restrict__ q, int64_t ldq,
+template <int HD, int NWH, int KSP, int KEYS, bool HALF, bool WIN>
+__global__ __launch_bounds__(256 * KSP, HD == 64 ? 4 : KEYS == 32 ? 3 : 2) void k_attn_prefill_mfma(const u16* __restrict__ q, int64_t ldq,
                                                                     const u16* __restrict__ kc, const u16* __restrict__ vc,
                                                                     const int32_t* __restrict__ pos, u16* __restrict__ y,
                                                                     int64_t ldy, int S, int Hq, int Hkv, int Smax,
@@ -343,18 +352,23 @@ __global__ __launch_bounds__(256 * KSP, KEYS == 32 ? 3 : 2) void k_attn_prefill_
   } else {
     p = p >= Smax ? Smax - 1 : p;
   }
-  // the last key of this wave's queries, and keys needed by anybody in the workgroup
-  int kmax = p;
+  // the last and the first key of this wave's queries (lanes without one do not count), and
+  // the keys needed by anybody in the workgroup
+  int kmax = p, pmin = valid ? p : 0x7fffffff;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
-    const int t = __shfl_xor(kmax, o, LR_WAVE);
+    const int t = __shfl_xor(kmax, o, LR_WAVE), u = __shfl_xor(pmin, o, LR_WAVE);
     kmax = t > kmax ? t : kmax;
+    pmin = u < pmin ? u : pmin;
   }
   const int pmax = __builtin_amdgcn_readfirstlane(kmax);
-  int* const s_kmax = reinterpret_cast<int*>(prefill_lds + L::KMAX);
-  if (lane == 0) s_kmax[wave] = kmax;
-  __syncthreads();
-  kmax = max(max(s_kmax[0], s_kmax[1]), max(s_kmax[2], s_kmax[3]));
+  pmin = __builtin_amdgcn_readfirstlane(pmin);
+  if constexpr (NWQ > 1) {   // (else all waves have the same queries)
+    int* const s_kmax = reinterpret_cast<int*>(prefill_lds + L::KMAX);
+    if (lane == 0) s_kmax[wave] = kmax;
+    __syncthreads();
+    kmax = max(max(s_kmax[0], s_kmax[1]), max(s_kmax[2], s_kmax[3]));
+  }
   const int nkeys = __builtin_amdgcn_readfirstlane(kmax + 1);
   // (WIN) the first portion anybody in the workgroup sees
   int t_first = 0;
@@ -391,14 +405,6 @@ __global__ __launch_bounds__(256 * KSP, KEYS == 32 ? 3 : 2) void k_attn_prefill_
   float m = -INFINITY, l = 0.0f;  // m: reference point in raw score units; l: this lane's half of the row sum
   const float c2 = (WIN ? w.scale : rsqrtf((float)HD)) * 1.4426950408889634f;  // e^(x / sqrt(HD)) = 2^(x c2)
   const float tau_raw = PREFILL_TAU2 / c2;
-  // the smallest position among the wave's queries (lanes without a query do not count)
-  int pmin = valid ? p : 0x7fffffff;
-#pragma unroll
-  for (int o_ = 32; o_ > 0; o_ >>= 1) {
-    const int t = __shfl_xor(pmin, o_, LR_WAVE);
-    pmin = t < pmin ? t : pmin;
-  }
-  pmin = __builtin_amdgcn_readfirstlane(pmin);
   const int krow = WIN ? w.ld : HD;   // elements from key to key
   const u16* kbase = WIN ? kc + (int64_t)b * w.n_keys * w.ld + kvh * w.dk : kc + ((int64_t)b * Hkv + kvh) * Smax * HD;
   const u16* vbase = WIN ? vc + (int64_t)b * w.n_keys * w.ld + kvh * w.dv : vc + ((int64_t)b * Hkv + kvh) * Smax * HD;
@@ -442,36 +448,35 @@ __global__ __launch_bounds__(256 * KSP, KEYS == 32 ? 3 : 2) void k_attn_prefill_
   }
   if (t_first < nkeys) stage(t_first, 0);
   int buf = 0;
-  for (int t0 = t_first; t0 < nkeys; t0 += KEYS, buf ^= 1) {
-    // this portion has arrived, for all waves, and nobody reads the one before any more
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (t0 + KEYS < nkeys) stage(t0 + KEYS, buf ^ 1);
+  // N 32-key tiles of the portion at t0, for this wave's queries
+  auto tiles = [&](auto N_, const int t0, const int buf) {
+    constexpr int N = decltype(N_)::value;
     const int tk = t0 + part * 32;
-    if (tk > pmax || (WIN && tk + 32 * NS - 1 <= pmin - w.window)) continue;   // nothing here for this wave's queries
+    if (tk > pmax || (WIN && tk + 32 * N - 1 <= pmin - w.window)) return;   // nothing here for them
     const unsigned char* const at = prefill_lds + buf * L::STAGE;
     // ---- S^T tiles: rows = keys, columns = queries
-    f32x16_t sacc[NS];
+    f32x16_t sacc[N];
 #pragma unroll
-    for (int n = 0; n < NS; ++n)
+    for (int n = 0; n < N; ++n)
 #pragma unroll
       for (int v = 0; v < 16; ++v) sacc[n][v] = 0.0f;
-    u32x4_t ka[KS][NS];   // (all on their way before the first product)
+    u32x4_t ka[KS][N];   // (all on their way before the first product)
 #pragma unroll
     for (int i = 0; i < KS; ++i)
 #pragma unroll
-      for (int n = 0; n < NS; ++n) ka[i][n] = *reinterpret_cast<const u32x4_t*>(at + (kat ^ (32 * i)) + n * 32 * RB);
+      for (int n = 0; n < N; ++n) ka[i][n] = *reinterpret_cast<const u32x4_t*>(at + (kat ^ (32 * i)) + n * 32 * RB);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < KS; ++i)
 #pragma unroll
-      for (int n = 0; n < NS; ++n)
+      for (int n = 0; n < N; ++n)
         sacc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, ka[i][n]), __builtin_bit_cast(bf16x8_t, qb[i]),
                                                           sacc[n], 0, 0, 0);
     // element v of tile n is key tk + 32 n + (v / 4) * 8 + half * 4 + v % 4 for query `col`; only a portion that reaches past the
     // smallest position of the wave's queries has anything to mask
-    if (tk + 32 * NS - 1 > pmin || (WIN && tk <= pmax - w.window)) {
+    if (tk + 32 * N - 1 > pmin || (WIN && tk <= pmax - w.window)) {
 #pragma unroll
-      for (int n = 0; n < NS; ++n)
+      for (int n = 0; n < N; ++n)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const int key = tk + 32 * n + (v / 4) * 8 + half * 4 + (v % 4);
@@ -480,7 +485,7 @@ __global__ __launch_bounds__(256 * KSP, KEYS == 32 ? 3 : 2) void k_attn_prefill_
     }
     float tmax = max_med3(sacc[0][0], sacc[0][1]);
 #pragma unroll
-    for (int v = 2; v < 16 * NS; ++v) tmax = max_med3(tmax, sacc[v / 16][v % 16]);
+    for (int v = 2; v < 16 * N; ++v) tmax = max_med3(tmax, sacc[v / 16][v % 16]);
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32, LR_WAVE));
     // The reference point m of the exponentials follows the running maximum lazily: it moves only when a portion's
     // maximum exceeds it by more than PREFILL_TAU2 / c2, so the weights stay below 2^PREFILL_TAU2 (harmless in fp32,
@@ -499,7 +504,7 @@ __global__ __launch_bounds__(256 * KSP, KEYS == 32 ? 3 : 2) void k_attn_prefill_
         for (int v = 0; v < 16; ++v) o[d][v] *= corr;
     }
 #pragma unroll
-    for (int n = 0; n < NS; ++n) {
+    for (int n = 0; n < N; ++n) {
       u32x4_t phi[2], plo[2];
 #pragma unroll
       for (int h2 = 0; h2 < 2; ++h2)
@@ -534,6 +539,19 @@ __global__ __launch_bounds__(256 * KSP, KEYS == 32 ? 3 : 2) void k_attn_prefill_
           o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[d], __builtin_bit_cast(bf16x8_t, plo[h2]), o[d], 0, 0, 0);
       }
     }
+  };
+  // (that portion has arrived, for all waves, and nobody reads the one before any more)
+  auto arrived = [] { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  constexpr int LAST = HALF ? 32 : 0;
+  int t0 = t_first;
+  for (; t0 + LAST < nkeys; t0 += KEYS, buf ^= 1) {
+    arrived();
+    if (t0 + KEYS < nkeys) stage(t0 + KEYS, buf ^ 1);
+    tiles(std::integral_constant<int, NS>{}, t0, buf);
+  }
+  if (HALF && t0 < nkeys) {   // at most 32 keys are left
+    arrived();
+    tiles(std::integral_constant<int, 1>{}, t0, buf);
   }
   if constexpr (KSP == 2) {
     // the second four waves' results to the first four, which saw the other keys of the same queries
@@ -575,13 +593,13 @@ __global__ __launch_bounds__(256 * KSP, KEYS == 32 ? 3 : 2) void k_attn_prefill_
   }
 }
 
-template <int HD, int NWH, int KSP, int KEYS, bool WIN>
+template <int HD, int NWH, int KSP, int KEYS, bool HALF, bool WIN>
 static int launch_prefill_as(unsigned workgroups, const u16* q, int64_t ldq, const u16* kc, const u16* vc, const int32_t* pos, u16* y, int64_t ldy,
                              int S, int Hq, int Hkv, int Smax, const WindowKeys& w, hipStream_t s) {
   constexpr size_t lds = PrefillLds<HD, KSP, KEYS>::BYTES;
   static std::atomic<unsigned long long> raised{0};
-  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_attn_prefill_mfma<HD, NWH, KSP, KEYS, WIN>), lds, raised)) return LR_E_LAUNCH;
-  k_attn_prefill_mfma<HD, NWH, KSP, KEYS, WIN><<<dim3(workgroups), dim3(256 * KSP), lds, s>>>(q, ldq, kc, vc, pos, y, ldy, S, Hq, Hkv, Smax, w);
+  if (!lr_raise_lds_limit(reinterpret_cast<const void*>(&k_attn_prefill_mfma<HD, NWH, KSP, KEYS, HALF, WIN>), lds, raised)) return LR_E_LAUNCH;
+  k_attn_prefill_mfma<HD, NWH, KSP, KEYS, HALF, WIN><<<dim3(workgroups), dim3(256 * KSP), lds, s>>>(q, ldq, kc, vc, pos, y, ldy, S, Hq, Hkv, Smax, w);
   return lr_launch_status();
 }
 template <int HD, int NWH, bool WIN>
@@ -590,10 +608,14 @@ static int launch_prefill_heads(const u16* q, int64_t ldq, const u16* kc, const 
   constexpr int queries = 32 * (4 / NWH);
   const int64_t n = (int64_t)((S + queries - 1) / queries) * (Hq / NWH) * B;
   const int cus = lr_num_cus();
-  auto run = &launch_prefill_as<HD, NWH, 1, 64, WIN>;
-  if constexpr (HD == 128)
-    if (n > 2 * cus || S <= 128) run = &launch_prefill_as<HD, NWH, 1, 32, WIN>;
-  if (n <= cus && S >= PREFILL_PARTS_FROM) run = &launch_prefill_as<HD, NWH, 2, 64, WIN>;
+  const int seen = WIN && w.window < S ? w.window : S;   // keys (at least: how long the history ahead of the queries is only the device knows)
+  auto run = &launch_prefill_as<HD, NWH, 1, 64, true, WIN>;
+  if constexpr (HD == 128) {
+    if (n > 2 * cus || (NWH == 2 && S > 32 && S <= 96)) run = &launch_prefill_as<HD, NWH, 1, 32, false, WIN>;
+  } else {
+    if (seen > PREFILL_HALF_TO) run = &launch_prefill_as<HD, NWH, 1, 64, false, WIN>;
+  }
+  if (n <= cus && seen >= PREFILL_PARTS_FROM) run = &launch_prefill_as<HD, NWH, 2, 64, false, WIN>;
   return run((unsigned)n, q, ldq, kc, vc, pos, y, ldy, S, Hq, Hkv, Smax, w, s);
 }
 // NWH heads of a kv head in a workgroup: as many of four as divide its share

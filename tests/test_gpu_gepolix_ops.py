@@ -326,6 +326,31 @@ def test_window_attention_over_a_cache(hip, dtype, H, G, dk, dv, window):
             assert torch.isnan(y[:, H * dv:]).all()
 
 
+# (eight waves to a workgroup: windows of 512 and more, from a first key that is an odd multiple of 32; 32 keys at a time: grids beyond twice
+# the CUs; a last half of a portion: heads of 128, and windows of up to 128; one, two and four heads to a workgroup)
+@pytest.mark.parametrize("B,S,H,G,d,window,start", [
+    (1, 520, 8, 2, 128, 512, 95), (1, 700, 4, 4, 128, 543, 1000), (2, 513, 6, 3, 64, 600, 607), (1, 600, 8, 1, 64, 513, 0), (1, 512, 4, 4, 64, 1000, 1100),
+    (6, 300, 32, 32, 128, 100, 40), (2, 200, 64, 1, 128, 64, 33), (1, 300, 8, 2, 128, 63, 100), (1, 161, 6, 3, 128, 64, 95), (1, 530, 4, 4, 128, 65, 0),
+    (1, 96, 8, 4, 128, 500, 200), (2, 300, 8, 2, 64, 128, 33), (1, 290, 6, 3, 64, 129, 31), (1, 600, 4, 4, 64, 33, 64), (1, 100, 8, 2, 64, 2000, 130)])
+def test_window_attention_portions_of_keys(hip, B, S, H, G, d, window, start):
+    """In each query's window one key stands out, alternately the first it sees and the last it does not; nothing beyond the last position, and
+    no key ahead of the first window, is used."""
+    L = start + S + 40
+    cache, q = rnd(B, L, 2 * G * d, seed=1, dtype=BF), rnd(B, S, H * d, seed=2, dtype=BF)
+    for i in range(S):
+        j = start + i - window + 1 - (i % 2)
+        if j >= 0:
+            for g in range(G):
+                cache[:, j, g * d:(g + 1) * d] = (q[:, i].view(B, H, d)[:, g * (H // G)] * 3).to(BF)
+    want = [O.grouped_window_attention(d64(q[b]).view(S, H, d), d64(cache[b, :start + S, :G * d]).reshape(-1, G, d),
+                                       d64(cache[b, :start + S, G * d:]).reshape(-1, G, d), start, window, d ** -0.5).reshape(S, -1) for b in range(B)]
+    cache[:, start + S:] = float("nan")
+    cache[:, :max(0, start - window + 1) // 32 * 32] = float("nan")
+    y = torch.full((B * S, H * d), float("nan"), dtype=BF, device=DEV)
+    hip.window_attention(q.view(B * S, -1), cache.view(B * L, -1), y, at_pos(start, S), B, S, H, d, d, window, L, L, d ** -0.5, kv_heads=G)
+    close(y.view(B, S, -1), torch.stack(want), BF)
+
+
 def test_window_decode_cuts_long_windows_into_ranges(hip):
     B, H, G, d, L = 1, 4, 1, 64, 5000
     cache, q = rnd(B, L, 2 * d, seed=1, dtype=BF), rnd(B, H * d, seed=2, dtype=BF)

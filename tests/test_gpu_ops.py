@@ -1211,7 +1211,11 @@ def test_attn_prefill(hip, B, S, Hq, Hkv, hd, Smax, start):
 @pytest.mark.parametrize("B,S,Hq,Hkv,hd,start", [
     (1, 16, 4, 1, 128, 0), (2, 33, 8, 2, 128, 31), (1, 128, 6, 3, 128, 64), (1, 129, 32, 8, 128, 0), (3, 161, 2, 2, 128, 95), (1, 511, 8, 2, 128, 1),
     (1, 512, 8, 1, 128, 0), (1, 545, 6, 3, 128, 63), (2, 600, 2, 2, 128, 200), (8, 520, 32, 8, 128, 0), (5, 610, 28, 7, 128, 17),
-    (1, 17, 4, 1, 64, 0), (1, 130, 6, 3, 64, 33), (1, 512, 32, 8, 64, 0), (1, 577, 2, 2, 64, 64), (8, 530, 32, 8, 64, 3)])
+    (1, 17, 4, 1, 64, 0), (1, 130, 6, 3, 64, 33), (1, 512, 32, 8, 64, 0), (1, 577, 2, 2, 64, 64), (8, 530, 32, 8, 64, 3),
+    # the last portion: one key, 32 and 33 of them, alone and behind others, where it is computed as half of one and where it is not
+    (1, 16, 4, 1, 128, 17), (2, 32, 8, 2, 128, 0), (1, 32, 4, 1, 128, 64), (1, 65, 8, 2, 128, 0), (3, 97, 8, 8, 128, 0), (1, 96, 6, 3, 128, 0),
+    (1, 33, 6, 3, 128, 64), (1, 97, 4, 2, 128, 63), (2, 32, 8, 2, 64, 0), (1, 33, 4, 1, 64, 0), (1, 65, 6, 3, 64, 0), (3, 96, 2, 2, 64, 0),
+    (1, 128, 4, 1, 64, 1), (1, 129, 4, 1, 64, 0), (1, 129, 4, 4, 64, 31)])
 def test_attn_prefill_portions_of_keys(hip, B, S, Hq, Hkv, hd, start):
     """Nothing beyond the last position is used, whatever lies there."""
     n = start + S
