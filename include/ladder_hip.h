@@ -127,6 +127,8 @@ typedef struct lr_linear_plan {
   size_t sums_bytes;            /* of the pieces' sums */
 } lr_linear_plan_t;
 int lr_linear_plan(int M, int N, int K, int pair, size_t scratch_bytes, lr_linear_plan_t* plan);
+/* The us that the costs behind that plan give the product, its own launches included; 0 where lr_linear_plan refuses. */
+float lr_linear_plan_us(int M, int N, int K, int pair, size_t scratch_bytes);
 int lr_linear_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, void* scratch,
                       size_t scratch_bytes, lr_stream_t stream);
 

@@ -1270,6 +1270,12 @@ extern "C" int lr_linear_plan(int M, int N, int K, int pair, size_t scratch_byte
   return LR_OK;
 }
 
+extern "C" float lr_linear_plan_us(int M, int N, int K, int pair, size_t scratch_bytes) {
+  if (M <= 0 || N <= 0 || K <= 0 || (pair && N % 2) || K % 8) return 0.0f;
+  const GemmPlan p = gemm_plan(M, pair ? N / 2 : N, K, pair ? GEMM_PAIR : GEMM_PLAIN, scratch_bytes);
+  return p.tile < 0 ? 0.0f : p.us;
+}
+
 extern "C" int lr_linear_scratch(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int M, int N, int K, void* scratch,
                                  size_t scratch_bytes, lr_stream_t stream) {
   LR_OPTIONAL_PTR(scratch);

@@ -30,6 +30,7 @@ _PROTOS = {
                                 c_void_p]),
     "lr_linear_scratch_bytes": (c_size_t, [c_int]),
     "lr_linear_plan": (c_int, [c_int, c_int, c_int, c_int, c_size_t, c_void_p]),
+    "lr_linear_plan_us": (c_float, [c_int, c_int, c_int, c_int, c_size_t]),
     "lr_linear_scratch": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_size_t,
                                   c_void_p]),
     "lr_linear_pieces": (c_int, [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_void_p, c_size_t, c_void_p, c_void_p]),
@@ -306,6 +307,11 @@ def linear_plan(rows: int, N: int, K: int, pair: bool = False, scratch_bytes: in
     n = linear_scratch_bytes(rows) if scratch_bytes is None else scratch_bytes
     _check(load().lr_linear_plan(rows, N, K, int(pair), n, ctypes.byref(p)), "lr_linear_plan")
     return p
+
+
+def linear_plan_us(rows: int, N: int, K: int, pair: bool = False) -> float:
+    """The us that its costs give such a product with all the scratch it could use (lr_linear_plan_us)."""
+    return float(load().lr_linear_plan_us(rows, N, K, int(pair), linear_scratch_bytes(rows)))
 
 
 def linear_sums_bytes(products) -> int:

@@ -38,6 +38,10 @@ class GPTParallel(GPTBase):
     family = "parallel"
     band_rows_from = 1   # six launches per block instead of nine also pay for a single row (5.6 -> 5.0 ms, 70B shard)
 
+    def __init__(self, config):
+        super().__init__(config)
+        self._parts_pay = {}   # (rows, of a decode step): see _in_parts
+
     def _make_block(self, config, layer_idx):
         return ParallelTransformerBlock(config)
 
@@ -53,7 +57,7 @@ class GPTParallel(GPTBase):
         nqkv = GPTBase._fused_width(self)
         for rows, N, K, pair in super()._products(B, S):
             yield rows, N, K, pair
-            if N == self._fused_width():   # (its two parts)
+            if N == self._fused_width() and (S == 1 and B <= 64 or self._in_parts(B, S)):   # (its two parts)
                 yield rows, nqkv, K, False
                 yield rows, N - nqkv, K, True
 
@@ -64,7 +68,7 @@ class GPTParallel(GPTBase):
         if not any(hasattr(m, "scales") for m in (att0.wqkv1, att0.wo, att0.w2)):
             if ws.S == 1 and self.band_rows_from <= ws.B <= 64:
                 return self._run_layers_decode(ws, pos, nqkv)
-            if 4 < ws.rows <= self.parts_to or ws.rows >= self.parts_from:
+            if self._in_parts(ws.B, ws.S):
                 return self._run_layers_prompt(ws, pos, nqkv)
         for blk in self.layers:
             att = blk.attention
@@ -78,11 +82,34 @@ class GPTParallel(GPTBase):
                 ws.x.copy_(ws.m)
         return None, None
 
-    # Rows of a prompt up to which, and from which on, the fused input weight is two products: few rows are launches, many are passes over
-    # the products' rows; in between one product leaves less of the last round of tiles empty (8B, us per prompt, one / two: 30 tokens
-    # 4391 / 4288, 50 4414 / 3797, 100 4986 / 4479, 150 5381 / 5165, 190 5462 / 5592, 400 7718 / 7878, 666 10134 / 10330, 4 x 2000 92032 / 89111, of which
-    # the attention's own gain is 1750; 220 to 300 and 600 to 2300 no difference but the attention's)
+    # Rows (of a prompt, or a decode batch above 64) whose fused input weight is two products with their output passes, eight launches for
+    # eleven and no passes over the products' rows: up to 32, from parts_from on, and up to parts_to where the products' costs say that
+    # they take no longer than one and what it leaves out: 8 us of passes, and 6 more for the launches of a prompt, which come one by one and take
+    # about 110 us per block, where one product takes up to 50 (the other half of such a block is no longer).
+    # us, one / two, one library, shapes of 8B, 1B, the 70B rank shard and Llama 3.2 3B.  A decode step's graph: 70 sequences 5198 / 4771,
+    # 1273 / 1306, 6884 / 7018, 3070 / 3300, 160 sequences 5902 / 5759, 1520 / 1582, 8649 / 8529, 4044 / 4134; only 8B's is two.  A prompt as it is
+    # called: 30 tokens 4390 / 4234, 1722 / 1602, 7725 / 7046, 3022 / 2772, 64 tokens 4437 / 3808, 1880 / 1769, 8468 / 7801, 3216 / 2920, 150 tokens
+    # 5375 / 5259, 1786 / 1579, 8655 / 8417, 3071 / 3195; above 32 all but 3B's are two, though 1B's take 3 to 5 % longer on the device (64 tokens
+    # 1092 / 1148) and the shard's up to 3.  Shapes that the line was not drawn from, of 6 and 12 layers: 70B 64 tokens 2161 / 1973, 160 sequences
+    # 2954 / 2749, 7B 40 tokens 1542 / 1314, 150 tokens 1886 / 1954 (one), the 405B rank shard 64 tokens 1118 / 1163 (one), 20 tokens 1217 / 1238
+    # (two).  190 tokens of 8B 5493 / 5618, 400 7397 / 7483; from 4096 rows on 2 to 5 % less (4 x 1100 52681 / 51065, 8782 / 8459, 69048 / 68578,
+    # 25597 / 24814), but 4 x 1250 of the 70B shard 77036 / 78132; in between either, by up to 5 %.
     parts_to, parts_from = 160, 4096
+    passes_us, launches_us, short_us = 8.0, 6.0, 50.0
+
+    def _in_parts(self, B: int, S: int) -> bool:
+        rows = B * S
+        if not 4 < rows <= self.parts_to:
+            return rows >= self.parts_from
+        if rows <= _hip.BANDS_TO:
+            return True
+        if (rows, S == 1) not in self._parts_pay:
+            dim, fused, nqkv = self.config.dim, self._fused_width(), GPTBase._fused_width(self)
+            one = _hip.linear_plan_us(rows, fused, dim)
+            two = _hip.linear_plan_us(rows, nqkv, dim) + _hip.linear_plan_us(rows, fused - nqkv, dim, True)
+            launches = self.launches_us if S > 1 and one <= self.short_us else 0.0
+            self._parts_pay[rows, S == 1] = two - one <= self.passes_us + launches
+        return self._parts_pay[rows, S == 1]
 
     def _run_layers_prompt(self, ws: Workspace, pos: Tensor, nqkv: int):
         """Prompts (and decode batches above 64): the rows of the fused input weight as two products, whose output passes rotate and cache, and

@@ -356,6 +356,31 @@ def test_the_plan_takes_no_tiles_that_measured_slower(lib, M, N, K, pair, mib, t
     assert times[(plan.tile_rows, plan.tile_cols, plan.pieces)] <= 1.03 * min(times.values())
 
 
+# (rows of a prompt, of a decode step; us of a measured one and two products beside the rule)
+@pytest.mark.parametrize("name,S,B,two", [
+    ("ladder-8b", 64, 0, True), ("ladder-8b", 150, 0, True), ("ladder-8b", 0, 70, True), ("ladder-8b", 0, 160, True), ("ladder-8b", 190, 0, False),
+    ("ladder-1b", 64, 0, True), ("ladder-1b", 150, 0, True), ("ladder-1b", 0, 70, False), ("ladder-1b", 0, 160, False),
+    ("ladder-70b-tp8", 64, 0, True), ("ladder-70b-tp8", 0, 70, False), ("ladder-70b-tp8", 4100, 0, True),
+    ("llama-3.2-3b", 30, 0, True), ("llama-3.2-3b", 100, 0, False), ("llama-3.2-3b", 150, 0, False), ("llama-3.2-3b", 0, 70, False),
+    ("llama-3.2-3b", 0, 160, False), ("7B", 40, 0, True), ("7B", 150, 0, False), ("70B", 0, 160, True), ("ladder-405b-tp8", 64, 0, False),
+    ("ladder-405b-tp8", 0, 100, False)])
+def test_parallel_blocks_take_the_form_that_measured_faster(lib, name, S, B, two):
+    """And hold memory for the two products' sums only where they run."""
+    model = meta_model("parallel", name)
+    B, S = (B, 1) if B else (1, S)
+    assert model._in_parts(B, S) == two
+    nqkv = (model.config.n_head_local + 2 * model.config.n_kv_local) * model.config.head_dim
+    assert any(N == nqkv for rows, N, K, pair in model._products(B, S) if rows == B * S) == two
+
+
+def test_the_plans_us_are_those_of_its_refusals(lib):
+    from gpt_fast import _hip
+
+    assert _hip.linear_plan_us(64, 4096, 4096) > 0 and _hip.linear_plan_us(64, 28672, 4096, True) > _hip.linear_plan_us(64, 4096, 4096)
+    for bad in ((0, 64, 64), (64, 0, 64), (64, 64, 0), (64, 65, 64, True), (64, 64, 60)):
+        assert _hip.linear_plan_us(*bad) == 0.0
+
+
 def test_a_model_without_bf16_projections_holds_no_memory_for_partial_sums(lib):
     from gpt_fast.quantize import quantize_model_fp8
 

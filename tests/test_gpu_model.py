@@ -1041,6 +1041,45 @@ def test_parallel_prompts_by_one_product_or_two(B, S, semi, monkeypatch):
         assert torch.isfinite(got).all() and (got.double() - want.double()).norm() <= 2.0 ** -6 * want.double().norm()
 
 
+@pytest.mark.parametrize("B,S", [(5, 33), (8, 60), (70, 1), (160, 1), (190, 1)])
+@pytest.mark.parametrize("semi", [False, True])
+@torch.no_grad()
+def test_parallel_blocks_of_many_rows_by_one_product_or_two(B, S, semi, monkeypatch):
+    """The same where the rule takes one product here or takes two from more rows on than a test has: prompts, and decode steps above 64
+    sequences at two positions; replays of the step equal to the eager one."""
+    from gpt_fast import _hip
+
+    model = build("parallel", **dict(TINY, tp_world_size=2, tp_rank=1, semi_compiled_model=semi))
+    model.setup_caches(B, 64)
+    toks = torch.randint(0, 512, (B, 2 * S), device=DEV, generator=torch.Generator(device=DEV).manual_seed(5))
+    passes, rope = [], _hip.rope_kv_write
+    monkeypatch.setattr(_hip, "rope_kv_write", lambda *a: (passes.append(a), rope(*a))[1])
+    results = []
+    for two in (True, False):
+        model._in_parts = lambda B, S: two
+        model.release_workspace()
+        passes.clear()
+        if S == 1:
+            model(toks[:, :1].contiguous(), torch.tensor([0], device=DEV))
+            idx, pos = toks[:, 1:].contiguous(), torch.tensor([1], dtype=torch.int32, device=DEV)
+        else:
+            idx, pos = toks[:, :S].contiguous(), torch.arange(S, dtype=torch.int32, device=DEV)
+        out = model(idx, pos).clone()
+        assert bool(passes) != two
+        graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+            replayed = model(idx, pos)
+        for _ in range(3):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(replayed, out)
+        model.check_device_errors()
+        kv = model.layers[-1].attention.kv_cache
+        results.append((out, kv.k_cache[:, :, :max(S, 2)].clone(), kv.v_cache[:, :, :max(S, 2)].clone()))
+    for got, want in zip(*results):
+        assert torch.isfinite(got).all() and (got.double() - want.double()).norm() <= 2.0 ** -6 * want.double().norm()
+
+
 @pytest.mark.parametrize("family", ["dense", "desync", "parallel"])
 @pytest.mark.parametrize("B", [3, 20])
 @pytest.mark.parametrize("semi", [False, True])
