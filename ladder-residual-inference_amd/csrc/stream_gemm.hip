@@ -157,8 +157,10 @@ extern "C" int lr_linear_residual_tanh(const void* x, int64_t ldx, const void* w
 // 8 rows 1001 / 941, 16 rows 1080 / 1043 (in part by the bands' slices of K, see stream_band).
 namespace {
 
+// (Bands of 32 columns with their inputs through LDS: one workgroup per CU, which is all that a grid of up to 8192 columns has.  Held to the
+// registers of two they kept six in memory: 9 rows of 8192 x 8192 and the 16384 x 8192 behind 74.3 us, now 72.3.)
 template <int UNITS, bool XL, int UROWS>
-__global__ __launch_bounds__(NWV * 64, 2) void k_stream_rms(const Proj p, const int M, const BandResidual rs) {
+__global__ __launch_bounds__(NWV * 64, XL && UNITS == 2 ? 1 : 2) void k_stream_rms(const Proj p, const int M, const BandResidual rs) {
   extern __shared__ __attribute__((aligned(16))) u16 sg_smem[];
   stream_band<16, UNITS, false, XL, false, RESID_RMS, NWV, UROWS, true, !XL>(p, M, blockIdx.x, sg_smem, nullptr, 1, rs);
 }

@@ -36,8 +36,7 @@ class LasivikWorkspace(HybridWorkspace):
                 self._y[key] = torch.zeros(rows, m.y_cols, dtype=dtype, device=device)
         # the parts of the rows' sums of squares behind a mixer and behind a feed-forward, see _run_layers_decode
         self.sq = None
-        if S == 1 and model.norms_in_projections_from <= B <= _hip.ROW_NORM_MAX_ROWS and dtype == torch.bfloat16 and device.type == "cuda" \
-                and model.config.width == model.config.dim:
+        if S == 1 and model.norms_in_projections(B) and dtype == torch.bfloat16 and device.type == "cuda" and model.config.width == model.config.dim:
             n = _hip.linear_residual_rms_sums(model.config.dim)
             self.sq = tuple(e(rows, n, dt=torch.float32) for _ in range(2)) if n else None
 
@@ -78,6 +77,12 @@ class GPTLasivik(GPTHybrid):
     # matrix-vector kernel's otherwise, see project, take 2 us longer in bands and the two norms of a layer 10: 4 % of an 8B step at 1000
     # tokens, 2 % of a 1B one.  One row is the matrix-vector kernel's throughout.)
     norms_in_projections_from = 2
+
+    def norms_in_projections(self, B: int) -> bool:
+        """Rows wider than 6144, two bands' worth of columns per workgroup and more: up to 8 of them (us of an output projection with its norm
+        and the projection behind, norm inside / in a launch of its own: 6144 x 6144 and 12288 x 6144, 16 rows 47.6 / 49.3; 8192 x 8192 and 16384 x
+        8192, 2 rows 68.2 / 71.2, 8 rows 70.4 / 70.5, 9 rows 72.3 / 71.0; 12288 x 4096 and 8192 x 12288, 8 rows 56.0 / 56.6, 16 rows 63.0 / 60.4)."""
+        return self.norms_in_projections_from <= B <= (_hip.ROW_NORM_MAX_ROWS if self.config.dim <= 6144 else 8)
 
     def _run_layers_decode(self, ws, pos):
         """Decode step of up to 16 rows: an output projection updates the residual and leaves the rows with the norm's gain and their

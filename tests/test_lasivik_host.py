@@ -170,6 +170,17 @@ def test_rank_shards_are_refused(monkeypatch):
         args_from_name("lasivik", "lasivik-1b")
 
 
+@pytest.mark.parametrize("dim,B,inside", [(2048, 1, False), (2048, 2, True), (4096, 16, True), (4096, 17, False), (6144, 16, True),
+                                          (8192, 2, True), (8192, 8, True), (8192, 9, False), (12288, 16, False)])
+def test_decode_norms_are_inside_the_projections_where_that_measured_faster(dim, B, inside):
+    from types import SimpleNamespace
+
+    from gpt_fast.gpt_lasivik import GPTLasivik
+
+    model = SimpleNamespace(norms_in_projections_from=GPTLasivik.norms_in_projections_from, config=SimpleNamespace(dim=dim))
+    assert GPTLasivik.norms_in_projections(model, B) == inside
+
+
 def test_weight_only_quantisation_is_refused():
     from gpt_fast import GPTLasivik
     from gpt_fast.quantize import quantize_model_fp8
