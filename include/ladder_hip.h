@@ -700,7 +700,8 @@ int lr_linear_residual_tanh(const void* x, int64_t ldx, const void* w, int M, in
  *     resid [M, N] = scale * X + x w^T (fp32),   x_compute [M, N] = bf16(resid * (gain_offset + gain)),
  *     sums [M, lr_linear_residual_rms_sums(N)] = parts of the new resid's sums of squares:
  * x_compute and sums are an input of lr_linear_multi_normed, resid, sums and gain what the next call takes as resid, `before` and
- * gain_before.  `sums` must not be before->sums, whose dim is N.  lr_linear_residual_rms_sums: 0 where rows of N are not served. */
+ * gain_before.  before->dim is N.  resid, x_compute and sums must overlap neither each other nor x, the gains or before->sums (LR_E_SHAPE): they are
+ * written while those are read.  lr_linear_residual_rms_sums: 0 where rows of N are not served. */
 int lr_linear_residual_rms_sums(int N);
 int lr_linear_residual_rms(const void* x, int64_t ldx, const void* w, int M, int N, int K, float* resid, float scale,
                            const lr_row_norm_t* before, const void* gain_before, const void* gain, float gain_offset,

@@ -157,6 +157,15 @@ extern "C" int lr_linear_residual_tanh(const void* x, int64_t ldx, const void* w
 // 8 rows 1001 / 941, 16 rows 1080 / 1043 (in part by the bands' slices of K, see stream_band).
 namespace {
 
+struct Range {
+  const void* p;
+  size_t bytes;
+  bool meets(const Range& r) const {
+    const uintptr_t a = (uintptr_t)p, b = (uintptr_t)r.p;
+    return r.p != nullptr && a < b + r.bytes && b < a + bytes;
+  }
+};
+
 // (Bands of 32 columns with their inputs through LDS: one workgroup per CU, which is all that a grid of up to 8192 columns has.  Held to the
 // registers of two they kept six in memory: 9 rows of 8192 x 8192 and the 16384 x 8192 behind 74.3 us, now 72.3.)
 template <int UNITS, bool XL, int UROWS>
@@ -193,13 +202,25 @@ extern "C" int lr_linear_residual_rms(const void* x, int64_t ldx, const void* w,
   LR_REQUIRE_PTR(x_compute);
   LR_OPTIONAL_PTR(gain_before);
   if (sums == nullptr || (before && (before->sums == nullptr || gain_before == nullptr))) return LR_E_NULL;
-  if (before && (before->dim != N || before->fold_sums || before->sums == sums)) return LR_E_SHAPE;   // (the sums are read while others are written)
+  if (before && (before->dim != N || before->fold_sums)) return LR_E_SHAPE;
   if (M < 1) return LR_E_SHAPE;
   const lr_projection_t q = {x, ldx, w, x_compute, N, N, K, LR_EPI_NONE, nullptr};
   Proj p{};
   int rc = sb_fill_projection(q, p);
   if (rc != LR_OK) return rc;
-  if (M > LR_ROW_NORM_MAX_ROWS || lr_linear_residual_rms_sums(N) == 0 || (int64_t)M * N * 4 >= 0x7fffffff) return LR_E_UNSUPPORTED;
+  if (M > LR_ROW_NORM_MAX_ROWS || (int64_t)M * N * 4 >= 0x7fffffff) return LR_E_UNSUPPORTED;
+  // Every band reads all of x and of the parts before while others write theirs of the results.
+  const int parts = lr_linear_residual_rms_sums(N);
+  const Range out[3] = {{resid, (size_t)M * N * 4}, {x_compute, (size_t)M * N * 2}, {sums, (size_t)M * (parts ? parts : 1) * 4}};
+  const Range in[4] = {{x, ((size_t)(M - 1) * ldx + K) * 2}, {gain, (size_t)N * 2}, {before ? before->sums : nullptr, before ? (size_t)M * before->count * 4 : 0},
+                       {before ? gain_before : nullptr, (size_t)N * 2}};
+  for (int i = 0; i < 3; ++i) {
+    for (int j = 0; j < i; ++j)
+      if (out[i].meets(out[j])) return LR_E_SHAPE;
+    for (const Range& r : in)
+      if (out[i].meets(r)) return LR_E_SHAPE;
+  }
+  if (parts == 0) return LR_E_UNSUPPORTED;
   if (before) {
     lr_row_norm_t of_input = *before;
     of_input.dim = K;   // (checked against N above: the sums are the residual's)

@@ -618,6 +618,92 @@ def test_two_products_of_one_launch_refuse_what_they_cannot_serve(lib):
     assert lib.lr_linear_pieces_two_bytes(64, 0, 1024, 1024) == 0 == lib.lr_linear_pieces_two_bytes(64, 64, 1028, 1024)
 
 
+def test_linear_residual_rms_refuses_what_it_cannot_serve(lib):
+    """Checked before anything is launched; memory that some bands would write while others read it among it."""
+    from gpt_fast import _hip
+
+    at = {n: (i + 1) << 24 for i, n in enumerate(("x", "w", "resid", "gain_before", "gain", "x_compute", "sums", "parts"))}
+
+    def rc(M=4, N=32768, K=64, ldx=64, before=True, norm={}, **kw):   # (wider than any rows that are served: nothing reaches a launch)
+        p = {**at, **kw}
+        b = _hip._RowNorm(**{**dict(sums=p["parts"], count=32, dim=N, eps=1e-5), **norm})
+        return lib.lr_linear_residual_rms(p["x"], ldx, p["w"], M, N, K, p["resid"], 1.0, ctypes.byref(b) if before else None, p["gain_before"], p["gain"],
+                                          1.0, p["x_compute"], p["sums"], None)
+
+    for name in ("x", "w", "resid", "gain_before", "gain", "x_compute", "sums", "parts"):
+        assert rc(**{name: None}) == -1, name
+    for name in ("x", "w", "resid", "gain_before", "gain", "x_compute"):
+        assert rc(**{name: at[name] + 8}) == -2, name
+    assert rc(M=0) == -3 and rc(N=0) == -3 and rc(K=0) == -3 and rc(K=60) == -2 and rc(ldx=56) == -3 and rc(M=17) == -4
+    assert rc(norm=dict(dim=64)) == -3 and rc(norm=dict(fold_sums=256)) == -3
+    ranges = dict(x=(3 * 64 + 64) * 2, resid=4 * 32768 * 4, x_compute=4 * 32768 * 2, sums=16, gain=65536, gain_before=65536, parts=4 * 32 * 4)
+    for out in ("resid", "x_compute", "sums"):
+        for other in ranges:
+            if other != out:
+                assert rc(**{out: at[other]}) == -3, (out, other)                              # the same place
+                assert rc(**{out: at[other] + ranges[other] - 16}) == -3, (out, other)         # its last 16 bytes
+                assert rc(**{other: at[out] + ranges[out] - 16}) == -3, (out, other)
+                assert rc(**{out: at[other] - ranges[out]}) == -4, (out, other)                # next to it
+    assert rc(before=False, sums=at["parts"], gain_before=None) == -4
+
+
+def test_products_on_e4m3_weights_refuse_what_they_cannot_serve(lib):
+    """Checked before anything is launched; shapes of the passes of 16 rows are declined."""
+    from gpt_fast import _hip
+
+    heads = dict(n_head=4, n_kv_head=2, head_dim=64, smax=64, block_size=64)
+
+    def one(x=256, ldx=128, w=256, scales=256, y=256, ldy=512, M=17, N=512, K=128, sums=256, size=0, rope=None):
+        r = None if rope is None else ctypes.byref(_hip._RopeKv(**{**dict(table=256, pos=256, k_cache=256, v_cache=256), **heads, **rope}))
+        return lib.lr_linear_fp8_product(x, ldx, w, scales, y, ldy, M, N, K, r, sums, size, None)
+
+    for name in ("x", "w", "scales", "y"):
+        assert one(**{name: None}) == -1, name
+    for name in ("x", "w", "y", "sums"):
+        assert one(**{name: 264}) == -2, name
+    assert one(M=0) == -3 and one(N=0) == -3 and one(K=0) == -3 and one(ldx=120) == -3 and one(ldy=504) == -3 and one(K=120) == -2 and one(ldx=132) == -2
+    assert one(M=16) == -4 and one(M=65) == -4 and one(K=64) == -4 and one(K=192, ldx=192) == -4
+    for name in ("table", "pos", "k_cache", "v_cache"):
+        assert one(rope={name: None}) == -1, name
+    for name in heads:
+        assert one(rope={name: 0}) == -3, name
+    assert one(rope=dict(n_head=5)) == -3
+
+    n0, n1 = ctypes.c_int32(), ctypes.c_int32()
+
+    def two(x0=256, w0=256, s0=256, K0=1024, sums0=1 << 30, n0=ctypes.byref(n0), x1=256, w1=256, s1=256, K1=1024, sums1=2 << 30, n1=ctypes.byref(n1),
+            M=64, N=64, size=1 << 20):
+        return lib.lr_linear_fp8_pieces_two(x0, w0, s0, K0, sums0, n0, x1, w1, s1, K1, sums1, n1, M, N, size, None)
+
+    for name in ("x0", "w0", "s0", "sums0", "n0", "x1", "w1", "s1", "sums1", "n1"):
+        assert two(**{name: None}) == -1, name
+    for name in ("x0", "w0", "sums0", "x1", "w1", "sums1"):
+        assert two(**{name: 264}) == -2, name
+    for name in ("M", "N", "K0", "K1"):
+        assert two(**{name: 0}) == -3, name
+    assert two(K0=1032) == -2 and two(sums1=1 << 30) == -3 and two(sums1=(1 << 30) + (1 << 20) - 256) == -3
+    assert two(M=16) == -4 and two(M=65) == -4 and two(N=66) == -4 and two(K0=1040) == -4 and two(size=0) == -4
+    assert lib.lr_linear_fp8_pieces_two_bytes(16, 64, 1024, 1024) == 0 == lib.lr_linear_fp8_pieces_two_bytes(64, 66, 1024, 1024)
+    assert lib.lr_linear_fp8_product_bytes(16, 512, 128, 0) == 0 == lib.lr_linear_fp8_product_bytes(64, 511, 128, 1)
+
+    def beside(scales=256, x=256, w=256, act=256, M=17, N=512, K=128, ldx=128, ldact=256, sums=256, q=256, Hq=8):
+        return lib.lr_attn_decode_beside_product_fp8(q, 1024, 256, 256, 256, 256, 1024, 32, Hq, 1, 128, 64, 256, 1 << 24, 256, x, ldx, w, scales, act, ldact, M,
+                                                     N, K, sums, 1 << 20, None)
+
+    for name in ("scales", "x", "w", "act", "q"):
+        assert beside(**{name: None}) == -1, name
+    assert beside(x=264) == -2 and beside(sums=264) == -2 and beside(N=511) == -3 and beside(ldx=120) == -3 and beside(ldact=248) == -3 and beside(Hq=0) == -3
+    assert beside(M=16) == -4 and beside(M=65) == -4 and beside(K=64) == -4
+
+
+def test_add_rmsnorm_of_partial_sums_refuses_what_it_cannot_serve(lib):
+    def rc(resid=256, d1=256, pieces=2, d2=None, gain=256, out=256, normed=256, rows=4, dim=64):
+        return lib.lr_add_rmsnorm_pieces(resid, d1, pieces, d2, gain, out, normed, rows, dim, 1e-5, None)
+
+    assert rc(d1=None) == -1 and rc(resid=None) == -1 and rc(gain=None) == -1 and rc(normed=None) == -1 and rc(pieces=-1) == -3
+    assert rc(d1=264) == -2 and rc(d2=264) == -2 and rc(dim=60) == -2 and rc(rows=0) == -3 and rc(dim=32768) == -4
+
+
 @pytest.mark.parametrize("entry", ["beside_merged", "beside_fp8_merged", "beside_product"])
 def test_attention_in_a_shared_launch_refuses_what_its_own_launch_refuses(lib, entry):
     """lr_attn_decode's arguments and the tickets; what is not for these grids is declined."""
