@@ -240,8 +240,8 @@ def test_ladder_decode_of_different_sequences_equals_each_alone(B, fp8):
 @pytest.mark.parametrize("B,fp8", [(17, False), (32, False), (33, False), (64, False), (17, True), (40, True), (64, True)])
 @torch.no_grad()
 def test_ladder_decode_of_many_different_sequences_equals_each_alone(B, fp8, monkeypatch):
-    """17 to 64 rows, the attention beside the up/gate product and wo beside w2, or e4m3 bands of up to 16 rows at a time: another
-    sequence in every row, each row's logits those of the sequence decoded alone, replays equal to eager steps."""
+    """17 to 64 rows, the attention beside the up/gate product and wo beside w2, on either weights: another sequence in every row, each row's
+    logits those of the sequence decoded alone, replays equal to eager steps."""
     from gpt_fast import _hip
     from gpt_fast.quantize import quantize_model_fp8
 
@@ -249,13 +249,24 @@ def test_ladder_decode_of_many_different_sequences_equals_each_alone(B, fp8, mon
     if fp8:
         quantize_model_fp8(model)
     model.setup_caches(B, 16)
-    beside, launches = _hip.attn_decode_beside_product, []
-    monkeypatch.setattr(_hip, "attn_decode_beside_product", lambda *a: (launches.append(beside(*a)), launches[-1])[1])
+    taken = {}
+
+    def spy(name):
+        call, taken[name] = getattr(_hip, name), []
+        monkeypatch.setattr(_hip, name, lambda *a: (taken[name].append(call(*a)), taken[name][-1])[1])
+
+    for name in ("attn_decode_beside_product", "linear_pieces_two", "attn_decode_beside_product_fp8", "linear_fp8_pieces_two", "linear_fp8_product",
+                 "linear_fp8_multi"):
+        spy(name)
     toks = torch.randint(0, 512, (B, 6), device=DEV, generator=torch.Generator(device=DEV).manual_seed(9))
     pos = torch.zeros(1, dtype=torch.int32, device=DEV)
     decode = lambda rows: torch.cat([model(rows[:, t:t + 1].contiguous(), torch.tensor([t], device=DEV)).clone() for t in range(6)], 1)
     together = decode(toks)
-    assert fp8 or (launches and all(launches))
+    n = len(model.layers)      # (the last block leaves no partial sums, and on e4m3 weights the head is a product, too)
+    count = {name: len(calls) for name, calls in taken.items() if all(calls)}
+    assert count == {"attn_decode_beside_product": 0 if fp8 else 6 * n, "linear_pieces_two": 0 if fp8 else 6 * (n - 1),
+                     "attn_decode_beside_product_fp8": 6 * n if fp8 else 0, "linear_fp8_pieces_two": 6 * (n - 1) if fp8 else 0,
+                     "linear_fp8_product": 6 * (n + 3) if fp8 else 0, "linear_fp8_multi": 0}
     for b in range(0, B, 5):
         assert rel_err(together[b], decode(toks[b:b + 1])[0]) <= REL_TOL, b
     decode(toks)
@@ -290,6 +301,49 @@ def test_ladder_decode_where_no_shared_grid_serves_equals_each_alone(B, chains, 
     decode = lambda rows: torch.cat([model(rows[:, t:t + 1].contiguous(), torch.tensor([t], device=DEV)).clone() for t in range(6)], 1)
     together = decode(toks)
     assert len(launches) == (6 if why == "declined" else 0) and hasattr(model, "_chain_stream") == chains
+    for b in range(0, B, 5):
+        assert rel_err(together[b], decode(toks[b:b + 1])[0]) <= REL_TOL, b
+    decode(toks)
+    idx = toks[:, 5:].contiguous()
+    pos.fill_(5)
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+        out = model(idx, pos)
+    for _ in range(4):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[:, 0], together[:, 5])
+
+
+@pytest.mark.parametrize("why", ["declined", "tickets", "pieces", "width"])
+@pytest.mark.parametrize("B", [17, 40, 64])
+@torch.no_grad()
+def test_ladder_decode_on_e4m3_weights_where_no_products_serve_equals_each_alone(B, why, monkeypatch):
+    """The library declines the shared grid, there are no tickets, or a width is no multiple of 128: passes of up to 16 rows; it declines the two
+    output products of one launch: one after the other."""
+    from gpt_fast import _hip
+    from gpt_fast.quantize import quantize_model_fp8
+
+    model = build("ladder", **dict(WIDER, dim=1024, intermediate_size=8256 if why == "width" else 8192))
+    quantize_model_fp8(model)
+    model.setup_caches(B, 16)
+    beside, passes, multi, one, products = [], [], _hip.linear_fp8_multi, _hip.linear_fp8_product, []
+    monkeypatch.setattr(_hip, "linear_fp8_multi", lambda *a: (passes.append(a), multi(*a))[1])
+    monkeypatch.setattr(_hip, "linear_fp8_product", lambda *a: (products.append(one(*a)), products[-1])[1])
+    if why == "declined":
+        monkeypatch.setattr(_hip, "attn_decode_beside_product_fp8", lambda *a: bool(beside.append(a)))
+    if why == "pieces":
+        monkeypatch.setattr(_hip, "linear_fp8_pieces_two", lambda *a: beside.append(a))
+    if why == "tickets":
+        model._workspace(B, 1).tickets = None
+    toks = torch.randint(0, 512, (B, 6), device=DEV, generator=torch.Generator(device=DEV).manual_seed(9))
+    pos = torch.zeros(1, dtype=torch.int32, device=DEV)
+    decode = lambda rows: torch.cat([model(rows[:, t:t + 1].contiguous(), torch.tensor([t], device=DEV)).clone() for t in range(6)], 1)
+    together = decode(toks)
+    n, parts = len(model.layers), -(-B // 16)
+    assert len(beside) == {"declined": 6, "pieces": 6 * (n - 1)}.get(why, 0)
+    assert len(passes) == (0 if why == "pieces" else 6 * n * 2 * parts) and all(products)
+    assert len(products) == 6 * {"declined": 2, "tickets": 1, "pieces": 3 * n + 1, "width": 0}[why]     # (the head's among them)
     for b in range(0, B, 5):
         assert rel_err(together[b], decode(toks[b:b + 1])[0]) <= REL_TOL, b
     decode(toks)
