@@ -264,25 +264,30 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
 #pragma unroll
     for (int mt = 0; mt < MTILES; ++mt) acc[u][mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-  // Which chunk of K is the wave's ci-th: bf16 bands are read in a slice of K per wave, one chunk behind the other.  (The waves'
-  // chunks in turn, g = ci KW + wave, as it was and as e4m3 bands and the two matrices of RN still are: a wave then skips three
-  // chunks of every row.  us, 8 rows, in turn / in slices: 128256 x 4096 194 / 157, 16384 x 2048 15.9 / 14.7, 6144 x 4096 12.4 / 11.7,
-  // 4096 x 14336 22.2 / 20.9; of RN, 8192 x (1024 | 3584) 18.4 / 19.6.)
-  // All workgroups walk K from the same end, over rows that lie a multiple of 4 KiB apart: the four waves' places should differ
-  // there too, or all of the grid asks for the same 1 KiB in four of the DRAM's interleaving.  Slices of whole 4 KiB (K 8192) begin
-  // at four different quarters and wrap around: 7168 x 8192 22.4 in turn, 26.3 in slices, 21.2 so, 16032 x 8192 54.7 / 51.5 / 42.7.
+  // Which chunk of K is the wave's ci-th: the waves' chunks in turn, g = ci KW + wave, or a slice of K per wave, one chunk behind the
+  // other.  All workgroups walk K from the same end: over rows that lie a multiple of 4 KiB apart the four waves' 1 KiB in turn are the same
+  // quarter of the DRAM's interleaving all over the grid, and places a slice apart are not.  Slices of whole 4 KiB begin at four
+  // different quarters and wrap around (8192 columns: 20.7 us for 7168 rows, 24.8 without).  us, 8 input rows, in turn / in slices, one library:
+  // 128256 x 2048 92.2 / 84.8, 16384 x 2048 15.3 / 14.1, 128256 x 4096 199 / 156, 6144 x 4096 11.7 / 11.0, 8192 x 8192 31.1 / 23.8, 16032 x 8192 55.9 /
+  // 42.2, 4096 x 14336 21.4 / 20.3, 8192 x 20480 55.2 / 51.4.
+  // In turn: other distances, which spread the rows by themselves (8192 x 22016 62.6 / 73.6, 18432 x 2304 19.5 / 20.6, 5120 x 12800 25.2 /
+  // 26.8, 20000 x 4352 31.5 / 32.6, 40 others 0.95 to 1.03, but 4096 x 11008 19.4 / 18.0), and multiples of 32 KiB (13312 x 16384 69.6 / 76.7, 2304 x
+  // 16384 15.6 / 16.8, 2048 x 32768 29.7 / 30.5; 8192 x 32768 96.2 / 88.5).  The two matrices of RN, where a wave that wraps around would mix them
+  // (8192 x (1024 | 3584) 18.4 / 19.6 without), and e4m3, where a row's chunk is half as long, are left in turn (e4m3, 5 input rows: 1280 x 8192 6.33 /
+  // 6.40, 28672 x 4096 22.9 / 22.5, 6144 x 4096 7.86 / 7.82, 16 rows 9.73 / 10.11; but 16032 x 8192 28.5 / 22.9, 128256 x 4096 92.3 / 82.2).
   // What lies beyond K or the wave's last chunk reads as zero (no branch around a load: the number of loads in flight is fixed, so
   // the waits between chunks are exact).  The order of a sum is a matter of K alone, not of how the rows are cut into bands.
   const int nck = nck1 + (RN ? (rn.K2 + KCW - 1) / KCW : 0);
   constexpr bool SLICES = !RN && !W8;
-  const int kper = (nck + KW - 1) / KW, kfirst = SLICES ? kwave * kper : kwave;
-  const int nch = kfirst >= nck ? 0 : SLICES ? (nck - kfirst < kper ? nck - kfirst : kper) : (nck - kfirst + KW - 1) / KW;  // chunks of this wave
+  const bool slices = SLICES && K % 2048 == 0 && K % 16384 != 0;
+  const int kper = (nck + KW - 1) / KW, kfirst = slices ? kwave * kper : kwave, kstep = slices ? 1 : KW;
+  const int nch = kfirst >= nck ? 0 : slices ? (nck - kfirst < kper ? nck - kfirst : kper) : (nck - kfirst + KW - 1) / KW;  // chunks of this wave
   constexpr int CHUNKS_4K = 4096 / (KCW * WB), QUARTER = CHUNKS_4K / 4;
-  const int kturn = SLICES && kper % CHUNKS_4K == 0 && nch == kper ? kwave * QUARTER % CHUNKS_4K : 0;
+  const int kturn = slices && kper % CHUNKS_4K == 0 ? kwave * QUARTER % CHUNKS_4K : 0;   // (K % 2048: all slices are as long)
   auto chunk_at = [&](int ci) {
     if (!SLICES) return ci * KW + kfirst;
     const int c = ci + kturn;
-    return ci < nch ? kfirst + (c < nch ? c : c - nch) : nck;
+    return ci < nch ? kfirst + (c < nch ? c : c - nch) * kstep : nck;
   };
   auto issue_w = [&](int ci, u32x4_t (&dst)[NLD]) {
     if constexpr (RN) {

@@ -638,9 +638,10 @@ def test_bands_of_few_rows_equal_the_bands_of_many(hip, M, N, K):
 
 
 @pytest.mark.parametrize("M", [3, 24, 60])
-@pytest.mark.parametrize("K", [8, 120, 136, 520, 8064, 8072, 8192, 8200, 16384, 16512])
+@pytest.mark.parametrize("K", [8, 120, 136, 520, 2040, 2048, 2056, 6144, 8064, 8072, 8192, 8200, 10240, 16384, 16512, 18432, 24576])
 def test_bands_in_slices_of_k(hip, M, K):
-    """Each wave's slice of K: fewer chunks than waves, a last wave with fewer or none, slices of whole 4 KiB (which wrap around)."""
+    """The waves' chunks in turn: fewer of them than waves, a last wave with fewer; a slice of K each where rows lie 4 KiB apart (2048 to 6144, 10240
+    and 18432), slices of whole 4 KiB, which wrap around (8192, 24576), and multiples of 32 KiB, in turn again."""
     x, w = rnd(M, K, seed=94), rnd(40, K, seed=95, scale=0.02)
     y = torch.empty(M, 40, dtype=BF, device=DEV)
     hip.linear_multi((x, w, y, hip.EPI_NONE))
