@@ -171,13 +171,17 @@ __global__ __launch_bounds__(256) void k_gemm(const u16* __restrict__ x, int64_t
 // weights' way from HBM, and a CU has at most some 48 KiB of requests on their way whoever waits for them, so a ring of two, of
 // which a k-tile and a half are, asks for too little; four are no faster (7168 x 8192, 64 rows, four pieces: two 31.0 us, three 27.4,
 // four 27.6).  And all workgroups walk K from the same end, over rows that lie a multiple of 4 KiB apart: at any time they ask for
-// one place of the DRAM's interleaving.  With a long ring column tile nt begins at k-tile GEMM_TURN * nt and goes round (a stream of
-// such operands without products, 128 rows, 7168 x 8192: ring of two 33.3 us, turned 30.9, ring of four 27.2, turned 23.3).  Not with
-// several row tiles, which share the rows and the weights in L2 while they go in step.  us before / now: 64 rows, 28672 x 4096 (pairs)
-// 47.5 / 39.9, 6144 x 4096 31.4 / 30.1 without pieces; 128 rows, 16032 x 8192 66.5 / 56.7, 28672 x 4096 (pairs) 54.7 / 50.6, 7168 x
-// 8192 (pairs) 36.0 / 32.3.
+// one place of the DRAM's interleaving.  With a long ring column tile nt begins where the fraction of nt times the golden ratio lies in K
+// and goes round, so that any run of column tiles is spread evenly over K (a stream of such operands without products, 128 rows, 7168 x
+// 8192: ring of two 33.3 us, turned 30.9, ring of four 27.2, turned 23.3).  Steps of so and so many k-tiles meet the interleaving's own
+// period at some K: 48 rows, 16384 x 6656 ring of two 42.6 us, steps of five 46.2, now 41.9; 8192 x 22016 75.3, 76.2, 63.9; of 84 products
+// of 48 and 112 rows steps of five take 0.934 of the ring of two's time, of three 0.929, now 0.925, at worst 1.086, 1.060, 1.019.  Not
+// with several row tiles, which share the rows and the weights in L2 while they go in step.  us, ring of two / now: 48 rows, 28672 x 4096
+// (pairs) 48.8 / 37.4, 16384 x 11008 78.2 / 62.1, 16032 x 8192 56.6 / 50.6; 112 rows, 28672 x 4096 (pairs) 55.5 / 47.7, 24576 x 8192
+// 105.7 / 85.7, 10240 x 8192 45.2 / 42.8.
 // ---------------------------------------------------------------------------------------------
-constexpr int GEMM_RING = 3, GEMM_TURN = 5;
+constexpr int GEMM_RING = 3;
+constexpr unsigned GEMM_TURN = 2654435761u;   // 2^32 / golden ratio, the prime next to it
 struct GemmRope {   // the projection is the fused q/k/v projection of a prefill: see lr_linear_rope_kv
   const u16* table;
   const int32_t* pos;
@@ -451,7 +455,7 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
   const int64_t xlast = GROUP ? gp.xrows - 1 : (M - m0 < T::TM ? M - m0 : T::TM) - 1;
   const int64_t wlast = MODE == GEMM_PAIR ? N + (int64_t)(N - n0 < T::TN / 2 ? N - n0 : T::TN / 2) - 1 : (N - n0 < T::TN ? N - n0 : T::TN) - 1;
   const int xbytes = (int)((xlast * ldx + klen) * 2), wbytes = (int)((wlast * K + klen) * WB);   // (below 2 GiB: gemm_reaches)
-  const int turn = LONG ? (int)((unsigned)(nt * GEMM_TURN) % (unsigned)nk) : 0;   // the k-tile that is multiplied first
+  const int turn = LONG ? (int)__umulhi((unsigned)nt * GEMM_TURN, (unsigned)nk) : 0;   // the k-tile that is multiplied first
   auto request = [&](auto ONCE, const u16* base, int bytes, int voff, int t, int per, int part, u32 lds) {   // (per: bytes of a row in a k-tile)
     const bool in = t < nk;
     if (LONG) t = t + turn < nk ? t + turn : t + turn - nk;

@@ -648,7 +648,7 @@ def test_bands_in_slices_of_k(hip, M, K):
     assert_close_ulp(y, linear_ref(x, w), what=f"slices M={M} K={K}")
 
 
-@pytest.mark.parametrize("M,N,K", [(33, 200, 64), (64, 136, 128), (40, 1030, 192), (64, 2000, 832), (48, 264, 8192), (64, 4096, 4160),
+@pytest.mark.parametrize("M,N,K", [(33, 200, 64), (64, 136, 128), (40, 1030, 192), (64, 2000, 832), (48, 264, 8192), (64, 4096, 4160), (48, 8200, 6656),
                                    (65, 200, 4096), (96, 264, 8192), (128, 1030, 8192), (127, 4104, 2112), (129, 200, 4160)])
 @pytest.mark.parametrize("memory", [0, 8 << 20])
 def test_products_in_long_rings(hip, M, N, K, memory):
