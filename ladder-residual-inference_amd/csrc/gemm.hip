@@ -821,9 +821,12 @@ constexpr GemmTileCost GEMM_TILES[GEMM_NTILES] = {{8, 2, 1, 16, 1.2f, 0.0f, 0.0f
                                                   {5, 2, 1, 16, 0.668f, 0.2935f, 0.581f, 0.0f, 0.0f, 3.12f, 5.41f},
                                                   {5, 1, 2, 8, 0.553f, 0.0159f, 0.173f, 1.103f, 4.77f, 3.88f, 0.0077f},
                                                   {6, 1, 1, 16, 0.617f, 0.0f, 0.0944f, 0.0f, 0.0f, 4.28f, 0.0f},
-                                                  {4, 1, 1, 16, 0.407f, 0.0508f, 0.206f, 0.0f, 0.0f, 5.0f, 0.101f}};
+                                                  {4, 1, 1, 16, 0.56f, 0.0508f, 0.08f, 0.0f, 0.0f, 5.0f, 0.101f}};
 // The long rings' costs are fitted to 25 weights of the model families: 17 to 64 rows (92 products; what the plan takes is 0.6 % above the
-// best of the pieces, 6 % at worst; with the ring of two's costs 1.7 and 17 %) and, beside 64 x 128 and 128 x 128, 65 to 128 (66; 0.7 and 6 %).
+// best of the pieces, 6 % at worst; with the ring of two's costs 1.7 and 17 %).  128 x 128's of 65 to 128 rows are fitted to 201 products of
+// 72 weights, each against the best of the other tiles, of whose time they take 0.961 on average and 1.05 at worst: with CUs to spare it is
+// the slower one (8192 x 15360, 112 rows: 192 workgroups 66.9 us, 256 of the ring of two 56.3), which costs that fell with them did not see
+// (0.974 and 1.19).  Lost by it: 13312 x 16384 (pairs), 66 rows, 115 us in 128 x 256, would be 88.
 constexpr GemmTileCost GEMM_FEW_COST = {2, 1, 2, 16, 0.353f, 0.201f, 0.281f, 0.737f, 1.19f, 3.17f, 0.0f};
 constexpr GemmTileCost GEMM_FEW8_COST = {2, 1, 2, 16, 0.547f, 0.201f, 0.242f, 0.8f, 1.405f, 1.78f, 0.0f};   // (64 products of 17 weights: 0.7 % above the best pieces)
 static const GemmTileCost& gemm_cost(int tile, int M) { return tile == GEMM_ROWS64 && M <= 64 ? GEMM_FEW_COST : GEMM_TILES[tile]; }
