@@ -240,8 +240,41 @@ def test_ladder_decode_of_different_sequences_equals_each_alone(B, fp8):
 @pytest.mark.parametrize("B,fp8", [(17, False), (32, False), (33, False), (64, False), (17, True), (40, True), (64, True)])
 @torch.no_grad()
 def test_ladder_decode_of_many_different_sequences_equals_each_alone(B, fp8, monkeypatch):
-    """17 to 64 rows, the attention beside the up/gate product and wo beside w2, on either weights: another sequence in every row, each row's
-    logits those of the sequence decoded alone, replays equal to eager steps."""
+    """17 to 64 rows, the attention beside the up/gate product and wo beside w2, or e4m3 bands of up to 16 rows at a time: another
+    sequence in every row, each row's logits those of the sequence decoded alone, replays equal to eager steps."""
+    from gpt_fast import _hip
+    from gpt_fast.quantize import quantize_model_fp8
+
+    model = build("ladder", **dict(WIDER, dim=1024, intermediate_size=8192))
+    if fp8:
+        quantize_model_fp8(model)
+    model.setup_caches(B, 16)
+    beside, launches = _hip.attn_decode_beside_product, []
+    monkeypatch.setattr(_hip, "attn_decode_beside_product", lambda *a: (launches.append(beside(*a)), launches[-1])[1])
+    toks = torch.randint(0, 512, (B, 6), device=DEV, generator=torch.Generator(device=DEV).manual_seed(9))
+    pos = torch.zeros(1, dtype=torch.int32, device=DEV)
+    decode = lambda rows: torch.cat([model(rows[:, t:t + 1].contiguous(), torch.tensor([t], device=DEV)).clone() for t in range(6)], 1)
+    together = decode(toks)
+    assert fp8 or (launches and all(launches))
+    for b in range(0, B, 5):
+        assert rel_err(together[b], decode(toks[b:b + 1])[0]) <= REL_TOL, b
+    decode(toks)
+    idx = toks[:, 5:].contiguous()
+    pos.fill_(5)
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+        out = model(idx, pos)
+    for _ in range(4):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[:, 0], together[:, 5])
+
+
+@pytest.mark.parametrize("B,fp8", [(17, False), (64, False), (17, True), (40, True), (64, True)])
+@torch.no_grad()
+def test_ladder_decode_of_17_to_64_rows_runs_the_products(B, fp8, monkeypatch):
+    """On either weights every block's attention beside its up/gate product and every two output products but the last block's in one launch, with
+    none declined; e4m3 weights in no pass of 16 rows."""
     from gpt_fast import _hip
     from gpt_fast.quantize import quantize_model_fp8
 
@@ -258,27 +291,15 @@ def test_ladder_decode_of_many_different_sequences_equals_each_alone(B, fp8, mon
     for name in ("attn_decode_beside_product", "linear_pieces_two", "attn_decode_beside_product_fp8", "linear_fp8_pieces_two", "linear_fp8_product",
                  "linear_fp8_multi"):
         spy(name)
-    toks = torch.randint(0, 512, (B, 6), device=DEV, generator=torch.Generator(device=DEV).manual_seed(9))
-    pos = torch.zeros(1, dtype=torch.int32, device=DEV)
-    decode = lambda rows: torch.cat([model(rows[:, t:t + 1].contiguous(), torch.tensor([t], device=DEV)).clone() for t in range(6)], 1)
-    together = decode(toks)
+    for t in range(2):
+        model(torch.full((B, 1), 7, dtype=torch.int64, device=DEV), torch.tensor([t], device=DEV))
+    model.check_device_errors()
     n = len(model.layers)      # (the last block leaves no partial sums, and on e4m3 weights the head is a product, too)
-    count = {name: len(calls) for name, calls in taken.items() if all(calls)}
-    assert count == {"attn_decode_beside_product": 0 if fp8 else 6 * n, "linear_pieces_two": 0 if fp8 else 6 * (n - 1),
-                     "attn_decode_beside_product_fp8": 6 * n if fp8 else 0, "linear_fp8_pieces_two": 6 * (n - 1) if fp8 else 0,
-                     "linear_fp8_product": 6 * (n + 3) if fp8 else 0, "linear_fp8_multi": 0}
-    for b in range(0, B, 5):
-        assert rel_err(together[b], decode(toks[b:b + 1])[0]) <= REL_TOL, b
-    decode(toks)
-    idx = toks[:, 5:].contiguous()
-    pos.fill_(5)
-    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
-    with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
-        out = model(idx, pos)
-    for _ in range(4):
-        graph.replay()
-        torch.cuda.synchronize()
-        assert torch.equal(out[:, 0], together[:, 5])
+    assert all(all(calls) for calls in taken.values())
+    assert {name: len(calls) for name, calls in taken.items()} == {
+        "attn_decode_beside_product": 0 if fp8 else 2 * n, "linear_pieces_two": 0 if fp8 else 2 * (n - 1),
+        "attn_decode_beside_product_fp8": 2 * n if fp8 else 0, "linear_fp8_pieces_two": 2 * (n - 1) if fp8 else 0,
+        "linear_fp8_product": 2 * (n + 3) if fp8 else 0, "linear_fp8_multi": 0}
 
 
 @pytest.mark.parametrize("why", ["declined", "tickets"])
@@ -928,10 +949,7 @@ def test_tokens_on_conditioned_weights(name, B, T):
     oracle differs from the SAME oracle run in fp32 by ~1e-1 of the largest logit, and two bf16
     implementations that differ in one rounding decorrelate to that level.  So the yardstick is
     the fp32 run, and what is asserted is
-      * the HIP logits are no farther from the fp32 logits than the eager bf16 reference is: on average over steps and rows (x 1.5), and in
-        the worst of them (x 2.5).  Six prompts to the 70B shard in two orders of the same sums gave 0.89 to 1.19 of the reference's average
-        and 0.8 to 1.9 times its worst step, six to the 8B model 0.90 to 1.25 and 0.7 to 1.6, the averages over the prompts 0.97 to 1.02: one
-        step's distance is a draw of last bits, the average over 48 is one five times as narrow;
+      * the HIP logits are no farther from the fp32 logits than the eager bf16 reference is (x 1.5);
       * at every step where the reference's choice is robust to its own bf16 error -- its margin
         over the runner-up exceeds twice its distance to the fp32 logits -- the HIP token is
         IDENTICAL, with no tie exemption; such steps must be the majority and their tokens must
@@ -955,9 +973,7 @@ def test_tokens_on_conditioned_weights(name, B, T):
     _, exact_logits = O.generate(ocfg, P32, prompt, new, 1, "ladder", forced=ref_tok[:1])
     del P32
     exact_logits = exact_logits.expand(new, B, -1)
-    each = lambda logits, i: [rel_err(got, want) for got, want in zip(logits.view(B, -1), exact_logits[i])]   # (a row's)
-    average = lambda e: float(sum(e)) / len(e)
-    oracle_errs = [err for i in range(new) for err in each(ref_logits[i], i)]
+    oracle_err = max(rel_err(ref_logits[i], exact_logits[i]) for i in range(new))
     top2 = ref_logits.float().topk(2, dim=-1).values                            # [new, B, 2]
     noise = (ref_logits.float() - exact_logits.float()).abs().amax(-1)          # [new, B]
     robust = ((top2[..., 0] - top2[..., 1]) > 2 * noise).T                      # [B, new]
@@ -969,21 +985,21 @@ def test_tokens_on_conditioned_weights(name, B, T):
 
     rows = prompt.view(1, -1).repeat(B, 1)
     logits = model(rows, torch.arange(T, device=DEV))
-    errs = each(logits[:, -1], 0)
+    errs = [rel_err(logits[:, -1], exact_logits[0])]
     forced = [model.greedy_next(logits).clone()]
     pos = torch.tensor([T], dtype=torch.int32, device=DEV)
     for i in range(new - 1):
         logits = model(ref_tok[:, i:i + 1].contiguous(), pos)
-        errs += each(logits[:, -1], i + 1)
+        errs.append(rel_err(logits[:, -1], exact_logits[i + 1]))
         forced.append(model.greedy_next(logits).clone())
         pos += 1
     forced = torch.cat(forced, dim=1)
     same = forced == ref_tok
     line = (f"conditioned weights {name} B={B}: tokens identical at {float(same.float().mean()):.4f} of all steps, at "
-            f"{float(same[robust].float().mean()):.4f} of the robust ones; distance to the fp32 logits: HIP {average(errs):.3e}, at worst "
-            f"{max(errs):.3e}, eager bf16 oracle {average(oracle_errs):.3e}, {max(oracle_errs):.3e}")
+            f"{float(same[robust].float().mean()):.4f} of the robust ones; distance to the fp32 logits: HIP {max(errs):.3e}, "
+            f"eager bf16 oracle {oracle_err:.3e}")
     progress(line)
-    assert average(errs) <= 1.5 * average(oracle_errs) and max(errs) <= 2.5 * max(oracle_errs)
+    assert max(errs) <= 1.5 * oracle_err
     assert bool(same[robust].all())
 
     empty = torch.empty(B, T + new, dtype=torch.int64, device=DEV)
@@ -1000,6 +1016,30 @@ def test_tokens_on_conditioned_weights(name, B, T):
     torch.cuda.synchronize()
     model.check_device_errors()
     assert torch.equal(dg.history[:, : new - 1], free[:, 1:])
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("name,B,T", [("ladder-70b-tp8", 1, 2048), ("ladder-8b", 16, 1024)])
+def test_average_distance_to_fp32_on_conditioned_weights(name, B, T):
+    """What the worst of 48 steps' distances above is a draw of: last bits move it by a factor of two, their average by a few per cent (six prompts
+    to the 70B shard in two orders of the same sums: 0.89 to 1.19 of the eager bf16 reference's average, to the 8B model 0.90 to 1.25)."""
+    new = 48
+    model = build("ladder", **shape_kw(name))
+    init_conditioned(model, seed=0)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(CONDITIONED_PROMPT_SEED)
+    prompt = torch.randint(0, model.config.vocab_size, (T,), device=DEV, generator=g)
+    P, ocfg = dict(model.state_dict()), oracle_cfg(model.config)
+    tokens, reference = O.generate(ocfg, P, prompt, new, 1, "ladder")
+    exact = O.generate(ocfg, {k: v.float() for k, v in P.items()}, prompt, new, 1, "ladder", forced=tokens)[1]
+    model.setup_caches(B, T + new)
+    logits = [model(prompt.view(1, -1).repeat(B, 1), torch.arange(T, device=DEV))[:, -1].clone()]
+    for i in range(new - 1):
+        logits.append(model(tokens[:, i:i + 1].expand(B, 1).contiguous(), torch.tensor([T + i], dtype=torch.int32, device=DEV))[:, -1].clone())
+    ours = sum(rel_err(row, exact[i, 0]) for i in range(new) for row in logits[i]) / (new * B)
+    theirs = sum(rel_err(reference[i, 0], exact[i, 0]) for i in range(new)) / new
+    progress(f"conditioned weights {name} B={B}: average distance to the fp32 logits: HIP {ours:.3e}, eager bf16 oracle {theirs:.3e}")
+    assert ours <= 1.5 * theirs
 
 
 # ---------------------------------------------------------------------------------------------------

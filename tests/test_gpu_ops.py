@@ -638,17 +638,23 @@ def test_bands_of_few_rows_equal_the_bands_of_many(hip, M, N, K):
 
 
 @pytest.mark.parametrize("M", [3, 24, 60])
-@pytest.mark.parametrize("K", [8, 120, 136, 520, 2040, 2048, 2056, 6144, 8064, 8072, 8192, 8200, 10240, 16384, 16512, 18432, 24576])
+@pytest.mark.parametrize("K", [8, 120, 136, 520, 8064, 8072, 8192, 8200, 16384, 16512])
 def test_bands_in_slices_of_k(hip, M, K):
-    """The waves' chunks in turn: fewer of them than waves, a last wave with fewer; a slice of K each where rows lie 4 KiB apart (2048 to 6144, 10240
-    and 18432), slices of whole 4 KiB, which wrap around (8192, 24576), and multiples of 32 KiB, in turn again."""
+    """Each wave's slice of K: fewer chunks than waves, a last wave with fewer or none, slices of whole 4 KiB (which wrap around)."""
     x, w = rnd(M, K, seed=94), rnd(40, K, seed=95, scale=0.02)
     y = torch.empty(M, 40, dtype=BF, device=DEV)
     hip.linear_multi((x, w, y, hip.EPI_NONE))
     assert_close_ulp(y, linear_ref(x, w), what=f"slices M={M} K={K}")
 
 
-@pytest.mark.parametrize("M,N,K", [(33, 200, 64), (64, 136, 128), (40, 1030, 192), (64, 2000, 832), (48, 264, 8192), (64, 4096, 4160), (48, 8200, 6656),
+@pytest.mark.parametrize("M", [3, 24, 60])
+@pytest.mark.parametrize("K", [2040, 2048, 2056, 6144, 10240, 18432, 24576])
+def test_bands_in_slices_of_k_where_rows_lie_4_kib_apart(hip, M, K):
+    """A slice of K per wave at multiples of 2048, wrapping around where it is whole 4 KiB (24576); the chunks in turn beside them."""
+    test_bands_in_slices_of_k(hip, M, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 200, 64), (64, 136, 128), (40, 1030, 192), (64, 2000, 832), (48, 264, 8192), (64, 4096, 4160),
                                    (65, 200, 4096), (96, 264, 8192), (128, 1030, 8192), (127, 4104, 2112), (129, 200, 4160)])
 @pytest.mark.parametrize("memory", [0, 8 << 20])
 def test_products_in_long_rings(hip, M, N, K, memory):
@@ -660,6 +666,12 @@ def test_products_in_long_rings(hip, M, N, K, memory):
     hip.linear(x, w, y[:, :N], scratch=scratch)
     assert_close_ulp(y[:, :N].contiguous(), linear_ref(x, w), what=f"long ring M={M} N={N} K={K}")
     assert bool((y[:, N:] == 3.0).all())
+
+
+@pytest.mark.parametrize("memory", [0, 8 << 20])
+def test_products_in_long_rings_of_many_column_tiles(hip, memory):
+    """More column tiles than k-tiles: several of them begin at the same one."""
+    test_products_in_long_rings(hip, 48, 8200, 6656, memory)
 
 
 @pytest.mark.parametrize("rows,dim", [(2, 4096), (2, 4104), (257, 8192), (3, 8200), (1, 16376)])
@@ -1212,11 +1224,7 @@ def test_attn_prefill(hip, B, S, Hq, Hkv, hd, Smax, start):
 @pytest.mark.parametrize("B,S,Hq,Hkv,hd,start", [
     (1, 16, 4, 1, 128, 0), (2, 33, 8, 2, 128, 31), (1, 128, 6, 3, 128, 64), (1, 129, 32, 8, 128, 0), (3, 161, 2, 2, 128, 95), (1, 511, 8, 2, 128, 1),
     (1, 512, 8, 1, 128, 0), (1, 545, 6, 3, 128, 63), (2, 600, 2, 2, 128, 200), (8, 520, 32, 8, 128, 0), (5, 610, 28, 7, 128, 17),
-    (1, 17, 4, 1, 64, 0), (1, 130, 6, 3, 64, 33), (1, 512, 32, 8, 64, 0), (1, 577, 2, 2, 64, 64), (8, 530, 32, 8, 64, 3),
-    # the last portion: one key, 32 and 33 of them, alone and behind others, where it is computed as half of one and where it is not
-    (1, 16, 4, 1, 128, 17), (2, 32, 8, 2, 128, 0), (1, 32, 4, 1, 128, 64), (1, 65, 8, 2, 128, 0), (3, 97, 8, 8, 128, 0), (1, 96, 6, 3, 128, 0),
-    (1, 33, 6, 3, 128, 64), (1, 97, 4, 2, 128, 63), (2, 32, 8, 2, 64, 0), (1, 33, 4, 1, 64, 0), (1, 65, 6, 3, 64, 0), (3, 96, 2, 2, 64, 0),
-    (1, 128, 4, 1, 64, 1), (1, 129, 4, 1, 64, 0), (1, 129, 4, 4, 64, 31)])
+    (1, 17, 4, 1, 64, 0), (1, 130, 6, 3, 64, 33), (1, 512, 32, 8, 64, 0), (1, 577, 2, 2, 64, 64), (8, 530, 32, 8, 64, 3)])
 def test_attn_prefill_portions_of_keys(hip, B, S, Hq, Hkv, hd, start):
     """Nothing beyond the last position is used, whatever lies there."""
     n = start + S
@@ -1228,6 +1236,15 @@ def test_attn_prefill_portions_of_keys(hip, B, S, Hq, Hkv, hd, start):
     mask = torch.arange(n, device=DEV).view(1, n) <= pos.view(S, 1)
     want = O.sdpa_math(q.view(B, S, Hq, hd).transpose(1, 2), kc[:, :, :n].contiguous(), vc[:, :, :n].contiguous(), mask)
     assert_close_ulp(y, want.transpose(1, 2).reshape(B, S, Hq * hd), max_frac=0.03, what="attn_prefill, portions")
+
+
+# (one key, 32 and 33 of them, alone and behind others, where they are computed as half a portion and where they are not)
+@pytest.mark.parametrize("B,S,Hq,Hkv,hd,start", [
+    (1, 16, 4, 1, 128, 17), (2, 32, 8, 2, 128, 0), (1, 32, 4, 1, 128, 64), (1, 65, 8, 2, 128, 0), (3, 97, 8, 8, 128, 0), (1, 96, 6, 3, 128, 0),
+    (1, 33, 6, 3, 128, 64), (1, 97, 4, 2, 128, 63), (2, 32, 8, 2, 64, 0), (1, 33, 4, 1, 64, 0), (1, 65, 6, 3, 64, 0), (3, 96, 2, 2, 64, 0),
+    (1, 128, 4, 1, 64, 1), (1, 129, 4, 1, 64, 0), (1, 129, 4, 4, 64, 31)])
+def test_attn_prefill_last_portion_of_keys(hip, B, S, Hq, Hkv, hd, start):
+    test_attn_prefill_portions_of_keys(hip, B, S, Hq, Hkv, hd, start)
 
 
 @pytest.mark.parametrize("qscale", [4.0, 12.0])
