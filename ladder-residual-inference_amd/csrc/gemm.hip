@@ -171,17 +171,17 @@ __global__ __launch_bounds__(256) void k_gemm(const u16* __restrict__ x, int64_t
 // weights' way from HBM, and a CU has at most some 48 KiB of requests on their way whoever waits for them, so a ring of two, of
 // which a k-tile and a half are, asks for too little; four are no faster (7168 x 8192, 64 rows, four pieces: two 31.0 us, three 27.4,
 // four 27.6).  And all workgroups walk K from the same end, over rows that lie a multiple of 4 KiB apart: at any time they ask for
-// one place of the DRAM's interleaving.  With a long ring column tile nt begins where the fraction of nt times the golden ratio lies in K
-// and goes round, so that any run of column tiles is spread evenly over K (a stream of such operands without products, 128 rows, 7168 x
-// 8192: ring of two 33.3 us, turned 30.9, ring of four 27.2, turned 23.3).  Steps of so and so many k-tiles meet the interleaving's own
-// period at some K: 48 rows, 16384 x 6656 ring of two 42.6 us, steps of five 46.2, now 41.9; 8192 x 22016 75.3, 76.2, 63.9; of 84 products
-// of 48 and 112 rows steps of five take 0.934 of the ring of two's time, of three 0.929, now 0.925, at worst 1.086, 1.060, 1.019.  Not
-// with several row tiles, which share the rows and the weights in L2 while they go in step.  us, ring of two / now: 48 rows, 28672 x 4096
-// (pairs) 48.8 / 37.4, 16384 x 11008 78.2 / 62.1, 16032 x 8192 56.6 / 50.6; 112 rows, 28672 x 4096 (pairs) 55.5 / 47.7, 24576 x 8192
-// 105.7 / 85.7, 10240 x 8192 45.2 / 42.8.
+// one place of the DRAM's interleaving.  With a long ring column tile nt begins at k-tile GEMM_TURN * nt and goes round (a stream of such
+// operands without products, 128 rows, 7168 x 8192: ring of two 33.3 us, turned 30.9, ring of four 27.2, turned 23.3).  Not with several row
+// tiles, which share the rows and the weights in L2 while they go in step.  us, ring of two / now: 48 rows, 28672 x 4096 (pairs) 48.8 / 39.9,
+// 16384 x 11008 78.2 / 64.9, 16032 x 8192 56.6 / 48.9; 112 rows, 28672 x 4096 (pairs) 55.5 / 52.5, 10240 x 8192 45.2 / 43.9.
+// Steps of so and so many k-tiles meet the interleaving's own period where rows are an odd multiple of 1 KiB: there, from 4096 columns on, a tile
+// begins where the fraction of nt times the golden ratio lies in K (48 rows, steps of five / so: 16384 x 6656 47.1 / 42.2, ring of two 42.6; 6656 x
+// 6656 24.6 / 23.8, 8192 x 22016 81.0 / 70.6; 5120 x 13824 32.6 / 32.7, 6656 x 17920 49.7 / 50.5).  Of 81 products of other
+// widths, 48 and 112 rows, it takes 0.94 to 1.04 of the steps' time, as long on average, and 26624 x 16384 (pairs), 112 rows, 204 us for 170.
 // ---------------------------------------------------------------------------------------------
-constexpr int GEMM_RING = 3;
-constexpr unsigned GEMM_TURN = 2654435761u;   // 2^32 / golden ratio, the prime next to it
+constexpr int GEMM_RING = 3, GEMM_TURN = 5;
+constexpr unsigned GEMM_TURN_GOLDEN = 2654435761u;   // 2^32 / golden ratio, the prime next to it
 struct GemmRope {   // the projection is the fused q/k/v projection of a prefill: see lr_linear_rope_kv
   const u16* table;
   const int32_t* pos;
@@ -455,7 +455,9 @@ __device__ __forceinline__ void gemm_tile(const int block, const int blocks, con
   const int64_t xlast = GROUP ? gp.xrows - 1 : (M - m0 < T::TM ? M - m0 : T::TM) - 1;
   const int64_t wlast = MODE == GEMM_PAIR ? N + (int64_t)(N - n0 < T::TN / 2 ? N - n0 : T::TN / 2) - 1 : (N - n0 < T::TN ? N - n0 : T::TN) - 1;
   const int xbytes = (int)((xlast * ldx + klen) * 2), wbytes = (int)((wlast * K + klen) * WB);   // (below 2 GiB: gemm_reaches)
-  const int turn = LONG ? (int)__umulhi((unsigned)nt * GEMM_TURN, (unsigned)nk) : 0;   // the k-tile that is multiplied first
+  // the k-tile that is multiplied first
+  const bool golden = !W8 && K % 1024 == 512 && K >= 4096;
+  const int turn = !LONG ? 0 : golden ? (int)__umulhi((unsigned)nt * GEMM_TURN_GOLDEN, (unsigned)nk) : (int)((unsigned)(nt * GEMM_TURN) % (unsigned)nk);
   auto request = [&](auto ONCE, const u16* base, int bytes, int voff, int t, int per, int part, u32 lds) {   // (per: bytes of a row in a k-tile)
     const bool in = t < nk;
     if (LONG) t = t + turn < nk ? t + turn : t + turn - nk;
@@ -824,12 +826,18 @@ constexpr GemmTileCost GEMM_TILES[GEMM_NTILES] = {{8, 2, 1, 16, 1.2f, 0.0f, 0.0f
                                                   {4, 1, 1, 16, 0.56f, 0.0508f, 0.08f, 0.0f, 0.0f, 5.0f, 0.101f}};
 // The long rings' costs are fitted to 25 weights of the model families: 17 to 64 rows (92 products; what the plan takes is 0.6 % above the
 // best of the pieces, 6 % at worst; with the ring of two's costs 1.7 and 17 %).  128 x 128's of 65 to 128 rows are fitted to 201 products of
-// 72 weights, each against the best of the other tiles, of whose time they take 0.961 on average and 1.05 at worst: with CUs to spare it is
-// the slower one (8192 x 15360, 112 rows: 192 workgroups 66.9 us, 256 of the ring of two 56.3), which costs that fell with them did not see
-// (0.974 and 1.19).  Lost by it: 13312 x 16384 (pairs), 66 rows, 115 us in 128 x 256, would be 88.
+// 72 weights, each against the best of the other tiles: with CUs to spare it is the slower one (8192 x 15360, 112 rows: 192 workgroups 66.6 us, 256 of
+// the ring of two 56.9; 20480 x 5120 (pairs) 62.5 / 54.1, 6144 x 17920 64.3 / 56.0), which costs that fell with them did not see.
 constexpr GemmTileCost GEMM_FEW_COST = {2, 1, 2, 16, 0.353f, 0.201f, 0.281f, 0.737f, 1.19f, 3.17f, 0.0f};
 constexpr GemmTileCost GEMM_FEW8_COST = {2, 1, 2, 16, 0.547f, 0.201f, 0.242f, 0.8f, 1.405f, 1.78f, 0.0f};   // (64 products of 17 weights: 0.7 % above the best pieces)
-static const GemmTileCost& gemm_cost(int tile, int M) { return tile == GEMM_ROWS64 && M <= 64 ? GEMM_FEW_COST : GEMM_TILES[tile]; }
+// The same over rows a power of two apart, where all row distances meet the same channels and the tiles that do not turn are the slower ones (us, they /
+// this one: 13312 x 16384 (pairs) 66 rows 115 / 90, 112 rows 117 / 98, 12288 x 4096 66 rows 29.4 / 27.5): fitted to 66 products beside 64 x 128
+// and 128 x 128, 0.7 % above the best, 6 % at worst.
+constexpr GemmTileCost GEMM_LONG_COST = {4, 1, 1, 16, 0.407f, 0.0508f, 0.206f, 0.0f, 0.0f, 5.0f, 0.101f};
+static const GemmTileCost& gemm_cost(int tile, int M, int K) {
+  if (tile == GEMM_LONG && (K & (K - 1)) == 0) return GEMM_LONG_COST;
+  return tile == GEMM_ROWS64 && M <= 64 ? GEMM_FEW_COST : GEMM_TILES[tile];
+}
 // whether a tile serves the product
 static bool gemm_takes(int tile, int M, int K) {
   if (tile < GEMM_TILES_ANY) return true;
@@ -899,7 +907,7 @@ static GemmPlan gemm_plan(int M, int N, int K, int mode, size_t scratch) {
   if (M > 0x7fffffff - 256 || N > 0x7fffffff - 256 || K > 0x7fffffff - 256) return best;   // (row, column and k of the last tile are ints)
   const float bytes_us = gemm_bytes_us(M, N, K, mode);
   for (int c = 0; c < GEMM_NTILES; ++c)
-    if (gemm_takes(c, M, K)) gemm_consider(gemm_cost(c, M), c, M, N, (K + 63) / 64, mode, bytes_us, scratch, best);
+    if (gemm_takes(c, M, K)) gemm_consider(gemm_cost(c, M, K), c, M, N, (K + 63) / 64, mode, bytes_us, scratch, best);
   return best;
 }
 // The same for e4m3 weights (K % 128 == 0): tiles of 64 x 128, k-tiles of 128.
@@ -1009,7 +1017,7 @@ int gemm_inputs(const void* x0, const void* wqkv, void* qkv, int S, const lr_rop
   int best = -1;
   for (int c = 0; c < GEMM_NTILES; ++c) {
     if (!gemm_shares(c, M, K)) continue;
-    const GemmTileCost& t = gemm_cost(c, M);
+    const GemmTileCost& t = gemm_cost(c, M, K);
     const int TM = 32 * t.a, slots = cus * t.per_cu;
     const int64_t tm = (M - 1) / TM + 1, tiles0 = tm * ((N - 1) / (128 * t.bh) + 1), tiles1 = tm * ((I - 1) / (64 * t.bh) + 1), tiles = tiles0 + tiles1;
     // (of several rounds only the last one leaves room, and q/k/v goes cold before the attention reads it: 8 x 2048 tokens of
@@ -1097,7 +1105,7 @@ static GemmOutputs outputs_plan(int M, int N, int K0, int K1, size_t sums_bytes)
   const int cus = gemm_cus(), pairs0 = (K0 / KT + 1) / 2, pairs1 = (K1 / KT + 1) / 2;
   const size_t row = (size_t)M * N * sizeof(float);
   for (int c = W8 ? GEMM_ROWS64 : 0; c < GEMM_TILES_ANY; ++c) {
-    const GemmTileCost& t = W8 ? GEMM_FEW8_COST : gemm_cost(c, M);
+    const GemmTileCost& t = W8 ? GEMM_FEW8_COST : gemm_cost(c, M, K0);
     const int TM = 32 * t.a, TN = 128 * t.bh, slots = cus * t.per_cu;
     const int64_t tiles = (int64_t)((M + TM - 1) / TM) * ((N + TN - 1) / TN);
     for (int s0 = 1; s0 <= 16 && 2 * s0 <= pairs0 + 1 && row * s0 <= sums_bytes; ++s0)
