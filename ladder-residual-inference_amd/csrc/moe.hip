@@ -478,7 +478,7 @@ extern "C" int lr_moe(const lr_moe_t* d, lr_stream_t stream) {
       return LR_E_UNSUPPORTED;
     const bool by_slot = d->rows == 1;
     Proj p = {};
-    p.x = (const u16*)d->x; p.ldx = d->ldx; p.w = (const u16*)d->w1; p.y = (u16*)act; p.ldy = I; p.N = 2 * I; p.K = D; p.pair_off = I;
+    p.x = (const u16*)d->x; p.ldx = d->ldx; p.w = (const u16*)d->w1; p.y = (u16*)act; p.ldy = I; p.N = 2 * I; p.K = D; p.pair_off = I; p.in_turn = band_in_turn(D);
     const int64_t busy = n < d->E ? n : d->E;      // experts, at most
     p.rpw = 16;
     p.nwg = (I + 15) / 16;
@@ -486,7 +486,7 @@ extern "C" int lr_moe(const lr_moe_t* d, lr_stream_t stream) {
     rc = launch_band<2>(p, (int64_t)2 * I * D, d->experts, n, d->E, by_slot, d->top, s, sh);
     if (rc != LR_OK) return rc;
     Proj o = {};
-    o.x = (const u16*)act; o.ldx = I; o.w = (const u16*)d->w2; o.y = (u16*)d->out; o.ldy = D; o.N = D; o.K = I;
+    o.x = (const u16*)act; o.ldx = I; o.w = (const u16*)d->w2; o.y = (u16*)d->out; o.ldy = D; o.N = D; o.K = I; o.in_turn = band_in_turn(I);
     const int64_t w2 = (int64_t)I * D;
     if (I <= 1024 && busy * ((D + 127) / 128) >= 256) {
       o.rpw = 32; o.nwg = (D + 127) / 128;

@@ -47,6 +47,7 @@ struct Proj {
   int rpw;       // rows (row pairs if pair_off) per workgroup
   int pair_off;  // 0, or the distance from an up row to its gate row (= outputs)
   int nwg;       // workgroups of this projection
+  int in_turn;   // how a band's four waves share K, see band_in_turn
   const u16* scales;  // weight-only e4m3 weights (the W8 kernels): one bf16 scale per weight row; else nullptr
   // RoPE + KV-cache epilogue of a fused q/k/v projection (rope_table == nullptr: none)
   const u16* rope_table;
@@ -64,6 +65,9 @@ struct Proj {
   float* fold_total;
   int fold_count;
 };
+// log2 of the distance between a wave's chunks of K in a bf16 band of four waves: 0 a slice each, 2 in turn.  A matter of K alone, measured: see
+// stream_band
+inline int band_in_turn(int K) { return (K % 2048 == 0 ? K % 16384 == 0 : K > 1024 && (K <= 3072 || (K >= 12288 && K % 1024 != 0))) ? 2 : 0; }
 __host__ __device__ constexpr int norm_pitch(int count) { return (count + 255) & ~255; }   // LDS row of parts: whole requests
 
 // What a layer's output projections leave for the next layer's input projections instead of their sums (stream_band, RN):
@@ -270,24 +274,28 @@ __device__ __forceinline__ void stream_band(const Proj& p, const int M, const in
   // different quarters and wrap around (8192 columns: 20.7 us for 7168 rows, 24.8 without).  us, 8 input rows, in turn / in slices, one library:
   // 128256 x 2048 92.2 / 84.8, 16384 x 2048 15.3 / 14.1, 128256 x 4096 199 / 156, 6144 x 4096 11.7 / 11.0, 8192 x 8192 31.1 / 23.8, 16032 x 8192 55.9 /
   // 42.2, 4096 x 14336 21.4 / 20.3, 8192 x 20480 55.2 / 51.4.
-  // In turn: other distances, which spread the rows by themselves (8192 x 22016 62.6 / 73.6, 18432 x 2304 19.5 / 20.6, 5120 x 12800 25.2 /
-  // 26.8, 20000 x 4352 31.5 / 32.6, 40 others 0.95 to 1.03, but 4096 x 11008 19.4 / 18.0), and multiples of 32 KiB (13312 x 16384 69.6 / 76.7, 2304 x
-  // 16384 15.6 / 16.8, 2048 x 32768 29.7 / 30.5; 8192 x 32768 96.2 / 88.5).  The two matrices of RN, where a wave that wraps around would mix them
-  // (8192 x (1024 | 3584) 18.4 / 19.6 without), and e4m3, where a row's chunk is half as long, are left in turn (e4m3, 5 input rows: 1280 x 8192 6.33 /
-  // 6.40, 28672 x 4096 22.9 / 22.5, 6144 x 4096 7.86 / 7.82, 16 rows 9.73 / 10.11; but 16032 x 8192 28.5 / 22.9, 128256 x 4096 92.3 / 82.2).
+  // Other widths gain less by slices or lose by them, and are in turn where they measured slower so (2048 to 16384 rows, 8 to 32 input rows, time in
+  // slices over that in turn): 1024 0.92 to 1.01; 1536 to 3072 1.02 to 1.11; 3584 to 9216 0.95 to 1.04, as long on average; 11008 0.93 to 0.97;
+  // 12800 1.01 to 1.06; 15360 0.97 to 1.01; 22016 1.08 to 1.20 (8192 rows, 8 input rows, 80.9 / 68.0 us); but 17920 0.95 to 1.00.  In turn, too:
+  // multiples of 32 KiB (13312 x 16384 76.7 / 69.6, 2304 x 16384 16.8 / 15.6, 2048 x 32768 30.5 / 29.7; 8192 x 32768 88.5 / 96.2), the two
+  // matrices of RN, where a wave that wraps around would mix them (8192 x (1024 | 3584) 19.6 / 18.4 without), and e4m3, where a row's chunk is half
+  // as long (5 input rows: 1280 x 8192 6.40 / 6.33, 28672 x 4096 22.5 / 22.9, 6144 x 4096 7.82 / 7.86, 16 rows 10.11 / 9.73; but 16032 x 8192 22.9 /
+  // 28.5, 128256 x 4096 82.2 / 92.3).
   // What lies beyond K or the wave's last chunk reads as zero (no branch around a load: the number of loads in flight is fixed, so
   // the waits between chunks are exact).  The order of a sum is a matter of K alone, not of how the rows are cut into bands.
   const int nck = nck1 + (RN ? (rn.K2 + KCW - 1) / KCW : 0);
   constexpr bool SLICES = !RN && !W8;
-  const bool slices = SLICES && K % 2048 == 0 && K % 16384 != 0;
-  const int kper = (nck + KW - 1) / KW, kfirst = slices ? kwave * kper : kwave, kstep = slices ? 1 : KW;
-  const int nch = kfirst >= nck ? 0 : slices ? (nck - kfirst < kper ? nck - kfirst : kper) : (nck - kfirst + KW - 1) / KW;  // chunks of this wave
+  // (selects and shifts: a branch here is 0.1 us of a launch, 4 to 8 % of the smallest)
+  static_assert(KW == 1 || KW == 4 || (KW == 8 && !SLICES), "");
+  const int turn = !SLICES ? (KW == 8 ? 3 : KW == 4 ? 2 : 0) : KW == 1 ? 0 : p.in_turn;   // log2 of the distance between a wave's chunks
+  const int kper = (nck + KW - 1) / KW, kfirst = kwave * (turn ? 1 : kper), kend = min(nck, turn ? nck : kfirst + kper);
+  const int nch = max(kend - kfirst + (1 << turn) - 1, 0) >> turn;  // chunks of this wave
   constexpr int CHUNKS_4K = 4096 / (KCW * WB), QUARTER = CHUNKS_4K / 4;
-  const int kturn = slices && kper % CHUNKS_4K == 0 ? kwave * QUARTER % CHUNKS_4K : 0;   // (K % 2048: all slices are as long)
+  const int kturn = SLICES ? (kwave * QUARTER % CHUNKS_4K) & -(int)((turn == 0) & (kper % CHUNKS_4K == 0) & (nch == kper)) : 0;
   auto chunk_at = [&](int ci) {
     if (!SLICES) return ci * KW + kfirst;
-    const int c = ci + kturn;
-    return ci < nch ? kfirst + (c < nch ? c : c - nch) * kstep : nck;
+    const int c = ci + kturn, g = kfirst + ((c - (c < nch ? 0 : nch)) << turn);
+    return ci < nch ? g : nck;
   };
   auto issue_w = [&](int ci, u32x4_t (&dst)[NLD]) {
     if constexpr (RN) {
@@ -781,6 +789,7 @@ static int sb_fill_projection(const lr_projection_t& q, Proj& p) {
   p = Proj{};
   p.x = (const u16*)q.x; p.w = (const u16*)q.w; p.y = (u16*)q.y;
   p.ldx = q.ldx; p.ldy = q.ldy; p.N = q.N; p.K = q.K;
+  p.in_turn = band_in_turn(q.K);
   p.pair_off = pair ? q.N / 2 : 0;
   if (q.epilogue == LR_EPI_ROPE_KV) {
     const lr_rope_kv_t* r = q.rope;

@@ -11,10 +11,10 @@
 //
 // A workgroup (4 waves, one per SIMD, so each has the whole register budget) owns a band of up to
 // 32 weight rows -- the number of rows is chosen so that every CU gets the same share -- and its
-// waves walk K in 128-element chunks, in turn or, where rows lie a multiple of 4 KiB apart, a slice of K
-// each (stream_band).  Each wave keeps 4 chunks of weights (32 KiB) in flight in registers, 128 KiB per CU.
-// The input rows come from L2 straight into B-fragment layout.  The waves' partial sums meet in LDS and are
-// added in a fixed order.
+// waves walk K in 128-element chunks, in turn or, where that measured faster, a slice of K each
+// (stream_band).  Each wave keeps 4 chunks of weights (32 KiB) in flight in registers, 128 KiB per CU.
+// The input rows come from L2 straight into B-fragment layout.  The waves' partial sums meet in LDS and
+// are added in a fixed order.
 //
 // Two projections that read the same layer input can share one launch (the band index selects the
 // projection), and a projection whose weight holds [up; gate] rows can take the band as row PAIRS

@@ -648,9 +648,9 @@ def test_bands_in_slices_of_k(hip, M, K):
 
 
 @pytest.mark.parametrize("M", [3, 24, 60])
-@pytest.mark.parametrize("K", [2040, 2048, 2056, 6144, 10240, 18432, 24576])
-def test_bands_in_slices_of_k_where_rows_lie_4_kib_apart(hip, M, K):
-    """A slice of K per wave at multiples of 2048, wrapping around where it is whole 4 KiB (24576); the chunks in turn beside them."""
+@pytest.mark.parametrize("K", [1024, 1032, 1536, 2048, 2056, 3072, 3080, 5120, 6144, 10240, 11008, 12280, 12296, 13312, 18432, 22016, 24576])
+def test_bands_in_slices_of_k_and_in_turn(hip, M, K):
+    """Widths on both sides of each line between the two; slices of whole 4 KiB (24576), which wrap around."""
     test_bands_in_slices_of_k(hip, M, K)
 
 
