@@ -275,18 +275,23 @@ struct WindowKeys {
 // 128, 8 x 2048 tokens 401 / 397, 4 x 777 44.2 / 41.8, 4 x 1024 62.5 / 63.1, 4 x 1300 93.0 / 96.5; 2 x 1500 of window 128 27.2 / 25.0),
 // and for the 33 to 96 queries of two heads to a workgroup, whose first 32 have no use for the second 32 keys (28 heads, 14 kv heads, 64 tokens
 // 7.5 / 6.9).
-// HALF: a last portion of up to 32 keys is computed as such.  Short prompts are one (us without / with: 32 heads, 8 kv heads of 64, 32 tokens 5.31 /
-// 4.73, 100 tokens 6.29 / 5.78; of 128, 16 tokens 6.28 / 5.71, 32 tokens 7.02 / 6.49), and narrow windows have few others (1500 tokens, window of 128
-// 11.1 / 10.1).  Heads of 64: up to 128 keys, the loop is slower beside a second copy of its body (32 tokens at position 3000 47.5 / 51.0).
+// PREFILL_EACH: a portion's 32-key tiles one after the other, with a reference point each: up to 128 queries of heads of 128, which have KEYS 32's
+// results so, and a barrier per 64 keys (KEYS 32 / so: 32 heads, 8 kv heads, 64 tokens 7.28 / 7.07, 100 8.21 / 8.17, 128 9.21 / 8.74, 4 x 32 tokens
+// at position 3000 102 / 92.  Both tiles at a time would be 7.66, 8.37 and 74 us at 100, 128 and 4 x 32, in other last bits: a whole model's outputs,
+// 80 layers later, are 1 to 2 % of their norm apart by that, no nearer to 64 bits).
+// PREFILL_HALF: a last portion of up to 32 keys is computed as such (us without / with: 32 heads, 8 kv heads of 64, 32 tokens 5.32 / 4.64, 100 tokens
+// 6.42 / 5.70; of 128, 300 tokens 12.9 / 12.1), and narrow windows have few others (1500 tokens, window of 128 11.1 / 10.1).  Heads of 64: up to 128
+// keys, the loop is slower beside a second copy of its body (32 tokens at position 3000 47.5 / 51.0).
 // Heads of 64 keep to the 128 registers that let four workgroups share a CU (40 heads, 20 kv heads, 3000 tokens, window of 128: three to a CU
 // 22.6 us, four 19.0).
 // Bound: matrix instructions 48 % of a SIMD's cycles, vector instructions 46 % (exponentials at a quarter of the rate, splitting P), which hardly
 // run at the same time, in another wave or between the matrix instructions of the same one (written so, it took as long).  No bank
 // conflicts.  Before (32 keys in one LDS buffer through registers, V transposed on its way in, two barriers) / now, us: 32 heads of 128,
-// 8 kv heads: 8 x 2048 tokens 460 / 396 (598 / 694 TFLOP/s of products), 4 x 1300 112 / 96, 2 x 1000 50.8 / 35.9, 777 28.4 / 22.4, 300 14.0 / 12.3,
-// 100 8.2 / 8.0, 32 6.3 / 6.5, 16 5.6 / 5.7; of 64: 4 x 1024 59.9 / 40.1, 512 15.1 / 11.8, 100 6.3 / 5.8, 32 4.8 / 4.7.
+// 8 kv heads: 8 x 2048 tokens 460 / 396 (598 / 694 TFLOP/s of products), 4 x 1300 112 / 96, 2 x 1000 50.8 / 35.9, 777 28.4 / 22.4, 300 14.0 / 12.1,
+// 100 8.2 / 8.2, 32 6.3 / 6.4, 16 5.6 / 5.7; of 64: 4 x 1024 59.9 / 40.1, 512 15.1 / 11.8, 100 6.3 / 5.8, 32 4.8 / 4.7.
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
 constexpr int PREFILL_PARTS_FROM = 512, PREFILL_HALF_TO = 128;   // keys that are seen, see above
+enum { PREFILL_WHOLE, PREFILL_HALF, PREFILL_EACH };
 template <int HD, int KSP, int KEYS>
 struct PrefillLds {
   static constexpr int TILE = KEYS * HD * 2, STAGE = 2 * TILE;   // a portion's keys or values; both
@@ -302,7 +307,7 @@ __device__ __forceinline__ int value_swizzle(int key) { return HD == 128 ? (key 
 
 // WIN (lr_window_attention): a sliding window, the score scale as an argument, and the kv heads' keys and values side by
 // side as rows of a matrix, in the order lr_latent_window gives them; head sizes up to HD.
-template <int HD, int NWH, int KSP, int KEYS, bool HALF, bool WIN>
+template <int HD, int NWH, int KSP, int KEYS, int HALF, bool WIN>
 __global__ __launch_bounds__(256 * KSP, HD == 64 ? 4 : KEYS == 32 ? 3 : 2) void k_attn_prefill_mfma(const u16* __restrict__ q, int64_t ldq,
                                                                     const u16* __restrict__ kc, const u16* __restrict__ vc,
                                                                     const int32_t* __restrict__ pos, u16* __restrict__ y,
@@ -448,12 +453,12 @@ __global__ __launch_bounds__(256 * KSP, HD == 64 ? 4 : KEYS == 32 ? 3 : 2) void 
   }
   if (t_first < nkeys) stage(t_first, 0);
   int buf = 0;
-  // N 32-key tiles of the portion at t0, for this wave's queries
-  auto tiles = [&](auto N_, const int t0, const int buf) {
+  // N 32-key tiles of the portion at t0, from its tile `first` on, for this wave's queries
+  auto tiles = [&](auto N_, const int t0, const int buf, const int first) {
     constexpr int N = decltype(N_)::value;
-    const int tk = t0 + part * 32;
+    const int tk = t0 + (part + first) * 32;
     if (tk > pmax || (WIN && tk + 32 * N - 1 <= pmin - w.window)) return;   // nothing here for them
-    const unsigned char* const at = prefill_lds + buf * L::STAGE;
+    const unsigned char* const at = prefill_lds + buf * L::STAGE + first * 32 * RB;
     // ---- S^T tiles: rows = keys, columns = queries
     f32x16_t sacc[N];
 #pragma unroll
@@ -542,16 +547,21 @@ __global__ __launch_bounds__(256 * KSP, HD == 64 ? 4 : KEYS == 32 ? 3 : 2) void 
   };
   // (that portion has arrived, for all waves, and nobody reads the one before any more)
   auto arrived = [] { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-  constexpr int LAST = HALF ? 32 : 0;
+  constexpr int LAST = HALF == PREFILL_HALF ? 32 : 0;
   int t0 = t_first;
   for (; t0 + LAST < nkeys; t0 += KEYS, buf ^= 1) {
     arrived();
     if (t0 + KEYS < nkeys) stage(t0 + KEYS, buf ^ 1);
-    tiles(std::integral_constant<int, NS>{}, t0, buf);
+    if constexpr (HALF == PREFILL_EACH) {
+#pragma unroll 1
+      for (int first = 0; first < NS && t0 + 32 * first < nkeys; ++first) tiles(std::integral_constant<int, 1>{}, t0, buf, first);
+    } else {
+      tiles(std::integral_constant<int, NS>{}, t0, buf, 0);
+    }
   }
-  if (HALF && t0 < nkeys) {   // at most 32 keys are left
+  if (HALF == PREFILL_HALF && t0 < nkeys) {   // at most 32 keys are left
     arrived();
-    tiles(std::integral_constant<int, 1>{}, t0, buf);
+    tiles(std::integral_constant<int, 1>{}, t0, buf, 0);
   }
   if constexpr (KSP == 2) {
     // the second four waves' results to the first four, which saw the other keys of the same queries
@@ -593,7 +603,7 @@ __global__ __launch_bounds__(256 * KSP, HD == 64 ? 4 : KEYS == 32 ? 3 : 2) void 
   }
 }
 
-template <int HD, int NWH, int KSP, int KEYS, bool HALF, bool WIN>
+template <int HD, int NWH, int KSP, int KEYS, int HALF, bool WIN>
 static int launch_prefill_as(unsigned workgroups, const u16* q, int64_t ldq, const u16* kc, const u16* vc, const int32_t* pos, u16* y, int64_t ldy,
                              int S, int Hq, int Hkv, int Smax, const WindowKeys& w, hipStream_t s) {
   constexpr size_t lds = PrefillLds<HD, KSP, KEYS>::BYTES;
@@ -609,13 +619,14 @@ static int launch_prefill_heads(const u16* q, int64_t ldq, const u16* kc, const 
   const int64_t n = (int64_t)((S + queries - 1) / queries) * (Hq / NWH) * B;
   const int cus = lr_num_cus();
   const int seen = WIN && w.window < S ? w.window : S;   // keys (at least: how long the history ahead of the queries is only the device knows)
-  auto run = &launch_prefill_as<HD, NWH, 1, 64, true, WIN>;
+  auto run = &launch_prefill_as<HD, NWH, 1, 64, PREFILL_HALF, WIN>;
   if constexpr (HD == 128) {
-    if (n > 2 * cus || (NWH == 2 && S > 32 && S <= 96)) run = &launch_prefill_as<HD, NWH, 1, 32, false, WIN>;
+    if (n > 2 * cus || (NWH == 2 && S > 32 && S <= 96)) run = &launch_prefill_as<HD, NWH, 1, 32, PREFILL_WHOLE, WIN>;
+    else if (S <= 128) run = &launch_prefill_as<HD, NWH, 1, 64, PREFILL_EACH, WIN>;
   } else {
-    if (seen > PREFILL_HALF_TO) run = &launch_prefill_as<HD, NWH, 1, 64, false, WIN>;
+    if (seen > PREFILL_HALF_TO) run = &launch_prefill_as<HD, NWH, 1, 64, PREFILL_WHOLE, WIN>;
   }
-  if (n <= cus && seen >= PREFILL_PARTS_FROM) run = &launch_prefill_as<HD, NWH, 2, 64, false, WIN>;
+  if (n <= cus && seen >= PREFILL_PARTS_FROM) run = &launch_prefill_as<HD, NWH, 2, 64, PREFILL_WHOLE, WIN>;
   return run((unsigned)n, q, ldq, kc, vc, pos, y, ldy, S, Hq, Hkv, Smax, w, s);
 }
 // NWH heads of a kv head in a workgroup: as many of four as divide its share
