@@ -844,9 +844,9 @@ static bool gemm_takes(int tile, int M, int K) {
   if (tile == GEMM_LONG) return M > 64 && M <= 128 && K % 64 == 0;
   return M > 128 && K % 64 == 0;
 }
-// and the two input projections of a block in one grid (K % 64 == 0): q/k/v beside up/gate of 1B, 128 rows, ring of two 29.5 us, of three 28.2
-// (a prompt of 128 tokens 1041 us -> 1019, of 70 935 -> 913).  Its output projections, cut so that every CU has a workgroup, are 64 x 128 there
-// in 17.0 us and would be 18.0 with the long ring: they keep the first four.
+// and the two input projections of a block in one grid (K % 64 == 0): q/k/v beside up/gate of 1B, 128 rows, ring of two 29.5 us, of three 28.2,
+// which the whole prompt of 128 tokens, 1050 us, does not show beyond the 1.5 % that two runs of it differ by.  Its output projections, cut so
+// that every CU has a workgroup, are 64 x 128 there in 17.0 us and would be 18.0 with the long ring: they keep the first four.
 static bool gemm_shares(int tile, int M, int K) { return (tile < GEMM_TILES_ANY || tile == GEMM_LONG) && gemm_takes(tile, M, K); }
 constexpr size_t GEMM_SCRATCH = (size_t)64 << 20;   // pieces of one round of the largest tiles
 constexpr int GEMM_SCRATCH_FROM = 33;               // rows from which a projection that has memory for pieces is one of this file's
